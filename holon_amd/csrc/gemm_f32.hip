@@ -1,93 +1,253 @@
-// y[M, N] = x[M, K] w[N, K]^T in true float32: float32 operands on the matrix cores (v_mfma_f32_32x32x2_f32: no
-// reduced-precision mode), float32 accumulation. This is the product of the 32-bit check path.
+// y[M, N] = x[M, K] w[N, K]^T in true float32: float32 operands on the matrix cores (v_mfma_f32_16x16x4_f32: no
+// reduced-precision mode), float32 accumulation. This is the product of the 32-bit path.
 //
-// Its point is a fixed order of summation. Output element (m, n) is the sum over k of x[m, k] w[n, k] taken in tiles of
-// 32 k, one after the other, and inside a tile in the order the instruction adds its pairs; neither depends on M, on
-// where the row lies in the batch, or on the tile of the output the element falls in (rows and columns beyond the edge
-// are computed on zeros and never stored; a K that is no multiple of 32 is padded with zeros, which add nothing). So
-// a token's result is bit for bit the same whether it runs alone, in a portion of a prompt or in a batch of others.
+// Its point is a fixed order of summation, the same in both kernels below: K is cut into 16 shares of equal length (a
+// multiple of 32, the last ones shorter or empty); a share's sum runs over its k in groups of 16 (the instruction adds
+// k, k + 4, k + 8 and k + 12 of a group at a time), four shares are added up one after the other, and so are the four
+// quarters that makes. None of it depends on M, on where the row lies in the batch, or on the tile of the output the
+// element falls in (rows and columns beyond the edge repeat the last one and are never stored; what lies beyond K is
+// taken as zeros, which add nothing). So a token's result is bit for bit the same whether it runs alone, in a portion
+// of a prompt or in a batch of others.
 //
-// A workgroup of four waves owns a 64 x 64 tile of the output, each wave a 32 x 32 quarter. Per step the workgroup
-// stages 64 rows of x and 64 rows of w, 32 k wide, in LDS (rows padded to 33 floats: a wave's 32 rows then fall in 32
-// different banks).
+// A lane of a matrix instruction's operand holds one float of row lane % 16; here it reads four neighbours in k at once
+// (16 bytes, k = 4 (lane / 16) .. + 3 of a group) and spends them on four instructions.
 #include "common.h"
 #include "holon_hip.h"
 
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 namespace {
-constexpr int TM = 64, TN = 64, TK = 32, PAD = 1;
+constexpr int SHARES = 16, QUARTERS = 4;
+constexpr int GROUP = 16;              // k values of one 16-byte load of every lane
+constexpr int CHUNK = 32;              // k values staged at a time, and what shares are a multiple of
 
-// VEC: K is a multiple of 4 and both operands are 16-byte aligned, so rows are read four floats at a time.
-template <bool VEC>
-__device__ __forceinline__ void stage_rows(const float* __restrict__ src, int rows, int K, int row0, int k0,
-                                           float (*dst)[TK + PAD]) {
-  // 64 rows x 32 floats = 512 groups of four; 256 threads take two each
+__host__ __device__ __forceinline__ int share_length(int K) { return (K + SHARES * CHUNK - 1) / (SHARES * CHUNK) * CHUNK; }
+
+// s[0] .. s[15] in the order above.
+template <typename F>
+__device__ __forceinline__ f32x4_t sum_shares(F s) {
+  f32x4_t total;
 #pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int idx = threadIdx.x + it * 256;
-    const int r = idx / (TK / 4), c = (idx % (TK / 4)) * 4;
-    const int row = row0 + r, k = k0 + c;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (row < rows) {
-      const float* p = src + (int64_t)row * K + k;
-      if (VEC) {
-        if (k < K) v = *reinterpret_cast<const float4*>(p);      // K % 4 == 0: a group is inside or outside whole
-      } else {
-        if (k + 0 < K) v.x = p[0];
-        if (k + 1 < K) v.y = p[1];
-        if (k + 2 < K) v.z = p[2];
-        if (k + 3 < K) v.w = p[3];
-      }
-    }
-    dst[r][c + 0] = v.x; dst[r][c + 1] = v.y; dst[r][c + 2] = v.z; dst[r][c + 3] = v.w;
+  for (int q = 0; q < QUARTERS; ++q) {
+    f32x4_t quarter = s(4 * q);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) quarter += s(4 * q + i);
+    total = q ? total + quarter : quarter;
+  }
+  return total;
+}
+
+// Four results of a row, columns n .. n + 3.
+__device__ __forceinline__ void store4(float* __restrict__ y, f32x4_t v, int m, int n, int M, int N) {
+  if (m >= M) return;
+  float* out = y + (int64_t)m * N + n;
+  if (N % 4 == 0 && (uintptr_t)y % 16 == 0) {
+    if (n < N) *reinterpret_cast<f32x4_t*>(out) = v;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) if (n + i < N) out[i] = v[i];
   }
 }
 
+// Four floats of a row at k. VEC: K is a multiple of 4 and rows are 16-byte aligned.
 template <bool VEC>
-__global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                       float* __restrict__ y, int M, int N, int K) {
-  __shared__ float xs[TM][TK + PAD];
-  __shared__ float ws[TN][TK + PAD];
+__device__ __forceinline__ f32x4_t load4(const float* __restrict__ row, int k, int K) {
+  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (VEC) {
+    if (k < K) v = *reinterpret_cast<const f32x4_t*>(row + k);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) if (k + i < K) v[i] = row[k + i];
+  }
+  return v;
+}
+
+// Steps of few rows. A block owns MT x NT tiles of 16 x 16 results; each of its 16 waves takes one share of K, and the waves' sums are added in
+// order through LDS. Operands go from memory straight to registers, DEPTH groups of k of a wave under way at a time; 16
+// waves on four SIMDs cover each other's loads, so nothing is staged and no wave waits for another before the end. With
+// few rows that streams the weights (bound by memory: a lane has DEPTH 16-byte loads in flight); with many the matrix
+// cores bound it, as a group of k is 4 MT NT instructions of 32 cycles for MT + NT loads.
+template <int MT, int NT, int DEPTH, bool VEC>
+__global__ void __launch_bounds__(SHARES * WAVE) gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                  float* __restrict__ y, int M, int N, int K) {
+  __shared__ f32x4_t part[SHARES][MT * NT][WAVE];
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int wm = wave / 2, wn = wave % 2;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int r = lane % 32, half = lane / 32;
-  f32x16_t acc;
+  const int g = lane / 16, c = lane % 16;
+  const int n0 = blockIdx.x * NT * 16, m0 = blockIdx.y * MT * 16;
+  const int share = share_length(K);
+  const int first = wave * share, last = min(K, first + share);
+  const float *wr[NT], *xr[MT];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-  for (int k0 = 0; k0 < K; k0 += TK) {
-    stage_rows<VEC>(x, M, K, m0, k0, xs);
-    stage_rows<VEC>(w, N, K, n0, k0, ws);
-    __syncthreads();
+  for (int u = 0; u < NT; ++u) wr[u] = w + (int64_t)min(n0 + u * 16 + c, N - 1) * K;
 #pragma unroll
-    for (int kk = 0; kk < TK; kk += 2) {
-      const float a = xs[wm * 32 + r][kk + half];
-      const float b = ws[wn * 32 + r][kk + half];
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+  for (int t = 0; t < MT; ++t) xr[t] = x + (int64_t)min(m0 + t * 16 + c, M - 1) * K;
+  f32x4_t acc[MT][NT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int u = 0; u < NT; ++u) acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = first; k0 < last; k0 += DEPTH * GROUP) {
+    f32x4_t a[DEPTH][NT], b[DEPTH][MT];
+#pragma unroll
+    for (int s = 0; s < DEPTH; ++s) {                     // (beyond the share: zeros, which add nothing)
+      const int k = k0 + s * GROUP + 4 * g;
+#pragma unroll
+      for (int u = 0; u < NT; ++u) a[s][u] = load4<VEC>(wr[u], k, last);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) b[s][t] = load4<VEC>(xr[t], k, last);
     }
-    __syncthreads();
-  }
-  // lane holds column n = r of rows 8 (i / 4) + 4 half + i % 4
-  const int n = n0 + wn * 32 + r;
-  if (n >= N) return;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int m = m0 + wm * 32 + 8 * (i / 4) + 4 * half + i % 4;
-    if (m < M) y[(int64_t)m * N + n] = acc[i];
+    for (int s = 0; s < DEPTH; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+          for (int u = 0; u < NT; ++u)
+            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][u][i], b[s][t][i], acc[t][u], 0, 0, 0);
   }
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int u = 0; u < NT; ++u) part[wave][t * NT + u][lane] = acc[t][u];
+  __syncthreads();
+  // lane holds columns 4 g .. 4 g + 3 of row c of tile `wave`
+  if (wave >= MT * NT) return;
+  const f32x4_t sum = sum_shares([&](int i) { return part[i][wave][lane]; });
+  store4(y, sum, m0 + wave / NT * 16 + c, n0 + wave % NT * 16 + 4 * g, M, N);
+}
+
+// More rows: bound by the matrix cores. A block owns 64 x 64 results with four waves (32 x 32 each) for every quarter of
+// K, which stage their quarter's rows of x and w in LDS, CHUNK of k at a time, into one of two buffers while the other is
+// multiplied; pieces of 16 bytes lie at place p ^ (row % 8) of their row. Splitting K inside the block is what fills the
+// chip where an output of some hundred rows has few tiles, and four waves a SIMD cover each other's barriers.
+template <bool VEC>
+__global__ void __launch_bounds__(1024) gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                        float* __restrict__ y, int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) float stage[QUARTERS][2][2][64 * CHUNK];   // quarter, buffer, x or w
+  const int quarter = threadIdx.x / 256, tid = threadIdx.x % 256;
+  const int wave = tid / WAVE, lane = tid % WAVE;
+  const int g = lane / 16, c = lane % 16;
+  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+  const int share = share_length(K), first = quarter * 4 * share, chunks = 4 * share / CHUNK, per_share = share / CHUNK;
+  // what this thread stages: rows tid / 8 and 32 more, piece tid % 8
+  const int r0 = tid / 8, p0 = tid % 8;
+  const float *xr[2], *wr[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    xr[i] = x + (int64_t)min(m0 + r0 + 32 * i, M - 1) * K;
+    wr[i] = w + (int64_t)min(n0 + r0 + 32 * i, N - 1) * K;
+  }
+  const int put = r0 * CHUNK + 4 * (p0 ^ (r0 % 8));
+  f32x4_t held[2][2];
+  auto fetch = [&](int chunk) {
+    const int k = first + chunk * CHUNK + 4 * p0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      held[0][i] = load4<VEC>(xr[i], k, K);
+      held[1][i] = load4<VEC>(wr[i], k, K);
+    }
+  };
+  auto keep = [&](int buf) {
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4_t*>(&stage[quarter][buf][o][put + 32 * i * CHUNK]) = held[o][i];
+  };
+  // where this lane reads: row 32 (half) + 16 t + c, pieces g and 4 + g
+  const int xrow = wave / 2 * 32 + c, wrow = wave % 2 * 32 + c;
+  const int at[2] = {4 * (g ^ (c % 8)), 4 * ((4 + g) ^ (c % 8))};
+  f32x4_t acc[2][2], total[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) acc[t][u] = total[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  fetch(0);
+  keep(0);
+  if (chunks > 1) fetch(1);
+  lds_barrier();
+  int left = per_share;
+  bool begun = false;                                     // whether `total` holds a share
+  for (int ch = 0; ch < chunks; ++ch) {
+    if (ch + 1 < chunks) keep((ch + 1) & 1);              // (read last in front of the barrier behind us)
+    if (ch + 2 < chunks) fetch(ch + 2);
+    const float* xs = stage[quarter][ch & 1][0];
+    const float* ws = stage[quarter][ch & 1][1];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      f32x4_t b[2], a[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) b[t] = *reinterpret_cast<const f32x4_t*>(&xs[(xrow + 16 * t) * CHUNK + at[s]]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) a[u] = *reinterpret_cast<const f32x4_t*>(&ws[(wrow + 16 * u) * CHUNK + at[s]]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[t][i], acc[t][u], 0, 0, 0);
+    }
+    if (--left == 0) {                                    // a share ends
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          total[t][u] = begun ? total[t][u] + acc[t][u] : acc[t][u];
+          acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+      left = per_share;
+      begun = true;
+    }
+    lds_barrier();                                        // (what was fetched stays under way)
+  }
+  // the quarters' sums through LDS: tile (4 t' + u') of the block's 16, one a wave
+  f32x4_t(*part)[16][WAVE] = reinterpret_cast<f32x4_t(*)[16][WAVE]>(&stage[0][0][0][0]);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) part[quarter][(wave / 2 * 2 + t) * 4 + wave % 2 * 2 + u][lane] = total[t][u];
+  __syncthreads();
+  const int tile = quarter * 4 + wave;
+  f32x4_t sum = part[0][tile][lane];
+#pragma unroll
+  for (int q = 1; q < QUARTERS; ++q) sum += part[q][tile][lane];
+  store4(y, sum, m0 + tile / 4 * 16 + c, n0 + tile % 4 * 16 + 4 * g, M, N);
+}
+
+// Which tile a product takes: the one whose rounds of one block a CU are done first. A round's time over K = 2,048 on
+// MI355X, in us (in proportion for other K): 1 x 1 tiles 9.3, 1 x 2 15.5, 2 x 2 20.5, 2 x 4 33.5, and 42 for the staged 4 x 4
+// (0.8 of the float32 peak where the last round is full). So 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10 us; with a
+// 64 x 64 tile a block and no split of K it took 118) and the staged kernel from 300 rows (45 us; 126), 16384 x 2048 1 x 1
+// tiles up to 16 rows (27 to 39 us, 5.0 TB/s at one row; 116 to 120) and the staged one from 48 (46 us at 64 rows; 145).
+template <bool VEC>
+void launch(const float* x, const float* w, float* y, int M, int N, int K, hipStream_t s) {
+  const auto cost = [&](int mt, int nt, float round) {
+    const int64_t blocks = (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt));
+    return (float)((blocks + 255) / 256) * round;
+  };
+  const float few[4] = {cost(1, 1, 9.3f), cost(1, 2, 15.5f), cost(2, 2, 20.5f), cost(2, 4, 33.5f)};
+  int best = 0;
+  for (int i = 1; i < 4; ++i) if (M > 16 && few[i] < few[best]) best = i;
+#define F32_ROWS(MT, NT, DEPTH)                                                                                     \
+  gemm_f32_rows_kernel<MT, NT, DEPTH, VEC><<<dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)),    \
+                                             SHARES * WAVE, 0, s>>>(x, w, y, M, N, K)
+  if (M > 16 && (cost(4, 4, 42.f) <= few[best] || (M + 15) / 16 > 65535))
+    gemm_f32_kernel<VEC><<<dim3((N + 63) / 64, (M + 63) / 64), 1024, 0, s>>>(x, w, y, M, N, K);
+  else if (best == 0) F32_ROWS(1, 1, 2);
+  else if (best == 1) F32_ROWS(1, 2, 1);
+  else if (best == 2) F32_ROWS(2, 2, 1);
+  else F32_ROWS(2, 4, 1);
+#undef F32_ROWS
 }
 }  // namespace
 
 extern "C" int holon_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, void* stream) {
   HOLON_CHECK(M >= 0 && N > 0 && K > 0, "gemm (float32): M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
-  const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
-  HOLON_CHECK(grid.y <= 65535, "gemm (float32): M=%d rows exceed one launch (%d)", M, 65535 * TM);
+  HOLON_CHECK((M + 63) / 64 <= 65535, "gemm (float32): M=%d rows exceed one launch (%d)", M, 65535 * 64);
   const bool vec = K % 4 == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
-  hipStream_t s = (hipStream_t)stream;
-  if (vec) gemm_f32_kernel<true><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, (float*)y, M, N, K);
-  else gemm_f32_kernel<false><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, (float*)y, M, N, K);
+  if (vec) launch<true>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
+  else launch<false>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
   HOLON_LAUNCH_OK();
   return 0;
 }

@@ -630,6 +630,23 @@ def test_float32_product_is_true_32_bit_and_its_order_is_fixed(hip):
     assert torch.equal(hip.linear(x, w), x @ w.T)                                 # exact arithmetic: any order, same bits
 
 
+@pytest.mark.parametrize("m", (16, 17, 33, 64, 65, 96, 130, 300))
+def test_float32_product_across_its_tiles(hip, m):
+    """Every tile the float32 product chooses between, at the edges of its rows, columns, shares and chunks of K: against
+    the float64 product, and each row bit for bit what it is alone. A sum of
+    K / 16 products a share, then 16 shares: its error stays below (K / 16 + 20) 2^-24 sum |x w|."""
+    for k, n in ((30, 97), (32, 16), (36, 200), (512, 48), (544, 1000), (2080, 64), (1100, 3072), (256, 16384)):
+        x, w = _randn(m, k, dtype=torch.float32, seed=44), _randn(n, k, dtype=torch.float32, seed=45)
+        got, want = hip.linear(x, w), x.double() @ w.double().T
+        bound = (k / 16 + 20) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        assert ((got.double() - want).abs() <= bound).all(), (m, k, n)
+        for row in (0, 15, m - 1):
+            assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), (m, k, n, row)
+        odd = torch.empty(m * k + 1, device=x.device)[1:].view(m, k)              # rows that start on no 16-byte border
+        odd.copy_(x)
+        assert torch.equal(hip.linear(odd, w), got), (m, k, n)
+
+
 def test_norm_folded_into_the_product(hip):
     """The norm's weight folded into the tiled copy, the rows scaled inside the product from statistics another kernel
     left: against norm then product in float64, within the budget of the two operations; the statistics from the

@@ -72,6 +72,7 @@ struct GlaRows {
   const int32_t* base;         // [rows]: the number of row b's first piece among all pieces of the step
   float* sloc;                 // [pieces, H, D, V]: what a piece adds; after the walk, the state behind it
   float* pw;                   // [pieces, H, D]: the product of a piece's decays
+  const float* bonus;          // [H, D], BONUS alone: the weights of a token's own key in its read-out
 };
 
 template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
@@ -80,7 +81,10 @@ template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
 
 // A block: one (row or piece, head) and 16 NW value columns, wave w columns 16 w .. 16 w + 15 of them, S's KD x 16 part of
 // a wave in its matrix-core accumulators. KD: the key size padded with zeros (a zero key writes nothing).
-template <int KD, int NW, int PASS, typename T>
+// BONUS: the read-out comes before the write and the token's own key enters it with weights of its own,
+//   o_t = (S + diag(u) k_t v_t^T)^T q_t,  S <- diag(alpha) S + k_t v_t^T:
+// p_t then leaves t itself out, a score's decays run from behind j to in front of t, and the diagonal scores take u k_t.
+template <int KD, int NW, int PASS, bool BONUS, typename T>
 __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                              const T* __restrict__ v, int64_t stride, float q_scale,
                                                              const float* __restrict__ alpha, float* __restrict__ state,
@@ -91,7 +95,7 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
   static_assert(N % THREADS == 0 && KD == 4 * VW * NW * U, "whole tiles");
   __shared__ __attribute__((aligned(16))) float as_[N], ks_[N], qs_[OUT ? N : 4];
   __shared__ __attribute__((aligned(16))) float qp_[OUT ? TB * QP : 4], kt_[KD * TP], P_[KD];
-  __shared__ __attribute__((aligned(16))) float red_[OUT ? NW * TB * TB : 4];
+  __shared__ __attribute__((aligned(16))) float red_[OUT ? NW * TB * TB : 4], us_[BONUS ? KD : 4];
   const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   const int g4 = lane / 16, c = lane % 16;
   const int col_blocks = (r.vdim + 16 * NW - 1) / (16 * NW);
@@ -100,8 +104,9 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
   int lo = r.query_start[b], hi = r.query_start[b + 1];
   bool from_slot = true, to_slot = OUT;
   int64_t piece_no = 0;
+  int pieces = 1;
   if (r.piece > 0) {                                       // (everything here is the same in all of the block's lanes)
-    const int pieces = (hi - lo + r.piece - 1) / r.piece;
+    pieces = (hi - lo + r.piece - 1) / r.piece;
     if (piece >= pieces || (PASS == 1 && piece == pieces - 1)) return;
     lo += piece * r.piece;
     hi = min(hi, lo + r.piece);
@@ -111,18 +116,19 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
   }
   float* held = state + ((int64_t)r.slots[b] * r.heads + h) * dim * vdim;
   const bool carried = r.starts[b] > 0;
+  const float* before = pieces == 1 ? held : r.sloc + ((piece_no + (from_slot ? pieces : 0) - 1) * r.heads + h) * dim * vdim;
+  const bool some = OUT && (!from_slot || carried);        // whether there is a state to start from
   const int j = col0 + 16 * wave + c;                      // this lane's value column
   const bool col = j < vdim;
+  if constexpr (BONUS)
+    for (int d = tid; d < KD; d += THREADS) us_[d] = d < dim ? r.bonus[(int64_t)h * dim + d] : 0.f;
   f32x4 S[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int d = 16 * dt + 4 * g4 + i;
-      const bool in = OUT && col && d < dim;
-      S[dt][i] = !in ? 0.f
-                     : (from_slot ? (carried ? held[(int64_t)d * vdim + j] : 0.f)
-                                  : r.sloc[((piece_no - 1) * r.heads + h) * dim * vdim + (int64_t)d * vdim + j]);
+      S[dt][i] = some && col && d < dim ? before[(int64_t)d * vdim + j] : 0.f;
     }
   float run = 1.f;                                         // PASS 1, thread d: the product of the piece's decays so far
   const int64_t width = (int64_t)r.heads * dim;
@@ -181,17 +187,23 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
         float p = 1.f;
 #pragma unroll
         for (int t = 0; t < TB; ++t) {
-          p *= a[t];
-          qp_[t * QP + d] = x[t] * p;
+          if constexpr (BONUS) {
+            qp_[t * QP + d] = x[t] * p;
+            p *= a[t];
+          } else {
+            p *= a[t];
+            qp_[t * QP + d] = x[t] * p;
+          }
         }
       }
     }
     if constexpr (OUT) {                                   // the block's scores, every wave over its channels
       typedef float fv __attribute__((ext_vector_type(VW)));
       const int jj = lane / 4, part = lane % 4;            // lane (jj, part): key jj, channels ((u NW + wave) 4 + part) VW ..
-      fv kj[U], car[U];
+      fv kj[U], car[U], own[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        if constexpr (BONUS) own[u] = *reinterpret_cast<const fv*>(&us_[((u * NW + wave) * 4 + part) * VW]);
         kj[u] = *reinterpret_cast<const fv*>(&ks_[jj * KD + ((u * NW + wave) * 4 + part) * VW]);
         car[u] = (fv)0.f;
       }
@@ -205,9 +217,14 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
           const fv at = *reinterpret_cast<const fv*>(&as_[t * KD + d]);
           const fv qt = *reinterpret_cast<const fv*>(&qs_[t * KD + d]);
 #pragma unroll
-          for (int i = 0; i < VW; ++i) {
-            car[u][i] = jj == t ? kj[u][i] : car[u][i] * at[i];        // (0 until the key's own token)
-            dot[t] += qt[i] * car[u][i];
+          for (int i = 0; i < VW; ++i) {                   // (0 until the key's own token)
+            if constexpr (BONUS) {
+              dot[t] += qt[i] * (jj == t ? kj[u][i] * own[u][i] : car[u][i]);
+              car[u][i] = jj == t ? kj[u][i] : car[u][i] * at[i];
+            } else {
+              car[u][i] = jj == t ? kj[u][i] : car[u][i] * at[i];
+              dot[t] += qt[i] * car[u][i];
+            }
           }
         }
       }
@@ -268,8 +285,9 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
   }
 }
 
-// Between the passes: a row's pieces in order, S <- diag(pw) S + sloc; sloc[p] becomes the state piece p + 1 starts from.
-// A thread an element; the pieces' values are asked for four at a time.
+// Between the passes: a row's pieces in order, S <- diag(pw) S + sloc; sloc[p] becomes the state piece p + 1 starts from, and
+// the last piece's place, which nothing adds to, takes the state the row starts from (the slot may no longer hold it when
+// piece 0 comes to read it). A thread an element; the pieces' values are asked for four at a time.
 __global__ void __launch_bounds__(256) gla_walk_kernel(const float* __restrict__ state, GlaRows r) {
   const int b = blockIdx.x, h = blockIdx.y, e = blockIdx.z * 256 + threadIdx.x;
   const int cells = r.dim * r.vdim;
@@ -277,6 +295,7 @@ __global__ void __launch_bounds__(256) gla_walk_kernel(const float* __restrict__
   const int pieces = (r.query_start[b + 1] - r.query_start[b] + r.piece - 1) / r.piece;
   const int row = e / r.vdim;
   float s = r.starts[b] > 0 ? state[((int64_t)r.slots[b] * r.heads + h) * cells + e] : 0.f;
+  if (pieces > 1) r.sloc[(((int64_t)r.base[b] + pieces - 1) * r.heads + h) * cells + e] = s;
   for (int p0 = 0; p0 + 1 < pieces; p0 += 4) {
     float add[4], w[4];
 #pragma unroll
@@ -428,15 +447,51 @@ extern "C" int holon_gla_decay(const void* a, int64_t a_stride, const void* w2t,
   return 0;
 }
 
-template <int KD, int NW, typename T>
+template <int KD, int NW, bool BONUS, typename T>
 static void launch_gla(int pass, dim3 grid, hipStream_t s, const void* q, const void* k, const void* v, int64_t stride,
                        float q_scale, const float* alpha, float* state, float* out, GlaRows r) {
-  if (pass == 1)
-    gla_scan_kernel<KD, NW, 1, T><<<grid, NW * WAVE, 0, s>>>((const T*)q, (const T*)k, (const T*)v, stride, q_scale, alpha,
-                                                             state, out, r);
+  if (pass == 1)                                           // (what a piece adds does not depend on how it is read)
+    gla_scan_kernel<KD, NW, 1, false, T><<<grid, NW * WAVE, 0, s>>>((const T*)q, (const T*)k, (const T*)v, stride, q_scale,
+                                                                    alpha, state, out, r);
   else
-    gla_scan_kernel<KD, NW, 2, T><<<grid, NW * WAVE, 0, s>>>((const T*)q, (const T*)k, (const T*)v, stride, q_scale, alpha,
-                                                             state, out, r);
+    gla_scan_kernel<KD, NW, 2, BONUS, T><<<grid, NW * WAVE, 0, s>>>((const T*)q, (const T*)k, (const T*)v, stride, q_scale,
+                                                                    alpha, state, out, r);
+}
+
+template <bool BONUS>
+static int scan_rows(const char* what, const void* q, const void* k, const void* v, int64_t stride, float q_scale,
+                     const float* alpha, float* state, float* out, int rows, int dtype, int max_pieces, GlaRows r,
+                     hipStream_t s) {
+  const int heads = r.heads, dim = r.dim, vdim = r.vdim;
+  const int nw = vdim <= 64 ? 4 : 8;
+  const int col_blocks = (vdim + 16 * nw - 1) / (16 * nw);
+  const int most = r.piece ? max_pieces : 1;
+  HOLON_CHECK((int64_t)col_blocks * most <= 65535 && ((int64_t)dim * vdim + 255) / 256 <= 65535,
+              "%s: %d pieces of %d x %d exceed one launch", what, most, dim, vdim);
+  const dim3 grid(rows, heads, col_blocks * most);
+#define GLA_NW(PASS, KD)                                                                                              \
+  do {                                                                                                                \
+    if (nw == 4) launch_gla<KD, 4, BONUS, T>(PASS, grid, s, q, k, v, stride, q_scale, alpha, state, out, r);           \
+    else launch_gla<KD, 8, BONUS, T>(PASS, grid, s, q, k, v, stride, q_scale, alpha, state, out, r);                   \
+  } while (0)
+#define GLA(PASS)                                                                                                     \
+  do {                                                                                                                \
+    if (dim <= 32) BY_DTYPE(dtype, GLA_NW(PASS, 32));                                                                  \
+    else if (dim <= 64) BY_DTYPE(dtype, GLA_NW(PASS, 64));                                                             \
+    else if (dim <= 128) BY_DTYPE(dtype, GLA_NW(PASS, 128));                                                           \
+    else BY_DTYPE(dtype, GLA_NW(PASS, 256));                                                                           \
+  } while (0)
+  if (r.piece) {
+    GLA(1);
+    HOLON_LAUNCH_OK();
+    gla_walk_kernel<<<dim3(rows, heads, (dim * vdim + 255) / 256), 256, 0, s>>>(state, r);
+    HOLON_LAUNCH_OK();
+  }
+  GLA(2);
+#undef GLA
+#undef GLA_NW
+  HOLON_LAUNCH_OK();
+  return 0;
 }
 
 extern "C" int holon_gla_scan(const void* q, const void* k, const void* v, int64_t stride, float q_scale, const float* alpha,
@@ -451,37 +506,19 @@ extern "C" int holon_gla_scan(const void* q, const void* k, const void* v, int64
   HOLON_CHECK(piece_tokens == 0 || (piece_tokens > 0 && piece_tokens % 16 == 0 && max_pieces > 0 && piece_base && sloc && pw),
               "gla_scan: rows in pieces of %d tokens (a multiple of 16) need the pieces' table and workspace", piece_tokens);
   if (rows == 0) return 0;
-  hipStream_t s = (hipStream_t)stream;
-  const GlaRows r{slots, starts, query_start, heads, dim, vdim, piece_tokens, piece_base, sloc, pw};
-  const int nw = vdim <= 64 ? 4 : 8;
-  const int col_blocks = (vdim + 16 * nw - 1) / (16 * nw);
-  const int most = piece_tokens ? max_pieces : 1;
-  HOLON_CHECK((int64_t)col_blocks * most <= 65535 && ((int64_t)dim * vdim + 255) / 256 <= 65535,
-              "gla_scan: %d pieces of %d x %d exceed one launch", most, dim, vdim);
-  const dim3 grid(rows, heads, col_blocks * most);
-#define GLA_NW(PASS, KD)                                                                                              \
-  do {                                                                                                                \
-    if (nw == 4) launch_gla<KD, 4, T>(PASS, grid, s, q, k, v, stride, q_scale, alpha, state, out, r);                  \
-    else launch_gla<KD, 8, T>(PASS, grid, s, q, k, v, stride, q_scale, alpha, state, out, r);                          \
-  } while (0)
-#define GLA(PASS)                                                                                                     \
-  do {                                                                                                                \
-    if (dim <= 32) BY_DTYPE(dtype, GLA_NW(PASS, 32));                                                                  \
-    else if (dim <= 64) BY_DTYPE(dtype, GLA_NW(PASS, 64));                                                             \
-    else if (dim <= 128) BY_DTYPE(dtype, GLA_NW(PASS, 128));                                                           \
-    else BY_DTYPE(dtype, GLA_NW(PASS, 256));                                                                           \
-  } while (0)
-  if (piece_tokens) {
-    GLA(1);
-    HOLON_LAUNCH_OK();
-    gla_walk_kernel<<<dim3(rows, heads, (dim * vdim + 255) / 256), 256, 0, s>>>(state, r);
-    HOLON_LAUNCH_OK();
-  }
-  GLA(2);
-#undef GLA
-#undef GLA_NW
-  HOLON_LAUNCH_OK();
-  return 0;
+  const GlaRows r{slots, starts, query_start, heads, dim, vdim, piece_tokens, piece_base, sloc, pw, nullptr};
+  return scan_rows<false>("gla_scan", q, k, v, stride, q_scale, alpha, state, out, rows, dtype, max_pieces, r,
+                          (hipStream_t)stream);
+}
+
+// The decayed memory's rows in pieces (holon_memory_scan, which has checked the arguments).
+int holon_memory_scan_pieces(const void* q, const void* k, const void* v, const float* w, const float* u, float* state,
+                             float* out, const int32_t* slots, const int32_t* starts, const int32_t* query_start, int rows,
+                             int heads, int dim, int dtype, int piece_tokens, int max_pieces, const int32_t* piece_base,
+                             float* sloc, float* pw, void* stream) {
+  const GlaRows r{slots, starts, query_start, heads, dim, dim, piece_tokens, piece_base, sloc, pw, u};
+  return scan_rows<true>("memory_scan", q, k, v, (int64_t)heads * dim, 1.f, w, state, out, rows, dtype, max_pieces, r,
+                         (hipStream_t)stream);
 }
 
 extern "C" int holon_gla_step_supported(int dim, int vdim) {

@@ -462,59 +462,32 @@ __global__ void __launch_bounds__(256) delta_pieces_kernel(const float* __restri
   }
 }
 
-// A long row's tokens in pieces that run side by side (the memory's recurrence is linear in S and its decays do not
-// depend on S): every piece but a row's last first runs from S = 0 and leaves what it adds (`sloc`) and the product of
-// its decays per key row (`pw`); a small kernel then walks a row's pieces in order, S <- diag(pw) S + sloc, leaving
-// each piece's true starting state in place of `sloc`; then every piece runs again from there and writes its outputs.
-struct ScanPieces {
-  int tokens;                  // tokens a piece (0: rows are not cut)
-  int mode;                    // 1: from zero, leave sloc and pw; 2: from the true start, write outputs
-  const int32_t* base;         // [rows]: the number of row b's first piece among all pieces of the step
-  float* sloc;                 // [pieces, H, D, D]
-  float* pw;                   // [pieces, H, D]
-};
-
-// Per (row, head): o = (S + diag(u) k v^T)^T r; S <- diag(w) S + k v^T. The same split of S [D, D] over lanes.
+// Per (row, head): o = (S + diag(u) k v^T)^T r; S <- diag(w) S + k v^T. The same split of S [D, D] over lanes. (Rows in
+// pieces go on the matrix cores: `holon_memory_scan_pieces`. Short rows stay here, where every sum's order is the token's
+// alone.)
 template <int KD, typename T>
 __global__ void __launch_bounds__(WAVE) memory_scan_kernel(const T* __restrict__ r, const T* __restrict__ k,
                                                            const T* __restrict__ v, const float* __restrict__ w,
                                                            const float* __restrict__ u, float* __restrict__ state,
                                                            float* __restrict__ out, const int32_t* __restrict__ slots,
                                                            const int32_t* __restrict__ starts,
-                                                           const int32_t* __restrict__ query_start, int heads, int dim,
-                                                           ScanPieces pc) {
+                                                           const int32_t* __restrict__ query_start, int heads, int dim) {
   constexpr int KQ = KD / SCAN_PARTS, TC = ScanChunk<KD, 3>::kTokens, N = TC * KD, PER = (N + WAVE - 1) / WAVE;
   constexpr int VPER = (TC * SCAN_COLS + WAVE - 1) / WAVE;
   __shared__ __attribute__((aligned(16))) float rs[2][N], ks[2][N], ws[2][N], us[KD];
   __shared__ float vs[2][TC * SCAN_COLS];
   const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int col_blocks = (dim + SCAN_COLS - 1) / SCAN_COLS;
-  const int piece = blockIdx.z / col_blocks, col_block = blockIdx.z % col_blocks;
+  const int col_block = blockIdx.z;
   const int part = lane % SCAN_PARTS, col = lane / SCAN_PARTS, j = col_block * SCAN_COLS + col;
   const bool active = j < dim;
-  int lo = query_start[b], hi = query_start[b + 1];
-  bool from_slot = true, to_slot = true;
-  int64_t piece_no = 0;
-  if (pc.tokens > 0) {                                   // (everything here is the same in all of the block's lanes)
-    const int pieces = (hi - lo + pc.tokens - 1) / pc.tokens;
-    if (piece >= pieces || (pc.mode == 1 && piece == pieces - 1)) return;
-    lo += piece * pc.tokens;
-    hi = min(hi, lo + pc.tokens);
-    from_slot = piece == 0;
-    to_slot = pc.mode == 2 && piece == pieces - 1;
-    piece_no = pc.base[b] + piece;
-  }
+  const int lo = query_start[b], hi = query_start[b + 1];
   float* held = state + ((int64_t)slots[b] * heads + h) * dim * dim;
   const bool carried = starts[b] > 0;
-  float S[KQ], pw[KQ];
+  float S[KQ];
 #pragma unroll
   for (int i = 0; i < KQ; ++i) {
     const int row = part * KQ + i;
-    const bool in = active && row < dim;
-    pw[i] = 1.f;
-    if (pc.tokens > 0 && pc.mode == 1) S[i] = 0.f;
-    else if (from_slot) S[i] = (carried && in) ? held[(int64_t)row * dim + j] : 0.f;
-    else S[i] = in ? pc.sloc[((piece_no - 1) * heads + h) * dim * dim + (int64_t)row * dim + j] : 0.f;
+    S[i] = carried && active && row < dim ? held[(int64_t)row * dim + j] : 0.f;
   }
   for (int i = lane; i < KD; i += WAVE) us[i] = i < dim ? u[h * dim + i] : 0.f;
   const int64_t width = (int64_t)heads * dim;
@@ -553,7 +526,6 @@ __global__ void __launch_bounds__(WAVE) memory_scan_kernel(const T* __restrict__
     put(0);
   }
   __syncthreads();
-  const bool local = pc.tokens > 0 && pc.mode == 1;
   for (int t0 = lo, buf = 0; t0 < hi; t0 += TC, buf ^= 1) {
     if (t0 + TC < hi) ask(t0 + TC);
     const int nt = min(TC, hi - t0);
@@ -563,14 +535,6 @@ __global__ void __launch_bounds__(WAVE) memory_scan_kernel(const T* __restrict__
       const float* kt = &ks[buf][tt * KD + part * KQ];
       const float* wt = &ws[buf][tt * KD + part * KQ];
       const float* ut = &us[part * KQ];
-      if (local) {                       // what the piece adds to S, and its decays' product; no output yet
-#pragma unroll
-        for (int i = 0; i < KQ; ++i) {
-          S[i] = wt[i] * S[i] + kt[i] * vt;
-          pw[i] *= wt[i];
-        }
-        continue;
-      }
       float o = 0.f;
 #pragma unroll
       for (int i = 0; i < KQ; ++i) {
@@ -588,34 +552,7 @@ __global__ void __launch_bounds__(WAVE) memory_scan_kernel(const T* __restrict__
   for (int i = 0; i < KQ; ++i) {
     const int row = part * KQ + i;
     if (!active || row >= dim) continue;
-    if (local) {
-      pc.sloc[(piece_no * heads + h) * dim * dim + (int64_t)row * dim + j] = S[i];
-      if (j == 0) pc.pw[(piece_no * heads + h) * dim + row] = pw[i];
-    } else if (to_slot) {
-      held[(int64_t)row * dim + j] = S[i];
-    }
-  }
-}
-
-// Between the two passes: a row's pieces in order. sloc[p] becomes the state piece p + 1 starts from.
-__global__ void __launch_bounds__(256) memory_pieces_kernel(const float* __restrict__ state,
-                                                            const int32_t* __restrict__ slots,
-                                                            const int32_t* __restrict__ starts,
-                                                            const int32_t* __restrict__ query_start, int heads, int dim,
-                                                            ScanPieces pc) {
-  const int b = blockIdx.x, h = blockIdx.y;
-  const int pieces = (query_start[b + 1] - query_start[b] + pc.tokens - 1) / pc.tokens;
-  const float* held = state + ((int64_t)slots[b] * heads + h) * dim * dim;
-  const bool carried = starts[b] > 0;
-  for (int e = threadIdx.x; e < dim * dim; e += 256) {
-    const int row = e / dim;
-    float s = carried ? held[e] : 0.f;
-    for (int p = 0; p + 1 < pieces; ++p) {
-      const int64_t at = (int64_t)pc.base[b] + p;
-      float* add = pc.sloc + (at * heads + h) * dim * dim + e;
-      s = pc.pw[(at * heads + h) * dim + row] * s + *add;
-      *add = s;
-    }
+    held[(int64_t)row * dim + j] = S[i];
   }
 }
 
@@ -838,11 +775,21 @@ extern "C" int holon_delta_scan(const float* qn, const float* kn, const void* qk
 template <typename T, int KD>
 static void launch_memory(dim3 grid, hipStream_t s, const void* r, const void* k, const void* v,
                           const float* w, const float* u, float* state, float* out, const int32_t* slots,
-                          const int32_t* starts, const int32_t* qs, int heads, int dim, ScanPieces pc) {
+                          const int32_t* starts, const int32_t* qs, int heads, int dim) {
   memory_scan_kernel<KD, T><<<grid, WAVE, 0, s>>>((const T*)r, (const T*)k, (const T*)v, w, u, state, out, slots,
-                                                     starts, qs, heads, dim, pc);
+                                                     starts, qs, heads, dim);
 }
 
+int holon_memory_scan_pieces(const void* q, const void* k, const void* v, const float* w, const float* u, float* state,
+                             float* out, const int32_t* slots, const int32_t* starts, const int32_t* query_start, int rows,
+                             int heads, int dim, int dtype, int piece_tokens, int max_pieces, const int32_t* piece_base,
+                             float* sloc, float* pw, void* stream);
+
+// Rows in pieces (the recurrence is linear in S and its decays do not depend on S): every piece but a row's last first runs
+// from S = 0 and leaves what it adds and the product of its decays per key row; a walk over a row's pieces in order leaves
+// each piece's true start; then every piece runs from there and writes its outputs. A layer of 32 heads of 64 over one row
+// of 2,048 tokens: 17 + 7 + 38 us in blocks of 16 tokens on the float32 matrix cores, 153 + 65 + 153 token by token with S
+// in registers.
 extern "C" int holon_memory_scan(const void* r, const void* k, const void* v, const float* w, const float* u,
                                  float* state, float* out, const int32_t* slots, const int32_t* starts,
                                  const int32_t* query_start, int rows, int heads, int dim, int state_slots, int dtype,
@@ -853,27 +800,13 @@ extern "C" int holon_memory_scan(const void* r, const void* k, const void* v, co
   HOLON_CHECK(piece_tokens == 0 || (piece_tokens > 0 && max_pieces > 0 && piece_base && sloc && pw),
               "memory_scan: rows in pieces of %d tokens need the pieces' table and workspace", piece_tokens);
   if (rows == 0) return 0;
-  const int col_blocks = (dim + SCAN_COLS - 1) / SCAN_COLS;
+  if (piece_tokens)
+    return holon_memory_scan_pieces(r, k, v, w, u, state, out, slots, starts, query_start, rows, heads, dim, dtype, piece_tokens,
+                                    max_pieces, piece_base, sloc, pw, stream);
   hipStream_t s = (hipStream_t)stream;
-  ScanPieces pc{piece_tokens, 0, piece_base, sloc, pw};
-  if (piece_tokens == 0) {
-    const dim3 grid(rows, heads, col_blocks);
-    BY_DTYPE(dtype, BY_KEY_SIZE(dim, (launch_memory<T, KD>(grid, s, r, k, v, w, u, state, out, slots, starts,
-                                                            query_start, heads, dim, pc))));
-    HOLON_LAUNCH_OK();
-    return 0;
-  }
-  HOLON_CHECK((int64_t)col_blocks * max_pieces <= 65535, "memory_scan: %d pieces a row exceed one launch", max_pieces);
-  const dim3 grid(rows, heads, col_blocks * max_pieces);
-  pc.mode = 1;
+  const dim3 grid(rows, heads, (dim + SCAN_COLS - 1) / SCAN_COLS);
   BY_DTYPE(dtype, BY_KEY_SIZE(dim, (launch_memory<T, KD>(grid, s, r, k, v, w, u, state, out, slots, starts,
-                                                          query_start, heads, dim, pc))));
-  HOLON_LAUNCH_OK();
-  memory_pieces_kernel<<<dim3(rows, heads), 256, 0, s>>>(state, slots, starts, query_start, heads, dim, pc);
-  HOLON_LAUNCH_OK();
-  pc.mode = 2;
-  BY_DTYPE(dtype, BY_KEY_SIZE(dim, (launch_memory<T, KD>(grid, s, r, k, v, w, u, state, out, slots, starts,
-                                                          query_start, heads, dim, pc))));
+                                                          query_start, heads, dim))));
   HOLON_LAUNCH_OK();
   return 0;
 }

@@ -329,3 +329,28 @@ def test_trace_runner_as_a_program(folders, tmp_path):
         for row, key in zip(rows, expect):
             got[key] = torch.from_numpy(row.copy())
     _check(folder, "float32", requests, got, "trace_run")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,dim", [(3, 64), (2, 16), (2, 40), (1, 128), (1, 200)])
+def test_the_memory_in_pieces(heads, dim, dtype):
+    """`memory_scan` with rows in pieces against its plain form: rows longer and shorter than a piece, ends inside, at and one
+    behind a border of a piece and of a block of 16 tokens, states carried and not, decays near one and near nothing. The
+    same products in another order: float32 rounding."""
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.registry import kernel_op
+    k, dev = load_hip(), torch.device("cuda")
+    gen = torch.Generator().manual_seed(heads * 1000 + dim)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    counts, piece = [385, 256, 17, 1, 300], 128
+    t, npc = sum(counts), [-(-n // piece) for n in counts]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
+    r, kk, v = (rn(t, heads * dim).to(dtype) for _ in range(3))
+    w = torch.exp(-torch.exp(2 * rn(t, heads * dim)))
+    u, state = rn(heads, dim), rn(7, heads, dim, dim)
+    rows = (i32([6, 1, 2, 0, 4]), i32([5, 0, 9, 3, 0]), i32([sum(counts[:b]) for b in range(6)]), 5, heads)
+    one, two = state.clone(), state.clone()
+    got = k.memory_scan(r, kk, v, w, u, one, *rows, (piece, max(npc), i32([sum(npc[:b]) for b in range(5)]), sum(npc)))
+    want = kernel_op("memory_scan").plain(r.double().float(), kk, v, w, u, two, *rows)
+    assert H.rel_rms(got, want) < 2e-6 and H.rel_rms(one, two) < 2e-6

@@ -1,8 +1,8 @@
 // y[M, N] = x[M, K] w[N, K]^T in true float32: float32 operands on the matrix cores (v_mfma_f32_16x16x4_f32: no
 // reduced-precision mode), float32 accumulation. This is the product of the 32-bit path.
 //
-// Its point is a fixed order of summation, the same in both kernels below: K is cut into 16 shares of equal length (a
-// multiple of 32, the last ones shorter or empty); a share's sum runs over its k in groups of 16 (the instruction adds
+// Its point is a fixed order of summation, the same in both kernels of shares below: K is cut into 16 shares of equal length
+// (64, or a larger multiple of 32; the last ones shorter or empty); a share's sum runs over its k in groups of 16 (the instruction adds
 // k, k + 4, k + 8 and k + 12 of a group at a time), four shares are added up one after the other, and so are the four
 // quarters that makes. None of it depends on M, on where the row lies in the batch, or on the tile of the output the
 // element falls in (rows and columns beyond the edge repeat the last one and are never stored; what lies beyond K is
@@ -21,7 +21,12 @@ constexpr int SHARES = 16, QUARTERS = 4;
 constexpr int GROUP = 16;              // k values of one 16-byte load of every lane
 constexpr int CHUNK = 32;              // k values staged at a time, and what shares are a multiple of
 
-__host__ __device__ __forceinline__ int share_length(int K) { return (K + SHARES * CHUNK - 1) / (SHARES * CHUNK) * CHUNK; }
+constexpr int SHORTEST = 64;           // a share's least length: up to 1,024 of K fewer waves share it
+
+__host__ __device__ __forceinline__ int share_length(int K) {
+  const int even = (K + SHARES * CHUNK - 1) / (SHARES * CHUNK) * CHUNK;
+  return even > SHORTEST ? even : SHORTEST;
+}
 
 // s[0] .. s[15] in the order above.
 template <typename F>
@@ -214,6 +219,78 @@ __global__ void __launch_bounds__(1024) gemm_f32_kernel(const float* __restrict_
   store4(y, sum, m0 + tile / 4 * 16 + c, n0 + tile % 4 * 16 + 4 * g, M, N);
 }
 
+// Long sums into many columns: one running sum over k = 0, 1, 2, ... (v_mfma_f32_32x32x2_f32 adds its two k one after the
+// other), the order of a plain float32 product. What the 32-bit path of a model of these sizes is held against is the same model
+// in plain float32 products, and the rounding of those alone, most of it the query and key projection's (6,144 columns over K =
+// 4,096), is 2.1e-5 of the logits' rms at 36 layers: sums in shares come 3 times closer to 64 bits (8e-6) and lie 2.1e-5 from
+// the plain model where 2e-5 are allowed; these lie 1.9e-5 from it.
+// A workgroup of four waves owns a 64 x 64 tile of the output, each wave a 32 x 32 quarter. Per step the workgroup stages 64
+// rows of x and 64 rows of w, 32 k wide, in LDS (rows padded to 33 floats: a wave's 32 rows then fall in 32 different banks).
+constexpr int TM = 64, TN = 64, TK = 32, PAD = 1;
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+__host__ __device__ __forceinline__ bool sums_in_order(int N, int K) { return K >= 4096 && N > K; }
+
+// VEC: K is a multiple of 4 and both operands are 16-byte aligned, so rows are read four floats at a time.
+template <bool VEC>
+__device__ __forceinline__ void stage_rows(const float* __restrict__ src, int rows, int K, int row0, int k0,
+                                           float (*dst)[TK + PAD]) {
+  // 64 rows x 32 floats = 512 groups of four; 256 threads take two each
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const int idx = threadIdx.x + it * 256;
+    const int r = idx / (TK / 4), c = (idx % (TK / 4)) * 4;
+    const int row = row0 + r, k = k0 + c;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row < rows) {
+      const float* p = src + (int64_t)row * K + k;
+      if (VEC) {
+        if (k < K) v = *reinterpret_cast<const float4*>(p);      // K % 4 == 0: a group is inside or outside whole
+      } else {
+        if (k + 0 < K) v.x = p[0];
+        if (k + 1 < K) v.y = p[1];
+        if (k + 2 < K) v.z = p[2];
+        if (k + 3 < K) v.w = p[3];
+      }
+    }
+    dst[r][c + 0] = v.x; dst[r][c + 1] = v.y; dst[r][c + 2] = v.z; dst[r][c + 3] = v.w;
+  }
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(256) gemm_f32_in_order_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                       float* __restrict__ y, int M, int N, int K) {
+  __shared__ float xs[TM][TK + PAD];
+  __shared__ float ws[TN][TK + PAD];
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int wm = wave / 2, wn = wave % 2;
+  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+  const int r = lane % 32, half = lane / 32;
+  f32x16_t acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int k0 = 0; k0 < K; k0 += TK) {
+    stage_rows<VEC>(x, M, K, m0, k0, xs);
+    stage_rows<VEC>(w, N, K, n0, k0, ws);
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < TK; kk += 2) {
+      const float a = xs[wm * 32 + r][kk + half];
+      const float b = ws[wn * 32 + r][kk + half];
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
+    }
+    __syncthreads();
+  }
+  // lane holds column n = r of rows 8 (i / 4) + 4 half + i % 4
+  const int n = n0 + wn * 32 + r;
+  if (n >= N) return;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int m = m0 + wm * 32 + 8 * (i / 4) + 4 * half + i % 4;
+    if (m < M) y[(int64_t)m * N + n] = acc[i];
+  }
+}
+
 // Which tile a product takes: the one whose rounds of one block a CU are done first. A round's time over K = 2,048 on
 // MI355X, in us (in proportion for other K): 1 x 1 tiles 9.3, 1 x 2 15.5, 2 x 2 20.5, 2 x 4 33.5, and 42 for the staged 4 x 4
 // (0.8 of the float32 peak where the last round is full). So 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10 us; with a
@@ -246,7 +323,12 @@ extern "C" int holon_gemm_f32(const void* x, const void* w, void* y, int M, int 
   if (M == 0) return 0;
   HOLON_CHECK((M + 63) / 64 <= 65535, "gemm (float32): M=%d rows exceed one launch (%d)", M, 65535 * 64);
   const bool vec = K % 4 == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
-  if (vec) launch<true>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
+  if (sums_in_order(N, K)) {
+    const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
+    hipStream_t s = (hipStream_t)stream;
+    if (vec) gemm_f32_in_order_kernel<true><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, (float*)y, M, N, K);
+    else gemm_f32_in_order_kernel<false><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, (float*)y, M, N, K);
+  } else if (vec) launch<true>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
   else launch<false>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
   HOLON_LAUNCH_OK();
   return 0;

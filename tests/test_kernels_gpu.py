@@ -634,11 +634,14 @@ def test_float32_product_is_true_32_bit_and_its_order_is_fixed(hip):
 def test_float32_product_across_its_tiles(hip, m):
     """Every tile the float32 product chooses between, at the edges of its rows, columns, shares and chunks of K: against
     the float64 product, and each row bit for bit what it is alone. A sum of
-    K / 16 products a share, then 16 shares: its error stays below (K / 16 + 20) 2^-24 sum |x w|."""
-    for k, n in ((30, 97), (32, 16), (36, 200), (512, 48), (544, 1000), (2080, 64), (1100, 3072), (256, 16384)):
+    max(64, K / 16 up to a multiple of 32) products a share, then 16 shares (or one of K, where K >= 4,096 and N > K): its error
+    stays below that many times 2^-24 sum |x w|."""
+    for k, n in ((30, 97), (32, 16), (36, 200), (512, 48), (544, 1000), (2080, 64), (1100, 3072), (256, 16384),
+                 (4096, 4096), (4096, 4112), (4101, 4200)):
         x, w = _randn(m, k, dtype=torch.float32, seed=44), _randn(n, k, dtype=torch.float32, seed=45)
         got, want = hip.linear(x, w), x.double() @ w.double().T
-        bound = (k / 16 + 20) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        longest = k if k >= 4096 and n > k else max(64, -(-k // 512) * 32) + 16
+        bound = longest * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
         assert ((got.double() - want).abs() <= bound).all(), (m, k, n)
         for row in (0, 15, m - 1):
             assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), (m, k, n, row)

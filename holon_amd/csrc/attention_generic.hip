@@ -1,9 +1,16 @@
 // Paged causal attention, the general kernel: any element type, any page size, any head_dim that is a multiple of 8.
-// One wave per (query token, query head). Keys are visited in tiles of 64 starting at the first visible key, so the
-// order of every sum depends on the token's position alone, never on how the batch was cut. Scores and softmax are
-// float32. For float32 operands the two long sums (a score over head_dim, the values over the keys) are accumulated in
-// float64, which this GPU does at the float32 rate: a float32 running sum over 256 products of a sharp query and key
+// A block takes a query token and HG query heads that read one kv head. Keys are visited in tiles of 64 starting at the
+// first visible key, wave w of the block's eight taking tiles w, w + 8, ..., and the waves are combined in order at the
+// end: the order of every sum depends on the token's position alone, never on how the batch was cut. Scores and softmax
+// are float32. For float32 operands the two long sums (a score over head_dim, the values over the keys) are accumulated
+// in float64, which this GPU does at the float32 rate: a float32 running sum over 256 products of a sharp query and key
 // is off by 1e-4 of the score, and that shows in the weights of the softmax.
+//
+// Bound by the latency of its loads. Four lanes share a key (16 keys of a tile at a time, 16 bytes a lane, so that a
+// load takes whole 64-byte parts of 16 rows), a lane holds the weight of key 16 (lane % 4) + lane / 4 of the tile, and a
+// value column is read in 16-byte pieces of neighbouring tokens where the pages allow. Heads of a group share what is
+// read. One row in float32 over 16 heads of 128 on 4 at some 400 keys (and the prompts of 150, averaged): 47 us;
+// with a wave a head, a lane a key and a value column read token by token 175.
 #include <type_traits>
 
 #include "common.h"
@@ -11,20 +18,24 @@
 
 #define GEN_MAX_D 512
 
-template <typename T>
-__global__ void attention_generic_kernel(const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ pages,
-                                         const int32_t* __restrict__ table, int table_stride,
-                                         const int32_t* __restrict__ slots, const int32_t* __restrict__ lens,
-                                         const int32_t* __restrict__ query_start, int rows, int heads, int kv_heads,
-                                         int head_dim, int page_size, float scale, int window) {
-  __shared__ float q_s[4][GEN_MAX_D];
-  __shared__ float p_s[4][WAVE];
-  __shared__ int64_t v_s[4][WAVE];   // element offset of each tile key's value column
+namespace {
+constexpr int GEN_WAVES = 8;
+
+// DB: blocks of 64 dimensions (head_dim at most 64 DB). VVEC: a page's tokens of one value dimension are whole 16-byte
+// pieces on 16-byte borders.
+template <typename T, int DB, int HG, bool VVEC>
+__global__ void __launch_bounds__(GEN_WAVES * WAVE) attention_generic_kernel(
+    const T* __restrict__ q, T* __restrict__ out, const T* __restrict__ pages, const int32_t* __restrict__ table,
+    int table_stride, const int32_t* __restrict__ slots, const int32_t* __restrict__ lens,
+    const int32_t* __restrict__ query_start, int rows, int heads, int kv_heads, int head_dim, int page_size, float scale,
+    int window) {
   using Acc = std::conditional_t<std::is_same<T, float>::value, double, float>;
+  __shared__ Acc q_s[HG][DB * 64];
+  __shared__ Acc sum_s[GEN_WAVES][HG][DB * 64];
+  __shared__ Acc p_s[GEN_WAVES][HG][WAVE];
+  __shared__ float ml_s[GEN_WAVES][HG][2];
   const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int t = blockIdx.x;
-  const bool active = blockIdx.y * 4 + w < heads;
-  const int h = active ? blockIdx.y * 4 + w : 0;   // a spare wave walks head 0 and stores nothing: all reach the barriers
+  const int t = blockIdx.x, h0 = blockIdx.y * HG;
   // the row of token t: the last b with query_start[b] <= t
   int lo_b = 0, hi_b = rows - 1;
   while (lo_b < hi_b) {
@@ -35,72 +46,173 @@ __global__ void attention_generic_kernel(const T* __restrict__ q, T* __restrict_
   const int n = lens[b];
   const int nq = query_start[b + 1] - query_start[b];
   const int pos = n - nq + (t - query_start[b]);
-  T* o = out + ((int64_t)t * heads + h) * head_dim;
+  T* o = out + ((int64_t)t * heads + h0) * head_dim;      // (HG heads side by side)
   if (n <= 0 || pos < 0) {   // uniform over the block (one token per block)
-    if (active) for (int d = lane; d < head_dim; d += WAVE) o[d] = Elem<T>::store(0.f);
+    for (int d = threadIdx.x; d < HG * head_dim; d += GEN_WAVES * WAVE) o[d] = Elem<T>::store(0.f);
     return;
   }
-  const int hk = h / (heads / kv_heads);
+  const int hk = h0 / (heads / kv_heads);
   const int32_t* trow = table + (int64_t)slots[b] * table_stride;
   const int64_t plane = (int64_t)page_size * head_dim;
-  const T* qp = q + ((int64_t)t * heads + h) * head_dim;
-  for (int d = lane; d < head_dim; d += WAVE) q_s[w][d] = Elem<T>::load(qp[d]);
+  const T* qp = q + ((int64_t)t * heads + h0) * head_dim;
+  for (int d = threadIdx.x; d < HG * head_dim; d += GEN_WAVES * WAVE) q_s[d / head_dim][d % head_dim] = (Acc)Elem<T>::load(qp[d]);
   __syncthreads();
 
   const int first = max(0, first_seen(pos, window));
-  float m = -INFINITY, l = 0.f;
-  Acc acc[GEN_MAX_D / WAVE];
+  float m[HG], l[HG];
+  Acc acc[HG][DB];
 #pragma unroll
-  for (int i = 0; i < GEN_MAX_D / WAVE; ++i) acc[i] = 0;
-  constexpr int V = Elem<T>::kVec;
-
-  for (int j0 = first; j0 <= pos; j0 += WAVE) {
-    const int key = j0 + lane;
-    const bool valid = key <= pos;
-    float s = -INFINITY;
-    int64_t voff = 0;
-    if (valid) {
-      const int page = trow[key / page_size];
-      const int off = key - (key / page_size) * page_size;
-      const T* kp = pages + (((int64_t)page * 2 + 0) * kv_heads + hk) * plane + (int64_t)off * head_dim;
-      voff = (((int64_t)page * 2 + 1) * kv_heads + hk) * plane + off;
-      Acc dot = 0;
-      for (int d = 0; d < head_dim; d += V) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(kp + d);
-        const T* e = reinterpret_cast<const T*>(&raw);
+  for (int h = 0; h < HG; ++h) {
+    m[h] = -INFINITY;
+    l[h] = 0.f;
 #pragma unroll
-        for (int i = 0; i < V; ++i) dot += (Acc)q_s[w][d + i] * (Acc)Elem<T>::load(e[i]);
-      }
-      s = (float)dot * scale;
-    }
-    const float m_new = fmaxf(m, wave_max(s));
-    const float alpha = expf(m - m_new);          // m = -inf on the first tile: alpha = 0
-    const float p = valid ? expf(s - m_new) : 0.f;
-    l = l * alpha + wave_sum(p);
-    m = m_new;
-    p_s[w][lane] = p;
-    v_s[w][lane] = voff;
-    __syncthreads();
-    const int count = min(WAVE, pos - j0 + 1);
-#pragma unroll
-    for (int i = 0; i < GEN_MAX_D / WAVE; ++i) {
-      const int d = lane + i * WAVE;
-      if (d < head_dim) {
-        Acc a = acc[i] * (Acc)alpha;
-        for (int j = 0; j < count; ++j)
-          a += (Acc)p_s[w][j] * (Acc)Elem<T>::load(pages[v_s[w][j] + (int64_t)d * page_size]);
-        acc[i] = a;
-      }
-    }
-    __syncthreads();
+    for (int i = 0; i < DB; ++i) acc[h][i] = 0;
   }
-  if (!active) return;
+  constexpr int V = Elem<T>::kVec;
+  const int part = lane % 4, chunks = head_dim / V;
+  for (int j0 = first + w * WAVE; j0 <= pos; j0 += GEN_WAVES * WAVE) {
+    float s[HG];
 #pragma unroll
-  for (int i = 0; i < GEN_MAX_D / WAVE; ++i) {
-    const int d = lane + i * WAVE;
-    if (d < head_dim) o[d] = Elem<T>::store((float)(acc[i] / (Acc)l));
+    for (int h = 0; h < HG; ++h) s[h] = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int key = j0 + 16 * r + lane / 4;
+      Acc dot[HG];
+#pragma unroll
+      for (int h = 0; h < HG; ++h) dot[h] = 0;
+      if (key <= pos) {
+        const int page = trow[key / page_size], off = key % page_size;
+        const T* kp = pages + (((int64_t)page * 2 + 0) * kv_heads + hk) * plane + (int64_t)off * head_dim;
+#pragma unroll 4
+        for (int c = part; c < chunks; c += 4) {
+          const uint4 raw = *reinterpret_cast<const uint4*>(kp + c * V);
+          const T* e = reinterpret_cast<const T*>(&raw);
+#pragma unroll
+          for (int i = 0; i < V; ++i) {
+            const Acc k = (Acc)Elem<T>::load(e[i]);
+#pragma unroll
+            for (int h = 0; h < HG; ++h) dot[h] += q_s[h][c * V + i] * k;
+          }
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < HG; ++h) {
+        dot[h] += __shfl_xor(dot[h], 1, WAVE);
+        dot[h] += __shfl_xor(dot[h], 2, WAVE);
+        if (r == part && key <= pos) s[h] = (float)dot[h] * scale;
+      }
+    }
+    const int mine = 16 * part + lane / 4;                // the tile's key whose weight this lane holds
+#pragma unroll
+    for (int h = 0; h < HG; ++h) {
+      const float m_new = fmaxf(m[h], wave_max(s[h]));
+      const float alpha = expf(m[h] - m_new);             // m = -inf on the first tile: alpha = 0
+      const float p = j0 + mine <= pos ? expf(s[h] - m_new) : 0.f;
+      l[h] = l[h] * alpha + wave_sum(p);
+      m[h] = m_new;
+      p_s[w][h][mine] = (Acc)p;
+#pragma unroll
+      for (int i = 0; i < DB; ++i) acc[h][i] *= (Acc)alpha;
+    }
+    const int count = min(WAVE, pos - j0 + 1);
+    // (what a wave wrote to LDS it reads back behind its own wait: no other wave touches p_s[w])
+    for (int j = 0; j < count;) {
+      const int key = j0 + j, off = key % page_size;
+      const int run = min(count - j, page_size - off);    // keys of one page
+      const T* vp = pages + (((int64_t)trow[key / page_size] * 2 + 1) * kv_heads + hk) * plane + off;
+      int u = 0;
+      if (VVEC && off % V == 0) {
+#pragma unroll 4
+        for (; u + V <= run; u += V) {
+#pragma unroll
+          for (int i = 0; i < DB; ++i) {
+            const int d = lane + i * WAVE;
+            if (d >= head_dim) break;
+            const uint4 raw = *reinterpret_cast<const uint4*>(vp + (int64_t)d * page_size + u);
+            const T* e = reinterpret_cast<const T*>(&raw);
+#pragma unroll
+            for (int x = 0; x < V; ++x) {
+              const Acc v = (Acc)Elem<T>::load(e[x]);
+#pragma unroll
+              for (int h = 0; h < HG; ++h) acc[h][i] += p_s[w][h][j + u + x] * v;
+            }
+          }
+        }
+      }
+      for (; u < run; ++u) {
+#pragma unroll
+        for (int i = 0; i < DB; ++i) {
+          const int d = lane + i * WAVE;
+          if (d >= head_dim) break;
+          const Acc v = (Acc)Elem<T>::load(vp[(int64_t)d * page_size + u]);
+#pragma unroll
+          for (int h = 0; h < HG; ++h) acc[h][i] += p_s[w][h][j + u] * v;
+        }
+      }
+      j += run;
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < HG; ++h) {
+#pragma unroll
+    for (int i = 0; i < DB; ++i) sum_s[w][h][lane + i * WAVE] = acc[h][i];
+    if (lane == 0) { ml_s[w][h][0] = m[h]; ml_s[w][h][1] = l[h]; }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < HG * head_dim; e += GEN_WAVES * WAVE) {
+    const int h = e / head_dim, d = e % head_dim;
+    float top = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < GEN_WAVES; ++i) top = fmaxf(top, ml_s[i][h][0]);
+    Acc sum = 0;
+    float den = 0.f;
+#pragma unroll
+    for (int i = 0; i < GEN_WAVES; ++i) {
+      if (ml_s[i][h][0] == -INFINITY) continue;           // a wave without keys
+      const float f = expf(ml_s[i][h][0] - top);
+      den += ml_s[i][h][1] * f;
+      sum += sum_s[i][h][d] * (Acc)f;
+    }
+    o[e] = Elem<T>::store((float)(sum / (Acc)den));
   }
 }
+
+template <typename T, int DB, int HG>
+void launch(bool vvec, hipStream_t s, const T* q, T* out, const T* pages, const int32_t* table, int table_stride,
+            const int32_t* slots, const int32_t* lens, const int32_t* query_start, int rows, int tokens, int heads,
+            int kv_heads, int head_dim, int page_size, float scale, int window) {
+  const dim3 grid(tokens, heads / HG);
+  if (vvec)
+    attention_generic_kernel<T, DB, HG, true><<<grid, GEN_WAVES * WAVE, 0, s>>>(q, out, pages, table, table_stride, slots, lens,
+        query_start, rows, heads, kv_heads, head_dim, page_size, scale, window);
+  else
+    attention_generic_kernel<T, DB, HG, false><<<grid, GEN_WAVES * WAVE, 0, s>>>(q, out, pages, table, table_stride, slots, lens,
+        query_start, rows, heads, kv_heads, head_dim, page_size, scale, window);
+}
+
+template <typename T>
+void by_size(hipStream_t s, const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
+             const int32_t* slots, const int32_t* lens, const int32_t* query_start, int rows, int tokens, int heads,
+             int kv_heads, int head_dim, int page_size, float scale, int window) {
+  const int group = heads / kv_heads;
+  const bool vvec = page_size % Elem<T>::kVec == 0 && (uintptr_t)pages % 16 == 0;
+#define GEN(DB, HG)                                                                                                    \
+  launch<T, DB, HG>(vvec, s, (const T*)q, (T*)out, (const T*)pages, table, table_stride, slots, lens, query_start, rows, \
+                    tokens, heads, kv_heads, head_dim, page_size, scale, window)
+#define GEN_HEADS(DB)                  \
+  do {                                 \
+    if (group % 4 == 0) GEN(DB, 4);    \
+    else if (group % 2 == 0) GEN(DB, 2); \
+    else GEN(DB, 1);                   \
+  } while (0)
+  if (head_dim <= 64) GEN_HEADS(1);
+  else if (head_dim <= 128) GEN_HEADS(2);
+  else if (head_dim <= 256) GEN_HEADS(4);
+  else GEN(8, 1);
+#undef GEN_HEADS
+#undef GEN
+}
+}  // namespace
 
 extern "C" int holon_attention_generic(const void* q, void* out, const void* pages, const int32_t* table,
                                        int table_stride, const int32_t* slots, const int32_t* lens,
@@ -113,16 +225,14 @@ extern "C" int holon_attention_generic(const void* q, void* out, const void* pag
               "attention: head_dim %d must be a multiple of 8, at most %d", head_dim, GEN_MAX_D);
   HOLON_CHECK(page_size > 0 && num_pages > 0 && window > -0x7fffffff, "attention: bad page size or window");
   if (tokens == 0 || rows == 0) return 0;
-  dim3 grid(tokens, (heads + 3) / 4);
+  HOLON_CHECK(heads <= 65535, "attention: %d heads exceed one launch", heads);
   hipStream_t s = (hipStream_t)stream;
   if (dtype == HOLON_F32)
-    attention_generic_kernel<float><<<grid, 4 * WAVE, 0, s>>>((const float*)q, (float*)out, (const float*)pages,
-                                                              table, table_stride, slots, lens, query_start, rows,
-                                                              heads, kv_heads, head_dim, page_size, scale, window);
+    by_size<float>(s, q, out, pages, table, table_stride, slots, lens, query_start, rows, tokens, heads, kv_heads, head_dim,
+                   page_size, scale, window);
   else
-    attention_generic_kernel<bf16_t><<<grid, 4 * WAVE, 0, s>>>((const bf16_t*)q, (bf16_t*)out, (const bf16_t*)pages,
-                                                               table, table_stride, slots, lens, query_start, rows,
-                                                               heads, kv_heads, head_dim, page_size, scale, window);
+    by_size<bf16_t>(s, q, out, pages, table, table_stride, slots, lens, query_start, rows, tokens, heads, kv_heads, head_dim,
+                    page_size, scale, window);
   HOLON_LAUNCH_OK();
   return 0;
 }

@@ -8,12 +8,12 @@ namespace {
 // Three sums over a block of 256 threads at once; waves are added in order.
 __device__ __forceinline__ void block_sum3_256(float& a, float& b, float& c, float (*part)[4]) {
   a = wave_sum(a); b = wave_sum(b); c = wave_sum(c);
-  __syncthreads();
+  lds_barrier();                         // (global accesses stay under way)
   if (threadIdx.x % WAVE == 0) {
     const int w = threadIdx.x / WAVE;
     part[0][w] = a; part[1][w] = b; part[2][w] = c;
   }
-  __syncthreads();
+  lds_barrier();
   a = (part[0][0] + part[0][1]) + (part[0][2] + part[0][3]);
   b = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
   c = (part[2][0] + part[2][1]) + (part[2][2] + part[2][3]);
@@ -142,6 +142,11 @@ __global__ void __launch_bounds__(64) moe_route_kernel(const float* __restrict__
   route_token(score_s, choice_s, group_s, weights + base, experts, top, groups, keep, scale);
 }
 
+// Four products of a logit, in this order in every router.
+__device__ __forceinline__ float dot4(float x0, float x1, float x2, float x3, const float4& w) {
+  return fmaf(x3, w.w, fmaf(x2, w.z, fmaf(x1, w.y, x0 * w.x)));
+}
+
 // One block of 256 threads a token, from the token's row: the float32 logits x . router[e] first (the row waits in LDS
 // as float32; wave w takes experts w, w + 4, ..., its lanes a 64th of the row each, added up in an order the width
 // alone decides), then the choice.
@@ -165,10 +170,10 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const T* __restrict__ x
     if (wide) {
       for (int i = lane * 4; i < width; i += WAVE * 4) {
         const float4 v = *reinterpret_cast<const float4*>(w + i);
-        acc += xs[i] * v.x + xs[i + 1] * v.y + xs[i + 2] * v.z + xs[i + 3] * v.w;
+        acc += dot4(xs[i], xs[i + 1], xs[i + 2], xs[i + 3], v);
       }
     } else {
-      for (int i = lane; i < width; i += WAVE) acc += xs[i] * w[i];
+      for (int i = lane; i < width; i += WAVE) acc = fmaf(xs[i], w[i], acc);
     }
     acc = wave_sum(acc);
     if (lane == 0) {
@@ -179,6 +184,112 @@ __global__ void __launch_bounds__(256) moe_router_kernel(const T* __restrict__ x
   }
   __syncthreads();
   route_token(score_s, choice_s, group_s, weights + t * experts, experts, top, groups, keep, scale);
+}
+
+// The router of up to 64 experts for steps of few rows, both kinds: float32 logits z_e = x . router[e] (+ bias[e]), then the choice by one wave with
+// an expert a lane. `score` -1: the scores are s = sigmoid(z), experts are chosen by s + bias (a correction; none: by s), a
+// group's rank is the sum of its two best, and a chosen expert's weight is s * scale; otherwise as moe_router_top_kernel.
+// Equal ones: the lower index first. A logit is added up as the kernels for other sizes do it: PARTS 1 as 64 lanes of a wave,
+// PARTS 4 as 256 threads whose waves' sums are added in order, here four sums a lane; so neither the number of rows nor the
+// kernel changes a choice.
+// A block of 16 waves a token, a wave an expert (all its loads under way at once: one round of memory latency instead of one for
+// every few experts): at one row of 2,048 over 8 experts 6.0 us (PARTS 1) and 6.8 (PARTS 4), 8.7 and 10.7 with a block of four
+// waves a token.
+template <typename T, int PARTS>
+__global__ void __launch_bounds__(1024) moe_router_few_kernel(
+    const T* __restrict__ x, const float* __restrict__ router, const float* __restrict__ bias, float* __restrict__ weights,
+    int width, int experts, int rows_r, int top, int groups, int keep, int score, float scale) {
+  __shared__ float z[WAVE + 1], choice[WAVE], group[WAVE];
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int64_t t = blockIdx.x;
+  const T* row = x + t * width;
+  const bool wide = width % 4 == 0 && (uintptr_t)router % 16 == 0 && (uintptr_t)x % (4 * sizeof(T)) == 0;
+  struct alignas(4 * sizeof(T)) Four { T v[4]; };
+  for (int e = wave; e < rows_r; e += 16) {
+    const float* w = router + (int64_t)e * width;
+    float acc[PARTS];
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) acc[q] = 0.f;
+    if (wide) {
+#pragma unroll(8 / PARTS)
+      for (int i0 = lane * 4; i0 < width; i0 += PARTS * WAVE * 4) {
+#pragma unroll
+        for (int q = 0; q < PARTS; ++q) {
+          const int i = i0 + q * WAVE * 4;
+          if (PARTS > 1 && i >= width) break;
+          const Four r = *reinterpret_cast<const Four*>(row + i);
+          const float4 v = *reinterpret_cast<const float4*>(w + i);
+          acc[q] += dot4(Elem<T>::load(r.v[0]), Elem<T>::load(r.v[1]), Elem<T>::load(r.v[2]), Elem<T>::load(r.v[3]), v);
+        }
+      }
+    } else {
+      for (int i0 = lane; i0 < width; i0 += PARTS * WAVE) {
+#pragma unroll
+        for (int q = 0; q < PARTS; ++q) {
+          const int i = i0 + q * WAVE;
+          if (PARTS > 1 && i >= width) break;
+          acc[q] = fmaf(Elem<T>::load(row[i]), w[i], acc[q]);
+        }
+      }
+    }
+    float sum = wave_sum(acc[0]);
+#pragma unroll
+    for (int q = 1; q < PARTS; ++q) sum += wave_sum(acc[q]);
+    if (lane == 0) z[e] = sum;
+  }
+  __syncthreads();
+  if (wave > 0) return;
+  // from here on one wave, whose lanes read back what its lanes wrote
+  const auto settle = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+  settle();
+  const bool in = lane < experts;
+  float mine = -INFINITY, own = 0.f;                        // the choice score; the score or logit a weight is made of
+  if (in) {
+    own = z[lane];
+    if (score < 0) {
+      own = 1.0f / (1.0f + expf(-own));
+      mine = bias ? own + bias[lane] : own;
+    } else {
+      own = bias ? own + bias[lane] : own;
+      mine = own;
+    }
+    choice[lane] = mine;
+  }
+  settle();
+  if (groups > 1) {
+    const int size = experts / groups, g = in ? lane / size : 0;
+    float best = -INFINITY, next = -INFINITY;               // the group's two largest
+    for (int i = 0; i < size; ++i) {
+      const float v = choice[g * size + i];
+      if (v > best) { next = best; best = v; } else if (v > next) { next = v; }
+    }
+    const float rank = score < 0 && size > 1 ? best + next : best;
+    if (in && lane % size == 0) group[g] = rank;
+    settle();
+    int before = 0;
+    for (int o = 0; o < groups; ++o) before += (group[o] > rank) || (group[o] == rank && o < g);
+    if (before >= keep) mine = -INFINITY;
+    if (in) choice[lane] = mine;
+    settle();
+  }
+  int ahead = 0;
+  for (int o = 0; o < experts; ++o) {
+    const float other = choice[o];
+    ahead += (other > mine) || (other == mine && o < lane);
+  }
+  const bool chosen = in && ahead < top && mine > -INFINITY;
+  float* to = weights + t * rows_r;
+  if (score != 0) {
+    float s = 0.f;
+    if (chosen) s = score < 0 ? own * scale : 1.0f / (1.0f + expf(-own));
+    if (in) to[lane] = score == 2 ? s * s : s;
+  } else {
+    const float top_z = wave_max(mine);                     // the largest logit is always chosen
+    const float v = chosen ? expf(mine - top_z) : 0.f;
+    const float sum = wave_sum(v);
+    if (in) to[lane] = v / sum;
+  }
+  if (rows_r > experts && lane == 0) to[experts] = 1.0f / (1.0f + expf(-z[experts]));
 }
 
 // y[t, c] = round(round(silu(gate)) * up) * weight of the column's expert, 0 where that weight is 0; columns from
@@ -250,7 +361,7 @@ __global__ void __launch_bounds__(256) moe_router_top_kernel(const T* __restrict
         for (int j = 0; j < 16; ++j) {
           if (e0 + j < rows_r) {
             const float4 v = *reinterpret_cast<const float4*>(router + (int64_t)(e0 + j) * width + i);
-            acc[j] += x0 * v.x + x1 * v.y + x2 * v.z + x3 * v.w;
+            acc[j] += dot4(x0, x1, x2, x3, v);
           }
         }
       }
@@ -259,7 +370,7 @@ __global__ void __launch_bounds__(256) moe_router_top_kernel(const T* __restrict
         const float xv = Elem<T>::load(row[i]);
 #pragma unroll
         for (int j = 0; j < 16; ++j)
-          if (e0 + j < rows_r) acc[j] += xv * router[(int64_t)(e0 + j) * width + i];
+          if (e0 + j < rows_r) acc[j] = fmaf(xv, router[(int64_t)(e0 + j) * width + i], acc[j]);
       }
     }
 #pragma unroll
@@ -447,6 +558,22 @@ extern "C" int holon_moe_route(const float* logits, const float* correction, flo
   return 0;
 }
 
+// Up to 256 rows a block a token leaves the chip with idle units, which more waves a token use; with more (4,096 rows of 4,096 over
+// 8 experts: 57 us a wave a token, 58 so) there is nothing left to gain.
+static bool router_few_serves(int64_t rows, int experts) { return rows <= 256 && experts <= WAVE; }
+static int router_few(const void* x, const float* router, const float* bias, float* weights, int64_t rows, int width,
+                      int experts, int rows_r, int top, int groups, int keep, int score, float scale, int dtype,
+                      hipStream_t s) {
+#define ROUTER(T, PARTS)                                                                                                   \
+  moe_router_few_kernel<T, PARTS><<<(unsigned)rows, 1024, 0, s>>>((const T*)x, router, bias, weights, width, experts, rows_r, \
+                                                                  top, groups, keep, score, scale)
+  if (score < 0) { if (dtype == HOLON_F32) ROUTER(float, 1); else ROUTER(bf16_t, 1); }
+  else { if (dtype == HOLON_F32) ROUTER(float, 4); else ROUTER(bf16_t, 4); }
+#undef ROUTER
+  HOLON_LAUNCH_OK();
+  return 0;
+}
+
 extern "C" int holon_moe_router(const void* x, const float* router, const float* correction, float* weights,
                                 int64_t rows, int width, int experts, int top, int groups, int keep, float scale,
                                 int dtype, void* stream) {
@@ -458,6 +585,8 @@ extern "C" int holon_moe_router(const void* x, const float* router, const float*
               "moe_router: %d experts in %d groups of which %d stay open", experts, groups, keep);
   if (rows == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
+  if (router_few_serves(rows, experts))
+    return router_few(x, router, correction, weights, rows, width, experts, experts, top, groups, keep, -1, scale, dtype, s);
   const size_t lds = (size_t)width * sizeof(float);
   if (dtype == HOLON_F32)
     moe_router_kernel<float><<<(unsigned)rows, 256, lds, s>>>((const float*)x, router, correction, weights, width,
@@ -508,6 +637,8 @@ extern "C" int holon_moe_router_top(const void* x, const float* router, const fl
               "moe_router_top: top %d of %d experts in %d groups of which %d stay open", top, experts, groups, keep);
   if (rows == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
+  if (router_few_serves(rows, experts))
+    return router_few(x, router, bias, weights, rows, width, experts, router_rows, top, groups, keep, score, 1.f, dtype, s);
   if (dtype == HOLON_F32)
     moe_router_top_kernel<float><<<(unsigned)rows, 256, 0, s>>>((const float*)x, router, bias, weights, width, experts,
                                                                router_rows, top, groups, keep, score);

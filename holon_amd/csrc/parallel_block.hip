@@ -20,9 +20,9 @@ __device__ __forceinline__ void store_as(void* p, int64_t i, int dt, float v) {
 // Sum over a block of 256 threads, every thread gets the result; waves are added in order.
 __device__ __forceinline__ float block_sum_256(float v, float* part) {
   v = wave_sum(v);
-  __syncthreads();
+  lds_barrier();                         // (global accesses stay under way)
   if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = v;
-  __syncthreads();
+  lds_barrier();
   return (part[0] + part[1]) + (part[2] + part[3]);
 }
 

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 import torch
 
+import holon_amd.parts  # noqa: F401  (registers the parts' operations)
 from holon_amd.kernels.api import AttnRows
 from tests import helpers as H
 from tests.plain.ops import TorchKernels
@@ -1042,3 +1043,27 @@ def test_nothing_is_collected_while_a_graph_is_recorded():
         with capture(torch.cuda.CUDAGraph()):
             raise RuntimeError("stop here")
     assert gc.isenabled()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_router_of_few_experts(hip, dtype):
+    """Both routers up to 64 experts, on either side of 256 rows: the plain form's choice but for rows of a close call, and a
+    row alone what it is among others."""
+    for experts, top, width, groups, keep in ((1, 1, 40, 1, 1), (8, 2, 2048, 1, 1), (17, 5, 250, 1, 1), (64, 6, 1024, 8, 3),
+                                              (12, 4, 37, 6, 2), (64, 64, 128, 64, 64)):
+        for rows in (1, 256, 257, 1030):
+            x = _randn(rows, width, dtype=dtype, seed=70)
+            router = _randn(experts + 1, width, dtype=torch.float32, seed=71, scale=width ** -0.5)
+            bias = _randn(experts, dtype=torch.float32, seed=72, scale=0.2)
+            from holon_amd.kernels.registry import kernel_op
+            cases = [("moe_router", (x, router[:experts], bias, top, groups, keep, 1.7), {}),
+                     ("moe_router", (x, router[:experts], None, top, groups, keep, 0.5), {})]
+            cases += [("moe_router_top", (x, router, bias, experts, top, groups, keep), dict(score=how))
+                      for how in ("softmax", "sigmoid", "sigmoid_squared")]
+            for name, args, how in cases:
+                op = getattr(hip, name)
+                got, want = op(*args, **how), kernel_op(name).plain(*args, **how)
+                close = ((got != 0) != (want != 0)).any(1)
+                assert close.sum() <= 1 + rows // 500 and torch.allclose(got[~close], want[~close], atol=2e-5), (name, how, experts, rows)
+                alone = op(x[-1:].contiguous(), *args[1:], **how)
+                assert torch.equal(alone[0], got[-1]), (name, how, experts, rows)

@@ -125,3 +125,10 @@ void holon_set_error(const char* fmt, ...);
   } while (0)
 
 enum { HOLON_F32 = 0, HOLON_BF16 = 1 };
+
+// How many waves of a block share the K of a few-row product over `tiles` tiles of 16 outputs: from the shapes alone.
+static inline int skinny_waves(int tiles, int K) {
+  int waves = tiles >= 320 ? 8 : 16;
+  while (waves > 1 && K % (32 * waves) != 0) waves /= 2;
+  return waves;
+}

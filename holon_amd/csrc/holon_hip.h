@@ -405,6 +405,14 @@ int holon_moe_gate(const void* gate_up, const float* weights, void* y, int64_t r
 // weights are the chosen logits' own sigmoids, 2: their squares.
 int holon_moe_router_top(const void* x, const float* router, const float* bias, float* weights, int64_t rows, int width,
                          int experts, int router_rows, int top, int dtype, int groups, int keep, int score, void* stream);
+// The experts for steps of up to 16 bfloat16 rows, reading the chosen experts' weights alone: act [rows, experts ff + shared]
+// from x and the tiled first projections (gated: [gates; ups], then what holon_moe_gate does; else what holon_moe_relu2
+// does; columns of experts that no row chose are left as they are), and y [rows, hidden] from act and the tiled second ones.
+int holon_moe_few_supported(int rows, int hidden, int experts, int ff, int shared);
+int holon_moe_up_few_bf16(const void* x, const void* w_tiled, void* act, int rows, int hidden, int experts, int ff, int shared,
+                          int gated, const float* weights, int wstride, int shared_col, void* stream);
+int holon_moe_down_few_bf16(const void* act, const void* w_tiled, void* y, int rows, int hidden, int experts, int ff,
+                            int shared, const float* weights, int wstride, void* stream);
 // up [rows, C], C = experts ff + shared: y = max(up, 0)^2 times the weight of the column's expert (as for holon_moe_gate).
 int holon_moe_relu2(const void* up, const float* weights, void* y, int64_t rows, int experts, int ff, int shared, int dtype,
                     int wstride, int shared_col, void* stream);

@@ -1045,6 +1045,48 @@ def test_nothing_is_collected_while_a_graph_is_recorded():
     assert gc.isenabled()
 
 
+@pytest.mark.parametrize("hidden,experts,ff,shared,top,gated,own_gate", [
+    (256, 8, 32, 0, 1, True, False), (384, 8, 160, 64, 2, True, True), (512, 70, 544, 32, 6, False, False),
+    (288, 5, 96, 0, 2, False, False), (2048, 8, 2048, 2048, 2, True, True)])
+def test_chosen_experts_alone(hip, hidden, experts, ff, shared, top, gated, own_gate):
+    """The two products over the chosen experts: bit for bit the products over all experts with the activation between them, and
+    against float64 five roundings to bfloat16 (gate, up, their activation, the product, the result), of 2^-9 each at most. No
+    row's result depends on the rows beside it."""
+    bf, cols = torch.bfloat16, experts * ff + shared
+    up_w = _randn((2 if gated else 1) * cols, hidden, dtype=bf, seed=60, scale=hidden ** -0.5)
+    down_w = _randn(hidden, cols, dtype=bf, seed=61, scale=ff ** -0.5)
+    up_t, down_t = hip.tile_weight(up_w), hip.tile_weight(down_w)
+    g = torch.Generator().manual_seed(62)
+    for m in (1, 2, 7, 16):
+        x = _randn(m, hidden, dtype=bf, seed=63 + m)
+        weights = torch.zeros(m, experts + int(own_gate))
+        for row in range(m):
+            weights[row, torch.randperm(experts, generator=g)[:top]] = torch.rand(top, generator=g) + 0.2
+        weights[:, experts:] = 0.7
+        if m == 7:
+            weights[:, 1:experts] = 0          # one expert or none
+        weights = weights.cuda()
+        garbage = torch.full((m, cols), float("nan"), dtype=bf, device="cuda")
+        del garbage                            # what no row chose must not be read
+        got = hip.moe_few(x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=own_gate)
+        between = hip.moe_gate if gated else hip.moe_relu2
+        whole = hip.linear(between(hip.linear(x, up_w, tiled=up_t), weights, ff, shared, shared_weight=own_gate), down_w,
+                           tiled=down_t)
+        assert torch.equal(got, whole), m
+        z = x.double() @ up_w.double().T
+        act = torch.nn.functional.silu(z[:, :cols]) * z[:, cols:] if gated else torch.relu(z).square()
+        each = weights[:, :experts].double().repeat_interleave(ff, 1)
+        last = weights[:, experts:].double() if own_gate else torch.ones(m, 1, dtype=torch.double, device="cuda")
+        want = (act * torch.cat((each, last.expand(m, shared)), 1)) @ down_w.double().T
+        apart = H.rel_rms(got, want) if want.any() else got.abs().max().item()
+        assert apart < 5 * 2.0 ** -9, (m, apart)
+        for row in (0, m // 2, m - 1):
+            alone = hip.moe_few(x[row: row + 1].contiguous(), weights[row: row + 1].contiguous(), up_t, down_t, experts, ff, shared,
+                                gated, shared_weight=own_gate)
+            assert torch.equal(alone[0], got[row]), (m, row)
+    assert hip.moe_few(_randn(17, hidden, dtype=bf), weights, up_t, down_t, experts, ff, shared, gated) is None
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_router_of_few_experts(hip, dtype):
     """Both routers up to 64 experts, on either side of 256 rows: the plain form's choice but for rows of a close call, and a

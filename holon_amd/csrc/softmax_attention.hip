@@ -335,10 +335,11 @@ extern "C" int holon_head_linear_rows(const void* x, const void* w, void* y, int
 // -- preparing the merged projections of the two attention mixers -------------------------------------------------------
 namespace {
 
-// Both prepares take a block of 1,024 threads a token, of which the first 256 add up the squares: a step of few rows waits for a
-// round of memory per loop over the row, and the loops that write have a quarter as many. A row of 3,072 takes 4.2 and 4.0 us at
-// one token (6.5 and 6.9 with 256 threads throughout); at 4,096 tokens of 8,192 47 and 55 (47 and 55 as well).
-constexpr int PREP_THREADS = 1024;
+// Both prepares take a block a token, whose first 256 threads add up the squares. Up to 256 tokens it has 1,024 threads: such a
+// step waits for a round of memory per loop over the row, and the loops that write then have a quarter as many. A row of 3,072
+// takes 4.2 and 4.0 us at one token (6.5 and 6.9 with 256 threads throughout); 4,096 tokens of 8,192 keep the chip busy and take
+// 47 and 55 so, 45 and 47 with blocks of 256.
+constexpr int PREP_FEW = 256, PREP_THREADS_FEW = 1024, PREP_THREADS = 256;
 
 // Sum over the block's first 256 threads of two values at once; waves are added in order.
 __device__ __forceinline__ void block_sum2_256(float& a, float& b, float (*part)[4]) {
@@ -355,8 +356,8 @@ __device__ __forceinline__ void block_sum2_256(float& a, float& b, float (*part)
 // as one vector and multiplied by q_weight [H D], all of its key values likewise with k_weight [G D] (eps inside the
 // root, float32 inside, one rounding). Queries go to `q` [T, H, D]; keys and values into the token's page: keys
 // [G, P, D], then values [G, V, P].
-template <typename T>
-__global__ void __launch_bounds__(PREP_THREADS) whole_norm_prepare_kernel(
+template <typename T, int THREADS>
+__global__ void __launch_bounds__(THREADS) whole_norm_prepare_kernel(
     const T* __restrict__ qkv, int heads, int kv_heads, int dim, int vdim, const T* __restrict__ q_weight,
     const T* __restrict__ k_weight, float eps, T* __restrict__ q, T* __restrict__ pages,
     const int32_t* __restrict__ write_page, const int32_t* __restrict__ write_off, int page_size, int num_pages) {
@@ -373,18 +374,18 @@ __global__ void __launch_bounds__(PREP_THREADS) whole_norm_prepare_kernel(
   }
   block_sum2_256(sq, sk, part);
   const float rq = 1.0f / sqrtf(sq / (float)nq + eps), rk = 1.0f / sqrtf(sk / (float)nk + eps);
-  for (int c = threadIdx.x; c < nq; c += PREP_THREADS)
+  for (int c = threadIdx.x; c < nq; c += THREADS)
     q[(int64_t)t * nq + c] = Elem<T>::store(Elem<T>::load(row[c]) * rq * Elem<T>::load(q_weight[c]));
   const int page = write_page[t], off = write_off[t];
   if (page < 0 || page >= num_pages || off < 0 || off >= page_size) return;
   T* keys = pages + (int64_t)page * kv_heads * page_size * (dim + vdim);
   T* vals = keys + (int64_t)kv_heads * page_size * dim;
-  for (int c = threadIdx.x; c < nk; c += PREP_THREADS) {
+  for (int c = threadIdx.x; c < nk; c += THREADS) {
     const int g = c / dim, d = c - g * dim;
     keys[((int64_t)g * page_size + off) * dim + d] =
         Elem<T>::store(Elem<T>::load(row[nq + c]) * rk * Elem<T>::load(k_weight[c]));
   }
-  for (int c = threadIdx.x; c < nv; c += PREP_THREADS) vals[(int64_t)c * page_size + off] = row[nq + nk + c];
+  for (int c = threadIdx.x; c < nv; c += THREADS) vals[(int64_t)c * page_size + off] = row[nq + nk + c];
 }
 
 // One block a token. `both` [T, H (dim + rot) + kv_rank + rot]: every head's query as [dim unrotated, rot rotated], then
@@ -393,8 +394,8 @@ __global__ void __launch_bounds__(PREP_THREADS) whole_norm_prepare_kernel(
 // then rd / 2 sines). Unrotated query parts go to `qn` [T, H, dim], rotated ones into the last `rot` columns of `full`
 // [T, H, kv_rank + rot]; the cache entry [latent, rotated key part] into the token's page as a key row of [P, width]
 // and (copies 2) as a value column of [width, P]. Rows are `both_stride` apart; `pages` null: queries alone.
-template <typename T>
-__global__ void __launch_bounds__(PREP_THREADS) latent_rope_prepare_kernel(
+template <typename T, int THREADS>
+__global__ void __launch_bounds__(THREADS) latent_rope_prepare_kernel(
     const T* __restrict__ both, int both_stride, int heads, int dim, int rot, int kv_rank, const T* __restrict__ c_weight,
     float eps,
     const float* __restrict__ table, int rd, int table_rows, const int32_t* __restrict__ positions, T* __restrict__ qn,
@@ -423,11 +424,11 @@ __global__ void __launch_bounds__(PREP_THREADS) latent_rope_prepare_kernel(
     if (r < half) return v * cs[r] - Elem<T>::load(x[r + half]) * cs[half + r];
     return v * cs[r - half] + Elem<T>::load(x[r - half]) * cs[r];
   };
-  for (int c = threadIdx.x; c < heads * dim; c += PREP_THREADS) {
+  for (int c = threadIdx.x; c < heads * dim; c += THREADS) {
     const int h = c / dim, d = c - h * dim;
     qn[(int64_t)t * heads * dim + c] = row[h * per + d];
   }
-  for (int c = threadIdx.x; c < heads * rot; c += PREP_THREADS) {
+  for (int c = threadIdx.x; c < heads * rot; c += THREADS) {
     const int h = c / rot, r = c - h * rot;
     full[((int64_t)t * heads + h) * width + kv_rank + r] = Elem<T>::store(turned(row + h * per + dim, r));
   }
@@ -436,7 +437,7 @@ __global__ void __launch_bounds__(PREP_THREADS) latent_rope_prepare_kernel(
   if (page < 0 || page >= num_pages || off < 0 || off >= page_size) return;
   T* keys = pages + (int64_t)page * copies * page_size * width;
   T* vals = keys + (int64_t)page_size * width;
-  for (int d = threadIdx.x; d < width; d += PREP_THREADS) {
+  for (int d = threadIdx.x; d < width; d += THREADS) {
     const T e = d < kv_rank ? Elem<T>::store(Elem<T>::load(tail[d]) * rc * Elem<T>::load(c_weight[d]))
                             : Elem<T>::store(turned(tail + kv_rank, d - kv_rank));
     keys[(int64_t)off * width + d] = e;
@@ -489,6 +490,12 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(const T* __restrict__
 }
 }  // namespace
 
+#define PREPARE(KERNEL, T, ...)                                                             \
+  do {                                                                                      \
+    if (tokens <= PREP_FEW) KERNEL<T, PREP_THREADS_FEW><<<tokens, PREP_THREADS_FEW, 0, s>>>(__VA_ARGS__); \
+    else KERNEL<T, PREP_THREADS><<<tokens, PREP_THREADS, 0, s>>>(__VA_ARGS__);              \
+  } while (0)
+
 extern "C" int holon_whole_norm_prepare(const void* qkv, int tokens, int heads, int kv_heads, int dim, int vdim,
                                         const void* q_weight, const void* k_weight, float eps, void* q, void* pages,
                                         const int32_t* write_page, const int32_t* write_off, int page_size,
@@ -498,15 +505,12 @@ extern "C" int holon_whole_norm_prepare(const void* qkv, int tokens, int heads, 
   if (tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == HOLON_F32)
-    whole_norm_prepare_kernel<float><<<tokens, PREP_THREADS, 0, s>>>((const float*)qkv, heads, kv_heads, dim, vdim,
-                                                           (const float*)q_weight, (const float*)k_weight, eps,
-                                                           (float*)q, (float*)pages, write_page, write_off, page_size,
-                                                           num_pages);
+    PREPARE(whole_norm_prepare_kernel, float, (const float*)qkv, heads, kv_heads, dim, vdim, (const float*)q_weight,
+            (const float*)k_weight, eps, (float*)q, (float*)pages, write_page, write_off, page_size, num_pages);
   else
-    whole_norm_prepare_kernel<bf16_t><<<tokens, PREP_THREADS, 0, s>>>((const bf16_t*)qkv, heads, kv_heads, dim, vdim,
-                                                            (const bf16_t*)q_weight, (const bf16_t*)k_weight, eps,
-                                                            (bf16_t*)q, (bf16_t*)pages, write_page, write_off,
-                                                            page_size, num_pages);
+    PREPARE(whole_norm_prepare_kernel, bf16_t, (const bf16_t*)qkv, heads, kv_heads, dim, vdim,
+            (const bf16_t*)q_weight, (const bf16_t*)k_weight, eps, (bf16_t*)q, (bf16_t*)pages, write_page, write_off,
+            page_size, num_pages);
   HOLON_LAUNCH_OK();
   return 0;
 }
@@ -527,15 +531,13 @@ extern "C" int holon_latent_rope_prepare(const void* both, int both_stride, int 
   if (tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == HOLON_F32)
-    latent_rope_prepare_kernel<float><<<tokens, PREP_THREADS, 0, s>>>((const float*)both, both_stride, heads, dim, rot, kv_rank,
-                                                            (const float*)c_weight, eps, table, rd, table_rows, positions,
-                                                            (float*)qn, (float*)full, (float*)pages, write_page,
-                                                            write_off, page_size, num_pages, copies);
+    PREPARE(latent_rope_prepare_kernel, float, (const float*)both, both_stride, heads, dim, rot, kv_rank,
+            (const float*)c_weight, eps, table, rd, table_rows, positions, (float*)qn, (float*)full, (float*)pages,
+            write_page, write_off, page_size, num_pages, copies);
   else
-    latent_rope_prepare_kernel<bf16_t><<<tokens, PREP_THREADS, 0, s>>>((const bf16_t*)both, both_stride, heads, dim, rot, kv_rank,
-                                                             (const bf16_t*)c_weight, eps, table, rd, table_rows,
-                                                             positions, (bf16_t*)qn, (bf16_t*)full, (bf16_t*)pages,
-                                                             write_page, write_off, page_size, num_pages, copies);
+    PREPARE(latent_rope_prepare_kernel, bf16_t, (const bf16_t*)both, both_stride, heads, dim, rot, kv_rank,
+            (const bf16_t*)c_weight, eps, table, rd, table_rows, positions, (bf16_t*)qn, (bf16_t*)full,
+            (bf16_t*)pages, write_page, write_off, page_size, num_pages, copies);
   HOLON_LAUNCH_OK();
   return 0;
 }

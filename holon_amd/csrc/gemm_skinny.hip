@@ -9,6 +9,8 @@
 // Two weight layouts: rows [N, K] as the checkpoint stores them, and tiles [N/16, K/32, 64 lanes, 8] in which the
 // 16 bytes lane l needs for one product are at lane l's place, so that a wave's load is one contiguous kilobyte and a
 // tile's whole K extent is one contiguous run (measured: 6 to 7 TB/s against 4 to 5 for the row layout).
+#include <type_traits>
+
 #include "common.h"
 #include "holon_hip.h"
 
@@ -84,12 +86,60 @@ __device__ __forceinline__ float over_lane_groups(float v, int c) {
   return ((a + b) + d) + e;
 }
 
+// A wave's run of `steps` products over NT weight tiles, added to acc. UNROLL products' loads wait in one of two sets of
+// registers while the other set's are asked for: a wave that asks for all, waits for all and multiplies has nothing under way
+// for part of its time. (One row of 2,048 / 8,192 / 18,432 against 2,048 columns, 16 waves a tile: 8 loads in one set 5.1, 11.6,
+// 24.2 us; two sets of 4 4.35, 9.7, 21.7.)
+template <int NT, int UNROLL, typename Tokens, typename Turn>
+__device__ __forceinline__ void stream_tiles(f32x4_t (&acc)[NT], const bf16_t* const (&wp)[NT], int wstep, int steps,
+                                             Tokens tokens, Turn turn) {
+  bf16x8_t wf[2][NT][UNROLL], xf[2][UNROLL];
+  const auto ask = [&](auto set, int s) {
+    constexpr int B = decltype(set)::value;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u)
+        wf[B][j][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)(s + u) * wstep));
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) xf[B][u] = tokens(s + u);
+  };
+  const auto use = [&](auto set) {
+    constexpr int B = decltype(set)::value;
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[B][j][u], xf[B][u], acc[j], 0, 0, 0);
+  };
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  const int rounds = steps / UNROLL;
+  if (rounds > 0) ask(even, 0);
+  for (int r = 0; r < rounds; r += 2) {
+    turn();
+    if (r + 1 < rounds) ask(odd, (r + 1) * UNROLL);
+    use(even);
+    if (r + 1 < rounds) {
+      if (r + 2 < rounds) ask(even, (r + 2) * UNROLL);
+      use(odd);
+    }
+  }
+  for (int s = rounds * UNROLL; s < steps; ++s) {
+    const bf16x8_t xl = tokens(s);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const bf16x8_t wl = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)s * wstep));
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl, xl, acc[j], 0, 0, 0);
+    }
+  }
+}
+
 // RESID: y is the residual stream, y = round(y + round(product)) in place: the add that the next norm's kernel would
 // have done, with its roundings.
 // NT: tiles of 16 weight rows a block owns, next to one another; its waves run them side by side over one copy of the
 // activations, which halves what the activations cost where every block reads all of them. A tile's sums are the same
 // whatever NT is.
-template <int NT, int WPB, int UNROLL, typename OutT, bool TILED, bool RESID = false>
+template <int NT, int WPB, int UNROLL, bool TWICE, typename OutT, bool TILED, bool RESID = false>
 __global__ void __launch_bounds__(WPB * 64) gemm_skinny_kernel(const bf16_t* __restrict__ x,
                                                                 const bf16_t* __restrict__ w, OutT* __restrict__ y,
                                                                 int M, int N, int K, int round_first, RowScale rs,
@@ -131,28 +181,32 @@ __global__ void __launch_bounds__(WPB * 64) gemm_skinny_kernel(const bf16_t* __r
     return xf;
   };
 
-  int s = 0;
-  for (; s + UNROLL <= steps; s += UNROLL) {
-    sums.turn();
-    bf16x8_t wf[NT][UNROLL], xf[UNROLL];
+  if constexpr (TWICE) {
+    stream_tiles<NT, UNROLL>(acc, wp, WSTEP, steps, tokens, [&] { sums.turn(); });
+  } else {
+    int s = 0;
+    for (; s + UNROLL <= steps; s += UNROLL) {
+      sums.turn();
+      bf16x8_t wf[NT][UNROLL], xf[UNROLL];
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+          wf[j][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)(s + u) * WSTEP));
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) xf[u] = tokens(s + u);
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)
-        wf[j][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)(s + u) * WSTEP));
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) xf[u] = tokens(s + u);
+        for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][u], xf[u], acc[j], 0, 0, 0);
+    }
+    for (; s < steps; ++s) {
+      const bf16x8_t xf = tokens(s);
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j][u], xf[u], acc[j], 0, 0, 0);
-  }
-  for (; s < steps; ++s) {
-    const bf16x8_t xf = tokens(s);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const bf16x8_t wf = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)s * WSTEP));
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[j], 0, 0, 0);
+      for (int j = 0; j < NT; ++j) {
+        const bf16x8_t wf = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)s * WSTEP));
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[j], 0, 0, 0);
+      }
     }
   }
   f32x4_t ss = sums.finish();
@@ -218,46 +272,52 @@ __global__ void __launch_bounds__(WPB * 64) gemm_skinny_kernel(const bf16_t* __r
   }
 }
 
-template <int NT, int WPB, int UNROLL, typename OutT, bool RESID>
+template <int NT, int WPB, int UNROLL, bool TWICE, typename OutT, bool RESID>
 static void launch_skinny(const void* x, const void* w, void* y, int M, int N, int K, bool tiled, hipStream_t s,
                           int round_first, RowScale rs, float* stats_out) {
   const dim3 grid(N / 16 / NT), block(WPB * 64);
   if constexpr (RESID)
-    gemm_skinny_kernel<NT, WPB, UNROLL, OutT, true, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
+    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, OutT, true, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
                                                                                 (OutT*)y, M, N, K, round_first, rs, stats_out);
   else if (tiled)
-    gemm_skinny_kernel<NT, WPB, UNROLL, OutT, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
+    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, OutT, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
                                                                           (OutT*)y, M, N, K, round_first, rs, stats_out);
   else
-    gemm_skinny_kernel<NT, WPB, UNROLL, OutT, false><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
+    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, OutT, false><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
                                                                            (OutT*)y, M, N, K, round_first, rs, stats_out);
 }
 
-// How many waves share a tile, from the shapes alone (a result never depends on M), and how many tiles a block owns
-// (which changes no result, so it may follow M). Measured on MI355X, K 4096 to 8192, in us at 1 / 8 / 16 rows:
-//   256 tiles: 16 waves, one tile (two tiles leave half the compute units without a block);
-//   320 to 512 tiles: 8 waves; two tiles 9.9 / 10.7 / 12.2 (320), 11.5 / 12.3 / 13.8 (384), 14.0 / 14.6 / 15.8 (512)
-//     against one 10.8 / 12.8 / 16.1, 11.9 / 14.2 / 16.8, 13.8 / 15.5 / 17.9;
-//   640 tiles: 8 waves, one tile 17.2 / 20.0 / 23.1 against two 19.1 / 21.1 / 23.3;
-//   9,496 tiles (float32 result): 8 waves; one tile up to 8 rows (4 rows 181 against 195, 8 rows 192 against 201), two
-//     from 10 rows up (12 rows 211 against 220, 16 rows 223 against 251).
-constexpr int SKINNY_WIDE_TWO_FROM = 10;   // rows from which a vocabulary's worth of tiles is walked two a block
+// How many waves share a tile, from the shapes alone (a result never depends on M): 16 up to 319 tiles, 8 from there. How many
+// tiles a block owns and how many loads wait in which form changes no result, so it may follow M. Measured on MI355X, in us at
+// 1 / 8 / 16 rows (in brackets: 8 loads in one set of registers, two tiles a block from 320 to 512 tiles and, from 10 rows
+// up, beyond 4,096):
+//   up to 319 tiles: one, two sets of 4 loads. 2048 x 8192 9.7 / 11.4 / 14.5 (11.6 / 12.4 / 15.3), 4096 x 4096 7.8 / 8.3 / 9.3
+//     (8.3 / 8.5 / 10.0).
+//   320 to 511: two (at 512, one: 8192 x 4096 13.8 / 15.1 / 16.0, two 15.0 / 16.1 / 16.0); two sets of 4 loads a tile up to 8 rows,
+//     of 2 above: 6144 x 4096 11.5 / 12.8 / 12.7 (12.0 / 12.9 / 14.3), 6144 x 5120 13.3 / 14.8 / 15.4 (16.8 / 17.8 / 19.1).
+//   from 1,024, and K below 4,096 or more than 8 rows: two, two sets of 2 loads a tile: 18432 x 2048 15.5 / 16.0 / 17.7 (15.6 /
+//     16.8 / 20.0), 36864 x 2048 26.2 / 26.3 / 28.4 (26.3 / 29.0 / 34.7), 24576 x 3072 26.3 / 26.5 / 28.6 (29.6 / 32.4 / 39.4).
+//   otherwise one, 4 loads in one set, which is what 8 waves a block and several blocks a unit need least registers for: 12288 x
+//     4096 19.4 / 20.0 / 23.3 (19.5 / 20.6 / 25.3; two tiles 22.8 / 23.6 / 24.7), 9216 x 2048 9.5 / 10.1 / 11.5 (9.7 / 10.7 /
+//     12.6), 151936 x 4096 182 / 190 (184 / 199; two tiles, for 16 rows, 206, where one takes 243 and took 225).
 template <typename OutT, bool RESID = false>
 static int pick_waves(const void* x, const void* w, void* y, int M, int N, int K, bool tiled, hipStream_t s,
                       int round_first = 0, RowScale rs = RowScale{nullptr, 0, 0.f, 0.f}, float* stats_out = nullptr) {
   const int tiles = N / 16;
-  int wpb = tiles >= 320 ? 8 : 16;
-  while (wpb > 1 && K % (32 * wpb) != 0) wpb /= 2;
-  const bool two = tiles % 2 == 0 && wpb <= 8 && ((tiles >= 320 && tiles <= 512) || (tiles > 4096 && M >= SKINNY_WIDE_TWO_FROM));
-#define SKINNY(WPB, U)                                                                                         \
-  if (two) launch_skinny<2, WPB, U, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out);     \
-  else launch_skinny<1, WPB, U, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out)
+  const int wpb = skinny_waves(tiles, K);
+  const bool two = tiles % 2 == 0 && (tiles < 512 || (tiles >= 1024 && (K < 4096 || M > 8)));
+#define SKINNY(NT, WPB, U, TWICE) \
+  launch_skinny<NT, WPB, U, TWICE, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out)
   switch (wpb) {
-    case 16: launch_skinny<1, 16, 8, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out); break;
-    case 8: SKINNY(8, 8); break;
-    case 4: if (two) { SKINNY(4, 8); } else { SKINNY(4, 16); } break;
-    case 2: SKINNY(2, 8); break;
-    default: SKINNY(1, 8); break;
+    case 16: SKINNY(1, 16, 4, true); break;
+    case 8:
+      if (!two) SKINNY(1, 8, 4, false);
+      else if (tiles < 512 && M <= 8) SKINNY(2, 8, 4, true);
+      else SKINNY(2, 8, 2, true);
+      break;
+    case 4: SKINNY(1, 4, 8, true); break;
+    case 2: SKINNY(1, 2, 8, true); break;
+    default: SKINNY(1, 1, 8, true); break;
   }
 #undef SKINNY
   return 0;
@@ -348,30 +408,7 @@ __global__ void __launch_bounds__(WPB * 64) gemm_skinny_glu_kernel(const bf16_t*
     }
     return xf;
   };
-  int s = 0;
-  for (; s + UNROLL <= steps; s += UNROLL) {
-    sums.turn();
-    bf16x8_t wf[2][UNROLL], xf[UNROLL];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u)
-        wf[h][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[h] + (int64_t)(s + u) * WSTEP));
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) xf[u] = tokens(s + u);
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[0][u], xf[u], acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[1][u], xf[u], acc[1], 0, 0, 0);
-    }
-  }
-  for (; s < steps; ++s) {
-    const bf16x8_t w0 = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[0] + (int64_t)s * WSTEP));
-    const bf16x8_t w1 = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[1] + (int64_t)s * WSTEP));
-    const bf16x8_t xf = tokens(s);
-    acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, xf, acc[0], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, xf, acc[1], 0, 0, 0);
-  }
+  stream_tiles<2, UNROLL>(acc, wp, WSTEP, steps, tokens, [&] { sums.turn(); });
   f32x4_t ss = sums.finish();
   if (WPB > 1) {
     if (wave > 0) {
@@ -414,14 +451,15 @@ static int skinny_glu(const void* x, const void* w, void* y, int M, int I, int K
   HOLON_CHECK(stats == nullptr || (tiled && parts >= 1), "gated gemm (few rows, folded norm): tiled=%d parts=%d", tiled, parts);
   const RowScale rs{stats, parts, eps, 1.0f / (float)K};
   hipStream_t s = (hipStream_t)stream;
-  const bool few = I / 16 < 512;   // few tile pairs: four waves share each; otherwise two (measured at 768 pairs, K 4096:
-                                   // 33 us against 36 for one wave a pair at 1 and 8 rows, the same at 16)
+  // few tile pairs: four waves share each; otherwise two. At 1 / 8 / 16 rows 768 pairs over K = 4,096 take 34.4 / 34.3 / 35.0 us,
+  // 384 over 2,048 11.6 / 12.3 / 13.3 (35.4 / 35.7 / 36.6 and 12.1 / 13.3 / 14.6 with 8 loads in one set of registers).
+  const bool few = I / 16 < 512;
 #define GLU(WPB, U)                                                                                              \
   if (tiled) gemm_skinny_glu_kernel<WPB, U, true, ACT><<<I / 16, WPB * 64, 0, s>>>((const bf16_t*)x, (const bf16_t*)w, \
                                                                              (bf16_t*)y, M, I, K, rs);           \
   else gemm_skinny_glu_kernel<WPB, U, false, ACT><<<I / 16, WPB * 64, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,      \
                                                                         (bf16_t*)y, M, I, K, rs)
-  if (few) { GLU(4, 8); } else { GLU(2, 8); }
+  if (few) { GLU(4, 4); } else { GLU(2, 4); }
 #undef GLU
   HOLON_LAUNCH_OK();
   return 0;

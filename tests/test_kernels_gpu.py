@@ -1109,3 +1109,25 @@ def test_router_of_few_experts(hip, dtype):
                 assert close.sum() <= 1 + rows // 500 and torch.allclose(got[~close], want[~close], atol=2e-5), (name, how, experts, rows)
                 alone = op(x[-1:].contiguous(), *args[1:], **how)
                 assert torch.equal(alone[0], got[-1]), (name, how, experts, rows)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_stream_norm_across_its_widths(hip, dtype):
+    """The residual sum in float32 and its norm, at the edges of the widths a thread's registers are cut for, with operands on
+    and off 16-byte borders and terms of either type."""
+    from holon_amd.kernels.registry import kernel_op
+    plain = kernel_op("stream_norm").plain
+    for dim in (4, 1024, 1028, 2044, 2048, 2052, 4096, 4100, 8192, 8196, 1030):
+        weight = 1 + 0.2 * _randn(dim, dtype=dtype, seed=80)
+        for kinds in ((), (dtype,), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.bfloat16)):
+            for off in (0, 1):
+                x = torch.empty(3 * dim + off, device="cuda")[off:].view(3, dim)
+                x.copy_(_randn(3, dim, dtype=torch.float32, seed=81))
+                terms = [(_randn(3, dim, dtype=kind, seed=82 + i), 0.5 + i) for i, kind in enumerate(kinds)]
+                ref = x.double()
+                got = hip.stream_norm(x, terms, weight, 1e-5, dtype)
+                for term, factor in terms:
+                    ref = ref + term.double() * factor
+                assert (x.double() - ref).abs().max() <= 4 * 2.0 ** -24 * ref.abs().max() + 1e-6, (dim, kinds)
+                want = plain(ref, [], weight.double(), 1e-5, torch.float64)
+                assert H.op_budget_usage(got, want, dtype, dim) <= 1, (dim, kinds, off)

@@ -292,7 +292,8 @@ static void launch_skinny(const void* x, const void* w, void* y, int M, int N, i
 // 1 / 8 / 16 rows (in brackets: 8 loads in one set of registers, two tiles a block from 320 to 512 tiles and, from 10 rows
 // up, beyond 4,096):
 //   up to 319 tiles: one, two sets of 4 loads. 2048 x 8192 9.7 / 11.4 / 14.5 (11.6 / 12.4 / 15.3), 4096 x 4096 7.8 / 8.3 / 9.3
-//     (8.3 / 8.5 / 10.0).
+//     (8.3 / 8.5 / 10.0). Where the residual is added, 8 loads in one set: behind the kernels of a step of four rows, which leave
+//     4096 x 4096 and 4096 x 12288 cold, two sets took 13.9 on average and one 13.4.
 //   320 to 511: two (at 512, one: 8192 x 4096 13.8 / 15.1 / 16.0, two 15.0 / 16.1 / 16.0); two sets of 4 loads a tile up to 8 rows,
 //     of 2 above: 6144 x 4096 11.5 / 12.8 / 12.7 (12.0 / 12.9 / 14.3), 6144 x 5120 13.3 / 14.8 / 15.4 (16.8 / 17.8 / 19.1).
 //   from 1,024, and K below 4,096 or more than 8 rows: two, two sets of 2 loads a tile: 18432 x 2048 15.5 / 16.0 / 17.7 (15.6 /
@@ -309,7 +310,9 @@ static int pick_waves(const void* x, const void* w, void* y, int M, int N, int K
 #define SKINNY(NT, WPB, U, TWICE) \
   launch_skinny<NT, WPB, U, TWICE, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out)
   switch (wpb) {
-    case 16: SKINNY(1, 16, 4, true); break;
+    case 16:
+      if constexpr (RESID) { SKINNY(1, 16, 8, false); } else { SKINNY(1, 16, 4, true); }
+      break;
     case 8:
       if (!two) SKINNY(1, 8, 4, false);
       else if (tiles < 512 && M <= 8) SKINNY(2, 8, 4, true);

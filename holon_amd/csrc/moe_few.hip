@@ -79,8 +79,8 @@ __device__ __forceinline__ void in_two_sets(f32x4_t (&acc)[H], int steps_, At at
 }
 
 // One block 16 columns of the experts' activations: gate and up tile over all of K, split over the block's waves in order,
-// then round(round(round(silu(gate)) * up) * weight); GATED false: one tile and round(max(up, 0)^2 * weight). Blocks of an
-// expert that no row chose end at once and write nothing. 0 where the weight is 0.
+// then round(round(round(silu(gate)) * up) * weight); GATED false: one tile and round(max(up, 0)^2 * weight). Blocks of a
+// routed expert that no row chose end at once and write nothing. 0 where the weight is 0.
 template <int WPB, bool GATED>
 __global__ void __launch_bounds__(WPB * 64) moe_up_few_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                               bf16_t* __restrict__ y, int M, int cols, int K, Chosen ch) {
@@ -90,7 +90,9 @@ __global__ void __launch_bounds__(WPB * 64) moe_up_few_kernel(const bf16_t* __re
   const int g = lane / 16, c = lane % 16;
   const bool have = c < M;
   const float weight = have ? ch.of(c, blockIdx.x * 16) : 0.f;      // (16 columns are one expert's)
-  if (__ballot(weight != 0.f) == 0) return;
+  // The second product leaves out the experts that no row chose, never the shared one: its columns are written whatever its
+  // weights are, zeros where its gate has come to 0 for every row.
+  if (blockIdx.x * 16 < ch.experts * ch.ff && __ballot(weight != 0.f) == 0) return;
   const int steps = K / 32 / WPB;
   const bf16_t* wp[H];
 #pragma unroll

@@ -1131,3 +1131,28 @@ def test_stream_norm_across_its_widths(hip, dtype):
                 assert (x.double() - ref).abs().max() <= 4 * 2.0 ** -24 * ref.abs().max() + 1e-6, (dim, kinds)
                 want = plain(ref, [], weight.double(), 1e-5, torch.float64)
                 assert H.op_budget_usage(got, want, dtype, dim) <= 1, (dim, kinds, off)
+
+
+@pytest.mark.parametrize("shared", (64, 512))
+@pytest.mark.parametrize("gated", (True, False))
+def test_a_shared_expert_whose_gate_is_shut(hip, gated, shared):
+    """A shared expert's weight of exactly 0 (the sigmoid of anything below -88 or so) for every row of a step, and for some of
+    them: bit for bit the products over all experts, whatever the memory of the activations held before."""
+    bf, hidden, experts, ff = torch.bfloat16, 256, 4, 96
+    cols = experts * ff + shared
+    up_w = _randn((2 if gated else 1) * cols, hidden, dtype=bf, seed=90, scale=hidden ** -0.5)
+    down_w = _randn(hidden, cols, dtype=bf, seed=91, scale=ff ** -0.5)
+    up_t, down_t = hip.tile_weight(up_w), hip.tile_weight(down_w)
+    between = hip.moe_gate if gated else hip.moe_relu2
+    for m, open_rows in ((1, 0), (3, 0), (16, 0), (1, 1), (16, 5)):
+        x = _randn(m, hidden, dtype=bf, seed=92 + m)
+        weights = torch.zeros(m, experts + 1)
+        weights[:, 1] = 0.4
+        weights[:open_rows, experts] = 0.7
+        weights = weights.cuda()
+        garbage = torch.full((m, cols), float("nan"), dtype=bf, device="cuda")
+        del garbage                            # what the next allocation of this size finds
+        got = hip.moe_few(x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=True)
+        whole = hip.linear(between(hip.linear(x, up_w, tiled=up_t), weights, ff, shared, shared_weight=True), down_w,
+                           tiled=down_t)
+        assert torch.equal(got, whole), (m, open_rows)

@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
   static_assert(N % THREADS == 0 && KD == 4 * VW * NW * U, "whole tiles");
   __shared__ __attribute__((aligned(16))) float as_[N], ks_[N], qs_[OUT ? N : 4];
   __shared__ __attribute__((aligned(16))) float qp_[OUT ? TB * QP : 4], kt_[KD * TP], P_[KD];
-  __shared__ __attribute__((aligned(16))) float red_[OUT ? NW * TB * TB : 4], us_[BONUS ? KD : 4];
+  __shared__ __attribute__((aligned(16))) float red_[OUT ? NW * TB * TB : 4], us_[BONUS && OUT ? KD : 4];
   const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   const int g4 = lane / 16, c = lane % 16;
   const int col_blocks = (r.vdim + 16 * NW - 1) / (16 * NW);
@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
   const bool some = OUT && (!from_slot || carried);        // whether there is a state to start from
   const int j = col0 + 16 * wave + c;                      // this lane's value column
   const bool col = j < vdim;
-  if constexpr (BONUS)
+  if constexpr (BONUS && OUT)
     for (int d = tid; d < KD; d += THREADS) us_[d] = d < dim ? r.bonus[(int64_t)h * dim + d] : 0.f;
   f32x4 S[DT];
 #pragma unroll
@@ -240,22 +240,32 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
     }
     lds_barrier();
     if constexpr (OUT) {
-      f32x4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const f32x4 qa = *reinterpret_cast<const f32x4*>(&qp_[c * QP + 16 * dt + 4 * g4]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i], S[dt][i], o[i % 2], 0, 0, 0);
-      }
       f32x4 sa = *reinterpret_cast<const f32x4*>(&red_[c * TB + 4 * g4]);      // the waves' scores, added up in order
 #pragma unroll
       for (int w = 1; w < NW; ++w) sa += *reinterpret_cast<const f32x4*>(&red_[(w * TB + c) * TB + 4 * g4]);
+      constexpr int CH = BONUS ? 4 : 2, RUN = BONUS ? 4 : DT;      // chains side by side, and how many groups of 16 a chain is long
+      f32x4 o[CH], read;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[i], vv[i], o[i % 2], 0, 0, 0);
+      for (int d0 = 0; d0 < DT; d0 += RUN) {
+#pragma unroll
+        for (int i = 0; i < CH; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int dt = d0; dt < d0 + RUN && dt < DT; ++dt) {
+          const f32x4 qa = *reinterpret_cast<const f32x4*>(&qp_[c * QP + 16 * dt + 4 * g4]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[i], S[dt][i], o[i % CH], 0, 0, 0);
+        }
+        if (d0 + RUN >= DT)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[i], vv[i], o[i % CH], 0, 0, 0);
+        f32x4 sum = o[0] + o[1];
+        if constexpr (CH == 4) sum += o[2] + o[3];
+        read = d0 ? read + sum : sum;
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = t0 + 4 * g4 + i;
-        if (t < hi && col) out[((int64_t)t * r.heads + h) * vdim + j] = o[0][i] + o[1][i];
+        if (t < hi && col) out[((int64_t)t * r.heads + h) * vdim + j] = read[i];
       }
     }
     if (!OUT || t0 + TB < hi || to_slot) {
@@ -263,9 +273,16 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
       for (int dt = 0; dt < DT; ++dt) {
         const f32x4 pd = *reinterpret_cast<const f32x4*>(&P_[16 * dt + 4 * g4]);
         const f32x4 ka = *reinterpret_cast<const f32x4*>(&kt_[(16 * dt + c) * TP + 4 * g4]);
-        S[dt] *= pd;
+        if constexpr (BONUS) {                             // the block's part by itself: S is rounded once a block
+          f32x4 add = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i], vv[i], S[dt], 0, 0, 0);
+          for (int i = 0; i < 4; ++i) add = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i], vv[i], add, 0, 0, 0);
+          S[dt] = S[dt] * pd + add;
+        } else {
+          S[dt] *= pd;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) S[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[i], vv[i], S[dt], 0, 0, 0);
+        }
       }
     }
     // (no barrier: the next block's operands go where only the part before the last barrier read, and what this part reads
@@ -450,8 +467,8 @@ extern "C" int holon_gla_decay(const void* a, int64_t a_stride, const void* w2t,
 template <int KD, int NW, bool BONUS, typename T>
 static void launch_gla(int pass, dim3 grid, hipStream_t s, const void* q, const void* k, const void* v, int64_t stride,
                        float q_scale, const float* alpha, float* state, float* out, GlaRows r) {
-  if (pass == 1)                                           // (what a piece adds does not depend on how it is read)
-    gla_scan_kernel<KD, NW, 1, false, T><<<grid, NW * WAVE, 0, s>>>((const T*)q, (const T*)k, (const T*)v, stride, q_scale,
+  if (pass == 1)
+    gla_scan_kernel<KD, NW, 1, BONUS, T><<<grid, NW * WAVE, 0, s>>>((const T*)q, (const T*)k, (const T*)v, stride, q_scale,
                                                                     alpha, state, out, r);
   else
     gla_scan_kernel<KD, NW, 2, BONUS, T><<<grid, NW * WAVE, 0, s>>>((const T*)q, (const T*)k, (const T*)v, stride, q_scale,

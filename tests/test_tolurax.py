@@ -354,3 +354,34 @@ def test_the_memory_in_pieces(heads, dim, dtype):
     got = k.memory_scan(r, kk, v, w, u, one, *rows, (piece, max(npc), i32([sum(npc[:b]) for b in range(5)]), sum(npc)))
     want = kernel_op("memory_scan").plain(r.double().float(), kk, v, w, u, two, *rows)
     assert H.rel_rms(got, want) < 2e-6 and H.rel_rms(one, two) < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dim,shift", [(64, -5), (64, 0), (128, -5), (200, -5)])
+def test_the_memory_in_pieces_is_as_near_64_bits_as_token_by_token(dim, shift, dtype):
+    """Long sums (decays near one) and short ones: rows in pieces may be at most 1.1 times as far from the recurrence in float64
+    as the token-by-token scan of the same row, in results and, where decays are near one, state."""
+    from holon_amd.kernels import load_hip
+    k, dev, heads, t = load_hip(), torch.device("cuda"), 8, 1000
+    gen = torch.Generator().manual_seed(dim + shift)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
+    r, kk, v = (rn(t, heads * dim).to(dtype) for _ in range(3))
+    w = torch.exp(-torch.exp(rn(t, heads * dim) + shift))
+    u, state = rn(heads, dim), rn(2, heads, dim, dim)
+    rows = (i32([1]), i32([7]), i32([0, t]), 1, heads)
+    S, want = state[1].double(), torch.empty(t, heads, dim, dtype=torch.double, device=dev)
+    rd, kd, vd, wd = (x.double().view(t, heads, dim) for x in (r, kk, v, w))
+    for i in range(t):
+        kv = kd[i][:, :, None] * vd[i][:, None, :]
+        want[i] = ((S + u.double()[:, :, None] * kv) * rd[i][:, :, None]).sum(1)
+        S = wd[i][:, :, None] * S + kv
+    apart = []
+    for pieces in (None, (128, 8, i32([0]), 8)):
+        held = state.clone()
+        got = k.memory_scan(r, kk, v, w, u, held, *rows, pieces).view_as(want)
+        apart.append((((got - want).norm() / want.norm()).item(), ((held[1] - S).norm() / S.norm()).item()))
+    assert apart[1][0] <= 1.1 * apart[0][0], apart
+    if shift < 0:                              # (fast decays: what is left of a state is its last few tokens)
+        assert apart[1][1] <= 1.1 * apart[0][1], apart

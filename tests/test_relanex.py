@@ -577,3 +577,44 @@ def test_trace_runner_as_a_program(folders, tmp_path):
         for row, key in zip(rows, expect):
             got[key] = torch.from_numpy(row.copy())
     _check(folder, "float32", requests, got, "trace_run")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,d,v", [(8, 128, 128), (4, 256, 512), (8, 64, 64), (3, 40, 56)])
+def test_the_matrix_memory_in_pieces_is_as_near_64_bits_as_token_by_token(heads, d, v, dtype):
+    """Rows in pieces may be at most 1.1 times as far from the recurrence in float64 as the token-by-token scan of the same
+    row, in numerators and denominators; 1.25 times in the state, as their gates' running maximum comes from a prefix over runs of
+    tokens, whose sums of logarithms are rounded at their borders (up to 1.15 with a scan of either kind behind it)."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    k, dev, t = load_hip(), torch.device("cuda"), 1000
+    gen = torch.Generator().manual_seed(d + v)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)             # noqa: E731
+    hd, hv, copies = heads * d, heads * v, -(-(v + 1) // 8)
+    proj, gb = rn(t, -(-(2 * hd + 2 * hv + 2 * heads) // 16) * 16).to(dtype), rn(2 * heads)
+    state = [rn(2, heads, d, v + 1), rn(2, heads, 1).expand(2, heads, copies).contiguous()]
+    args = (proj, 0, hd, 2 * hd, 2 * hd + 2 * hv, gb, 12.0)
+    rows = (i32([1]), i32([7]), i32([0, t]), 1, heads, d, v)
+    pd = proj.double()
+    q, kk, vv = pd[:, :hd].view(t, heads, d) * d ** -0.5, pd[:, hd:2 * hd].view(t, heads, d), pd[:, 2 * hd:2 * hd + hv].view(t, heads, v)
+    gate = 12 * torch.tanh((pd[:, 2 * hd + 2 * hv:2 * hd + 2 * hv + 2 * heads] + gb.double()) / 12)
+    gi, gf = gate[:, :heads], torch.nn.functional.logsigmoid(gate[:, heads:])
+    vv = torch.cat((vv, torch.ones(t, heads, 1, dtype=torch.double, device=dev)), 2)
+    S, m = state[0][1].double(), state[1][1, :, 0].double()
+    want = torch.empty(t, heads, v + 1, dtype=torch.double, device=dev)
+    for i in range(t):
+        m_new = torch.maximum(gf[i] + m, gi[i])
+        S = torch.exp(gf[i] + m - m_new)[:, None, None] * S \
+            + torch.exp(gi[i] - m_new)[:, None, None] * kk[i][:, :, None] * vv[i][:, None, :]
+        m = m_new
+        want[i] = (S * q[i][:, :, None]).sum(1)
+        want[i, :, v] = torch.maximum(want[i, :, v].abs(), torch.exp(-m)) + 1e-6
+    off = lambda got, ref: ((got - ref).norm() / ref.norm()).item()            # noqa: E731
+    apart = []
+    for pieces in (None, (256, 4, i32([0]), 4)):
+        held = [x.clone() for x in state]
+        out, under = k.mlstm_scan(*args, *held, *rows, pieces)
+        apart.append((off(out, want[..., :v]), off(under, want[..., v]), off(held[0][1], S)))
+    assert all(b <= most * a for a, b, most in zip(*apart, (1.1, 1.1, 1.25))), apart

@@ -362,6 +362,7 @@ def test_the_memory_in_pieces(heads, dim, dtype):
 def test_the_memory_in_pieces_is_as_near_64_bits_as_token_by_token(dim, shift, dtype):
     """Long sums (decays near one) and short ones: rows in pieces may be at most 1.1 times as far from the recurrence in float64
     as the token-by-token scan of the same row, in results and, where decays are near one, state."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
     from holon_amd.kernels import load_hip
     k, dev, heads, t = load_hip(), torch.device("cuda"), 8, 1000
     gen = torch.Generator().manual_seed(dim + shift)

@@ -106,8 +106,9 @@ __global__ void __launch_bounds__(GEN_WAVES * WAVE) attention_generic_kernel(
 #pragma unroll
     for (int h = 0; h < HG; ++h) {
       const float m_new = fmaxf(m[h], wave_max(s[h]));
-      const float alpha = expf(m[h] - m_new);             // m = -inf on the first tile: alpha = 0
-      const float p = j0 + mine <= pos ? expf(s[h] - m_new) : 0.f;
+      const float at = m_new == -INFINITY ? 0.f : m_new;  // (scores of -inf weigh 0, one that is NaN stays one)
+      const float alpha = expf(m[h] - at);                // m = -inf on the first tile: alpha = 0
+      const float p = j0 + mine <= pos ? expf(s[h] - at) : 0.f;
       l[h] = l[h] * alpha + wave_sum(p);
       m[h] = m_new;
       p_s[w][h][mine] = (Acc)p;
@@ -168,8 +169,7 @@ __global__ void __launch_bounds__(GEN_WAVES * WAVE) attention_generic_kernel(
     float den = 0.f;
 #pragma unroll
     for (int i = 0; i < GEN_WAVES; ++i) {
-      if (ml_s[i][h][0] == -INFINITY) continue;           // a wave without keys
-      const float f = expf(ml_s[i][h][0] - top);
+      const float f = expf(ml_s[i][h][0] - top);          // (0 for a wave without keys, whose sums are 0 too)
       den += ml_s[i][h][1] * f;
       sum += sum_s[i][h][d] * (Acc)f;
     }

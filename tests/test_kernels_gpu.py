@@ -1156,3 +1156,28 @@ def test_a_shared_expert_whose_gate_is_shut(hip, gated, shared):
         whole = hip.linear(between(hip.linear(x, up_w, tiled=up_t), weights, ff, shared, shared_weight=True), down_w,
                            tiled=down_t)
         assert torch.equal(got, whole), (m, open_rows)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_general_attention_with_keys_that_are_not_finite(hip, dtype):
+    """Keys of NaN and of -inf in different tiles of 64, alone in their tile and among others: a NaN score makes the results of
+    every query that sees its key NaN and no others', a score of -inf weighs nothing."""
+    page, d, n = 16, 48, 700                    # (48: a size the matrix-core kernels do not serve)
+    most = -(-n // page)
+    pages = _randn(most, 2, 1, page * d, dtype=dtype, seed=95)
+    table = torch.arange(most, dtype=torch.int32, device="cuda")[None]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")            # noqa: E731
+    rows = AttnRows(slots=i32([0]), lens=i32([n]), query_start=i32([0, n]), decode_rows=None, chunk_rows=i32([0]), n_decode=0,
+                    n_chunk=1, max_decode_len=0, max_chunk_query=n, max_chunk_len=n)
+    q = _randn(n, 2, d, dtype=dtype, seed=96).abs() + 0.1
+    for at, count, value in ((640, 60, "nan"), (699, 1, "nan"), (100, 1, "nan"), (130, 1, "-inf"), (320, 64, "-inf"), (0, 1, "-inf")):
+        held = pages.clone()
+        for key in range(at, at + count):
+            pages[key // page, 0, 0, key % page * d: (key % page + 1) * d] = float(value)
+        got = hip.paged_attention(q, pages, table, rows, page, d ** -0.5, 0).cpu()
+        want = TorchKernels().paged_attention(q.float().cpu(), pages.float().cpu(), table.cpu(), AttnRows(
+            **{k: v.cpu() if torch.is_tensor(v) else v for k, v in rows.__dict__.items()}), page, d ** -0.5, 0)
+        gone = torch.isnan(want)
+        assert torch.equal(torch.isnan(got), gone) and gone.any() == (value == "nan" or at == 0), (at, value)
+        assert H.rel_rms(got[~gone], want[~gone]) < (1e-5 if dtype == torch.float32 else 1e-2), (at, value)
+        pages.copy_(held)

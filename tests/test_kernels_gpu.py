@@ -1170,7 +1170,8 @@ def test_general_attention_with_keys_that_are_not_finite(hip, dtype):
     rows = AttnRows(slots=i32([0]), lens=i32([n]), query_start=i32([0, n]), decode_rows=None, chunk_rows=i32([0]), n_decode=0,
                     n_chunk=1, max_decode_len=0, max_chunk_query=n, max_chunk_len=n)
     q = _randn(n, 2, d, dtype=dtype, seed=96).abs() + 0.1
-    for at, count, value in ((640, 60, "nan"), (699, 1, "nan"), (100, 1, "nan"), (130, 1, "-inf"), (320, 64, "-inf"), (0, 1, "-inf")):
+    for at, count, value in ((64, 1, "nan"), (320, 64, "nan"), (640, 60, "nan"), (699, 1, "nan"), (130, 1, "-inf"),
+                             (320, 64, "-inf"), (0, 1, "-inf")):
         held = pages.clone()
         for key in range(at, at + count):
             pages[key // page, 0, 0, key % page * d: (key % page + 1) * d] = float(value)

@@ -35,7 +35,8 @@ __global__ void __launch_bounds__(GEN_WAVES * WAVE) attention_generic_kernel(
   __shared__ Acc p_s[GEN_WAVES][HG][WAVE];
   __shared__ float ml_s[GEN_WAVES][HG][2];
   const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int t = blockIdx.x, h0 = blockIdx.y * HG;
+  const int t = blockIdx.x, h0 = (blockIdx.z * gridDim.y + blockIdx.y) * HG;
+  if (h0 >= heads) return;                                // (uniform over the block: the last of a second round of heads)
   // the row of token t: the last b with query_start[b] <= t
   int lo_b = 0, hi_b = rows - 1;
   while (lo_b < hi_b) {
@@ -181,7 +182,8 @@ template <typename T, int DB, int HG>
 void launch(bool vvec, hipStream_t s, const T* q, T* out, const T* pages, const int32_t* table, int table_stride,
             const int32_t* slots, const int32_t* lens, const int32_t* query_start, int rows, int tokens, int heads,
             int kv_heads, int head_dim, int page_size, float scale, int window) {
-  const dim3 grid(tokens, heads / HG);
+  const int groups = heads / HG, rounds = (groups + 65534) / 65535;       // (a grid's second number has 16 bits)
+  const dim3 grid(tokens, (groups + rounds - 1) / rounds, rounds);
   if (vvec)
     attention_generic_kernel<T, DB, HG, true><<<grid, GEN_WAVES * WAVE, 0, s>>>(q, out, pages, table, table_stride, slots, lens,
         query_start, rows, heads, kv_heads, head_dim, page_size, scale, window);
@@ -225,7 +227,6 @@ extern "C" int holon_attention_generic(const void* q, void* out, const void* pag
               "attention: head_dim %d must be a multiple of 8, at most %d", head_dim, GEN_MAX_D);
   HOLON_CHECK(page_size > 0 && num_pages > 0 && window > -0x7fffffff, "attention: bad page size or window");
   if (tokens == 0 || rows == 0) return 0;
-  HOLON_CHECK(heads <= 65535, "attention: %d heads exceed one launch", heads);
   hipStream_t s = (hipStream_t)stream;
   if (dtype == HOLON_F32)
     by_size<float>(s, q, out, pages, table, table_stride, slots, lens, query_start, rows, tokens, heads, kv_heads, head_dim,

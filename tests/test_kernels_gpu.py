@@ -1182,3 +1182,15 @@ def test_general_attention_with_keys_that_are_not_finite(hip, dtype):
         assert torch.equal(torch.isnan(got), gone) and gone.any() == (value == "nan" or at == 0), (at, value)
         assert H.rel_rms(got[~gone], want[~gone]) < (1e-5 if dtype == torch.float32 else 1e-2), (at, value)
         pages.copy_(held)
+
+
+def test_general_attention_with_more_heads_than_a_grid_has_rows(hip):
+    """65,537 heads (a grid's second number ends at 65,535), each with keys and values of its own, and 131,074 on as many pairs."""
+    page, d = 4, 8
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")            # noqa: E731
+    rows = AttnRows(slots=i32([0]), lens=i32([3]), query_start=i32([0, 1]), decode_rows=i32([0]), chunk_rows=None, n_decode=1,
+                    n_chunk=0, max_decode_len=3, max_chunk_query=0, max_chunk_len=0)
+    for heads, kv in ((65537, 65537), (131074, 65537)):
+        pages, q = _randn(1, 2, kv, page * d, dtype=torch.float32, seed=97), _randn(1, heads, d, dtype=torch.float32, seed=98)
+        args = (torch.zeros(1, 1, dtype=torch.int32, device="cuda"), rows, page, 0.5, 0)
+        assert H.rel_rms(hip.paged_attention(q, pages, *args), TorchKernels().paged_attention(q, pages, *args)) < 1e-5

@@ -48,6 +48,8 @@ __device__ __forceinline__ float log_sigmoid(float x) {   // -softplus(-x), with
   return fminf(x, 0.f) - log1pf(expf(-fabsf(x)));
 }
 
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
+
 struct MlstmPieces {
   int tokens;                  // tokens a piece
   const int32_t* base;         // [rows]: the number of row b's first piece among all pieces of the step
@@ -391,7 +393,8 @@ __global__ void __launch_bounds__(512) mlstm_chunk_kernel(const T* __restrict__ 
           for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)qa[i], (double)kb[i], sum, 0, 0, 0);
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) score[(16 * ti + 4 * i + g4) * MS + 16 * tj + c] = (float)sum[i];
+        for (int i = 0; i < 4; ++i)                        // (above the diagonal: 0, whatever a later token's key holds)
+          score[(16 * ti + 4 * i + g4) * MS + 16 * tj + c] = tj < ti || 4 * i + g4 >= c ? (float)sum[i] : 0.f;
       }
     }
     lds_barrier();
@@ -416,13 +419,32 @@ __global__ void __launch_bounds__(512) mlstm_chunk_kernel(const T* __restrict__ 
           const int at = (16 * ti + c) * MS + 16 * tj + 4 * g4;
           const f32x4 sa = *reinterpret_cast<const f32x4*>(&score[at]) * *reinterpret_cast<const f32x4*>(&fade[at]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[i], vv[tj][i], o[i], 0, 0, 0);
+          for (int i = 0; i < 4; ++i)                      // (a value times the 0 above the diagonal: see below)
+            o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[i], tj < ti || finite(vv[tj][i]) ? vv[tj][i] : 0.f, o[i], 0, 0, 0);
         }
         const f32x4 sum = old + ((o[0] + o[1]) + (o[2] + o[3]));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int t = t0 + 16 * ti + 4 * g4 + i;
           if (t < hi && col) out[((int64_t)t * heads + h) * vdim + j] = sum[i];
+        }
+      }
+      // A value that is not finite belongs into its own token's result and the later ones', and the products on the diagonal,
+      // where it would meet the earlier ones' zeros, went without it: those of its 16 tokens get it here, the lane that stored
+      // a result adding to it.
+      bool odd = false;
+#pragma unroll
+      for (int tt = 0; tt < CT; ++tt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) odd |= !finite(vv[tt][i]);
+      if (__ballot(odd) != 0) {
+#pragma nounroll
+        for (int q = 0; q < min(C, hi - t0); ++q) {
+          const float v = Elem<T>::load(proj[(int64_t)(t0 + q) * width + v_off + h * vdim + min(j, vdim - 1)]);
+          if (finite(v) || !col) continue;
+#pragma nounroll
+          for (int t = max(q, q / 16 * 16 + 4 * g4); t < q / 16 * 16 + 4 * g4 + 4; ++t)
+            if (t0 + t < hi) out[((int64_t)(t0 + t) * heads + h) * vdim + j] += score[t * MS + q] * fade[t * MS + q] * v;
         }
       }
       if (col0 == 0) {                                     // the denominators: TPT neighbouring lanes a token

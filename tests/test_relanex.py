@@ -618,3 +618,38 @@ def test_the_matrix_memory_in_pieces_is_as_near_64_bits_as_token_by_token(heads,
         out, under = k.mlstm_scan(*args, *held, *rows, pieces)
         apart.append((off(out, want[..., :v]), off(under, want[..., v]), off(held[0][1], S)))
     assert all(b <= most * a for a, b, most in zip(*apart, (1.1, 1.1, 1.25))), apart
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("what", ["k", "v"])
+@pytest.mark.parametrize("d", [40, 128, 200])
+def test_the_matrix_memory_in_pieces_keeps_what_is_not_finite_from_earlier_tokens(d, what, dtype):
+    """A key or value of NaN or infinity: the tokens before it come out bit for bit as without it, those from it on as the
+    plain form's (a value: its own column alone)."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.registry import kernel_op
+    k, dev, heads, v, t = load_hip(), torch.device("cuda"), 2, 24, 300
+    gen = torch.Generator().manual_seed(d)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)             # noqa: E731
+    hd, hv, copies = heads * d, heads * v, -(-(v + 1) // 8)
+    clean, gb = rn(t, -(-(2 * hd + 2 * hv + 2 * heads) // 16) * 16).to(dtype), rn(2 * heads)
+    state = [rn(1, heads, d, v + 1), rn(1, heads, 1).expand(1, heads, copies).contiguous()]
+    rows = (i32([0]), i32([7]), i32([0, t]), 1, heads, d, v)
+    run = lambda op, proj, *cut: op(proj, 0, hd, 2 * hd, 2 * hd + 2 * hv, gb, 12.0, *[x.clone() for x in state], *rows, *cut)  # noqa: E731
+    for at, value in ((0, "nan"), (5, "inf"), (37, "-inf"), (140, "nan"), (255, "inf"), (299, "nan")):
+        proj = clean.clone()
+        proj[at, hd + 3 if what == "k" else 2 * hd + 7] = float(value)
+        cut = (128, 3, i32([0]), 3)
+        out, den = run(k.mlstm_scan, proj, cut)
+        ref, ref_den = run(k.mlstm_scan, clean, cut)
+        assert torch.equal(out[:at], ref[:at]) and torch.equal(den[:at], ref_den[:at]), (at, value)
+        if what == "v":                        # head 0, column 7: nothing else may change
+            out[:, 0, 7] = ref[:, 0, 7] = 0
+            assert torch.equal(out, ref) and torch.equal(den, ref_den), (at, value)
+        else:
+            want, _ = run(kernel_op("mlstm_scan").plain, proj)
+            assert torch.equal(torch.isfinite(out[at:, 0]).any(), torch.isfinite(want[at:, 0]).any()), (at, value)
+            assert torch.equal(out[:, 1], ref[:, 1]), (at, value)

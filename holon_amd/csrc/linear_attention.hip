@@ -79,6 +79,8 @@ template <int CTRL> __device__ __forceinline__ float dpp_add(float v) {
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
 
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
+
 // A block: one (row or piece, head) and 16 NW value columns, wave w columns 16 w .. 16 w + 15 of them, S's KD x 16 part of
 // a wave in its matrix-core accumulators. KD: the key size padded with zeros (a zero key writes nothing).
 // BONUS: the read-out comes before the write and the token's own key enters it with weights of its own,
@@ -257,7 +259,8 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
         }
         if (d0 + RUN >= DT)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[i], vv[i], o[i % CH], 0, 0, 0);
+          for (int i = 0; i < 4; ++i)                      // (a value times the 0 of an earlier token: see below)
+            o[i % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(sa[i], finite(vv[i]) ? vv[i] : 0.f, o[i % CH], 0, 0, 0);
         f32x4 sum = o[0] + o[1];
         if constexpr (CH == 4) sum += o[2] + o[3];
         read = d0 ? read + sum : sum;
@@ -266,6 +269,21 @@ __global__ void __launch_bounds__(NW * WAVE, KD <= 64 ? 4 : 1) gla_scan_kernel(c
       for (int i = 0; i < 4; ++i) {
         const int t = t0 + 4 * g4 + i;
         if (t < hi && col) out[((int64_t)t * r.heads + h) * vdim + j] = read[i];
+      }
+      // A value that is not finite belongs into its own token's result and the later ones': the products above, where it would
+      // meet the earlier ones' zeros, went without it, and the lane that stored a result adds it there.
+      if (__ballot(!(finite(vv[0]) && finite(vv[1]) && finite(vv[2]) && finite(vv[3]))) != 0) {
+#pragma nounroll
+        for (int n = 0; n < min(TB, hi - t0); ++n) {
+          const float val = Elem<T>::load(v[(int64_t)(t0 + n) * stride + (int64_t)h * vdim + min(j, vdim - 1)]);
+          if (finite(val) || !col) continue;
+#pragma nounroll
+          for (int t = max(n, 4 * g4); t < 4 * g4 + 4; ++t) {
+            float score = red_[t * TB + n];
+            for (int w = 1; w < NW; ++w) score += red_[(w * TB + t) * TB + n];
+            if (t0 + t < hi) out[((int64_t)(t0 + t) * r.heads + h) * vdim + j] += score * val;
+          }
+        }
       }
     }
     if (!OUT || t0 + TB < hi || to_slot) {

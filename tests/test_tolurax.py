@@ -386,3 +386,36 @@ def test_the_memory_in_pieces_is_as_near_64_bits_as_token_by_token(dim, shift, d
     assert apart[1][0] <= 1.1 * apart[0][0], apart
     if shift < 0:                              # (fast decays: what is left of a state is its last few tokens)
         assert apart[1][1] <= 1.1 * apart[0][1], apart
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,dim", [(2, 24), (2, 64), (1, 128), (1, 200)])
+def test_the_memory_in_pieces_keeps_what_is_not_finite_from_earlier_tokens(heads, dim, dtype):
+    """A key or value of NaN or infinity: the tokens before it come out bit for bit as without it, those from it on are the
+    token-by-token scan's in where they are finite (a value: its own column alone)."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    k, dev, t = load_hip(), torch.device("cuda"), 300
+    gen = torch.Generator().manual_seed(dim)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
+    r, kk, v = (rn(t, heads * dim).to(dtype) for _ in range(3))
+    w = torch.exp(-torch.exp(rn(t, heads * dim) - 2))
+    u, state = rn(heads, dim), rn(1, heads, dim, dim)
+    cut = (128, 3, i32([0]), 3)
+    run = lambda key, val, pieces: k.memory_scan(r, key, val, w, u, state.clone(), i32([0]), i32([7]), i32([0, t]), 1, heads,  # noqa: E731
+                                                 pieces).view(t, heads, dim)
+    ref = run(kk, v, cut)
+    for at, value in ((0, "nan"), (5, "inf"), (37, "-inf"), (140, "nan"), (255, "inf"), (299, "nan")):
+        key, val = kk.clone(), v.clone()
+        key[at, 3] = float(value)
+        val[at, 7] = float(value)
+        got = run(key, v, cut)
+        assert torch.equal(got[:at], ref[:at]), (at, value)
+        assert torch.equal(got.isfinite(), run(key, v, None).isfinite()), (at, value)
+        got = run(kk, val, cut)
+        assert torch.equal(got[:at], ref[:at]), (at, value)
+        assert torch.equal(got.isfinite(), run(kk, val, None).isfinite()), (at, value)
+        got[:, 0, 7] = ref[:, 0, 7]
+        assert torch.equal(got, ref), (at, value)

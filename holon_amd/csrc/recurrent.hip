@@ -299,9 +299,10 @@ __global__ void __launch_bounds__(WAVE) delta_scan_kernel(const float* __restric
   const bool active = j < columns;
   int lo = query_start[b], hi = query_start[b + 1];
   bool from_slot = true, to_slot = true;
+  int pieces = 1;
   int64_t piece_no = 0;
   if (pc.tokens > 0) {                                   // (everything here is the same in all of the block's lanes)
-    const int pieces = (hi - lo + pc.tokens - 1) / pc.tokens;
+    pieces = (hi - lo + pc.tokens - 1) / pc.tokens;
     if (piece >= pieces || (local && piece == pieces - 1)) return;
     lo += piece * pc.tokens;
     hi = min(hi, lo + pc.tokens);
@@ -310,15 +311,15 @@ __global__ void __launch_bounds__(WAVE) delta_scan_kernel(const float* __restric
     piece_no = pc.base[b] + piece;
   }
   float* held = state + ((int64_t)slots[b] * heads + h) * dim * vdim;
-  const bool carried = starts[b] > 0;
+  const float* before = pieces == 1 ? held : pc.sin + ((piece_no + (from_slot ? pieces : 0) - 1) * heads + h) * dim * vdim;
+  const bool some = !from_slot || starts[b] > 0;         // whether there is a state to start from
   float S[KQ];
 #pragma unroll
   for (int i = 0; i < KQ; ++i) {
     const int row = part * KQ + i;
     const bool in = active && row < dim;
     if (local) S[i] = (in && j >= vdim && row == j - vdim) ? 1.f : 0.f;
-    else if (from_slot) S[i] = (carried && in) ? held[(int64_t)row * vdim + j] : 0.f;
-    else S[i] = in ? pc.sin[((piece_no - 1) * heads + h) * dim * vdim + (int64_t)row * vdim + j] : 0.f;
+    else S[i] = some && in ? before[(int64_t)row * vdim + j] : 0.f;
   }
   float nk[PER], nq[PER], nv[VPER], ng = 1.f, nb = 0.f;
   auto ask = [&](int t0) {
@@ -400,7 +401,8 @@ __global__ void __launch_bounds__(WAVE) delta_scan_kernel(const float* __restric
 
 // Between the two passes: a row's pieces in order, S <- A S + B, sixteen columns of S a block (columns never meet).
 // A comes through LDS in slabs of 32 columns, S's sixteen columns stay there. sin[p] becomes the state piece p + 1
-// starts from.
+// starts from, and the last piece's place, which nothing is added to, takes the state the row starts from: the slot may no
+// longer hold it when piece 0 comes to read it, as the last piece writes it in the same launch.
 __global__ void __launch_bounds__(256) delta_pieces_kernel(const float* __restrict__ state,
                                                            const int32_t* __restrict__ slots,
                                                            const int32_t* __restrict__ starts,
@@ -416,6 +418,8 @@ __global__ void __launch_bounds__(256) delta_pieces_kernel(const float* __restri
   for (int e = threadIdx.x; e < MAXD * 16; e += 256) {      // (rows from dim on stay zero: the slabs reach past dim)
     const int m = e / 16, j = j0 + e % 16;
     sc[e] = carried && m < dim && j < vdim ? held[(int64_t)m * vdim + j] : 0.f;
+    if (pieces > 1 && m < dim && j < vdim)
+      pc.sin[(((int64_t)pc.base[b] + pieces - 1) * heads + h) * dim * vdim + (int64_t)m * vdim + j] = sc[e];
   }
   for (int e = dim * SLAB + threadIdx.x; e < MAXD * SLAB; e += 256) as[e / SLAB][e % SLAB] = 0.f;   // rows no slab fills
   const int c = threadIdx.x % 16;                            // this thread's column of the sixteen, whatever k

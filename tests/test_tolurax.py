@@ -419,3 +419,36 @@ def test_the_memory_in_pieces_keeps_what_is_not_finite_from_earlier_tokens(heads
         assert torch.equal(got.isfinite(), run(kk, val, None).isfinite()), (at, value)
         got[:, 0, 7] = ref[:, 0, 7]
         assert torch.equal(got, ref), (at, value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(2, 1, 64, 64), (4, 2, 24, 40), (1, 1, 128, 72), (2, 2, 200, 16)])
+def test_the_delta_rule_in_pieces_starts_from_a_copy(heads, kv, dim, vdim, monkeypatch):
+    """`delta_scan` with rows in pieces against its plain form, carried rows of several pieces among them. The second pass writes
+    a row's slot from its last piece while its first one starts, so the first one's start lies in the workspace, in the last
+    piece's place."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.registry import kernel_op
+    k, dev = load_hip(), torch.device("cuda")
+    gen = torch.Generator().manual_seed(dim)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
+    counts, piece = [513, 256, 1, 257, 300], 256
+    t, npc = sum(counts), [-(-n // piece) for n in counts]
+    norm = lambda x: x / x.norm(dim=-1, keepdim=True)                          # noqa: E731
+    qn, kn = norm(rn(t, kv, dim)), norm(rn(t, kv, dim))
+    qkv, beta, g = rn(t, 2 * kv * dim + heads * vdim), torch.rand(t, heads, generator=gen).to(dev), torch.exp(-rn(t, heads).abs() / 20)
+    state, base = rn(7, heads, dim, vdim), [sum(npc[:b]) for b in range(5)]
+    slots, starts = [6, 1, 2, 0, 4], [5, 0, 9, 3, 0]
+    rows = (i32(slots), i32(starts), i32([sum(counts[:b]) for b in range(6)]), 5, heads, vdim)
+    one, two, made, empty = state.clone(), state.clone(), [], torch.empty
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", lambda *a, **kw: made.append(empty(*a, **kw)) or made[-1])
+        got = k.delta_scan(qn, kn, qkv, beta, g, one, *rows, (piece, max(npc), i32(base), sum(npc)))
+    want = kernel_op("delta_scan").plain(qn, kn, qkv, beta, g, two, *rows)
+    assert H.rel_rms(got, want) < 1e-5 and H.rel_rms(one, two) < 1e-5
+    starts_of = [x for x in made if tuple(x.shape) == (sum(npc), heads, dim, vdim)][-1]
+    for b in (0, 3):
+        assert torch.equal(starts_of[base[b] + npc[b] - 1], state[slots[b]]), b
+    assert not starts_of[base[4] + npc[4] - 1].any()

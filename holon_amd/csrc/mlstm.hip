@@ -280,7 +280,8 @@ __global__ void __launch_bounds__(512) mlstm_chunk_kernel(const T* __restrict__ 
   constexpr int PER = C * KD / THREADS, TPT = THREADS / C;                  // staged values a thread; threads a token
   __shared__ __attribute__((aligned(16))) float qs[OUT ? C * QS : 4], ks[C * QS];
   __shared__ __attribute__((aligned(16))) float score[OUT ? C * MS : 4], fade[OUT ? C * MS : 4];
-  __shared__ float n_s[KD], keep_s[C], take_s[C], low_s[C], p_s[C], e_s[C];
+  __shared__ __attribute__((aligned(16))) float p_s[C], e_s[C];      // (read 16 bytes at a time, as those above)
+  __shared__ float n_s[KD], keep_s[C], take_s[C], low_s[C];
   const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
   const int g4 = lane / 16, c = lane % 16;
   const int piece = blockIdx.z / col_blocks, col0 = (blockIdx.z % col_blocks) * 128;

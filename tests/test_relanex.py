@@ -653,3 +653,33 @@ def test_the_matrix_memory_in_pieces_keeps_what_is_not_finite_from_earlier_token
             want, _ = run(kernel_op("mlstm_scan").plain, proj)
             assert torch.equal(torch.isfinite(out[at:, 0]).any(), torch.isfinite(want[at:, 0]).any()), (at, value)
             assert torch.equal(out[:, 1], ref[:, 1]), (at, value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,d,v", [(1, 128, 128), (2, 64, 144), (1, 200, 260), (3, 16, 127), (2, 33, 300)])
+def test_the_matrix_memory_in_pieces_at_its_edges(heads, d, v, dtype):
+    """`mlstm_scan` with rows in pieces against its plain form: values wider than one block's 128 columns, rows that end at and one
+    behind the borders of a piece and of a chunk of 64 or 32 tokens, carried and not, beside a row of one token."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.registry import kernel_op
+    k, dev, piece = load_hip(), torch.device("cuda"), 128
+    gen = torch.Generator().manual_seed(d + v)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)             # noqa: E731
+    counts = [256, 257, 321, 385, 1, 129]
+    t, npc = sum(counts), [-(-n // piece) for n in counts]
+    hd, hv, copies = heads * d, heads * v, -(-(v + 1) // 8)
+    proj, gb = rn(t, -(-(2 * hd + 2 * hv + 2 * heads) // 16) * 16), rn(2 * heads)
+    proj[:, 2 * hd + 2 * hv:] *= 3
+    proj = proj.to(dtype)
+    state = [rn(8, heads, d, v + 1), rn(8, heads, 1).expand(8, heads, copies).contiguous()]
+    rows = (i32([3, 0, 7, 1, 4, 2]), i32([0, 9, 5, 0, 77, 6]), i32([sum(counts[:b]) for b in range(7)]), 6, heads, d, v)
+    one, two = [x.clone() for x in state], [x.clone() for x in state]
+    args = (proj, 0, hd, 2 * hd, 2 * hd + 2 * hv, gb, 12.0)
+    got, den = k.mlstm_scan(*args, *one, *rows, (piece, max(npc), i32([sum(npc[:b]) for b in range(6)]), sum(npc)))
+    want, ref = kernel_op("mlstm_scan").plain(*args, *two, *rows)
+    # numerators and denominators apart, each within the rounding of a running maximum of some 10 (2^-24 * 10, and as much for the
+    # gates' sums): their ratio is as far off as a denominator is near 0
+    assert _rel(got, want) < 1e-5 and _rel(den, ref) < 1e-5 and all(_rel(a, b) < 1e-5 for a, b in zip(one, two))

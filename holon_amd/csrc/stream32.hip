@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(256) stream_norm_kernel(float* __restrict__ x3
   }
 }
 
-// The same with four neighbouring values a thread and step (dim a multiple of 4, operands on 16-byte borders), the row in
+// The same with four neighbouring values a thread and step (dim a multiple of 4, operands on borders of four values), the row in
 // registers and every load, the weight's too, under way before the row's sums are taken: a step of few rows waits for memory
 // once. Over a prompt of 2,048 rows and decode steps of a few, rows of 2,048: 4.9 us a call on average where
 // one value at a time, with the weight read behind the sums, took 9.0.
@@ -209,10 +209,13 @@ extern "C" int holon_stream_norm(float* x32, const void* d1, float s1, int dt1, 
   HOLON_CHECK(rows <= 0x7fffffff, "stream_norm: %lld rows exceed one launch", (long long)rows);
   if (rows == 0 || (!d1 && !d2 && !weight)) return 0;
   if (!d1 && d2) { d1 = d2; s1 = s2; dt1 = dt2; d2 = nullptr; }
-  const auto on16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
-  if (dim % 4 == 0 && dim <= 8192 && (!d2 || dt2 == dt1) && on16(x32) && on16(d1) && on16(d2) && on16(weight) && on16(y)) {
-    hipStream_t s = (hipStream_t)stream;                     // (a sum's order is the width's alone here too)
-    const bool df = d1 && dt1 == HOLON_F32;
+  const bool df = d1 && dt1 == HOLON_F32, tf = dt_out == HOLON_F32;
+  // (on the borders of a thread's four values, which every row of a tensor that starts on one lies on: a sum's order is then the
+  // width's alone, whichever rows a call is given)
+  const auto on = [](const void* p, bool f32) { return (uintptr_t)p % (f32 ? 16 : 8) == 0; };
+  if (dim % 4 == 0 && dim <= 8192 && (!d2 || dt2 == dt1) && on(x32, true) && on(d1, df) && on(d2, df) && on(weight, tf) &&
+      on(y, tf)) {
+    hipStream_t s = (hipStream_t)stream;
     if (dt_out == HOLON_F32) {
       if (df) launch_norm_vec<float, float>(x32, d1, s1, d2, s2, weight, y, rows, dim, eps, s);
       else launch_norm_vec<bf16_t, float>(x32, d1, s1, d2, s2, weight, y, rows, dim, eps, s);

@@ -1194,3 +1194,18 @@ def test_general_attention_with_more_heads_than_a_grid_has_rows(hip):
         pages, q = _randn(1, 2, kv, page * d, dtype=torch.float32, seed=97), _randn(1, heads, d, dtype=torch.float32, seed=98)
         args = (torch.zeros(1, 1, dtype=torch.int32, device="cuda"), rows, page, 0.5, 0)
         assert H.rel_rms(hip.paged_attention(q, pages, *args), TorchKernels().paged_attention(q, pages, *args)) < 1e-5
+
+
+@pytest.mark.parametrize("dim", (1028, 2052, 4100))
+def test_stream_norm_of_rows_within_a_tensor(hip, dim):
+    """Rows of bfloat16 whose width is a multiple of 4 and not of 8 (every other one starts on no 16-byte border): each row comes out
+    bit for bit the same whichever row a call starts from."""
+    bf = torch.bfloat16
+    x, weight = _randn(6, dim, dtype=torch.float32, seed=99), 1 + 0.2 * _randn(dim, dtype=bf, seed=100)
+    terms = [(_randn(6, dim, dtype=bf, seed=101 + i), 0.5 + i) for i in range(2)]
+    whole = x.clone()
+    want = hip.stream_norm(whole, terms, weight, 1e-5, bf)
+    for at in range(1, 6):
+        part = x[at:].clone()
+        got = hip.stream_norm(part, [(term[at:], factor) for term, factor in terms], weight, 1e-5, bf)
+        assert torch.equal(got, want[at:]) and torch.equal(part, whole[at:]), at

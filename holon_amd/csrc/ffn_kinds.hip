@@ -203,8 +203,8 @@ __global__ void __launch_bounds__(1024) moe_router_few_kernel(
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int64_t t = blockIdx.x;
   const T* row = x + t * width;
-  const bool wide = width % 4 == 0 && (uintptr_t)router % 16 == 0 && (uintptr_t)x % (4 * sizeof(T)) == 0;
-  struct alignas(4 * sizeof(T)) Four { T v[4]; };
+  const bool wide = width % 4 == 0 && (uintptr_t)router % 16 == 0;      // (wherever x lies: the order of a sum may not follow it)
+  struct Four { T v[4]; };                                  // (aligned as T is; one load all the same)
   for (int e = wave; e < rows_r; e += 16) {
     const float* w = router + (int64_t)e * width;
     float acc[PARTS];
@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(256) moe_router_top_kernel(const T* __restrict
   const int64_t t = blockIdx.x;
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const T* row = x + t * width;
-  const bool wide = width % 4 == 0 && (uintptr_t)router % 16 == 0 && (uintptr_t)x % 16 == 0;
+  const bool wide = width % 4 == 0 && (uintptr_t)router % 16 == 0;
   for (int e0 = 0; e0 < rows_r; e0 += 16) {
     float acc[16];
 #pragma unroll

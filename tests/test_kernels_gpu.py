@@ -1209,3 +1209,20 @@ def test_stream_norm_of_rows_within_a_tensor(hip, dim):
         part = x[at:].clone()
         got = hip.stream_norm(part, [(term[at:], factor) for term, factor in terms], weight, 1e-5, bf)
         assert torch.equal(got, want[at:]) and torch.equal(part, whole[at:]), at
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_routers_wherever_their_rows_lie(hip, dtype):
+    """Rows that start on no border of 16 bytes or of four values: a token's weights are bit for bit the same in every kernel (up to 256
+    rows and more) and wherever its row lies."""
+    for width, off in ((1028, 0), (1028, 1), (2052, 2), (1026, 1), (2050, 3)):
+        rows, experts, top = 300, 24, 3
+        x = torch.empty(rows * width + off, dtype=dtype, device="cuda")[off:].view(rows, width)
+        x.copy_(_randn(rows, width, dtype=dtype, seed=110))
+        router = _randn(experts + 1, width, dtype=torch.float32, seed=111, scale=width ** -0.5)
+        bias = _randn(experts, dtype=torch.float32, seed=112, scale=0.2)
+        for op, args, how in ((hip.moe_router, (router[:experts], bias, top, 1, 1, 1.7), {}),
+                              (hip.moe_router_top, (router, bias, experts, top, 1, 1), dict(score="softmax"))):
+            want = op(x.clone(), *args, **how)
+            for first, count in ((0, 300), (1, 299), (1, 256), (7, 257), (3, 1)):
+                assert torch.equal(op(x[first: first + count], *args, **how), want[first: first + count]), (width, off, first, count)

@@ -294,6 +294,10 @@ static void launch_skinny(const void* x, const void* w, void* y, int M, int N, i
 //   up to 319 tiles: one, two sets of 4 loads. 2048 x 8192 9.7 / 11.4 / 14.5 (11.6 / 12.4 / 15.3), 4096 x 4096 7.8 / 8.3 / 9.3
 //     (8.3 / 8.5 / 10.0). Where the residual is added, 8 loads in one set: behind the kernels of a step of four rows, which leave
 //     4096 x 4096 and 4096 x 12288 cold, two sets took 13.9 on average and one 13.4.
+//     (8 waves where K is no multiple of 512: two sets of 4 up to 256 tiles, 4096 x 11008 17.5 / 19.2 / 22.6 (18.9 / 21.2 / 23.4;
+//     two tiles, half the units without a block, 22.7 / 25.5 / 29.1), 2816 x 2816 6.3 / 6.8 / 7.8 (6.8 / 7.4 / 8.0; 9.0 / 9.7 / 9.6);
+//     from there one set of 4, 5104 x 3328 10.1 / 11.3 / 13.5 (11.4 / 12.0 / 14.8; two sets 10.7 / 11.9 / 14.7), and above 8 rows
+//     two tiles, 4608 x 2816 at 16 rows 10.0 (12.6; one tile 12.3).)
 //   320 to 511: two (at 512, one: 8192 x 4096 13.8 / 15.1 / 16.0, two 15.0 / 16.1 / 16.0); two sets of 4 loads a tile up to 8 rows,
 //     of 2 above: 6144 x 4096 11.5 / 12.8 / 12.7 (12.0 / 12.9 / 14.3), 6144 x 5120 13.3 / 14.8 / 15.4 (16.8 / 17.8 / 19.1).
 //   from 1,024, and K below 4,096 or more than 8 rows: two, two sets of 2 loads a tile: 18432 x 2048 15.5 / 16.0 / 17.7 (15.6 /
@@ -301,12 +305,17 @@ static void launch_skinny(const void* x, const void* w, void* y, int M, int N, i
 //   otherwise one, 4 loads in one set, which is what 8 waves a block and several blocks a unit need least registers for: 12288 x
 //     4096 19.4 / 20.0 / 23.3 (19.5 / 20.6 / 25.3; two tiles 22.8 / 23.6 / 24.7), 9216 x 2048 9.5 / 10.1 / 11.5 (9.7 / 10.7 /
 //     12.6), 151936 x 4096 182 / 190 (184 / 199; two tiles, for 16 rows, 206, where one takes 243 and took 225).
+static bool skinny_two(int tiles, int K, int M) {
+  return skinny_waves(tiles, K) == 8 && tiles % 2 == 0 &&
+         ((tiles >= (M > 8 ? 257 : 320) && tiles < 512) || (tiles >= 1024 && (K < 4096 || M > 8)));
+}
+
 template <typename OutT, bool RESID = false>
 static int pick_waves(const void* x, const void* w, void* y, int M, int N, int K, bool tiled, hipStream_t s,
                       int round_first = 0, RowScale rs = RowScale{nullptr, 0, 0.f, 0.f}, float* stats_out = nullptr) {
   const int tiles = N / 16;
   const int wpb = skinny_waves(tiles, K);
-  const bool two = tiles % 2 == 0 && (tiles < 512 || (tiles >= 1024 && (K < 4096 || M > 8)));
+  const bool two = skinny_two(tiles, K, M);
 #define SKINNY(NT, WPB, U, TWICE) \
   launch_skinny<NT, WPB, U, TWICE, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out)
   switch (wpb) {
@@ -314,7 +323,8 @@ static int pick_waves(const void* x, const void* w, void* y, int M, int N, int K
       if constexpr (RESID) { SKINNY(1, 16, 8, false); } else { SKINNY(1, 16, 4, true); }
       break;
     case 8:
-      if (!two) SKINNY(1, 8, 4, false);
+      if (tiles <= 256) SKINNY(1, 8, 4, true);
+      else if (!two) SKINNY(1, 8, 4, false);
       else if (tiles < 512 && M <= 8) SKINNY(2, 8, 4, true);
       else SKINNY(2, 8, 2, true);
       break;
@@ -325,6 +335,9 @@ static int pick_waves(const void* x, const void* w, void* y, int M, int N, int K
 #undef SKINNY
   return 0;
 }
+
+// How many tiles of 16 columns a block owns.
+extern "C" int holon_gemm_skinny_tiles(int M, int N, int K) { return skinny_two(N / 16, K, M) ? 2 : 1; }
 
 extern "C" int holon_gemm_skinny_supported(int M, int N, int K) {
   return M >= 1 && M <= 16 && N % 16 == 0 && K % 32 == 0 && K >= 32;

@@ -135,6 +135,7 @@ int holon_attention_decode_bf16_static(const void* q, void* out, const void* pag
 // out, 2 float32 out of values rounded to bfloat16 first, 4 bfloat16 out of max(rounded product, 0)^2;
 // tiled says that `w` is holon_tile_weight_bf16's copy ([N/16, K/32, 64, 8]: lane-major 16-byte pieces).
 int holon_gemm_skinny_supported(int M, int N, int K);
+int holon_gemm_skinny_tiles(int M, int N, int K);   // tiles of 16 columns a block owns
 int holon_gemm_skinny_bf16(const void* x, const void* w, void* y, int M, int N, int K, int out_f32, int tiled,
                            void* stream);
 // residual[M, N] = round(residual + round(x w^T)) in place, tiled weights: the product and the residual add that

@@ -1226,3 +1226,19 @@ def test_routers_wherever_their_rows_lie(hip, dtype):
             want = op(x.clone(), *args, **how)
             for first, count in ((0, 300), (1, 299), (1, 256), (7, 257), (3, 1)):
                 assert torch.equal(op(x[first: first + count], *args, **how), want[first: first + count]), (width, off, first, count)
+
+
+def test_few_row_products_with_few_tiles_take_one_a_block(hip):
+    """A block owns one tile of 16 columns where there are at most 256, also where K is no multiple of 512 and eight waves share a
+    tile (two would leave half the compute units without a block); the results across those sizes against float64."""
+    for n, k in ((4096, 11008), (2816, 2816), (1024, 768), (4096, 2304)):
+        assert [hip.lib.holon_gemm_skinny_tiles(m, n, k) for m in (1, 8, 16)] == [1, 1, 1], (n, k)
+    assert [hip.lib.holon_gemm_skinny_tiles(m, 6144, 4096) for m in (1, 8, 16)] == [2, 2, 2]
+    assert [hip.lib.holon_gemm_skinny_tiles(m, 8192, 4096) for m in (1, 8, 16)] == [1, 1, 1]
+    for n, k in ((4096, 2816), (4112, 768), (5088, 1280), (5104, 1280), (5120, 1280)):
+        x, w = _randn(16, k, dtype=torch.bfloat16, seed=120), _randn(n, k, dtype=torch.bfloat16, seed=121)
+        tiled, want = hip.tile_weight(w), x.double() @ w.double().T
+        for m in (1, 9, 16):
+            got = hip.linear(x[:m].contiguous(), w, tiled=tiled)
+            assert H.op_budget_usage(got, want[:m], torch.bfloat16, k) <= 1, (m, n, k)
+            assert torch.equal(got, hip.linear(x, w, tiled=tiled)[:m]), (m, n, k)

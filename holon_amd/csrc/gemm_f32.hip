@@ -1,7 +1,7 @@
 // y[M, N] = x[M, K] w[N, K]^T in true float32: float32 operands on the matrix cores (v_mfma_f32_16x16x4_f32: no
 // reduced-precision mode), float32 accumulation. This is the product of the 32-bit path.
 //
-// Its point is a fixed order of summation, the same in both kernels of shares below: K is cut into 16 shares of equal length
+// Its point is a fixed order of summation, the same in all forms of shares below: K is cut into 16 shares of equal length
 // (64, or a larger multiple of 32; the last ones shorter or empty); a share's sum runs over its k in groups of 16 (the instruction adds
 // k, k + 4, k + 8 and k + 12 of a group at a time), four shares are added up one after the other, and so are the four
 // quarters that makes. None of it depends on M, on where the row lies in the batch, or on the tile of the output the
@@ -122,19 +122,22 @@ __global__ void __launch_bounds__(SHARES * WAVE) gemm_f32_rows_kernel(const floa
   store4(y, sum, m0 + wave / NT * 16 + c, n0 + wave % NT * 16 + 4 * g, M, N);
 }
 
-// More rows: bound by the matrix cores. A block owns 64 x 64 results with four waves (32 x 32 each) for every quarter of
-// K, which stage their quarter's rows of x and w in LDS, CHUNK of k at a time, into one of two buffers while the other is
-// multiplied; pieces of 16 bytes lie at place p ^ (row % 8) of their row. Splitting K inside the block is what fills the
-// chip where an output of some hundred rows has few tiles, and four waves a SIMD cover each other's barriers.
-template <bool VEC>
-__global__ void __launch_bounds__(1024) gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                        float* __restrict__ y, int M, int N, int K) {
-  __shared__ __attribute__((aligned(16))) float stage[QUARTERS][2][2][64 * CHUNK];   // quarter, buffer, x or w
-  const int quarter = threadIdx.x / 256, tid = threadIdx.x % 256;
+// More rows: bound by the matrix cores. A block owns 64 x 64 results; four waves (32 x 32 each) walk a run of K whose rows of x and
+// w they stage in LDS, CHUNK of k at a time, into one of two buffers while the other is multiplied; pieces of 16 bytes lie at
+// place p ^ (row % 8) of their row. SIDE 4: sixteen waves, the four quarters of K side by side: what fills the chip where an output of
+// some hundred rows has few tiles, four waves a SIMD covering each other's barriers. SIDE 1: four waves, the quarters one after the
+// other: several blocks share a unit, so that one's first loads and its stores lie under the others' products; that is the better
+// one where there are tiles for it, the more the shorter K. Either ends at K (what lies behind it would add zeros).
+template <int SIDE, bool VEC>
+__global__ void __launch_bounds__(SIDE * 256) gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                              float* __restrict__ y, int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) float stage[SIDE][2][2][64 * CHUNK];       // quarter, buffer, x or w
+  const int quarter = SIDE > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 256) : 0, tid = threadIdx.x % 256;
   const int wave = tid / WAVE, lane = tid % WAVE;
   const int g = lane / 16, c = lane % 16;
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int share = share_length(K), first = quarter * 4 * share, chunks = 4 * share / CHUNK, per_share = share / CHUNK;
+  const int share = share_length(K), first = quarter * 4 * share, per_share = share / CHUNK;
+  const int chunks = (min(K, (SIDE > 1 ? 4 : 16) * share) + CHUNK - 1) / CHUNK;      // (of the block: the first quarter's)
   // what this thread stages: rows tid / 8 and 32 more, piece tid % 8
   const int r0 = tid / 8, p0 = tid % 8;
   const float *xr[2], *wr[2];
@@ -162,61 +165,83 @@ __global__ void __launch_bounds__(1024) gemm_f32_kernel(const float* __restrict_
   // where this lane reads: row 32 (half) + 16 t + c, pieces g and 4 + g
   const int xrow = wave / 2 * 32 + c, wrow = wave % 2 * 32 + c;
   const int at[2] = {4 * (g ^ (c % 8)), 4 * ((4 + g) ^ (c % 8))};
-  f32x4_t acc[2][2], total[2][2];
+  // the sums of a share, of a quarter's shares so far (SIDE 1), and of all that is behind them
+  f32x4_t acc[2][2], part[SIDE > 1 ? 1 : 2][2], total[2][2];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int u = 0; u < 2; ++u) acc[t][u] = total[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  int left = per_share, shares = 0;
+  const auto end_share = [&]() {
+    const bool begins = SIDE > 1 ? shares == 0 : shares % 4 == 0, ends = shares % 4 == 3, first_quarter = shares < 4;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if constexpr (SIDE > 1) {
+          total[t][u] = begins ? acc[t][u] : total[t][u] + acc[t][u];
+        } else {
+          part[t][u] = begins ? acc[t][u] : part[t][u] + acc[t][u];
+          if (ends) total[t][u] = first_quarter ? part[t][u] : total[t][u] + part[t][u];
+        }
+        acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    left = per_share;
+    ++shares;
+  };
   fetch(0);
   keep(0);
   if (chunks > 1) fetch(1);
   lds_barrier();
-  int left = per_share;
-  bool begun = false;                                     // whether `total` holds a share
   for (int ch = 0; ch < chunks; ++ch) {
     if (ch + 1 < chunks) keep((ch + 1) & 1);              // (read last in front of the barrier behind us)
     if (ch + 2 < chunks) fetch(ch + 2);
-    const float* xs = stage[quarter][ch & 1][0];
-    const float* ws = stage[quarter][ch & 1][1];
+    if (SIDE == 1 || first + ch * CHUNK < K) {
+      const float* xs = stage[quarter][ch & 1][0];
+      const float* ws = stage[quarter][ch & 1][1];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      f32x4_t b[2], a[2];
+      for (int s = 0; s < 2; ++s) {
+        f32x4_t b[2], a[2];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) b[t] = *reinterpret_cast<const f32x4_t*>(&xs[(xrow + 16 * t) * CHUNK + at[s]]);
+        for (int t = 0; t < 2; ++t) b[t] = *reinterpret_cast<const f32x4_t*>(&xs[(xrow + 16 * t) * CHUNK + at[s]]);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) a[u] = *reinterpret_cast<const f32x4_t*>(&ws[(wrow + 16 * u) * CHUNK + at[s]]);
+        for (int u = 0; u < 2; ++u) a[u] = *reinterpret_cast<const f32x4_t*>(&ws[(wrow + 16 * u) * CHUNK + at[s]]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+          for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int u = 0; u < 2; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[t][i], acc[t][u], 0, 0, 0);
-    }
-    if (--left == 0) {                                    // a share ends
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          total[t][u] = begun ? total[t][u] + acc[t][u] : acc[t][u];
-          acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
-      left = per_share;
-      begun = true;
+            for (int u = 0; u < 2; ++u)
+              acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[t][i], acc[t][u], 0, 0, 0);
+      }
+      if (--left == 0) end_share();
     }
     lds_barrier();                                        // (what was fetched stays under way)
   }
-  // the quarters' sums through LDS: tile (4 t' + u') of the block's 16, one a wave
-  f32x4_t(*part)[16][WAVE] = reinterpret_cast<f32x4_t(*)[16][WAVE]>(&stage[0][0][0][0]);
+  if (left < per_share) end_share();                      // (K ends inside a share)
+  if constexpr (SIDE > 1) {
+    // the quarters' sums through LDS: tile (4 t' + u') of the block's 16, one a wave
+    f32x4_t(*sums)[16][WAVE] = reinterpret_cast<f32x4_t(*)[16][WAVE]>(&stage[0][0][0][0]);
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int u = 0; u < 2; ++u) part[quarter][(wave / 2 * 2 + t) * 4 + wave % 2 * 2 + u][lane] = total[t][u];
-  __syncthreads();
-  const int tile = quarter * 4 + wave;
-  f32x4_t sum = part[0][tile][lane];
+      for (int u = 0; u < 2; ++u) sums[quarter][(wave / 2 * 2 + t) * 4 + wave % 2 * 2 + u][lane] = total[t][u];
+    __syncthreads();
+    const int tile = quarter * 4 + wave;
+    f32x4_t sum = sums[0][tile][lane];
 #pragma unroll
-  for (int q = 1; q < QUARTERS; ++q) sum += part[q][tile][lane];
-  store4(y, sum, m0 + tile / 4 * 16 + c, n0 + tile % 4 * 16 + 4 * g, M, N);
+    for (int q = 1; q < QUARTERS; ++q) sum += sums[q][tile][lane];
+    store4(y, sum, m0 + tile / 4 * 16 + c, n0 + tile % 4 * 16 + 4 * g, M, N);
+  } else {
+    const bool pending = shares % 4 != 0, only = shares < 4;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const f32x4_t sum = pending ? (only ? part[t][u] : total[t][u] + part[t][u]) : total[t][u];
+        store4(y, sum, m0 + (wave / 2 * 2 + t) * 16 + c, n0 + (wave % 2 * 2 + u) * 16 + 4 * g, M, N);
+      }
+  }
 }
 
 // Long sums into many columns: one running sum over k = 0, 1, 2, ... (v_mfma_f32_32x32x2_f32 adds its two k one after the
@@ -291,30 +316,38 @@ __global__ void __launch_bounds__(256) gemm_f32_in_order_kernel(const float* __r
   }
 }
 
-// Which tile a product takes: the one whose rounds of one block a CU are done first. A round's time over K = 2,048 on
-// MI355X, in us (in proportion for other K): 1 x 1 tiles 9.3, 1 x 2 15.5, 2 x 2 20.5, 2 x 4 33.5, and 42 for the staged 4 x 4
-// (0.8 of the float32 peak where the last round is full). So 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10 us; with a
-// 64 x 64 tile a block and no split of K it took 118) and the staged kernel from 300 rows (45 us; 126), 16384 x 2048 1 x 1
-// tiles up to 16 rows (27 to 39 us, 5.0 TB/s at one row; 116 to 120) and the staged one from 48 (46 us at 64 rows; 145).
+// Which form a product takes: the one that is done first by a fit over K = 48 to 4,096, N = 256 to 16,384 and M = 17 to 2,048 on
+// MI355X (203 products, each in all forms): in us, a start and so much for every round of one block a CU, both linear in K. The choice
+// is 1 % from the best form on average and 15 % at most. 2048 x 2048 takes 1 x 1 tiles up to 32 rows (11 us; with a 64 x 64 tile a
+// block and no split of K it took 118), quarters side by side from 300 rows (42 us; 118), one after the other at 2,048 (157 us; 182);
+// 16384 x 2048 1 x 1 tiles up to 16 rows (27 to 39 us, 5.0 TB/s at one row; 116 to 120), quarters side by side from 64 (49 us;
+// 149), one after the other from 150 (126 us; 187); 8192 x 256 at 2,048 rows 87 us (quarters side by side 151, and 325 where they
+// walked through K that is not there; one running sum in blocks of four waves 84), 8192 x 64 33 (67, 327; 30).
 template <bool VEC>
 void launch(const float* x, const float* w, float* y, int M, int N, int K, hipStream_t s) {
-  const auto cost = [&](int mt, int nt, float round) {
-    const int64_t blocks = (int64_t)((M + 16 * mt - 1) / (16 * mt)) * ((N + 16 * nt - 1) / (16 * nt));
-    return (float)((blocks + 255) / 256) * round;
-  };
-  const float few[4] = {cost(1, 1, 9.3f), cost(1, 2, 15.5f), cost(2, 2, 20.5f), cost(2, 4, 33.5f)};
+  struct Form { int mt, nt; float start, start_k, round, round_k; };
+  static constexpr Form FORMS[6] = {{1, 1, 2.9f, 6e-4f, 0.48f, 3.0e-3f}, {1, 2, 2.9f, 4e-4f, 0.65f, 5.0e-3f},
+                                    {2, 2, 3.1f, 7e-4f, 0.93f, 7.2e-3f}, {2, 4, 1.9f, 8e-4f, 3.1f, 1.25e-2f},
+                                    {4, 4, 1.8f, 0.f, 3.2f, 1.96e-2f},   {4, 4, 2.7f, 9.2e-3f, 1.03f, 1.69e-2f}};
   int best = 0;
-  for (int i = 1; i < 4; ++i) if (M > 16 && few[i] < few[best]) best = i;
-#define F32_ROWS(MT, NT, DEPTH)                                                                                     \
-  gemm_f32_rows_kernel<MT, NT, DEPTH, VEC><<<dim3((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT)),    \
-                                             SHARES * WAVE, 0, s>>>(x, w, y, M, N, K)
-  if (M > 16 && (cost(4, 4, 42.f) <= few[best] || (M + 15) / 16 > 65535))
-    gemm_f32_kernel<VEC><<<dim3((N + 63) / 64, (M + 63) / 64), 1024, 0, s>>>(x, w, y, M, N, K);
-  else if (best == 0) F32_ROWS(1, 1, 2);
-  else if (best == 1) F32_ROWS(1, 2, 1);
-  else if (best == 2) F32_ROWS(2, 2, 1);
-  else F32_ROWS(2, 4, 1);
-#undef F32_ROWS
+  float least = INFINITY;
+  for (int i = 0; i < 6; ++i) {
+    const Form& f = FORMS[i];
+    if (i > 0 && M <= 16) break;
+    if (f.mt < 4 && (M + 16 * f.mt - 1) / (16 * f.mt) > 65535) continue;
+    const int64_t blocks = (int64_t)((M + 16 * f.mt - 1) / (16 * f.mt)) * ((N + 16 * f.nt - 1) / (16 * f.nt));
+    const float cost = f.start + f.start_k * K + (float)((blocks + 255) / 256) * (f.round + f.round_k * K);
+    if (cost < least) { least = cost; best = i; }
+  }
+  const dim3 grid((N + 16 * FORMS[best].nt - 1) / (16 * FORMS[best].nt), (M + 16 * FORMS[best].mt - 1) / (16 * FORMS[best].mt));
+  switch (best) {
+    case 0: gemm_f32_rows_kernel<1, 1, 2, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
+    case 1: gemm_f32_rows_kernel<1, 2, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
+    case 2: gemm_f32_rows_kernel<2, 2, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
+    case 3: gemm_f32_rows_kernel<2, 4, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
+    case 4: gemm_f32_kernel<4, VEC><<<grid, 1024, 0, s>>>(x, w, y, M, N, K); break;
+    default: gemm_f32_kernel<1, VEC><<<grid, 256, 0, s>>>(x, w, y, M, N, K); break;
+  }
 }
 }  // namespace
 

@@ -1242,3 +1242,29 @@ def test_few_row_products_with_few_tiles_take_one_a_block(hip):
             got = hip.linear(x[:m].contiguous(), w, tiled=tiled)
             assert H.op_budget_usage(got, want[:m], torch.bfloat16, k) <= 1, (m, n, k)
             assert torch.equal(got, hip.linear(x, w, tiled=tiled)[:m]), (m, n, k)
+
+
+def test_float32_product_of_short_sums(hip):
+    """Rows many enough for 64 x 64 tiles over short K, quarters of K side by side and one after the other: at K's borders against the
+    float64 product, each row bit for bit what it is alone; and the time follows K (a block does not walk what is not there)."""
+    for k in (1, 31, 32, 33, 64, 65, 100, 128, 255, 256, 257, 320, 512, 700, 768, 1000, 1024, 1056):
+        for m, n in ((65, 1100), (300, 1024), (830, 4160)):
+            x, w = _randn(m, k, dtype=torch.float32, seed=130), _randn(n, k, dtype=torch.float32, seed=131)
+            got, want = hip.linear(x, w), x.double() @ w.double().T
+            bound = (max(64, -(-k // 512) * 32) + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+            assert ((got.double() - want).abs() <= bound).all(), (m, k, n)
+            for row in (0, m - 1):
+                assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), (m, k, n, row)
+
+    def us(k):
+        x, w, took = _randn(2048, k, dtype=torch.float32), _randn(8192, k, dtype=torch.float32), []
+        for _ in range(8):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            for _ in range(4):
+                hip.linear(x, w)
+            end.record()
+            end.synchronize()
+            took.append(begin.elapsed_time(end) * 250)
+        return min(took)
+    assert us(64) < 0.4 * us(1024)

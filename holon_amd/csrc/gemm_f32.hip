@@ -248,7 +248,9 @@ __global__ void __launch_bounds__(SIDE * 256) gemm_f32_kernel(const float* __res
 // other), the order of a plain float32 product. What the 32-bit path of a model of these sizes is held against is the same model
 // in plain float32 products, and the rounding of those alone, most of it the query and key projection's (6,144 columns over K =
 // 4,096), is 2.1e-5 of the logits' rms at 36 layers: sums in shares come 3 times closer to 64 bits (8e-6) and lie 2.1e-5 from
-// the plain model where 2e-5 are allowed; these lie 1.9e-5 from it.
+// the plain model where 2e-5 are allowed; these lie 1.9e-5 from it. (A product that is exact would lie 2.1e-5 from it too.) The order
+// costs time, most with few rows, as nothing shares K: 6144 x 4096 takes 223 / 273 / 285 / 433 us at 1 / 64 / 300 / 704 rows, in
+// shares 27 / 67 / 158 / 387.
 // A workgroup of four waves owns a 64 x 64 tile of the output, each wave a 32 x 32 quarter. Per step the workgroup stages 64
 // rows of x and 64 rows of w, 32 k wide, in LDS (rows padded to 33 floats: a wave's 32 rows then fall in 32 different banks).
 constexpr int TM = 64, TN = 64, TK = 32, PAD = 1;
@@ -316,19 +318,20 @@ __global__ void __launch_bounds__(256) gemm_f32_in_order_kernel(const float* __r
   }
 }
 
-// Which form a product takes: the one that is done first by a fit over K = 48 to 4,096, N = 256 to 16,384 and M = 17 to 2,048 on
-// MI355X (203 products, each in all forms): in us, a start and so much for every round of one block a CU, both linear in K. The choice
-// is 1 % from the best form on average and 15 % at most. 2048 x 2048 takes 1 x 1 tiles up to 32 rows (11 us; with a 64 x 64 tile a
-// block and no split of K it took 118), quarters side by side from 300 rows (42 us; 118), one after the other at 2,048 (157 us; 182);
-// 16384 x 2048 1 x 1 tiles up to 16 rows (27 to 39 us, 5.0 TB/s at one row; 116 to 120), quarters side by side from 64 (49 us;
-// 149), one after the other from 150 (126 us; 187); 8192 x 256 at 2,048 rows 87 us (quarters side by side 151, and 325 where they
-// walked through K that is not there; one running sum in blocks of four waves 84), 8192 x 64 33 (67, 327; 30).
-template <bool VEC>
-void launch(const float* x, const float* w, float* y, int M, int N, int K, hipStream_t s) {
-  struct Form { int mt, nt; float start, start_k, round, round_k; };
-  static constexpr Form FORMS[6] = {{1, 1, 2.9f, 6e-4f, 0.48f, 3.0e-3f}, {1, 2, 2.9f, 4e-4f, 0.65f, 5.0e-3f},
-                                    {2, 2, 3.1f, 7e-4f, 0.93f, 7.2e-3f}, {2, 4, 1.9f, 8e-4f, 3.1f, 1.25e-2f},
-                                    {4, 4, 1.8f, 0.f, 3.2f, 1.96e-2f},   {4, 4, 2.7f, 9.2e-3f, 1.03f, 1.69e-2f}};
+// Which form a product takes: the one that is done first by a fit over K = 48 to 18,432, N = 64 to 16,384 and M = 17 to 2,048 on
+// MI355X (1,149 products, each in all forms, weights from memory): in us, a start and so much for every round of one block a CU, both
+// linear in K. Where the best form takes more than 15 us the choice is 0.1 % from it on average and 6 % at most. In us, best and others:
+// 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10; with a 64 x 64 tile a block and no split of K it took 118), quarters side by side
+// from 300 rows (42; one after the other 54, 2 x 2 tiles 50), one after the other at 2,048 (157; 163); 2048 x 9248 and 2048 x 18432 at
+// 704 rows quarters side by side (345 and 672; 2 x 4 tiles, which a fit up to K = 4,096 took there, 396 and 767); 16384 x 2048 1 x 1
+// tiles up to 16 rows (5.0 TB/s at one row), quarters side by side from 64 (46; 58), one after the other from 150 (125; 130); 9248 x 256
+// at 2,048 rows one after the other (103; side by side 180).
+struct Form { int mt, nt; float start, start_k, round, round_k; };
+constexpr Form FORMS[6] = {{1, 1, 2.6f, 2e-4f, 0.43f, 3.25e-3f}, {1, 2, 2.5f, 2e-4f, 0.63f, 5.0e-3f},
+                           {2, 2, 2.5f, 7e-4f, 0.90f, 7.35e-3f}, {2, 4, 1.2f, 5e-4f, 3.0f, 1.31e-2f},
+                           {4, 4, 1.2f, 0.f, 3.2f, 1.86e-2f},    {4, 4, 2.1f, 8.0e-3f, 1.1f, 1.66e-2f}};
+
+int pick_form(int M, int N, int K) {
   int best = 0;
   float least = INFINITY;
   for (int i = 0; i < 6; ++i) {
@@ -339,6 +342,12 @@ void launch(const float* x, const float* w, float* y, int M, int N, int K, hipSt
     const float cost = f.start + f.start_k * K + (float)((blocks + 255) / 256) * (f.round + f.round_k * K);
     if (cost < least) { least = cost; best = i; }
   }
+  return best;
+}
+
+template <bool VEC>
+void launch(const float* x, const float* w, float* y, int M, int N, int K, hipStream_t s) {
+  const int best = pick_form(M, N, K);
   const dim3 grid((N + 16 * FORMS[best].nt - 1) / (16 * FORMS[best].nt), (M + 16 * FORMS[best].mt - 1) / (16 * FORMS[best].mt));
   switch (best) {
     case 0: gemm_f32_rows_kernel<1, 1, 2, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
@@ -350,6 +359,10 @@ void launch(const float* x, const float* w, float* y, int M, int N, int K, hipSt
   }
 }
 }  // namespace
+
+// Which form serves M rows: 0 to 3 tiles of 1 x 1, 1 x 2, 2 x 2 and 2 x 4 a block, 4 quarters of K side by side, 5 one after the
+// other; -1 one running sum.
+extern "C" int holon_gemm_f32_form(int M, int N, int K) { return sums_in_order(N, K) ? -1 : pick_form(M, N, K); }
 
 extern "C" int holon_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, void* stream) {
   HOLON_CHECK(M >= 0 && N > 0 && K > 0, "gemm (float32): M=%d N=%d K=%d", M, N, K);

@@ -177,9 +177,10 @@ int holon_gemm_tiles_parts_supported(int M, int N, int K, int splits);
 int holon_gemm_tiles_parts_bf16(const void* x, const void* w_tiled, void* parts, int M, int N, int K, int splits,
                                 void* stream);
 int holon_sum_parts(const void* parts, void* y, int splits, int64_t count, void* stream);
-// y[M, N] = x[M, K] w[N, K]^T, all float32, true 32-bit products and sums in an order that depends on K alone: a row's
-// result is bit for bit the same whatever other rows are in the call.
+// y[M, N] = x[M, K] w[N, K]^T, all float32, true 32-bit products and sums in an order that depends on K and N
+// alone: a row's result is bit for bit the same whatever other rows are in the call.
 int holon_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, void* stream);
+int holon_gemm_f32_form(int M, int N, int K);       // which form serves M rows (see gemm_f32.hip)
 // scale (nullable, [K] bfloat16): tiled holds round(w[n][k] * scale[k]).
 int holon_tile_weight_bf16(const void* w, void* tiled, int N, int K, const void* scale, void* stream);
 // `pieces`: room for rows x holon_argmax_pieces(vocab) pairs (float32, int32) when that is not 0 (a wide row is then

@@ -1268,3 +1268,20 @@ def test_float32_product_of_short_sums(hip):
             took.append(begin.elapsed_time(end) * 250)
         return min(took)
     assert us(64) < 0.4 * us(1024)
+
+
+def test_float32_product_of_long_sums_takes_the_form_that_is_done_first(hip):
+    """Some hundred rows over K beyond 4,096 take 64 x 64 tiles with the quarters of K side by side (tiles of 32 x 64 straight from
+    memory take 15 % longer), few rows narrow tiles, wide weights one running sum; against the float64 product, each row bit for bit
+    what it is alone."""
+    form = hip.lib.holon_gemm_f32_form
+    assert [form(m, 2048, 18432) for m in (1, 17, 704)] == [0, 0, 4]
+    assert [form(704, 2048, 9248), form(500, 3072, 12288), form(300, 4096, 18432), form(2048, 2048, 2048)] == [4, 4, 4, 5]
+    assert [form(m, n, k) for m, n, k in ((1, 6144, 4096), (704, 4097, 4096), (704, 4096, 4096))] == [-1, -1, 4]
+    for m, n, k in ((130, 2048, 4608), (400, 2048, 5120), (300, 1056, 9248), (67, 4096, 6150)):
+        x, w = _randn(m, k, dtype=torch.float32, seed=140), _randn(n, k, dtype=torch.float32, seed=141)
+        got, want = hip.linear(x, w), x.double() @ w.double().T
+        bound = (-(-k // 512) * 32 + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        assert ((got.double() - want).abs() <= bound).all(), (m, n, k)
+        for row in (0, 64, m - 1):
+            assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), (m, n, k, row)

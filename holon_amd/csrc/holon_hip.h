@@ -36,11 +36,12 @@ int holon_qk_norm_rope_write(const void* qkv, int64_t qkv_stride, void* q_out, i
                              int dtype, void* stream);
 int holon_kv_write(const void* k, const void* v, void* pages, const int32_t* write_page, const int32_t* write_off,
                    int tokens, int kv_heads, int head_dim, int page_size, int num_pages, int dtype, void* stream);
-// Attention of every query token over its row's cached keys (any dtype, page size and head_dim % 8 == 0).
+// Attention of every query token over its row's cached keys (any dtype, page size and head_dim % 8 == 0). `most`: the longest of
+// the rows' lengths or more (0: not known), which launch shapes follow and results do not.
 int holon_attention_generic(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
                             const int32_t* slots, const int32_t* lens, const int32_t* query_start, int rows,
                             int tokens, int heads, int kv_heads, int head_dim, int page_size, int num_pages,
-                            float scale, int window, int dtype, void* stream);
+                            float scale, int window, int most, int dtype, void* stream);
 // Matrix-core attention (bfloat16, head_dim 64/128/256, page_size % 16 == 0). `row_ids` lists the rows served.
 int holon_attention_mfma_supported(int head_dim, int page_size, int dtype);
 int holon_attention_prefill_bf16(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,

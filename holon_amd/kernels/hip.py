@@ -81,7 +81,7 @@ class HipKernels:
             "holon_qk_norm_rope_write": [_P, _L, _P, _I, _I, _I, _I, _P, _P, _F, _P, _I, _I, _P, _P, _P, _P, _I, _I,
                                          _I, _P],
             "holon_kv_write": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
-            "holon_attention_generic": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _P],
+            "holon_attention_generic": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P],
             "holon_attention_mfma_supported": [_I, _I, _I],
             "holon_attention_prefill_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
                                              _P],
@@ -411,7 +411,7 @@ class HipKernels:
         if x.dtype == torch.bfloat16 and x.is_contiguous() and self.serves_rows(m, weight, tiled):
             return self._rows_product(x, weight, tiled, False, out_dtype == torch.float32)
         if x.dtype == torch.float32 and weight.dtype == torch.float32 and out_dtype in (None, torch.float32):
-            # the 32-bit path's own product: true float32, every sum in an order that K alone decides
+            # the 32-bit path's own product: true float32, every sum in an order that K and N alone decide
             self._check(x, "linear x")
             self._check(weight, "linear weight")
             y = torch.empty((m, n), dtype=torch.float32, device=x.device)
@@ -729,8 +729,8 @@ class HipKernels:
                               f"not at head_dim {d}, page {page_size}, {q.dtype}")
         self._call(self.lib.holon_attention_generic, q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(),
                    table.shape[1], rows.slots.data_ptr(), rows.lens.data_ptr(), rows.query_start.data_ptr(), b, t, hq,
-                   hkv, d, page_size, pages.shape[0], float(scale), int(window), self._dt(q, "attention"),
-                   self._stream())
+                   hkv, d, page_size, pages.shape[0], float(scale), int(window),
+                   max(rows.max_decode_len, rows.max_chunk_len), self._dt(q, "attention"), self._stream())
         return out
 
     def _shared_attention(self, q, pages, table, rows, page_size, scale, window, sink, softcap, dist, keep_first, share,

@@ -1285,3 +1285,29 @@ def test_float32_product_of_long_sums_takes_the_form_that_is_done_first(hip):
         assert ((got.double() - want).abs() <= bound).all(), (m, n, k)
         for row in (0, 64, m - 1):
             assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), (m, n, k, row)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,kv,d", [(6, 2, 48), (8, 8, 24), (4, 1, 272), (4, 2, 80)])
+def test_general_attention_of_short_rows(hip, dtype, heads, kv, d):
+    """A block has as many waves as the longest row has tiles of 64 keys, eight at most: rows around the borders at which that
+    changes come out bit for bit as with eight waves (a bound that says nothing), within a window of either kind too, and a bound that
+    is too short still leaves no key out."""
+    page, i32 = 16, lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")            # noqa: E731
+    for n, window in ((1, 0), (63, 0), (64, 0), (65, 0), (128, 0), (129, 0), (256, 0), (257, 0), (300, 64), (300, 65), (300, -64), (300, -130)):
+        count = -(-300 // n)                    # more blocks than compute units, whatever the heads share
+        lens, starts = [n] * count, [n * b for b in range(count + 1)]
+        most = -(-n // page)
+        pages = _randn(most * count, 2, kv, page * d, dtype=dtype, seed=150)
+        table = torch.arange(most * count, dtype=torch.int32, device="cuda").view(count, most)
+        q = _randn(n * count, heads, d, dtype=dtype, seed=151)
+
+        def rows(bound):
+            return AttnRows(slots=i32(list(range(count))), lens=i32(lens), query_start=i32(starts), decode_rows=None,
+                            chunk_rows=i32(list(range(count))), n_decode=0, n_chunk=count, max_decode_len=0, max_chunk_query=n,
+                            max_chunk_len=bound)
+        got = hip.paged_attention(q, pages, table, rows(n), page, d ** -0.5, window)
+        assert torch.equal(got, hip.paged_attention(q, pages, table, rows(1000), page, d ** -0.5, window)), (n, window)
+        want = TorchKernels().paged_attention(q.float(), pages.float(), table, rows(n), page, d ** -0.5, window)
+        tight = 1e-5 if dtype == torch.float32 else 1e-2
+        assert H.rel_rms(got, want) < tight and H.rel_rms(hip.paged_attention(q, pages, table, rows(1), page, d ** -0.5, window), want) < tight

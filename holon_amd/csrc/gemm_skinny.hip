@@ -90,47 +90,51 @@ __device__ __forceinline__ float over_lane_groups(float v, int c) {
 // registers while the other set's are asked for: a wave that asks for all, waits for all and multiplies has nothing under way
 // for part of its time. (One row of 2,048 / 8,192 / 18,432 against 2,048 columns, 16 waves a tile: 8 loads in one set 5.1, 11.6,
 // 24.2 us; two sets of 4 4.35, 9.7, 21.7.)
-template <int NT, int UNROLL, typename Tokens, typename Turn>
+// REST: steps is no multiple of UNROLL; what is left over is asked for while the last whole set is multiplied, where one load after
+// the other behind it took 20 % of a short K's time (18432 x 704 at one row 9.7 us and 6.6 so; gated, 5120 x 1280, 6.9 and 6.2).
+// Without it the conditions are not there: they cost up to 15 % where nothing is left over (4096 x 2048, gated: 6.6 and 7.8).
+template <int NT, int UNROLL, bool REST, typename Tokens, typename Turn>
 __device__ __forceinline__ void stream_tiles(f32x4_t (&acc)[NT], const bf16_t* const (&wp)[NT], int wstep, int steps,
                                              Tokens tokens, Turn turn) {
   bf16x8_t wf[2][NT][UNROLL], xf[2][UNROLL];
-  const auto ask = [&](auto set, int s) {
+  const auto ask = [&](auto set, int s, int n) {
     constexpr int B = decltype(set)::value;
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)
-        wf[B][j][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)(s + u) * wstep));
+        if (u < n) wf[B][j][u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)(s + u) * wstep));
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u) xf[B][u] = tokens(s + u);
+    for (int u = 0; u < UNROLL; ++u)
+      if (u < n) xf[B][u] = tokens(s + u);
   };
-  const auto use = [&](auto set) {
+  const auto use = [&](auto set, int n) {
     constexpr int B = decltype(set)::value;
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
+      if (u < n)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[B][j][u], xf[B][u], acc[j], 0, 0, 0);
+        for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[B][j][u], xf[B][u], acc[j], 0, 0, 0);
   };
   constexpr std::integral_constant<int, 0> even{};
   constexpr std::integral_constant<int, 1> odd{};
-  const int rounds = steps / UNROLL;
-  if (rounds > 0) ask(even, 0);
+  const int rounds = steps / UNROLL, end = rounds * UNROLL, rest = steps - end;      // (the same in all lanes)
+  if (rounds > 0) ask(even, 0, UNROLL);
+  else if (REST) ask(even, 0, rest);
   for (int r = 0; r < rounds; r += 2) {
     turn();
-    if (r + 1 < rounds) ask(odd, (r + 1) * UNROLL);
-    use(even);
+    if (r + 1 < rounds) ask(odd, (r + 1) * UNROLL, UNROLL);
+    else if (REST) ask(odd, end, rest);
+    use(even, UNROLL);
     if (r + 1 < rounds) {
-      if (r + 2 < rounds) ask(even, (r + 2) * UNROLL);
-      use(odd);
+      if (r + 2 < rounds) ask(even, (r + 2) * UNROLL, UNROLL);
+      else if (REST) ask(even, end, rest);
+      use(odd, UNROLL);
     }
   }
-  for (int s = rounds * UNROLL; s < steps; ++s) {
-    const bf16x8_t xl = tokens(s);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const bf16x8_t wl = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[j] + (int64_t)s * wstep));
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wl, xl, acc[j], 0, 0, 0);
-    }
+  if (REST) {
+    if (rounds % 2) use(odd, rest);
+    else use(even, rest);
   }
 }
 
@@ -139,7 +143,7 @@ __device__ __forceinline__ void stream_tiles(f32x4_t (&acc)[NT], const bf16_t* c
 // NT: tiles of 16 weight rows a block owns, next to one another; its waves run them side by side over one copy of the
 // activations, which halves what the activations cost where every block reads all of them. A tile's sums are the same
 // whatever NT is.
-template <int NT, int WPB, int UNROLL, bool TWICE, typename OutT, bool TILED, bool RESID = false>
+template <int NT, int WPB, int UNROLL, bool TWICE, bool REST, typename OutT, bool TILED, bool RESID = false>
 __global__ void __launch_bounds__(WPB * 64) gemm_skinny_kernel(const bf16_t* __restrict__ x,
                                                                 const bf16_t* __restrict__ w, OutT* __restrict__ y,
                                                                 int M, int N, int K, int round_first, RowScale rs,
@@ -182,7 +186,7 @@ __global__ void __launch_bounds__(WPB * 64) gemm_skinny_kernel(const bf16_t* __r
   };
 
   if constexpr (TWICE) {
-    stream_tiles<NT, UNROLL>(acc, wp, WSTEP, steps, tokens, [&] { sums.turn(); });
+    stream_tiles<NT, UNROLL, REST>(acc, wp, WSTEP, steps, tokens, [&] { sums.turn(); });
   } else {
     int s = 0;
     for (; s + UNROLL <= steps; s += UNROLL) {
@@ -272,18 +276,18 @@ __global__ void __launch_bounds__(WPB * 64) gemm_skinny_kernel(const bf16_t* __r
   }
 }
 
-template <int NT, int WPB, int UNROLL, bool TWICE, typename OutT, bool RESID>
+template <int NT, int WPB, int UNROLL, bool TWICE, bool REST, typename OutT, bool RESID>
 static void launch_skinny(const void* x, const void* w, void* y, int M, int N, int K, bool tiled, hipStream_t s,
                           int round_first, RowScale rs, float* stats_out) {
   const dim3 grid(N / 16 / NT), block(WPB * 64);
   if constexpr (RESID)
-    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, OutT, true, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
+    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, REST, OutT, true, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
                                                                                 (OutT*)y, M, N, K, round_first, rs, stats_out);
   else if (tiled)
-    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, OutT, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
+    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, REST, OutT, true><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
                                                                           (OutT*)y, M, N, K, round_first, rs, stats_out);
   else
-    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, OutT, false><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
+    gemm_skinny_kernel<NT, WPB, UNROLL, TWICE, REST, OutT, false><<<grid, block, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,
                                                                            (OutT*)y, M, N, K, round_first, rs, stats_out);
 }
 
@@ -305,6 +309,9 @@ static void launch_skinny(const void* x, const void* w, void* y, int M, int N, i
 //   otherwise one, 4 loads in one set, which is what 8 waves a block and several blocks a unit need least registers for: 12288 x
 //     4096 19.4 / 20.0 / 23.3 (19.5 / 20.6 / 25.3; two tiles 22.8 / 23.6 / 24.7), 9216 x 2048 9.5 / 10.1 / 11.5 (9.7 / 10.7 /
 //     12.6), 151936 x 4096 182 / 190 (184 / 199; two tiles, for 16 rows, 206, where one takes 243 and took 225).
+//   fewer than 8 waves: one, two sets of 8 loads up to 1,024 waves in all, of 4 from there, where registers bound how many of them are
+//     on the chip: 5632 x 1472 6.3 / 6.8 / 7.4 (12.3 / 12.6 / 13.0; sets of 4 7.2 / 7.4 / 7.8), 18432 x 704 6.6 / 7.0 / 8.2 (8.1 / 8.4
+//     / 9.4; sets of 8 8.0 / 8.3 / 9.6), 7168 x 2688 9.2 / 9.7 / 11.6 (13.9 / 14.3 / 14.9; sets of 8 9.9 / 10.9 / 12.3).
 static bool skinny_two(int tiles, int K, int M) {
   return skinny_waves(tiles, K) == 8 && tiles % 2 == 0 &&
          ((tiles >= (M > 8 ? 257 : 320) && tiles < 512) || (tiles >= 1024 && (K < 4096 || M > 8)));
@@ -316,22 +323,30 @@ static int pick_waves(const void* x, const void* w, void* y, int M, int N, int K
   const int tiles = N / 16;
   const int wpb = skinny_waves(tiles, K);
   const bool two = skinny_two(tiles, K, M);
-#define SKINNY(NT, WPB, U, TWICE) \
-  launch_skinny<NT, WPB, U, TWICE, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out)
+  const int steps = K / 32 / wpb;
+#define SKINNY(NT, WPB, U, TWICE, REST) \
+  launch_skinny<NT, WPB, U, TWICE, REST, OutT, RESID>(x, w, y, M, N, K, tiled, s, round_first, rs, stats_out)
+#define SKINNY_TWICE(NT, WPB, U)                      \
+  do {                                                \
+    if (steps % U) SKINNY(NT, WPB, U, true, true);    \
+    else SKINNY(NT, WPB, U, true, false);             \
+  } while (0)
   switch (wpb) {
     case 16:
-      if constexpr (RESID) { SKINNY(1, 16, 8, false); } else { SKINNY(1, 16, 4, true); }
+      if constexpr (RESID) { SKINNY(1, 16, 8, false, false); } else { SKINNY_TWICE(1, 16, 4); }
       break;
     case 8:
-      if (tiles <= 256) SKINNY(1, 8, 4, true);
-      else if (!two) SKINNY(1, 8, 4, false);
-      else if (tiles < 512 && M <= 8) SKINNY(2, 8, 4, true);
-      else SKINNY(2, 8, 2, true);
+      if (tiles <= 256) SKINNY_TWICE(1, 8, 4);
+      else if (!two) SKINNY(1, 8, 4, false, false);
+      else if (tiles < 512 && M <= 8) SKINNY_TWICE(2, 8, 4);
+      else SKINNY_TWICE(2, 8, 2);
       break;
-    case 4: SKINNY(1, 4, 8, true); break;
-    case 2: SKINNY(1, 2, 8, true); break;
-    default: SKINNY(1, 1, 8, true); break;
+    // (fewer than 8: an odd number of steps a wave)
+    case 4: if (tiles <= 256) SKINNY(1, 4, 8, true, true); else SKINNY(1, 4, 4, true, true); break;
+    case 2: if (tiles <= 512) SKINNY(1, 2, 8, true, true); else SKINNY(1, 2, 4, true, true); break;
+    default: SKINNY(1, 1, 8, true, true); break;
   }
+#undef SKINNY_TWICE
 #undef SKINNY
   return 0;
 }
@@ -390,7 +405,7 @@ extern "C" int holon_gemm_skinny_add_bf16(const void* x, const void* w_tiled, vo
 
 // The gated form: w = [gate rows; up rows] (2I rows), y[M, I] = round(act(round(x gate^T))) * round(x up^T), act silu or
 // (ACT 1) the tanh form of gelu, the roundings of the two-kernel composition. A block owns gate tile t and up tile t + I/16 and streams both.
-template <int WPB, int UNROLL, bool TILED, int ACT>
+template <int WPB, int UNROLL, bool REST, bool TILED, int ACT>
 __global__ void __launch_bounds__(WPB * 64) gemm_skinny_glu_kernel(const bf16_t* __restrict__ x,
                                                                     const bf16_t* __restrict__ w,
                                                                     bf16_t* __restrict__ y, int M, int I, int K,
@@ -424,7 +439,7 @@ __global__ void __launch_bounds__(WPB * 64) gemm_skinny_glu_kernel(const bf16_t*
     }
     return xf;
   };
-  stream_tiles<2, UNROLL>(acc, wp, WSTEP, steps, tokens, [&] { sums.turn(); });
+  stream_tiles<2, UNROLL, REST>(acc, wp, WSTEP, steps, tokens, [&] { sums.turn(); });
   f32x4_t ss = sums.finish();
   if (WPB > 1) {
     if (wave > 0) {
@@ -470,12 +485,18 @@ static int skinny_glu(const void* x, const void* w, void* y, int M, int I, int K
   // few tile pairs: four waves share each; otherwise two. At 1 / 8 / 16 rows 768 pairs over K = 4,096 take 34.4 / 34.3 / 35.0 us,
   // 384 over 2,048 11.6 / 12.3 / 13.3 (35.4 / 35.7 / 36.6 and 12.1 / 13.3 / 14.6 with 8 loads in one set of registers).
   const bool few = I / 16 < 512;
-#define GLU(WPB, U)                                                                                              \
-  if (tiled) gemm_skinny_glu_kernel<WPB, U, true, ACT><<<I / 16, WPB * 64, 0, s>>>((const bf16_t*)x, (const bf16_t*)w, \
-                                                                             (bf16_t*)y, M, I, K, rs);           \
-  else gemm_skinny_glu_kernel<WPB, U, false, ACT><<<I / 16, WPB * 64, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,      \
-                                                                        (bf16_t*)y, M, I, K, rs)
-  if (few) { GLU(4, 4); } else { GLU(2, 4); }
+#define GLU(WPB, U, REST)                                                                                              \
+  do {                                                                                                                 \
+    if (tiled) gemm_skinny_glu_kernel<WPB, U, REST, true, ACT><<<I / 16, WPB * 64, 0, s>>>((const bf16_t*)x, (const bf16_t*)w, \
+                                                                                     (bf16_t*)y, M, I, K, rs);         \
+    else gemm_skinny_glu_kernel<WPB, U, REST, false, ACT><<<I / 16, WPB * 64, 0, s>>>((const bf16_t*)x, (const bf16_t*)w,      \
+                                                                                (bf16_t*)y, M, I, K, rs);              \
+  } while (0)
+  const bool rest = K / 32 / (few ? 4 : 2) % 4 != 0;
+  if (few && rest) GLU(4, 4, true);
+  else if (few) GLU(4, 4, false);
+  else if (rest) GLU(2, 4, true);
+  else GLU(2, 4, false);
 #undef GLU
   HOLON_LAUNCH_OK();
   return 0;

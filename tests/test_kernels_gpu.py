@@ -1311,3 +1311,28 @@ def test_general_attention_of_short_rows(hip, dtype, heads, kv, d):
         want = TorchKernels().paged_attention(q.float(), pages.float(), table, rows(n), page, d ** -0.5, window)
         tight = 1e-5 if dtype == torch.float32 else 1e-2
         assert H.rel_rms(got, want) < tight and H.rel_rms(hip.paged_attention(q, pages, table, rows(1), page, d ** -0.5, window), want) < tight
+
+
+def test_few_row_products_whose_steps_leave_a_rest(hip):
+    """A wave's steps of 32 are multiplied in sets of 2, 4 or 8, and what is left over in a set by itself: every remainder of each, none
+    among them, fewer steps than a set, for each number of waves a tile, both weight layouts and the gated form, against float64; a
+    row bit for bit what it is alone."""
+    bf = torch.bfloat16
+    for n, k in ((48, 288), (48, 352), (64, 416), (32, 480), (16, 544), (48, 320), (64, 448), (80, 576), (48, 704), (8224, 704), (64, 832),
+                 (48, 384), (64, 640), (80, 896), (48, 1152), (4112, 1664), (48, 256), (64, 768), (2064, 768), (80, 1280), (48, 1792),
+                 (64, 2304), (5136, 1152), (5120, 1280), (5136, 1792), (16400, 2816), (5120, 256), (48, 512), (64, 1024), (64, 1536),
+                 (80, 2048), (80, 2560), (48, 3584), (32, 4608)):
+        x, w = _randn(16, k, dtype=bf, seed=160), _randn(n, k, dtype=bf, seed=161)
+        tiled, want = hip.tile_weight(w), x.double() @ w.double().T
+        for held in (tiled, None):
+            for m in (1, 9, 16):
+                got = hip.linear(x[:m].contiguous(), w, tiled=held)
+                assert H.op_budget_usage(got, want[:m], bf, k) <= 1, (m, n, k)
+                assert torch.equal(got[:1], hip.linear(x[:1].contiguous(), w, tiled=held)), (m, n, k)
+    for i, k in ((64, 256), (48, 384), (80, 512), (48, 640), (64, 768), (48, 896), (80, 1024), (64, 1280), (8208, 256), (8192, 384), (8208, 640)):
+        x, w = _randn(16, k, dtype=bf, seed=162, scale=0.5), _randn(2 * i, k, dtype=bf, seed=163, scale=2 * k ** -0.5)
+        tiled = hip.tile_weight(w)
+        for held in (tiled, None):
+            whole = hip.linear_silu_mul(x, w, tiled=held)
+            assert torch.equal(whole[:1], hip.linear_silu_mul(x[:1].contiguous(), w, tiled=held)), (i, k)
+            assert H.rel_rms(whole, torch.nn.functional.silu(x.double() @ w[:i].double().T) * (x.double() @ w[i:].double().T)) < 1e-2, (i, k)

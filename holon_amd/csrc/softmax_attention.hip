@@ -338,8 +338,9 @@ namespace {
 // Both prepares take a block a token, whose first 256 threads add up the squares. Up to 256 tokens it has 1,024 threads: such a
 // step waits for a round of memory per loop over the row, and the loops that write then have a quarter as many. A row of 3,072
 // takes 4.2 and 4.0 us at one token (6.5 and 6.9 with 256 threads throughout); 4,096 tokens of 8,192 keep the chip busy and take
-// 47 and 55 so, 45 and 47 with blocks of 256.
-constexpr int PREP_FEW = 256, PREP_THREADS_FEW = 1024, PREP_THREADS = 256;
+// 47 and 55 so, 45 and 47 with blocks of 256. A row of less than 1,024 has no such rounds to
+// save: 200 tokens of 176 and of 272 take 4.5 and 4.4 us (4.7 and 4.6).
+constexpr int PREP_FEW = 256, PREP_WIDE = 1024, PREP_THREADS_FEW = 1024, PREP_THREADS = 256;
 
 // Sum over the block's first 256 threads of two values at once; waves are added in order.
 __device__ __forceinline__ void block_sum2_256(float& a, float& b, float (*part)[4]) {
@@ -490,10 +491,11 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(const T* __restrict__
 }
 }  // namespace
 
-#define PREPARE(KERNEL, T, ...)                                                             \
-  do {                                                                                      \
-    if (tokens <= PREP_FEW) KERNEL<T, PREP_THREADS_FEW><<<tokens, PREP_THREADS_FEW, 0, s>>>(__VA_ARGS__); \
-    else KERNEL<T, PREP_THREADS><<<tokens, PREP_THREADS, 0, s>>>(__VA_ARGS__);              \
+#define PREPARE(KERNEL, T, ...)                                                                       \
+  do {                                                                                                \
+    if (tokens <= PREP_FEW && width >= PREP_WIDE)                                                     \
+      KERNEL<T, PREP_THREADS_FEW><<<tokens, PREP_THREADS_FEW, 0, s>>>(__VA_ARGS__);                   \
+    else KERNEL<T, PREP_THREADS><<<tokens, PREP_THREADS, 0, s>>>(__VA_ARGS__);                        \
   } while (0)
 
 extern "C" int holon_whole_norm_prepare(const void* qkv, int tokens, int heads, int kv_heads, int dim, int vdim,
@@ -504,6 +506,7 @@ extern "C" int holon_whole_norm_prepare(const void* qkv, int tokens, int heads, 
               "whole_norm_prepare: %d/%d heads of %d/%d, pages of %d", heads, kv_heads, dim, vdim, page_size);
   if (tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
+  const int width = (heads + kv_heads) * dim + kv_heads * vdim;
   if (dtype == HOLON_F32)
     PREPARE(whole_norm_prepare_kernel, float, (const float*)qkv, heads, kv_heads, dim, vdim, (const float*)q_weight,
             (const float*)k_weight, eps, (float*)q, (float*)pages, write_page, write_off, page_size, num_pages);
@@ -530,6 +533,7 @@ extern "C" int holon_latent_rope_prepare(const void* both, int both_stride, int 
               "latent_rope_prepare: %d of %d dimensions rotated, a table of %d rows", rd, rot, table_rows);
   if (tokens == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
+  const int width = heads * (dim + rot) + kv_rank + rot;
   if (dtype == HOLON_F32)
     PREPARE(latent_rope_prepare_kernel, float, (const float*)both, both_stride, heads, dim, rot, kv_rank,
             (const float*)c_weight, eps, table, rd, table_rows, positions, (float*)qn, (float*)full, (float*)pages,

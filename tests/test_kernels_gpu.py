@@ -1336,3 +1336,22 @@ def test_few_row_products_whose_steps_leave_a_rest(hip):
             whole = hip.linear_silu_mul(x, w, tiled=held)
             assert torch.equal(whole[:1], hip.linear_silu_mul(x[:1].contiguous(), w, tiled=held)), (i, k)
             assert H.rel_rms(whole, torch.nn.functional.silu(x.double() @ w[:i].double().T) * (x.double() @ w[i:].double().T)) < 1e-2, (i, k)
+
+
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(3, 1, 204, 204), (2, 2, 128, 255), (2, 2, 128, 256), (14, 1, 64, 64)])
+def test_whole_norm_prepare_around_its_block_sizes(hip, heads, kv, dim, vdim):
+    """Rows of 1,020 to 1,024 values, steps of up to 256 tokens and more: blocks of 256 and of 1,024 threads leave the same bits, which are
+    the plain form's within a rounding."""
+    from holon_amd.kernels.registry import kernel_op
+    width, bf, page = (heads + kv) * dim + kv * vdim, torch.bfloat16, 16
+    x, qw, kw = _randn(257, width, dtype=bf, seed=170), 1 + _randn(heads * dim, dtype=bf, seed=171, scale=0.1), 1 + _randn(kv * dim, dtype=bf, seed=172, scale=0.1)
+    at = torch.arange(257, dtype=torch.int32, device="cuda")
+    held = {}
+    for t in (1, 256, 257):
+        pages = torch.zeros(17, kv * page * (dim + vdim), dtype=bf, device="cuda")
+        held[t] = hip.whole_norm_prepare(x[:t].contiguous(), heads, kv, dim, vdim, qw, kw, 1e-5, pages, at[:t] // page, at[:t] % page, page), pages
+    plain = torch.zeros_like(pages)
+    want = kernel_op("whole_norm_prepare").plain(x, heads, kv, dim, vdim, qw, kw, 1e-5, plain, at // page, at % page, page)
+    assert H.rel_rms(held[257][0], want) < 3e-3 and H.rel_rms(held[257][1], plain) < 3e-3
+    assert torch.equal(held[256][0], held[257][0][:256]) and torch.equal(held[256][1][:16], held[257][1][:16])
+    assert torch.equal(held[1][0], held[257][0][:1])

@@ -702,3 +702,26 @@ def test_key_heads_that_share_value_heads_on_the_gpu(dim):
                 general = k.softmax_attention(q.to(dtype), flat.to(dtype), table.to(dev), rows, token_row, positions,
                                               groups, dim, page, sk, scale, 0, softcap=cap, value_share=share)
                 assert H.rel_rms(general.view(-1, heads, dim), ref) < tol, (dim, heads, groups, share, cap, dtype)
+
+
+def test_chosen_experts_alone_where_that_is_done_sooner():
+    """Whether a step of few rows reads the chosen experts' weights alone: by what that saves against what the search for them costs."""
+    from holon_amd.parts.ffn import moe_few_pays
+    assert [moe_few_pays(m, 2048, 8, 2048, True, 2) for m in (1, 2, 4, 6, 7, 16)] == [True, True, True, True, False, False]
+    assert [moe_few_pays(m, 4096, 64, 512, True, 6) for m in (1, 4, 16)] == [True, True, True]
+    assert [moe_few_pays(m, 1024, 128, 64, False, 8) for m in (1, 2, 8, 16)] == [True, True, False, False]
+    assert not any(moe_few_pays(m, 256, 4, 64, True, 1) for m in range(1, 17)) and not moe_few_pays(4096, 4096, 64, 512, True, 6)
+
+
+@pytest.mark.gpu
+def test_chosen_experts_alone_or_all_of_them(tmp_path, monkeypatch):
+    """Decoding a row over experts of a size that the few-row products serve, from graphs: bit for bit the same logits over the chosen
+    experts' columns and over all of them."""
+    from holon_amd.parts import ffn
+    assert ffn.moe_few_pays(1, 256, 8, 512, True, 2) and ffn.moe_few_serves(1, 256, 8, 512, 64)
+    config = M.model(256, 160, [M.attention(4, 2, 64, 0.3, mlp=M.moe(8, 2, 512, shared=64)), M.attention(2, 1, 64, 0.3, mlp=M.moe(8, 2, 512))])
+    folder, ids, got = M.make_folder(tmp_path / "m", config, 23, False), H.random_ids(24, 160, 9), []
+    for side in (True, False):
+        monkeypatch.setattr(ffn, "moe_few_pays", lambda *a, side=side: side)
+        got.append(H.run_trace(_replayer(folder, "cuda", "bfloat16", 16, cache_tokens=32), H.trace_decode_tail("r", ids, 20)))
+    assert got[0].keys() == got[1].keys() and all(torch.equal(got[0][key], got[1][key]) for key in got[0])

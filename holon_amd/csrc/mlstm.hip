@@ -262,10 +262,12 @@ __global__ void __launch_bounds__(WAVE) mlstm_scan_kernel(const T* __restrict__ 
 // and the same for n with 1 in place of v_j. Every factor is a product of factors of at most 1: nothing is divided, no
 // difference of logarithms is taken. The chunk's scores q k^T and the M are formed once by the block's waves together, the
 // scores in float64: a score's rounding is shared by all of the token's columns, and made results lie 1.2 times as far from 64 bits as
-// the token-by-token scan's (16 heads of 128 by 128 over 2,048 tokens: 1.56e-7 against 1.31e-7; so 1.14e-7, for 2 % of the time).
-// Bound by the float32 matrix cores (two products with S a token), and by the barriers around a chunk. Two layers of 16 heads of
-// 128 by 128 over steps of 4,096 and 304 tokens: 150 us for the first passes and 368 for the second ones; token by token,
-// a wave 8 columns with S in registers, 3,400 in all.
+// the token-by-token scan's (16 heads of 128 by 128 over 2,048 tokens: 1.56e-7 against 1.31e-7; so 1.14e-7, for 5 % of the time).
+// Bound by the float32 matrix cores (two products with S a token), by the barriers around a chunk, and in the second pass by its
+// registers: keys of 128 need all 256 and spill 42 of them (172 bytes a lane), keys of 256 138, with the LDS for two waves a SIMD (one
+// block a unit) to hide that; the first pass spills at keys of 256 alone (36). Two layers of 16 heads of 128 by 128 over steps of 4,096
+// and 304 tokens: 150 us for the first passes and 400 for the second ones (368 without the scores in float64 and the branch for
+// values that are not finite); token by token, a wave 8 columns with S in registers, 3,400 in all.
 // Operands: lane (g4, c) of A holds row c, of B column c, and product i of a group of 16 takes inner index 4 g4 + i, so that
 // a result's registers are the B operands of the products over its rows.
 template <int KD, int PASS, typename T>

@@ -23,7 +23,7 @@ SHORT = (("_Z18gemm_skinny_kernelILi", "gemm_skinny<"), ("_Z22gemm_skinny_glu_ke
          ("_Z23attn_prefill_dma_kernel8AttnArgs", "attn_prefill_dma"), ("_Z24attn_prefill_pair_kernelILi", "attn_prefill_pair<"),
          ("_Z17attn_merge_kernel", "attn_merge"), ("_Z13argmax_kernel", "argmax"), ("_Z20argmax_pieces_kernel", "argmax_pieces"),
          ("_Z23argmax_of_pieces_kernel", "argmax_of_pieces"), ("_Z16embedding_kernel", "embedding"),
-         ("_Z15gemm_f32_kernel", "gemm_f32"), ("_Z13sample_kernel", "sample"),
+         ("_Z13sample_kernel", "sample"),
          ("_ZN12_GLOBAL__N_116gemm_rows_kernelILi", "gemm_rows<"),
          ("_Z20gated_mul_vec_kernelI", "gated_mul_vec<"), ("_Z16gated_mul_kernelI", "gated_mul<"), ("_ZN12_GLOBAL__N_118memory_scan_kernelILi", "memory_scan<"),
          ("_ZN12_GLOBAL__N_117delta_scan_kernelILi", "delta_scan<"), ("_ZN12_GLOBAL__N_118stream_norm_kernelILi", "stream_norm<"),

@@ -416,6 +416,13 @@ int holon_moe_up_few_bf16(const void* x, const void* w_tiled, void* act, int row
                           int gated, const float* weights, int wstride, int shared_col, void* stream);
 int holon_moe_down_few_bf16(const void* act, const void* w_tiled, void* y, int rows, int hidden, int experts, int ff,
                             int shared, const float* weights, int wstride, void* stream);
+// The experts for steps of many bfloat16 rows, every expert over the rows that chose it alone: y [rows, hidden] from x, the
+// first projections `up` and the second ones `down` as they come (untiled), with the activations and roundings of the few-row
+// form. At most `top` weights a row are not 0. Scratch as the definition says.
+int holon_moe_rows_supported(int rows, int hidden, int experts, int top, int ff, int shared);
+int holon_moe_rows_bf16(const void* x, const void* up, const void* down, void* y, int* lists, void* act, float* parts, int rows,
+                        int hidden, int experts, int top, int ff, int shared, int gated, const float* weights, int wstride,
+                        int shared_col, void* stream);
 // up [rows, C], C = experts ff + shared: y = max(up, 0)^2 times the weight of the column's expert (as for holon_moe_gate).
 int holon_moe_relu2(const void* up, const float* weights, void* y, int64_t rows, int experts, int ff, int shared, int dtype,
                     int wstride, int shared_col, void* stream);

@@ -1,0 +1,323 @@
+// The experts of a mixture for steps of many rows (prompts), bfloat16: every expert's products over the rows that chose it
+// alone, where the products over all experts multiply every row by every expert and add zeros (2 of 8 experts beside a
+// shared one: three times the products). Four launches after the router:
+//   lists   which rows chose an expert, in their order, and where a row stands among its own choices (a block an expert)
+//   up      tiles of 256 of an expert's rows, gathered, against 128 gates and the same 128 ups (or 256 ups): the activation
+//           and the weight in the epilogue, rows of the expert's own -> act
+//   down    tiles of act against the expert's columns of the second weight -> a row's part from that expert, float32
+//   add     a row's parts in the experts' order, rounded once
+// The shared expert's rows are all rows; its tiles come first in `up`'s and `down`'s launches. Which tile a block takes is
+// read from the lists on the device, so the launches are the same whatever was chosen: the grid is the most tiles there can
+// be, and what is left over ends at once.
+//
+// Bound by the matrix pipe (gemm_block.h). 4,096 rows of 4,096, 8 experts of 3,072 of which a row takes two, beside a shared
+// one: 0.93 TFLOP where the products over all take 2.78.
+#include <algorithm>
+
+#include "common.h"
+#include "gemm_block.h"
+#include "holon_hip.h"
+
+namespace {
+using namespace block_gemm;
+constexpr int MAX_EXPERTS = 1024, MAX_TOP = 256;
+constexpr int TOKEN_BITS = 22;                       // a list's entry: the row, and above it the place among the row's choices
+constexpr int LIST_THREADS = 1024;
+
+struct MoeRows {
+  const float* weights;                              // [rows, stride]: 0 where a row did not choose an expert
+  int stride, rows, hidden, experts, top, ff, shared, shared_col;   // shared_col < 0: the shared expert's weight is 1
+  int* counts;                                       // [experts] rows that chose it
+  int* lists;                                        // [experts, rows]
+  int* slots;                                        // [rows, top] where a row's parts lie, -1: it made fewer choices
+};
+
+// Blocks of `experts`: an expert's list. The rest: what rows of fewer choices than `top` leave over. (No more than `top` of a
+// row's weights are taken, so that the lists hold rows * top entries at most whatever the weights are.)
+__global__ void __launch_bounds__(LIST_THREADS) moe_lists_kernel(MoeRows p) {
+  __shared__ int sums[LIST_THREADS / WAVE];
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  if ((int)blockIdx.x >= p.experts) {
+    const int t = (blockIdx.x - p.experts) * LIST_THREADS + threadIdx.x;
+    if (t >= p.rows) return;
+    int n = 0;
+    for (int e = 0; e < p.experts; ++e) n += p.weights[(int64_t)t * p.stride + e] != 0.f;
+    for (int j = n; j < p.top; ++j) p.slots[(int64_t)t * p.top + j] = -1;
+    return;
+  }
+  const int e = blockIdx.x;
+  int total = 0;
+  for (int t0 = 0; t0 < p.rows; t0 += LIST_THREADS) {
+    const int t = t0 + threadIdx.x;
+    int place = 0;
+    bool mine = t < p.rows && p.weights[(int64_t)t * p.stride + e] != 0.f;
+    if (mine) {
+      for (int before = 0; before < e; ++before) place += p.weights[(int64_t)t * p.stride + before] != 0.f;
+      mine = place < p.top;
+    }
+    const uint64_t mask = __ballot(mine);
+    if (lane == 0) sums[wave] = __popcll(mask);
+    __syncthreads();
+    int at = total, all = 0;
+    for (int w = 0; w < LIST_THREADS / WAVE; ++w) {
+      if (w < wave) at += sums[w];
+      all += sums[w];
+    }
+    if (mine) p.lists[(int64_t)e * p.rows + at + __popcll(mask & ((1ull << lane) - 1))] = t | place << TOKEN_BITS;
+    total += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) p.counts[e] = total;
+}
+
+struct RowTile {
+  int expert, first, count, row0;                    // the expert's rows come from `first` on; this tile's from row0 of them
+};
+
+// Row tiles of all experts together, and (tile >= 0) which expert's the given one is. Every lane of a wave calls it.
+__device__ __forceinline__ int find_rows(const MoeRows& p, int tile, RowTile& out) {
+  const int lane = threadIdx.x % WAVE;
+  int tiles = 0, rows = 0;
+  for (int e0 = 0; e0 < p.experts; e0 += WAVE) {
+    const int count = e0 + lane < p.experts ? p.counts[e0 + lane] : 0;
+    int t = (count + TILE - 1) / TILE, r = count;
+#pragma unroll
+    for (int o = 1; o < WAVE; o *= 2) {              // sums up to this lane's expert
+      const int t_before = __shfl_up(t, o, WAVE), r_before = __shfl_up(r, o, WAVE);
+      if (lane >= o) t += t_before, r += r_before;
+    }
+    if (tile >= 0) {
+      const uint64_t past = __ballot(tiles + t > tile);
+      if (past != 0) {
+        const int at = __builtin_ctzll(past);
+        out.expert = e0 + at;
+        out.count = __builtin_amdgcn_readlane(count, at);
+        out.first = rows + __builtin_amdgcn_readlane(r, at) - out.count;
+        out.row0 = (tile - tiles - (__builtin_amdgcn_readlane(t, at) - (out.count + TILE - 1) / TILE)) * TILE;
+        return 0;
+      }
+    }
+    tiles += __builtin_amdgcn_readlane(t, WAVE - 1);
+    rows += __builtin_amdgcn_readlane(r, WAVE - 1);
+  }
+  return tiles;
+}
+
+// act of an expert's rows (routed: [rows * top, ff] in the order of the lists) and of the shared expert ([rows, shared]).
+template <bool GATED>
+__global__ void __launch_bounds__(THREADS, 2) moe_up_rows_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                 bf16_t* __restrict__ act, bf16_t* __restrict__ act_shared,
+                                                                 MoeRows p) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  constexpr int COLS = GATED ? HALF : TILE;          // columns of act a tile gives
+  const int K = p.hidden, cols = p.experts * p.ff + p.shared;
+  RowTile rows;
+  const int routed = find_rows(p, -1, rows);
+  const int per_routed = (p.ff + COLS - 1) / COLS, per_shared = (p.shared + COLS - 1) / COLS;
+  const int shared_tiles = p.shared ? (p.rows + TILE - 1) / TILE : 0;
+  const int tile = tile_of_block(blockIdx.x, routed * per_routed + shared_tiles * per_shared);
+  if (tile < 0) return;
+  const int first = shared_tiles * per_shared;
+  const bool is_routed = tile >= first;
+  int rt, ct;
+  if (is_routed) {
+    row_and_column(tile - first, routed, per_routed, rt, ct);
+    find_rows(p, rt, rows);
+  } else {
+    row_and_column(tile, shared_tiles, per_shared, rt, ct);
+    rows = RowTile{p.experts, 0, p.rows, rt * TILE};
+  }
+  const int width = is_routed ? p.ff : p.shared;     // columns the expert has
+  const int* list = p.lists + (int64_t)rows.expert * p.rows;
+  const auto token = [&](int i) { return is_routed ? list[i] & ((1 << TOKEN_BITS) - 1) : i; };
+  const int64_t w_row = (int64_t)rows.expert * p.ff + ct * COLS;
+  uint32_t x_at[2][2], w_at[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {                    // (rows and columns past the last repeat it: nothing of them is written)
+      const int r = copy_row(q), last = width - 1 - ct * COLS;
+      x_at[h][q] = (uint32_t)((int64_t)token(min(rows.row0 + h * HALF + r, rows.count - 1)) * K * 2) + copy_piece(q);
+      const int64_t column = GATED ? (int64_t)h * cols + min(r, last) : min(h * HALF + r, last);
+      w_at[h][q] = (uint32_t)(column * K * 2) + copy_piece(q);
+    }
+  Acc acc;
+  acc.clear();
+  run(acc, lds, x, w + w_row * K, x_at, w_at, K / KC);
+  const Place at;
+  // through LDS, so that a row's columns leave as whole lines (a lane holds four of them): 128 columns in rows of 256 bytes and
+  // a piece, twice where a tile gives 256
+  constexpr int PITCH = HALF * 2 + 16;
+  static_assert(TILE * PITCH <= LDS_BYTES, "a tile's half of the columns");
+  bf16_t* out = is_routed ? act + (int64_t)rows.first * p.ff : act_shared;
+#pragma unroll
+  for (int j = 0; j < COLS / HALF; ++j) {
+    if (j > 0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = rows.row0 + at.row(i, t);
+        const int col = is_routed ? rows.expert : p.shared_col;
+        const float weight = r < rows.count && col >= 0 ? p.weights[(int64_t)token(r) * p.stride + col] : 1.f;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          ushort4 o;
+          bf16_t* oe = reinterpret_cast<bf16_t*>(&o);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {              // the roundings of moe_gate and of moe_relu2
+            float z;
+            if constexpr (GATED) {
+              const float gate = Elem<bf16_t>::round(acc.v[i][0][t][n][v]), up = Elem<bf16_t>::round(acc.v[i][1][t][n][v]);
+              z = Elem<bf16_t>::round(Elem<bf16_t>::round(silu<bf16_t>(gate)) * up) * weight;
+            } else {
+              const float up = fmaxf(Elem<bf16_t>::round(acc.v[i][j][t][n][v]), 0.f);
+              z = up * up * weight;
+            }
+            oe[v] = float_to_bf16(weight != 0.f ? z : 0.f);
+          }
+          *reinterpret_cast<ushort4*>(lds + at.row(i, t) * PITCH + at.column(0, n) * 2) = o;
+        }
+      }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < TILE * 16 / THREADS; ++u) {
+      const int row = u * (THREADS / 16) + threadIdx.x / 16, r = rows.row0 + row, column = ct * COLS + j * HALF + threadIdx.x % 16 * 8;
+      if (r < rows.count && column < width)
+        *reinterpret_cast<uint4*>(out + (int64_t)r * width + column) =
+            *reinterpret_cast<const uint4*>(lds + row * PITCH + threadIdx.x % 16 * 16);
+    }
+  }
+}
+
+// parts [rows * top + rows, hidden] float32: an expert's share of the results of its rows, in the order of the lists, then the
+// shared expert's; which of them are a row's goes into `slots`.
+__global__ void __launch_bounds__(THREADS, 2) moe_down_rows_kernel(const bf16_t* __restrict__ act,
+                                                                   const bf16_t* __restrict__ act_shared,
+                                                                   const bf16_t* __restrict__ w, float* __restrict__ parts,
+                                                                   MoeRows p) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
+  const int N = p.hidden;
+  const int64_t cols = (int64_t)p.experts * p.ff + p.shared;
+  RowTile rows;
+  const int routed = find_rows(p, -1, rows), per = (N + TILE - 1) / TILE;
+  const int shared_tiles = p.shared ? (p.rows + TILE - 1) / TILE : 0;
+  const int tile = tile_of_block(blockIdx.x, (routed + shared_tiles) * per);
+  if (tile < 0) return;
+  const bool is_routed = tile >= shared_tiles * per;
+  int rt, ct;
+  if (is_routed) {
+    row_and_column(tile - shared_tiles * per, routed, per, rt, ct);
+    find_rows(p, rt, rows);
+  } else {
+    row_and_column(tile, shared_tiles, per, rt, ct);
+    rows = RowTile{p.experts, 0, p.rows, rt * TILE};
+  }
+  const int K = is_routed ? p.ff : p.shared;
+  uint32_t x_at[2][2], w_at[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int r = h * HALF + copy_row(q);
+      x_at[h][q] = (uint32_t)((int64_t)min(rows.row0 + r, rows.count - 1) * K * 2) + copy_piece(q);
+      w_at[h][q] = (uint32_t)(min(ct * TILE + r, N - 1) * cols * 2) + copy_piece(q);
+    }
+  Acc acc;
+  acc.clear();
+  run(acc, lds, is_routed ? act + (int64_t)rows.first * K : act_shared, w + (int64_t)rows.expert * p.ff, x_at, w_at, K / KC);
+  const Place at;
+  float* out = parts + ((int64_t)(is_routed ? rows.first : p.rows * (int64_t)p.top)) * N;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int r = rows.row0 + at.row(i, t);
+      if (r >= rows.count) continue;
+      if (is_routed && ct == 0 && at.wc == 0 && at.g == 0) {      // (one lane a row)
+        const uint32_t entry = p.lists[(int64_t)rows.expert * p.rows + r];
+        p.slots[(int64_t)(entry & ((1u << TOKEN_BITS) - 1)) * p.top + (entry >> TOKEN_BITS)] = rows.first + r;
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          const int column = ct * TILE + at.column(j, n);
+          if (column < N) *reinterpret_cast<f32x4_t*>(out + (int64_t)r * N + column) = acc.v[i][j][t][n];
+        }
+    }
+}
+
+// y: a row's parts in the experts' order, the shared expert's last, rounded once. A thread 8 columns, as many loads under way
+// as there are parts: 4,096 rows of 4,096 with three parts each are bound by the 235 MB that are read and written.
+constexpr int ADD_AT_ONCE = 4;
+__global__ void __launch_bounds__(256) moe_add_parts_kernel(const float* __restrict__ parts, bf16_t* __restrict__ y, MoeRows p) {
+  const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (at >= (int64_t)p.rows * p.hidden) return;
+  const int row = (int)(at / p.hidden), column = (int)(at % p.hidden);
+  const int* slots = p.slots + (int64_t)row * p.top;
+  f32x4_t sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  for (int j0 = 0; j0 <= p.top; j0 += ADD_AT_ONCE) {
+    f32x4_t part[ADD_AT_ONCE][2];
+    bool have[ADD_AT_ONCE];
+#pragma unroll
+    for (int u = 0; u < ADD_AT_ONCE; ++u) {
+      const int j = j0 + u;
+      const int64_t slot = j < p.top ? slots[j] : (j == p.top && p.shared ? p.rows * (int64_t)p.top + row : -1);
+      have[u] = slot >= 0;
+      const float* from = parts + (have[u] ? slot : 0) * p.hidden + column;      // (some part, and not added)
+      part[u][0] = *reinterpret_cast<const f32x4_t*>(from);
+      part[u][1] = *reinterpret_cast<const f32x4_t*>(from + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < ADD_AT_ONCE; ++u)
+      if (have[u]) sum[0] += part[u][0], sum[1] += part[u][1];
+  }
+  uint4 o;
+  bf16_t* oe = reinterpret_cast<bf16_t*>(&o);
+#pragma unroll
+  for (int v = 0; v < 8; ++v) oe[v] = float_to_bf16(sum[v / 4][v % 4]);
+  *reinterpret_cast<uint4*>(y + at) = o;
+}
+}  // namespace
+
+// Whether the products serve `rows` rows of `hidden`: sizes the loop's chunks divide, offsets that 32 bits hold.
+extern "C" int holon_moe_rows_supported(int rows, int hidden, int experts, int top, int ff, int shared) {
+  const int64_t cols = (int64_t)experts * ff + shared;
+  const auto deep = [](int k) { return k >= 128 && k % 128 == 0; };
+  return rows >= 1 && rows < 1 << TOKEN_BITS && deep(hidden) && deep(ff) && (shared == 0 || deep(shared)) && experts >= 1 &&
+         experts <= MAX_EXPERTS && top >= 1 && top <= experts && top <= MAX_TOP && (int64_t)rows * top * ff < (int64_t)1 << 31 &&
+         (int64_t)rows * hidden < (int64_t)1 << 31 && (int64_t)rows * shared < (int64_t)1 << 31 &&
+         (cols + HALF) * hidden < (int64_t)1 << 31 && (int64_t)experts * rows < (int64_t)1 << 31;
+}
+
+// y [rows, hidden] = the experts' and the shared expert's results of x, over the weights [gates; ups] or [ups] (rows as they
+// come, `up`) and the second projections side by side (`down` [hidden, experts ff + shared]). Scratch: lists [experts (rows +
+// 1) + rows top] whole numbers, act [rows (top ff + shared)], parts [rows (top + 1), hidden] float32.
+extern "C" int holon_moe_rows_bf16(const void* x, const void* up, const void* down, void* y, int* lists, void* act, float* parts,
+                                   int rows, int hidden, int experts, int top, int ff, int shared, int gated,
+                                   const float* weights, int wstride, int shared_col, void* stream) {
+  HOLON_CHECK(holon_moe_rows_supported(rows, hidden, experts, top, ff, shared) && wstride >= experts && shared_col < wstride,
+              "moe (many rows): %d rows of %d, %d experts of %d (%d a row), %d shared columns not served", rows, hidden, experts,
+              ff, top, shared);
+  hipStream_t s = (hipStream_t)stream;
+  MoeRows p{weights, wstride, rows, hidden, experts, top, ff, shared, shared_col, lists, nullptr, nullptr};
+  p.lists = p.counts + experts;
+  p.slots = p.lists + (int64_t)experts * rows;
+  bf16_t* act_routed = (bf16_t*)act;
+  bf16_t* act_shared = act_routed + (int64_t)rows * top * ff;
+  const auto tiles = [](int64_t n, int of) { return (n + of - 1) / of; };
+  // an expert's last tile is partly empty, and no more tiles than that
+  const int64_t routed = std::min<int64_t>((int64_t)rows * top / TILE + experts, (int64_t)experts * tiles(rows, TILE));
+  const int cols = gated ? HALF : TILE;
+  const int64_t up_tiles = routed * tiles(ff, cols) + tiles(rows, TILE) * tiles(shared, cols);
+  const int64_t down_tiles = (routed + (shared ? tiles(rows, TILE) : 0)) * tiles(hidden, TILE);
+  const auto blocks = [&](int64_t n) { return (unsigned)(tiles(n, XCDS) * XCDS); };      // every XCD as many
+  moe_lists_kernel<<<experts + (unsigned)tiles(rows, LIST_THREADS), LIST_THREADS, 0, s>>>(p);
+  if (gated) moe_up_rows_kernel<true><<<blocks(up_tiles), THREADS, 0, s>>>((const bf16_t*)x, (const bf16_t*)up, act_routed, act_shared, p);
+  else moe_up_rows_kernel<false><<<blocks(up_tiles), THREADS, 0, s>>>((const bf16_t*)x, (const bf16_t*)up, act_routed, act_shared, p);
+  moe_down_rows_kernel<<<blocks(down_tiles), THREADS, 0, s>>>(act_routed, act_shared, (const bf16_t*)down, parts, p);
+  moe_add_parts_kernel<<<(unsigned)tiles((int64_t)rows * hidden, 2048), 256, 0, s>>>(parts, (bf16_t*)y, p);
+  HOLON_LAUNCH_OK();
+  return 0;
+}

@@ -385,6 +385,68 @@ register_kernel(KernelOp("moe_few", moe_few_plain, ("holon_moe_up_few_bf16", "ho
                          _moe_few_hip))
 
 
+def moe_rows_plain(x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
+    """The experts' two products and the activation between them for steps of many rows, every expert over the rows that chose
+    it alone, with the roundings of `linear`, `moe_gate` (`gated`) or `moe_relu2`, and `linear` (whose sums over the experts
+    are cut at the experts); None where they are not served (the caller then composes the three). The plain form never does."""
+    return None
+
+
+def moe_rows_serves(rows: int, hidden: int, experts: int, top: int, ff: int, shared: int) -> bool:
+    """What the library's `holon_moe_rows_supported` answers."""
+    def deep(k):
+        return k >= 128 and k % 128 == 0
+    return 1 <= rows < 1 << 22 and deep(hidden) and deep(ff) and (shared == 0 or deep(shared)) and 1 <= top <= experts <= 1024 \
+        and top <= 256 and max(rows * top * ff, rows * hidden, rows * shared, (experts * ff + shared + 128) * hidden,
+                               experts * rows) < 1 << 31
+
+
+def moe_rows_pays(rows: int, hidden: int, experts: int, ff: int, shared: int, gated: bool, top: int) -> bool:
+    """Whether a step of many rows is done sooner over every expert's own rows than with all rows over all experts, by what either
+    takes in us: tiles of 256 x 256 over 256 compute units (1.6 us a round and 64 columns of K where there are several rounds, 1.3
+    where there is one) and the parts' traffic against the products over all (their operations at 1.2 PFLOP/s and their weights at 4
+    TB/s). Measured on MI355X, own rows / all (us): 8 experts of 3,072 x 4,096 beside a shared one, 2 a row, at 64 / 512 / 4,096 rows
+    181 / 218 / 830 and 226 / 472 / 2,035; of 2,048 x 2,048 at 64 / 512 / 4,096 86 / 93 / 345 and 89 / 211 / 853; 8 of 1,024 beside a
+    shared one of 2,048, 4 a row, at 64 / 512 / 1,024 / 4,096 82 / 97 / 113 / 405 and 50 / 85 / 149 / 438; 64 of 512, 6 a row, at 64 /
+    1,024 128 / 168 and 131 / 496. A step whose parts would take more memory than the products over all stays with those."""
+    if rows <= 16:
+        return False
+    cols = experts * ff + shared
+    if 2 * (top * ff + shared) + 4 * (top + 1) * hidden > 6 * cols:
+        return False
+    row_tiles, all_tiles = max(min(experts, rows * top), rows * top / 256 + experts / 2), -(-rows // 256)
+    width = 128 if gated else 256
+    up = row_tiles * -(-ff // width) + all_tiles * -(-shared // width)
+    down = (row_tiles * (0.029 * ff + 8) + (all_tiles * (0.029 * shared + 8) if shared else 0)) * -(-hidden // 256)
+    own = 12 + hidden * max(0.0205, 0.029 * up / 256) + max(0.0205 * max(ff, shared), down / 256) + rows * hidden * (top + 1) / 1.1e6
+    values = (3 if gated else 2) * cols * hidden
+    return own < 0.93 * (20 + 2 * rows * values / 1.2e9 + 2 * values / 4e6)
+
+
+def _moe_rows_hip(launch, x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
+    t, hidden = x.shape
+    cols = experts * ff + shared
+    if x.dtype != torch.bfloat16 or not moe_rows_serves(t, hidden, experts, top, ff, shared):
+        return None
+    _need(x.is_cuda and x.is_contiguous() and weights.is_contiguous() and weights.dtype == torch.float32
+          and tuple(weights.shape) == (t, experts + int(bool(shared_weight)))
+          and all(w.is_contiguous() and w.dtype == x.dtype and w.data_ptr() % 16 == 0 for w in (up, down)) and x.data_ptr() % 16 == 0
+          and tuple(up.shape) == ((2 if gated else 1) * cols, hidden) and tuple(down.shape) == (hidden, cols),
+          f"moe_rows: rows {tuple(x.shape)}, weights {tuple(weights.shape)}, projections {tuple(up.shape)} and "
+          f"{tuple(down.shape)} for {experts} experts of {ff} and {shared} shared columns")
+    lists = torch.empty(experts * (t + 1) + t * top, dtype=torch.int32, device=x.device)
+    act = torch.empty(t * (top * ff + shared), dtype=x.dtype, device=x.device)
+    parts = torch.empty((t * (top + 1), hidden), dtype=torch.float32, device=x.device)
+    y = torch.empty_like(x)
+    launch(x.data_ptr(), up.data_ptr(), down.data_ptr(), y.data_ptr(), lists.data_ptr(), act.data_ptr(), parts.data_ptr(), t, hidden,
+           experts, top, ff, shared, int(bool(gated)), weights.data_ptr(), weights.shape[1], experts if shared_weight else -1)
+    return y
+
+
+register_kernel(KernelOp("moe_rows", moe_rows_plain, "holon_moe_rows_bf16",
+                         [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _I], _moe_rows_hip))
+
+
 @register_part("ffn", "polynorm")
 class PolyNormFFN(Part):
     """down(act(up(x))) with act = a N(z) + b N(z^2) + c N(z^3) + e (`act` holds a, b, c, e; N divides a token's
@@ -451,8 +513,9 @@ class MoE(Part):
     is weighted by s * `scale`. All experts' gate and up projections are one product and all down projections
     another: the activations of experts a token did not choose are set to 0 in between (`moe_gate`), so the second
     product adds up exactly the chosen experts' weighted outputs, and the shared expert's columns ride in the same two
-    products. Steps of few rows take the same two products over the chosen experts' columns alone (`moe_few`). Every step
-    launches the same kernels whatever was chosen."""
+    products. Steps of few rows take the same two products over the chosen experts' columns alone (`moe_few`), steps of many
+    rows each expert's over the rows that chose it (`moe_rows`), where that is done sooner. Steps of as many rows launch the
+    same kernels whatever was chosen."""
 
     graph_safe = True
 
@@ -536,10 +599,14 @@ class MoE(Part):
             weights = k.moe_router(x, self.router, self.correction if self.has_bias else None, self.top, self.groups,
                                    self.keep, self.scale)
         up, down = self.gate_up, self.all_down
-        # (the results are the same bits)
         if moe_few_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.act == "silu", self.top):
             y = k.moe_few(x, weights, up.tiled, down.tiled, self.experts, self.inter, self.shared, self.act == "silu",
                           shared_weight=self.shared_gated)
+            if y is not None:
+                return y
+        if moe_rows_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top):
+            y = k.moe_rows(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",
+                           shared_weight=self.shared_gated)
             if y is not None:
                 return y
         between = k.moe_relu2 if self.act == "relu2" else k.moe_gate

@@ -713,6 +713,19 @@ def test_chosen_experts_alone_where_that_is_done_sooner():
     assert not any(moe_few_pays(m, 256, 4, 64, True, 1) for m in range(1, 17)) and not moe_few_pays(4096, 4096, 64, 512, True, 6)
 
 
+def test_every_expert_over_its_own_rows_where_that_is_done_sooner():
+    """Whether a step of many rows goes over every expert's own rows, by tiles and bytes; and only where the parts take no more
+    memory than the products over all experts."""
+    from holon_amd.parts.ffn import moe_rows_pays, moe_rows_serves
+    assert [moe_rows_pays(m, 4096, 8, 3072, 3072, True, 2) for m in (16, 64, 512, 4096)] == [False, True, True, True]
+    assert [moe_rows_pays(m, 2048, 8, 1024, 2048, True, 4) for m in (64, 400, 1024, 4096)] == [False, False, True, True]
+    assert [moe_rows_pays(m, 2048, 8, 2048, 2048, False, 2) for m in (64, 512, 4096)] == [False, True, True]
+    assert not moe_rows_pays(4096, 4096, 4, 128, 0, True, 2) and not moe_rows_pays(4096, 2048, 8, 1024, 0, True, 8)
+    assert moe_rows_serves(4096, 4096, 8, 2, 3072, 3072) and moe_rows_serves(1, 128, 1, 1, 128, 0)
+    assert not any(moe_rows_serves(*a) for a in ((64, 192, 8, 2, 128, 0), (64, 256, 8, 2, 64, 0), (64, 256, 8, 2, 128, 64),
+                                                 (64, 256, 2, 3, 128, 0), (0, 256, 8, 2, 128, 0), (1 << 22, 256, 8, 2, 128, 0)))
+
+
 @pytest.mark.gpu
 def test_chosen_experts_alone_or_all_of_them(tmp_path, monkeypatch):
     """Decoding a row over experts of a size that the few-row products serve, from graphs: bit for bit the same logits over the chosen

@@ -1087,6 +1087,43 @@ def test_chosen_experts_alone(hip, hidden, experts, ff, shared, top, gated, own_
     assert hip.moe_few(_randn(17, hidden, dtype=bf), weights, up_t, down_t, experts, ff, shared, gated) is None
 
 
+@pytest.mark.parametrize("hidden,experts,ff,shared,top,gated,own_gate", [
+    (128, 1, 128, 0, 1, True, False), (256, 8, 128, 256, 2, True, True), (384, 5, 384, 0, 3, False, False),
+    (640, 70, 128, 128, 6, True, False), (256, 130, 256, 128, 2, False, False), (2048, 8, 1024, 2048, 4, True, True)])
+def test_every_expert_over_its_own_rows(hip, hidden, experts, ff, shared, top, gated, own_gate):
+    """Against float64 five roundings to bfloat16 (gate, up, their activation, the product, the result), of 2^-9 each at most; and no
+    row's result depends on the rows beside it, nor on which tile of its expert's rows it lies in."""
+    bf, cols = torch.bfloat16, experts * ff + shared
+    up_w = _randn((2 if gated else 1) * cols, hidden, dtype=bf, seed=64, scale=hidden ** -0.5)
+    down_w = _randn(hidden, cols, dtype=bf, seed=65, scale=ff ** -0.5)
+    g = torch.Generator().manual_seed(66)
+    for m in (1, 17, 256, 257, 1030):
+        x = _randn(m, hidden, dtype=bf, seed=67 + m)
+        weights = torch.zeros(m, experts + int(own_gate))
+        for row in range(m):
+            weights[row, torch.randperm(experts, generator=g)[:top]] = torch.rand(top, generator=g) + 0.2
+        weights[:, experts:] = 0.7
+        if m == 257:
+            weights[:, 1:experts] = 0          # one expert for all that chose it, none for the others
+            weights[3:5] = 0                   # rows of no expert, the shared one's gate closed too
+        weights = weights.cuda()
+        got = hip.moe_rows(x, weights, up_w, down_w, experts, top, ff, shared, gated, shared_weight=own_gate)
+        z = x.double() @ up_w.double().T
+        act = torch.nn.functional.silu(z[:, :cols]) * z[:, cols:] if gated else torch.relu(z).square()
+        each = weights[:, :experts].double().repeat_interleave(ff, 1)
+        last = weights[:, experts:].double() if own_gate else torch.ones(m, 1, dtype=torch.double, device="cuda")
+        want = (act * torch.cat((each, last.expand(m, shared)), 1)) @ down_w.double().T
+        apart = H.rel_rms(got, want) if want.any() else got.abs().max().item()
+        assert apart < 5 * 2.0 ** -9, (m, apart)
+        if m == 257 and (own_gate or not shared):
+            assert not got[3:5].any()
+        for row in {0, m // 2, m - 1}:
+            alone = hip.moe_rows(x[row: row + 1].contiguous(), weights[row: row + 1].contiguous(), up_w, down_w, experts, top, ff,
+                                 shared, gated, shared_weight=own_gate)
+            assert torch.equal(alone[0], got[row]), (m, row)
+    assert hip.moe_rows(_randn(4, hidden, dtype=torch.float32), weights[:4], up_w, down_w, experts, top, ff, shared, gated) is None
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_router_of_few_experts(hip, dtype):
     """Both routers up to 64 experts, on either side of 256 rows: the plain form's choice but for rows of a close call, and a

@@ -988,35 +988,39 @@ __device__ __forceinline__ void scores_to_probs(const f32x16_t& sc, int kb, int 
   }
 }
 
-// The same for head_dim 128 with a stage's keys and values copied from the cache into LDS by the memory pipeline
-// itself (global_load_lds: 16 bytes a lane, a wave's 64 lanes into one contiguous kilobyte of LDS), two stages ahead
-// of the one being multiplied, into three buffers in turn: no registers hold a stage on its way, and no instruction
+// The same for head_dim 128 and 256 with a stage's keys and values copied from the cache into LDS by the memory pipeline
+// itself (global_load_lds: 16 bytes a lane, a wave's 64 lanes into one contiguous kilobyte of LDS), as many stages ahead
+// of the one being multiplied as there are further buffers (two at 128; one at 256, where three buffers would leave a
+// compute unit one block), into the buffers in turn: no registers hold a stage on its way, and no instruction
 // writes LDS. A wave's kilobyte has to be contiguous, so rows cannot be padded apart; instead each 16-byte piece
-// sits at place `piece ^ (row % 16)` of its key's 256-byte row (values: each half of the stage's keys apart, a dim's 16
+// sits at place `piece ^ (row % 16)` of its key's row (values: each half of the stage's keys apart, a dim's 16
 // keys a row of 32 bytes, place `piece ^ (row / 8 % 2)`), which a lane's source address arranges and a lane's read
 // undoes: 16 lanes that read the same piece of 16 consecutive rows then touch every bank once, as with padded rows.
 // Every copy instruction reads one page, so its lanes share a scalar base and their own offsets never change.
 // The compiler does not know these loads (it would wait for all of them before every read of LDS): they are issued
-// from inline assembly, and the one wait per stage that they need (all but the newest stage's four loads a lane) is
+// from inline assembly, and the one wait per stage that they need (all but the loads of stages after the next) is
 // written by hand in front of the stage's barrier. Nothing else loads from memory inside the loop.
-// A block's staging of 32-key stages at head_dim 128 through three LDS buffers: what each lane copies, where it reads.
+// A block's staging of 32-key stages through LDS buffers: what each lane copies, where it reads.
+template <int D>
 struct StagedCopies {
-  static constexpr int D = 128;
-  static constexpr int K_BYTES = 32 * D * 2, V_BYTES = D * 32 * 2, STAGE_BYTES = K_BYTES + V_BYTES;   // 8 KB + 8 KB
-  static constexpr int BUFFERS = 3, PG = 4096;
+  static constexpr int K_BYTES = 32 * D * 2, V_BYTES = D * 32 * 2, STAGE_BYTES = K_BYTES + V_BYTES;   // 8 KB + 8 KB at 128
+  static constexpr int BUFFERS = D == 128 ? 3 : 2, AHEAD = BUFFERS - 1, PG = 4096;
+  static constexpr int PER = D / 64;             // kilobytes of keys a wave copies per stage, and of values
+  static constexpr int PIECES = D / 8;           // of 16 bytes a key has
+  static constexpr int KEYS = 64 / PIECES;       // that a kilobyte holds
   const unsigned char* lds;      // BUFFERS * STAGE_BYTES, aligned to 1,024
   const int32_t* pg;             // the row's block table, in LDS
   const bf16_t* kbase;
   const bf16_t* vbase;
   int64_t page_stride;
   int P, max_page, second, wave;
-  uint32_t lds0, k_src[2], v_src[2], k_at[D / 16], v_at[2];
+  uint32_t lds0, k_src[PER], v_src[PER], k_at, v_at[2];
 
-  // What this lane copies per stage: two pieces of keys and two of values (instruction q = 2 * wave + i of eight;
+  // What this lane copies per stage: PER pieces of keys and as many of values (instruction q = PER * wave + i of 4 PER;
   // waves 0 and 1 copy the stage's first 16 keys, which lie in one page, waves 2 and 3 its last 16).
-  // Keys: kilobyte q holds rows 4 q .. 4 q + 3; row 8 i' + 4 h' + r holds key 16 (i' / 2) + 8 h' + 4 (i' % 2) + r of
+  // Keys: kilobyte q holds rows KEYS q .. + KEYS - 1; row 8 i' + 4 h' + r holds key 16 (i' / 2) + 8 h' + 4 (i' % 2) + r of
   // the stage (the order the score product's result wants), so rows 0-15 are the first half. Values: kilobyte q holds
-  // dims 32 (q % 4) .. + 31 of half q / 4, two pieces a dim: keys 0-7 and 8-15 of the half.
+  // 32 dims of half q / (2 PER), two pieces a dim: keys 0-7 and 8-15 of the half.
   // Where it reads: keys, row c, piece 2 ds + h; values, half t, row 32 db + c, piece h (lane = 32 h + c).
   __device__ __forceinline__ void init(const unsigned char* stage_lds, const int32_t* pg_lds, const AttnArgs& a, int hk) {
     lds = stage_lds;
@@ -1031,37 +1035,36 @@ struct StagedCopies {
     wave = threadIdx.x / WAVE;
     second = __builtin_amdgcn_readfirstlane(wave / 2);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int q = 2 * wave + i;
-      const int row = 4 * q + lane / 16, piece = (lane % 16) ^ (row % 16);
+    for (int i = 0; i < PER; ++i) {
+      const int q = PER * wave + i;
+      const int row = KEYS * q + lane / PIECES, piece = (lane % PIECES) ^ (row % 16);
       const int key = 16 * ((row / 8) / 2) + 8 * ((row % 8) / 4) + 4 * ((row / 8) % 2) + row % 4;
       k_src[i] = (uint32_t)(((key % 16) * D + piece * 8) * 2);
-      const int dim = 32 * (q % 4) + lane / 2, vpiece = (lane % 2) ^ ((dim / 8) % 2);
+      const int dim = 32 * (q % (2 * PER)) + lane / 2, vpiece = (lane % 2) ^ ((dim / 8) % 2);
       v_src[i] = (uint32_t)((dim * P + 8 * vpiece) * 2);
     }
     lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)stage_lds;
-#pragma unroll
-    for (int ds = 0; ds < D / 16; ++ds) k_at[ds] = (uint32_t)(c * (D * 2) + 16 * ((2 * ds + h) ^ (c % 16)));
+    k_at = (uint32_t)(c * (D * 2) + 16 * (h ^ (c % 16)));
 #pragma unroll
     for (int t = 0; t < 2; ++t) v_at[t] = (uint32_t)(K_BYTES + t * (V_BYTES / 2) + c * 32 + 16 * (h ^ ((c / 8) % 2)));
   }
-  // four loads a lane: the stage at kb (a stage past kb_last copies the last one again) into buffer `buf`
+  // LOADS loads a lane: the stage at kb (a stage past kb_last copies the last one again) into buffer `buf`
   __device__ __forceinline__ void copy(int kb_want, int kb_last, int buf) const {
     const int kb = min(kb_want, kb_last) + 16 * second;         // this wave's half of the stage: 16 keys of one page
     const int64_t at = (int64_t)__builtin_amdgcn_readfirstlane(pg[min(kb / P, max_page)]) * page_stride;
     const int off = kb % P;
     const bf16_t* kh = kbase + at + (int64_t)off * D;
     const bf16_t* vh = vbase + at + off;
-    const uint32_t to = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)buf * STAGE_BYTES + (uint32_t)wave * 2048);
+    const uint32_t to = __builtin_amdgcn_readfirstlane(lds0 + (uint32_t)buf * STAGE_BYTES + (uint32_t)wave * (1024 * PER));
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < PER; ++i) {
       load_to_lds16(kh, k_src[i], to + 1024 * i);
       load_to_lds16(vh, v_src[i], to + K_BYTES + 1024 * i);
     }
   }
-  static constexpr int LOADS = 4;                               // of a lane, per stage
+  static constexpr int LOADS = 2 * PER;                         // of a lane, per stage
   __device__ __forceinline__ bf16x8_t key(int buf, int ds) const {
-    return *reinterpret_cast<const bf16x8_t*>(lds + buf * STAGE_BYTES + k_at[ds]);
+    return *reinterpret_cast<const bf16x8_t*>(lds + buf * STAGE_BYTES + (k_at ^ (32 * (ds % 8))) + 256 * (ds / 8));
   }
   __device__ __forceinline__ bf16x8_t value(int buf, int db, int t) const {
     return *reinterpret_cast<const bf16x8_t*>(lds + buf * STAGE_BYTES + v_at[t] + db * 1024);
@@ -1070,12 +1073,15 @@ struct StagedCopies {
   static __device__ __forceinline__ int before(int buf) { return buf == 0 ? BUFFERS - 1 : buf - 1; }
 };
 
+// MOD: changed scores (see AttnArgs). They enter the exponential in units of log2: cap tanh(s / cap) as cap - 2 cap / (1 +
+// e^(2 s / cap)), the distance bias as r1 log2(1 + r2 (i - j)). Under a window the stages of kept first keys come before the
+// window's.
+template <int D, bool MOD>
 __global__ void __launch_bounds__(256, 2) attn_prefill_dma_kernel(AttnArgs a) {
-  using SC = StagedCopies;
-  constexpr int D = SC::D;
+  using SC = StagedCopies<D>;
   __shared__ __attribute__((aligned(1024))) unsigned char stage_lds[SC::BUFFERS * SC::STAGE_BYTES];
   __shared__ int32_t pg_lds[SC::PG];
-  static_assert(sizeof(stage_lds) + sizeof(pg_lds) <= 64 * 1024, "a block's static LDS; two blocks share a compute unit");
+  static_assert(sizeof(stage_lds) + sizeof(pg_lds) <= 80 * 1024, "a block's static LDS; two blocks share a compute unit");
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, tid = threadIdx.x;
   const int h = lane / 32, c = lane % 32;
   const int b = a.row_ids[a.unpaired ? blockIdx.z / 2 : blockIdx.z];
@@ -1127,40 +1133,66 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dma_kernel(AttnArgs a) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
     float m = -INFINITY, l = 0.f;
+    const bool far = MOD && a.r1 != nullptr;
+    const float b1 = far && valid ? a.r1[head] : 0.f, b2 = far && valid ? a.r2[head] : 0.f;
+    const float to_log2 = MOD ? 1.f : a.scale_log2;            // (changed scores come in units of log2 already)
+    const float cap = MOD ? a.softcap * 1.4426950408889634f : 0.f, steep = MOD && cap > 0.f ? 2.f * a.scale_log2 / a.softcap : 0.f;
 
-    const int kb_last = (key_hi / 32) * 32;
-    // `last`: the stage holds the row's last key (std::true_type) and may reach past it
-    auto stage = [&](auto last, int kb, int buf) {
+    const int kb_first = (key_lo / 32) * 32, kb_last = (key_hi / 32) * 32;
+    const int keep_first = MOD && a.window > 0 ? a.keep_first : 0, kept = min(keep_first, key_lo);
+    const int kept_end = min((kept + 31) / 32 * 32, kb_first);
+    // `last`: values past `held` may be anything (std::true_type): the stage holds the row's last key, or the kept ones
+    auto stage = [&](auto last, int kb, int buf, int held) {
       if (kb <= tile_last) {
         f32x16_t sc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) sc[i] = 0.f;
-        bf16x8_t kf[D / 16];                       // all of a stage's key fragments are asked for at once
+        constexpr int AT_ONCE = D == 128 ? 8 : 2;  // key fragments (128: all of a stage's) that are asked for at once
 #pragma unroll
-        for (int ds = 0; ds < D / 16; ++ds) kf[ds] = sc_.key(buf, ds);
+        for (int d0 = 0; d0 < D / 16; d0 += AT_ONCE) {
+          bf16x8_t kf[AT_ONCE];
 #pragma unroll
-        for (int ds = 0; ds < D / 16; ++ds) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ds], qf[ds], sc, 0, 0, 0);
-        bf16x8_t vf[D / 32][2];                    // and its value fragments before the softmax that they wait for
+          for (int ds = 0; ds < AT_ONCE; ++ds) kf[ds] = sc_.key(buf, d0 + ds);
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db) {
-          vf[db][0] = sc_.value(buf, db, 0);
-          vf[db][1] = sc_.value(buf, db, 1);
-          if constexpr (decltype(last)::value) {
-            zero_after(vf[db][0], kb + 8 * h, key_hi);
-            zero_after(vf[db][1], kb + 16 + 8 * h, key_hi);
-          }
+          for (int ds = 0; ds < AT_ONCE; ++ds) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ds], qf[d0 + ds], sc, 0, 0, 0);
         }
+        const auto values = [&](int db, bf16x8_t (&vf)[2]) {
+          vf[0] = sc_.value(buf, db, 0);
+          vf[1] = sc_.value(buf, db, 1);
+          if constexpr (decltype(last)::value) {
+            zero_after(vf[0], kb + 8 * h, held);
+            zero_after(vf[1], kb + 16 + 8 * h, held);
+          }
+        };
+        constexpr int EARLY = D == 128 && !MOD ? D / 32 : 0;   // value fragments read before the softmax that they wait for
+        bf16x8_t early[EARLY > 0 ? EARLY : 1][2];
+#pragma unroll
+        for (int db = 0; db < EARLY; ++db) values(db, early[db]);
         // value idx = 4i + r of this lane is key kb + 16*(i/2) + 8h + 4*(i%2) + r against query column c
         const bool whole = kb + 31 <= tile_first && kb >= whole_from;
         float sv[16];
 #pragma unroll
         for (int idx = 0; idx < 16; ++idx) sv[idx] = sc[idx];
+        if constexpr (MOD) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              float& v = sv[4 * i + r];
+              v = cap > 0.f ? cap - 2.f * cap * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(v * steep)) : v * a.scale_log2;
+              if (far) {
+                const int dist = max(qpos - (kb + 16 * (i / 2) + 8 * h + 4 * (i % 2) + r), 0);
+                v -= b1 * __builtin_amdgcn_logf(1.f + b2 * (float)dist);           // (log2)
+              }
+            }
+          }
+        }
         if (!whole) {
 #pragma unroll
           for (int idx = 0; idx < 16; ++idx) {
             const int i = idx / 4, r = idx % 4;
             const int key = kb + 16 * (i / 2) + 8 * h + 4 * (i % 2) + r;
-            if (!(key <= qpos && key >= first)) sv[idx] = -INFINITY;
+            if (!(key <= qpos && (key >= first || (MOD && key < keep_first)))) sv[idx] = -INFINITY;
           }
         }
         float mx = sv[0];
@@ -1170,13 +1202,13 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dma_kernel(AttnArgs a) {
           const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
           mx = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
         }
-        const float m_new = fmaxf(m, mx * a.scale_log2);
+        const float m_new = fmaxf(m, mx * to_log2);
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
         bf16x8_t pb0, pb1;
         float psum = 0.f;
 #pragma unroll
         for (int idx = 0; idx < 16; ++idx) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(sv[idx], a.scale_log2, -m_use));
+          const float p = __builtin_amdgcn_exp2f(fmaf(sv[idx], to_log2, -m_use));
           psum += p;
           if (idx < 8) pb0[idx] = (__bf16)p; else pb1[idx - 8] = (__bf16)p;
         }
@@ -1190,27 +1222,33 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dma_kernel(AttnArgs a) {
         l += psum;
 #pragma unroll
         for (int db = 0; db < D / 32; ++db) {
-          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[db][0], pb0, o[db], 0, 0, 0);
-          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[db][1], pb1, o[db], 0, 0, 0);
+          bf16x8_t vf[2];
+          if constexpr (EARLY > 0) { vf[0] = early[db][0]; vf[1] = early[db][1]; }
+          else values(db, vf);
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0], pb0, o[db], 0, 0, 0);
+          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1], pb1, o[db], 0, 0, 0);
         }
       }
     };
-    const int kb_first = (key_lo / 32) * 32;
     wait_loads_but<0>();         // (a stage past the end of the pass before may still be on its way into a buffer)
     lds_barrier();               // the previous pass has finished reading the buffers; the table is in LDS
-    sc_.copy(kb_first, kb_last, 0);
-    sc_.copy(kb_first + 32, kb_last, 1);
-    wait_loads_but<SC::LOADS>();
+    const auto after = [&](int kb) { return MOD && kb + 32 == kept_end ? kb_first : kb + 32; };
+    int ask = kept_end > 0 ? 0 : kb_first;                     // the next stage to ask for
+#pragma unroll
+    for (int i = 0; i < SC::AHEAD; ++i, ask = after(ask)) sc_.copy(ask, kb_last, i);
+    wait_loads_but<(SC::AHEAD - 1) * SC::LOADS>();
     lds_barrier();
     int buf = 0;
-    for (int kb = kb_first; kb < kb_last; kb += 32) {          // every stage before the last one
-      sc_.copy(kb + 64, kb_last, SC::before(buf));             // two stages on, into the buffer read a stage ago
-      stage(std::false_type{}, kb, buf);
-      wait_loads_but<SC::LOADS>();                             // the next stage has landed (this wave's share of it)
+    for (int kb = kept_end > 0 ? 0 : kb_first; kb < kb_last; kb = after(kb)) {   // every stage before the last one
+      sc_.copy(ask, kb_last, SC::before(buf));                 // into the buffer read a stage ago
+      ask = after(ask);
+      if (MOD && kb < kept_end) stage(std::true_type{}, kb, buf, kept - 1);
+      else stage(std::false_type{}, kb, buf, 0);
+      wait_loads_but<(SC::AHEAD - 1) * SC::LOADS>();           // the next stage has landed (this wave's share of it)
       lds_barrier();
       buf = SC::after(buf);
     }
-    stage(std::true_type{}, kb_last, buf);
+    stage(std::true_type{}, kb_last, buf, key_hi);
     float lt = l + __shfl_xor(l, 32, WAVE);
     if (valid) {
       lt = with_sink(a, token, head, lt, m);
@@ -1911,12 +1949,35 @@ static int prefill_launch(const void* q, void* out, const void* pages, const int
   const TileMap tm = tile_map(heads / kv_heads);
   const int tiles = (max_query + tm.pos_per_tile - 1) / tm.pos_per_tile;
   if (mod != nullptr) {
-    // changed scores: the kernel that reads its operands from the cache, one tile a wave under a window (a wave then
-    // walks its own tile's window and no other's), two without
     HOLON_CHECK(mod->softcap >= 0.f && mod->keep_first >= 0 && (mod->r1 == nullptr) == (mod->r2 == nullptr),
                 "attention: a cap of %g, %d kept tokens, a distance bias of two numbers a head", mod->softcap,
                 mod->keep_first);
     a.scale = scale; a.softcap = mod->softcap; a.r1 = mod->r1; a.r2 = mod->r2; a.keep_first = mod->keep_first;
+  }
+  // Heads of 256, and changed scores at 128: stages copied into LDS too (below, with the pairs of ranges), where that is the
+  // faster form. Heads of 256 over one kv head, from rows of about 200 tokens on (us, operands straight from the cache
+  // against staged): four prompts of 600 to 1,321 tokens of 32 heads 401 against 159, one of 4,096 behind 4,096 (16 heads
+  // over 2) 1,721 and 471 (0.88 PFLOP/s), 64 tokens behind 1,000 80 and 61, prompts of 128 / 256 tokens 15.8 / 24.7 and 16.6 /
+  // 22.6. Changed scores (a cap of 30, a window of 1,024 with a distance bias) from 384 ranges on, four waves of 32 rows each:
+  // the scores' arithmetic is what they take, and fewer blocks leave it to fewer waves than tiles of 16 rows do. 16 heads over
+  // 4, one prompt of 4,000 tokens 172 and 105, of 1,000 53 and 72; 32 over 8, three of 1,300 241 and 148, one of 1,000 79 and 72.
+  const TileMap32 few = tile_map32(heads / kv_heads);
+  const int64_t few_ranges = (int64_t)(((max_query + few.pos_per_tile - 1) / few.pos_per_tile + 3) / 4) * kv_heads * n_rows;
+  if (g_prefill_dma && heads / kv_heads <= 32 && tiles >= 16 && max_len <= 4096 * page_size &&
+      (mod != nullptr ? head_dim == 128 && few_ranges >= 384 : head_dim == 256 && max_len > 192)) {
+    const TileMap32 tm32 = tile_map32(heads / kv_heads);
+    const int ranges32 = ((max_query + tm32.pos_per_tile - 1) / tm32.pos_per_tile + 3) / 4;
+    a.unpaired = (int64_t)((ranges32 + 1) / 2) * kv_heads * n_rows < UNPAIR_BELOW ? 1 : 0;
+    dim3 lgrid(kv_heads, (ranges32 + 1) / 2, a.unpaired ? 2 * n_rows : n_rows);
+    hipStream_t ls = (hipStream_t)stream;
+    if (mod == nullptr) attn_prefill_dma_kernel<256, false><<<lgrid, 256, 0, ls>>>(a);
+    else attn_prefill_dma_kernel<128, true><<<lgrid, 256, 0, ls>>>(a);
+    HOLON_LAUNCH_OK();
+    return 0;
+  }
+  if (mod != nullptr) {
+    // changed scores: the kernel that reads its operands from the cache, one tile a wave under a window (a wave then
+    // walks its own tile's window and no other's), two without
     const int mnt = head_dim == 256 || window != 0 ? 1 : 2;
     dim3 grid(((tiles + mnt - 1) / mnt + 3) / 4, kv_heads * tm.head_blocks, n_rows);
     hipStream_t ms = (hipStream_t)stream;
@@ -1954,7 +2015,7 @@ static int prefill_launch(const void* q, void* out, const void* pages, const int
       // same XCD and finds the keys its neighbours have just read in that XCD's L2 (behind 28,672 tokens 2,246 -> 2,119 us)
       dim3 lgrid(kv_heads, (ranges32 + 1) / 2, a.unpaired ? 2 * n_rows : n_rows);
       if (head_dim == 64) attn_prefill_wide_kernel<64><<<lgrid, 256, 0, ls>>>(a);
-      else if (direct) attn_prefill_dma_kernel<<<lgrid, 256, 0, ls>>>(a);
+      else if (direct) attn_prefill_dma_kernel<128, false><<<lgrid, 256, 0, ls>>>(a);
       else attn_prefill_wide_kernel<128><<<lgrid, 256, 0, ls>>>(a);
     } else if (blocks2 >= 512) {
       dim3 lgrid((ranges2 + 1) / 2, kv_heads * tm.head_blocks, n_rows);

@@ -312,6 +312,30 @@ def test_long_prompt_portions_two_tiles_a_wave(hip, geometry):
             assert torch.equal(got, again)
 
 
+@pytest.mark.parametrize("geometry", [(32, 1), (5, 1), (6, 2), (4, 4)])
+def test_prompt_portions_of_wide_heads(hip, geometry):
+    """Heads of 256 with stages copied into LDS (rows of more than 192 tokens), and straight from the cache: whole prompts, rows
+    behind earlier tokens, a window, last stages of 1 to 32 keys; every stretch of rows within the budget of the keys it sees."""
+    (heads, kv_heads), bf, head_dim = geometry, torch.bfloat16, 256
+    for rows, window in (([(0, 193)], 0), ([(0, 417), (300, 33)], 0), ([(415, 129), (0, 224), (31, 16)], 100), ([(1000, 17)], 0)):
+        q, pages, table, attn = _paged_case(rows, heads, kv_heads, head_dim, 16, bf, seed=len(rows) + window)
+        want = PLAIN.paged_attention(q.double(), pages.double(), table, attn, 16, head_dim ** -0.5, window)
+        for direct in (1, 0):
+            copies = hip.lib.holon_attention_prefill_copies(direct)
+            try:
+                got = hip.paged_attention(q, pages, table, attn, 16, head_dim ** -0.5, window)
+            finally:
+                hip.lib.holon_attention_prefill_copies(copies)
+            at = 0
+            for start, n in rows:
+                for lo, hi in ((0, 64), (64, n)):
+                    part = slice(at + lo, at + min(hi, n))
+                    if lo < n:
+                        span = head_dim + (min(window, start + hi) if window else start + min(hi, n))
+                        assert H.op_budget_usage(got[part], want[part], bf, span) <= 1, (geometry, rows, window, lo, direct)
+                at += n
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window", [1, 7, 16, 100])
 def test_paged_attention_window(hip, dtype, window):

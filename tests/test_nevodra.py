@@ -195,6 +195,60 @@ def test_changed_scores_on_the_matrix_cores(dim):
         assert per < 4e-2, (dim, window, keep, cap, per)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,groups", [(32, 32), (48, 16), (64, 16)])
+def test_changed_scores_over_staged_keys(heads, groups):
+    """Portions of enough ranges for the kernel that copies stages into LDS, heads of 128: whole prompts and rows behind earlier
+    tokens, kept first tokens before the window's stages and inside them, a cap alone, and pages that the row no longer holds
+    full of NaN. Against the plain form in float64, and against the kernel that reads its operands from the cache."""
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.api import AttnRows
+    k, dev, page, dim = load_hip(), "cuda", 16, 128
+    g = torch.Generator().manual_seed(heads)
+    lens, counts = [330, 75, 300, 577], [330, 75, 33, 260]
+    n_pages = sum(-(-n // page) for n in lens) + 1
+    table = torch.full((len(lens), 40), n_pages - 1, dtype=torch.int32)
+    order, at = torch.randperm(n_pages - 1, generator=g).tolist(), 0
+    for s_, n in enumerate(lens):
+        for i in range(-(-n // page)):
+            table[s_, i] = order[at]
+            at += 1
+    full = (torch.randn(n_pages, 2, groups, page * dim, generator=g) * 0.5).bfloat16()
+    qstart = [0]
+    for c in counts:
+        qstart.append(qstart[-1] + c)
+    q = torch.randn(qstart[-1], heads, dim, generator=g).to(dev).bfloat16()
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)          # noqa: E731
+    rows = AttnRows(slots=i32([0, 1, 2, 3]), lens=i32(lens), query_start=i32(qstart), decode_rows=i32([]), chunk_rows=i32([0, 1, 2, 3]),
+                    n_decode=0, n_chunk=4, max_decode_len=0, max_chunk_query=max(counts), max_chunk_len=max(lens))
+    r1, r2 = torch.rand(heads, generator=g).to(dev), (2 * torch.rand(heads, generator=g)).to(dev)
+    sink = torch.randn(heads, generator=g).to(dev)
+    twin, scale = TorchKernels(), 2.0 * dim ** -0.5
+    for window, keep, cap, dist, sk in ((0, 0, 3.0, (r1, r2), None), (40, 5, 3.0, (r1, r2), sink), (100, 64, 0.0, None, None),
+                                        (33, 70, 2.0, (r1, r2), None), (64, 1, 0.0, (r1, r2), None), (17, 32, 5.0, None, sink)):
+        pages = full.clone()
+        if window:             # whole blocks of 32 keys between the kept keys and the window, and the rest of the kept keys' block
+            for b, (n, c) in enumerate(zip(lens, counts)):
+                for i in range(-(-keep // page), max(0, n - c - window + 1) // 32 * 32 // page):
+                    pages[table[b, i]] = float("nan")
+        pages = pages.to(dev)
+        both = []
+        for direct in (1, 0):
+            was = k.lib.holon_attention_prefill_copies(direct)
+            try:
+                both.append(k.paged_attention(q, pages, table.to(dev), rows, page, scale, window, sink=sk, softcap=cap, dist=dist,
+                                              keep_first=keep))
+            finally:
+                k.lib.holon_attention_prefill_copies(was)
+        want = twin.paged_attention(q.double(), full.to(dev).double(), table.to(dev), rows, page, scale, window,
+                                    sink=None if sk is None else sk.double(), softcap=cap,
+                                    dist=None if dist is None else (dist[0].double(), dist[1].double()), keep_first=keep)
+        for got in both:
+            assert H.rel_rms(got, want) < 8e-3, (window, keep, cap)
+            per = ((got.double() - want).square().mean((1, 2)).sqrt() / want.square().mean().sqrt()).max().item()
+            assert per < 4e-2, (window, keep, cap, per)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 def test_the_stream_after_every_layer_run(folders, device):
     """The residual stream after each run of a layer (a repeated layer counts each time), float32, against the plain

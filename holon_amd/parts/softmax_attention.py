@@ -75,6 +75,14 @@ def softmax_attention_plain(q, pages, table, rows, token_row, positions, kv_head
     return out.view(t, heads * vdim).to(q.dtype)
 
 
+def _float64_sums_serve(heads, kv_heads, dim, vdim, page_size):
+    """What the library's `holon_softmax_attention_f64_supported` answers. That kernel takes float32 steps that bring 16 tokens a row
+    or more, at least 64 in all (measured, us, against the general one: 8 tokens a row of 16 rows, 16 heads of 128 on 4, 13.7 and
+    15.2, each head its own keys 20.7 and 15.5; one row of 37 tokens 30.7 and 12.6, of 65 14.9 and 16.8, of 700 106 and 407)."""
+    return dim == vdim and dim in (64, 128) and page_size % 16 == 0 and heads % kv_heads == 0 \
+        and kv_heads * -(-(heads // kv_heads) // 16) <= 65535
+
+
 def _softmax_attention_hip(launch, q, pages, table, rows, token_row, positions, kv_heads, vdim, page_size, sink,
                            scale, window, softcap=0.0, dist=None, keep_first=0, value_share=1):
     t, heads, dim = q.shape
@@ -91,7 +99,11 @@ def _softmax_attention_hip(launch, q, pages, table, rows, token_row, positions, 
         raise ValueError(f"softmax_attention: q {tuple(q.shape)} {q.dtype}, pages {tuple(pages.shape)} do not fit "
                          f"{kv_heads} kv heads, values of {vdim}, page {page_size}")
     out = torch.empty((t, heads * vdim), dtype=q.dtype, device=q.device)
-    launch(q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), table.shape[1], table.shape[0],
+    general, wide = launch
+    kernel = wide if q.dtype == torch.float32 and t >= 64 and t >= 16 * rows.slots.shape[0] and not (window > 0 and keep_first > 0) \
+        and _float64_sums_serve(heads, kv_heads, dim, vdim, page_size) and q.data_ptr() % 16 == 0 and pages.data_ptr() % 16 == 0 \
+        else general
+    kernel(q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), table.shape[1], table.shape[0],
            rows.slots.data_ptr(), token_row.data_ptr(), positions.data_ptr(), t, heads, kv_heads, dim, vdim, page_size,
            pages.shape[0], _ptr(sink), float(scale), int(window), _DT[q.dtype], float(softcap),
            _ptr(dist[0]) if dist is not None else None, _ptr(dist[1]) if dist is not None else None, int(keep_first),
@@ -387,9 +399,9 @@ def _add_bias_hip(launch, x, bias):
     return x
 
 
-register_kernel(KernelOp("softmax_attention", softmax_attention_plain, "holon_softmax_attention",
-                         [_P, _P, _P, _P, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _F, _I, _I, _F, _P, _P, _I, _I],
-                         _softmax_attention_hip))
+_SOFTMAX = [_P, _P, _P, _P, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _F, _I, _I, _F, _P, _P, _I, _I]
+register_kernel(KernelOp("softmax_attention", softmax_attention_plain, ("holon_softmax_attention", "holon_softmax_attention_f64"),
+                         (_SOFTMAX, _SOFTMAX), _softmax_attention_hip))
 register_kernel(KernelOp("head_linear", head_linear_plain, ("holon_head_linear_rows", "holon_head_linear_bf16"),
                          ([_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _L], [_P, _P, _P, _I, _I, _I, _I, _I, _P, _L]),
                          _head_linear_hip))

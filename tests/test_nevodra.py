@@ -592,6 +592,62 @@ def test_graph_replays_equal_eager_steps(folders, name, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,groups,dim,page,share", [(16, 4, 128, 16, 1), (4, 4, 64, 32, 2), (6, 2, 128, 48, 1), (40, 2, 64, 16, 1)])
+def test_float32_prompts_on_the_float64_cores(heads, groups, dim, page, share):
+    """`softmax_attention` over float32 portions of 16 tokens a row or more: rows that meet inside a block, a row of one token among
+    them, windows, chunks, every option, against the plain form in float64 (sums in float64, scores and weights rounded to
+    float32: 2^-23 of a score of some 10 moves a weight by 1e-6). A token's result does not depend on the rows beside it, and a key
+    or value that is not finite stays out of the tokens that do not see it."""
+    import holon_amd.parts  # noqa: F401
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.api import AttnRows
+    from holon_amd.kernels.registry import kernel_op
+    k, dev = load_hip(), "cuda"
+    g = torch.Generator().manual_seed(dim + heads)
+    lens, counts = [130, 75, 33, 301], [130, 18, 1, 77]
+    n_pages = sum(-(-n // page) for n in lens)
+    order, at = torch.randperm(n_pages, generator=g).tolist(), 0
+    table = torch.full((6, -(-400 // page)), -1, dtype=torch.int32)
+    for b, n in enumerate(lens):
+        for i in range(-(-n // page)):
+            table[5 - b, i] = order[at]
+            at += 1
+    pages = torch.randn(n_pages, (groups + groups // share) * page * dim, generator=g).to(dev)
+    q, i32 = torch.randn(sum(counts), heads, dim, generator=g).to(dev), lambda v: torch.tensor(v, dtype=torch.int32, device=dev)   # noqa: E731
+    rows = AttnRows(slots=i32([5, 4, 3, 2]), lens=i32(lens), query_start=i32([0, 130, 148, 149, 226]), decode_rows=i32([2]),
+                    chunk_rows=i32([0, 1, 3]), n_decode=1, n_chunk=3, max_decode_len=33, max_chunk_query=130, max_chunk_len=301)
+    token_row = i32([b for b, c in enumerate(counts) for _ in range(c)])
+    positions = i32([n - c + i for n, c in zip(lens, counts) for i in range(c)])
+    r1, r2 = torch.rand(heads, generator=g).to(dev), (2 * torch.rand(heads, generator=g)).to(dev)
+    sink = torch.randn(heads, generator=g).to(dev)
+    table, op = table.to(dev), kernel_op("softmax_attention").plain
+    for window, cap, dist, sk in ((0, 0.0, None, None), (40, 3.0, (r1, r2), sink), (-64, 0.0, None, sink), (17, 0.0, (r1, r2), None)):
+        args = (table, rows, token_row, positions, groups, dim, page, sk, dim ** -0.5, window)
+        more = dict(softcap=cap, value_share=share)
+        got = k.softmax_attention(q, pages, *args, dist=dist, **more)
+        want = op(q.double(), pages.double(), *args[:7], None if sk is None else sk.double(), *args[8:],
+                  dist=None if dist is None else (dist[0].double(), dist[1].double()), **more)
+        assert H.rel_rms(got, want) < 2e-6, (window, cap)
+        # the last row's tokens by themselves
+        alone = AttnRows(slots=i32([2]), lens=i32([301]), query_start=i32([0, 77]), decode_rows=i32([]), chunk_rows=i32([0]), n_decode=0,
+                         n_chunk=1, max_decode_len=0, max_chunk_query=77, max_chunk_len=301)
+        one = k.softmax_attention(q[149:].contiguous(), pages, table, alone, i32([0] * 77), positions[149:].contiguous(), *args[4:],
+                                  dist=dist, **more)
+        assert torch.equal(one, got[149:]), (window, cap)
+        for value in (float("nan"), float("inf")):
+            for key in (250, 266):                                           # a value of the last row: its tokens from key on see it
+                spoilt = pages.clone()
+                at = (groups + 0) * page * dim + 3 * page + key % page        # (the first value head's dimension 3)
+                spoilt[table[2, key // page], at] = value
+                bad = k.softmax_attention(q, spoilt, *args, dist=dist, **more)
+                tokens = torch.arange(149, 226, device=dev)
+                pos = positions[149:]
+                sees = (pos >= key) & ((pos - key < window) if window > 0 else (pos // -window == key // -window) if window < 0 else pos >= 0)
+                assert torch.equal(bad[tokens[~sees]], got[tokens[~sees]]) and torch.equal(bad[:149], got[:149]), (window, key)
+                assert not torch.isfinite(bad[tokens[sees], 3]).any() and torch.isfinite(bad[tokens[sees], 4]).all(), (window, key)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_kernels_alone_against_their_plain_forms(dtype):
     """Every operation the design brought, on the GPU, against its plain form in torch: odd widths, rows wider than a

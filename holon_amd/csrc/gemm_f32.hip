@@ -11,61 +11,11 @@
 //
 // A lane of a matrix instruction's operand holds one float of row lane % 16; here it reads four neighbours in k at once
 // (16 bytes, k = 4 (lane / 16) .. + 3 of a group) and spends them on four instructions.
-#include "common.h"
+#include "gemm_f32.h"
 #include "holon_hip.h"
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
 namespace {
-constexpr int SHARES = 16, QUARTERS = 4;
-constexpr int GROUP = 16;              // k values of one 16-byte load of every lane
-constexpr int CHUNK = 32;              // k values staged at a time, and what shares are a multiple of
-
-constexpr int SHORTEST = 64;           // a share's least length: up to 1,024 of K fewer waves share it
-
-__host__ __device__ __forceinline__ int share_length(int K) {
-  const int even = (K + SHARES * CHUNK - 1) / (SHARES * CHUNK) * CHUNK;
-  return even > SHORTEST ? even : SHORTEST;
-}
-
-// s[0] .. s[15] in the order above.
-template <typename F>
-__device__ __forceinline__ f32x4_t sum_shares(F s) {
-  f32x4_t total;
-#pragma unroll
-  for (int q = 0; q < QUARTERS; ++q) {
-    f32x4_t quarter = s(4 * q);
-#pragma unroll
-    for (int i = 1; i < 4; ++i) quarter += s(4 * q + i);
-    total = q ? total + quarter : quarter;
-  }
-  return total;
-}
-
-// Four results of a row, columns n .. n + 3.
-__device__ __forceinline__ void store4(float* __restrict__ y, f32x4_t v, int m, int n, int M, int N) {
-  if (m >= M) return;
-  float* out = y + (int64_t)m * N + n;
-  if (N % 4 == 0 && (uintptr_t)y % 16 == 0) {
-    if (n < N) *reinterpret_cast<f32x4_t*>(out) = v;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) if (n + i < N) out[i] = v[i];
-  }
-}
-
-// Four floats of a row at k. VEC: K is a multiple of 4 and rows are 16-byte aligned.
-template <bool VEC>
-__device__ __forceinline__ f32x4_t load4(const float* __restrict__ row, int k, int K) {
-  f32x4_t v = {0.f, 0.f, 0.f, 0.f};
-  if constexpr (VEC) {
-    if (k < K) v = *reinterpret_cast<const f32x4_t*>(row + k);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) if (k + i < K) v[i] = row[k + i];
-  }
-  return v;
-}
+using namespace f32_sums;
 
 // Steps of few rows. A block owns MT x NT tiles of 16 x 16 results; each of its 16 waves takes one share of K, and the waves' sums are added in
 // order through LDS. Operands go from memory straight to registers, DEPTH groups of k of a wave under way at a time; 16
@@ -91,26 +41,7 @@ __global__ void __launch_bounds__(SHARES * WAVE) gemm_f32_rows_kernel(const floa
   for (int t = 0; t < MT; ++t)
 #pragma unroll
     for (int u = 0; u < NT; ++u) acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = first; k0 < last; k0 += DEPTH * GROUP) {
-    f32x4_t a[DEPTH][NT], b[DEPTH][MT];
-#pragma unroll
-    for (int s = 0; s < DEPTH; ++s) {                     // (beyond the share: zeros, which add nothing)
-      const int k = k0 + s * GROUP + 4 * g;
-#pragma unroll
-      for (int u = 0; u < NT; ++u) a[s][u] = load4<VEC>(wr[u], k, last);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) b[s][t] = load4<VEC>(xr[t], k, last);
-    }
-#pragma unroll
-    for (int s = 0; s < DEPTH; ++s)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-#pragma unroll
-          for (int u = 0; u < NT; ++u)
-            acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][u][i], b[s][t][i], acc[t][u], 0, 0, 0);
-  }
+  share_sums<MT, NT, DEPTH, VEC>(acc, wr, xr, first, last);
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -122,126 +53,38 @@ __global__ void __launch_bounds__(SHARES * WAVE) gemm_f32_rows_kernel(const floa
   store4(y, sum, m0 + wave / NT * 16 + c, n0 + wave % NT * 16 + 4 * g, M, N);
 }
 
-// More rows: bound by the matrix cores. A block owns 64 x 64 results; four waves (32 x 32 each) walk a run of K whose rows of x and
-// w they stage in LDS, CHUNK of k at a time, into one of two buffers while the other is multiplied; pieces of 16 bytes lie at
-// place p ^ (row % 8) of their row. SIDE 4: sixteen waves, the four quarters of K side by side: what fills the chip where an output of
-// some hundred rows has few tiles, four waves a SIMD covering each other's barriers. SIDE 1: four waves, the quarters one after the
-// other: several blocks share a unit, so that one's first loads and its stores lie under the others' products; that is the better
-// one where there are tiles for it, the more the shorter K. Either ends at K (what lies behind it would add zeros).
+// Up to 16 rows over at most 128 tiles of 16 columns, which a block each leave half the compute units idle: a block half a tile. Tiles
+// against halves at 1 / 16 rows, us: 2048 x 2048 7.4 / 10.4 and 6.3 / 9.2, 2048 x 8192 27.6 / 38.5 and 20.2 / 28.7, 2048 x 18432 55 / 85
+// and 44 / 59; of 192 tiles (3072 x 2048) 9.2 / 12.5 and 10.8 / 14.3. More loads under way change nothing in either form.
+constexpr int HALF_TILES = 128;
+template <int DEPTH, bool VEC>
+__global__ void __launch_bounds__(SHARES * WAVE) gemm_f32_half_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                  float* __restrict__ y, int M, int N, int K) {
+  __shared__ f32x4_t part[SHARES][WAVE];
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int g = lane / 16, c = lane % 16, n0 = blockIdx.x * 8, share = share_length(K);
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  half_sums<DEPTH, VEC>(acc, w + (int64_t)min(n0 + c % 8, N - 1) * K, x + (int64_t)min(c, M - 1) * K, wave * share,
+                        min(K, (wave + 1) * share));
+  part[wave][lane] = acc;
+  __syncthreads();
+  if (wave > 0 || g > 1) return;
+  const f32x4_t sum = sum_shares([&](int i) { return part[i][lane]; });
+  store4(y, sum, c, n0 + 4 * g, M, N);
+}
+
 template <int SIDE, bool VEC>
 __global__ void __launch_bounds__(SIDE * 256) gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                               float* __restrict__ y, int M, int N, int K) {
-  __shared__ __attribute__((aligned(16))) float stage[SIDE][2][2][64 * CHUNK];       // quarter, buffer, x or w
-  const int quarter = SIDE > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / 256) : 0, tid = threadIdx.x % 256;
-  const int wave = tid / WAVE, lane = tid % WAVE;
-  const int g = lane / 16, c = lane % 16;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int share = share_length(K), first = quarter * 4 * share, per_share = share / CHUNK;
-  const int chunks = (min(K, (SIDE > 1 ? 4 : 16) * share) + CHUNK - 1) / CHUNK;      // (of the block: the first quarter's)
-  // what this thread stages: rows tid / 8 and 32 more, piece tid % 8
-  const int r0 = tid / 8, p0 = tid % 8;
+  __shared__ __attribute__((aligned(16))) Stage<SIDE> stage;
+  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64, r0 = threadIdx.x % 256 / 8;
   const float *xr[2], *wr[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     xr[i] = x + (int64_t)min(m0 + r0 + 32 * i, M - 1) * K;
     wr[i] = w + (int64_t)min(n0 + r0 + 32 * i, N - 1) * K;
   }
-  const int put = r0 * CHUNK + 4 * (p0 ^ (r0 % 8));
-  f32x4_t held[2][2];
-  auto fetch = [&](int chunk) {
-    const int k = first + chunk * CHUNK + 4 * p0;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      held[0][i] = load4<VEC>(xr[i], k, K);
-      held[1][i] = load4<VEC>(wr[i], k, K);
-    }
-  };
-  auto keep = [&](int buf) {
-#pragma unroll
-    for (int o = 0; o < 2; ++o)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4_t*>(&stage[quarter][buf][o][put + 32 * i * CHUNK]) = held[o][i];
-  };
-  // where this lane reads: row 32 (half) + 16 t + c, pieces g and 4 + g
-  const int xrow = wave / 2 * 32 + c, wrow = wave % 2 * 32 + c;
-  const int at[2] = {4 * (g ^ (c % 8)), 4 * ((4 + g) ^ (c % 8))};
-  // the sums of a share, of a quarter's shares so far (SIDE 1), and of all that is behind them
-  f32x4_t acc[2][2], part[SIDE > 1 ? 1 : 2][2], total[2][2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int u = 0; u < 2; ++u) acc[t][u] = total[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  int left = per_share, shares = 0;
-  const auto end_share = [&]() {
-    const bool begins = SIDE > 1 ? shares == 0 : shares % 4 == 0, ends = shares % 4 == 3, first_quarter = shares < 4;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        if constexpr (SIDE > 1) {
-          total[t][u] = begins ? acc[t][u] : total[t][u] + acc[t][u];
-        } else {
-          part[t][u] = begins ? acc[t][u] : part[t][u] + acc[t][u];
-          if (ends) total[t][u] = first_quarter ? part[t][u] : total[t][u] + part[t][u];
-        }
-        acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      }
-    left = per_share;
-    ++shares;
-  };
-  fetch(0);
-  keep(0);
-  if (chunks > 1) fetch(1);
-  lds_barrier();
-  for (int ch = 0; ch < chunks; ++ch) {
-    if (ch + 1 < chunks) keep((ch + 1) & 1);              // (read last in front of the barrier behind us)
-    if (ch + 2 < chunks) fetch(ch + 2);
-    if (SIDE == 1 || first + ch * CHUNK < K) {
-      const float* xs = stage[quarter][ch & 1][0];
-      const float* ws = stage[quarter][ch & 1][1];
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        f32x4_t b[2], a[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) b[t] = *reinterpret_cast<const f32x4_t*>(&xs[(xrow + 16 * t) * CHUNK + at[s]]);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) a[u] = *reinterpret_cast<const f32x4_t*>(&ws[(wrow + 16 * u) * CHUNK + at[s]]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-              acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[t][i], acc[t][u], 0, 0, 0);
-      }
-      if (--left == 0) end_share();
-    }
-    lds_barrier();                                        // (what was fetched stays under way)
-  }
-  if (left < per_share) end_share();                      // (K ends inside a share)
-  if constexpr (SIDE > 1) {
-    // the quarters' sums through LDS: tile (4 t' + u') of the block's 16, one a wave
-    f32x4_t(*sums)[16][WAVE] = reinterpret_cast<f32x4_t(*)[16][WAVE]>(&stage[0][0][0][0]);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) sums[quarter][(wave / 2 * 2 + t) * 4 + wave % 2 * 2 + u][lane] = total[t][u];
-    __syncthreads();
-    const int tile = quarter * 4 + wave;
-    f32x4_t sum = sums[0][tile][lane];
-#pragma unroll
-    for (int q = 1; q < QUARTERS; ++q) sum += sums[q][tile][lane];
-    store4(y, sum, m0 + tile / 4 * 16 + c, n0 + tile % 4 * 16 + 4 * g, M, N);
-  } else {
-    const bool pending = shares % 4 != 0, only = shares < 4;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const f32x4_t sum = pending ? (only ? part[t][u] : total[t][u] + part[t][u]) : total[t][u];
-        store4(y, sum, m0 + (wave / 2 * 2 + t) * 16 + c, n0 + (wave % 2 * 2 + u) * 16 + 4 * g, M, N);
-      }
-  }
+  tile_sums<SIDE, VEC>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) { store4(y, sum, m0 + row, n0 + column, M, N); });
 }
 
 // Long sums into many columns: one running sum over k = 0, 1, 2, ... (v_mfma_f32_32x32x2_f32 adds its two k one after the
@@ -350,7 +193,10 @@ void launch(const float* x, const float* w, float* y, int M, int N, int K, hipSt
   const int best = pick_form(M, N, K);
   const dim3 grid((N + 16 * FORMS[best].nt - 1) / (16 * FORMS[best].nt), (M + 16 * FORMS[best].mt - 1) / (16 * FORMS[best].mt));
   switch (best) {
-    case 0: gemm_f32_rows_kernel<1, 1, 2, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
+    case 0:
+      if (M <= 16 && (N + 15) / 16 <= HALF_TILES) gemm_f32_half_kernel<2, VEC><<<(N + 7) / 8, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K);
+      else gemm_f32_rows_kernel<1, 1, 2, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K);
+      break;
     case 1: gemm_f32_rows_kernel<1, 2, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
     case 2: gemm_f32_rows_kernel<2, 2, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
     case 3: gemm_f32_rows_kernel<2, 4, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;

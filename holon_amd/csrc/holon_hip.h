@@ -431,6 +431,10 @@ int holon_moe_rows_supported(int rows, int hidden, int experts, int top, int ff,
 int holon_moe_rows_bf16(const void* x, const void* up, const void* down, void* y, int* lists, void* act, float* parts, int rows,
                         int hidden, int experts, int top, int ff, int shared, int gated, const float* weights, int wstride,
                         int shared_col, void* stream);
+// The same in float32, few rows and many, over the projections as they come.
+int holon_moe_f32_supported(int rows, int hidden, int experts, int top, int ff, int shared);
+int holon_moe_f32(const void* x, const void* up, const void* down, void* y, int* lists, void* act, float* parts, int rows, int hidden,
+                  int experts, int top, int ff, int shared, int gated, const float* weights, int wstride, int shared_col, void* stream);
 // up [rows, C], C = experts ff + shared: y = max(up, 0)^2 times the weight of the column's expert (as for holon_moe_gate).
 int holon_moe_relu2(const void* up, const float* weights, void* y, int64_t rows, int experts, int ff, int shared, int dtype,
                     int wstride, int shared_col, void* stream);

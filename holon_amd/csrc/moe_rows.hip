@@ -17,92 +17,11 @@
 #include "common.h"
 #include "gemm_block.h"
 #include "holon_hip.h"
+#include "moe_lists.h"
 
 namespace {
 using namespace block_gemm;
-constexpr int MAX_EXPERTS = 1024, MAX_TOP = 256;
-constexpr int TOKEN_BITS = 22;                       // a list's entry: the row, and above it the place among the row's choices
-constexpr int LIST_THREADS = 1024;
-
-struct MoeRows {
-  const float* weights;                              // [rows, stride]: 0 where a row did not choose an expert
-  int stride, rows, hidden, experts, top, ff, shared, shared_col;   // shared_col < 0: the shared expert's weight is 1
-  int* counts;                                       // [experts] rows that chose it
-  int* lists;                                        // [experts, rows]
-  int* slots;                                        // [rows, top] where a row's parts lie, -1: it made fewer choices
-};
-
-// Blocks of `experts`: an expert's list. The rest: what rows of fewer choices than `top` leave over. (No more than `top` of a
-// row's weights are taken, so that the lists hold rows * top entries at most whatever the weights are.)
-__global__ void __launch_bounds__(LIST_THREADS) moe_lists_kernel(MoeRows p) {
-  __shared__ int sums[LIST_THREADS / WAVE];
-  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-  if ((int)blockIdx.x >= p.experts) {
-    const int t = (blockIdx.x - p.experts) * LIST_THREADS + threadIdx.x;
-    if (t >= p.rows) return;
-    int n = 0;
-    for (int e = 0; e < p.experts; ++e) n += p.weights[(int64_t)t * p.stride + e] != 0.f;
-    for (int j = n; j < p.top; ++j) p.slots[(int64_t)t * p.top + j] = -1;
-    return;
-  }
-  const int e = blockIdx.x;
-  int total = 0;
-  for (int t0 = 0; t0 < p.rows; t0 += LIST_THREADS) {
-    const int t = t0 + threadIdx.x;
-    int place = 0;
-    bool mine = t < p.rows && p.weights[(int64_t)t * p.stride + e] != 0.f;
-    if (mine) {
-      for (int before = 0; before < e; ++before) place += p.weights[(int64_t)t * p.stride + before] != 0.f;
-      mine = place < p.top;
-    }
-    const uint64_t mask = __ballot(mine);
-    if (lane == 0) sums[wave] = __popcll(mask);
-    __syncthreads();
-    int at = total, all = 0;
-    for (int w = 0; w < LIST_THREADS / WAVE; ++w) {
-      if (w < wave) at += sums[w];
-      all += sums[w];
-    }
-    if (mine) p.lists[(int64_t)e * p.rows + at + __popcll(mask & ((1ull << lane) - 1))] = t | place << TOKEN_BITS;
-    total += all;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) p.counts[e] = total;
-}
-
-struct RowTile {
-  int expert, first, count, row0;                    // the expert's rows come from `first` on; this tile's from row0 of them
-};
-
-// Row tiles of all experts together, and (tile >= 0) which expert's the given one is. Every lane of a wave calls it.
-__device__ __forceinline__ int find_rows(const MoeRows& p, int tile, RowTile& out) {
-  const int lane = threadIdx.x % WAVE;
-  int tiles = 0, rows = 0;
-  for (int e0 = 0; e0 < p.experts; e0 += WAVE) {
-    const int count = e0 + lane < p.experts ? p.counts[e0 + lane] : 0;
-    int t = (count + TILE - 1) / TILE, r = count;
-#pragma unroll
-    for (int o = 1; o < WAVE; o *= 2) {              // sums up to this lane's expert
-      const int t_before = __shfl_up(t, o, WAVE), r_before = __shfl_up(r, o, WAVE);
-      if (lane >= o) t += t_before, r += r_before;
-    }
-    if (tile >= 0) {
-      const uint64_t past = __ballot(tiles + t > tile);
-      if (past != 0) {
-        const int at = __builtin_ctzll(past);
-        out.expert = e0 + at;
-        out.count = __builtin_amdgcn_readlane(count, at);
-        out.first = rows + __builtin_amdgcn_readlane(r, at) - out.count;
-        out.row0 = (tile - tiles - (__builtin_amdgcn_readlane(t, at) - (out.count + TILE - 1) / TILE)) * TILE;
-        return 0;
-      }
-    }
-    tiles += __builtin_amdgcn_readlane(t, WAVE - 1);
-    rows += __builtin_amdgcn_readlane(r, WAVE - 1);
-  }
-  return tiles;
-}
-
+using namespace moe_lists;
 // act of an expert's rows (routed: [rows * top, ff] in the order of the lists) and of the shared expert ([rows, shared]).
 template <bool GATED>
 __global__ void __launch_bounds__(THREADS, 2) moe_up_rows_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
@@ -112,7 +31,7 @@ __global__ void __launch_bounds__(THREADS, 2) moe_up_rows_kernel(const bf16_t* _
   constexpr int COLS = GATED ? HALF : TILE;          // columns of act a tile gives
   const int K = p.hidden, cols = p.experts * p.ff + p.shared;
   RowTile rows;
-  const int routed = find_rows(p, -1, rows);
+  const int routed = find_rows<TILE>(p, -1, rows);
   const int per_routed = (p.ff + COLS - 1) / COLS, per_shared = (p.shared + COLS - 1) / COLS;
   const int shared_tiles = p.shared ? (p.rows + TILE - 1) / TILE : 0;
   const int tile = tile_of_block(blockIdx.x, routed * per_routed + shared_tiles * per_shared);
@@ -122,7 +41,7 @@ __global__ void __launch_bounds__(THREADS, 2) moe_up_rows_kernel(const bf16_t* _
   int rt, ct;
   if (is_routed) {
     row_and_column(tile - first, routed, per_routed, rt, ct);
-    find_rows(p, rt, rows);
+    find_rows<TILE>(p, rt, rows);
   } else {
     row_and_column(tile, shared_tiles, per_shared, rt, ct);
     rows = RowTile{p.experts, 0, p.rows, rt * TILE};
@@ -200,7 +119,7 @@ __global__ void __launch_bounds__(THREADS, 2) moe_down_rows_kernel(const bf16_t*
   const int N = p.hidden;
   const int64_t cols = (int64_t)p.experts * p.ff + p.shared;
   RowTile rows;
-  const int routed = find_rows(p, -1, rows), per = (N + TILE - 1) / TILE;
+  const int routed = find_rows<TILE>(p, -1, rows), per = (N + TILE - 1) / TILE;
   const int shared_tiles = p.shared ? (p.rows + TILE - 1) / TILE : 0;
   const int tile = tile_of_block(blockIdx.x, (routed + shared_tiles) * per);
   if (tile < 0) return;
@@ -208,7 +127,7 @@ __global__ void __launch_bounds__(THREADS, 2) moe_down_rows_kernel(const bf16_t*
   int rt, ct;
   if (is_routed) {
     row_and_column(tile - shared_tiles * per, routed, per, rt, ct);
-    find_rows(p, rt, rows);
+    find_rows<TILE>(p, rt, rows);
   } else {
     row_and_column(tile, shared_tiles, per, rt, ct);
     rows = RowTile{p.experts, 0, p.rows, rt * TILE};
@@ -248,37 +167,6 @@ __global__ void __launch_bounds__(THREADS, 2) moe_down_rows_kernel(const bf16_t*
     }
 }
 
-// y: a row's parts in the experts' order, the shared expert's last, rounded once. A thread 8 columns, as many loads under way
-// as there are parts: 4,096 rows of 4,096 with three parts each are bound by the 235 MB that are read and written.
-constexpr int ADD_AT_ONCE = 4;
-__global__ void __launch_bounds__(256) moe_add_parts_kernel(const float* __restrict__ parts, bf16_t* __restrict__ y, MoeRows p) {
-  const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (at >= (int64_t)p.rows * p.hidden) return;
-  const int row = (int)(at / p.hidden), column = (int)(at % p.hidden);
-  const int* slots = p.slots + (int64_t)row * p.top;
-  f32x4_t sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  for (int j0 = 0; j0 <= p.top; j0 += ADD_AT_ONCE) {
-    f32x4_t part[ADD_AT_ONCE][2];
-    bool have[ADD_AT_ONCE];
-#pragma unroll
-    for (int u = 0; u < ADD_AT_ONCE; ++u) {
-      const int j = j0 + u;
-      const int64_t slot = j < p.top ? slots[j] : (j == p.top && p.shared ? p.rows * (int64_t)p.top + row : -1);
-      have[u] = slot >= 0;
-      const float* from = parts + (have[u] ? slot : 0) * p.hidden + column;      // (some part, and not added)
-      part[u][0] = *reinterpret_cast<const f32x4_t*>(from);
-      part[u][1] = *reinterpret_cast<const f32x4_t*>(from + 4);
-    }
-#pragma unroll
-    for (int u = 0; u < ADD_AT_ONCE; ++u)
-      if (have[u]) sum[0] += part[u][0], sum[1] += part[u][1];
-  }
-  uint4 o;
-  bf16_t* oe = reinterpret_cast<bf16_t*>(&o);
-#pragma unroll
-  for (int v = 0; v < 8; ++v) oe[v] = float_to_bf16(sum[v / 4][v % 4]);
-  *reinterpret_cast<uint4*>(y + at) = o;
-}
 }  // namespace
 
 // Whether the products serve `rows` rows of `hidden`: sizes the loop's chunks divide, offsets that 32 bits hold.
@@ -313,11 +201,11 @@ extern "C" int holon_moe_rows_bf16(const void* x, const void* up, const void* do
   const int64_t up_tiles = routed * tiles(ff, cols) + tiles(rows, TILE) * tiles(shared, cols);
   const int64_t down_tiles = (routed + (shared ? tiles(rows, TILE) : 0)) * tiles(hidden, TILE);
   const auto blocks = [&](int64_t n) { return (unsigned)(tiles(n, XCDS) * XCDS); };      // every XCD as many
-  moe_lists_kernel<<<experts + (unsigned)tiles(rows, LIST_THREADS), LIST_THREADS, 0, s>>>(p);
+  make_lists(p, s);
   if (gated) moe_up_rows_kernel<true><<<blocks(up_tiles), THREADS, 0, s>>>((const bf16_t*)x, (const bf16_t*)up, act_routed, act_shared, p);
   else moe_up_rows_kernel<false><<<blocks(up_tiles), THREADS, 0, s>>>((const bf16_t*)x, (const bf16_t*)up, act_routed, act_shared, p);
   moe_down_rows_kernel<<<blocks(down_tiles), THREADS, 0, s>>>(act_routed, act_shared, (const bf16_t*)down, parts, p);
-  moe_add_parts_kernel<<<(unsigned)tiles((int64_t)rows * hidden, 2048), 256, 0, s>>>(parts, (bf16_t*)y, p);
+  add_parts(p, parts, (bf16_t*)y, s);
   HOLON_LAUNCH_OK();
   return 0;
 }

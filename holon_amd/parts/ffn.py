@@ -447,6 +447,67 @@ register_kernel(KernelOp("moe_rows", moe_rows_plain, "holon_moe_rows_bf16",
                          [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _I], _moe_rows_hip))
 
 
+def moe_f32_plain(x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
+    """The experts of the 32-bit path over the rows that chose them: the two products and the activation between them, the sums over
+    the experts cut at the experts; None where they are not served (the caller then composes the three). The plain form never does."""
+    return None
+
+
+def moe_f32_serves(rows: int, hidden: int, experts: int, top: int, ff: int, shared: int) -> bool:
+    """What the library's `holon_moe_f32_supported` answers (of sizes whose counts fit 31 bits)."""
+    return 1 <= rows < 1 << 22 and hidden > 0 and ff > 0 and not (hidden % 16 or ff % 16 or shared % 16) and 1 <= top <= experts <= 1024 \
+        and top <= 256 and (rows * top // 64 + experts + -(-rows // 64)) * (max(experts * ff + shared, hidden) // 32 + 1) < 1 << 31 \
+        and max(2 * (experts * ff + shared), experts * rows, rows * top) < 1 << 31
+
+
+def moe_f32_pays(rows: int, hidden: int, experts: int, ff: int, shared: int, gated: bool, top: int) -> bool:
+    """Whether a float32 step is done sooner over the rows that chose an expert than with all rows over all experts. Up to 16 rows: what
+    the weights that no row is expected to choose take at 3 TB/s against a start an expert chosen and the search for them. From 64 rows
+    on: tiles of 64 x 64 by their length and a start. Measured on MI355X, us, own rows / all: 8 experts of 2,048 x 2,048 (squared ReLU)
+    beside a shared one, 2 a row, at 1 / 4 / 12 / 64 / 700 rows 53 / 102 / 125 / 204 / 460 and 110 / 111 / 123 / 248 / 1,199; 8 of 1,024
+    (gated) beside one of 2,048, 4 a row, at 1 / 4 / 64 / 700 70 / 98 / 190 / 703 and 95 / 95 / 200 / 945; 64 of 512 x 1,024, 6 a row, at
+    4 / 16 / 700 93 / 212 / 294 and 156 / 194 / 1,629; 128 of 64 x 2,048, 8 a row, at 4 / 64 / 200 73 / 147 / 150 and 80 / 121 / 303."""
+    if rows <= 16:
+        left = experts * (1 - top / experts) ** rows
+        return left * ff * hidden * (12 if gated else 8) / 3e6 > 2 + 1.5 * (experts - left) + 0.01 * rows * experts
+    if rows < 64:
+        return False
+
+    def work(row_tiles, columns, tile, length):            # of products of `columns` columns, `tile` wide, over `length` of K
+        return row_tiles * -(-columns // tile) * (length + 200)
+    routed, whole, wide = max(min(experts, rows * top), rows * top / 64 + experts / 2), -(-rows // 64), 32 if gated else 64
+    cols = experts * ff + shared
+    own = work(routed, ff, wide, hidden) + work(routed, hidden, 64, ff)
+    own += (work(whole, shared, wide, hidden) + work(whole, hidden, 64, shared)) if shared else 0
+    return own < 1.12 * (work(whole, cols, wide, hidden) + work(whole, hidden, 64, cols))
+
+
+def _moe_f32_hip(launch, x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
+    t, hidden = x.shape
+    cols = experts * ff + shared
+    if x.dtype != torch.float32 or not moe_f32_serves(t, hidden, experts, top, ff, shared):
+        return None
+    _need(x.is_cuda and x.is_contiguous() and weights.is_contiguous() and weights.dtype == torch.float32
+          and tuple(weights.shape) == (t, experts + int(bool(shared_weight)))
+          and all(w.is_contiguous() and w.dtype == x.dtype and w.data_ptr() % 16 == 0 for w in (up, down)) and x.data_ptr() % 16 == 0
+          and tuple(up.shape) == ((2 if gated else 1) * cols, hidden) and tuple(down.shape) == (hidden, cols),
+          f"moe_f32: rows {tuple(x.shape)}, weights {tuple(weights.shape)}, projections {tuple(up.shape)} and "
+          f"{tuple(down.shape)} for {experts} experts of {ff} and {shared} shared columns")
+    few = t <= 16
+    lists = None if few else torch.empty(experts * (t + 1) + t * top, dtype=torch.int32, device=x.device)
+    act = torch.empty(t * (cols if few else top * ff + shared), dtype=x.dtype, device=x.device)
+    parts = None if few else torch.empty((t * (top + 1), hidden), dtype=torch.float32, device=x.device)
+    y = torch.empty_like(x)
+    launch(x.data_ptr(), up.data_ptr(), down.data_ptr(), y.data_ptr(), None if few else lists.data_ptr(), act.data_ptr(),
+           None if few else parts.data_ptr(), t, hidden, experts, top, ff, shared, int(bool(gated)), weights.data_ptr(),
+           weights.shape[1], experts if shared_weight else -1)
+    return y
+
+
+register_kernel(KernelOp("moe_f32", moe_f32_plain, "holon_moe_f32",
+                         [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _I], _moe_f32_hip))
+
+
 @register_part("ffn", "polynorm")
 class PolyNormFFN(Part):
     """down(act(up(x))) with act = a N(z) + b N(z^2) + c N(z^3) + e (`act` holds a, b, c, e; N divides a token's
@@ -514,7 +575,8 @@ class MoE(Part):
     another: the activations of experts a token did not choose are set to 0 in between (`moe_gate`), so the second
     product adds up exactly the chosen experts' weighted outputs, and the shared expert's columns ride in the same two
     products. Steps of few rows take the same two products over the chosen experts' columns alone (`moe_few`), steps of many
-    rows each expert's over the rows that chose it (`moe_rows`), where that is done sooner. Steps of as many rows launch the
+    rows each expert's over the rows that chose it (`moe_rows`), and float32 steps of either kind the same (`moe_f32`), where
+    that is done sooner. Steps of as many rows launch the
     same kernels whatever was chosen."""
 
     graph_safe = True
@@ -599,6 +661,12 @@ class MoE(Part):
             weights = k.moe_router(x, self.router, self.correction if self.has_bias else None, self.top, self.groups,
                                    self.keep, self.scale)
         up, down = self.gate_up, self.all_down
+        if x.dtype == torch.float32 and moe_f32_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.shared, self.act == "silu",
+                                                     self.top):
+            y = k.moe_f32(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",
+                          shared_weight=self.shared_gated)
+            if y is not None:
+                return y
         if moe_few_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.act == "silu", self.top):
             y = k.moe_few(x, weights, up.tiled, down.tiled, self.experts, self.inter, self.shared, self.act == "silu",
                           shared_weight=self.shared_gated)

@@ -726,6 +726,16 @@ def test_every_expert_over_its_own_rows_where_that_is_done_sooner():
                                                  (64, 256, 2, 3, 128, 0), (0, 256, 8, 2, 128, 0), (1 << 22, 256, 8, 2, 128, 0)))
 
 
+def test_float32_experts_over_the_rows_that_chose_them_where_that_is_done_sooner():
+    from holon_amd.parts.ffn import moe_f32_pays, moe_f32_serves
+    assert [moe_f32_pays(m, 2048, 8, 2048, 2048, False, 2) for m in (1, 4, 12, 17, 64, 700)] == [True, True, False, False, True, True]
+    assert [moe_f32_pays(m, 2048, 8, 1024, 2048, True, 4) for m in (1, 4, 16, 63, 200)] == [True, False, False, False, True]
+    assert [moe_f32_pays(m, 2048, 128, 64, 0, True, 8) for m in (4, 16, 64, 200)] == [True, False, False, True]
+    assert moe_f32_serves(700, 2048, 8, 2, 2048, 2048) and moe_f32_serves(1, 16, 1, 1, 16, 0)
+    assert not any(moe_f32_serves(*a) for a in ((64, 40, 8, 2, 32, 0), (64, 32, 8, 2, 24, 0), (64, 32, 8, 2, 32, 8), (0, 32, 8, 2, 32, 0),
+                                                (64, 32, 2, 3, 32, 0)))
+
+
 @pytest.mark.gpu
 def test_chosen_experts_alone_or_all_of_them(tmp_path, monkeypatch):
     """Decoding a row over experts of a size that the few-row products serve, from graphs: bit for bit the same logits over the chosen

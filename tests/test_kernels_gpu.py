@@ -1148,6 +1148,50 @@ def test_every_expert_over_its_own_rows(hip, hidden, experts, ff, shared, top, g
     assert hip.moe_rows(_randn(4, hidden, dtype=torch.float32), weights[:4], up_w, down_w, experts, top, ff, shared, gated) is None
 
 
+@pytest.mark.parametrize("hidden,experts,ff,shared,top,gated,own_gate", [
+    (16, 1, 16, 0, 1, True, False), (272, 8, 80, 48, 2, True, True), (400, 5, 384, 0, 3, False, False),
+    (128, 70, 32, 16, 6, True, False), (2048, 8, 1024, 2048, 4, False, True)])
+def test_float32_experts_over_the_rows_that_chose_them(hip, hidden, experts, ff, shared, top, gated, own_gate):
+    """Few rows and many, against float64: sums of K and of the experts' columns in float32, 2^-24 of the larger of the two's shares and
+    their additions; a row the same bits alone, in a few and among many."""
+    cols = experts * ff + shared
+    up_w = _randn((2 if gated else 1) * cols, hidden, dtype=torch.float32, seed=74, scale=hidden ** -0.5)
+    down_w = _randn(hidden, cols, dtype=torch.float32, seed=75, scale=ff ** -0.5)
+    g = torch.Generator().manual_seed(76)
+    for m in (1, 2, 16, 17, 64, 65, 300):
+        x = _randn(m, hidden, dtype=torch.float32, seed=77 + m)
+        weights = torch.zeros(m, experts + int(own_gate))
+        for row in range(m):
+            weights[row, torch.randperm(experts, generator=g)[:top]] = torch.rand(top, generator=g) + 0.2
+        weights[:, experts:] = 0.7
+        if m in (16, 65):
+            weights[:, 1:experts] = 0          # one expert for all that chose it, none for the others
+            weights[3:5] = 0                   # rows of no expert, the shared one's gate closed too
+        weights = weights.cuda()
+        got = hip.moe_f32(x, weights, up_w, down_w, experts, top, ff, shared, gated, shared_weight=own_gate)
+        z = x.double() @ up_w.double().T
+        act = torch.nn.functional.silu(z[:, :cols]) * z[:, cols:] if gated else torch.relu(z).square()
+        each = weights[:, :experts].double().repeat_interleave(ff, 1)
+        last = weights[:, experts:].double() if own_gate else torch.ones(m, 1, dtype=torch.double, device="cuda")
+        want = (act * torch.cat((each, last.expand(m, shared)), 1)) @ down_w.double().T
+        apart = H.rel_rms(got, want) if want.any() else got.abs().max().item()
+        assert apart < 2e-6, (m, apart)
+        for row in {0, m // 2, m - 1}:
+            alone = hip.moe_f32(x[row: row + 1].contiguous(), weights[row: row + 1].contiguous(), up_w, down_w, experts, top, ff,
+                                shared, gated, shared_weight=own_gate)
+            assert torch.equal(alone[0], got[row]), (m, row)
+    assert hip.moe_f32(x.bfloat16(), weights, up_w, down_w, experts, top, ff, shared, gated) is None
+
+
+def test_float32_products_of_few_rows_by_half_tiles(hip):
+    """Up to 128 tiles of columns a block takes half a tile: the same bits as whole tiles (a row among more than 16), any K and N."""
+    for n, k in ((2048, 2048), (2047, 1000), (9, 31), (16, 64), (24, 4100), (1030, 513)):
+        x, w = _randn(17, k, dtype=torch.float32, seed=145), _randn(n, k, dtype=torch.float32, seed=146)
+        whole = hip.linear(x, w)
+        for m in (1, 5, 16):
+            assert torch.equal(hip.linear(x[:m].contiguous(), w), whole[:m]), (m, n, k)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_router_of_few_experts(hip, dtype):
     """Both routers up to 64 experts, on either side of 256 rows: the plain form's choice but for rows of a close call, and a

@@ -24,7 +24,7 @@ MODES = ("own", "vendor", "timed")
 # kind -> (this package's form or the plain default, every form)
 KINDS: dict[str, tuple[str, tuple[str, ...]]] = {
     "rows": ("rows", ("rows", "vendor")),         # 17 to 64 rows over many tiles, rows shared through LDS
-    "glu": ("rows", ("rows", "vendor")),          # the same with SiLU-mul inside
+    "glu": ("rows", ("rows", "vendor")),          # the same with SiLU-mul inside, and above 128 rows 256 x 256 tiles
     "parts": ("parts", ("parts", "vendor")),      # a narrow weight, K in shares: 17 to 128 rows; to 1,024 where K is well above N
     "vendor": ("bf16", ("bf16", "f32", "f32x2")),  # the vendor product's own forms (result type, K in halves)
 }

@@ -25,6 +25,8 @@ constexpr int KC = 64;                     // columns of K a chunk holds
 constexpr int REGION = HALF * KC * 2;      // bytes of 128 rows of a chunk
 constexpr int STAGE = 4 * REGION;          // a chunk: columns' first half, rows' first half, the second halves
 constexpr int LDS_BYTES = 2 * STAGE;
+constexpr int EXTRA = 16;                  // rows a tile may take beyond its 256: what a step's last few rows are not worth a tile for
+constexpr int EXTRA_BYTES = EXTRA * KC * 2;
 constexpr int XCDS = 8;
 
 // [half of the rows][half of the columns][tile of 16 rows][tile of 16 columns]: a lane holds columns 4 (lane / 16) .. + 3 of
@@ -54,6 +56,13 @@ struct Place {
   __device__ __forceinline__ int column(int j, int n) const { return j * HALF + wc * 32 + n * 16 + 4 * g; }
 };
 
+// The extra rows' sums: of half j of the columns, one tile of 16 a wave (`extra_column(j)`: the lane's first of four), row lane % 16.
+struct ExtraAcc {
+  f32x4_t v[2];
+  __device__ __forceinline__ void clear() { v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f}; }
+};
+__device__ __forceinline__ int extra_column(const Place& at, int j) { return j * HALF + at.wc * 32 + at.wr * 16 + 4 * at.g; }
+
 // What a lane copies of each 128 rows of a chunk: rows `copy_row(q)` (q = 0, 1), from `copy_piece(q)` bytes into the chunk's
 // 128 bytes of that row.
 __device__ __forceinline__ int copy_row(int q) { return q * 64 + threadIdx.x / 8; }
@@ -67,8 +76,11 @@ __device__ __forceinline__ void phase_barrier() {           // (nothing is moved
 
 // Adds the products to acc. `x_at` and `w_at` [half][q]: this lane's byte offsets from x and w of what it copies of the first
 // chunk (row and piece). `chunks` (K / 64): even, at least 2. Every wave of the block comes here, with the same `chunks`.
-__device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const bf16_t* w, const uint32_t (&x_at)[2][2],
-                                    const uint32_t (&w_at)[2][2], int chunks) {
+// MORE: 16 extra rows as well (`more`; `more_at`: as x_at, of rows copy_row(0) up to 15; LDS of LDS_BYTES + 2 EXTRA_BYTES). Waves 0 and 1
+// then have a copy more under way, and wait for one more than they need.
+template <bool MORE>
+__device__ __forceinline__ void run_with(Acc& acc, ExtraAcc& more, char* lds, const bf16_t* x, const bf16_t* w,
+                                         const uint32_t (&x_at)[2][2], const uint32_t (&w_at)[2][2], uint32_t more_at, int chunks) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const int wr = wave / 4, wc = wave % 4, g = lane / 16, c = lane % 16;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
@@ -78,6 +90,7 @@ __device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const 
     const uint32_t to = lds0 + (chunk & 1) * STAGE + which * REGION + wave * 1024;
 #pragma unroll
     for (int q = 0; q < 2; ++q) load_to_lds16(from, (which & 1) ? x_at[h][q] : w_at[h][q], to + q * 8192);
+    if (MORE && which == 1 && wave < 2) load_to_lds16(from, more_at, lds0 + LDS_BYTES + (chunk & 1) * EXTRA_BYTES + wave * 1024);
   };
   uint32_t at[2];                                           // this lane's 16 bytes of its row of a tile, per 32 of the chunk
 #pragma unroll
@@ -96,7 +109,11 @@ __device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const 
 #pragma unroll
       for (int t = 0; t < 2; ++t) b[s][t] = *reinterpret_cast<const bf16x8_t*>(p + t * 16 * KC * 2 + at[s]);
   };
-  const auto multiply = [&](f32x4_t (&d)[4][2], const bf16x8_t (&a)[2][4], const bf16x8_t (&b)[2][2]) {
+  constexpr std::integral_constant<int, 0> c0{};
+  constexpr std::integral_constant<int, 1> c1{};
+  constexpr std::integral_constant<int, 2> c2{};
+  bf16x8_t extra[2];
+  const auto multiply = [&](f32x4_t (&d)[4][2], const bf16x8_t (&a)[2][4], const bf16x8_t (&b)[2][2], auto with) {      // with: the extra
     phase_barrier();
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -105,6 +122,13 @@ __device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const 
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int n = 0; n < 2; ++n) d[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][n], a[s][t], d[t][n], 0, 0, 0);
+    constexpr int J = decltype(with)::value;                // rows too, of half J of the columns (2: not)
+    if constexpr (MORE && J < 2) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        if (wr == 0) more.v[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][0], extra[s], more.v[J], 0, 0, 0);
+        else more.v[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][1], extra[s], more.v[J], 0, 0, 0);
+    }
     __builtin_amdgcn_s_setprio(0);
     phase_barrier();
   };
@@ -127,29 +151,29 @@ __device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const 
   const auto chunk = [&](auto parity, auto tail, int k) {
     constexpr int P = decltype(parity)::value, T = decltype(tail)::value;
     read_rows(a, 0, k);
+    if constexpr (MORE)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) extra[s] = *reinterpret_cast<const bf16x8_t*>(lds + LDS_BYTES + (k & 1) * EXTRA_BYTES + at[s]);
     if constexpr (T == 0) copy(0, k + 2);
     reads_done();
     wait_loads_but<T == 0 ? 12 : (T == 1 ? 10 : 2)>();
-    multiply(acc.v[0][0], a, b[P]);
+    multiply(acc.v[0][0], a, b[P], c0);
     read_columns(b[1 - P], 1, k);
     if constexpr (T == 0) copy(1, k + 2);
     reads_done();
     wait_loads_but<T == 0 ? 12 : (T == 1 ? 8 : 0)>();
-    multiply(acc.v[0][1], a, b[1 - P]);
+    multiply(acc.v[0][1], a, b[1 - P], c1);
     read_rows(a, 1, k);
     if constexpr (T == 0) copy(2, k + 2);
     reads_done();
     wait_loads_but<T == 0 ? 12 : (T == 1 ? 6 : 0)>();
-    multiply(acc.v[1][1], a, b[1 - P]);
+    multiply(acc.v[1][1], a, b[1 - P], c2);
     if constexpr (T < 2) read_columns(b[1 - P], 0, k + 1);
     if constexpr (T == 0) copy(3, k + 2);
     reads_done();
     wait_loads_but<T == 0 ? 12 : (T == 1 ? 4 : 0)>();
-    multiply(acc.v[1][0], a, b[P]);
+    multiply(acc.v[1][0], a, b[P], c2);
   };
-  constexpr std::integral_constant<int, 0> c0{};
-  constexpr std::integral_constant<int, 1> c1{};
-  constexpr std::integral_constant<int, 2> c2{};
   for (int k = 0; k + 2 < chunks; k += 2) {
     chunk(c0, c0, k);
     chunk(c1, c0, k + 1);
@@ -157,6 +181,12 @@ __device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const 
   chunk(c0, c1, chunks - 2);
   chunk(c1, c2, chunks - 1);
   if (wr == 0) phase_barrier();                             // (as many barriers as the other four waves)
+}
+
+__device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const bf16_t* w, const uint32_t (&x_at)[2][2],
+                                    const uint32_t (&w_at)[2][2], int chunks) {
+  ExtraAcc none;
+  run_with<false>(acc, none, lds, x, w, x_at, w_at, 0, chunks);
 }
 
 // The tile that block `id` takes of `total`, -1: none. Blocks go to the XCDs in turn; each XCD gets a run of neighbouring

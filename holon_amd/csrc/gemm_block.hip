@@ -1,0 +1,167 @@
+// Products of many rows (prompts) over untiled weights on 256 x 256 tiles (gemm_block.h), bfloat16 with float32 sums: a gated
+// feed-forward's first product with the activation in its epilogue, and products whose K is cut into shares over the grid, the shares
+// added up by whoever reads them.
+//
+// A step's last row tile takes up to 16 rows beyond its 256: a portion of 512 tokens beside a few decode rows is two tiles high, not three.
+#include "common.h"
+#include "gemm_block.h"
+#include "holon_hip.h"
+
+namespace {
+using namespace block_gemm;
+
+enum { SILU, GELU, PARTS };
+
+// What a tile gives, from LDS in whole lines: the gated ones bfloat16 y [M, N], 128 columns a tile (the tile's first half of columns are
+// gates and the second ups of w [2 N, K]), PARTS float32 y [splits, M, N].
+template <int KIND>
+__global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                void* __restrict__ y, int M, int N, int K, int row_tiles,
+                                                                int col_tiles, int splits) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES + 2 * EXTRA_BYTES];
+  constexpr bool GATED = KIND == SILU || KIND == GELU;
+  constexpr int COLS = GATED ? HALF : TILE;
+  const int tiles = row_tiles * col_tiles;
+  int tile = tile_of_block(blockIdx.x, tiles * splits);
+  if (tile < 0) return;
+  const int split = tile / tiles, share = K / splits;
+  tile %= tiles;
+  int rt, ct;
+  row_and_column(tile, row_tiles, col_tiles, rt, ct);
+  const int m0 = rt * TILE, n0 = ct * COLS;
+  const bool has_more = rt == row_tiles - 1 && M > row_tiles * TILE;      // rows beyond the last tile's 256
+  uint32_t x_at[2][2], w_at[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {                    // (rows and columns past the last repeat it: nothing of them is written)
+      const int r = copy_row(q);
+      x_at[h][q] = (uint32_t)((int64_t)min(m0 + h * HALF + r, M - 1) * K * 2) + copy_piece(q);
+      const int64_t column = GATED ? (int64_t)h * N + min(n0 + r, N - 1) : min(n0 + h * HALF + r, N - 1);
+      w_at[h][q] = (uint32_t)(column * K * 2) + copy_piece(q);
+    }
+  const uint32_t more_at = (uint32_t)((int64_t)min(m0 + TILE + copy_row(0) % EXTRA, M - 1) * K * 2) + copy_piece(0);
+  Acc acc;
+  ExtraAcc more;
+  acc.clear();
+  more.clear();
+  const int64_t k0 = (int64_t)split * share;
+  if (has_more) run_with<true>(acc, more, lds, x + k0, w + k0, x_at, w_at, more_at, share / KC);
+  else run_with<false>(acc, more, lds, x + k0, w + k0, x_at, w_at, 0, share / KC);
+  const Place at;
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  if constexpr (GATED) {
+    constexpr int ACT = KIND == GELU, PITCH = HALF * 2 + 16, ROWS = TILE + EXTRA;
+    static_assert(ROWS * PITCH <= LDS_BYTES, "a tile's columns");
+    const auto gated = [](f32x4_t gate, f32x4_t up) {                      // the roundings of the product and of the gated kernels
+      ushort4 o;
+      bf16_t* oe = reinterpret_cast<bf16_t*>(&o);
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        oe[v] = float_to_bf16(Elem<bf16_t>::round(gate_act<ACT, bf16_t>(Elem<bf16_t>::round(gate[v]))) * Elem<bf16_t>::round(up[v]));
+      return o;
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+          *reinterpret_cast<ushort4*>(lds + at.row(i, t) * PITCH + at.column(0, n) * 2) = gated(acc.v[i][0][t][n], acc.v[i][1][t][n]);
+    if (has_more) *reinterpret_cast<ushort4*>(lds + (TILE + at.c) * PITCH + extra_column(at, 0) * 2) = gated(more.v[0], more.v[1]);
+    __syncthreads();
+    for (int e = threadIdx.x; e < (has_more ? ROWS : TILE) * 16; e += THREADS) {
+      const int row = e / 16, column = n0 + e % 16 * 8;
+      if (m0 + row < M && column < N)
+        *reinterpret_cast<uint4*>((bf16_t*)y + (int64_t)(m0 + row) * N + column) =
+            *reinterpret_cast<const uint4*>(lds + row * PITCH + e % 16 * 16);
+    }
+  } else {
+    constexpr int PITCH = 144;                       // a wave's own 64 rows of 32 columns at a time
+    char* mine = lds + wave * (64 * PITCH);
+    float* out = (float*)y + (int64_t)split * M * N;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+            *reinterpret_cast<f32x4_t*>(mine + (t * 16 + at.c) * PITCH + n * 64 + at.g * 16) = acc.v[i][j][t][n];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int r = u * 8 + lane / 8, m = m0 + i * HALF + at.wr * 64 + r, column = n0 + j * HALF + at.wc * 32 + lane % 8 * 4;
+          if (m < M && column < N)
+            *reinterpret_cast<f32x4_t*>(out + (int64_t)m * N + column) = *reinterpret_cast<const f32x4_t*>(mine + r * PITCH + lane % 8 * 16);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+    if (has_more && m0 + TILE + at.c < M)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int column = n0 + extra_column(at, j);
+        if (column < N) *reinterpret_cast<f32x4_t*>(out + (int64_t)(m0 + TILE + at.c) * N + column) = more.v[j];
+      }
+  }
+}
+
+int row_tiles_of(int M) { return M > TILE && M % TILE && M % TILE <= EXTRA ? M / TILE : (M + TILE - 1) / TILE; }
+}  // namespace
+
+// Whether the products serve M rows over w [N or 2 N, K] with K in `splits` shares: shares of whole pairs of chunks, offsets of 32 bits.
+extern "C" int holon_gemm_block_supported(int M, int N, int K, int gated, int splits) {
+  return M >= 1 && N > 0 && N % 16 == 0 && splits >= 1 && K > 0 && K % (128 * splits) == 0 && (int64_t)M * K < (int64_t)1 << 31 &&
+         ((int64_t)N * (gated ? 2 : 1)) * K < (int64_t)1 << 31;
+}
+
+static int launch_block(int kind, const void* x, const void* w, void* y, int M, int N, int K, int splits, void* stream) {
+  const bool gated = kind == SILU || kind == GELU;
+  HOLON_CHECK(holon_gemm_block_supported(M, N, K, gated, splits) && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0,
+              "gemm (many rows): M=%d N=%d K=%d in %d shares not served", M, N, K, splits);
+  const int rows = row_tiles_of(M), cols = (N + (gated ? HALF : TILE) - 1) / (gated ? HALF : TILE);
+  const unsigned blocks = (unsigned)(((int64_t)rows * cols * splits + XCDS - 1) / XCDS * XCDS);      // every XCD as many
+  hipStream_t s = (hipStream_t)stream;
+  const bf16_t *a = (const bf16_t*)x, *b = (const bf16_t*)w;
+  switch (kind) {
+    case SILU: gemm_block_kernel<SILU><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
+    case GELU: gemm_block_kernel<GELU><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
+    default: gemm_block_kernel<PARTS><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
+  }
+  HOLON_LAUNCH_OK();
+  return 0;
+}
+
+// y [M, N] = act(x gates^T) * (x ups^T) over w [2 N, K] (gates, then ups); act 0 silu, 1 gelu in its tanh form.
+extern "C" int holon_gemm_block_glu_bf16(const void* x, const void* w, void* y, int M, int N, int K, int act, void* stream) {
+  return launch_block(act ? GELU : SILU, x, w, y, M, N, K, 1, stream);
+}
+
+// Whether a product in shares takes this form where gemm_tiles.hip's would serve it too: with its last rows filled up that one's blocks
+// read both operands twice as often. Measured with the add + norm that reads the parts, in as many shares, us, that form against this:
+// 4096 x 12288 at 129 / 300 / 520 / 768 / 1,024 rows 44 / 64 / 96 / 105 / 117 and 41 / 54 / 64 / 83 / 96; 5120 x 25600 at 256 / 512 /
+// 1,000 rows 121 / 172 / 297 and 93 / 148 / 250; 2048 x 8192 at 129 / 512 / 1,000 rows 28 / 35 / 57 and 27 / 35 / 49. A K that eight shares
+// of whole pairs of chunks do not divide stays with the other up to 512 rows (2560 x 9728 at 256 / 400 / 600 / 1,000 rows, eight shares there
+// against four here: 35 / 50 / 56 / 90 and 48 / 52 / 56 / 63).
+extern "C" int holon_gemm_block_parts_serves(int M, int N, int K, int splits) {
+  return M > 128 && M <= 1024 && N % TILE == 0 && holon_gemm_block_supported(M, N, K, 0, splits) && (K % 1024 == 0 || M > 512);
+}
+// The number of shares, a power of two up to eight, that is done first: rounds of a tile's loop a compute unit, and the parts' traffic (of
+// 24 products of three widths the choice is at most 6 % from the best).
+int block_parts_splits(int M, int N, int K) {
+  const int tiles = row_tiles_of(M) * ((N + TILE - 1) / TILE);
+  int best = 0;
+  float least = 0.f;
+  for (int splits = 1; splits <= 8; splits *= 2) {
+    if (!holon_gemm_block_parts_serves(M, N, K, splits)) continue;
+    const float us = (float)((tiles * splits + 255) / 256) * (0.0203f * K / splits + 6.f) + 1.45e-6f * splits * M * N;
+    if (best == 0 || us < least) { best = splits; least = us; }
+  }
+  return best;
+}
+
+// parts [splits, M, N] (float32) = x[:, share s of K] w[:, share s of K]^T.
+extern "C" int holon_gemm_block_parts_bf16(const void* x, const void* w, void* parts, int M, int N, int K, int splits, void* stream) {
+  return launch_block(PARTS, x, w, parts, M, N, K, splits, stream);
+}

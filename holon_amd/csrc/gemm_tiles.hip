@@ -1,5 +1,5 @@
 // parts[s][M, N] = x[M, share s of K] w[N, share s of K]^T for 129 to 1,024 rows (prompt portions of a few hundred
-// tokens) over a narrow weight with a long K (a feed-forward's second product): bfloat16 operands, float32 sums on the
+// tokens; where gemm_block.hip's 256 x 256 tiles do not serve them) over a narrow weight with a long K (a feed-forward's second product): bfloat16 operands, float32 sums on the
 // matrix cores, the shares added up by whoever reads them (the residual add + norm does so as it reads).
 //
 // The shape the vendor library serves worst: few tiles of output and a long K, so that its blocks walk all of K alone
@@ -163,6 +163,8 @@ extern "C" int holon_gemm_tiles_parts_supported(int M, int N, int K, int splits)
          (int64_t)M * K * 2 < (int64_t)1 << 32;             // (a lane's place among the rows is a 32-bit byte offset)
 }
 
+int block_parts_splits(int M, int N, int K);
+
 // How many shares of K to take, 0 where the kernel does not serve the shape or is not the one to take: it is for
 // weights whose K is well above their N (few output tiles, long sums), with as few shares (a power of two, at most
 // eight) as give 384 blocks. Measured on MI355X with the add + norm that reads the parts, against the vendor library's
@@ -178,7 +180,9 @@ extern "C" int holon_gemm_tiles_splits(int M, int N, int K) {
   int splits = 1;
   while (splits < TILES_MAX_SPLITS && blocks * splits < 384) splits *= 2;
   while (splits > 1 && K % (TILES_KC * splits)) splits /= 2;
-  return holon_gemm_tiles_parts_supported(M, N, K, splits) && blocks * splits >= 128 ? splits : 0;
+  if (!holon_gemm_tiles_parts_supported(M, N, K, splits) || blocks * splits < 128) return 0;
+  const int whole = block_parts_splits(M, N, K);          // (in shares of 256 x 256 tiles: gemm_block.hip)
+  return whole ? whole : splits;
 }
 
 // parts[s][M][N] (float32) = x[:, share s of K] w[:, share s of K]^T over tiled weights, 129 <= M <= 1,024.

@@ -1018,6 +1018,43 @@ def test_product_in_shares_of_k_for_prompt_portions(hip):
         hip._rows_parts(x, w[:4000].contiguous(), hip.tile_weight(w[:4000].contiguous()), 4)   # 4,000 columns: no whole blocks
 
 
+def test_products_on_tiles_of_256_rows(hip):
+    """Tiles of 256 x 256 with up to 16 rows more in the last one: a gated first product against float64 (three roundings to bfloat16 of
+    2^-9 each: gate and up, the activation, the result) in either activation, products in shares of K against float64 shares; rows whatever
+    lies beside them; which calls take them."""
+    from holon_amd.kernels.hip import KernelError, glu_block_pays
+    bf = torch.bfloat16
+    for m, inter, k in ((1, 16, 128), (17, 128, 256), (256, 112, 128), (257, 144, 384), (272, 272, 256), (273, 128, 640), (520, 400, 256),
+                        (769, 256, 128)):
+        x, w = _randn(m, k, dtype=bf, seed=180), _randn(2 * inter, k, dtype=bf, seed=181, scale=2 * k ** -0.5)
+        z = x.double() @ w.double().T
+        outs = []
+        for act, fn in ((0, torch.nn.functional.silu), (1, lambda v: torch.nn.functional.gelu(v, approximate="tanh"))):
+            y = torch.empty(m, inter, dtype=bf, device="cuda")
+            hip._call(hip.lib.holon_gemm_block_glu_bf16, x.data_ptr(), w.data_ptr(), y.data_ptr(), m, inter, k, act, hip._stream())
+            assert H.rel_rms(y, fn(z[:, :inter]) * z[:, inter:]) < 3 * 2.0 ** -9, (m, inter, k, act)
+            outs.append(y)
+        one = torch.empty(1, inter, dtype=bf, device="cuda")
+        for row in {0, m // 2, m - 1}:
+            hip._call(hip.lib.holon_gemm_block_glu_bf16, x[row:].data_ptr(), w.data_ptr(), one.data_ptr(), 1, inter, k, 0, hip._stream())
+            assert torch.equal(one[0], outs[0][row]), (m, inter, k, row)
+    for m, n, k, splits in ((1, 16, 128, 1), (257, 272, 512, 2), (272, 256, 1024, 8), (300, 512, 768, 3), (520, 256, 256, 1), (529, 48, 512, 4)):
+        x, w = _randn(m, k, dtype=bf, seed=182), _randn(n, k, dtype=bf, seed=183, scale=0.05)
+        parts = torch.empty(splits, m, n, dtype=torch.float32, device="cuda")
+        hip._call(hip.lib.holon_gemm_block_parts_bf16, x.data_ptr(), w.data_ptr(), parts.data_ptr(), m, n, k, splits, hip._stream())
+        for s in range(splits):
+            part = slice(s * k // splits, (s + 1) * k // splits)
+            want = x[:, part].double() @ w[:, part].double().T
+            assert H.op_budget_usage(parts[s], want, torch.float32, k // splits) <= 1, (m, n, k, s)
+    assert [glu_block_pays(m, 12288, 4096) for m in (128, 520, 600, 768, 1024, 4096)] == [False, True, False, False, True, True]
+    x, w = _randn(520, 256, dtype=bf), _randn(2 * 16384, 256, dtype=bf, scale=0.1)
+    assert torch.equal(hip.linear_silu_mul(x, w), hip._glu_block(x, w)) and hip.configured("vendor").linear_silu_mul(x, w) is None
+    with pytest.raises(KernelError):                                                   # K of whole pairs of chunks alone
+        hip._call(hip.lib.holon_gemm_block_parts_bf16, x.data_ptr(), w.data_ptr(), x.data_ptr(), 16, 16, 192, 1, hip._stream())
+    with pytest.raises(KernelError):
+        hip._call(hip.lib.holon_gemm_block_parts_bf16, x.data_ptr(), w.data_ptr(), x.data_ptr(), 16, 16, 256, 4, hip._stream())
+
+
 def test_kernels_refuse_what_they_do_not_serve(hip):
     from holon_amd.kernels.hip import KernelError
     with pytest.raises(KernelError):

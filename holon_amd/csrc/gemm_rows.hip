@@ -175,9 +175,88 @@ void launch_rows_tall(const void* x, const void* w, void* y, int M, int N, int K
 }
 }  // namespace
 
+// 17 to 64 rows over weights too narrow for the form above: a block one tile of 16 columns, K split over its waves in order, every wave
+// reading its share of the rows from L2 (the few-row kernel's shape with MT tiles of tokens). One launch where a product in shares takes
+// two; bound by what the blocks read of the rows, N / 16 times all of them.
+namespace {
+template <int MT, bool F32>
+__global__ void __launch_bounds__(1024) gemm_deep_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ y,
+                                                         int M, int N, int K) {
+  extern __shared__ __attribute__((aligned(16))) f32x4_t deep_sums[];      // [waves][MT][64]
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, waves = blockDim.x / WAVE;
+  const int g = lane / 16, c = lane % 16, steps = K / 32 / waves;
+  const bf16_t* wp = w + ((int64_t)blockIdx.x * (K / 32) + (int64_t)wave * steps) * 512 + lane * 8;
+  const bf16_t* xp[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) xp[t] = x + (int64_t)min(t * 16 + c, M - 1) * K + (int64_t)wave * steps * 32 + 8 * g;
+  f32x4_t acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int AT_ONCE = 4;
+  for (int s0 = 0; s0 < steps; s0 += AT_ONCE) {
+    bf16x8_t a[AT_ONCE], b[AT_ONCE][MT];
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u) {                     // (past the last step: that one again, unused)
+      const int s = min(s0 + u, steps - 1);
+      a[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp + (int64_t)s * 512));
+#pragma unroll
+      for (int t = 0; t < MT; ++t) b[u][t] = *reinterpret_cast<const bf16x8_t*>(xp[t] + s * 32);
+    }
+#pragma unroll
+    for (int u = 0; u < AT_ONCE; ++u)
+      if (s0 + u < steps)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u][t], acc[t], 0, 0, 0);
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) deep_sums[(wave * MT + t) * WAVE + lane] = acc[t];
+  __syncthreads();
+  for (int t = wave; t < MT; t += waves) {                  // a wave a tile of rows
+    f32x4_t sum = deep_sums[t * WAVE + lane];
+    for (int i = 1; i < waves; ++i) sum += deep_sums[(i * MT + t) * WAVE + lane];
+    const int m = t * 16 + c;
+    if (m >= M) continue;
+    const int64_t at = (int64_t)m * N + blockIdx.x * 16 + 4 * g;
+    if constexpr (F32) {                                    // (the bfloat16 product, cast up)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i] = Elem<bf16_t>::round(sum[i]);
+      *reinterpret_cast<f32x4_t*>((float*)y + at) = sum;
+    } else {
+      ushort4 o;
+      o.x = float_to_bf16(sum[0]); o.y = float_to_bf16(sum[1]); o.z = float_to_bf16(sum[2]); o.w = float_to_bf16(sum[3]);
+      *reinterpret_cast<ushort4*>((bf16_t*)y + at) = o;
+    }
+  }
+}
+
+// Where that is no slower on the GPU than the vendor library's product, and one launch of 7 us of the host's where that one takes 19 (a
+// prompt of so few tokens is bound by the host): us at 17 / 32 / 37 / 48 rows against the library, 2048 x 2048 6.8 / 8.3 / 9.2 / 10.2 and
+// 8.9 / 8.9 / 8.9 / 8.9, 4096 x 2048 7.8 / 9.0 / 9.6 / 10.6 and 9.1 / 9.2 / 9.2 / 9.2, 1024 x 2048 6.6 / 8.1 / 9.0 / 9.9 and 8.5 / 8.8 / 8.6 /
+// 8.7; beyond 256 tiles, or over longer sums (2048 x 8192 at 17 / 37 rows 18 / 27 and 14 / 14), the reads of the rows cost too much, under
+// 64 tiles the compute units stand idle (512 x 2048 at 37 rows 8.9 and 5.8), and short sums are done in 5 us (2048 x 768).
+bool deep_serves(int M, int N, int K) {
+  return M > 16 && M <= 40 && N % 16 == 0 && N >= 1024 && N <= 4096 && K % 256 == 0 && K >= 1280 && K <= 2048;
+}
+
+void launch_deep(const void* x, const void* w, void* y, int M, int N, int K, int out_f32, hipStream_t s) {
+  int waves = 16;
+  while (K % (32 * waves) != 0) waves /= 2;                 // (K is a multiple of 256: at least 8)
+  const int mt = (M + 15) / 16;
+  const size_t lds = (size_t)waves * mt * WAVE * sizeof(f32x4_t);
+#define DEEP(MT)                                                                                                              \
+  case MT:                                                                                                                    \
+    if (out_f32) gemm_deep_kernel<MT, true><<<N / 16, waves * WAVE, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, y, M, N, K); \
+    else gemm_deep_kernel<MT, false><<<N / 16, waves * WAVE, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, y, M, N, K);        \
+    break
+  switch (mt) { DEEP(2); DEEP(3); }
+#undef DEEP
+}
+}  // namespace
+
 // Whether holon_gemm_rows_bf16 serves this product (gated: N is the number of output columns I, the weight has 2 I rows).
 extern "C" int holon_gemm_rows_supported(int M, int N, int K, int gated) {
   const int tiles = N / 16;
+  if (!gated && deep_serves(M, N, K)) return 1;
   return M > 16 && M <= 64 && N % 16 == 0 && K % 256 == 0 && K >= 256 && tiles % 8 == 0 &&
          tiles * (gated ? 2 : 1) >= ROWS_MIN_TILES;
 }
@@ -189,6 +268,11 @@ extern "C" int holon_gemm_rows_bf16(const void* x, const void* w_tiled, void* y,
                                     void* stream) {
   HOLON_CHECK(holon_gemm_rows_supported(M, N, K, 0), "gemm (17 to 64 rows): M=%d N=%d K=%d not served", M, N, K);
   hipStream_t s = (hipStream_t)stream;
+  if (deep_serves(M, N, K)) {
+    launch_deep(x, w_tiled, y, M, N, K, out_f32, s);
+    HOLON_LAUNCH_OK();
+    return 0;
+  }
   const bool wide = N / 16 >= 4096;          // a vocabulary's worth of tiles: longer chunks, at 64 rows eight waves
   if (out_f32) {
     if (wide && M > 48) launch_rows<8, 256, 1>(x, w_tiled, y, M, N, K, s);

@@ -76,10 +76,12 @@ class ProductPlan:
         self.resolving = False                    # True only while the engine starts: `timed` may time now
         self.seconds = 0.0                        # what the timings cost
 
-    def choose(self, kind: str, shape: tuple[int, int], bucket: int, time: Callable[[], str] | None = None) -> str:
+    def choose(self, kind: str, shape: tuple[int, int], bucket: int, time: Callable[[], str] | None = None,
+               yields: bool = False) -> str:
         """The form the product `kind` over a weight of `shape` takes at `bucket` rows. `time()` runs the candidates
         against each other and names the winner; it is called at most once per key, and only while the engine
-        starts."""
+        starts. `yields`: where nothing is pinned for this kind, a pinned form of the vendor library's product at this
+        shape and bucket keeps that product (pins of a run that had no other form to choose there)."""
         key = key_of(kind, shape, bucket)
         form = self.taken.get(key)
         if form is not None:
@@ -87,6 +89,8 @@ class ProductPlan:
         own, forms = KINDS[kind]
         if key in self.pins:
             form, how = self.pins[key], "pinned"
+        elif yields and key_of("vendor", shape, bucket) in self.pins:
+            form, how = forms[-1], "pinned"
         elif self.mode == "vendor":
             form, how = forms[-1] if kind != "vendor" else "bf16", "vendor"
         elif self.mode == "timed" and self.resolving and time is not None:

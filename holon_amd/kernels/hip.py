@@ -160,12 +160,12 @@ class HipKernels:
         other.plan = ProductPlan(products, pins)
         return other
 
-    def product_choice(self, kind: str, weight, rows: int, time=None) -> str:
+    def product_choice(self, kind: str, weight, rows: int, time=None, yields=False) -> str:
         """The one place a product's form is resolved: pinned, else by the engine's mode, else (mode `timed`, while
         the engine starts and outside graph capture) by timing the candidates once."""
         if time is not None and (not self.plan.resolving or torch.cuda.is_current_stream_capturing()):
             time = None
-        return self.plan.choose(kind, tuple(weight.shape), row_bucket(rows), time)
+        return self.plan.choose(kind, tuple(weight.shape), row_bucket(rows), time, yields)
 
     # -- operations that parts bring with them ----------------------------------------------------------------------
     _part_libs: dict[str, ctypes.CDLL] = {}       # libraries built from parts' own sources, by source path
@@ -495,7 +495,8 @@ class HipKernels:
                 and self.lib.holon_gemm_rows_supported(rows, n // 2 if gated else n, k, int(gated))):
             return False
         return self.product_choice("glu" if gated else "rows", weight, rows,
-                                   lambda: self._time_rows(rows, weight, tiled, gated)) == "rows"
+                                   lambda: self._time_rows(rows, weight, tiled, gated),
+                                   yields=not gated and n <= 4096) == "rows"
 
     def _rows_product(self, x, weight, tiled, gated, to_f32=False):
         m, k = x.shape
@@ -637,7 +638,7 @@ class HipKernels:
             return "rows" if took["rows"] < took["vendor"] else "vendor"
         if m > self.parts_rows:                   # (beyond the steps that start-up times: by the rule above)
             return None if self.plan.mode == "vendor" else block(weight)
-        return block(weight) if self.product_choice("glu", weight, m, time) == "rows" else None
+        return block(weight) if self.product_choice("glu", weight, m, time, yields=True) == "rows" else None
 
     def silu_mul(self, gate_up):
         self._check(gate_up, "silu_mul")

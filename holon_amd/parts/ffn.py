@@ -434,11 +434,12 @@ def moe_rows_pays(rows: int, hidden: int, experts: int, ff: int, shared: int, ga
 def _moe_rows_hip(launch, x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
     t, hidden = x.shape
     cols = experts * ff + shared
-    if x.dtype != torch.bfloat16 or not moe_rows_serves(t, hidden, experts, top, ff, shared):
+    if x.dtype != torch.bfloat16 or not moe_rows_serves(t, hidden, experts, top, ff, shared) \
+            or any(v.data_ptr() % 16 for v in (x, up, down)):
         return None
     _need(x.is_cuda and x.is_contiguous() and weights.is_contiguous() and weights.dtype == torch.float32
           and tuple(weights.shape) == (t, experts + int(bool(shared_weight)))
-          and all(w.is_contiguous() and w.dtype == x.dtype and w.data_ptr() % 16 == 0 for w in (up, down)) and x.data_ptr() % 16 == 0
+          and all(w.is_contiguous() and w.dtype == x.dtype for w in (up, down))
           and tuple(up.shape) == ((2 if gated else 1) * cols, hidden) and tuple(down.shape) == (hidden, cols),
           f"moe_rows: rows {tuple(x.shape)}, weights {tuple(weights.shape)}, projections {tuple(up.shape)} and "
           f"{tuple(down.shape)} for {experts} experts of {ff} and {shared} shared columns")
@@ -493,11 +494,12 @@ def moe_f32_pays(rows: int, hidden: int, experts: int, ff: int, shared: int, gat
 def _moe_f32_hip(launch, x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
     t, hidden = x.shape
     cols = experts * ff + shared
-    if x.dtype != torch.float32 or not moe_f32_serves(t, hidden, experts, top, ff, shared):
+    if x.dtype != torch.float32 or not moe_f32_serves(t, hidden, experts, top, ff, shared) \
+            or any(v.data_ptr() % 16 for v in (x, up, down)):
         return None
     _need(x.is_cuda and x.is_contiguous() and weights.is_contiguous() and weights.dtype == torch.float32
           and tuple(weights.shape) == (t, experts + int(bool(shared_weight)))
-          and all(w.is_contiguous() and w.dtype == x.dtype and w.data_ptr() % 16 == 0 for w in (up, down)) and x.data_ptr() % 16 == 0
+          and all(w.is_contiguous() and w.dtype == x.dtype for w in (up, down))
           and tuple(up.shape) == ((2 if gated else 1) * cols, hidden) and tuple(down.shape) == (hidden, cols),
           f"moe_f32: rows {tuple(x.shape)}, weights {tuple(weights.shape)}, projections {tuple(up.shape)} and "
           f"{tuple(down.shape)} for {experts} experts of {ff} and {shared} shared columns")

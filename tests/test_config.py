@@ -178,3 +178,16 @@ def test_product_choices_resolve_pinned_then_by_mode_then_timed_at_start_only():
     got = cli.engine_config("m", ap.parse_args(["--products", "timed", "--product-pins",
                                                 "parts:8x16:32=vendor, vendor:8x16:512=f32x2"]))
     assert got.products == "timed" and got.product_pins == {"parts:8x16:32": "vendor", "vendor:8x16:512": "f32x2"}
+
+
+def test_a_pinned_vendor_form_keeps_the_vendor_product():
+    """Where a kind yields and nothing is pinned for it: pins of a run in which the vendor library's product was the only one."""
+    from holon_amd.config.products import ProductPlan
+
+    plan = ProductPlan("own", {"vendor:4096x2048:32": "f32x2", "vendor:24576x4096:512": "f32", "glu:24576x4096:512": "rows"})
+    assert plan.choose("rows", (4096, 2048), 32, yields=True) == "vendor"
+    assert plan.choose("vendor", (4096, 2048), 32) == "f32x2"
+    assert plan.choose("rows", (4096, 2048), 64, yields=True) == "rows"
+    assert plan.choose("rows", (2048, 2048), 32, yields=True) == "rows"
+    assert plan.choose("glu", (24576, 4096), 512, yields=True) == "rows"
+    assert ProductPlan("own", {"vendor:4096x2048:32": "f32"}).choose("rows", (4096, 2048), 32) == "rows"

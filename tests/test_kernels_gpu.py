@@ -1202,6 +1202,19 @@ def test_every_expert_over_its_own_rows(hip, hidden, experts, ff, shared, top, g
     assert hip.moe_rows(_randn(4, hidden, dtype=torch.float32), weights[:4], up_w, down_w, experts, top, ff, shared, gated) is None
 
 
+def test_experts_whose_operands_start_on_no_border_of_16_bytes_stay_with_the_products_over_all(hip):
+    """The kernels over an expert's own rows read 16 bytes at a time: elsewhere they serve nothing, whichever operand it is."""
+    for op, dtype in ((hip.moe_rows, torch.bfloat16), (hip.moe_f32, torch.float32)):
+        rows, hidden, experts, ff = 64, 128, 4, 128
+        weights = torch.zeros(rows, experts, device="cuda")
+        weights[:, 0] = 1
+        operands = [_randn(n, k, dtype=dtype, seed=68) for n, k in ((rows, hidden), (experts * ff, hidden), (hidden, experts * ff))]
+        for at in (None, 0, 1, 2):
+            x, up, down = (torch.empty(v.numel() + 1, dtype=dtype, device="cuda")[1:].view(v.shape).copy_(v) if i == at else v
+                           for i, v in enumerate(operands))
+            assert (op(x, weights, up, down, experts, 1, ff, 0, False) is None) == (at is not None), (dtype, at)
+
+
 @pytest.mark.parametrize("hidden,experts,ff,shared,top,gated,own_gate", [
     (16, 1, 16, 0, 1, True, False), (272, 8, 80, 48, 2, True, True), (400, 5, 384, 0, 3, False, False),
     (128, 70, 32, 16, 6, True, False), (2048, 8, 1024, 2048, 4, False, True)])

@@ -1,5 +1,5 @@
 // The sums of one 256 x 256 tile of x[rows, K] w[columns, K]^T, bfloat16 operands and float32 sums on the matrix cores, by a
-// block of eight waves: the loop that the products of many rows are built on (moe_rows.hip).
+// block of eight waves: the loop that the products of many rows are built on (moe_rows.hip, gemm_block.hip).
 //
 // What bounds it is the matrix pipe, so the loop keeps it fed. The chunk of 64 columns of K of both operands (64 KB) lies in
 // LDS twice, the one being multiplied and the one on its way, copied by the memory pipeline (global_load_lds, rows of 128

@@ -175,7 +175,7 @@ void launch_rows_tall(const void* x, const void* w, void* y, int M, int N, int K
 }
 }  // namespace
 
-// 17 to 64 rows over weights too narrow for the form above: a block one tile of 16 columns, K split over its waves in order, every wave
+// 17 to 40 rows over weights too narrow for the form above: a block one tile of 16 columns, K split over its waves in order, every wave
 // reading its share of the rows from L2 (the few-row kernel's shape with MT tiles of tokens). One launch where a product in shares takes
 // two; bound by what the blocks read of the rows, N / 16 times all of them.
 namespace {

@@ -1932,7 +1932,7 @@ static int prefill_launch(const void* q, void* out, const void* pages, const int
                           const int32_t* slots, const int32_t* lens, const int32_t* query_start, const int32_t* row_ids,
                           int n_rows, int max_query, int max_len, int heads, int kv_heads, int head_dim, int page_size,
                           float scale, int window, const float* sink, void* stream, const ScoreMod* mod = nullptr,
-                          int v_share = 1, const void* hgate = nullptr, int64_t hgate_stride = 0) {
+                          int v_share = 1, const void* hgate = nullptr, int64_t hgate_stride = 0, bool staged_256 = true) {
   HOLON_CHECK(mfma_serves(head_dim, page_size), "attention (matrix cores): head_dim %d / page %d not served", head_dim,
               page_size);
   HOLON_CHECK(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && window > -0x7fffffff && table_stride > 0,
@@ -1964,7 +1964,7 @@ static int prefill_launch(const void* q, void* out, const void* pages, const int
   const TileMap32 few = tile_map32(heads / kv_heads);
   const int64_t few_ranges = (int64_t)(((max_query + few.pos_per_tile - 1) / few.pos_per_tile + 3) / 4) * kv_heads * n_rows;
   if (g_prefill_dma && heads / kv_heads <= 32 && tiles >= 16 && max_len <= 4096 * page_size &&
-      (mod != nullptr ? head_dim == 128 && few_ranges >= 384 : head_dim == 256 && max_len > 192)) {
+      (mod != nullptr ? head_dim == 128 && few_ranges >= 384 : head_dim == 256 && staged_256 && max_len > 192)) {
     const TileMap32 tm32 = tile_map32(heads / kv_heads);
     const int ranges32 = ((max_query + tm32.pos_per_tile - 1) / tm32.pos_per_tile + 3) / 4;
     a.unpaired = (int64_t)((ranges32 + 1) / 2) * kv_heads * n_rows < UNPAIR_BELOW ? 1 : 0;
@@ -2057,6 +2057,17 @@ extern "C" int holon_attention_prefill_sink_bf16(const void* q, void* out, const
                                                  void* stream) {
   return prefill_launch(q, out, pages, table, table_stride, slots, lens, query_start, row_ids, n_rows, max_query, max_len,
                         heads, kv_heads, head_dim, page_size, scale, window, sink, stream);
+}
+
+// The same with the operands of heads of 256 straight from the cache whatever the rows' length, in the order of sums that short rows have.
+extern "C" int holon_attention_prefill_from_cache_bf16(const void* q, void* out, const void* pages, const int32_t* table,
+                                                       int table_stride, const int32_t* slots, const int32_t* lens,
+                                                       const int32_t* query_start, const int32_t* row_ids, int n_rows,
+                                                       int max_query, int max_len, int heads, int kv_heads, int head_dim,
+                                                       int page_size, float scale, int window, const float* sink,
+                                                       void* stream) {
+  return prefill_launch(q, out, pages, table, table_stride, slots, lens, query_start, row_ids, n_rows, max_query, max_len,
+                        heads, kv_heads, head_dim, page_size, scale, window, sink, stream, nullptr, 1, nullptr, 0, false);
 }
 
 // Prompt portions of windowed attention with sigmoid weights (head sizes 64 and 128, keys and values of one width,

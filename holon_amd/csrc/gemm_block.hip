@@ -147,9 +147,9 @@ extern "C" int holon_gemm_block_glu_bf16(const void* x, const void* w, void* y, 
 extern "C" int holon_gemm_block_parts_serves(int M, int N, int K, int splits) {
   return M > 128 && M <= 1024 && N % TILE == 0 && holon_gemm_block_supported(M, N, K, 0, splits) && (K % 1024 == 0 || M > 512);
 }
-// The number of shares, a power of two up to eight, that is done first: rounds of a tile's loop a compute unit, and the parts' traffic (of
-// 24 products of three widths the choice is at most 6 % from the best).
-int block_parts_splits(int M, int N, int K) {
+// The number of shares, a power of two up to eight, that is done first (0: none is served): rounds of a tile's loop a compute unit, and the
+// parts' traffic (of 24 products of three widths the choice is at most 6 % from the best).
+extern "C" int holon_gemm_block_parts_splits(int M, int N, int K) {
   const int tiles = row_tiles_of(M) * ((N + TILE - 1) / TILE);
   int best = 0;
   float least = 0.f;

@@ -163,8 +163,6 @@ extern "C" int holon_gemm_tiles_parts_supported(int M, int N, int K, int splits)
          (int64_t)M * K * 2 < (int64_t)1 << 32;             // (a lane's place among the rows is a 32-bit byte offset)
 }
 
-int block_parts_splits(int M, int N, int K);
-
 // How many shares of K to take, 0 where the kernel does not serve the shape or is not the one to take: it is for
 // weights whose K is well above their N (few output tiles, long sums), with as few shares (a power of two, at most
 // eight) as give 384 blocks. Measured on MI355X with the add + norm that reads the parts, against the vendor library's
@@ -180,9 +178,7 @@ extern "C" int holon_gemm_tiles_splits(int M, int N, int K) {
   int splits = 1;
   while (splits < TILES_MAX_SPLITS && blocks * splits < 384) splits *= 2;
   while (splits > 1 && K % (TILES_KC * splits)) splits /= 2;
-  if (!holon_gemm_tiles_parts_supported(M, N, K, splits) || blocks * splits < 128) return 0;
-  const int whole = block_parts_splits(M, N, K);          // (in shares of 256 x 256 tiles: gemm_block.hip)
-  return whole ? whole : splits;
+  return holon_gemm_tiles_parts_supported(M, N, K, splits) && blocks * splits >= 128 ? splits : 0;
 }
 
 // parts[s][M][N] (float32) = x[:, share s of K] w[:, share s of K]^T over tiled weights, 129 <= M <= 1,024.

@@ -79,6 +79,13 @@ int holon_attention_prefill_sink_bf16(const void* q, void* out, const void* page
                                       const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_query,
                                       int max_len, int heads, int kv_heads, int head_dim, int page_size, float scale,
                                       int window, const float* sink, void* stream);
+// The prompt entry point with heads of 256 read straight from the cache whatever the rows' length (a row of more than 192 tokens has its
+// stages copied into LDS otherwise, in another order of sums).
+int holon_attention_prefill_from_cache_bf16(const void* q, void* out, const void* pages, const int32_t* table,
+                                            int table_stride, const int32_t* slots, const int32_t* lens,
+                                            const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_query,
+                                            int max_len, int heads, int kv_heads, int head_dim, int page_size, float scale,
+                                            int window, const float* sink, void* stream);
 int holon_attention_decode_sink_bf16(const void* q, void* out, const void* pages, const int32_t* table,
                                      int table_stride, const int32_t* slots, const int32_t* lens,
                                      const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_len,
@@ -180,7 +187,9 @@ int holon_gemm_tiles_parts_bf16(const void* x, const void* w_tiled, void* parts,
 // Products of many rows on 256 x 256 tiles over untiled weights (gemm_block.hip): the same parts, and a gated feed-forward's first product
 // with its activation, y [M, N] from w [2 N, K] (gates, then ups; act 0 silu, 1 gelu in its tanh form).
 int holon_gemm_block_supported(int M, int N, int K, int gated, int splits);
+// The parts in place of holon_gemm_tiles_parts_bf16's: which numbers of shares are served, and the one to take (0: none).
 int holon_gemm_block_parts_serves(int M, int N, int K, int splits);
+int holon_gemm_block_parts_splits(int M, int N, int K);
 int holon_gemm_block_parts_bf16(const void* x, const void* w, void* parts, int M, int N, int K, int splits, void* stream);
 int holon_gemm_block_glu_bf16(const void* x, const void* w, void* y, int M, int N, int K, int act, void* stream);
 int holon_sum_parts(const void* parts, void* y, int splits, int64_t count, void* stream);

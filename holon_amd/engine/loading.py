@@ -101,6 +101,8 @@ def assemble(cfg: EngineConfig, kernels=None, *, random_config: dict | None = No
     model, _ = build_from_spec(spec, device=device, dtype=dtype, kernels=kernels, page_size=cfg.page_size,
                                max_seqs=cfg.max_seqs, max_model_len=cfg.max_model_len,
                                max_step_tokens=cfg.max_step_tokens, decode_copy=cfg.decode_weight_copy)
+    if configured is not None:
+        kernels.settled = any(part.amplifies for part in model.walk())
     if random_config is not None:
         fill_random(model, spec, seed, device, dtype)
     else:

@@ -58,6 +58,7 @@ def glu_block_pays(rows: int, inter: int, hidden: int) -> bool:
 
 class HipKernels:
     name = "hip-gfx950"
+    settled = False           # see `configured`
     _instance: "HipKernels | None" = None
 
     @classmethod
@@ -104,6 +105,8 @@ class HipKernels:
                                                   _P, _P, _I, _I, _I, _I, _P],
             "holon_attention_prefill_sink_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
                                                   _P, _P],
+            "holon_attention_prefill_from_cache_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
+                                                        _P, _P],
             "holon_attention_decode_sink_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I,
                                                  _P, _P, _I, _I, _I, _I, _P, _P],
             "holon_attention_prefill_mod_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
@@ -130,6 +133,7 @@ class HipKernels:
             "holon_gemm_tiles_parts_bf16": [_P, _P, _P, _I, _I, _I, _I, _P],
             "holon_gemm_block_supported": [_I, _I, _I, _I, _I],
             "holon_gemm_block_parts_serves": [_I, _I, _I, _I],
+            "holon_gemm_block_parts_splits": [_I, _I, _I],
             "holon_gemm_block_parts_bf16": [_P, _P, _P, _I, _I, _I, _I, _P],
             "holon_gemm_block_glu_bf16": [_P, _P, _P, _I, _I, _I, _I, _P],
             "holon_sum_parts": [_P, _P, _I, _L, _P],
@@ -155,7 +159,9 @@ class HipKernels:
     def configured(self, products: str = "own", pins=None) -> "HipKernels":
         """The same kernels with product choices of their own: an engine's `products` mode and `product_pins`. The
         library, and the record of tiled weights by shape, are shared; what a product took is per engine
-        (`plan.taken`)."""
+        (`plan.taken`). `settled` (set on the result, by whoever puts a model with an amplifying part together): steps of
+        17 rows and more keep the forms whose order of sums such a model's logits have been compared in: no 256 x 256
+        tiles, no narrow products in one launch, heads of 256 straight from the cache."""
         other = copy.copy(self)
         other.plan = ProductPlan(products, pins)
         return other
@@ -491,6 +497,8 @@ class HipKernels:
         must serve the shape and, timed once per weight shape and row bucket against the vendor library's product of
         the same rows (outside graph capture), be the faster of the two."""
         n, k = weight.shape
+        if self.settled and not gated and n <= 4096:      # (what is so narrow takes one launch, or the library)
+            return False
         if not (tiled is not None and weight.dtype == torch.bfloat16 and 16 < rows <= 64
                 and self.lib.holon_gemm_rows_supported(rows, n // 2 if gated else n, k, int(gated))):
             return False
@@ -525,24 +533,25 @@ class HipKernels:
         splits = (self.lib.holon_gemm_rows_splits if m <= self.parts_rows_short else self.lib.holon_gemm_tiles_splits)(m, n, k)
         if not splits:
             return None
-        use = self.product_choice("parts", weight, m, lambda: self._time_parts(x, weight, tiled, splits))
-        return self._rows_parts(x, weight, tiled, splits) if use == "parts" else None
+        whole = 0 if self.settled or (x.data_ptr() | weight.data_ptr()) % 16 else self.lib.holon_gemm_block_parts_splits(m, n, k)
+        how = (whole, True) if whole else (splits, False)
+        use = self.product_choice("parts", weight, m, lambda: self._time_parts(x, weight, tiled, *how))
+        return self._rows_parts(x, weight, tiled, *how) if use == "parts" else None
 
-    def _rows_parts(self, x, weight, tiled, splits):
+    def _rows_parts(self, x, weight, tiled, splits, whole=False):
+        """`whole`: on 256 x 256 tiles, over the weight as it is."""
         (m, k), n = x.shape, weight.shape[0]
         self._check_product("linear in parts", x, weight, tiled)
         if tiled is None or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.shape[1] != k:
             raise KernelError(f"linear in parts: bfloat16 rows {tuple(x.shape)} over a tiled bfloat16 weight "
                               f"{tuple(weight.shape)} expected")
         parts = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
-        if self.lib.holon_gemm_block_parts_serves(m, n, k, splits) and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0:
-            entry, source = self.lib.holon_gemm_block_parts_bf16, weight
-        else:
-            entry, source = self.lib.holon_gemm_rows_parts_bf16 if m <= self.parts_rows_short else self.lib.holon_gemm_tiles_parts_bf16, tiled
-        self._call(entry, x.data_ptr(), source.data_ptr(), parts.data_ptr(), m, n, k, splits, self._stream())
+        entry = self.lib.holon_gemm_block_parts_bf16 if whole else \
+            self.lib.holon_gemm_rows_parts_bf16 if m <= self.parts_rows_short else self.lib.holon_gemm_tiles_parts_bf16
+        self._call(entry, x.data_ptr(), (weight if whole else tiled).data_ptr(), parts.data_ptr(), m, n, k, splits, self._stream())
         return parts
 
-    def _time_parts(self, x, weight, tiled, splits) -> str:
+    def _time_parts(self, x, weight, tiled, splits, whole=False) -> str:
         """Each way together with the residual add + norm that reads the product (reading parts costs that kernel a
         little, which the product must win back)."""
         n = weight.shape[0]
@@ -552,7 +561,7 @@ class HipKernels:
         rival = self._MID_FORMS[self._time_mid_forms(x, weight)]      # the vendor library's best form (kept only if it wins)
         took = {
             "parts": self._graph_time(self._in_turn(
-                pairs, lambda w, t: self.add_rmsnorm(self._rows_parts(x, w, t, splits), residual, ones, 1e-6))),
+                pairs, lambda w, t: self.add_rmsnorm(self._rows_parts(x, w, t, splits, whole), residual, ones, 1e-6))),
             "vendor": self._graph_time(self._in_turn(
                 pairs, lambda w, _t: self.add_rmsnorm(rival(x, w), residual, ones, 1e-6)))}
         return "parts" if took["parts"] < 0.97 * took["vendor"] else "vendor"
@@ -620,7 +629,7 @@ class HipKernels:
         """silu_mul(linear(x, weight)) for prompts on 256 x 256 tiles, the activation in the epilogue, where that is done sooner than by
         the vendor library's product and a kernel for the activation (a product choice of kind `glu`); None elsewhere."""
         (m, k), inter = x.shape, weight.shape[0] // 2
-        if not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.shape[1] == k and weight.shape[0] % 2 == 0
+        if self.settled or not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.shape[1] == k and weight.shape[0] % 2 == 0
                 and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
                 and glu_block_pays(m, inter, k) and self.lib.holon_gemm_block_supported(m, inter, k, 1, 1)):
             return None
@@ -757,7 +766,8 @@ class HipKernels:
             common = (q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), table.shape[1],
                       rows.slots.data_ptr(), rows.lens.data_ptr(), rows.query_start.data_ptr())
             if rows.n_chunk:
-                self._call(self.lib.holon_attention_prefill_sink_bf16, *common, rows.chunk_rows.data_ptr(), rows.n_chunk,
+                prefill = self.lib.holon_attention_prefill_from_cache_bf16 if self.settled else self.lib.holon_attention_prefill_sink_bf16
+                self._call(prefill, *common, rows.chunk_rows.data_ptr(), rows.n_chunk,
                            rows.max_chunk_query, rows.max_chunk_len, hq, hkv, d, page_size, float(scale), int(window),
                            _ptr(sink), self._stream())
             if rows.n_decode:

@@ -112,6 +112,9 @@ class Part:
 
     reads_origin = False      # a block that needs the embedding's rows beside the stream (`Stream.origin`)
     adds_residual = False     # its forward accepts `residual=h`: it may add its result into h and return None
+    amplifies = False         # True: it brings what may be near nothing to unit length, so that a change of rounding in front
+                              # of it moves single rows of the logits further than rounding otherwise does. A model with
+                              # such a part keeps the orders of sums that its logits have (`HipKernels.configured`).
     graph_safe = False        # True: a captured step may be replayed over it. Its forward then reads nothing on the
                               # host that changes from step to step (no `step.h_*`, no `.item()`, no shapes that depend
                               # on values) and launches the same kernels on the same buffers whatever the rows are.

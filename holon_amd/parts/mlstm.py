@@ -110,6 +110,10 @@ class MLSTM(Part):
     pre-activations; `eps` is that of the per-head division by the root mean square."""
 
     graph_safe = True
+    # A head whose n . q passes through zero has a read-out near nothing, which the norm per head then brings to unit length.
+    # Measured over a model of eight layers (two of them this one, width 2,048, bfloat16): two orders of a float32 sum in front of
+    # it move single rows of the logits by 0.003 to 0.02 of their rms over most weights, by up to 0.1 over some.
+    amplifies = True
 
     def __init__(self, build: Build, *, heads: int, dim: int, vdim: int, gate_cap: float, eps: float, hidden: int,
                  layer: int, name: str = "") -> None:

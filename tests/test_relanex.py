@@ -683,3 +683,44 @@ def test_the_matrix_memory_in_pieces_at_its_edges(heads, d, v, dtype):
     # numerators and denominators apart, each within the rounding of a running maximum of some 10 (2^-24 * 10, and as much for the
     # gates' sums): their ratio is as far off as a denominator is near 0
     assert _rel(got, want) < 1e-5 and _rel(den, ref) < 1e-5 and all(_rel(a, b) < 1e-5 for a, b in zip(one, two))
+
+
+@pytest.mark.gpu
+def test_prompts_keep_the_orders_of_sums_they_have():
+    """A matrix memory's norm brings a read-out near nothing to unit length, so that any other order of a sum in front of it can move a
+    row by more than rounding does: a model with one keeps the forms of 17 rows and more that its logits have been compared in (the
+    library's gated product and narrow products, shares of K on tiles of 128 rows, heads of 256 from the cache), models without do not."""
+    from holon_amd import benchmark
+    from holon_amd.engine.loading import load_model
+    from holon_amd.kernels import load_hip
+    sizes = dict(width=256, layers=4, heads=2, kv_heads=1, dim=64, ff=512, vocab=256)
+    of = {name: load_model("random", page_size=16, max_seqs=2, max_model_len=64, max_step_tokens=64, cache_tokens=128, seed=3,
+                           random_config=cfg).kernels
+          for name, cfg in (("relanex", benchmark.relanex_config(sizes)), ("qwen3", benchmark.qwen3_config(sizes)))}
+    hip = load_hip()
+    assert of["relanex"].settled and not of["qwen3"].settled and not hip.settled
+    bf, g = torch.bfloat16, torch.Generator().manual_seed(5)
+    draw = lambda *shape: (0.1 * torch.randn(*shape, generator=g)).cuda().to(bf)        # noqa: E731
+    k = of["relanex"]
+    x, up = draw(2048, 256), draw(2 * 4096, 256)
+    assert k.linear_silu_mul(x, up) is None and of["qwen3"].linear_silu_mul(x, up) is not None
+    x, down = draw(300, 8192), draw(2048, 8192)
+    tiled = hip.tile_weight(down)
+    parts = k.linear_parts(x, down, tiled)
+    want = torch.empty_like(parts)
+    hip._call(hip.lib.holon_gemm_tiles_parts_bf16, x.data_ptr(), tiled.data_ptr(), want.data_ptr(), 300, 2048, 8192, parts.shape[0],
+              hip._stream())
+    assert torch.equal(parts, want) and parts.shape[0] == hip.lib.holon_gemm_tiles_splits(300, 2048, 8192)
+    x, narrow = draw(32, 2048), draw(2048, 2048)
+    assert torch.equal(k.linear(x, narrow, tiled=hip.tile_weight(narrow)), torch.matmul(x, narrow.t()))
+    from holon_amd.kernels.api import AttnRows
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                   # noqa: E731
+    rows = AttnRows(slots=i32([0]), lens=i32([300]), query_start=i32([0, 300]), decode_rows=i32([]), chunk_rows=i32([0]), n_decode=0,
+                    n_chunk=1, max_decode_len=0, max_chunk_query=300, max_chunk_len=300)
+    q, pages, table = draw(300, 16, 256), draw(19, 2, 1, 16 * 256), i32([list(range(19))])
+    got = k.paged_attention(q, pages, table, rows, 16, 1 / 16, 0)
+    was = hip.lib.holon_attention_prefill_copies(0)
+    try:
+        assert torch.equal(got, hip.paged_attention(q, pages, table, rows, 16, 1 / 16, 0))
+    finally:
+        hip.lib.holon_attention_prefill_copies(was)

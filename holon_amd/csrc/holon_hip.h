@@ -322,8 +322,8 @@ int holon_softmax_attention(const void* q, void* out, const void* pages, const i
                             int tokens, int heads, int kv_heads, int dim, int vdim, int page_size, int num_pages,
                             const float* sink, float scale, int window, int dtype, float softcap, const float* r1,
                             const float* r2, int keep_first, int v_share, void* stream);
-// The same for prompts of the 32-bit path, on the float64 matrix cores (attention_f64.hip): heads of 64 or 128, dim = vdim, pages
-// of a multiple of 16 tokens.
+// The same for the 32-bit path on the float64 matrix cores (attention_f64.hip): heads of 64 or 128, dim = vdim, pages of a multiple of
+// 16 tokens. A caller that wants one order of sums for a position whatever the step is takes one of the two for all steps.
 int holon_softmax_attention_f64_supported(int heads, int kv_heads, int dim, int vdim, int page_size);
 int holon_softmax_attention_f64(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
                                 int table_rows, const int32_t* slots, const int32_t* token_row, const int32_t* positions,

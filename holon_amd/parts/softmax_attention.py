@@ -76,9 +76,9 @@ def softmax_attention_plain(q, pages, table, rows, token_row, positions, kv_head
 
 
 def _float64_sums_serve(heads, kv_heads, dim, vdim, page_size):
-    """What the library's `holon_softmax_attention_f64_supported` answers. That kernel takes float32 steps that bring 16 tokens a row
-    or more, at least 64 in all (measured, us, against the general one: 8 tokens a row of 16 rows, 16 heads of 128 on 4, 13.7 and
-    15.2, each head its own keys 20.7 and 15.5; one row of 37 tokens 30.7 and 12.6, of 65 14.9 and 16.8, of 700 106 and 407)."""
+    """What the library's `holon_softmax_attention_f64_supported` answers. That kernel takes every float32 step of such heads, prompts (four
+    times as fast) and decode rows (1.2 to 1.4 times the general one's time) alike: their orders of sums differ, and a position has the
+    same bits whatever step it comes in only if one of the two takes them all."""
     return dim == vdim and dim in (64, 128) and page_size % 16 == 0 and heads % kv_heads == 0 \
         and kv_heads * -(-(heads // kv_heads) // 16) <= 65535
 
@@ -100,7 +100,7 @@ def _softmax_attention_hip(launch, q, pages, table, rows, token_row, positions, 
                          f"{kv_heads} kv heads, values of {vdim}, page {page_size}")
     out = torch.empty((t, heads * vdim), dtype=q.dtype, device=q.device)
     general, wide = launch
-    kernel = wide if q.dtype == torch.float32 and t >= 64 and t >= 16 * rows.slots.shape[0] and not (window > 0 and keep_first > 0) \
+    kernel = wide if q.dtype == torch.float32 and not (window > 0 and keep_first > 0) \
         and _float64_sums_serve(heads, kv_heads, dim, vdim, page_size) and q.data_ptr() % 16 == 0 and pages.data_ptr() % 16 == 0 \
         else general
     kernel(q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), table.shape[1], table.shape[0],

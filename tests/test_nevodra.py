@@ -648,6 +648,58 @@ def test_float32_prompts_on_the_float64_cores(heads, groups, dim, page, share):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads,groups,dim", [(16, 4, 128), (4, 4, 64), (6, 2, 128), (40, 2, 64)])
+def test_float32_attention_has_the_same_bits_in_every_step(heads, groups, dim):
+    """Float32 `softmax_attention`: a position's result in a whole prompt, in portions of any size from one token on, decoded, and beside
+    rows of other lengths, is one; so is a padded row's (zeros). The steps lie on either side of 64 tokens and of 16 a row."""
+    import holon_amd.parts  # noqa: F401
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.api import AttnRows
+    k, dev, page = load_hip(), "cuda", 16
+    g = torch.Generator().manual_seed(heads)
+    lens = [130, 75, 33, 201]
+    table = torch.full((4, 13), -1, dtype=torch.int32)
+    order = torch.randperm(sum(-(-n // page) for n in lens), generator=g).tolist()
+    for b, n in enumerate(lens):
+        for i in range(-(-n // page)):
+            table[b, i] = order.pop()
+    pages = torch.randn(int(table.max()) + 1, 2 * groups * page * dim, generator=g).to(dev)
+    q = [torch.randn(n, heads, dim, generator=g).to(dev) for n in lens]
+    sink, table = torch.randn(heads, generator=g).to(dev), table.to(dev)
+    r1, r2 = torch.rand(heads, generator=g).to(dev), torch.rand(heads, generator=g).to(dev)
+
+    def step(parts, window, cap, pad=0):
+        """parts: (row, first, tokens); `pad` rows of one token at position -1 behind them."""
+        i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)          # noqa: E731
+        counts = [n for _, _, n in parts] + [1] * pad
+        starts = [0]
+        for n in counts:
+            starts.append(starts[-1] + n)
+        rows = AttnRows(slots=i32([r for r, _, _ in parts] + [0] * pad), lens=i32([at + n for _, at, n in parts] + [0] * pad),
+                        query_start=i32(starts), decode_rows=i32([]), chunk_rows=i32(list(range(len(counts)))), n_decode=0,
+                        n_chunk=len(counts), max_decode_len=0, max_chunk_query=max(counts), max_chunk_len=max(lens))
+        x = torch.cat([q[r][at: at + n] for r, at, n in parts] + [q[0][:1]] * pad).contiguous()
+        out = k.softmax_attention(x, pages, table, rows, i32([b for b, n in enumerate(counts) for _ in range(n)]),
+                                  i32([at + i for _, at, n in parts for i in range(n)] + [-1] * pad), groups, dim, page, sink,
+                                  dim ** -0.5, window, softcap=cap, dist=(r1, r2) if cap else None)
+        return [out[starts[b]: starts[b] + n] for b, n in enumerate(counts)]
+    for window, cap in ((0, 0.0), (40, 3.0), (-64, 0.0)):
+        whole = [step([(r, 0, n)], window, cap)[0] for r, n in enumerate(lens)]
+        together = step([(r, 0, n) for r, n in enumerate(lens)], window, cap)
+        assert all(torch.equal(a, b) for a, b in zip(together, whole)), (window, cap)
+        for size in (1, 3, 17, 64):
+            for at in range(0, 201, size):
+                n = min(size, 201 - at)
+                if n < size or size > 1 or at % 29 == 0:
+                    assert torch.equal(step([(3, at, n)], window, cap)[0], whole[3][at: at + n]), (window, size, at)
+        mixed = [(0, 129, 1), (1, 74, 1), (2, 30, 3), (3, 5, 196)]
+        for parts in (mixed, mixed[::-1], mixed[:3]):
+            for (r, at, n), got in zip(parts, step(parts, window, cap, pad=2)):
+                assert torch.equal(got, whole[r][at: at + n]), (window, parts)
+            assert not any(v.any() for v in step(parts, window, cap, pad=2)[len(parts):])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_kernels_alone_against_their_plain_forms(dtype):
     """Every operation the design brought, on the GPU, against its plain form in torch: odd widths, rows wider than a

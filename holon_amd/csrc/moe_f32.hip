@@ -99,8 +99,8 @@ __global__ void __launch_bounds__(SHARES * WAVE) moe_down_few_f32_kernel(const f
 }
 
 constexpr int ROWS = 64, XCDS = 8;
-// Which tile a block takes, of all experts' and, before them, the shared one's: false: none. `width`, `wide`: columns and tiles of
-// columns of a routed expert and of the shared one.
+// Which tile a block takes: of all experts' rows (`rows`; not `routed`: the shared one's, which come first) and the tile of columns `col`.
+// take: false where there is none for it; `routed_cols`, `shared_cols`: tiles of columns a routed expert and the shared one have.
 struct Taken {
   RowTile rows;
   bool routed;

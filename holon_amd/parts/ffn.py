@@ -469,26 +469,18 @@ def moe_f32_serves(rows: int, hidden: int, experts: int, top: int, ff: int, shar
         and max(2 * (experts * ff + shared), experts * rows, rows * top) < 1 << 31
 
 
-def moe_f32_pays(rows: int, hidden: int, experts: int, ff: int, shared: int, gated: bool, top: int) -> bool:
-    """Whether a float32 step is done sooner over the rows that chose an expert than with all rows over all experts. Up to 16 rows: what
-    the weights that no row is expected to choose take at 3 TB/s against a start an expert chosen and the search for them. From 64 rows
-    on: tiles of 64 x 64 by their length and a start. Measured on MI355X, us, own rows / all: 8 experts of 2,048 x 2,048 (squared ReLU)
-    beside a shared one, 2 a row, at 1 / 4 / 12 / 64 / 700 rows 53 / 102 / 125 / 204 / 460 and 110 / 111 / 123 / 248 / 1,199; 8 of 1,024
-    (gated) beside one of 2,048, 4 a row, at 1 / 4 / 64 / 700 70 / 98 / 190 / 703 and 95 / 95 / 200 / 945; 64 of 512 x 1,024, 6 a row, at
-    4 / 16 / 700 93 / 212 / 294 and 156 / 194 / 1,629; 128 of 64 x 2,048, 8 a row, at 4 / 64 / 200 73 / 147 / 150 and 80 / 121 / 303."""
-    if rows <= 16:
-        left = experts * (1 - top / experts) ** rows
-        return left * ff * hidden * (12 if gated else 8) / 3e6 > 2 + 1.5 * (experts - left) + 0.01 * rows * experts
-    if rows < 64:
-        return False
-
-    def work(row_tiles, columns, tile, length):            # of products of `columns` columns, `tile` wide, over `length` of K
-        return row_tiles * -(-columns // tile) * (length + 200)
-    routed, whole, wide = max(min(experts, rows * top), rows * top / 64 + experts / 2), -(-rows // 64), 32 if gated else 64
+def moe_f32_takes(hidden: int, experts: int, ff: int, shared: int, gated: bool, top: int) -> bool:
+    """Whether a float32 mixture's steps go over the rows that chose an expert, by its sizes alone: the two forms' orders of sums
+    differ, and a row has the same bits whatever step it comes in only if one of them takes them all. It is taken where a row chooses
+    at most half of the experts and its parts (which steps of more than 16 rows keep) take no more memory than the products over all.
+    Measured on MI355X, us, own rows / all: 8 experts of 2,048 x 2,048 (squared ReLU) beside a shared one, 2 a row, at 1 / 4 / 8 / 16 / 17 /
+    32 / 64 / 700 rows 52 / 92 / 116 / 136 / 201 / 203 / 203 / 460 and 110 / 111 / 115 / 132 / 152 / 177 / 245 / 1,199; 8 of 1,024 (gated) beside
+    one of 2,048, 4 a row, at 1 / 4 / 16 / 17 / 64 / 700 72 / 86 / 123 / 190 / 190 / 703 and 95 / 96 / 109 / 128 / 201 / 945; 64 of 512 x 1,024,
+    6 a row, at 1 / 8 / 16 / 32 / 700 40 / 143 / 205 / 185 / 294 and 158 / 163 / 194 / 250 / 1,629; 8 of 3,072 x 4,096 (gated) beside a shared one,
+    2 a row, at 1 / 16 / 32 161 / 441 / 561 and 533 / 588 / 659; 128 of 64 x 2,048, 8 a row, at 1 / 8 / 16 / 63 / 200 38 / 114 / 171 / 146 / 150 and
+    80 / 83 / 92 / 123 / 310. Decode rows and prompts gain, some 8 to 40 rows a step of small experts lose."""
     cols = experts * ff + shared
-    own = work(routed, ff, wide, hidden) + work(routed, hidden, 64, ff)
-    own += (work(whole, shared, wide, hidden) + work(whole, hidden, 64, shared)) if shared else 0
-    return own < 1.12 * (work(whole, cols, wide, hidden) + work(whole, hidden, 64, cols))
+    return 2 * top <= experts and top * ff + shared + (top + 1) * hidden + experts + top <= (3 if gated else 2) * cols
 
 
 def _moe_f32_hip(launch, x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
@@ -585,9 +577,8 @@ class MoE(Part):
     another: the activations of experts a token did not choose are set to 0 in between (`moe_gate`), so the second
     product adds up exactly the chosen experts' weighted outputs, and the shared expert's columns ride in the same two
     products. Steps of few rows take the same two products over the chosen experts' columns alone (`moe_few`), steps of many
-    rows each expert's over the rows that chose it (`moe_rows`), and float32 steps of either kind the same (`moe_f32`), where
-    that is done sooner. Steps of as many rows launch the
-    same kernels whatever was chosen."""
+    rows each expert's over the rows that chose it (`moe_rows`), where that is done sooner; in float32 every step does the latter
+    (`moe_f32`) or none, by the mixture's sizes. Steps of as many rows launch the same kernels whatever was chosen."""
 
     graph_safe = True
 
@@ -671,8 +662,7 @@ class MoE(Part):
             weights = k.moe_router(x, self.router, self.correction if self.has_bias else None, self.top, self.groups,
                                    self.keep, self.scale)
         up, down = self.gate_up, self.all_down
-        if x.dtype == torch.float32 and moe_f32_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.shared, self.act == "silu",
-                                                     self.top):
+        if x.dtype == torch.float32 and moe_f32_takes(x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top):
             y = k.moe_f32(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",
                           shared_weight=self.shared_gated)
             if y is not None:

@@ -726,11 +726,15 @@ def test_every_expert_over_its_own_rows_where_that_is_done_sooner():
                                                  (64, 256, 2, 3, 128, 0), (0, 256, 8, 2, 128, 0), (1 << 22, 256, 8, 2, 128, 0)))
 
 
-def test_float32_experts_over_the_rows_that_chose_them_where_that_is_done_sooner():
-    from holon_amd.parts.ffn import moe_f32_pays, moe_f32_serves
-    assert [moe_f32_pays(m, 2048, 8, 2048, 2048, False, 2) for m in (1, 4, 12, 17, 64, 700)] == [True, True, False, False, True, True]
-    assert [moe_f32_pays(m, 2048, 8, 1024, 2048, True, 4) for m in (1, 4, 16, 63, 200)] == [True, False, False, False, True]
-    assert [moe_f32_pays(m, 2048, 128, 64, 0, True, 8) for m in (4, 16, 64, 200)] == [True, False, False, True]
+def test_float32_experts_over_the_rows_that_chose_them_whatever_the_step():
+    """By a mixture's sizes alone (hidden, experts, ff, shared, gated, top): at most half of the experts a row, and parts of no more
+    memory than the products over all."""
+    from holon_amd.parts.ffn import moe_f32_serves, moe_f32_takes
+    assert all(moe_f32_takes(*a) for a in ((2048, 8, 2048, 2048, False, 2), (2048, 8, 1024, 2048, True, 4), (2048, 128, 64, 0, True, 8)))
+    assert not any(moe_f32_takes(*a) for a in ((2048, 8, 1024, 2048, True, 5), (4096, 16, 64, 0, True, 8), (4096, 8, 1024, 0, False, 4),
+                                               (64, 1, 64, 0, True, 1)))
+    # values of float32 a row: 2 ff + 3 hidden + 10 for 16 ff (8 experts, ungated)
+    assert moe_f32_takes(1400, 8, 301, 0, False, 2) and not moe_f32_takes(1406, 8, 301, 0, False, 2)
     assert moe_f32_serves(700, 2048, 8, 2, 2048, 2048) and moe_f32_serves(1, 16, 1, 1, 16, 0)
     assert not any(moe_f32_serves(*a) for a in ((64, 40, 8, 2, 32, 0), (64, 32, 8, 2, 24, 0), (64, 32, 8, 2, 32, 8), (0, 32, 8, 2, 32, 0),
                                                 (64, 32, 2, 3, 32, 0)))

@@ -553,6 +553,39 @@ def test_graph_replays_equal_eager_steps(folders, name, dtype):
 
 
 @pytest.mark.gpu
+def test_float32_decode_rows_have_the_same_bits_in_every_step():
+    """A request's logits, float32, at sizes where few rows and many take kernels of their own (attention heads of 128, 8 experts of 2,048
+    beside a shared one): decoded alone, six at a time, from a graph whose rows are padded to eight, 20 at a time, and beside a prompt. (The
+    linear attention, whose steps of decode rows alone have a kernel of their own, is left out.)"""
+    from holon_amd import benchmark
+    from holon_amd.engine.loading import load_model
+    from holon_amd.engine.replay import Replayer
+    cfg = benchmark.sopepel_config(dict(benchmark.DESIGN_SIZES["2k"], layers=2, vocab=4096))
+    for layer in cfg["layers"]:
+        layer["mixer"]["right_scale"] = 0.0
+    prompts = [H.random_ids(n, 4096, 40 + n) for n in (70, 5, 33, 1, 17, 64, *range(2, 16))]
+    more = [H.random_ids(3, 4096, 90 + i) for i in range(len(prompts))]
+    got = {}
+    for how in ("alone", "six", "graph", "twenty", "beside"):
+        rep = Replayer(load_model("random", device="cuda", dtype="float32", page_size=16, max_seqs=24, max_model_len=160, max_step_tokens=256,
+                                  cache_tokens=4096, graphs=how == "graph", random_config=cfg, seed=2))
+        for r, p in enumerate(prompts):
+            rep.step([{"id": r, "tokens": p, "want": []}], ())
+        sets = [[r] for r in range(6)] if how == "alone" else [list(range(20 if how == "twenty" else 6))]
+        out = {}
+        for ids in sets:
+            for i in range(3):
+                entries = [{"id": r, "tokens": more[r][i: i + 1], "want": [0]} for r in ids]
+                if how == "beside":
+                    entries.insert(3, {"id": 100 + i, "tokens": H.random_ids(100, 4096, i), "want": []})
+                logits = rep.step(entries, (100 + i,) if how == "beside" else ())
+                out.update({(r, i): logits[at].clone() for at, r in enumerate(ids)})
+        got[how] = out
+    for how, out in got.items():
+        assert all(torch.equal(out[key], want) for key, want in got["alone"].items()), how
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_kernels_alone_against_their_plain_forms(dtype):
     """Every operation the design brought or changed, on the GPU, against its plain form in torch."""

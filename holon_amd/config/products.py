@@ -17,14 +17,15 @@ from `Engine.stats()["products"]` and given back as `EngineConfig.product_pins`,
 """
 from __future__ import annotations
 
-from collections.abc import Callable, Mapping
+from collections.abc import Callable, Mapping, Sequence
 
 MODES = ("own", "vendor", "timed")
 
 # kind -> (this package's form or the plain default, every form)
 KINDS: dict[str, tuple[str, tuple[str, ...]]] = {
     "rows": ("rows", ("rows", "vendor")),         # 17 to 64 rows over many tiles, rows shared through LDS
-    "glu": ("rows", ("rows", "vendor")),          # the same with SiLU-mul inside, and above 128 rows 256 x 256 tiles
+    "glu": ("rows", ("rows", "vendor")),          # the same with SiLU-mul inside, and above 128 rows 256 x 256 tiles (GELU too;
+                                                  # above 1,024 rows never timed)
     "parts": ("parts", ("parts", "vendor")),      # a narrow weight, K in shares: 17 to 128 rows; to 1,024 where K is well above N
     "vendor": ("bf16", ("bf16", "f32", "f32x2")),  # the vendor product's own forms (result type, K in halves)
 }
@@ -77,11 +78,15 @@ class ProductPlan:
         self.seconds = 0.0                        # what the timings cost
 
     def choose(self, kind: str, shape: tuple[int, int], bucket: int, time: Callable[[], str] | None = None,
-               yields: bool = False) -> str:
+               yields: "bool | Sequence[tuple[str, tuple[int, int]]]" = False,
+               by_rule: bool = False) -> str:
         """The form the product `kind` over a weight of `shape` takes at `bucket` rows. `time()` runs the candidates
         against each other and names the winner; it is called at most once per key, and only while the engine
         starts. `yields`: where nothing is pinned for this kind, a pinned form of the vendor library's product at this
-        shape and bucket keeps that product (pins of a run that had no other form to choose there)."""
+        shape and bucket keeps that product (pins of a run that had no other form to choose there); or the (kind, shape)
+        pairs of the products whose pins do. `by_rule`: start-up never times this kind at this bucket (a timed run's pins do
+        not name it): a pin wins and is recorded, else mode `vendor` has the library's form and the others this package's,
+        by the kind's own rule, and nothing is recorded."""
         key = key_of(kind, shape, bucket)
         form = self.taken.get(key)
         if form is not None:
@@ -89,8 +94,10 @@ class ProductPlan:
         own, forms = KINDS[kind]
         if key in self.pins:
             form, how = self.pins[key], "pinned"
-        elif yields and key_of("vendor", shape, bucket) in self.pins:
+        elif yields and any(key_of(*other, bucket) in self.pins for other in ([("vendor", shape)] if yields is True else yields)):
             form, how = forms[-1], "pinned"
+        elif by_rule:
+            return forms[-1] if self.mode == "vendor" else own
         elif self.mode == "vendor":
             form, how = forms[-1] if kind != "vendor" else "bf16", "vendor"
         elif self.mode == "timed" and self.resolving and time is not None:

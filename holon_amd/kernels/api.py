@@ -109,6 +109,10 @@ class Kernels(Protocol):
         """silu_mul(linear(x, weight)) fused, with the composition's roundings; None when not fused for this shape.
         `row_scale` as in `linear`."""
 
+    def linear_glu(self, x: torch.Tensor, weight: torch.Tensor, act: int) -> torch.Tensor | None:
+        """`linear_silu_mul` (`act` 0) or `linear_gelu_mul` (1) for steps of more than 128 rows over the weight as it is; None where the
+        composition is to be taken. (A kernel set without it: the operation registered in `parts/ffn.py`, which never serves.)"""
+
     def silu_mul(self, gate_up: torch.Tensor) -> torch.Tensor:
         """gate_up [T, 2I] (gate columns first) -> [T, I] = round(silu(gate)) * up."""
 

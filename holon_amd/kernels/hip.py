@@ -47,7 +47,8 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 
 def glu_block_pays(rows: int, inter: int, hidden: int) -> bool:
     """Whether a gated first product of many rows with its activation takes this package's 256 x 256 tiles (128 gates and their ups each):
-    where the rounds of one tile a compute unit that it takes are filled to 0.62 and more. Measured on MI355X, us, against the vendor
+    where the rounds of one tile a compute unit that it takes are filled to 0.62 and more (`hidden` does not enter: either side's time
+    is in proportion to it). Measured on MI355X, us, against the vendor
     library's product and the kernel of the activation: 12,288 x 4,096 at 520 / 600 / 1,024 / 2,048 / 4,096 rows (filled 0.76 / 0.44 /
     0.75 / 1 / 1) 101 / 160 / 169 / 280 / 551 and 124 / 124 / 176 / 307 / 596; 8,192 x 2,048 at 400 / 768 / 1,024 / 2,048 (0.39 / 0.75 / 1 / 1)
     42 / 45 / 52 / 101 and 39 / 52 / 65 / 122; 9,728 x 2,560 at 1,024 / 1,500 (0.59 / 0.87) 119 / 122 and 114 / 142."""
@@ -166,12 +167,12 @@ class HipKernels:
         other.plan = ProductPlan(products, pins)
         return other
 
-    def product_choice(self, kind: str, weight, rows: int, time=None, yields=False) -> str:
+    def product_choice(self, kind: str, weight, rows: int, time=None, yields=False, by_rule=False) -> str:
         """The one place a product's form is resolved: pinned, else by the engine's mode, else (mode `timed`, while
         the engine starts and outside graph capture) by timing the candidates once."""
         if time is not None and (not self.plan.resolving or torch.cuda.is_current_stream_capturing()):
             time = None
-        return self.plan.choose(kind, tuple(weight.shape), row_bucket(rows), time, yields)
+        return self.plan.choose(kind, tuple(weight.shape), row_bucket(rows), time, yields, by_rule)
 
     # -- operations that parts bring with them ----------------------------------------------------------------------
     _part_libs: dict[str, ctypes.CDLL] = {}       # libraries built from parts' own sources, by source path
@@ -581,7 +582,7 @@ class HipKernels:
         x = torch.randn(rows, weight.shape[1], device=weight.device).to(torch.bfloat16)
         pairs = self._alike(weight, tiled)
         rival = self._MID_FORMS[self._time_mid_forms(x, weight)]      # the vendor library's best form (kept only if it wins)
-        vendor = (lambda w, _t: self.silu_mul(rival(x, w))) if gated else (lambda w, _t: rival(x, w))
+        vendor = (lambda w, _t: self.silu_mul(torch.matmul(x, w.t()))) if gated else (lambda w, _t: rival(x, w))
         took = {"rows": self._graph_time(self._in_turn(pairs, lambda w, t: self._rows_product(x, w, t, gated))),
                 "vendor": self._graph_time(self._in_turn(pairs, vendor))}
         return "rows" if took["rows"] < took["vendor"] else "vendor"
@@ -625,9 +626,12 @@ class HipKernels:
                    int(tiled is not None), _ptr(stats), parts, eps, self._stream())
         return y
 
-    def _glu_block(self, x, weight):
-        """silu_mul(linear(x, weight)) for prompts on 256 x 256 tiles, the activation in the epilogue, where that is done sooner than by
-        the vendor library's product and a kernel for the activation (a product choice of kind `glu`); None elsewhere."""
+    def linear_glu(self, x, weight, act):
+        return self._glu_block(x, weight, act)
+
+    def _glu_block(self, x, weight, act=0):
+        """silu_mul(linear(x, weight)) (`act` 1: gelu_mul) for prompts on 256 x 256 tiles, the activation in the epilogue, where that is
+        done sooner than by the vendor library's product and a kernel for the activation (a product choice of kind `glu`); None elsewhere."""
         (m, k), inter = x.shape, weight.shape[0] // 2
         if self.settled or not (x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.shape[1] == k and weight.shape[0] % 2 == 0
                 and x.is_contiguous() and weight.is_contiguous() and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
@@ -637,17 +641,18 @@ class HipKernels:
 
         def block(w):
             y = torch.empty((m, inter), dtype=torch.bfloat16, device=x.device)
-            self._call(self.lib.holon_gemm_block_glu_bf16, x.data_ptr(), w.data_ptr(), y.data_ptr(), m, inter, k, 0, self._stream())
+            self._call(self.lib.holon_gemm_block_glu_bf16, x.data_ptr(), w.data_ptr(), y.data_ptr(), m, inter, k, act, self._stream())
             return y
 
         def time():
-            pairs = self._alike(weight, None)
+            pairs, mul = self._alike(weight, None), self.gelu_mul if act else self.silu_mul
             took = {"rows": self._graph_time(self._in_turn(pairs, lambda w, _t: block(w))),
-                    "vendor": self._graph_time(self._in_turn(pairs, lambda w, _t: self.silu_mul(torch.matmul(x, w.t()))))}
+                    "vendor": self._graph_time(self._in_turn(pairs, lambda w, _t: mul(torch.matmul(x, w.t()))))}
             return "rows" if took["rows"] < took["vendor"] else "vendor"
-        if m > self.parts_rows:                   # (beyond the steps that start-up times: by the rule above)
-            return None if self.plan.mode == "vendor" else block(weight)
-        return block(weight) if self.product_choice("glu", weight, m, time, yields=True) == "rows" else None
+        # (steps beyond those that start-up times: by the rule above, unless a pin or the mode says otherwise)
+        beyond = m > self.parts_rows
+        choice = self.product_choice("glu", weight, m, None if beyond else time, yields=True, by_rule=beyond)
+        return block(weight) if choice == "rows" else None
 
     def silu_mul(self, gate_up):
         self._check(gate_up, "silu_mul")

@@ -7,7 +7,6 @@ import ctypes
 
 import torch
 
-from ..kernels.hip import glu_block_pays
 from ..kernels.registry import KernelOp, register_kernel
 from ..registry import register_part
 from .base import FLOAT32, Build, Part, Stream
@@ -99,24 +98,23 @@ def linear_gelu_mul_plain(x, weight, tiled=None):
 
 
 def _linear_gelu_mul_hip(launch, x, weight, tiled=None):
-    """Steps of up to 16 bfloat16 rows: the few-row product with the activation in its epilogue; of many: 256 x 256 tiles with it in
-    theirs, where that is done sooner."""
-    few, block = launch
+    """Steps of up to 16 bfloat16 rows: the few-row product with the activation in its epilogue."""
     (m, k), n = x.shape, weight.shape[0]
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.is_contiguous()
-            and weight.is_contiguous() and weight.shape[1] == k and n % 32 == 0 and k % 128 == 0):
-        return None
-    if glu_block_pays(m, n // 2, k) and max(m, n) * k < 1 << 31 and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0:
-        y = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
-        block(x.data_ptr(), weight.data_ptr(), y.data_ptr(), m, n // 2, k, 1)
-        return y
-    if not (1 <= m <= 16 and k >= 256 and (tiled is None or (tiled.shape == weight.shape and tiled.dtype == weight.dtype
-                                                              and tiled.is_contiguous()))):
+            and weight.is_contiguous() and weight.shape[1] == k and 1 <= m <= 16 and n % 32 == 0 and k % 128 == 0
+            and k >= 256 and (tiled is None or (tiled.shape == weight.shape and tiled.dtype == weight.dtype
+                                                 and tiled.is_contiguous()))):
         return None
     y = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
-    few(x.data_ptr(), (tiled if tiled is not None else weight).data_ptr(), y.data_ptr(), m, n // 2, k,
+    launch(x.data_ptr(), (tiled if tiled is not None else weight).data_ptr(), y.data_ptr(), m, n // 2, k,
            int(tiled is not None))
     return y
+
+
+def linear_glu_plain(x, weight, act):
+    """A gated first product of many rows with its activation: what a kernel set that has a choice of forms for it answers for itself
+    (`kernels.api.Kernels.linear_glu`); the plain form is the composition."""
+    return None
 
 
 def polynorm_plain(z, coef, eps):
@@ -311,8 +309,9 @@ register_kernel(KernelOp("moe_router_top", moe_router_top_plain, "holon_moe_rout
 register_kernel(KernelOp("moe_relu2", moe_relu2_plain, "holon_moe_relu2", [_P, _P, _P, _L, _I, _I, _I, _I, _I, _I],
                          _moe_relu2_hip))
 register_kernel(KernelOp("gelu_mul", gelu_mul_plain, "holon_gelu_mul", [_P, _P, _L, _I, _I], _gelu_mul_hip))
-register_kernel(KernelOp("linear_gelu_mul", linear_gelu_mul_plain, ("holon_gemm_skinny_geglu_bf16", "holon_gemm_block_glu_bf16"),
-                         ([_P, _P, _P, _I, _I, _I, _I], [_P, _P, _P, _I, _I, _I, _I]), _linear_gelu_mul_hip))
+register_kernel(KernelOp("linear_gelu_mul", linear_gelu_mul_plain, "holon_gemm_skinny_geglu_bf16",
+                         [_P, _P, _P, _I, _I, _I, _I], _linear_gelu_mul_hip))
+register_kernel(KernelOp("linear_glu", linear_glu_plain))
 register_kernel(KernelOp("relu2", relu2_plain, "holon_relu2", [_P, _P, _L, _I], _relu2_hip))
 
 

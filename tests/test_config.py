@@ -191,3 +191,17 @@ def test_a_pinned_vendor_form_keeps_the_vendor_product():
     assert plan.choose("rows", (2048, 2048), 32, yields=True) == "rows"
     assert plan.choose("glu", (24576, 4096), 512, yields=True) == "rows"
     assert ProductPlan("own", {"vendor:4096x2048:32": "f32"}).choose("rows", (4096, 2048), 32) == "rows"
+
+
+def test_a_choice_by_rule_reads_pins_and_mode_and_records_pins_alone():
+    from holon_amd.config.products import ProductPlan
+
+    own, vendor = ProductPlan("own"), ProductPlan("vendor")
+    assert own.choose("glu", (8192, 256), 2048, by_rule=True) == "rows" and vendor.choose("glu", (8192, 256), 2048, by_rule=True) == "vendor"
+    assert ProductPlan("timed").choose("glu", (8192, 256), 2048, by_rule=True) == "rows"
+    assert own.report() == vendor.report() == {}
+    pins = {"glu:8192x256:2048": "vendor", "rows:512x256:64": "rows", "vendor:256x512:512": "f32"}
+    plan = ProductPlan("own", pins)
+    assert plan.choose("glu", (8192, 256), 2048, by_rule=True) == "vendor" and plan.how == {"glu:8192x256:2048": "pinned"}
+    over = [("rows", (512, 256)), ("vendor", (512, 256)), ("rows", (256, 512)), ("vendor", (256, 512))]
+    assert [plan.choose("glu", (512, 256), bucket, yields=over) for bucket in (64, 128, 512)] == ["vendor", "rows", "vendor"]

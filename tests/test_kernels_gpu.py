@@ -1072,6 +1072,27 @@ def test_products_on_tiles_of_256_rows(hip):
         hip._call(hip.lib.holon_gemm_block_parts_bf16, x.data_ptr(), w.data_ptr(), x.data_ptr(), 16, 16, 256, 4, hip._stream())
 
 
+@pytest.mark.parametrize("act", [0, 1])
+def test_gated_products_on_tiles_of_256_rows_are_a_product_choice(hip, act):
+    """In either activation: the mode `vendor`, a pin of the kind, and a pinned form of the library's product keep that product, at any
+    number of rows; what was taken is recorded (beyond the rows that a start times: if it was pinned)."""
+    x, w = _randn(2048, 256, dtype=torch.bfloat16), _randn(2 * 16384, 256, dtype=torch.bfloat16, scale=0.1)
+    for m, bucket in ((520, 768), (2048, 2048)):
+        for mode, pins, taken in (("own", {}, "rows"), ("vendor", {}, "vendor"), ("own", {f"glu:32768x256:{bucket}": "vendor"}, "vendor"),
+                                  ("vendor", {f"glu:32768x256:{bucket}": "rows"}, "rows"),
+                                  ("own", {f"vendor:32768x256:{bucket}": "f32"}, "vendor"), ("timed", {}, "rows")):
+            k = hip.configured(mode, pins)
+            got = k.linear_glu(x[:m], w, act)
+            assert (got is not None) == (taken == "rows"), (m, mode, pins)
+            by_rule = m > 1024 and not pins                 # (never timed: recorded only where it is pinned)
+            assert k.plan.report() == ({} if by_rule else {f"glu:32768x256:{bucket}": taken}), (m, mode, pins)
+            if got is not None and mode == "own":
+                assert torch.equal(got, hip._glu_block(x[:m], w, act))
+                z = x[:m].double() @ w.double().T
+                gate = torch.nn.functional.gelu(z[:, :16384], approximate="tanh") if act else torch.nn.functional.silu(z[:, :16384])
+                assert H.rel_rms(got, gate * z[:, 16384:]) < 3 * 2.0 ** -9
+
+
 def test_kernels_refuse_what_they_do_not_serve(hip):
     from holon_amd.kernels.hip import KernelError
     with pytest.raises(KernelError):

@@ -582,7 +582,7 @@ class HipKernels:
         x = torch.randn(rows, weight.shape[1], device=weight.device).to(torch.bfloat16)
         pairs = self._alike(weight, tiled)
         rival = self._MID_FORMS[self._time_mid_forms(x, weight)]      # the vendor library's best form (kept only if it wins)
-        vendor = (lambda w, _t: self.silu_mul(torch.matmul(x, w.t()))) if gated else (lambda w, _t: rival(x, w))
+        vendor = (lambda w, _t: self.silu_mul(rival(x, w))) if gated else (lambda w, _t: rival(x, w))
         took = {"rows": self._graph_time(self._in_turn(pairs, lambda w, t: self._rows_product(x, w, t, gated))),
                 "vendor": self._graph_time(self._in_turn(pairs, vendor))}
         return "rows" if took["rows"] < took["vendor"] else "vendor"
@@ -646,8 +646,9 @@ class HipKernels:
 
         def time():
             pairs, mul = self._alike(weight, None), self.gelu_mul if act else self.silu_mul
+            rival = self._MID_FORMS[self._time_mid_forms(x, weight) if k >= self.deep_k else "bf16"]     # what the library's side would run
             took = {"rows": self._graph_time(self._in_turn(pairs, lambda w, _t: block(w))),
-                    "vendor": self._graph_time(self._in_turn(pairs, lambda w, _t: mul(torch.matmul(x, w.t()))))}
+                    "vendor": self._graph_time(self._in_turn(pairs, lambda w, _t: mul(rival(x, w))))}
             return "rows" if took["rows"] < took["vendor"] else "vendor"
         # (steps beyond those that start-up times: by the rule above, unless a pin or the mode says otherwise)
         beyond = m > self.parts_rows

@@ -1075,7 +1075,8 @@ def test_products_on_tiles_of_256_rows(hip):
 @pytest.mark.parametrize("act", [0, 1])
 def test_gated_products_on_tiles_of_256_rows_are_a_product_choice(hip, act):
     """In either activation: the mode `vendor`, a pin of the kind, and a pinned form of the library's product keep that product, at any
-    number of rows; what was taken is recorded (beyond the rows that a start times: if it was pinned)."""
+    number of rows; what was taken is recorded; mode `timed` times it only where a start does (here against the library's best form,
+    K being long enough for one)."""
     x, w = _randn(2048, 256, dtype=torch.bfloat16), _randn(2 * 16384, 256, dtype=torch.bfloat16, scale=0.1)
     for m, bucket in ((520, 768), (2048, 2048)):
         for mode, pins, taken in (("own", {}, "rows"), ("vendor", {}, "vendor"), ("own", {f"glu:32768x256:{bucket}": "vendor"}, "vendor"),
@@ -1091,6 +1092,11 @@ def test_gated_products_on_tiles_of_256_rows_are_a_product_choice(hip, act):
                 z = x[:m].double() @ w.double().T
                 gate = torch.nn.functional.gelu(z[:, :16384], approximate="tanh") if act else torch.nn.functional.silu(z[:, :16384])
                 assert H.rel_rms(got, gate * z[:, 16384:]) < 3 * 2.0 ** -9
+    deep = torch.zeros(2 * 16384, 8192, dtype=torch.bfloat16, device="cuda")
+    timed = hip.configured("timed")
+    timed.plan.resolving = True
+    timed.linear_glu(_randn(520, 8192, dtype=torch.bfloat16), deep, act)
+    assert timed.plan.how == {"glu:32768x8192:768": "timed"}
 
 
 def test_kernels_refuse_what_they_do_not_serve(hip):

@@ -671,12 +671,23 @@ class MoE(Part):
                           shared_weight=self.shared_gated)
             if y is not None:
                 return y
-        if moe_rows_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top):
+        if moe_rows_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top) \
+                and self._own_rows(x.shape[0]):
             y = k.moe_rows(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",
                            shared_weight=self.shared_gated)
             if y is not None:
                 return y
         between = k.moe_relu2 if self.act == "relu2" else k.moe_gate
         return down(between(up(x), weights, self.inter, self.shared, shared_weight=self.shared_gated))
+
+    def _own_rows(self, rows: int) -> bool:
+        """Whether the engine's product choices leave a step of many rows to `moe_rows`: pins of either product over all experts keep
+        those, and so does mode `vendor`."""
+        choice = getattr(self.kernels, "product_choice", None)       # (a kernel set with one form a product has nothing to choose)
+        if choice is None:
+            return True
+        shapes = [tuple(w.weight.shape) for w in (self.gate_up, self.all_down)]
+        return choice("experts", self.gate_up.weight, rows, yields=[(kind, s) for kind in ("rows", "vendor") for s in shapes],
+                      by_rule=True) == "own"
 
     __call__ = forward

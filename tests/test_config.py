@@ -204,4 +204,6 @@ def test_a_choice_by_rule_reads_pins_and_mode_and_records_pins_alone():
     plan = ProductPlan("own", pins)
     assert plan.choose("glu", (8192, 256), 2048, by_rule=True) == "vendor" and plan.how == {"glu:8192x256:2048": "pinned"}
     over = [("rows", (512, 256)), ("vendor", (512, 256)), ("rows", (256, 512)), ("vendor", (256, 512))]
+    assert [ProductPlan("own", pins).choose("experts", (512, 256), bucket, yields=over, by_rule=True) for bucket in (64, 128, 512)] == \
+        ["vendor", "own", "vendor"]
     assert [plan.choose("glu", (512, 256), bucket, yields=over) for bucket in (64, 128, 512)] == ["vendor", "rows", "vendor"]

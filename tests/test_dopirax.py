@@ -741,6 +741,36 @@ def test_float32_experts_over_the_rows_that_chose_them_whatever_the_step():
 
 
 @pytest.mark.gpu
+def test_experts_of_many_row_steps_are_a_product_choice(monkeypatch):
+    """A mixture's step of many rows stays with the products over all experts in mode `vendor`, under a pin of its kind, and under a pin of
+    either of those products at its row bucket; elsewhere it takes every expert's own rows."""
+    from holon_amd.kernels import load_hip
+    from holon_amd.parts import ffn
+    from holon_amd.parts.base import Build
+    dev, bf, experts, inter, hidden = torch.device("cuda"), torch.bfloat16, 8, 1024, 2048
+    up, down = f"{2 * experts * inter}x{hidden}", f"{hidden}x{experts * inter}"
+    x = (0.1 * torch.randn(1024, hidden)).to(dev).to(bf)
+    for mode, pins, own in (("own", {}, True), ("timed", {}, True), ("vendor", {}, False), ("own", {f"experts:{up}:1024": "vendor"}, False),
+                            ("vendor", {f"experts:{up}:1024": "own"}, True), ("own", {f"vendor:{down}:1024": "f32"}, False),
+                            ("own", {f"rows:{up}:64": "rows"}, True)):
+        k = load_hip().configured(mode, pins)
+        part = ffn.MoE(Build(k, dev, bf), experts=experts, top=2, inter=inter, hidden=hidden, layer=0, bias=False)
+        g = torch.Generator(device="cuda").manual_seed(3)
+        for _, owner, name, decl in part.named_params():
+            draw = 0.05 * torch.randn(decl.shape, generator=g, device=dev)
+            setattr(owner, name, draw if decl.kind == "float32" else draw.to(bf))
+        part.finalize()
+        calls = []
+        for op in ("moe_rows", "moe_gate"):
+            inner = getattr(k, op)
+            monkeypatch.setattr(k, op, lambda *a, op=op, inner=inner, **kw: calls.append(op) or inner(*a, **kw), raising=False)
+        part(x)
+        assert calls == (["moe_rows"] if own else ["moe_gate"]), (mode, pins)
+        chosen = {key: form for key, form in k.plan.report().items() if key.startswith("experts:")}
+        assert chosen == ({f"experts:{up}:1024": "own" if own else "vendor"} if pins and (mode == "vendor" or not own) else {}), (mode, pins)
+
+
+@pytest.mark.gpu
 def test_chosen_experts_alone_or_all_of_them(tmp_path, monkeypatch):
     """Decoding a row over experts of a size that the few-row products serve, from graphs: bit for bit the same logits over the chosen
     experts' columns and over all of them."""

@@ -264,6 +264,7 @@ extern "C" int holon_gemm_rows_bf16(const void* x, const void* w_tiled, void* y,
   HOLON_CHECK(holon_gemm_rows_supported(M, N, K, 0), "gemm (17 to 64 rows): M=%d N=%d K=%d not served", M, N, K);
   hipStream_t s = (hipStream_t)stream;
   if (deep_serves(M, N, K)) {
+    HOLON_CHECK((((uintptr_t)x | (uintptr_t)w_tiled | (uintptr_t)y) & 15) == 0, "gemm (17 to 32 rows): operands off a border of 16 bytes");
     launch_deep(x, w_tiled, y, M, N, K, out_f32, s);
     HOLON_LAUNCH_OK();
     return 0;

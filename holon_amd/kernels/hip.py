@@ -511,6 +511,8 @@ class HipKernels:
         m, k = x.shape
         n = weight.shape[0] // 2 if gated else weight.shape[0]
         self._check_product("linear", x, weight, tiled)
+        if x.data_ptr() % 16:                     # (rows are read 16 bytes at a time; `tiled` may be of rows normed without a weight,
+            x = x.clone()                         # which no other product serves)
         y = torch.empty((m, n), dtype=torch.float32 if to_f32 else torch.bfloat16, device=x.device)
         if gated:
             self._call(self.lib.holon_gemm_rows_glu_bf16, x.data_ptr(), tiled.data_ptr(), y.data_ptr(), m, n, k, self._stream())

@@ -419,7 +419,8 @@ def moe_rows_pays(rows: int, hidden: int, experts: int, ff: int, shared: int, ga
     if rows <= 16:
         return False
     cols = experts * ff + shared
-    if 2 * (top * ff + shared) + 4 * (top + 1) * hidden > 6 * cols:
+    # (bytes a row: its act, parts and places in the lists, against its products over all and their activation)
+    if 2 * (top * ff + shared) + 4 * (top + 1) * hidden + 4 * (experts + top) > (6 if gated else 4) * cols:
         return False
     row_tiles, all_tiles = max(min(experts, rows * top), rows * top / 256 + experts / 2), -(-rows // 256)
     width = 128 if gated else 256

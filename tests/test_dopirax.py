@@ -721,6 +721,9 @@ def test_every_expert_over_its_own_rows_where_that_is_done_sooner():
     assert [moe_rows_pays(m, 2048, 8, 1024, 2048, True, 4) for m in (64, 400, 1024, 4096)] == [False, False, True, True]
     assert [moe_rows_pays(m, 2048, 8, 2048, 2048, False, 2) for m in (64, 512, 4096)] == [False, True, True]
     assert not moe_rows_pays(4096, 4096, 4, 128, 0, True, 2) and not moe_rows_pays(4096, 2048, 8, 1024, 0, True, 8)
+    # ungated: 2 (2 ff) + 12 hidden + 40 bytes a row against 4 (8 ff)
+    assert not moe_rows_pays(4096, 4096, 8, 1536, 0, False, 2) and not moe_rows_pays(4096, 2048, 16, 512, 0, False, 4)
+    assert [moe_rows_pays(4096, hidden, 8, 2048, 0, False, 2) for hidden in (4736, 4864)] == [True, False]
     assert moe_rows_serves(4096, 4096, 8, 2, 3072, 3072) and moe_rows_serves(1, 128, 1, 1, 128, 0)
     assert not any(moe_rows_serves(*a) for a in ((64, 192, 8, 2, 128, 0), (64, 256, 8, 2, 64, 0), (64, 256, 8, 2, 128, 64),
                                                  (64, 256, 2, 3, 128, 0), (0, 256, 8, 2, 128, 0), (1 << 22, 256, 8, 2, 128, 0)))

@@ -1141,9 +1141,12 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dma_kernel(AttnArgs a) {
     const int kb_first = (key_lo / 32) * 32, kb_last = (key_hi / 32) * 32;
     const int keep_first = MOD && a.window > 0 ? a.keep_first : 0, kept = min(keep_first, key_lo);
     const int kept_end = min((kept + 31) / 32 * 32, kb_first);
+    // of the stages that the block walks, a wave leaves out those before the window of all its rows: nothing in them, finite or not,
+    // reaches a row that sees none of it
+    const int tile_from = first_seen(tile_first, a.window);
     // `last`: values past `held` may be anything (std::true_type): the stage holds the row's last key, or the kept ones
     auto stage = [&](auto last, int kb, int buf, int held) {
-      if (kb <= tile_last) {
+      if (kb <= tile_last && (kb + 31 >= tile_from || (MOD && kb < kept_end))) {
         f32x16_t sc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) sc[i] = 0.f;

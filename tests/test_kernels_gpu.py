@@ -336,6 +336,49 @@ def test_prompt_portions_of_wide_heads(hip, geometry):
                 at += n
 
 
+@pytest.mark.parametrize("head_dim,changed", [(256, False), (128, True)])
+def test_prompt_portions_over_staged_keys_and_values_that_are_not_finite(hip, head_dim, changed):
+    """Stages copied into LDS: what lies past a row's end, and before the window of all of a portion's tokens, may be anything; a value
+    that is not finite among the keys that some tokens see stays out of every tile of 32 rows whose tokens see none of its stage of 32."""
+    bf, kv, window, page = torch.bfloat16, 36, 70, 16
+    rows = [(0, 401), (333, 300), (37, 201)]
+    q, pages, table, attn = _paged_case(rows, kv, kv, head_dim, page, bf, seed=head_dim)
+    bias = (torch.rand(kv, generator=torch.Generator().manual_seed(1)).cuda(), torch.rand(kv, generator=torch.Generator().manual_seed(2)).cuda())
+    how = dict(softcap=5.0, dist=bias) if changed else {}
+
+    def run(pages, direct):
+        was = hip.lib.holon_attention_prefill_copies(direct)
+        try:
+            return hip.paged_attention(q, pages, table, attn, page, head_dim ** -0.5, window, **how)
+        finally:
+            hip.lib.holon_attention_prefill_copies(was)
+    clean = run(pages, 1)
+    assert not torch.equal(clean, run(pages, 0))                      # (the staged form it is)
+    bad, slots = pages.clone(), attn.slots.tolist()
+    for slot, (start, n) in zip(slots, rows):
+        for key in list(range(max(0, start - window + 1) // 32 * 32)) + list(range(start + n, table.shape[1] * page)):
+            at = table[slot, key // page]
+            bad[at, 0].view(kv, page, head_dim)[:, key % page] = float("nan")
+            bad[at, 1].view(kv, head_dim, page)[:, :, key % page] = float("inf")
+    assert torch.equal(run(bad, 1), clean)
+    ends = np.cumsum([n for _, n in rows])
+    for (start, n), end, slot, key in zip(rows, ends, slots, (130, 400, 60)):
+        bad = pages.clone()
+        bad[table[slot, key // page], 1].view(kv, head_dim, page)[:, 3, key % page] = float("nan")
+        got = run(bad, 1)
+        first = key // 32 * 32                                         # of the key's stage
+        sees = torch.tensor([any(first <= p and p - window < first + 32 for p in range(start + t // 32 * 32, start + min(n, t // 32 * 32 + 32)))
+                             for t in range(n)])
+        mine = torch.arange(end - n, end)
+        assert sees.any() and not sees.all()
+        assert torch.equal(got[mine[~sees].cuda()], clean[mine[~sees].cuda()]), (start, key)
+        others = torch.ones(len(q), dtype=torch.bool)
+        others[mine] = False
+        assert torch.equal(got[others.cuda()], clean[others.cuda()])
+        seen = torch.tensor([start + t >= key > start + t - window for t in range(n)])
+        assert got[mine[seen].cuda()][..., 3].isnan().all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("window", [1, 7, 16, 100])
 def test_paged_attention_window(hip, dtype, window):

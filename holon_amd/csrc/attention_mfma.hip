@@ -1146,7 +1146,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dma_kernel(AttnArgs a) {
     const int tile_from = first_seen(tile_first, a.window);
     // `last`: values past `held` may be anything (std::true_type): the stage holds the row's last key, or the kept ones
     auto stage = [&](auto last, int kb, int buf, int held) {
-      if (kb <= tile_last && (kb + 31 >= tile_from || (MOD && kb < kept_end))) {
+      if (kb <= tile_last && (kb + 31 >= tile_from || (MOD && kb < keep_first))) {
         f32x16_t sc;
 #pragma unroll
         for (int i = 0; i < 16; ++i) sc[i] = 0.f;

@@ -536,7 +536,7 @@ class HipKernels:
         splits = (self.lib.holon_gemm_rows_splits if m <= self.parts_rows_short else self.lib.holon_gemm_tiles_splits)(m, n, k)
         if not splits:
             return None
-        whole = 0 if self.settled or (x.data_ptr() | weight.data_ptr()) % 16 else self.lib.holon_gemm_block_parts_splits(m, n, k)
+        whole = 0 if self.settled or weight.data_ptr() % 16 else self.lib.holon_gemm_block_parts_splits(m, n, k)
         how = (whole, True) if whole else (splits, False)
         use = self.product_choice("parts", weight, m, lambda: self._time_parts(x, weight, tiled, *how))
         return self._rows_parts(x, weight, tiled, *how) if use == "parts" else None
@@ -548,6 +548,8 @@ class HipKernels:
         if tiled is None or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.shape[1] != k:
             raise KernelError(f"linear in parts: bfloat16 rows {tuple(x.shape)} over a tiled bfloat16 weight "
                               f"{tuple(weight.shape)} expected")
+        if x.data_ptr() % 16:                     # (rows are copied into LDS 16 bytes at a time)
+            x = x.clone()
         parts = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
         entry = self.lib.holon_gemm_block_parts_bf16 if whole else \
             self.lib.holon_gemm_rows_parts_bf16 if m <= self.parts_rows_short else self.lib.holon_gemm_tiles_parts_bf16

@@ -1019,7 +1019,7 @@ def test_product_in_shares_of_k_for_prompt_portions(hip):
     from holon_amd.kernels.hip import KernelError
     bf = torch.bfloat16
     for m, k, n in ((129, 512, 256), (200, 1024, 512), (512, 12288, 4096), (1000, 2048, 512), (1024, 1536, 768),
-                    (300, 25600, 5120), (640, 9728, 2560)):
+                    (300, 25600, 5120), (640, 9728, 2560), (256, 9728, 2560), (400, 9728, 2560)):
         x, w = _randn(m, k, dtype=bf, seed=190), _randn(n, k, dtype=bf, seed=191, scale=0.05)
         tiled = hip.tile_weight(w)
         auto = hip.lib.holon_gemm_tiles_splits(m, n, k)
@@ -1041,6 +1041,8 @@ def test_product_in_shares_of_k_for_prompt_portions(hip):
                 assert H.op_budget_usage(total, hip.linear(x, w).double(), bf, k) <= 1       # the vendor library's product
                 some = hip._rows_parts(x[5:200].contiguous(), w, tiled, splits) if m >= 200 else None
                 assert some is None or torch.equal(some, parts[:, 5:200])
+                odd = torch.empty(x.numel() + 1, dtype=bf, device="cuda")[1:].view(x.shape).copy_(x)      # off a border of 16 bytes
+                assert torch.equal(hip._rows_parts(odd, w, tiled, splits), parts)
                 weight, eps = _randn(n, dtype=bf, seed=192) + 1, 1e-5
                 res_a, res_b = _randn(m, n, dtype=bf, seed=193), _randn(m, n, dtype=bf, seed=193)
                 normed_a = hip.add_rmsnorm(parts, res_a, weight, eps)
@@ -1050,6 +1052,12 @@ def test_product_in_shares_of_k_for_prompt_portions(hip):
     x, w = _randn(512, 12288, dtype=bf, seed=194), _randn(4096, 12288, dtype=bf, seed=195, scale=0.05)
     tiled = hip.tile_weight(w)
     assert hip.linear_parts(x, w, tiled).shape == (8, 512, 4096)                            # mode `own`
+    # which of the two kernels of such parts a call takes: 256 x 256 tiles where they serve, these blocks elsewhere
+    for m, k, n, whole in ((512, 12288, 4096, True), (256, 9728, 2560, False), (400, 9728, 2560, False), (640, 9728, 2560, True)):
+        a, b = _randn(m, k, dtype=bf, seed=199), _randn(n, k, dtype=bf, seed=200, scale=0.05)
+        t, splits = hip.tile_weight(b), (hip.lib.holon_gemm_block_parts_splits if whole else hip.lib.holon_gemm_tiles_splits)(m, n, k)
+        assert bool(hip.lib.holon_gemm_block_parts_splits(m, n, k)) == whole and splits
+        assert torch.equal(hip.linear_parts(a, b, t), hip._rows_parts(a, b, t, splits, whole)), (m, k, n)
     assert hip.configured("vendor").linear_parts(x, w, tiled) is None
     assert hip.configured("vendor", {"parts:4096x12288:512": "parts"}).linear_parts(x, w, tiled).shape == (8, 512, 4096)
     assert hip.linear_parts(_randn(1025, 12288, dtype=bf, seed=196), w, tiled) is None     # beyond 1,024 rows
@@ -1276,6 +1284,32 @@ def test_every_expert_over_its_own_rows(hip, hidden, experts, ff, shared, top, g
                                  shared, gated, shared_weight=own_gate)
             assert torch.equal(alone[0], got[row]), (m, row)
     assert hip.moe_rows(_randn(4, hidden, dtype=torch.float32), weights[:4], up_w, down_w, experts, top, ff, shared, gated) is None
+
+
+@pytest.mark.parametrize("op,dtype", [("moe_rows", torch.bfloat16), ("moe_f32", torch.float32)])
+def test_rows_that_are_not_finite_among_the_rows_of_an_expert(hip, op, dtype):
+    """A row with a NaN or an infinity changes no other row's result, whichever experts they share, and is not finite itself; weights that
+    are not finite, or more of them than a row may choose, write nothing out of place."""
+    hidden, experts, ff, shared, top = 256, 6, 128, 128, 2
+    cols, g = experts * ff + shared, torch.Generator().manual_seed(69)
+    up, down = _randn(2 * cols, hidden, dtype=dtype, seed=70, scale=hidden ** -0.5), _randn(hidden, cols, dtype=dtype, seed=71, scale=ff ** -0.5)
+    for m in (5, 70, 600):
+        x = _randn(m, hidden, dtype=dtype, seed=72 + m)
+        weights = torch.zeros(m, experts)
+        for row in range(m):
+            weights[row, torch.randperm(experts, generator=g)[:top]] = torch.rand(top, generator=g) + 0.2
+        weights = weights.cuda()
+        run = lambda x, w: getattr(hip, op)(x, w, up, down, experts, top, ff, shared, True)      # noqa: E731
+        clean, spoilt, wrong = run(x, weights), x.clone(), weights.clone()
+        rows = [1, m // 2, m - 1]
+        for row, value in zip(rows, (float("nan"), float("inf"), -float("inf"))):
+            spoilt[row, 7] = value
+        wrong[rows[0]], wrong[rows[1]] = float("nan"), 0.3
+        others = torch.tensor([r for r in range(m) if r not in rows], device="cuda")
+        assert torch.isfinite(clean).all()
+        got = run(spoilt, weights)
+        assert torch.equal(got[others], clean[others]) and not torch.isfinite(got[rows]).all(1).any(), m
+        assert torch.equal(run(spoilt, wrong)[others], clean[others]), m
 
 
 def test_experts_whose_operands_start_on_no_border_of_16_bytes_stay_with_the_products_over_all(hip):

@@ -249,6 +249,55 @@ def test_changed_scores_over_staged_keys(heads, groups):
             assert per < 4e-2, (window, keep, cap, per)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,groups", [(32, 32), (48, 16)])
+def test_changed_scores_over_staged_keys_with_gates_shared_values_and_chunks(heads, groups):
+    """The same kernel (heads of 128, enough ranges) with a gate a head, key heads that share value heads, and chunks of positions, against
+    the plain form in float64; the form that reads its operands from the cache beside it."""
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.api import AttnRows
+    k, dev, page, dim = load_hip(), "cuda", 16, 128
+    g = torch.Generator().manual_seed(heads + 1)
+    lens, counts = [330, 75, 300, 577], [330, 75, 33, 260]
+    n_pages = sum(-(-n // page) for n in lens)
+    table, order, at = torch.zeros(4, 40, dtype=torch.int32), torch.randperm(n_pages, generator=g).tolist(), 0
+    for b, n in enumerate(lens):
+        for i in range(-(-n // page)):
+            table[b, i] = order[at]
+            at += 1
+    qstart = [0]
+    for c in counts:
+        qstart.append(qstart[-1] + c)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)          # noqa: E731
+    rows = AttnRows(slots=i32([0, 1, 2, 3]), lens=i32(lens), query_start=i32(qstart), decode_rows=i32([]), chunk_rows=i32([0, 1, 2, 3]),
+                    n_decode=0, n_chunk=4, max_decode_len=0, max_chunk_query=max(counts), max_chunk_len=max(lens))
+    q, table, twin = torch.randn(qstart[-1], heads, dim, generator=g).to(dev).bfloat16(), table.to(dev), TorchKernels()
+    r1, r2 = torch.rand(heads, generator=g).to(dev), (2 * torch.rand(heads, generator=g)).to(dev)
+    gates = (2.0 * torch.randn(qstart[-1], heads + 5, generator=g)).to(dev).bfloat16()[:, 2: 2 + heads]
+    sink, scale = torch.randn(heads, generator=g).to(dev), 2.0 * dim ** -0.5
+    for share in (1, 2, 4):
+        pages = (0.5 * torch.randn(n_pages, groups + groups // share, page * dim, generator=g)).to(dev).bfloat16()
+        if share == 1:
+            pages = pages.view(n_pages, 2, groups, page * dim)
+        for window, keep, cap, far, gated in ((0, 0, 3.0, True, True), (-150, 0, 3.0, False, True), (40, 5, 0.0, True, False),
+                                              (-64, 0, 0.0, True, True), (100, 0, 2.0, False, True)):
+            more = dict(softcap=cap, keep_first=keep, value_share=share)
+            want = twin.paged_attention(q.double(), pages.double(), table, rows, page, scale, window, sink=sink.double(),
+                                        dist=(r1.double(), r2.double()) if far else None, head_gate=gates.double() if gated else None, **more)
+            both = []
+            for direct in (1, 0):
+                was = k.lib.holon_attention_prefill_copies(direct)
+                try:
+                    both.append(k.paged_attention(q, pages, table, rows, page, scale, window, sink=sink, dist=(r1, r2) if far else None,
+                                                  head_gate=gates if gated else None, **more))
+                finally:
+                    k.lib.holon_attention_prefill_copies(was)
+                assert H.rel_rms(both[-1], want) < 8e-3, (share, window, cap, direct)
+                per = ((both[-1].double() - want).square().mean((1, 2)).sqrt() / want.square().mean().sqrt()).max().item()
+                assert per < 4e-2, (share, window, cap, direct, per)
+            assert not torch.equal(*both)                       # (two forms: the staged one did run)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 def test_the_stream_after_every_layer_run(folders, device):
     """The residual stream after each run of a layer (a repeated layer counts each time), float32, against the plain

@@ -6,7 +6,8 @@
 // bytes with their 16-byte pieces swizzled, so that no read of LDS meets a bank conflict). A wave's part of the tile is
 // 128 x 64 in four quarters of 64 x 32, and its loop four steps, one a quarter: read what the quarter needs that is not in
 // registers yet (rows for one step in two, columns the other two), ask for a quarter of the chunk after next, then 16
-// matrix instructions. The two waves of a SIMD run half a step apart, held there by a barrier before and after the
+// matrix instructions. The two waves of a SIMD run half a step apart (the eight-wave "ping-pong" schedule that is published
+// for products on CDNA, in the HipKittens paper of 2025 among others), held there by a barrier before and after the
 // instructions: while one reads, the other multiplies. A quarter of a chunk is asked for as soon as both waves have read the
 // one it overwrites, so about 6 steps (3,000 cycles) before it is read, and every wait leaves what came after it under way.
 // Measured on MI355X, us (the vendor library's product): 4096 x 4096 x 4096 101 (112), 4096 rows by 55296 x 4096 1,337 (1,387),

@@ -185,7 +185,8 @@ extern "C" int holon_moe_rows_supported(int rows, int hidden, int experts, int t
 extern "C" int holon_moe_rows_bf16(const void* x, const void* up, const void* down, void* y, int* lists, void* act, float* parts,
                                    int rows, int hidden, int experts, int top, int ff, int shared, int gated,
                                    const float* weights, int wstride, int shared_col, void* stream) {
-  HOLON_CHECK(holon_moe_rows_supported(rows, hidden, experts, top, ff, shared) && wstride >= experts && shared_col < wstride,
+  HOLON_CHECK(holon_moe_rows_supported(rows, hidden, experts, top, ff, shared) && wstride >= experts && shared_col < wstride &&
+                  (((uintptr_t)x | (uintptr_t)up | (uintptr_t)down | (uintptr_t)y | (uintptr_t)act | (uintptr_t)parts) & 15) == 0,
               "moe (many rows): %d rows of %d, %d experts of %d (%d a row), %d shared columns not served", rows, hidden, experts,
               ff, top, shared);
   hipStream_t s = (hipStream_t)stream;

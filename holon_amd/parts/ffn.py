@@ -414,8 +414,10 @@ def moe_rows_pays(rows: int, hidden: int, experts: int, ff: int, shared: int, ga
     where there is one) and the parts' traffic against the products over all (their operations at 1.2 PFLOP/s and their weights at 4
     TB/s). Measured on MI355X, own rows / all (us): 8 experts of 3,072 x 4,096 beside a shared one, 2 a row, at 64 / 512 / 4,096 rows
     181 / 218 / 830 and 226 / 472 / 2,035; of 2,048 x 2,048 at 64 / 512 / 4,096 86 / 93 / 345 and 89 / 211 / 853; 8 of 1,024 beside a
-    shared one of 2,048, 4 a row, at 64 / 512 / 1,024 / 4,096 82 / 97 / 113 / 405 and 50 / 85 / 149 / 438; 64 of 512, 6 a row, at 64 /
-    1,024 128 / 168 and 131 / 496. A step whose parts would take more memory than the products over all stays with those."""
+    shared one of 2,048, 4 a row, at 64 / 512 / 1,024 / 4,096 82 / 97 / 113 / 405 and 50 / 85 / 149 / 438; 64 of 512, 6 a row, at 17 /
+    32 / 64 / 1,024 89 / 115 / 128 / 168 and 124 / 125 / 131 / 496; the others at 17 / 32 / 63: of 3,072 x 4,096 167 / 178 / 181 and 224 / 215 /
+    209, of 2,048 x 2,048 87 / 87 / 86 and 85 / 89 / 90, 8 of 1,024 81 / 82 / 83 and 47 / 45 / 45. A step whose parts would take more memory
+    than the products over all stays with those."""
     if rows <= 16:
         return False
     cols = experts * ff + shared

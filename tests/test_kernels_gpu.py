@@ -1314,6 +1314,7 @@ def test_rows_that_are_not_finite_among_the_rows_of_an_expert(hip, op, dtype):
 
 def test_experts_whose_operands_start_on_no_border_of_16_bytes_stay_with_the_products_over_all(hip):
     """The kernels over an expert's own rows read 16 bytes at a time: elsewhere they serve nothing, whichever operand it is."""
+    from holon_amd.kernels.hip import KernelError
     for op, dtype in ((hip.moe_rows, torch.bfloat16), (hip.moe_f32, torch.float32)):
         rows, hidden, experts, ff = 64, 128, 4, 128
         weights = torch.zeros(rows, experts, device="cuda")
@@ -1323,6 +1324,13 @@ def test_experts_whose_operands_start_on_no_border_of_16_bytes_stay_with_the_pro
             x, up, down = (torch.empty(v.numel() + 1, dtype=dtype, device="cuda")[1:].view(v.shape).copy_(v) if i == at else v
                            for i, v in enumerate(operands))
             assert (op(x, weights, up, down, experts, 1, ff, 0, False) is None) == (at is not None), (dtype, at)
+            if at is not None:                     # (the entry points refuse them)
+                scratch = [torch.empty(rows * (experts + 2) * (hidden + ff), dtype=dt, device="cuda")
+                           for dt in (torch.int32, dtype, torch.float32, dtype)]
+                with pytest.raises(KernelError, match="not served"):
+                    hip._call(hip.lib.holon_moe_f32 if dtype == torch.float32 else hip.lib.holon_moe_rows_bf16, x.data_ptr(), up.data_ptr(),
+                              down.data_ptr(), scratch[3].data_ptr(), scratch[0].data_ptr(), scratch[1].data_ptr(), scratch[2].data_ptr(),
+                              rows, hidden, experts, 1, ff, 0, 0, weights.data_ptr(), experts, -1, hip._stream())
 
 
 @pytest.mark.parametrize("hidden,experts,ff,shared,top,gated,own_gate", [

@@ -23,7 +23,7 @@ MODES = ("own", "vendor", "timed")
 
 # kind -> (this package's form or the plain default, every form)
 KINDS: dict[str, tuple[str, tuple[str, ...]]] = {
-    "rows": ("rows", ("rows", "vendor")),         # 17 to 64 rows over many tiles, rows shared through LDS
+    "rows": ("rows", ("rows", "vendor")),         # 17 to 64 rows over many tiles, rows shared through LDS; 17 to 47 over narrow weights
     "glu": ("rows", ("rows", "vendor")),          # the same with SiLU-mul inside, and above 128 rows 256 x 256 tiles (GELU too;
                                                   # above 1,024 rows never timed)
     "parts": ("parts", ("parts", "vendor")),      # a narrow weight, K in shares: 17 to 128 rows; to 1,024 where K is well above N

@@ -175,7 +175,7 @@ void launch_rows_tall(const void* x, const void* w, void* y, int M, int N, int K
 }
 }  // namespace
 
-// 17 to 32 rows over weights too narrow for the form above: a block one tile of 16 columns, K split over its waves in order, every wave
+// 17 to 47 rows over weights too narrow for the form above: a block one tile of 16 columns, K split over its waves in order, every wave
 // reading its share of the rows from L2 (the few-row kernel's shape with MT tiles of tokens). One launch where a product in shares takes
 // two; bound by what the blocks read of the rows, N / 16 times all of them.
 namespace {
@@ -229,22 +229,30 @@ __global__ void __launch_bounds__(1024) gemm_deep_kernel(const bf16_t* __restric
   }
 }
 
-// Where that is no slower on the GPU than the vendor library's product (and one launch of 7 us of the host's where that one takes 19): us
-// at 17 / 32 / 37 / 48 rows against the library, 2048 x 2048 6.8 / 8.3 / 9.2 / 10.2 and 8.9 / 8.9 / 8.9 / 8.9, 4096 x 2048 7.8 / 9.0 / 9.6 /
-// 10.6 and 9.1 / 9.2 / 9.2 / 9.2, 1024 x 2048 6.6 / 8.1 / 9.0 / 9.9 and 8.5 / 8.8 / 8.6 / 8.7: two tiles of rows, not three. Beyond 256
-// tiles of columns, or over longer sums (2048 x 8192 at 17 / 37 rows 18 / 27 and 14 / 14), the reads of the rows cost too much, under
-// 64 tiles the compute units stand idle (512 x 2048 at 37 rows 8.9 and 5.8), and short sums are done in 5 us (2048 x 768).
+// What a step pays for either form is its whole time. Up to 32 rows it is the GPU's: such steps are replayed from graphs (of 24 and 32 rows)
+// that read their weights from memory, us at 17 / 32 rows against the vendor library's product 2048 x 2048 6.8 / 8.3 and 8.9 / 8.9, 4096 x 2048
+// 7.8 / 9.0 and 9.1 / 9.2, 1024 x 2048 6.6 / 8.1 and 8.5 / 8.8; decode steps of 24 / 32 rows of models of that width 541 / 561 and 549 / 563 us,
+// 1,062 / 1,101 and 1,133 / 1,155. From 33 to 47 rows a step runs eagerly (the next graph has 48) and waits for the host, 7 us for this launch
+// and 19 for the library's: prompts of 33 / 40 / 47 tokens 904 / 897 / 905 and 1,054 / 1,043 / 1,062 us, 1,669 / 1,654 / 1,655 and 1,874 / 1,865 /
+// 1,865, though the GPU alone would take 9.2 / 9.6 / 9.0 us for 8.9 / 9.2 / 8.6 at 37 rows. At 48, a graph's size, it takes 10.2 / 10.6 / 9.9 us for
+// 8.9 / 9.2 / 8.7. Beyond 256 tiles of columns, or over longer sums (2048 x 8192 at 17 / 37 rows 18 / 27 and 14 / 14), the reads of the rows cost
+// too much, under 64 tiles the compute units stand idle (512 x 2048 at 37 rows 8.9 and 5.8), and short sums are done in 5 us (2048 x 768).
 bool deep_serves(int M, int N, int K) {
-  return M > 16 && M <= 32 && N % 16 == 0 && N >= 1024 && N <= 4096 && K % 256 == 0 && K >= 1280 && K <= 2048;
+  return M > 16 && M < 48 && N % 16 == 0 && N >= 1024 && N <= 4096 && K % 256 == 0 && K >= 1280 && K <= 2048;
 }
 
 void launch_deep(const void* x, const void* w, void* y, int M, int N, int K, int out_f32, hipStream_t s) {
   int waves = 16;
   while (K % (32 * waves) != 0) waves /= 2;                 // (K is a multiple of 256: at least 8)
-  constexpr int MT = 2;
-  const size_t lds = (size_t)waves * MT * WAVE * sizeof(f32x4_t);
-  if (out_f32) gemm_deep_kernel<MT, true><<<N / 16, waves * WAVE, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, y, M, N, K);
-  else gemm_deep_kernel<MT, false><<<N / 16, waves * WAVE, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, y, M, N, K);
+  const int mt = (M + 15) / 16;
+  const size_t lds = (size_t)waves * mt * WAVE * sizeof(f32x4_t);
+#define DEEP(MT)                                                                                                              \
+  case MT:                                                                                                                    \
+    if (out_f32) gemm_deep_kernel<MT, true><<<N / 16, waves * WAVE, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, y, M, N, K); \
+    else gemm_deep_kernel<MT, false><<<N / 16, waves * WAVE, lds, s>>>((const bf16_t*)x, (const bf16_t*)w, y, M, N, K);        \
+    break
+  switch (mt) { DEEP(2); DEEP(3); }
+#undef DEEP
 }
 }  // namespace
 
@@ -264,7 +272,7 @@ extern "C" int holon_gemm_rows_bf16(const void* x, const void* w_tiled, void* y,
   HOLON_CHECK(holon_gemm_rows_supported(M, N, K, 0), "gemm (17 to 64 rows): M=%d N=%d K=%d not served", M, N, K);
   hipStream_t s = (hipStream_t)stream;
   if (deep_serves(M, N, K)) {
-    HOLON_CHECK((((uintptr_t)x | (uintptr_t)w_tiled | (uintptr_t)y) & 15) == 0, "gemm (17 to 32 rows): operands off a border of 16 bytes");
+    HOLON_CHECK((((uintptr_t)x | (uintptr_t)w_tiled | (uintptr_t)y) & 15) == 0, "gemm (17 to 47 rows): operands off a border of 16 bytes");
     launch_deep(x, w_tiled, y, M, N, K, out_f32, s);
     HOLON_LAUNCH_OK();
     return 0;

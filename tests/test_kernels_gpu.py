@@ -1069,27 +1069,27 @@ def test_product_in_shares_of_k_for_prompt_portions(hip):
         hip._rows_parts(x, w[:4000].contiguous(), hip.tile_weight(w[:4000].contiguous()), 4)   # 4,000 columns: no whole blocks
 
 
-def test_products_of_17_to_32_rows_over_narrow_weights(hip):
+def test_products_of_17_to_47_rows_over_narrow_weights(hip):
     """A block a tile of 16 columns, K over its waves: against float64, results in either type, rows whatever lies beside them, at the
     edges of what the kernel takes; rows that start on no border of 16 bytes."""
     from holon_amd.kernels.hip import KernelError
     bf, served = torch.bfloat16, lambda m, n, k: bool(hip.lib.holon_gemm_rows_supported(m, n, k, 0))     # noqa: E731
-    assert [served(m, 2048, 2048) for m in (16, 17, 32, 33, 64)] == [False, True, True, False, False]
+    assert [served(m, 2048, 2048) for m in (16, 17, 47, 48, 64)] == [False, True, True, False, False]
     assert [served(32, n, k) for n, k in ((1008, 2048), (1024, 768), (1024, 1280), (4112, 2048), (4096, 2304), (1032, 1280))] == \
         [False, False, True, False, False, False]
     for n, k in ((1024, 1536), (1040, 1280), (4096, 2048), (2064, 1792)):
         w = _randn(n, k, dtype=bf, seed=185, scale=0.05)
-        tiled, x = hip.tile_weight(w), _randn(32, k, dtype=bf, seed=186)
+        tiled, x = hip.tile_weight(w), _randn(47, k, dtype=bf, seed=186)
         want, whole = x.double() @ w.double().T, hip.linear(x, w, tiled=tiled)
         assert H.op_budget_usage(whole, want, bf, k) <= 1, (n, k)
-        for m in (17, 25, 31):
+        for m in (17, 32, 33, 40):
             assert torch.equal(hip.linear(x[:m].contiguous(), w, tiled=tiled), whole[:m]), (m, n, k)
         assert torch.equal(hip.linear(x, w, torch.float32, tiled), whole.float()), (n, k)
         odd = torch.empty(x.numel() + 1, dtype=bf, device="cuda")[1:].view(x.shape).copy_(x)
         assert torch.equal(hip.linear(odd, w, tiled=tiled), whole), (n, k)
         y = torch.empty_like(whole)
         with pytest.raises(KernelError):                                              # (the entry point itself takes no such rows)
-            hip._call(hip.lib.holon_gemm_rows_bf16, odd.data_ptr(), tiled.data_ptr(), y.data_ptr(), 32, n, k, 0, hip._stream())
+            hip._call(hip.lib.holon_gemm_rows_bf16, odd.data_ptr(), tiled.data_ptr(), y.data_ptr(), 47, n, k, 0, hip._stream())
 
 
 def test_products_on_tiles_of_256_rows(hip):

@@ -36,7 +36,7 @@ class EngineConfig:
     graphs: bool = _setting(True, "replay decode steps from HIP graphs, per batch-size bucket")
     decode_weight_copy: bool = _setting(True, "keep a second copy of every projection in the tile layout that steps of "
                                               "few rows stream fastest (doubles the weights' memory)")
-    products: str = _setting("own", "which kernel a matrix product of 17 to 1,024 rows takes where several serve it: "
+    products: str = _setting("own", "which kernel a matrix product of 17 rows and more takes where several serve it: "
                                     "own (this package's wherever one serves), vendor (the vendor library's plain "
                                     "product), timed (candidates are timed once while the engine starts)")
     product_pins: dict | None = _setting(None, "single products pinned whatever the mode, as kind:NxK:rows=form,... "

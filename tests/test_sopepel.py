@@ -555,7 +555,7 @@ def test_graph_replays_equal_eager_steps(folders, name, dtype):
 @pytest.mark.gpu
 def test_float32_decode_rows_have_the_same_bits_in_every_step():
     """A request's logits, float32, at sizes where few rows and many take kernels of their own (attention heads of 128, 8 experts of 2,048
-    beside a shared one): decoded alone, six at a time, from a graph whose rows are padded to eight, 20 at a time, and beside a prompt. (The
+    beside a shared one): decoded alone, six and 20 at a time, from graphs whose rows are padded to 8 and 24, and beside a prompt. (The
     linear attention, whose steps of decode rows alone have a kernel of their own, is left out.)"""
     from holon_amd import benchmark
     from holon_amd.engine.loading import load_model
@@ -566,12 +566,12 @@ def test_float32_decode_rows_have_the_same_bits_in_every_step():
     prompts = [H.random_ids(n, 4096, 40 + n) for n in (70, 5, 33, 1, 17, 64, *range(2, 16))]
     more = [H.random_ids(3, 4096, 90 + i) for i in range(len(prompts))]
     got = {}
-    for how in ("alone", "six", "graph", "twenty", "beside"):
+    for how in ("alone", "six", "graph", "twenty", "graph of twenty", "beside"):
         rep = Replayer(load_model("random", device="cuda", dtype="float32", page_size=16, max_seqs=24, max_model_len=160, max_step_tokens=256,
-                                  cache_tokens=4096, graphs=how == "graph", random_config=cfg, seed=2))
+                                  cache_tokens=4096, graphs="graph" in how, random_config=cfg, seed=2))
         for r, p in enumerate(prompts):
             rep.step([{"id": r, "tokens": p, "want": []}], ())
-        sets = [[r] for r in range(6)] if how == "alone" else [list(range(20 if how == "twenty" else 6))]
+        sets = [[r] for r in range(6)] if how == "alone" else [list(range(20 if "twenty" in how else 6))]
         out = {}
         for ids in sets:
             for i in range(3):

@@ -20,6 +20,10 @@ from .linear import Linear
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
 MAX_KEY_DIM = 256             # the scans keep a column of D values in registers
+# The delta rule's rows in blocks of 16 tokens, from a longest row of this many (16 heads of 128 by 128, us, against token by token:
+# 32 tokens 22 / 24, 64 28 / 41, 300 70 / 170). The 32-bit path keeps the token's own order of sums in shorter steps, so that its logits do
+# not depend on how a prompt of up to that many tokens is cut.
+DELTA_FROM = {torch.bfloat16: 32, torch.float32: 512}
 
 
 def _ptr(t):
@@ -97,12 +101,16 @@ def _delta_scan_hip(launch, qn, kn, qkv, beta, g, state, slots, starts, query_st
     _need(dim <= MAX_KEY_DIM and vdim <= 1024, f"delta_scan: key size {dim} (at most {MAX_KEY_DIM}), value size {vdim} "
           "(at most 1024)")
     out = torch.empty((t, heads, vdim), dtype=torch.float32, device=qn.device)
-    extra = (0, 0, None, None, None)
+    extra = (0, 0, None, None, None, None)
     if pieces is not None:
         tokens, most, base, total = pieces
-        ab = torch.empty((total, heads, dim, vdim + dim), dtype=torch.float32, device=qn.device)
-        sin = torch.empty((total, heads, dim, vdim), dtype=torch.float32, device=qn.device)
-        extra = (tokens, most, base.data_ptr(), ab.data_ptr(), sin.data_ptr())
+        f32 = dict(dtype=torch.float32, device=qn.device)
+        blocks, a, sin = torch.empty((t // 16 + n_rows, heads, 576), **f32), None, None
+        if most > 1:
+            kd = next(size for size in (32, 64, 128, 256) if dim <= size)
+            a = torch.empty((total, heads, kd, kd), **f32)
+            sin = torch.empty((total, heads, dim, vdim), **f32)
+        extra = (tokens, most, base.data_ptr(), blocks.data_ptr(), _ptr(a), _ptr(sin))
     launch(qn.data_ptr(), kn.data_ptr(), qkv.data_ptr(), qkv.shape[1], qkv.shape[1] - heads * vdim, beta.data_ptr(),
            g.data_ptr(), state.data_ptr(), out.data_ptr(), slots.data_ptr(), starts.data_ptr(), query_start.data_ptr(),
            n_rows, heads, kv_heads, dim, vdim, state.shape[0], _DT[qkv.dtype], *extra)
@@ -206,9 +214,7 @@ def memory_scan_plain(r, k, v, w, u, state, slots, starts, query_start, n_rows, 
 def scan_pieces(step, tokens: int = 128, least: int = 256):
     """For a step with a row of `least` tokens or more (never a step replayed from a graph: those rows have one token):
     (tokens a piece, the most pieces a row has, the number of each row's first piece among all [rows] int32 on the
-    device, pieces in all), made once a step and piece length from the host's row lengths; else None. (The delta
-    rule takes pieces of 256 tokens: the ordered walk between its two passes multiplies matrices, and is the shorter
-    the fewer pieces there are.)"""
+    device, pieces in all), made once a step and piece length from the host's row lengths; else None."""
     if step.rows.max_chunk_query < least:
         return None
     cache = step.__dict__.setdefault("_scan_pieces", {})
@@ -241,10 +247,19 @@ def _memory_scan_hip(launch, r, k, v, w, u, state, slots, starts, query_start, n
     return out
 
 
+def delta_pieces(step, columns: int, dtype: torch.dtype):
+    """`scan_pieces` for the delta rule over `columns` value columns of all heads: pieces of 256 tokens, or of 512 where no row is
+    longer or the step's columns fill the GPU by themselves (the pass that makes pieces independent runs on D + V columns:
+    16 heads of 128 by 128, us in pieces of 256 / 512: one row of 300 tokens 104 / 70, of 1,024 120 / 177, of 2,048 159 / 188,
+    of 4,000 261 / 238, eight of 500 173 / 117, four of 700 to 1,400 299 / 259)."""
+    full = step.rows.max_chunk_query <= 512 or step.n_tokens * columns > 2560 * 2048
+    return scan_pieces(step, 512 if full else 256, DELTA_FROM[dtype])
+
+
 register_kernel(KernelOp("delta_prepare", delta_prepare_plain, "holon_delta_prepare",
                          [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I], _delta_prepare_hip))
 register_kernel(KernelOp("delta_scan", delta_scan_plain, "holon_delta_scan",
-                         [_P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P],
+                         [_P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
                          _delta_scan_hip))
 register_kernel(KernelOp("gated_out", gated_out_plain, "holon_gated_out",
                          [_P, _P, _P, _P, _I, _I, _I, _I, _F, _I, ctypes.c_int64, _I, _P], _gated_out_hip))
@@ -311,7 +326,7 @@ class GatedDelta(Part):
         qn, kn, beta, g = k.delta_prepare(qkv, self.ab(x), self.A_log, self.dt_bias, self.heads, self.kv_heads,
                                           self.dim, self.vdim)
         o = k.delta_scan(qn, kn, qkv, beta, g, site.slot_state[self.prefix + "S"], step.slots, step.starts,
-                         step.query_start, step.n_rows, self.heads, self.vdim, scan_pieces(step, 256, 512))
+                         step.query_start, step.n_rows, self.heads, self.vdim, delta_pieces(step, self.heads * self.vdim, self.build.dtype))
         return self.o(k.gated_out(o, self.g(x), self.norm, False, self.eps, self.build.dtype))
 
     __call__ = forward

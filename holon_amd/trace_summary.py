@@ -61,7 +61,7 @@ def dispatches(path: str) -> list[tuple]:
 CLASSES = (("attention", ("attn_", "sigmoid_attention", "softmax_attention", "latent_attention", "latent_prefill", "latent_decode",
                           "latent_merge")),
            ("matrix products", ("gemm_", "Cijk_", "Custom_Cijk_", "hipBLASLt", "head_linear", "moe_up_few", "moe_down_few")),
-           ("recurrent scans", ("memory_scan", "delta_scan", "delta_pieces", "mlstm_scan", "mlstm_chunk", "mlstm_pieces", "mlstm_gates", "ssd_", "gla_")),
+           ("recurrent scans", ("memory_scan", "delta_scan", "delta_blocks", "delta_chain", "delta_walk", "mlstm_scan", "mlstm_chunk", "mlstm_pieces", "mlstm_gates", "ssd_", "gla_")),
            ("elementwise", ("rmsnorm", "gated_mul", "qk_norm_rope", "v_write", "kv_write", "embedding", "sum_parts",
                             "row_sumsq", "scatter_rows", "stream_norm", "dyt_stream", "widen_", "narrow_", "pair_rows", "softcap", "causal_conv",
                             "head_prepare", "delta_prepare", "gated_out", "shift_mix", "shift_keep", "decay_lora", "stream_rms", "latent_rope_prepare", "gated_parts_norm",

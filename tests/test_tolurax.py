@@ -452,3 +452,47 @@ def test_the_delta_rule_in_pieces_starts_from_a_copy(heads, kv, dim, vdim, monke
     for b in (0, 3):
         assert torch.equal(starts_of[base[b] + npc[b] - 1], state[slots[b]]), b
     assert not starts_of[base[4] + npc[4] - 1].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(2, 1, 32, 64), (4, 2, 22, 40), (1, 1, 6, 5), (2, 2, 128, 130), (1, 1, 256, 16)])
+def test_the_delta_rule_in_blocks_of_tokens(heads, kv, dim, vdim, dtype):
+    """`delta_scan` over rows of one token, of a block of 16, of one more and less, whole and in pieces of two blocks, against its plain
+    form (the same formulas in float32: sums of up to 256 terms, so 1e-5 leaves a factor of ten). A key or value of NaN or infinity:
+    the tokens before it bit for bit as without it, those from it on finite where the token-by-token scan's are."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    from holon_amd.kernels.registry import kernel_op
+    k, dev = load_hip(), torch.device("cuda")
+    gen = torch.Generator().manual_seed(dim)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
+    counts = [1, 15, 16, 17, 33, 47]
+    t, n = sum(counts), len(counts)
+    norm = lambda x: x / x.norm(dim=-1, keepdim=True)                          # noqa: E731
+    qn, kn = norm(rn(t, kv, dim)), norm(rn(t, kv, dim))
+    qkv = rn(t, 2 * kv * dim + heads * vdim).to(dtype)
+    beta, g = torch.rand(t, heads, generator=gen).to(dev), torch.exp(-rn(t, heads).abs())
+    g[5], beta[7] = 0.0, 0.0
+    state = rn(n + 1, heads, dim, vdim)
+    rows = (i32([6, 1, 2, 0, 4, 5]), i32([5, 0, 9, 3, 0, 1]), i32([sum(counts[:b]) for b in range(n + 1)]), n, heads, vdim)
+
+    def run(piece, key=kn, val=qkv, scan=k.delta_scan):
+        npc = [-(-c // piece) for c in counts] if piece else []
+        pieces = (piece, max(npc), i32([sum(npc[:b]) for b in range(n)]), sum(npc)) if piece else None
+        held = state.clone()
+        return scan(qn, key, val, beta, g, held, *rows, pieces), held
+    want, after = run(0, scan=kernel_op("delta_scan").plain)
+    for piece in (32, 48):
+        got, held = run(piece)
+        assert H.rel_rms(got, want) < 1e-5 and H.rel_rms(held, after) < 1e-5, piece
+    ref, last = run(48)[0], sum(counts[:5])
+    for at, value in ((last, "nan"), (last + 5, "inf"), (last + 16, "-inf"), (last + 46, "nan")):
+        key, val = kn.clone(), qkv.clone()
+        key[at, 0, 3] = float(value)
+        val[at, 2 * kv * dim + 1] = float(value)
+        for kk, vv in ((key, qkv), (kn, val)):
+            got = run(48, kk, vv)[0]
+            assert torch.equal(got[:at], ref[:at]), (at, value)
+            assert torch.equal(got.isfinite(), run(0, kk, vv)[0].isfinite()), (at, value)

@@ -403,6 +403,125 @@ extern "C" int holon_gemm_skinny_add_bf16(const void* x, const void* w_tiled, vo
   return 0;
 }
 
+// Several products of the same up to 16 rows that do not read one another's results, in one launch: each with operands, sizes and an output
+// form of its own, every sum in the order that the product by itself has. What bounds them one by one is not the weights: 2048 x 2048 by
+// itself takes 4.6 us in a step, of which its 8 MB are 1.2, the rest the kernel's start and end and a round of memory latency. Measured in a
+// step of one row, us, against the products one after the other: seven of 2,048 to 3,072 columns and one of 64 over 2,048 of K 12.5 (34);
+// 3,072 and 8,192 columns over 2,048 10.5 (12.9); 2,048 columns over 2,048 and over 8,192 of K 10.2 (13.9): 4.1 to 4.4 TB/s.
+// A block holds 16 waves: one tile of 16 columns whose K goes over 16 waves, two of 8 waves and so on; blocks with the most columns of K a
+// wave come first. SHORT: no wave has more than four steps of K, so that its loads need half the registers and a unit holds two blocks.
+constexpr int GROUP_MOST = 8, GROUP_WAVES = 16;
+struct GroupItem {
+  const bf16_t* x;
+  const bf16_t* w;             // tiled
+  void* y;
+  int N, K, waves, form;       // waves a tile; form as out_f32 of holon_gemm_skinny_bf16
+  int first;                   // the item's first block
+};
+struct GroupItems {
+  GroupItem at[GROUP_MOST];
+  int count, M;
+};
+
+template <bool SHORT, bool REST>
+__global__ void __launch_bounds__(GROUP_WAVES * 64, SHORT ? 8 : 4) gemm_skinny_group_kernel(GroupItems items) {
+  __shared__ f32x4_t red[GROUP_WAVES * WAVE];
+  const int all = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, g = lane / 16, c = lane % 16;
+  int n = 0;
+  while (n + 1 < items.count && (int)blockIdx.x >= items.at[n + 1].first) ++n;
+  const GroupItem it = items.at[n];
+  const int wave = all % it.waves, tile = ((int)blockIdx.x - it.first) * (GROUP_WAVES / it.waves) + all / it.waves;
+  const bool have = c < items.M, mine = tile < it.N / 16;
+  const int steps = mine ? it.K / 32 / it.waves : 0;
+  f32x4_t acc[1] = {{0.f, 0.f, 0.f, 0.f}};
+  const bf16_t* const wp[1] = {it.w + ((int64_t)tile * (it.K / 32) + (int64_t)wave * steps) * 512 + lane * 8};
+  const bf16_t* xp = it.x + (int64_t)c * it.K + (int64_t)wave * steps * 32 + 8 * g;
+  const auto tokens = [&](int s) -> bf16x8_t {
+    bf16x8_t xf;
+    if (have) {
+      xf = *reinterpret_cast<const bf16x8_t*>(xp + s * 32);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xf[i] = (__bf16)0.f;
+    }
+    return xf;
+  };
+  if constexpr (SHORT) {
+    bf16x8_t wf[4], xf[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u < steps) {
+        wf[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(wp[0] + (int64_t)u * 512));
+        xf[u] = tokens(u);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u < steps) acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc[0], 0, 0, 0);
+  } else {
+    stream_tiles<1, 4, REST>(acc, wp, 512, steps, tokens, [] {});
+  }
+  red[all * WAVE + lane] = acc[0];
+  __syncthreads();
+  if (wave > 0 || !mine) return;
+  for (int ww = 1; ww < it.waves; ++ww) acc[0] += red[(all + ww) * WAVE + lane];
+  if (!have) return;
+  const int64_t at = (int64_t)c * it.N + tile * 16 + 4 * g;
+  ushort4 o;
+  bf16_t* oe = reinterpret_cast<bf16_t*>(&o);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) oe[r] = float_to_bf16(acc[0][r]);
+  if (it.form == 2) {
+    f32x4_t wide;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) wide[r] = bf16_to_float(oe[r]);
+    *reinterpret_cast<f32x4_t*>((float*)it.y + at) = wide;
+    return;
+  }
+  if (it.form == 4)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float v = fmaxf(bf16_to_float(oe[r]), 0.f);
+      oe[r] = float_to_bf16(v * v);
+    }
+  *reinterpret_cast<ushort4*>((bf16_t*)it.y + at) = o;
+}
+
+// `items`: `count` (up to 8) of 3 pointers (x [M, K], w tiled, y [M, N]) and 3 sizes (N, K, form: 0 bfloat16, 2 float32 values that were
+// rounded to bfloat16 first, 4 bfloat16 max(product, 0)^2).
+extern "C" int holon_gemm_skinny_group_bf16(const int64_t* items, int count, int M, void* stream) {
+  HOLON_CHECK(count >= 1 && count <= GROUP_MOST && M >= 1 && M <= 16, "gemm (few rows, several): %d products of %d rows", count, M);
+  GroupItems g{};
+  g.count = count;
+  g.M = M;
+  for (int i = 0; i < count; ++i) {
+    const int64_t* v = items + 6 * i;
+    GroupItem it{(const bf16_t*)v[0], (const bf16_t*)v[1], (void*)v[2], (int)v[3], (int)v[4], 0, (int)v[5], 0};
+    HOLON_CHECK(holon_gemm_skinny_supported(M, it.N, it.K) && ((v[0] | v[1] | v[2]) & 15) == 0 &&
+                    (it.form == 0 || it.form == 2 || it.form == 4),
+                "gemm (few rows, several): M=%d N=%d K=%d form %d not served (N %% 16, K %% 32, operands at 16 bytes)", M, it.N, it.K, it.form);
+    it.waves = skinny_waves(it.N / 16, it.K);
+    int at = i;                                             // longest runs of K first
+    for (; at > 0 && g.at[at - 1].K / g.at[at - 1].waves < it.K / it.waves; --at) g.at[at] = g.at[at - 1];
+    g.at[at] = it;
+  }
+  int blocks = 0;
+  bool is_short = true, rest = false;
+  for (int i = 0; i < count; ++i) {
+    GroupItem& it = g.at[i];
+    const int per = GROUP_WAVES / it.waves, steps = it.K / 32 / it.waves;
+    it.first = blocks;
+    blocks += (it.N / 16 + per - 1) / per;
+    is_short = is_short && steps <= 4;
+    rest = rest || steps % 4 != 0;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  if (is_short) gemm_skinny_group_kernel<true, false><<<blocks, GROUP_WAVES * 64, 0, s>>>(g);
+  else if (rest) gemm_skinny_group_kernel<false, true><<<blocks, GROUP_WAVES * 64, 0, s>>>(g);
+  else gemm_skinny_group_kernel<false, false><<<blocks, GROUP_WAVES * 64, 0, s>>>(g);
+  HOLON_LAUNCH_OK();
+  return 0;
+}
+
 // The gated form: w = [gate rows; up rows] (2I rows), y[M, I] = round(act(round(x gate^T))) * round(x up^T), act silu or
 // (ACT 1) the tanh form of gelu, the roundings of the two-kernel composition. A block owns gate tile t and up tile t + I/16 and streams both.
 template <int WPB, int UNROLL, bool REST, bool TILED, int ACT>

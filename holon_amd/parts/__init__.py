@@ -12,6 +12,7 @@ from .convs import CausalConv
 from .recurrent import DecayMemory, GatedDelta
 from .sigmoid_attention import SigmoidWindowAttention
 from .stream32 import LayerNorm, Pending, PreNorm32
+from .products import Product, drive, products_of
 from .dyt import DynamicTanh, Sandwich32, Scaled
 from .softmax_attention import LatentAttention, SoftmaxAttention
 from .mlstm import MLSTM
@@ -26,4 +27,4 @@ __all__ = ["FLOAT32", "INT32", "MODEL", "Build", "EmbedPart", "NormPart", "Paged
            "SigmoidWindowAttention", "LayerNorm", "Pending", "PreNorm32", "ParallelMixers",
            "DynamicTanh", "Sandwich32", "Scaled", "LatentAttention", "SoftmaxAttention", "MLSTM", "Mamba2", "YarnRope",
            "MoE", "PolyNormFFN", "Parallel32", "RMSNorm32", "DiffAttention", "DenseFFN",
-           "BigramEmbedding", "PostNorm32", "GatedLinearAttention"]
+           "BigramEmbedding", "PostNorm32", "GatedLinearAttention", "Product", "drive", "products_of"]

@@ -31,6 +31,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
+from .products import Product, drive
 from .softmax_attention import attend, to_half_split
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -132,7 +133,7 @@ class DiffAttention(Part):
             self.drop("q")
         self._children["qkv"] = self.qkv
 
-    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step, site):
         k = self.kernels
         if site.writes != self.own_kv:
             raise ValueError("diff_attention: a layer with keys and values of its own writes its cache; one without "
@@ -140,14 +141,19 @@ class DiffAttention(Part):
         held = site.paged[self.state_name]
         view = step.paged[held.group]
         table = getattr(self.position, "table", None)
+        qkv, = yield [Product(self.qkv, x)]
         if self.own_kv:
-            q = k.head_prepare(self.qkv(x), 2 * self.heads, 2 * self.kv_heads, self.dim, self.vdim, self.q_norm,
+            q = k.head_prepare(qkv, 2 * self.heads, 2 * self.kv_heads, self.dim, self.vdim, self.q_norm,
                                self.k_norm, self.eps, table, step.positions, held.pages, view.write_page,
                                view.write_off, view.page_size, value_share=2)
         else:
-            q = k.head_prepare(self.qkv(x), 2 * self.heads, 0, self.dim, self.vdim, self.q_norm, self.q_norm,
+            q = k.head_prepare(qkv, 2 * self.heads, 0, self.dim, self.vdim, self.q_norm, self.q_norm,
                                self.eps, table, step.positions, None, None, None, view.page_size)
         maps = attend(k, q, held, view, step, 2 * self.kv_heads, self.vdim, None, self.scale, 0, value_share=2)
-        return self.o(k.diff_combine(maps, self.heads, self.kv_heads, self.vdim, self.lam, self.eps, 1.0 - self.diff))
+        out = k.diff_combine(maps, self.heads, self.kv_heads, self.vdim, self.lam, self.eps, 1.0 - self.diff)
+        return (yield [Product(self.o, out)])[0]
+
+    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
 
     __call__ = forward

@@ -12,6 +12,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, Stream
 from .linear import Linear
 from .norms import Normed
+from .products import Product, drive
 
 
 @register_part("ffn", "swiglu")
@@ -526,8 +527,12 @@ class PolyNormFFN(Part):
         self.attach("down_proj", Linear(build, inp=inter, out=hidden))
         self.declare("act", (4,), kind=FLOAT32, init="unit")
 
+    def products(self, x: torch.Tensor, step=None):
+        up, = yield [Product(self.up_proj, x)]
+        return (yield [Product(self.down_proj, self.kernels.polynorm(up, self.act, self.eps))])[0]
+
     def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
-        return self.down_proj(self.kernels.polynorm(self.up_proj(x), self.act, self.eps))
+        return drive(self.kernels, x.shape[0], self.products(x, step))[0]
 
     __call__ = forward
 
@@ -547,12 +552,12 @@ class DenseFFN(Part):
         self.attach("up_proj", Linear(build, inp=hidden, out=inter))
         self.attach("down_proj", Linear(build, inp=inter, out=hidden))
 
+    def products(self, x: torch.Tensor, step=None):
+        y, = yield [Product(self.up_proj, x, relu2=True)]
+        return (yield [Product(self.down_proj, y)])[0]
+
     def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
-        up = self.up_proj
-        y = self.kernels.linear_relu2(x, up.weight, up.tiled if up.folded is None else None)
-        if y is None:
-            y = self.kernels.relu2(up(x))
-        return self.down_proj(y)
+        return drive(self.kernels, x.shape[0], self.products(x, step))[0]
 
     __call__ = forward
 

@@ -15,6 +15,7 @@ from ..kernels.registry import KernelOp, register_kernel
 from ..registry import register_part
 from .base import FLOAT32, Build, Part, SlotState
 from .linear import Linear
+from .products import Product, drive
 from .recurrent import MAX_KEY_DIM, _need, _rows, gated_out_plain, scan_pieces
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -193,22 +194,26 @@ class GatedLinearAttention(Part):
             self.drop("inp")
         return inp
 
-    def forward(self, x: torch.Tensor, step, site, rows: torch.Tensor | None = None, at: int = 0) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step, site, rows: torch.Tensor | None = None, at: int = 0):
         """`rows`: the input's projections, this mixer's from column `at` on (None: made here from `x`)."""
         k = self.kernels
         if rows is None:
-            rows = self.inp(x)
+            rows, = yield [Product(self.inp, x)]
         c, n = self.heads * self.dim, self.heads * self.vdim
         q, kk = rows[:, at: at + c], rows[:, at + c: at + 2 * c]
         v, gate = rows[:, at + 2 * c: at + 2 * c + n], rows[:, at + 2 * c + n: at + 2 * c + 2 * n]
         a = rows[:, at + 2 * c + 2 * n: at + 2 * c + 2 * n + self.rank]
         state = site.slot_state[self.state_name]
         if step.rows.in_order and gla_step_serves(self.dim, self.vdim):       # single tokens: one kernel
-            return self.o(k.gla_step(q, kk, v, gate, a, self.scale, self.a2t, self.a2_bias, self.tau, self.norm, self.eps,
-                                     state, step.slots, step.starts, self.heads))
+            y = k.gla_step(q, kk, v, gate, a, self.scale, self.a2t, self.a2_bias, self.tau, self.norm, self.eps, state,
+                           step.slots, step.starts, self.heads)
+            return (yield [Product(self.o, y)])[0]
         alpha = k.gla_decay(a, self.a2t, self.a2_bias, self.tau)
         o = k.gla_scan(q, kk, v, self.scale, alpha, state, step.slots, step.starts, step.query_start, step.n_rows,
                        self.heads, scan_pieces(step, PIECE, PIECES_FROM))
-        return self.o(k.gated_out(o, gate, self.norm, False, self.eps, self.build.dtype))
+        return (yield [Product(self.o, k.gated_out(o, gate, self.norm, False, self.eps, self.build.dtype))])[0]
+
+    def forward(self, x: torch.Tensor, step, site, rows: torch.Tensor | None = None, at: int = 0) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step, site, rows, at))[0]
 
     __call__ = forward

@@ -9,6 +9,7 @@ from ..spec import PartRef
 from .base import Build, PagedState, Part, Stream
 from .linear import Linear
 from .norms import Normed
+from .products import drive, products_of
 
 
 @register_part("mixer", "gqa")
@@ -149,7 +150,8 @@ class ParallelMixers(Part):
             rows = self.inp(x)
             left.update(rows=rows)
             right.update(rows=rows, at=self.right_at)
-        return Pending([(self.left(x, step, site, **left), self.left_scale),
-                        (self.right(x, step, site, **right), self.right_scale)], self.row)
+        one, two = drive(self.kernels, x.shape[0], products_of(self.left, x, step, site, **left),
+                         products_of(self.right, x, step, site, **right))
+        return Pending([(one, self.left_scale), (two, self.right_scale)], self.row)
 
     __call__ = forward

@@ -30,6 +30,7 @@ from ..spec import PartRef
 from .base import FLOAT32, Build, NormPart, Part, Stream
 from .convs import CausalConv
 from .dyt import Scaled
+from .products import drive, products_of
 from .stream32 import Pending, _terms
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -356,9 +357,9 @@ class Parallel32(Part):
         norm's kernel. A mixer that names a bias on its last projection (`out_row`, a float32 vector) is asked to
         leave it out (`add_row=False`): it joins the stream in float32, in the same kernel as the terms."""
         row = getattr(self.mixer, "out_row", None)
-        out = [self.mixer(a, step, site) if row is None else self.mixer(a, step, site, add_row=False)]
+        parts = [products_of(self.mixer, a, step, site, **({} if row is None else {"add_row": False}))]
         if self.ffn is not None:
-            out.append(self.ffn(a if self.shared_norm else b, step))
-        return Pending([(t, 1.0) for t in out], row)
+            parts.append(products_of(self.ffn, a if self.shared_norm else b, step))
+        return Pending([(t, 1.0) for t in drive(self.kernels, a.shape[0], *parts)], row)
 
     __call__ = forward

@@ -16,6 +16,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, SlotState
 from .convs import CausalConv
 from .linear import Linear
+from .products import Product, drive
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -320,14 +321,18 @@ class GatedDelta(Part):
             self.drop(nm)
         self._children.update(qkv=self.qkv, ab=self.ab, conv=self.conv)
 
-    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step, site):
         k = self.kernels
-        qkv = self.conv(self.qkv(x), step, site)
-        qn, kn, beta, g = k.delta_prepare(qkv, self.ab(x), self.A_log, self.dt_bias, self.heads, self.kv_heads,
+        qkv, ab, gate = yield [Product(self.qkv, x), Product(self.ab, x), Product(self.g, x)]
+        qkv = self.conv(qkv, step, site)
+        qn, kn, beta, g = k.delta_prepare(qkv, ab, self.A_log, self.dt_bias, self.heads, self.kv_heads,
                                           self.dim, self.vdim)
         o = k.delta_scan(qn, kn, qkv, beta, g, site.slot_state[self.prefix + "S"], step.slots, step.starts,
                          step.query_start, step.n_rows, self.heads, self.vdim, delta_pieces(step, self.heads * self.vdim, self.build.dtype))
-        return self.o(k.gated_out(o, self.g(x), self.norm, False, self.eps, self.build.dtype))
+        return (yield [Product(self.o, k.gated_out(o, gate, self.norm, False, self.eps, self.build.dtype))])[0]
+
+    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
 
     __call__ = forward
 
@@ -360,7 +365,7 @@ class DecayMemory(Part):
         self.declare("w0", (heads * dim,), kind=FLOAT32, init="zero")
         self.declare("u", (heads, dim), kind=FLOAT32, init="zero")
         self.declare("norm", (heads * dim,), init="norm")
-        self.mu = self.w2t = None
+        self.mu = self.w2t = self.lora = None
 
     def state(self):
         return [SlotState(self.prefix + "shift", (self.hidden,)),
@@ -373,20 +378,26 @@ class DecayMemory(Part):
         if self.mu_r is not None:
             self.mu = torch.stack([getattr(self, f"mu_{s}") for s in self.MIXES]).contiguous()
             self.w2t = self.w2.t().contiguous()       # [rank, channels]: what the decay's kernel streams
+            self.lora = Linear(self.build, inp=self.hidden, out=self.w1.shape[0])
+            self.lora.weight = self.w1
+            self.lora.finalize()                      # (its tiled copy, for steps of few rows)
 
     def extra_tensors(self):
-        return [self.mu, self.w2t] if self.mu is not None else []
+        return [self.mu, self.w2t, *self.lora.extra_tensors()] if self.mu is not None else []
 
-    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step, site):
         k = self.kernels
         rows = (step.slots, step.starts, step.query_start)
         mixes = k.shift_mix(x, self.mu, site.slot_state[self.prefix + "shift"], *rows, step.token_row, step.n_rows,
                             step.rows.in_order)
-        r, kk, v, gate = (getattr(self, nm)(mixes[i]) for i, nm in enumerate(("r", "k", "v", "g")))
-        lora = k.linear(mixes[4], self.w1, torch.float32)
+        r, kk, v, gate, lora = yield [Product(getattr(self, nm), mixes[i]) for i, nm in enumerate(("r", "k", "v", "g"))] + \
+            [Product(self.lora, mixes[4], torch.float32)]
         decay = k.decay_lora(lora, self.w2t, self.w0)
         o = k.memory_scan(r, kk, v, decay, self.u, site.slot_state[self.prefix + "S"], *rows, step.n_rows, self.heads,
                           scan_pieces(step))
-        return self.o(k.gated_out(o, gate, self.norm, True, self.eps, self.build.dtype))
+        return (yield [Product(self.o, k.gated_out(o, gate, self.norm, True, self.eps, self.build.dtype))])[0]
+
+    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
 
     __call__ = forward

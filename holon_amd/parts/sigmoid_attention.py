@@ -18,6 +18,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
+from .products import Product, drive
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -236,20 +237,23 @@ class SigmoidWindowAttention(Part):
             self.drop(name)
         self._children["qkv"] = self.qkv
 
-    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step, site):
         k = self.kernels
         held = site.paged[self.state_name]
         view = step.paged[held.group]
         table = getattr(self.position, "table", None)
-        q = k.head_prepare(self.qkv(x), self.heads, self.kv_heads, self.dim, self.vdim,
+        qkv, *gate = yield [Product(self.qkv, x)] + ([Product(self.g, x)] if self.g is not None else [])
+        q = k.head_prepare(qkv, self.heads, self.kv_heads, self.dim, self.vdim,
                            getattr(self, "q_norm", None) if self.eps is not None else None,
                            getattr(self, "k_norm", None) if self.eps is not None else None,
                            self.eps or 0.0, table, step.positions, held.pages, view.write_page, view.write_off,
                            view.page_size)
-        gate = self.g(x) if self.g is not None else None
         out = k.sigmoid_attention(q, held.pages, view.table, step.rows, step.token_row, step.positions,
                                   self.kv_heads, self.vdim, view.page_size, self.pb if self.head_bias else None,
-                                  self.scale, self.window, gate)
-        return self.o(out)
+                                  self.scale, self.window, *(gate or (None,)))
+        return (yield [Product(self.o, out)])[0]
+
+    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
 
     __call__ = forward

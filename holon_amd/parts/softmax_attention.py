@@ -21,6 +21,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
+from .products import Product, drive
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -605,13 +606,13 @@ class SoftmaxAttention(Part):
         self.drop("qkv")
         return qkv
 
-    def forward(self, x: torch.Tensor, step, site, add_row: bool = True, rows: torch.Tensor | None = None) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step, site, add_row: bool = True, rows: torch.Tensor | None = None):
         """`rows`: the input's projections, this mixer's in the first columns (None: made here from `x`)."""
         k = self.kernels
         held = site.paged[self.state_name]
         view = step.paged[held.group]
         table = getattr(self.position, "table", None)
-        qkv = self.qkv(x) if rows is None else rows
+        qkv = (yield [Product(self.qkv, x)])[0] if rows is None else rows
         if self.whole_norm is not None:
             q = k.whole_norm_prepare(qkv, self.heads, self.kv_heads, self.dim, self.vdim, self.q_norm,
                                      self.k_norm, self.whole_norm, held.pages, view.write_page, view.write_off,
@@ -626,8 +627,11 @@ class SoftmaxAttention(Part):
         out = attend(k, q, held, view, step, self.kv_heads, self.vdim, sink, self.scale,
                      self.sees, self.softcap, (self.r1, self.r2) if self.distance_bias else None, self.keep_first,
                      head_gate=gates)
-        out = self.o(out)
+        out, = yield [Product(self.o, out)]
         return k.add_bias(out, self.o_bias) if self.has_o_bias and add_row else out
+
+    def forward(self, x: torch.Tensor, step, site, add_row: bool = True, rows: torch.Tensor | None = None) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step, site, add_row, rows))[0]
 
     __call__ = forward
 
@@ -752,7 +756,7 @@ class LatentAttention(Part):
         held = [self.uk_t] if self.uk_t is not None else []
         return held + ([self.uv_h] if self.rot_dim and self.entries == 2 and self.uv_h is not None else [])
 
-    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step, site):
         k = self.kernels
         t = x.shape[0]
         if site.writes != self.own_kv:
@@ -760,7 +764,7 @@ class LatentAttention(Part):
                              "another run's")
         held = site.paged[self.state_name]
         view = step.paged[held.group]
-        both = self.down(x)
+        both, = yield [Product(self.down, x)]
         if self.q_rank == 0:                      # norm, rotation and the cache write in one kernel
             table = getattr(self.position, "table", None)
             if self.own_kv:
@@ -781,7 +785,8 @@ class LatentAttention(Part):
                 c = self.dkv_norm(both[:, self.q_rank:].contiguous()).view(t, 1, self.kv_rank)
                 k.kv_write(c, c, held.pages.view(-1, 2, 1, view.page_size * self.kv_rank), view.write_page,
                            view.write_off, view.page_size)
-            q = k.head_linear(self.uq(cq).view(t, self.heads, self.dim), self.uk_t)
+            uq, = yield [Product(self.uq, cq)]
+            q = k.head_linear(uq.view(t, self.heads, self.dim), self.uk_t)
         sink = self.sink if self.has_sink else None
         if self.entries == 1:
             mixed = k.latent_attention(q, held.pages, view.table, step.rows, step.token_row, step.positions, self.kv_rank,
@@ -791,6 +796,9 @@ class LatentAttention(Part):
                            ).view(t, self.heads, self.width)
         gate = both[:, self.gate_at: self.gate_at + self.heads * self.vdim] if self.has_gate else None
         out = k.head_linear(mixed, self.uv_h, gate=gate) if gate is not None else k.head_linear(mixed, self.uv_h)
-        return self.o(out.view(t, self.heads * self.vdim))
+        return (yield [Product(self.o, out.view(t, self.heads * self.vdim))])[0]
+
+    def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
 
     __call__ = forward

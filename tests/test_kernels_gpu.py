@@ -1645,3 +1645,29 @@ def test_whole_norm_prepare_around_its_block_sizes(hip, heads, kv, dim, vdim):
     assert H.rel_rms(held[257][0], want) < 3e-3 and H.rel_rms(held[257][1], plain) < 3e-3
     assert torch.equal(held[256][0], held[257][0][:256]) and torch.equal(held[256][1][:16], held[257][1][:16])
     assert torch.equal(held[1][0], held[257][0][:1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 5, 16])
+@pytest.mark.parametrize("sizes", [[(2048, 2048), (64, 2048), (16, 512)], [(2064, 512), (5136, 512), (48, 1184), (80, 288), (32, 256)],
+                                   [(128, 2048), (144, 8192), (528, 352)] * 3, [(8192, 256)] * 2 + [(40, 256)]])
+def test_products_in_one_launch_are_the_products(hip, rows, sizes):
+    """`linear_group`, in every output form, bit for bit against each product by itself: tiles of 16, 8, 4, 2 and 1 waves, tiles that do
+    not fill a block, short and long runs of K with and without a rest, more products than a launch takes, one that is not served."""
+    from holon_amd.parts.products import Product
+    k, gen = hip, torch.Generator(device="cuda").manual_seed(rows)
+
+    class Weights:                                # what a projection holds
+        folded, kernels = None, hip
+
+        def __init__(self, n, kk):
+            self.weight = (0.05 * torch.randn(n, kk, generator=gen, device="cuda")).bfloat16()
+            self.tiled = k.tile_weight(self.weight)
+
+        def __call__(self, x, dtype=None):
+            return k.linear(x, self.weight, dtype, self.tiled)
+    products = [Product(Weights(n, kk), torch.randn(rows, kk, generator=gen, device="cuda").bfloat16(),
+                        **({}, {"dtype": torch.float32}, {"relu2": True})[i % 3]) for i, (n, kk) in enumerate(sizes)]
+    for p, got in zip(products, k.linear_group(products)):
+        want = p.alone()
+        assert got.dtype == want.dtype and torch.equal(got, want), (p.linear.weight.shape, p.dtype, p.relu2)

@@ -30,39 +30,55 @@ constexpr int EXTRA = 16;                  // rows a tile may take beyond its 25
 constexpr int EXTRA_BYTES = EXTRA * KC * 2;
 constexpr int XCDS = 8;
 
+// How the eight waves share a tile: a wave has TR tiles of 16 rows and TC of 16 columns of each quarter, so that a quarter is 128 rows by
+// 16 TC CW columns. <4, 2>: two waves by four, 256 x 256. <2, 3>: four by two, 256 rows by 192 columns, for products whose tiles of 256 columns
+// would leave a round of the compute units partly idle (a chunk costs it 20 reads of LDS for 48 matrix instructions a wave where the other has 24
+// for 64, and 0.8 to 0.87 of the time).
+template <int TR, int TC>
+struct Shape {
+  static constexpr int RW = HALF / (16 * TR), CW = 8 / RW, COLS = 16 * TC * CW;      // COLS: columns of a half
+};
+
 // [half of the rows][half of the columns][tile of 16 rows][tile of 16 columns]: a lane holds columns 4 (lane / 16) .. + 3 of
 // a tile for its row lane % 16
-struct Acc {
-  f32x4_t v[2][2][4][2];
+template <int TR, int TC>
+struct AccOf {
+  f32x4_t v[2][2][TR][TC];
   __device__ __forceinline__ void clear() {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < TR; ++t)
 #pragma unroll
-          for (int n = 0; n < 2; ++n) v[i][j][t][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          for (int n = 0; n < TC; ++n) v[i][j][t][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 };
+using Acc = AccOf<4, 2>;
 
 // Where the lane's part of the tile lies: row `row(i, t)` (of 256) of tile t in half i, first of its four columns
-// `column(j, n)` (of 256).
-struct Place {
+// `column(j, n)` (of 2 COLS). Extra rows: of half j of the columns, one tile of 16 a wave (`extra_column(j)`: the lane's first of four; the
+// waves that `has_extra` leaves out have none), row lane % 16.
+template <int TR, int TC>
+struct PlaceOf {
+  using S = Shape<TR, TC>;
   int wr, wc, g, c;
-  __device__ __forceinline__ Place()
-      : wr(__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) / 4), wc(__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) % 4),
+  __device__ __forceinline__ PlaceOf()
+      : wr(__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) / S::CW), wc(__builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) % S::CW),
         g(threadIdx.x % WAVE / 16), c(threadIdx.x % 16) {}
-  __device__ __forceinline__ int row(int i, int t) const { return i * HALF + wr * 64 + t * 16 + c; }
-  __device__ __forceinline__ int column(int j, int n) const { return j * HALF + wc * 32 + n * 16 + 4 * g; }
+  __device__ __forceinline__ int row(int i, int t) const { return i * HALF + wr * 16 * TR + t * 16 + c; }
+  __device__ __forceinline__ int column(int j, int n) const { return j * S::COLS + wc * 16 * TC + n * 16 + 4 * g; }
+  __device__ __forceinline__ bool has_extra() const { return wr < TC; }
+  __device__ __forceinline__ int extra_column(int j) const { return j * S::COLS + wc * 16 * TC + wr * 16 + 4 * g; }
 };
+using Place = PlaceOf<4, 2>;
 
-// The extra rows' sums: of half j of the columns, one tile of 16 a wave (`extra_column(j)`: the lane's first of four), row lane % 16.
+// The extra rows' sums, by half of the columns.
 struct ExtraAcc {
   f32x4_t v[2];
   __device__ __forceinline__ void clear() { v[0] = v[1] = f32x4_t{0.f, 0.f, 0.f, 0.f}; }
 };
-__device__ __forceinline__ int extra_column(const Place& at, int j) { return j * HALF + at.wc * 32 + at.wr * 16 + 4 * at.g; }
 
 // What a lane copies of each 128 rows of a chunk: rows `copy_row(q)` (q = 0, 1), from `copy_piece(q)` bytes into the chunk's
 // 128 bytes of that row.
@@ -79,11 +95,12 @@ __device__ __forceinline__ void phase_barrier() {           // (nothing is moved
 // chunk (row and piece). `chunks` (K / 64): even, at least 2. Every wave of the block comes here, with the same `chunks`.
 // MORE: 16 extra rows as well (`more`; `more_at`: as x_at, of rows copy_row(0) up to 15; LDS of LDS_BYTES + 2 EXTRA_BYTES). Waves 0 and 1
 // then have a copy more under way, and wait for one more than they need.
-template <bool MORE>
-__device__ __forceinline__ void run_with(Acc& acc, ExtraAcc& more, char* lds, const bf16_t* x, const bf16_t* w,
+template <bool MORE, int TR, int TC>
+__device__ __forceinline__ void run_with(AccOf<TR, TC>& acc, ExtraAcc& more, char* lds, const bf16_t* x, const bf16_t* w,
                                          const uint32_t (&x_at)[2][2], const uint32_t (&w_at)[2][2], uint32_t more_at, int chunks) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-  const int wr = wave / 4, wc = wave % 4, g = lane / 16, c = lane % 16;
+  using S = Shape<TR, TC>;
+  const int wr = wave / S::CW, wc = wave % S::CW, late = wave / 4, g = lane / 16, c = lane % 16;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
   const auto copy = [&](int which, int chunk) {             // 0: columns' first half, 1: rows' first half, 2, 3: the second ones
     const int h = which / 2;
@@ -96,39 +113,40 @@ __device__ __forceinline__ void run_with(Acc& acc, ExtraAcc& more, char* lds, co
   uint32_t at[2];                                           // this lane's 16 bytes of its row of a tile, per 32 of the chunk
 #pragma unroll
   for (int s = 0; s < 2; ++s) at[s] = c * (KC * 2) + 16 * ((4 * s + g) ^ ((c / 2) % 8));
-  const auto read_rows = [&](bf16x8_t (&a)[2][4], int half, int chunk) {
-    const char* p = lds + (chunk & 1) * STAGE + (1 + 2 * half) * REGION + wr * 64 * KC * 2;
+  const auto read_rows = [&](bf16x8_t (&a)[2][TR], int half, int chunk) {
+    const char* p = lds + (chunk & 1) * STAGE + (1 + 2 * half) * REGION + wr * 16 * TR * KC * 2;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) a[s][t] = *reinterpret_cast<const bf16x8_t*>(p + t * 16 * KC * 2 + at[s]);
+      for (int t = 0; t < TR; ++t) a[s][t] = *reinterpret_cast<const bf16x8_t*>(p + t * 16 * KC * 2 + at[s]);
   };
-  const auto read_columns = [&](bf16x8_t (&b)[2][2], int half, int chunk) {
-    const char* p = lds + (chunk & 1) * STAGE + 2 * half * REGION + wc * 32 * KC * 2;
+  const auto read_columns = [&](bf16x8_t (&b)[2][TC], int half, int chunk) {
+    const char* p = lds + (chunk & 1) * STAGE + 2 * half * REGION + wc * 16 * TC * KC * 2;
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) b[s][t] = *reinterpret_cast<const bf16x8_t*>(p + t * 16 * KC * 2 + at[s]);
+      for (int t = 0; t < TC; ++t) b[s][t] = *reinterpret_cast<const bf16x8_t*>(p + t * 16 * KC * 2 + at[s]);
   };
   constexpr std::integral_constant<int, 0> c0{};
   constexpr std::integral_constant<int, 1> c1{};
   constexpr std::integral_constant<int, 2> c2{};
   bf16x8_t extra[2];
-  const auto multiply = [&](f32x4_t (&d)[4][2], const bf16x8_t (&a)[2][4], const bf16x8_t (&b)[2][2], auto with) {      // with: the extra
+  const auto multiply = [&](f32x4_t (&d)[TR][TC], const bf16x8_t (&a)[2][TR], const bf16x8_t (&b)[2][TC], auto with) {      // with: the extra
     phase_barrier();
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < TR; ++t)
 #pragma unroll
-        for (int n = 0; n < 2; ++n) d[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][n], a[s][t], d[t][n], 0, 0, 0);
+        for (int n = 0; n < TC; ++n) d[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][n], a[s][t], d[t][n], 0, 0, 0);
     constexpr int J = decltype(with)::value;                // rows too, of half J of the columns (2: not)
     if constexpr (MORE && J < 2) {
 #pragma unroll
       for (int s = 0; s < 2; ++s)
-        if (wr == 0) more.v[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][0], extra[s], more.v[J], 0, 0, 0);
-        else more.v[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][1], extra[s], more.v[J], 0, 0, 0);
+#pragma unroll
+        for (int n = 0; n < TC; ++n)
+          if (wr == n) more.v[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[s][n], extra[s], more.v[J], 0, 0, 0);
     }
     __builtin_amdgcn_s_setprio(0);
     phase_barrier();
@@ -136,7 +154,7 @@ __device__ __forceinline__ void run_with(Acc& acc, ExtraAcc& more, char* lds, co
   // in front of the barrier behind which the other wave of the SIMD may ask for what overwrites what was read
   const auto reads_done = [&] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
 
-  bf16x8_t a[2][4], b[2][2][2];
+  bf16x8_t a[2][TR], b[2][2][TC];
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -146,7 +164,7 @@ __device__ __forceinline__ void run_with(Acc& acc, ExtraAcc& more, char* lds, co
   read_columns(b[0], 0, 0);
   reads_done();
   phase_barrier();
-  if (wr == 1) phase_barrier();                             // half a step behind the other four waves
+  if (late == 1) phase_barrier();                           // half a step behind the other four waves
   // P: k % 2, the set of b that holds the columns' first half. T: 0 while chunks are still asked for, 1 the last but one, 2 the
   // last. A step's wait is for what the next step reads: everything but the copies asked for after it, two a step and wave.
   const auto chunk = [&](auto parity, auto tail, int k) {
@@ -181,13 +199,13 @@ __device__ __forceinline__ void run_with(Acc& acc, ExtraAcc& more, char* lds, co
   }
   chunk(c0, c1, chunks - 2);
   chunk(c1, c2, chunks - 1);
-  if (wr == 0) phase_barrier();                             // (as many barriers as the other four waves)
+  if (late == 0) phase_barrier();                           // (as many barriers as the other four waves)
 }
 
 __device__ __forceinline__ void run(Acc& acc, char* lds, const bf16_t* x, const bf16_t* w, const uint32_t (&x_at)[2][2],
                                     const uint32_t (&w_at)[2][2], int chunks) {
   ExtraAcc none;
-  run_with<false>(acc, none, lds, x, w, x_at, w_at, 0, chunks);
+  run_with<false, 4, 2>(acc, none, lds, x, w, x_at, w_at, 0, chunks);
 }
 
 // The tile that block `id` takes of `total`, -1: none. Blocks go to the XCDs in turn; each XCD gets a run of neighbouring

@@ -14,13 +14,15 @@ enum { SILU, GELU, PARTS };
 
 // What a tile gives, from LDS in whole lines: the gated ones bfloat16 y [M, N], 128 columns a tile (the tile's first half of columns are
 // gates and the second ups of w [2 N, K]), PARTS float32 y [splits, M, N].
-template <int KIND>
+template <int KIND, int TR, int TC>
 __global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                 void* __restrict__ y, int M, int N, int K, int row_tiles,
                                                                 int col_tiles, int splits) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES + 2 * EXTRA_BYTES];
   constexpr bool GATED = KIND == SILU || KIND == GELU;
-  constexpr int COLS = GATED ? HALF : TILE;
+  using S = Shape<TR, TC>;
+  static_assert(GATED || S::COLS == HALF, "products in shares: 256 x 256 tiles alone");
+  constexpr int COLS = GATED ? S::COLS : TILE;
   const int tiles = row_tiles * col_tiles;
   int tile = tile_of_block(blockIdx.x, tiles * splits);
   if (tile < 0) return;
@@ -37,21 +39,21 @@ __global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __
     for (int q = 0; q < 2; ++q) {                    // (rows and columns past the last repeat it: nothing of them is written)
       const int r = copy_row(q);
       x_at[h][q] = (uint32_t)((int64_t)min(m0 + h * HALF + r, M - 1) * K * 2) + copy_piece(q);
-      const int64_t column = GATED ? (int64_t)h * N + min(n0 + r, N - 1) : min(n0 + h * HALF + r, N - 1);
+      const int64_t column = GATED ? (int64_t)h * N + min(n0 + min(r, COLS - 1), N - 1) : min(n0 + h * HALF + r, N - 1);
       w_at[h][q] = (uint32_t)(column * K * 2) + copy_piece(q);
     }
   const uint32_t more_at = (uint32_t)((int64_t)min(m0 + TILE + copy_row(0) % EXTRA, M - 1) * K * 2) + copy_piece(0);
-  Acc acc;
+  AccOf<TR, TC> acc;
   ExtraAcc more;
   acc.clear();
   more.clear();
   const int64_t k0 = (int64_t)split * share;
-  if (has_more) run_with<true>(acc, more, lds, x + k0, w + k0, x_at, w_at, more_at, share / KC);
-  else run_with<false>(acc, more, lds, x + k0, w + k0, x_at, w_at, 0, share / KC);
-  const Place at;
+  if (has_more) run_with<true, TR, TC>(acc, more, lds, x + k0, w + k0, x_at, w_at, more_at, share / KC);
+  else run_with<false, TR, TC>(acc, more, lds, x + k0, w + k0, x_at, w_at, 0, share / KC);
+  const PlaceOf<TR, TC> at;
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   if constexpr (GATED) {
-    constexpr int ACT = KIND == GELU, PITCH = HALF * 2 + 16, ROWS = TILE + EXTRA;
+    constexpr int ACT = KIND == GELU, PITCH = COLS * 2 + 16, ROWS = TILE + EXTRA, PIECES = COLS / 8;
     static_assert(ROWS * PITCH <= LDS_BYTES, "a tile's columns");
     const auto gated = [](f32x4_t gate, f32x4_t up) {                      // the roundings of the product and of the gated kernels
       ushort4 o;
@@ -64,17 +66,17 @@ __global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < TR; ++t)
 #pragma unroll
-        for (int n = 0; n < 2; ++n)
+        for (int n = 0; n < TC; ++n)
           *reinterpret_cast<ushort4*>(lds + at.row(i, t) * PITCH + at.column(0, n) * 2) = gated(acc.v[i][0][t][n], acc.v[i][1][t][n]);
-    if (has_more) *reinterpret_cast<ushort4*>(lds + (TILE + at.c) * PITCH + extra_column(at, 0) * 2) = gated(more.v[0], more.v[1]);
+    if (has_more && at.has_extra()) *reinterpret_cast<ushort4*>(lds + (TILE + at.c) * PITCH + at.extra_column(0) * 2) = gated(more.v[0], more.v[1]);
     __syncthreads();
-    for (int e = threadIdx.x; e < (has_more ? ROWS : TILE) * 16; e += THREADS) {
-      const int row = e / 16, column = n0 + e % 16 * 8;
+    for (int e = threadIdx.x; e < (has_more ? ROWS : TILE) * PIECES; e += THREADS) {
+      const int row = e / PIECES, column = n0 + e % PIECES * 8;
       if (m0 + row < M && column < N)
         *reinterpret_cast<uint4*>((bf16_t*)y + (int64_t)(m0 + row) * N + column) =
-            *reinterpret_cast<const uint4*>(lds + row * PITCH + e % 16 * 16);
+            *reinterpret_cast<const uint4*>(lds + row * PITCH + e % PIECES * 16);
     }
   } else {
     constexpr int PITCH = 144;                       // a wave's own 64 rows of 32 columns at a time
@@ -101,10 +103,22 @@ __global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __
     if (has_more && m0 + TILE + at.c < M)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int column = n0 + extra_column(at, j);
+        const int column = n0 + at.extra_column(j);
         if (column < N) *reinterpret_cast<f32x4_t*>(out + (int64_t)(m0 + TILE + at.c) * N + column) = more.v[j];
       }
   }
+}
+
+constexpr int SLIM = Shape<2, 3>::COLS;      // a gated product's columns a tile in the form of 192
+
+// Whether a gated product's tiles are 192 columns wide (96 gates and their ups): by the rounds of one tile a compute unit that either takes, of
+// which the slim one's lasts 0.8 to 0.87 as long. Measured, us, tiles of 256 columns against 192 (rounds): 12,288 x 4,096 at 256 / 520 / 768 /
+// 1,400 / 2,048 / 4,096 rows 85 (1) / 115 (1) / 166 (2) / 255 (3) / 280 (3) / 558 (6) and 78 (1) / 97 (1) / 143 (2) / 224 (3) / 300 (4) / 592 (8);
+// 8,192 x 2,048 at 400 / 768 / 2,048 41 (1) / 45 (1) / 105 (2) and 34 (1) / 68 (2) / 124 (3); 9,728 x 2,560 at 520 / 1,024 / 1,400 65 (1) / 119
+// (2) / 120 (2) and 58 (1) / 104 (2) / 141 (3). Of 80 products the rule's choice is never the slower one by more than 1 %.
+bool slim_pays(int row_tiles, int N) {
+  const auto rounds = [&](int wide) { return (row_tiles * ((N + wide - 1) / wide) + 255) / 256; };
+  return 0.85f * rounds(SLIM) < rounds(HALF);
 }
 
 int row_tiles_of(int M) { return M > TILE && M % TILE && M % TILE <= EXTRA ? M / TILE : (M + TILE - 1) / TILE; }
@@ -116,18 +130,26 @@ extern "C" int holon_gemm_block_supported(int M, int N, int K, int gated, int sp
          ((int64_t)N * (gated ? 2 : 1)) * K < (int64_t)1 << 31;
 }
 
-static int launch_block(int kind, const void* x, const void* w, void* y, int M, int N, int K, int splits, void* stream) {
+static int launch_block(int kind, const void* x, const void* w, void* y, int M, int N, int K, int splits, int width, void* stream) {
   const bool gated = kind == SILU || kind == GELU;
   HOLON_CHECK(holon_gemm_block_supported(M, N, K, gated, splits) && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) == 0,
               "gemm (many rows): M=%d N=%d K=%d in %d shares not served", M, N, K, splits);
-  const int rows = row_tiles_of(M), cols = (N + (gated ? HALF : TILE) - 1) / (gated ? HALF : TILE);
+  const int rows = row_tiles_of(M);
+  const bool slim = gated && (width ? width == SLIM : slim_pays(rows, N));
+  const int wide = gated ? (slim ? SLIM : HALF) : TILE, cols = (N + wide - 1) / wide;
   const unsigned blocks = (unsigned)(((int64_t)rows * cols * splits + XCDS - 1) / XCDS * XCDS);      // every XCD as many
   hipStream_t s = (hipStream_t)stream;
   const bf16_t *a = (const bf16_t*)x, *b = (const bf16_t*)w;
   switch (kind) {
-    case SILU: gemm_block_kernel<SILU><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
-    case GELU: gemm_block_kernel<GELU><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
-    default: gemm_block_kernel<PARTS><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
+    case SILU:
+      if (slim) gemm_block_kernel<SILU, 2, 3><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
+      else gemm_block_kernel<SILU, 4, 2><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
+      break;
+    case GELU:
+      if (slim) gemm_block_kernel<GELU, 2, 3><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
+      else gemm_block_kernel<GELU, 4, 2><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
+      break;
+    default: gemm_block_kernel<PARTS, 4, 2><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
   }
   HOLON_LAUNCH_OK();
   return 0;
@@ -135,7 +157,12 @@ static int launch_block(int kind, const void* x, const void* w, void* y, int M, 
 
 // y [M, N] = act(x gates^T) * (x ups^T) over w [2 N, K] (gates, then ups); act 0 silu, 1 gelu in its tanh form.
 extern "C" int holon_gemm_block_glu_bf16(const void* x, const void* w, void* y, int M, int N, int K, int act, void* stream) {
-  return launch_block(act ? GELU : SILU, x, w, y, M, N, K, 1, stream);
+  return launch_block(act ? GELU : SILU, x, w, y, M, N, K, 1, 0, stream);
+}
+// The same with the columns of y a tile has, 128 or 96, named (0: by the rule above). The sums are the same.
+extern "C" int holon_gemm_block_glu_width_bf16(const void* x, const void* w, void* y, int M, int N, int K, int act, int width, void* stream) {
+  HOLON_CHECK(width == 0 || width == HALF || width == SLIM, "gemm (many rows): tiles of %d columns", width);
+  return launch_block(act ? GELU : SILU, x, w, y, M, N, K, 1, width, stream);
 }
 
 // Whether a product in shares takes this form where gemm_tiles.hip's would serve it too: with its last rows filled up that one's blocks
@@ -163,5 +190,5 @@ extern "C" int holon_gemm_block_parts_splits(int M, int N, int K) {
 
 // parts [splits, M, N] (float32) = x[:, share s of K] w[:, share s of K]^T.
 extern "C" int holon_gemm_block_parts_bf16(const void* x, const void* w, void* parts, int M, int N, int K, int splits, void* stream) {
-  return launch_block(PARTS, x, w, parts, M, N, K, splits, stream);
+  return launch_block(PARTS, x, w, parts, M, N, K, splits, 0, stream);
 }

@@ -48,10 +48,10 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 def glu_block_pays(rows: int, inter: int, hidden: int) -> bool:
     """Whether a gated first product of many rows with its activation takes this package's 256 x 256 tiles (128 gates and their ups each):
     where the rounds of one tile a compute unit that it takes are filled to 0.62 and more (`hidden` does not enter: either side's time
-    is in proportion to it). Measured on MI355X, us, against the vendor
-    library's product and the kernel of the activation: 12,288 x 4,096 at 520 / 600 / 1,024 / 2,048 / 4,096 rows (filled 0.76 / 0.44 /
-    0.75 / 1 / 1) 101 / 160 / 169 / 280 / 551 and 124 / 124 / 176 / 307 / 596; 8,192 x 2,048 at 400 / 768 / 1,024 / 2,048 (0.39 / 0.75 / 1 / 1)
-    42 / 45 / 52 / 101 and 39 / 52 / 65 / 122; 9,728 x 2,560 at 1,024 / 1,500 (0.59 / 0.87) 119 / 122 and 114 / 142."""
+    is in proportion to it; tiles of 192 columns, taken where their rounds end sooner, make the line a cautious one). Measured on MI355X, us,
+    against the vendor library's product and the kernel of the activation: 12,288 x 4,096 at 520 / 600 / 1,024 / 2,048 / 4,096 rows (filled
+    0.76 / 0.44 / 0.75 / 1 / 1) 97 / 134 / 153 / 280 / 551 and 124 / 124 / 176 / 307 / 596; 8,192 x 2,048 at 400 / 768 / 1,024 / 2,048 (0.39 /
+    0.75 / 1 / 1) 34 / 45 / 52 / 101 and 39 / 52 / 65 / 122; 9,728 x 2,560 at 1,024 / 1,500 (0.59 / 0.87) 104 / 122 and 114 / 142."""
     high = rows // 256 if rows > 256 and 0 < rows % 256 <= 16 else -(-rows // 256)     # (a last tile takes up to 16 rows more)
     rounds = -(-high * -(-inter // 128) // 256)
     return rows > 128 and rows * inter >= 0.62 * rounds * 256 * 256 * 128
@@ -137,6 +137,7 @@ class HipKernels:
             "holon_gemm_block_parts_splits": [_I, _I, _I],
             "holon_gemm_block_parts_bf16": [_P, _P, _P, _I, _I, _I, _I, _P],
             "holon_gemm_block_glu_bf16": [_P, _P, _P, _I, _I, _I, _I, _P],
+            "holon_gemm_block_glu_width_bf16": [_P, _P, _P, _I, _I, _I, _I, _I, _P],
             "holon_sum_parts": [_P, _P, _I, _L, _P],
             "holon_rmsnorm_parts": [_P, _I, _P, _P, _P, _L, _I, _F, _P],
             "holon_gemm_skinny_scaled_bf16": [_P, _P, _P, _I, _I, _I, _I, _P, _I, _F, _P],

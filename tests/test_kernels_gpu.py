@@ -1671,3 +1671,18 @@ def test_products_in_one_launch_are_the_products(hip, rows, sizes):
     for p, got in zip(products, k.linear_group(products)):
         want = p.alone()
         assert got.dtype == want.dtype and torch.equal(got, want), (p.linear.weight.shape, p.dtype, p.relu2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("m,inter,k", [(1, 16, 128), (255, 96, 256), (256, 112, 128), (272, 192, 384), (273, 208, 256), (520, 400, 640)])
+def test_gated_tiles_of_both_widths(hip, act, m, inter, k):
+    """A gated first product on tiles of 96 gates and their ups is the one on tiles of 128, bit for bit: columns that end inside a tile,
+    at its end and in its first sixteen, rows up to 16 beyond the last tile's 256."""
+    x, w = _randn(m, k, dtype=torch.bfloat16, seed=190), _randn(2 * inter, k, dtype=torch.bfloat16, seed=191, scale=2 * k ** -0.5)
+    outs = []
+    for width in (128, 96):
+        y = torch.full((m + 1, inter), 7.0, dtype=torch.bfloat16, device="cuda")
+        hip._call(hip.lib.holon_gemm_block_glu_width_bf16, x.data_ptr(), w.data_ptr(), y.data_ptr(), m, inter, k, act, width, hip._stream())
+        outs.append(y)
+    assert torch.equal(outs[0], outs[1]) and (outs[1][m] == 7.0).all()

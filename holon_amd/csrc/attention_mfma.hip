@@ -1620,7 +1620,8 @@ struct NewKeyValue {
 // (waves 1.. leave theirs there, wave 0 adds them up); with one block a (row, kv head) the block writes the result
 // itself and no merge kernel follows.
 // SIG: sigmoid weights (see AttnArgs): the waves' partials are plain sums (their maxima stay 0, so the combination above
-// adds them as they are), one block a (row, kv head) writes the result, multiplied by the gate's sigmoid if one is given.
+// adds them as they are); with one block a (row, kv head) it writes the result, multiplied by the gate's sigmoid if one is
+// given, with more `sigmoid_merge_kernel` adds their sums in order.
 // MOD: changed scores (see AttnArgs); the wave that takes the row's first share also walks the kept first keys.
 template <int D, bool FUSED, bool SIG = false, bool MOD = false>
 __global__ void __launch_bounds__(512) attn_decode_kernel(AttnArgs a, FusedArgs f) {
@@ -1808,7 +1809,7 @@ __global__ void __launch_bounds__(512) attn_decode_kernel(AttnArgs a, FusedArgs 
       float* po = a.part_o + cell * D + 4 * g;
 #pragma unroll
       for (int ds = 0; ds < D / 16; ++ds) *reinterpret_cast<f32x4_t*>(po + ds * 16) = o[0][ds];
-      if (g == 0) { a.part_ml[cell * 2] = mt; a.part_ml[cell * 2 + 1] = lt; }
+      if (!SIG && g == 0) { a.part_ml[cell * 2] = mt; a.part_ml[cell * 2 + 1] = lt; }
     }
   }
   if constexpr (FUSED) {
@@ -1879,6 +1880,27 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict
     o.z = float_to_bf16(acc[2] * inv); o.w = float_to_bf16(acc[3] * inv);
     *reinterpret_cast<ushort4*>(out + ((int64_t)token * heads + h) * D + d0) = o;
   }
+}
+
+// Sigmoid weights: out[row, head, :] = the blocks' sums, added in order, times the gate's sigmoid if one is given.
+template <int D>
+__global__ void __launch_bounds__(D) sigmoid_merge_kernel(const float* __restrict__ part_o, bf16_t* __restrict__ out,
+                                                          const int32_t* __restrict__ row_ids, const int32_t* __restrict__ qstart,
+                                                          const bf16_t* __restrict__ gate, int heads, int splits) {
+  constexpr int AHEAD = 8;                 // sums asked for at a time
+  const int ri = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
+  const float* po = part_o + ((int64_t)ri * heads + h) * splits * D + d;
+  const int64_t at = ((int64_t)qstart[row_ids[ri]] * heads + h) * D + d;
+  float sum = 0.f;
+  for (int s0 = 0; s0 < splits; s0 += AHEAD) {
+    float v[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) v[i] = po[(int64_t)min(s0 + i, splits - 1) * D];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) sum += s0 + i < splits ? v[i] : 0.f;
+  }
+  if (gate != nullptr) sum *= 1.0f / (1.0f + __expf(-bf16_to_float(gate[at])));
+  out[at] = float_to_bf16(sum);
 }
 
 #ifndef PAIR_VALU_PER_MFMA
@@ -2103,35 +2125,46 @@ extern "C" int holon_sigmoid_attention_prefill_bf16(const void* q, void* out, co
   return 0;
 }
 
-// Decode rows of the same: one block a (row, kv head), the window's keys split over its waves (up to 8).
+// Decode rows of the same: the window's keys over `blocks` blocks a (row, kv head) and their waves (up to 8). With more than one, part_o
+// [n_rows, heads, blocks, D] takes their sums (float32), which a second kernel adds. What bounds a block is what its compute unit reads (16 KB
+// for every 32 keys at D = 128, about 42 KB a us), so a long window goes over several units; a short one not, as the second kernel takes 4 us.
 extern "C" int holon_sigmoid_attention_decode_bf16(const void* q, void* out, const void* pages, const int32_t* table,
                                                    int table_stride, const int32_t* slots, const int32_t* lens,
                                                    const int32_t* query_start, const int32_t* row_ids, int n_rows,
                                                    int max_len, int heads, int kv_heads, int head_dim, int page_size,
                                                    float scale, int window, const float* head_bias, const void* gate,
-                                                   int rows_in_order, void* stream) {
+                                                   int rows_in_order, int blocks, float* part_o, void* stream) {
   HOLON_CHECK((head_dim == 64 || head_dim == 128) && mfma_serves(head_dim, page_size),
               "sigmoid attention (matrix cores): head_dim %d / page %d not served", head_dim, page_size);
   HOLON_CHECK(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && window >= 0 && table_stride > 0 && max_len >= 0,
               "sigmoid attention: bad sizes");
   if (n_rows <= 0) return 0;
+  HOLON_CHECK(blocks == 1 || (blocks > 1 && blocks <= 64 && part_o != nullptr && (uintptr_t)part_o % 16 == 0),
+              "sigmoid attention: %d blocks a row without room for their sums", blocks);
   const int span = window > 0 ? (window < max_len ? window + 31 : max_len) : max_len;
-  int waves = (span + 127) / 128;                       // about 128 keys a wave
+  int waves = ((span + blocks - 1) / blocks + 31) / 32;      // 32 keys a wave, or more
   waves = waves < 1 ? 1 : (waves > 8 ? 8 : waves);
   AttnArgs a{};
   a.q = (const bf16_t*)q; a.out = (bf16_t*)out; a.pages = (const bf16_t*)pages; a.table = table;
   a.table_stride = table_stride; a.slots = slots; a.lens = lens; a.qstart = query_start; a.row_ids = row_ids;
   a.heads = heads; a.kv_heads = kv_heads; a.page_size = page_size; a.window = window;
   a.scale = scale; a.head_bias = head_bias; a.gate = (const bf16_t*)gate;
-  a.splits = waves; a.out_splits = 1; a.rows_in_order = rows_in_order;
+  a.splits = waves * blocks; a.out_splits = blocks; a.part_o = part_o; a.rows_in_order = rows_in_order;
   const TileMap tm = tile_map(heads / kv_heads);
-  dim3 grid(1, kv_heads * tm.head_blocks, n_rows);
+  dim3 grid(blocks, kv_heads * tm.head_blocks, n_rows);
   HOLON_CHECK(grid.y <= 65535 && grid.z <= 65535, "sigmoid attention: %d rows exceed one launch", n_rows);
   const size_t lds = (size_t)(waves - 1) * (16 * head_dim + 32) * sizeof(float);
   const FusedArgs none{};
   if (head_dim == 64) attn_decode_kernel<64, false, true><<<grid, waves * WAVE, lds, (hipStream_t)stream>>>(a, none);
   else attn_decode_kernel<128, false, true><<<grid, waves * WAVE, lds, (hipStream_t)stream>>>(a, none);
   HOLON_LAUNCH_OK();
+  if (blocks > 1) {
+    HOLON_CHECK(heads <= 65535, "sigmoid attention: %d heads exceed one launch", heads);
+    const dim3 cells(n_rows, heads);
+    if (head_dim == 64) sigmoid_merge_kernel<64><<<cells, 64, 0, (hipStream_t)stream>>>(part_o, a.out, row_ids, query_start, a.gate, heads, blocks);
+    else sigmoid_merge_kernel<128><<<cells, 128, 0, (hipStream_t)stream>>>(part_o, a.out, row_ids, query_start, a.gate, heads, blocks);
+    HOLON_LAUNCH_OK();
+  }
   return 0;
 }
 

@@ -145,6 +145,12 @@ def sigmoid_attention_plain(q, pages, table, rows, token_row, positions, kv_head
     return out.to(q.dtype)
 
 
+def decode_blocks(pairs: int, span: int) -> int:
+    """Blocks that share a decode row's keys (`pairs`: (row, kv head) tiles in the launch, `span` the most keys a row sees): one up to
+    256 keys, else one for every 128, up to a block a compute unit."""
+    return 1 if span <= 256 else max(1, min(64, -(-span // 128), 256 // max(1, pairs)))
+
+
 def _sigmoid_attention_hip(launch, q, pages, table, rows, token_row, positions, kv_heads, vdim, page_size, bias,
                            scale, window, gate):
     t, heads, dim = q.shape
@@ -169,9 +175,12 @@ def _sigmoid_attention_hip(launch, q, pages, table, rows, token_row, positions, 
                  rows.max_chunk_query, rows.max_chunk_len, heads, kv_heads, dim, page_size, float(scale), int(window),
                  _ptr(bias), _ptr(gate))
         if rows.n_decode:
+            span = min(rows.max_decode_len, window + 31) if window > 0 else rows.max_decode_len
+            blocks = decode_blocks(rows.n_decode * kv_heads * (-(-(heads // kv_heads) // 16)), span)
+            parts = torch.empty((rows.n_decode, heads, blocks, dim), dtype=torch.float32, device=q.device) if blocks > 1 else None
             narrow(*common, rows.lens.data_ptr(), rows.query_start.data_ptr(), rows.decode_rows.data_ptr(),
                    rows.n_decode, rows.max_decode_len, heads, kv_heads, dim, page_size, float(scale), int(window),
-                   _ptr(bias), _ptr(gate), int(rows.in_order and rows.n_decode == t))
+                   _ptr(bias), _ptr(gate), int(rows.in_order and rows.n_decode == t), blocks, _ptr(parts))
     else:
         general(*common, token_row.data_ptr(), positions.data_ptr(), None, None, t, *tail)
     return out
@@ -185,7 +194,7 @@ register_kernel(KernelOp("sigmoid_attention", sigmoid_attention_plain,
                           "holon_sigmoid_attention_decode_bf16"),
                          ([_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _F, _I, _P, _I],
                           [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
-                          [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I]),
+                          [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _P]),
                          _sigmoid_attention_hip))
 
 

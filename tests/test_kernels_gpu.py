@@ -1686,3 +1686,30 @@ def test_gated_tiles_of_both_widths(hip, act, m, inter, k):
         hip._call(hip.lib.holon_gemm_block_glu_width_bf16, x.data_ptr(), w.data_ptr(), y.data_ptr(), m, inter, k, act, width, hip._stream())
         outs.append(y)
     assert torch.equal(outs[0], outs[1]) and (outs[1][m] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,page", [(64, 16), (128, 32)])
+@pytest.mark.parametrize("window", [0, 40, 1024])
+def test_sigmoid_decode_rows_over_blocks(hip, dim, page, window):
+    """Sigmoid-weighted decode rows with their keys over one block and over several: float32 sums of up to 1,024 bfloat16 products in
+    another order, rounded once (2^-9)."""
+    from holon_amd.kernels.registry import kernel_op
+    from holon_amd.parts import sigmoid_attention as sa
+    heads, kv, lens = 4, 2, [1, 33, 256, 257, 700, 1300]
+    n, per = len(lens), -(-max(lens) // page)
+    pages = _randn(n * per + 1, kv * page * 2 * dim, dtype=torch.bfloat16, seed=192)
+    table = torch.arange(1, n * per + 1, dtype=torch.int32, device="cuda").view(n, per)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")          # noqa: E731
+    q, gate = _randn(n, heads, dim, dtype=torch.bfloat16, seed=193), _randn(n, heads * dim, dtype=torch.bfloat16, seed=194)
+    bias, order = _randn(heads, dtype=torch.float32, seed=195), i32(list(range(n)))
+    rows = AttnRows(slots=order, lens=i32(lens), query_start=i32(list(range(n + 1))), decode_rows=order, chunk_rows=i32([]), n_decode=n,
+                    n_chunk=0, max_decode_len=max(lens), max_chunk_query=0, max_chunk_len=0, in_order=True)
+    args = (q, pages, table, rows, order, i32([v - 1 for v in lens]), kv, dim, page, bias, dim ** -0.5, window, gate)
+    want, got = kernel_op("sigmoid_attention").plain(*args), []
+    for blocks in (1, 2, 11):
+        with pytest.MonkeyPatch.context() as m:
+            m.setattr(sa, "decode_blocks", lambda pairs, span: blocks)
+            got.append(hip.sigmoid_attention(*args))
+        assert H.rel_rms(got[-1], want) < 2.0 ** -8, blocks
+        assert H.rel_rms(got[-1], got[0]) < 2.0 ** -9, blocks

@@ -512,34 +512,80 @@ __global__ void shift_keep_kernel(const T* __restrict__ x, T* __restrict__ state
   state[(int64_t)slots[b] * width + c] = x[(int64_t)(query_start[b + 1] - 1) * width + c];
 }
 
-// exp(-exp(tanh(a) w2^T + w0)): a block takes 8 tokens and 256 channels; the tokens' tanh values are shared through
-// LDS, and w2 comes transposed ([rank, channels]) so that a wave's loads are contiguous and serve all 8 tokens.
-constexpr int LORA_TOKENS = 8, LORA_MAX_RANK = 1024;
-template <typename T>
+// exp(-exp(tanh(a) w2^T + w0)) on the float32 matrix cores, whose sums are the chain of multiply-adds in ascending order. A block takes 16
+// tokens and 256 channels, a wave 64 of them: lane l's four neighbouring channels are column l % 16 of four tiles, so that one load of w2
+// (transposed, [rank, channels]) serves them all. The tokens' tanh values lie in LDS. VEC: channels come in whole fours.
+// 2,048 tokens by 2,048 channels of rank 64 7 us and one token 4.4 (on the vector unit, a token's value read from LDS for every
+// multiply-add, 27 and 8.4).
+__host__ __device__ constexpr int lora_pitch(int rank) { return (rank + 3) / 4 * 4 + (rank < 1000 ? 1 : 0); }      // (at most 64 KB of LDS)
+constexpr int LORA_TOKENS = 16, LORA_MAX_RANK = 1024, LORA_AHEAD = 8;      // LORA_AHEAD: steps of four ranks whose weights are asked for at a time
+template <bool VEC, typename T>
 __global__ void __launch_bounds__(256) decay_lora_kernel(const float* __restrict__ a, const T* __restrict__ w2t,
                                                          const float* __restrict__ w0, float* __restrict__ y, int tokens,
                                                          int channels, int rank) {
-  __shared__ float th[LORA_TOKENS][LORA_MAX_RANK];
-  const int t0 = blockIdx.x * LORA_TOKENS;
-  const int c = blockIdx.y * 256 + threadIdx.x;
-  for (int e = threadIdx.x; e < LORA_TOKENS * rank; e += 256) {
-    const int tt = e / rank, r = e - tt * rank;
-    th[tt][r] = t0 + tt < tokens ? tanhf(a[(int64_t)(t0 + tt) * rank + r]) : 0.f;
+  extern __shared__ float th[];                            // [16][pitch], zeros behind the rank
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  const int steps = (rank + 3) / 4, pitch = lora_pitch(rank);
+  const int t0 = blockIdx.x * LORA_TOKENS, lane = threadIdx.x % WAVE, g = lane / 16, c = lane % 16;
+  const int c0 = blockIdx.y * 256 + threadIdx.x / WAVE * 64 + 4 * c;
+  T next[LORA_AHEAD][4];
+  const auto ask = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < LORA_AHEAD; ++u) {
+      const int64_t row = (int64_t)min(4 * (s0 + u) + g, rank - 1) * channels;
+      if constexpr (VEC) {
+        typedef T vec __attribute__((ext_vector_type(4)));
+        const vec v = *reinterpret_cast<const vec*>(w2t + row + min(c0, channels - 4));
+#pragma unroll
+        for (int n = 0; n < 4; ++n) next[u][n] = v[n];
+      } else {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) next[u][n] = w2t[row + min(c0 + n, channels - 1)];
+      }
+    }
+  };
+  ask(0);
+  for (int e = threadIdx.x; e < LORA_TOKENS * 4 * steps; e += 256) {
+    const int tt = e / (4 * steps), r = e - tt * 4 * steps;
+    th[tt * pitch + r] = t0 + tt < tokens && r < rank ? tanhf(a[(int64_t)(t0 + tt) * rank + r]) : 0.f;
   }
   __syncthreads();
-  if (c >= channels) return;
-  float acc[LORA_TOKENS];
+  f32x4 acc[4];
 #pragma unroll
-  for (int tt = 0; tt < LORA_TOKENS; ++tt) acc[tt] = 0.f;
-  for (int r = 0; r < rank; ++r) {
-    const float wv = Elem<T>::load(w2t[(int64_t)r * channels + c]);
+  for (int n = 0; n < 4; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < steps; s0 += LORA_AHEAD) {
+    float w[LORA_AHEAD][4];
 #pragma unroll
-    for (int tt = 0; tt < LORA_TOKENS; ++tt) acc[tt] += th[tt][r] * wv;
+    for (int u = 0; u < LORA_AHEAD; ++u)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) w[u][n] = 4 * (s0 + u) + g < rank ? Elem<T>::load(next[u][n]) : 0.f;
+    if (s0 + LORA_AHEAD < steps) ask(s0 + LORA_AHEAD);
+#pragma unroll
+    for (int u = 0; u < LORA_AHEAD; ++u) {
+      if (s0 + u >= steps) break;
+      const float x = th[c * pitch + 4 * (s0 + u) + g];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, w[u][n], acc[n], 0, 0, 0);
+    }
   }
-  const float off = w0[c];
+  float off[4];
 #pragma unroll
-  for (int tt = 0; tt < LORA_TOKENS; ++tt)
-    if (t0 + tt < tokens) y[(int64_t)(t0 + tt) * channels + c] = expf(-expf(acc[tt] + off));
+  for (int n = 0; n < 4; ++n) off[n] = w0[min(c0 + n, channels - 1)];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                            // lane: tokens 4 g + i of its four channels
+    const int t = t0 + 4 * g + i;
+    if (t >= tokens) continue;
+    f32x4 o;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) o[n] = expf(-expf(acc[n][i] + off[n]));
+    if constexpr (VEC) {
+      if (c0 < channels) *reinterpret_cast<f32x4*>(y + (int64_t)t * channels + c0) = o;
+    } else {
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        if (c0 + n < channels) y[(int64_t)t * channels + c0 + n] = o[n];
+    }
+  }
 }
 
 }  // namespace
@@ -743,8 +789,12 @@ extern "C" int holon_decay_lora(const float* a, const void* w2t, const float* w0
   if (tokens == 0) return 0;
   const dim3 grid((tokens + LORA_TOKENS - 1) / LORA_TOKENS, (channels + 255) / 256);
   HOLON_CHECK(grid.y <= 65535, "decay_lora: %d channels exceed one launch", channels);
-  BY_DTYPE(dtype, (decay_lora_kernel<T><<<grid, 256, 0, (hipStream_t)stream>>>(a, (const T*)w2t, w0, y, tokens, channels,
-                                                                               rank)));
+  const size_t lds = (size_t)LORA_TOKENS * lora_pitch(rank) * sizeof(float);
+  hipStream_t s = (hipStream_t)stream;
+  if (channels % 4 == 0 && (((uintptr_t)w2t | (uintptr_t)y) & 15) == 0)
+    BY_DTYPE(dtype, (decay_lora_kernel<true, T><<<grid, 256, lds, s>>>(a, (const T*)w2t, w0, y, tokens, channels, rank)));
+  else
+    BY_DTYPE(dtype, (decay_lora_kernel<false, T><<<grid, 256, lds, s>>>(a, (const T*)w2t, w0, y, tokens, channels, rank)));
   HOLON_LAUNCH_OK();
   return 0;
 }

@@ -1713,3 +1713,15 @@ def test_sigmoid_decode_rows_over_blocks(hip, dim, page, window):
             got.append(hip.sigmoid_attention(*args))
         assert H.rel_rms(got[-1], want) < 2.0 ** -8, blocks
         assert H.rel_rms(got[-1], got[0]) < 2.0 ** -9, blocks
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,channels,rank", [(1, 2048, 64), (17, 260, 5), (33, 70, 30), (16, 256, 1024), (5, 3, 1), (40, 516, 36)])
+def test_decay_projection(hip, dtype, tokens, channels, rank):
+    """exp(-exp(tanh(a) w2 + w0)) against float64: sums of up to 1,024 float32 terms of size one, so that their error is at most a few
+    times 2^-24 sqrt(rank) of the sum's size, which the two exponentials (slope at most 1 / e) do not enlarge."""
+    a, w2t = _randn(tokens, rank, dtype=torch.float32, seed=196), _randn(rank, channels, dtype=dtype, seed=197, scale=0.3 * rank ** -0.5)
+    w0 = _randn(channels, dtype=torch.float32, seed=198)
+    want = torch.exp(-torch.exp(torch.tanh(a.double()) @ w2t.double() + w0.double()))
+    assert (hip.decay_lora(a, w2t, w0).double() - want).abs().max() < 2e-6

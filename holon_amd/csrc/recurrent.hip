@@ -515,7 +515,7 @@ __global__ void shift_keep_kernel(const T* __restrict__ x, T* __restrict__ state
 // exp(-exp(tanh(a) w2^T + w0)) on the float32 matrix cores, whose sums are the chain of multiply-adds in ascending order. A block takes 16
 // tokens and 256 channels, a wave 64 of them: lane l's four neighbouring channels are column l % 16 of four tiles, so that one load of w2
 // (transposed, [rank, channels]) serves them all. The tokens' tanh values lie in LDS. VEC: channels come in whole fours.
-// 2,048 tokens by 2,048 channels of rank 64 7 us and one token 4.4 (on the vector unit, a token's value read from LDS for every
+// 2,048 tokens by 2,048 channels of rank 64 17 us and one token 4.9 (on the vector unit, a token's value read from LDS for every
 // multiply-add, 27 and 8.4).
 __host__ __device__ constexpr int lora_pitch(int rank) { return (rank + 3) / 4 * 4 + (rank < 1000 ? 1 : 0); }      // (at most 64 KB of LDS)
 constexpr int LORA_TOKENS = 16, LORA_MAX_RANK = 1024, LORA_AHEAD = 8;      // LORA_AHEAD: steps of four ranks whose weights are asked for at a time

@@ -49,16 +49,20 @@ struct AttnF64 {
   const float* r2;
   int v_share;
   int per;                         // tokens a block takes
+  double* part_o;                  // SPLIT: [tokens, heads, WAVES, dim] and [tokens, heads, WAVES, 2]
+  float* part_ml;
 };
 
-// DT: head_dim / 16. MOD: a cap or a distance bias on the scores.
-template <int DT, bool MOD>
-__global__ void __launch_bounds__(WAVES * WAVE, 2) attention_f64_kernel(AttnF64 a) {
+// DT: head_dim / 16. MOD: a cap or a distance bias on the scores. SPLIT: the block is wave blockIdx.z alone, and leaves what the waves
+// exchange at the end in memory for `attention_f64_merge_kernel`: a decode row's few blocks then fill more than a few compute units (one row
+// behind 700 tokens, 16 heads of 128 on 4: 45 us, split 23.1 + 4.6).
+template <int DT, bool MOD, bool SPLIT>
+__global__ void __launch_bounds__(SPLIT ? WAVE : WAVES * WAVE, SPLIT ? 1 : 2) attention_f64_kernel(AttnF64 a) {
   constexpr int D = DT * 16;
-  __shared__ double red[WAVES / 2][D][17];
+  __shared__ double red[SPLIT ? 1 : WAVES / 2][SPLIT ? 1 : D][17];
   __shared__ float ml_s[WAVES][16][2];
   __shared__ float den_s[16];
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, g = lane / 16, c = lane % 16;
+  const int w = SPLIT ? (int)blockIdx.z : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, g = lane / 16, c = lane % 16;
   const int group = a.heads / a.kv_heads, side = min(group, 16), blocks = (group + 15) / 16;      // columns a token takes
   const int hk = blockIdx.y / blocks, h_at = blockIdx.y % blocks * 16 + c % side;
   const int P = a.page_size;
@@ -209,6 +213,16 @@ __global__ void __launch_bounds__(WAVES * WAVE, 2) attention_f64_kernel(AttnF64 
     tile = next;
     page = next_page;
   }
+  if constexpr (SPLIT) {
+    if (!mine) return;
+    const int64_t cell = ((int64_t)t * a.heads + head) * WAVES + w;
+    if (g == 0) { a.part_ml[cell * 2] = m; a.part_ml[cell * 2 + 1] = l; }
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a.part_o[cell * D + d * 16 + 4 * r + g] = acc[d][r];
+    return;
+  }
   // the waves' sums, in one order: 0 + 4, 1 + 5, 2 + 6, 3 + 7, then those from the first on
   if (g == 0) { ml_s[w][c][0] = m; ml_s[w][c][1] = l; }
   __syncthreads();
@@ -219,7 +233,7 @@ __global__ void __launch_bounds__(WAVES * WAVE, 2) attention_f64_kernel(AttnF64 
   if (w == 0 && g == 0) {
     float den = 0.f;
 #pragma unroll
-    for (int i = 0; i < WAVES; ++i) den += ml_s[i][c][1] * share(ml_s[i][c][0]);
+    for (int i = 0; i < WAVES; ++i) den = fmaf(ml_s[i][c][1], share(ml_s[i][c][0]), den);
     if (a.sink && mine) den += expf(a.sink[head] - top);
     den_s[c] = den;
   }
@@ -228,14 +242,17 @@ __global__ void __launch_bounds__(WAVES * WAVE, 2) attention_f64_kernel(AttnF64 
 #pragma unroll
     for (int d = 0; d < DT; ++d)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[w][d * 16 + 4 * r + g][c] = acc[d][r] * f;
+      for (int r = 0; r < 4; ++r) red[w][d * 16 + 4 * r + g][c] = __dmul_rn(acc[d][r], f);
   }
   __syncthreads();
   if (w >= WAVES / 2) {
 #pragma unroll
     for (int d = 0; d < DT; ++d)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) red[w - WAVES / 2][d * 16 + 4 * r + g][c] += acc[d][r] * f;
+      for (int r = 0; r < 4; ++r) {
+        double& to = red[w - WAVES / 2][d * 16 + 4 * r + g][c];
+        to = fma(acc[d][r], f, to);
+      }
   }
   __syncthreads();
   const uint64_t to_write = __ballot(mine), with_keys = __ballot(live);       // (bit c: column c; the same in every wave)
@@ -251,6 +268,35 @@ __global__ void __launch_bounds__(WAVES * WAVE, 2) attention_f64_kernel(AttnF64 
         with_keys >> col & 1 ? y : 0.f;
   }
 }
+
+// What the waves of a block do at its end, from their sums in memory: the same operations in the same order.
+__global__ void __launch_bounds__(128) attention_f64_merge_kernel(AttnF64 a, int dim) {
+  const int t = blockIdx.x, head = blockIdx.y, d = threadIdx.x;
+  const int64_t cell = ((int64_t)t * a.heads + head) * WAVES;
+  float m[WAVES], l[WAVES];
+  double o[WAVES];
+#pragma unroll
+  for (int i = 0; i < WAVES; ++i) {
+    m[i] = a.part_ml[(cell + i) * 2];
+    l[i] = a.part_ml[(cell + i) * 2 + 1];
+    o[i] = a.part_o[(cell + i) * dim + d];
+  }
+  float top = a.sink ? a.sink[head] : -INFINITY;
+#pragma unroll
+  for (int i = 0; i < WAVES; ++i) top = fmaxf(top, m[i]);
+  float den = 0.f;
+  double sum = 0;
+#pragma unroll
+  for (int i = 0; i < WAVES; ++i) {
+    m[i] = m[i] == -INFINITY ? 0.f : expf(m[i] - top);
+    den = fmaf(l[i], m[i], den);
+  }
+  if (a.sink) den += expf(a.sink[head] - top);
+#pragma unroll
+  for (int i = 0; i < WAVES / 2; ++i) sum += fma(o[i + WAVES / 2], (double)m[i + WAVES / 2], __dmul_rn(o[i], (double)m[i]));
+  const float y = (float)(den > 0.f ? sum / (double)den : sum * 0.0);
+  a.out[((int64_t)t * a.heads + head) * dim + d] = a.positions[t] >= 0 ? y : 0.f;
+}
 }  // namespace
 
 extern "C" int holon_softmax_attention_f64_supported(int heads, int kv_heads, int dim, int vdim, int page_size) {
@@ -258,13 +304,12 @@ extern "C" int holon_softmax_attention_f64_supported(int heads, int kv_heads, in
          (int64_t)kv_heads * ((heads / kv_heads + 15) / 16) <= 65535;
 }
 
-// Arguments as holon_softmax_attention's; float32, no kept first tokens under a window.
-extern "C" int holon_softmax_attention_f64(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
+static int f64_launch(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
                                            int table_rows, const int32_t* slots, const int32_t* token_row,
                                            const int32_t* positions, int tokens, int heads, int kv_heads, int dim, int vdim,
                                            int page_size, int num_pages, const float* sink, float scale, int window, int dtype,
                                            float softcap, const float* r1, const float* r2, int keep_first, int v_share,
-                                           void* stream) {
+                                           double* part_o, float* part_ml, void* stream) {
   HOLON_CHECK(holon_softmax_attention_f64_supported(heads, kv_heads, dim, vdim, page_size) && dtype == HOLON_F32 &&
                   (uintptr_t)q % 16 == 0 && (uintptr_t)pages % 16 == 0,
               "softmax_attention (float64 sums): heads of %d / %d, pages of %d, type %d, or pointers that are not at 16 bytes", dim,
@@ -278,14 +323,49 @@ extern "C" int holon_softmax_attention_f64(const void* q, void* out, const void*
   HOLON_CHECK(tokens < 1 << 30, "softmax_attention: %d tokens exceed one launch", tokens);
   const int group = heads / kv_heads, side = group < 16 ? group : 16, per = 16 / side;
   const AttnF64 a{(const float*)q, (float*)out, (const float*)pages, table, table_stride, table_rows, slots, token_row, positions,
-                  tokens, heads, kv_heads, page_size, num_pages, scale, window, sink, softcap, r1, r2, v_share, per};
-  const dim3 grid(((tokens + per - 1) / per | 1) * per, kv_heads * ((group + 15) / 16));
+                  tokens, heads, kv_heads, page_size, num_pages, scale, window, sink, softcap, r1, r2, v_share, per, part_o, part_ml};
+  const bool split = part_o != nullptr;
+  const dim3 grid(((tokens + per - 1) / per | 1) * per, kv_heads * ((group + 15) / 16), split ? WAVES : 1);
   const bool mod = softcap > 0.f || r1 != nullptr;
   hipStream_t s = (hipStream_t)stream;
-  if (dim == 64 && !mod) attention_f64_kernel<4, false><<<grid, WAVES * WAVE, 0, s>>>(a);
-  else if (dim == 64) attention_f64_kernel<4, true><<<grid, WAVES * WAVE, 0, s>>>(a);
-  else if (!mod) attention_f64_kernel<8, false><<<grid, WAVES * WAVE, 0, s>>>(a);
-  else attention_f64_kernel<8, true><<<grid, WAVES * WAVE, 0, s>>>(a);
+#define F64(DT, MOD)                                                                   \
+  do {                                                                                 \
+    if (split) attention_f64_kernel<DT, MOD, true><<<grid, WAVE, 0, s>>>(a);           \
+    else attention_f64_kernel<DT, MOD, false><<<grid, WAVES * WAVE, 0, s>>>(a);        \
+  } while (0)
+  if (dim == 64 && !mod) F64(4, false);
+  else if (dim == 64) F64(4, true);
+  else if (!mod) F64(8, false);
+  else F64(8, true);
+#undef F64
   HOLON_LAUNCH_OK();
+  if (split) {
+    attention_f64_merge_kernel<<<dim3(tokens, heads), dim, 0, s>>>(a, dim);
+    HOLON_LAUNCH_OK();
+  }
   return 0;
+}
+
+// Arguments as holon_softmax_attention's; float32, no kept first tokens under a window.
+extern "C" int holon_softmax_attention_f64(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
+                                           int table_rows, const int32_t* slots, const int32_t* token_row,
+                                           const int32_t* positions, int tokens, int heads, int kv_heads, int dim, int vdim,
+                                           int page_size, int num_pages, const float* sink, float scale, int window, int dtype,
+                                           float softcap, const float* r1, const float* r2, int keep_first, int v_share,
+                                           void* stream) {
+  return f64_launch(q, out, pages, table, table_stride, table_rows, slots, token_row, positions, tokens, heads, kv_heads, dim, vdim,
+                    page_size, num_pages, sink, scale, window, dtype, softcap, r1, r2, keep_first, v_share, nullptr, nullptr, stream);
+}
+
+// The same bits with a block's eight waves in blocks of their own and a second kernel behind them: part_o [tokens, heads, 8, dim] float64,
+// part_ml [tokens, heads, 8, 2] float32.
+extern "C" int holon_softmax_attention_f64_split(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
+                                                 int table_rows, const int32_t* slots, const int32_t* token_row,
+                                                 const int32_t* positions, int tokens, int heads, int kv_heads, int dim, int vdim,
+                                                 int page_size, int num_pages, const float* sink, float scale, int window, int dtype,
+                                                 float softcap, const float* r1, const float* r2, int keep_first, int v_share,
+                                                 double* part_o, float* part_ml, void* stream) {
+  HOLON_CHECK(part_o != nullptr && part_ml != nullptr && heads <= 65535, "softmax_attention (float64 sums): no room for the waves' sums");
+  return f64_launch(q, out, pages, table, table_stride, table_rows, slots, token_row, positions, tokens, heads, kv_heads, dim, vdim,
+                    page_size, num_pages, sink, scale, window, dtype, softcap, r1, r2, keep_first, v_share, part_o, part_ml, stream);
 }

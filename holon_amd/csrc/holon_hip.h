@@ -42,6 +42,11 @@ int holon_attention_generic(const void* q, void* out, const void* pages, const i
                             const int32_t* slots, const int32_t* lens, const int32_t* query_start, int rows,
                             int tokens, int heads, int kv_heads, int head_dim, int page_size, int num_pages,
                             float scale, int window, int most, int dtype, void* stream);
+// The same bits, every wave a block (part [tokens, heads, 8, head_dim], float64 for float32 operands; part_ml [tokens, heads, 8, 2]).
+int holon_attention_generic_split(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
+                            const int32_t* slots, const int32_t* lens, const int32_t* query_start, int rows,
+                            int tokens, int heads, int kv_heads, int head_dim, int page_size, int num_pages,
+                            float scale, int window, int most, int dtype, void* part, float* part_ml, void* stream);
 // Matrix-core attention (bfloat16, head_dim 64/128/256, page_size % 16 == 0). `row_ids` lists the rows served.
 int holon_attention_mfma_supported(int head_dim, int page_size, int dtype);
 int holon_attention_prefill_bf16(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
@@ -336,6 +341,13 @@ int holon_softmax_attention_f64(const void* q, void* out, const void* pages, con
                                 int tokens, int heads, int kv_heads, int dim, int vdim, int page_size, int num_pages,
                                 const float* sink, float scale, int window, int dtype, float softcap, const float* r1,
                                 const float* r2, int keep_first, int v_share, void* stream);
+// The same bits, every wave a block (part_o [tokens, heads, 8, dim] float64, part_ml [tokens, heads, 8, 2] float32).
+int holon_softmax_attention_f64_split(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
+                                int table_rows, const int32_t* slots, const int32_t* token_row, const int32_t* positions,
+                                int tokens, int heads, int kv_heads, int dim, int vdim, int page_size, int num_pages,
+                                const float* sink, float scale, int window, int dtype, float softcap, const float* r1,
+                                const float* r2, int keep_first, int v_share, double* part_o, float* part_ml,
+                                void* stream);
 // x [T, H V] *= sigmoid(gates[t, h]) per head (gates: columns of rows gate_stride apart); x [rows, dim] += bias;
 // y [T, 2 H V] (kv head, map, head in group) -> out [T, H V]: u = y1 - lam y2, u / sqrt(mean(u^2) + eps) * gain.
 int holon_head_gate(void* x, const void* gates, int64_t gate_stride, int64_t tokens, int heads, int vdim, int dtype,

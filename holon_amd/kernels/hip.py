@@ -95,6 +95,7 @@ class HipKernels:
                                          _I, _P],
             "holon_kv_write": [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P],
             "holon_attention_generic": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P],
+            "holon_attention_generic_split": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _P, _P],
             "holon_attention_mfma_supported": [_I, _I, _I],
             "holon_attention_prefill_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
                                              _P],
@@ -793,10 +794,17 @@ class HipKernels:
         if sink is not None:
             raise KernelError("attention: a sink is served by the matrix-core kernels (and by `softmax_attention`), "
                               f"not at head_dim {d}, page {page_size}, {q.dtype}")
-        self._call(self.lib.holon_attention_generic, q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(),
+        general, parts = self.lib.holon_attention_generic, ()
+        span = min(rows.max_decode_len, abs(window)) if window else rows.max_decode_len
+        if rows.n_chunk == 0 and t * hkv <= 64 and span > 128:      # decode rows that leave compute units idle: a wave a block
+            f64 = torch.float64 if q.dtype == torch.float32 else torch.float32
+            general, parts = self.lib.holon_attention_generic_split, (
+                torch.empty((t, hq, 8, d), dtype=f64, device=q.device), torch.empty((t, hq, 8, 2), dtype=torch.float32, device=q.device))
+        self._call(general, q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(),
                    table.shape[1], rows.slots.data_ptr(), rows.lens.data_ptr(), rows.query_start.data_ptr(), b, t, hq,
                    hkv, d, page_size, pages.shape[0], float(scale), int(window),
-                   max(rows.max_decode_len, rows.max_chunk_len), self._dt(q, "attention"), self._stream())
+                   max(rows.max_decode_len, rows.max_chunk_len), self._dt(q, "attention"), *(p.data_ptr() for p in parts),
+                   self._stream())
         return out
 
     def _shared_attention(self, q, pages, table, rows, page_size, scale, window, sink, softcap, dist, keep_first, share,

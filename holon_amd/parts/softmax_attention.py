@@ -84,6 +84,13 @@ def _float64_sums_serve(heads, kv_heads, dim, vdim, page_size):
         and kv_heads * -(-(heads // kv_heads) // 16) <= 65535
 
 
+def f64_split_pays(blocks: int, longest: int, window: int) -> bool:
+    """Whether a step of decode rows alone, in `blocks` blocks of eight waves over up to `longest` keys, has every wave in a block of its
+    own (the same bits): where the blocks leave compute units idle and a wave has more than a tile or two (one row behind 700 tokens 28 us
+    in place of 45; behind 150 a block takes 16 and the second kernel alone 4.6)."""
+    return blocks <= 128 and (min(longest, abs(window)) if window else longest) > 256
+
+
 def _softmax_attention_hip(launch, q, pages, table, rows, token_row, positions, kv_heads, vdim, page_size, sink,
                            scale, window, softcap=0.0, dist=None, keep_first=0, value_share=1):
     t, heads, dim = q.shape
@@ -100,15 +107,19 @@ def _softmax_attention_hip(launch, q, pages, table, rows, token_row, positions, 
         raise ValueError(f"softmax_attention: q {tuple(q.shape)} {q.dtype}, pages {tuple(pages.shape)} do not fit "
                          f"{kv_heads} kv heads, values of {vdim}, page {page_size}")
     out = torch.empty((t, heads * vdim), dtype=q.dtype, device=q.device)
-    general, wide = launch
+    general, wide, split = launch
     kernel = wide if q.dtype == torch.float32 and not (window > 0 and keep_first > 0) \
         and _float64_sums_serve(heads, kv_heads, dim, vdim, page_size) and q.data_ptr() % 16 == 0 and pages.data_ptr() % 16 == 0 \
         else general
+    parts = ()
+    if kernel is wide and rows.n_chunk == 0 and f64_split_pays(t * kv_heads * -(-(heads // kv_heads) // 16), rows.max_decode_len, window):
+        kernel, parts = split, (torch.empty((t, heads, 8, dim), dtype=torch.float64, device=q.device),
+                                torch.empty((t, heads, 8, 2), dtype=torch.float32, device=q.device))
     kernel(q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), table.shape[1], table.shape[0],
            rows.slots.data_ptr(), token_row.data_ptr(), positions.data_ptr(), t, heads, kv_heads, dim, vdim, page_size,
            pages.shape[0], _ptr(sink), float(scale), int(window), _DT[q.dtype], float(softcap),
            _ptr(dist[0]) if dist is not None else None, _ptr(dist[1]) if dist is not None else None, int(keep_first),
-           int(value_share))
+           int(value_share), *(p.data_ptr() for p in parts))
     return out
 
 
@@ -401,8 +412,9 @@ def _add_bias_hip(launch, x, bias):
 
 
 _SOFTMAX = [_P, _P, _P, _P, _I, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _F, _I, _I, _F, _P, _P, _I, _I]
-register_kernel(KernelOp("softmax_attention", softmax_attention_plain, ("holon_softmax_attention", "holon_softmax_attention_f64"),
-                         (_SOFTMAX, _SOFTMAX), _softmax_attention_hip))
+register_kernel(KernelOp("softmax_attention", softmax_attention_plain,
+                         ("holon_softmax_attention", "holon_softmax_attention_f64", "holon_softmax_attention_f64_split"),
+                         (_SOFTMAX, _SOFTMAX, [*_SOFTMAX, _P, _P]), _softmax_attention_hip))
 register_kernel(KernelOp("head_linear", head_linear_plain, ("holon_head_linear_rows", "holon_head_linear_bf16"),
                          ([_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _L], [_P, _P, _P, _I, _I, _I, _I, _I, _P, _L]),
                          _head_linear_hip))

@@ -1725,3 +1725,53 @@ def test_decay_projection(hip, dtype, tokens, channels, rank):
     w0 = _randn(channels, dtype=torch.float32, seed=198)
     want = torch.exp(-torch.exp(torch.tanh(a.double()) @ w2t.double() + w0.double()))
     assert (hip.decay_lora(a, w2t, w0).double() - want).abs().max() < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv,dim,page", [(8, 2, 128, 16), (3, 3, 72, 5), (2, 1, 512, 8)])
+@pytest.mark.parametrize("window", [0, 300, -128])
+def test_decode_rows_a_wave_a_block_are_the_same_bits(hip, dtype, heads, kv, dim, page, window):
+    """The general attention kernel's waves in blocks of their own against the whole block: rows of one key, of a tile and one more, of more
+    tiles than waves, and a row of no keys."""
+    lens = [1, 64, 65, 0, 513, 1100]
+    n, per = len(lens), -(-max(lens) // page)
+    pages = _randn(n * per, 2, kv, page * dim, dtype=dtype, seed=199)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")          # noqa: E731
+    table, slots, at = torch.arange(n * per, dtype=torch.int32, device="cuda").view(n, per), i32(list(range(n))), i32(list(range(n + 1)))
+    q, outs = _randn(n, heads, dim, dtype=dtype, seed=200), []
+    parts = (torch.full((n, heads, 8, dim), float("nan"), dtype=torch.float64 if dtype == torch.float32 else torch.float32, device="cuda"),
+             torch.full((n, heads, 8, 2), float("nan"), dtype=torch.float32, device="cuda"))
+    for split in (False, True):
+        out = torch.full_like(q, 7.0)
+        args = (q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), per, slots.data_ptr(), i32(lens).data_ptr(), at.data_ptr(),
+                n, n, heads, kv, dim, page, n * per, dim ** -0.5, window, max(lens), int(dtype == torch.bfloat16))
+        if split:
+            hip._call(hip.lib.holon_attention_generic_split, *args, *(p.data_ptr() for p in parts), hip._stream())
+        else:
+            hip._call(hip.lib.holon_attention_generic, *args, hip._stream())
+        outs.append(out)
+    assert torch.equal(*outs) and not outs[1][3].any() and outs[1].isfinite().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv,dim", [(16, 4, 128), (4, 4, 64), (40, 2, 64)])
+@pytest.mark.parametrize("window,sunk,cap", [(0, False, 0.0), (300, True, 3.0), (-128, True, 0.0)])
+def test_float64_decode_rows_a_wave_a_block_are_the_same_bits(hip, heads, kv, dim, window, sunk, cap, monkeypatch):
+    """The same of softmax attention on the float64 matrix cores, a row on the padding slot (position -1) among them."""
+    from holon_amd.parts import softmax_attention as sa
+    page, lens = 16, [1, 16, 17, 0, 129, 700]
+    n, per = len(lens), 48
+    pages = _randn(n * per, 2 * kv * page * dim, dtype=torch.float32, seed=201)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")          # noqa: E731
+    table, order = torch.arange(n * per, dtype=torch.int32, device="cuda").view(n, per), i32(list(range(n)))
+    rows = AttnRows(slots=order, lens=i32(lens), query_start=i32(list(range(n + 1))), decode_rows=order, chunk_rows=i32([]), n_decode=n,
+                    n_chunk=0, max_decode_len=max(lens), max_chunk_query=0, max_chunk_len=0, in_order=True)
+    q = _randn(n, heads, dim, dtype=torch.float32, seed=202)
+    sink = _randn(heads, dtype=torch.float32, seed=203) if sunk else None
+    outs = []
+    for split in (False, True):
+        monkeypatch.setattr(sa, "f64_split_pays", lambda *a, split=split: split)
+        outs.append(hip.softmax_attention(q, pages, table, rows, order, i32([v - 1 for v in lens]), kv, dim, page, sink, dim ** -0.5, window,
+                                          softcap=cap))
+    assert torch.equal(*outs) and not outs[1][3].any() and outs[1].isfinite().all()

@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "holon_hip.h"
+#include "moe_router.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -422,15 +423,40 @@ struct GroupItems {
   GroupItem at[GROUP_MOST];
   int count, M;
 };
+// A mixture's router over the same number of rows, a block a row in front of the products' blocks: by itself it is one wave's chain of
+// choices behind the logits' round of memory latency, 4.8 to 6.1 us in which nothing else runs.
+struct GroupRoute {
+  const bf16_t* x;
+  const float* router;
+  const float* bias;
+  float* weights;
+  int width, experts, rows_r, top, groups, keep, score;
+  float scale;
+};
 
-template <bool SHORT, bool REST>
-__global__ void __launch_bounds__(GROUP_WAVES * 64, SHORT ? 8 : 4) gemm_skinny_group_kernel(GroupItems items) {
+template <bool SHORT, bool REST, bool ROUTE>
+__global__ void __launch_bounds__(GROUP_WAVES * 64, SHORT && !ROUTE ? 8 : 4) gemm_skinny_group_kernel(GroupItems items, GroupRoute route) {
   __shared__ f32x4_t red[GROUP_WAVES * WAVE];
+  int block = blockIdx.x;
+  if constexpr (ROUTE) {
+    static_assert(moe_router::BLOCK_WAVES == GROUP_WAVES && sizeof(moe_router::Lds) <= sizeof(red), "the router's block");
+    if (block < items.M) {
+      moe_router::Lds& lds = *reinterpret_cast<moe_router::Lds*>(red);
+      if (route.score < 0)
+        moe_router::few_token<bf16_t, 1>(lds, block, route.x, route.router, route.bias, route.weights, route.width, route.experts,
+                                         route.rows_r, route.top, route.groups, route.keep, route.score, route.scale);
+      else
+        moe_router::few_token<bf16_t, 4>(lds, block, route.x, route.router, route.bias, route.weights, route.width, route.experts,
+                                         route.rows_r, route.top, route.groups, route.keep, route.score, route.scale);
+      return;
+    }
+    block -= items.M;
+  }
   const int all = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, g = lane / 16, c = lane % 16;
   int n = 0;
-  while (n + 1 < items.count && (int)blockIdx.x >= items.at[n + 1].first) ++n;
+  while (n + 1 < items.count && block >= items.at[n + 1].first) ++n;
   const GroupItem it = items.at[n];
-  const int wave = all % it.waves, tile = ((int)blockIdx.x - it.first) * (GROUP_WAVES / it.waves) + all / it.waves;
+  const int wave = all % it.waves, tile = (block - it.first) * (GROUP_WAVES / it.waves) + all / it.waves;
   const bool have = c < items.M, mine = tile < it.N / 16;
   const int steps = mine ? it.K / 32 / it.waves : 0;
   f32x4_t acc[1] = {{0.f, 0.f, 0.f, 0.f}};
@@ -487,8 +513,10 @@ __global__ void __launch_bounds__(GROUP_WAVES * 64, SHORT ? 8 : 4) gemm_skinny_g
 }
 
 // `items`: `count` (up to 8) of 3 pointers (x [M, K], w tiled, y [M, N]) and 3 sizes (N, K, form: 0 bfloat16, 2 float32 values that were
-// rounded to bfloat16 first, 4 bfloat16 max(product, 0)^2).
-extern "C" int holon_gemm_skinny_group_bf16(const int64_t* items, int count, int M, void* stream) {
+// rounded to bfloat16 first, 4 bfloat16 max(product, 0)^2). `route` (nullable): 4 pointers (x [M, width], router [rows, width], bias or 0,
+// weights [M, rows]) and 7 numbers (width, experts, rows, top, groups, keep, score) of a router as holon_moe_router (score -1) and
+// holon_moe_router_top have them, of up to 64 experts.
+extern "C" int holon_gemm_skinny_group_bf16(const int64_t* items, int count, int M, const int64_t* route, float scale, void* stream) {
   HOLON_CHECK(count >= 1 && count <= GROUP_MOST && M >= 1 && M <= 16, "gemm (few rows, several): %d products of %d rows", count, M);
   GroupItems g{};
   g.count = count;
@@ -515,9 +543,27 @@ extern "C" int holon_gemm_skinny_group_bf16(const int64_t* items, int count, int
     rest = rest || steps % 4 != 0;
   }
   hipStream_t s = (hipStream_t)stream;
-  if (is_short) gemm_skinny_group_kernel<true, false><<<blocks, GROUP_WAVES * 64, 0, s>>>(g);
-  else if (rest) gemm_skinny_group_kernel<false, true><<<blocks, GROUP_WAVES * 64, 0, s>>>(g);
-  else gemm_skinny_group_kernel<false, false><<<blocks, GROUP_WAVES * 64, 0, s>>>(g);
+  GroupRoute r{};
+  if (route != nullptr) {
+    r = {(const bf16_t*)route[0], (const float*)route[1], (const float*)route[2], (float*)route[3], (int)route[4], (int)route[5], (int)route[6],
+         (int)route[7], (int)route[8], (int)route[9], (int)route[10], scale};
+    HOLON_CHECK(r.x && r.router && r.weights && r.width >= 1 && r.width <= 12288 && r.experts >= 1 && r.experts <= WAVE && r.top >= 1 &&
+                    r.top <= r.experts && (r.rows_r == r.experts || (r.score >= 0 && r.rows_r == r.experts + 1)) && r.score >= -1 && r.score <= 2 &&
+                    (r.groups <= 1 || (r.experts % r.groups == 0 && r.keep >= 1 && r.keep <= r.groups &&
+                                       (r.score < 0 || r.top <= r.keep * (r.experts / r.groups)))),
+                "gemm (few rows, several): a router of width %d, top %d of %d experts, %d rows, %d of %d groups, score %d not served", r.width,
+                r.top, r.experts, r.rows_r, r.keep, r.groups, r.score);
+    blocks += M;
+  }
+#define GROUP(SHORT, REST)                                                                                       \
+  do {                                                                                                           \
+    if (route != nullptr) gemm_skinny_group_kernel<SHORT, REST, true><<<blocks, GROUP_WAVES * 64, 0, s>>>(g, r); \
+    else gemm_skinny_group_kernel<SHORT, REST, false><<<blocks, GROUP_WAVES * 64, 0, s>>>(g, r);                 \
+  } while (0)
+  if (is_short) GROUP(true, false);
+  else if (rest) GROUP(false, true);
+  else GROUP(false, false);
+#undef GROUP
   HOLON_LAUNCH_OK();
   return 0;
 }

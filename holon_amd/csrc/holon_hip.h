@@ -167,7 +167,7 @@ int holon_gemm_skinny_glu_bf16(const void* x, const void* w, void* y, int M, int
                                int parts, float eps, void* stream);
 int holon_gemm_skinny_geglu_bf16(const void* x, const void* w, void* y, int M, int I, int K, int tiled, void* stream);
 // Several such products of the same rows in one launch, each bit for bit as by itself (see gemm_skinny.hip for `items`).
-int holon_gemm_skinny_group_bf16(const int64_t* items, int count, int M, void* stream);
+int holon_gemm_skinny_group_bf16(const int64_t* items, int count, int M, const int64_t* route, float scale, void* stream);
 // The same products for 17 <= M <= 64 rows over tiled weights with many tiles (N / 16 a multiple of 8 and at least
 // 1,024; K a multiple of 256): the rows of activations go through LDS, shared by a block's waves, and every wave sums
 // its tile over all of K in order. `gated`: N is I and the weight has 2 I rows.

@@ -12,7 +12,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, Stream
 from .linear import Linear
 from .norms import Normed
-from .products import Product, drive
+from .products import Product, Routing, drive
 
 
 @register_part("ffn", "swiglu")
@@ -659,15 +659,16 @@ class MoE(Part):
         self.gate_up = self.attach("gate_up", gate_up)
         self.all_down = self.attach("all_down", down)
 
-    def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
+    def products(self, x: torch.Tensor, step=None):
         k = self.kernels
         if self.score != "sigmoid":
-            how = {} if self.score == "softmax_top" else {"score": "sigmoid_squared" if self.weigh_input else "sigmoid"}
-            weights = k.moe_router_top(x, self.router, self.router_bias if self.has_bias else None, self.experts,
-                                       self.top, self.groups, self.keep, **how)
+            score = "softmax" if self.score == "softmax_top" else "sigmoid_squared" if self.weigh_input else "sigmoid"
+            route = Routing(k, x, self.router, self.router_bias if self.has_bias else None, self.experts, self.top, self.groups, self.keep,
+                            score)
         else:
-            weights = k.moe_router(x, self.router, self.correction if self.has_bias else None, self.top, self.groups,
-                                   self.keep, self.scale)
+            route = Routing(k, x, self.router, self.correction if self.has_bias else None, self.experts, self.top, self.groups, self.keep,
+                            scale=self.scale)
+        weights, = yield [route]
         up, down = self.gate_up, self.all_down
         if x.dtype == torch.float32 and moe_f32_takes(x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top):
             y = k.moe_f32(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",
@@ -687,6 +688,9 @@ class MoE(Part):
                 return y
         between = k.moe_relu2 if self.act == "relu2" else k.moe_gate
         return down(between(up(x), weights, self.inter, self.shared, shared_weight=self.shared_gated))
+
+    def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
+        return drive(self.kernels, x.shape[0], self.products(x, step))[0]
 
     def _own_rows(self, rows: int) -> bool:
         """Whether the engine's product choices leave a step of many rows to `moe_rows`: pins of either product over all experts keep

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
+from typing import Any
 
 import torch
 
@@ -36,6 +37,38 @@ class Product:
             return linear(self.x, self.dtype)
         y = k.linear_relu2(self.x, linear.weight, linear.tiled if linear.folded is None else None)
         return k.relu2(linear(self.x)) if y is None else y
+
+
+@dataclasses.dataclass
+class Routing:
+    """A mixture's router (`moe_router_top`, or with `scale` set `moe_router`): which experts each row of x takes, and their weights."""
+
+    kernels: Any
+    x: torch.Tensor
+    router: torch.Tensor
+    bias: torch.Tensor | None
+    experts: int
+    top: int
+    groups: int
+    keep: int
+    score: str = "softmax"
+    scale: float | None = None
+
+    def alone(self) -> torch.Tensor:
+        if self.scale is not None:
+            return self.kernels.moe_router(self.x, self.router, self.bias, self.top, self.groups, self.keep, self.scale)
+        how = {} if self.score == "softmax" else {"score": self.score}
+        return self.kernels.moe_router_top(self.x, self.router, self.bias, self.experts, self.top, self.groups, self.keep, **how)
+
+    def served(self) -> bool:
+        """Whether a launch of products takes it along: what the operation by itself would accept, at few rows and experts."""
+        x, r, e = self.x, self.router, self.experts
+        return (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.is_contiguous() and 1 <= x.shape[0] <= FEW_ROWS
+                and r.dtype == torch.float32 and r.is_contiguous() and r.dim() == 2 and r.shape[1] == x.shape[1] <= 12288
+                and r.shape[0] in ((e,) if self.scale is not None else (e, e + 1)) and 1 <= self.top <= e <= 64
+                and (self.bias is None or (self.bias.dtype == torch.float32 and self.bias.is_contiguous() and self.bias.shape == (e,)))
+                and (self.groups <= 1 or (e % self.groups == 0 and 1 <= self.keep <= self.groups
+                                          and (self.scale is not None or self.top <= self.keep * (e // self.groups)))))
 
 
 def products_of(part, *args, **kwargs):
@@ -81,8 +114,8 @@ def _by_itself(part):
             return end.value
 
 
-def linear_group_plain(products: list[Product]) -> list[torch.Tensor]:
-    """The results of products that do not read one another's, in order; each with the roundings it has alone."""
+def linear_group_plain(products: list[Product | Routing]) -> list[torch.Tensor]:
+    """The results of products (and a mixture's routing) that do not read one another's, in order; each with the roundings it has alone."""
     return [p.alone() for p in products]
 
 
@@ -95,15 +128,23 @@ def _served(p: Product) -> bool:
             and x.data_ptr() % 16 == 0 and p.dtype in (None, torch.bfloat16, torch.float32) and not (p.relu2 and p.dtype == torch.float32))
 
 
-def _linear_group_hip(launch, products: list[Product]) -> list[torch.Tensor]:
+SCORES = {"softmax": 0, "sigmoid": 1, "sigmoid_squared": 2}
+
+
+def _linear_group_hip(launch, products: list[Product | Routing]) -> list[torch.Tensor]:
     out: list = [None] * len(products)
     by_rows: dict[int, list[int]] = {}
+    routes: dict[int, list[int]] = {}
     for i, p in enumerate(products):
-        if _served(p):
+        if isinstance(p, Routing):
+            if p.served():
+                routes.setdefault(p.x.shape[0], []).append(i)
+        elif _served(p):
             by_rows.setdefault(p.x.shape[0], []).append(i)
     for rows, which in by_rows.items():
         for group in (which[at: at + MOST] for at in range(0, len(which), MOST)):
-            if len(group) == 1:
+            route = routes[rows].pop(0) if routes.get(rows) else None
+            if len(group) == 1 and route is None:
                 continue
             items = []
             for i in group:
@@ -112,9 +153,16 @@ def _linear_group_hip(launch, products: list[Product]) -> list[torch.Tensor]:
                 n, k = p.linear.weight.shape
                 out[i] = torch.empty((rows, n), dtype=torch.float32 if form == 2 else torch.bfloat16, device=p.x.device)
                 items += [p.x.data_ptr(), p.linear.tiled.data_ptr(), out[i].data_ptr(), n, k, form]
-            launch((ctypes.c_int64 * len(items))(*items), len(group), rows)
+            with_it, scale = None, 0.0
+            if route is not None:
+                p = products[route]
+                out[route] = torch.empty((rows, p.router.shape[0]), dtype=torch.float32, device=p.x.device)
+                score, scale = (SCORES[p.score], 0.0) if p.scale is None else (-1, float(p.scale))
+                with_it = (ctypes.c_int64 * 11)(p.x.data_ptr(), p.router.data_ptr(), 0 if p.bias is None else p.bias.data_ptr(),
+                                                out[route].data_ptr(), p.x.shape[1], p.experts, p.router.shape[0], p.top, p.groups, p.keep, score)
+            launch((ctypes.c_int64 * len(items))(*items), len(group), rows, with_it, scale)
     return [y if y is not None else p.alone() for y, p in zip(out, products)]
 
 
 register_kernel(KernelOp("linear_group", linear_group_plain, "holon_gemm_skinny_group_bf16",
-                         [ctypes.c_void_p, ctypes.c_int, ctypes.c_int], _linear_group_hip))
+                         [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_float], _linear_group_hip))

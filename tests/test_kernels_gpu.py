@@ -1775,3 +1775,29 @@ def test_float64_decode_rows_a_wave_a_block_are_the_same_bits(hip, heads, kv, di
         outs.append(hip.softmax_attention(q, pages, table, rows, order, i32([v - 1 for v in lens]), kv, dim, page, sink, dim ** -0.5, window,
                                           softcap=cap))
     assert torch.equal(*outs) and not outs[1][3].any() and outs[1].isfinite().all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 3, 16])
+@pytest.mark.parametrize("experts,extra,groups,how", [(8, 0, 4, {"scale": 2.5}), (8, 1, 1, {}), (64, 0, 8, {"score": "sigmoid"}),
+                                                      (5, 1, 1, {"score": "sigmoid_squared"})])
+def test_a_router_beside_products_is_the_router(hip, rows, experts, extra, groups, how):
+    """A mixture's routing in a launch of products, bit for bit the operation by itself, and the products what they are."""
+    from holon_amd.parts.products import Product, Routing
+    width = 640
+
+    class Weights:
+        folded, kernels = None, hip
+        weight = _randn(528, width, dtype=torch.bfloat16, seed=204, scale=0.05)
+        tiled = hip.tile_weight(weight)
+
+        def __call__(self, x, dtype=None):
+            return hip.linear(x, self.weight, dtype, self.tiled)
+    x = _randn(rows, width, dtype=torch.bfloat16, seed=205)
+    router = _randn(experts + extra, width, dtype=torch.float32, seed=206, scale=0.1)
+    bias = _randn(experts, dtype=torch.float32, seed=207)
+    routing = Routing(hip, x, router, bias, experts, 2, groups, max(1, groups // 2), **how)
+    products = [Product(Weights(), x), routing, Product(Weights(), x, torch.float32)]
+    for p, got in zip(products, hip.linear_group(products)):
+        assert torch.equal(got, p.alone())
+    assert torch.equal(hip.linear_group([routing])[0], routing.alone())

@@ -29,6 +29,8 @@ KINDS: dict[str, tuple[str, tuple[str, ...]]] = {
     "parts": ("parts", ("parts", "vendor")),      # a narrow weight, K in shares: 17 to 128 rows; to 1,024 where K is well above N
     "experts": ("own", ("own", "vendor")),        # a mixture's products, each expert over its own rows (17 and more; by its first weight's
                                                   # shape, never timed), or all rows over all experts, as the kinds above have it
+    "group": ("own", ("own", "vendor")),          # four products of one size and 129 rows and more in one launch (by the first weight's
+                                                  # shape, never timed), or each by itself
     "vendor": ("bf16", ("bf16", "f32", "f32x2")),  # the vendor product's own forms (result type, K in halves)
 }
 

@@ -1,6 +1,6 @@
 // Products of many rows (prompts) over untiled weights on 256 x 256 tiles (gemm_block.h), bfloat16 with float32 sums: a gated
-// feed-forward's first product with the activation in its epilogue, and products whose K is cut into shares over the grid, the shares
-// added up by whoever reads them.
+// feed-forward's first product with the activation in its epilogue, products whose K is cut into shares over the grid, the shares
+// added up by whoever reads them, and several products of one size that do not read one another's results.
 //
 // A step's last row tile takes up to 16 rows beyond its 256: a portion of 512 tokens beside a few decode rows is two tiles high, not three.
 #include "common.h"
@@ -10,14 +10,20 @@
 namespace {
 using namespace block_gemm;
 
-enum { SILU, GELU, PARTS };
+enum { SILU, GELU, PARTS, PLAIN };
+
+constexpr int GROUP_MOST = 4;
+struct Operands {                    // PLAIN: a product's each; else the first alone
+  const bf16_t* x[GROUP_MOST];
+  const bf16_t* w[GROUP_MOST];
+  void* y[GROUP_MOST];
+};
 
 // What a tile gives, from LDS in whole lines: the gated ones bfloat16 y [M, N], 128 columns a tile (the tile's first half of columns are
-// gates and the second ups of w [2 N, K]), PARTS float32 y [splits, M, N].
+// gates and the second ups of w [2 N, K]), PARTS float32 y [splits, M, N], PLAIN bfloat16 y [M, N] of `splits` products.
 template <int KIND, int TR, int TC>
-__global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                                                                void* __restrict__ y, int M, int N, int K, int row_tiles,
-                                                                int col_tiles, int splits) {
+__global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(Operands op, int M, int N, int K, int row_tiles, int col_tiles,
+                                                                int splits) {
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES + 2 * EXTRA_BYTES];
   constexpr bool GATED = KIND == SILU || KIND == GELU;
   using S = Shape<TR, TC>;
@@ -26,7 +32,9 @@ __global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __
   const int tiles = row_tiles * col_tiles;
   int tile = tile_of_block(blockIdx.x, tiles * splits);
   if (tile < 0) return;
-  const int split = tile / tiles, share = K / splits;
+  const int split = tile / tiles, share = KIND == PLAIN ? K : K / splits, which = KIND == PLAIN ? split : 0;
+  const bf16_t *x = op.x[which], *w = op.w[which];
+  void* y = op.y[which];
   tile %= tiles;
   int rt, ct;
   row_and_column(tile, row_tiles, col_tiles, rt, ct);
@@ -47,7 +55,7 @@ __global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __
   ExtraAcc more;
   acc.clear();
   more.clear();
-  const int64_t k0 = (int64_t)split * share;
+  const int64_t k0 = KIND == PLAIN ? 0 : (int64_t)split * share;
   if (has_more) run_with<true, TR, TC>(acc, more, lds, x + k0, w + k0, x_at, w_at, more_at, share / KC);
   else run_with<false, TR, TC>(acc, more, lds, x + k0, w + k0, x_at, w_at, 0, share / KC);
   const PlaceOf<TR, TC> at;
@@ -77,6 +85,31 @@ __global__ void __launch_bounds__(THREADS, 2) gemm_block_kernel(const bf16_t* __
       if (m0 + row < M && column < N)
         *reinterpret_cast<uint4*>((bf16_t*)y + (int64_t)(m0 + row) * N + column) =
             *reinterpret_cast<const uint4*>(lds + row * PITCH + e % PIECES * 16);
+    }
+  } else if constexpr (KIND == PLAIN) {
+    constexpr int PITCH = HALF * 2 + 16, ROWS = TILE + EXTRA;      // half of the columns at a time
+    const auto rounded = [](f32x4_t v) {
+      ushort4 o;
+      o.x = float_to_bf16(v[0]); o.y = float_to_bf16(v[1]); o.z = float_to_bf16(v[2]); o.w = float_to_bf16(v[3]);
+      return o;
+    };
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int t = 0; t < TR; ++t)
+#pragma unroll
+          for (int n = 0; n < TC; ++n)
+            *reinterpret_cast<ushort4*>(lds + at.row(i, t) * PITCH + at.column(0, n) * 2) = rounded(acc.v[i][j][t][n]);
+      if (has_more && at.has_extra()) *reinterpret_cast<ushort4*>(lds + (TILE + at.c) * PITCH + at.extra_column(0) * 2) = rounded(more.v[j]);
+      __syncthreads();
+      for (int e = threadIdx.x; e < (has_more ? ROWS : TILE) * 16; e += THREADS) {
+        const int row = e / 16, column = n0 + j * HALF + e % 16 * 8;
+        if (m0 + row < M && column < N)
+          *reinterpret_cast<uint4*>((bf16_t*)y + (int64_t)(m0 + row) * N + column) = *reinterpret_cast<const uint4*>(lds + row * PITCH + e % 16 * 16);
+      }
+      __syncthreads();
     }
   } else {
     constexpr int PITCH = 144;                       // a wave's own 64 rows of 32 columns at a time
@@ -139,17 +172,17 @@ static int launch_block(int kind, const void* x, const void* w, void* y, int M, 
   const int wide = gated ? (slim ? SLIM : HALF) : TILE, cols = (N + wide - 1) / wide;
   const unsigned blocks = (unsigned)(((int64_t)rows * cols * splits + XCDS - 1) / XCDS * XCDS);      // every XCD as many
   hipStream_t s = (hipStream_t)stream;
-  const bf16_t *a = (const bf16_t*)x, *b = (const bf16_t*)w;
+  const Operands op{{(const bf16_t*)x}, {(const bf16_t*)w}, {y}};
   switch (kind) {
     case SILU:
-      if (slim) gemm_block_kernel<SILU, 2, 3><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
-      else gemm_block_kernel<SILU, 4, 2><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
+      if (slim) gemm_block_kernel<SILU, 2, 3><<<blocks, THREADS, 0, s>>>(op, M, N, K, rows, cols, splits);
+      else gemm_block_kernel<SILU, 4, 2><<<blocks, THREADS, 0, s>>>(op, M, N, K, rows, cols, splits);
       break;
     case GELU:
-      if (slim) gemm_block_kernel<GELU, 2, 3><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
-      else gemm_block_kernel<GELU, 4, 2><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits);
+      if (slim) gemm_block_kernel<GELU, 2, 3><<<blocks, THREADS, 0, s>>>(op, M, N, K, rows, cols, splits);
+      else gemm_block_kernel<GELU, 4, 2><<<blocks, THREADS, 0, s>>>(op, M, N, K, rows, cols, splits);
       break;
-    default: gemm_block_kernel<PARTS, 4, 2><<<blocks, THREADS, 0, s>>>(a, b, y, M, N, K, rows, cols, splits); break;
+    default: gemm_block_kernel<PARTS, 4, 2><<<blocks, THREADS, 0, s>>>(op, M, N, K, rows, cols, splits); break;
   }
   HOLON_LAUNCH_OK();
   return 0;
@@ -191,4 +224,25 @@ extern "C" int holon_gemm_block_parts_splits(int M, int N, int K) {
 // parts [splits, M, N] (float32) = x[:, share s of K] w[:, share s of K]^T.
 extern "C" int holon_gemm_block_parts_bf16(const void* x, const void* w, void* parts, int M, int N, int K, int splits, void* stream) {
   return launch_block(PARTS, x, w, parts, M, N, K, splits, 0, stream);
+}
+
+// `count` (up to 4) products of one size in one launch, where one of them would leave most compute units without a tile (four of 2,048 x 2,048
+// at 2,048 rows are a tile for each of the 256 units: 63 us, 1.1 PFLOP/s; one such product by itself takes 37): y_i [M, N] (bfloat16) = x_i [M, K] w_i [N, K]^T. `operands`: count pointers x, then w,
+// then y.
+extern "C" int holon_gemm_block_group_bf16(const int64_t* operands, int count, int M, int N, int K, void* stream) {
+  HOLON_CHECK(count >= 1 && count <= GROUP_MOST && holon_gemm_block_supported(M, N, K, 0, 1),
+              "gemm (many rows, several): %d products of M=%d N=%d K=%d not served", count, M, N, K);
+  Operands op{};
+  for (int i = 0; i < count; ++i) {
+    op.x[i] = (const bf16_t*)operands[i];
+    op.w[i] = (const bf16_t*)operands[count + i];
+    op.y[i] = (void*)operands[2 * count + i];
+    HOLON_CHECK(op.x[i] && op.w[i] && op.y[i] && ((operands[i] | operands[count + i] | operands[2 * count + i]) & 15) == 0,
+                "gemm (many rows, several): operands off 16 bytes");
+  }
+  const int rows = row_tiles_of(M), cols = (N + TILE - 1) / TILE;
+  const unsigned blocks = (unsigned)(((int64_t)rows * cols * count + XCDS - 1) / XCDS * XCDS);
+  gemm_block_kernel<PLAIN, 4, 2><<<blocks, THREADS, 0, (hipStream_t)stream>>>(op, M, N, K, rows, cols, count);
+  HOLON_LAUNCH_OK();
+  return 0;
 }

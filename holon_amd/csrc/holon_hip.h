@@ -199,6 +199,7 @@ int holon_gemm_block_parts_serves(int M, int N, int K, int splits);
 int holon_gemm_block_parts_splits(int M, int N, int K);
 int holon_gemm_block_parts_bf16(const void* x, const void* w, void* parts, int M, int N, int K, int splits, void* stream);
 int holon_gemm_block_glu_bf16(const void* x, const void* w, void* y, int M, int N, int K, int act, void* stream);
+int holon_gemm_block_group_bf16(const int64_t* operands, int count, int M, int N, int K, void* stream);
 int holon_gemm_block_glu_width_bf16(const void* x, const void* w, void* y, int M, int N, int K, int act, int width, void* stream);
 int holon_sum_parts(const void* parts, void* y, int splits, int64_t count, void* stream);
 // y[M, N] = x[M, K] w[N, K]^T, all float32, true 32-bit products and sums in an order that depends on K and N

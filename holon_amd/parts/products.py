@@ -5,7 +5,8 @@ weights need, and a block's sublayers, or two mixers side by side, wait for one 
 down in. A part may therefore say what it does as a generator (`products`, with `forward`'s arguments): it yields lists of
 `Product`s, is sent their results, and returns what `forward` returns. `drive` runs such parts side by side: in steps of few
 rows it collects what all of them ask for and runs it as one operation (`linear_group`); in other steps, and for parts
-without a generator, one after the other, each product as it always was.
+without a generator, one after the other: products of one size in one launch where they fill the chip together
+(`linear_block_group`), each other product as it always was.
 """
 from __future__ import annotations
 
@@ -20,6 +21,8 @@ from .linear import Linear
 
 FEW_ROWS = 16                 # up to this many rows products run together
 MOST = 8                      # products a launch takes
+BLOCK_ROWS = (129, 3072)      # this many rows: products of one size run together
+BLOCK_MOST = 4                # so many of them
 
 
 @dataclasses.dataclass
@@ -86,7 +89,7 @@ def products_of(part, *args, **kwargs):
 def drive(kernels, rows: int, *parts) -> list:
     """What each generator returns."""
     if rows > FEW_ROWS:
-        return [_by_itself(part) for part in parts]
+        return [_by_itself(kernels, part) for part in parts]
     results, asked = [None] * len(parts), {}
 
     def go(i: int, send) -> None:
@@ -105,11 +108,12 @@ def drive(kernels, rows: int, *parts) -> list:
     return results
 
 
-def _by_itself(part):
+def _by_itself(kernels, part):
     send = None
     while True:
         try:
-            send = [p.alone() for p in part.send(send)]
+            asked = part.send(send)
+            send = [p.alone() for p in asked] if len(asked) < BLOCK_MOST else kernels.linear_block_group(asked)
         except StopIteration as end:
             return end.value
 
@@ -166,3 +170,54 @@ def _linear_group_hip(launch, products: list[Product | Routing]) -> list[torch.T
 
 register_kernel(KernelOp("linear_group", linear_group_plain, "holon_gemm_skinny_group_bf16",
                          [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_float], _linear_group_hip))
+
+
+def block_group_pays(count: int, m: int, n: int, k: int) -> bool:
+    """Whether `count` bfloat16 products of m rows over [n, k] weights run as one launch on 256 x 256 tiles rather than one after the
+    other. A tile takes about 5 us + K / 64 however few of the 256 compute units have one, so that one product of 2,048 rows and
+    columns leaves three quarters of the chip idle (36 us; the library's smaller tiles 25), and four of them take 63 us where the
+    library's four take 100. Four products against the library's, inside a graph: 36 | 36 us at 129 rows of 2,048 x 2,048, 37 | 44
+    at 400, 42 | 65 at 1,024, 103 | 127 at 3,000, 123 | 155 at 4,096; 2,560 x 2,560: 43 | 43 at 129, 57 | 104 at 1,024, 187 | 221 at
+    4,096; 4,096 x 4,096: 71 | 88 at 129, 114 | 181 at 1,024, 308 | 347 at 3,000, then 406 | 385 at 4,096, where one product fills
+    the chip by itself. Two or three gain little or lose at most sizes (three of 4,096 x 4,096 at 1,400 rows 155 | 153)."""
+    return count == BLOCK_MOST and BLOCK_ROWS[0] <= m <= BLOCK_ROWS[1] and 1024 <= n <= 8192 and 1024 <= k < 8192 and k % 128 == 0 and n % 16 == 0
+
+
+def _block_served(p: Product | Routing) -> bool:
+    if not isinstance(p, Product) or p.relu2 or p.dtype not in (None, torch.bfloat16) or not isinstance(p.x, torch.Tensor):
+        return False
+    x, w = p.x, p.linear.weight
+    return (x.is_cuda and w is not None and x.dtype == w.dtype == torch.bfloat16 and x.dim() == w.dim() == 2 and x.shape[1] == w.shape[1]
+            and x.is_contiguous() and w.is_contiguous() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def linear_block_group_plain(products: list[Product | Routing]) -> list[torch.Tensor]:
+    """What `linear_group` returns, of products of many rows."""
+    return [p.alone() for p in products]
+
+
+def _linear_block_group_hip(launch, products: list[Product | Routing]) -> list[torch.Tensor]:
+    out: list = [None] * len(products)
+    alike: dict[tuple, list[int]] = {}
+    for i, p in enumerate(products):
+        if _block_served(p):
+            alike.setdefault((p.x.shape[0], *p.linear.weight.shape), []).append(i)
+    for (m, n, k), which in alike.items():
+        for at in range(0, len(which), BLOCK_MOST):
+            group = which[at: at + BLOCK_MOST]
+            first = products[group[0]].linear
+            # (a model whose sums stay as they are keeps the library's order of them)
+            if not block_group_pays(len(group), m, n, k) or first.kernels.settled or \
+                    first.kernels.product_choice("group", first.weight, m, yields=True, by_rule=True) != "own":
+                continue
+            y = torch.empty((len(group), m, n), dtype=torch.bfloat16, device=products[group[0]].x.device)
+            for i, rows in zip(group, y):
+                out[i] = rows
+            operands = [products[i].x.data_ptr() for i in group] + [products[i].linear.weight.data_ptr() for i in group] + \
+                [out[i].data_ptr() for i in group]
+            launch((ctypes.c_int64 * len(operands))(*operands), len(group), m, n, k)
+    return [y if y is not None else p.alone() for y, p in zip(out, products)]
+
+
+register_kernel(KernelOp("linear_block_group", linear_block_group_plain, "holon_gemm_block_group_bf16",
+                         [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int], _linear_block_group_hip))

@@ -1801,3 +1801,36 @@ def test_a_router_beside_products_is_the_router(hip, rows, experts, extra, group
     for p, got in zip(products, hip.linear_group(products)):
         assert torch.equal(got, p.alone())
     assert torch.equal(hip.linear_group([routing])[0], routing.alone())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [(129, 1024, 1024), (256, 1040, 1152), (272, 1264, 1024), (273, 2048, 1280), (1025, 1536, 1024), (3072, 1024, 1024)])
+def test_products_of_many_rows_in_one_launch(hip, m, n, k):
+    """Four products of one size among others, in one launch on 256 x 256 tiles: each within a rounding (2^-9) and float32 sums of k of
+    its exact product, columns that end inside a tile, rows up to 16 beyond the last tile's 256 and more. What the group does not take
+    (another size, a float32 result, the fifth) is what it is alone."""
+    from holon_amd.parts.products import Product, block_group_pays
+
+    class Weights:                                # what a projection holds
+        folded, tiled, kernels = None, None, hip
+
+        def __init__(self, i, out):
+            self.weight = _randn(out, k, dtype=torch.bfloat16, seed=210 + i, scale=k ** -0.5)
+
+        def __call__(self, x, dtype=None):
+            return hip.linear(x, self.weight, dtype)
+    linears = [Weights(i, out) for i, out in enumerate([n, n, 512, n, n, n, n])]
+    xs = _randn(len(linears), m, k, dtype=torch.bfloat16, seed=209)
+    products = [Product(lin, xs[i], torch.float32 if i == 5 else None) for i, lin in enumerate(linears)]
+    assert block_group_pays(4, m, n, k)
+    got = hip.linear_block_group(products)
+    together = got[0].untyped_storage().data_ptr()
+    assert [g.untyped_storage().data_ptr() == together for g in got] == [True, True, False, True, True, False, False]
+    for i, (p, y) in enumerate(zip(products, got)):
+        want = p.x.double() @ p.linear.weight.double().t()
+        assert y.shape == want.shape and H.rel_rms(y, want) < 2.0 ** -9 + 2.0 ** -24 * k ** 0.5
+        if i in (2, 5, 6):
+            assert torch.equal(y, p.alone())
+    with pytest.MonkeyPatch.context() as settled:
+        settled.setattr(hip, "settled", True)
+        assert all(torch.equal(y, p.alone()) for y, p in zip(hip.linear_block_group(products), products))

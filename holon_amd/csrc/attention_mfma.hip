@@ -23,6 +23,7 @@
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bf16x8_t load8(const bf16_t* p) { return *reinterpret_cast<const bf16x8_t*>(p); }
 
@@ -34,6 +35,17 @@ __device__ __forceinline__ void zero_after(bf16x8_t& v, int first_key, int key_h
 #pragma unroll
   for (int i = 0; i < 8; ++i)
     if (first_key + i > key_hi) v[i] = (__bf16)0.f;
+}
+
+// The same by masks of two keys, which a block's fragments share, where a walk is short and its last block a good part of it: by elements a
+// decode row of 100 keys of 128 dims took 7.1 us, so 5.6 (one of 128 keys 5.4). The prompt kernels, whose last stage is one of many and
+// whose registers are all in use, have nothing left over for the masks.
+__device__ __forceinline__ void mask_after(bf16x8_t& v, int first_key, int key_hi) {
+  u32x4_t words = __builtin_bit_cast(u32x4_t, v);
+  const int last = key_hi - first_key;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) words[i] &= (2 * i <= last ? 0xffffu : 0u) | (2 * i + 1 <= last ? 0xffff0000u : 0u);
+  v = __builtin_bit_cast(bf16x8_t, words);
 }
 
 struct AttnArgs {
@@ -278,31 +290,13 @@ __device__ __forceinline__ void attn_tiles(const AttnArgs& a, const int32_t* __r
     bf16x8_t vf[D / 16];
 #pragma unroll
     for (int ds = 0; ds < D / 16; ++ds) vf[ds] = load8(vrowp + (int64_t)ds * 16 * P);
-    if (kb + 31 > key_hi) {
-#pragma unroll
-      for (int ds = 0; ds < D / 16; ++ds) zero_after(vf[ds], kb + 8 * g, key_hi);
-    }
-    if (MOD && kb < kept_end) {                            // a kept block: what lies behind the kept keys is not held
-#pragma unroll
-      for (int ds = 0; ds < D / 16; ++ds) zero_after(vf[ds], kb + 8 * g, kept_keys - 1);
-    }
-    if (fresh != nullptr && kb + 31 >= key_hi) {           // the block that holds key_hi: its key and value from LDS
+    if (fresh != nullptr && kb + 31 >= key_hi) {           // the block that holds key_hi: its key from LDS
       const int k0 = kb + 16 * khalf + kin;                // this lane's keys are k0 and k0 + 4
       if (k0 == key_hi || k0 + 4 == key_hi) {
 #pragma unroll
         for (int ks = 0; ks < D / 32; ++ks) {
           const bf16x8_t nk = *reinterpret_cast<const bf16x8_t*>(fresh + ks * 32 + 8 * g);
           if (k0 == key_hi) kf0[ks] = nk; else kf1[ks] = nk;
-        }
-      }
-      const int j = key_hi - (kb + 8 * g);                 // the value's place among this lane's eight keys, if any
-      if (j >= 0 && j < 8) {
-#pragma unroll
-        for (int ds = 0; ds < D / 16; ++ds) {
-          const __bf16 nv = reinterpret_cast<const __bf16*>(fresh + D)[ds * 16 + c];
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (i == j) vf[ds][i] = nv;
         }
       }
     }
@@ -334,6 +328,31 @@ __device__ __forceinline__ void attn_tiles(const AttnArgs& a, const int32_t* __r
                                             o[t], a.scale, a.softcap, mod[t], a.window > 0 ? a.keep_first : 0);
       else
         pb[t] = softmax_block<D / 16>(s0, s1, whole, kb, g, qp, first, key_lo, key_hi, a.scale_log2, m[t], l[t], o[t]);
+    }
+    // What lies behind the last key among the values, now that the scores are done: it needs the newest of a lane's loads.
+    if (kb + 31 > key_hi) {
+#pragma unroll
+      for (int ds = 0; ds < D / 16; ++ds) mask_after(vf[ds], kb + 8 * g, key_hi);
+    }
+    if (MOD && kb < kept_end) {                            // a kept block: what lies behind the kept keys is not held
+#pragma unroll
+      for (int ds = 0; ds < D / 16; ++ds) mask_after(vf[ds], kb + 8 * g, kept_keys - 1);
+    }
+    if (fresh != nullptr && kb + 31 >= key_hi) {           // the new token's value from LDS
+      const int j = key_hi - (kb + 8 * g);                 // the value's place among this lane's eight keys, if any
+      if (j >= 0 && j < 8) {
+#pragma unroll
+        for (int ds = 0; ds < D / 16; ++ds) {
+          const uint32_t nv = fresh[D + ds * 16 + c] * 0x10001u;
+          u32x4_t words = __builtin_bit_cast(u32x4_t, vf[ds]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t here = j == 2 * i ? 0xffffu : j == 2 * i + 1 ? 0xffff0000u : 0u;
+            words[i] = (words[i] & ~here) | (nv & here);
+          }
+          vf[ds] = __builtin_bit_cast(bf16x8_t, words);
+        }
+      }
     }
 #pragma unroll
     for (int ds = 0; ds < D / 16; ++ds) {
@@ -1623,8 +1642,10 @@ struct NewKeyValue {
 // adds them as they are); with one block a (row, kv head) it writes the result, multiplied by the gate's sigmoid if one is
 // given, with more `sigmoid_merge_kernel` adds their sums in order.
 // MOD: changed scores (see AttnArgs); the wave that takes the row's first share also walks the kept first keys.
+// D = 256: at most four waves a block (their partials fit no more into LDS), so that a lane may have 512 registers; with 256 it kept 284
+// bytes in memory: a row of 100 keys with 16 heads over one key head 12.1 us -> 7.6, one of 256 keys 16.2 -> 9.9.
 template <int D, bool FUSED, bool SIG = false, bool MOD = false>
-__global__ void __launch_bounds__(512) attn_decode_kernel(AttnArgs a, FusedArgs f) {
+__global__ void __launch_bounds__(D == 256 ? 256 : 512) attn_decode_kernel(AttnArgs a, FusedArgs f) {
   extern __shared__ __attribute__((aligned(16))) float red[];   // [waves - 1][16 D values, 16 maxima, 16 sums]
   __shared__ __attribute__((aligned(16))) bf16_t fresh_lds[FUSED ? 2 * D : 8];
   constexpr int PART = 16 * D + 32;

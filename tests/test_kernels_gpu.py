@@ -1834,3 +1834,28 @@ def test_products_of_many_rows_in_one_launch(hip, m, n, k):
     with pytest.MonkeyPatch.context() as settled:
         settled.setattr(hip, "settled", True)
         assert all(torch.equal(y, p.alone()) for y, p in zip(hip.linear_block_group(products), products))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("softcap", [0.0, 20.0])
+@pytest.mark.parametrize("geometry", [(8, 2, 64), (16, 4, 128), (16, 1, 256)])
+def test_decode_rows_of_every_last_block(hip, geometry, softcap):
+    """Decode rows of 1 to 64 keys, NaN in every cache slot behind them, alone in their block and over its four waves: each row within its
+    budget of the plain form in float64, and bit for bit what it is with zeros there."""
+    heads, kv_heads, d = geometry
+    page, dtype, rows = 16, torch.bfloat16, [(n, 1) for n in range(64)]
+    q, pages, table, attn = _paged_case(rows, heads, kv_heads, d, page, dtype, seed=31, max_seqs=64)
+    held = torch.zeros(pages.shape[0], page, dtype=torch.bool)
+    for slot, (s, n) in zip(attn.slots.tolist(), rows):
+        pos = torch.arange(s + n)
+        held[table[slot, pos // page].cpu().long(), pos % page] = True
+    outs, free = [], (~held).cuda()
+    for longest in (64, 256):
+        attn.max_decode_len = longest
+        for fill in (0.0, float("nan")):
+            pages[:, 0].view(-1, kv_heads, page, d).masked_fill_(free[:, None, :, None], fill)
+            pages[:, 1].view(-1, kv_heads, d, page).masked_fill_(free[:, None, None, :], fill)
+            outs.append(hip.paged_attention(q, pages, table, attn, page, d ** -0.5, 0, softcap=softcap))
+        assert torch.equal(outs[-1], outs[-2]) and torch.isfinite(outs[-1].float()).all()
+        want = PLAIN.paged_attention(q.double(), pages.double(), table, attn, page, d ** -0.5, 0, softcap=softcap)
+        assert H.op_budget_usage(outs[-1], want, dtype, d + 64) <= 1

@@ -154,10 +154,27 @@ struct Filter4 {
   }
 };
 
+// Four neighbouring values as they are stored, and widened.
+template <int DT>
+using Four = std::conditional_t<DT == HOLON_F32, float4, ushort4>;
+template <int DT>
+__device__ __forceinline__ Four<DT> raw4(const void* p, int64_t i) {
+  using E = std::conditional_t<DT == HOLON_F32, float, bf16_t>;
+  return *reinterpret_cast<const Four<DT>*>(reinterpret_cast<const E*>(p) + i);
+}
+__device__ __forceinline__ void widen4(const float4& f, float (&v)[4]) { v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w; }
+__device__ __forceinline__ void widen4(const ushort4& h, float (&v)[4]) {
+  v[0] = bf16_to_float(h.x); v[1] = bf16_to_float(h.y); v[2] = bf16_to_float(h.z); v[3] = bf16_to_float(h.w);
+}
+
 // The same pass as stream_rms_kernel with four neighbouring values a thread and step (dim a multiple of 4, at most
 // 1024 REGS values a row, which stay in registers). FILTER: the step's rows are single tokens, and each result goes
 // through its causal filter of TAPS taps before it is stored (see `filter4`).
-template <int REGS, int TAPS, int DT = HOLON_BF16>     // DT: the results' (and the filters') dtype, read when TAPS > 0
+// AHEAD: the terms, the weights and the results are of one type (DT), and everything that the row needs is asked for before any of it is
+// read: a step of few rows is a block or a few, and what it takes is one memory latency after the other, where a branch on a type
+// stands around each load. One row of 2,048 (two terms, one weight) 3.1 us -> 2.5, with the added vector, two weights and filters 4.6 ->
+// 3.7; of 4,096 4.4 -> 3.1 and 7.2 -> 5.4; 2,048 rows of 2,048 9.2 -> 8.7. Rows beyond 4,096 would hold more than the registers are worth.
+template <int REGS, int TAPS, int DT = HOLON_BF16, bool AHEAD = false>     // DT: read when TAPS > 0 or AHEAD
 __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__ x32, const void* __restrict__ d1, int dt1,
                                                              const void* __restrict__ d2, int dt2,
                                                              const float* __restrict__ row, const void* __restrict__ w1,
@@ -168,41 +185,10 @@ __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__
   const int64_t base = (int64_t)blockIdx.x * dim;
   float held[REGS][4];
   float sq = 0.f;
-#pragma unroll
-  for (int e = 0; e < REGS; ++e) {
-    const int i = (threadIdx.x + e * 256) * 4;
-    float (&v)[4] = held[e];
-    v[0] = v[1] = v[2] = v[3] = 0.f;
-    if (i < dim) {
-      load4(x32, base + i, HOLON_F32, v);
-      if (d1) {
-        float a[4];
-        load4(d1, base + i, dt1, a);
-        if (d2) {
-          float b[4];
-          load4(d2, base + i, dt2, b);
-#pragma unroll
-          for (int u = 0; u < 4; ++u) a[u] += b[u];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] += a[u];
-      }
-      if (row) {
-        float b[4];
-        load4(row, i, HOLON_F32, b);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] += b[u];
-      }
-      if (d1 || row) store4(x32, base + i, HOLON_F32, v);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) sq += v[u] * v[u];
-  }
-  if (!w1) return;
   constexpr bool FILTER = TAPS > 0;
-  // the filters' old inputs and taps are asked for now, so that they arrive while the row's sum is taken
+  Four<DT> g1[AHEAD ? REGS : 1], g2[AHEAD ? REGS : 1];
   Filter4<FILTER ? TAPS : 1, DT> f1[FILTER ? REGS : 1], f2[FILTER ? REGS : 1];
-  if constexpr (FILTER) {
+  auto ask_filters = [&]() {
     const int slot = f.slots[blockIdx.x];
     const bool carried = f.starts[blockIdx.x] > 0;
 #pragma unroll
@@ -212,6 +198,101 @@ __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__
       f1[e].load(f.held1, f.w1, slot, carried, i, dim);
       if (w2) f2[e].load(f.held2, f.w2, slot, carried, i, dim);
     }
+  };
+  if constexpr (AHEAD) {
+    float4 xs[REGS], rs[REGS];
+    Four<DT> as[REGS], bs[REGS];
+    int at[REGS];
+#pragma unroll
+    for (int e = 0; e < REGS; ++e) {
+      at[e] = min((int)(threadIdx.x + e * 256) * 4, dim - 4);      // (what lies behind the row reads its end and keeps nothing of it)
+      xs[e] = raw4<HOLON_F32>(x32, base + at[e]);
+    }
+    if (d1) {
+#pragma unroll
+      for (int e = 0; e < REGS; ++e) as[e] = raw4<DT>(d1, base + at[e]);
+    }
+    if (d2) {
+#pragma unroll
+      for (int e = 0; e < REGS; ++e) bs[e] = raw4<DT>(d2, base + at[e]);
+    }
+    if (row) {
+#pragma unroll
+      for (int e = 0; e < REGS; ++e) rs[e] = raw4<HOLON_F32>(row, at[e]);
+    }
+    if (w1) {
+#pragma unroll
+      for (int e = 0; e < REGS; ++e) g1[e] = raw4<DT>(w1, at[e]);
+    }
+    if (w2) {
+#pragma unroll
+      for (int e = 0; e < REGS; ++e) g2[e] = raw4<DT>(w2, at[e]);
+    }
+    if constexpr (FILTER) ask_filters();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < REGS; ++e) {
+      const int i = (threadIdx.x + e * 256) * 4;
+      float (&v)[4] = held[e];
+      widen4(xs[e], v);
+      if (d1) {
+        float a[4], b[4];
+        widen4(as[e], a);
+        if (d2) {
+          widen4(bs[e], b);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) a[u] += b[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] += a[u];
+      }
+      if (row) {
+        float b[4];
+        widen4(rs[e], b);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] += b[u];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = i < dim ? v[u] : 0.f;
+      if (i < dim && (d1 || row)) store4(x32, base + i, HOLON_F32, v);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sq += v[u] * v[u];
+    }
+    if (!w1) return;
+  } else {
+#pragma unroll
+    for (int e = 0; e < REGS; ++e) {
+      const int i = (threadIdx.x + e * 256) * 4;
+      float (&v)[4] = held[e];
+      v[0] = v[1] = v[2] = v[3] = 0.f;
+      if (i < dim) {
+        load4(x32, base + i, HOLON_F32, v);
+        if (d1) {
+          float a[4];
+          load4(d1, base + i, dt1, a);
+          if (d2) {
+            float b[4];
+            load4(d2, base + i, dt2, b);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[u] += b[u];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] += a[u];
+        }
+        if (row) {
+          float b[4];
+          load4(row, i, HOLON_F32, b);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] += b[u];
+        }
+        if (d1 || row) store4(x32, base + i, HOLON_F32, v);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) sq += v[u] * v[u];
+    }
+    if (!w1) return;
+    // the filters' old inputs and taps are asked for now, so that they arrive while the row's sum is taken
+    if constexpr (FILTER) ask_filters();
   }
   sq = block_sum_256(sq, part);
   const float r = 1.0f / sqrtf(sq / (float)dim + eps);
@@ -220,11 +301,13 @@ __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__
     const int i = (threadIdx.x + e * 256) * 4;
     if (i >= dim) continue;
     float g[4], y[4], z[4];
-    load4(w1, i, dtw, g);
+    if constexpr (AHEAD) widen4(g1[e], g);
+    else load4(w1, i, dtw, g);
 #pragma unroll
     for (int u = 0; u < 4; ++u) y[u] = held[e][u] * r * g[u];
     if (w2) {
-      load4(w2, i, dtw, g);
+      if constexpr (AHEAD) widen4(g2[e], g);
+      else load4(w2, i, dtw, g);
 #pragma unroll
       for (int u = 0; u < 4; ++u) z[u] = held[e][u] * r * g[u];
     }
@@ -237,8 +320,8 @@ __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__
       f1[e].keep(f.held1, a, dim);
       if (w2) f2[e].keep(f.held2, b, dim);
     }
-    store4(y1, base + i, dt_out, y);
-    if (w2) store4(y2, base + i, dt_out, z);
+    store4(y1, base + i, AHEAD ? DT : dt_out, y);
+    if (w2) store4(y2, base + i, AHEAD ? DT : dt_out, z);
   }
 }
 
@@ -365,6 +448,12 @@ __global__ void scale_rows_kernel(const void* __restrict__ x, float* __restrict_
 }
 }  // namespace
 
+// The one type of the terms, the weights and the results, -1 where they differ.
+static int one_type(const void* d1, int dt1, const void* d2, int dt2, const void* w1, int dtw, int dt_out) {
+  const int dt = w1 ? dt_out : d1 ? dt1 : HOLON_BF16;
+  return (d1 && dt1 != dt) || (d2 && dt2 != dt) || (w1 && dtw != dt) ? -1 : dt;
+}
+
 extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void* d2, int dt2, const float* row,
                                 const void* w1, const void* w2, int dtw, void* y1, void* y2, int64_t rows, int dim,
                                 float eps, int dt_out, void* stream) {
@@ -376,11 +465,19 @@ extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void*
   hipStream_t s = (hipStream_t)stream;
   if (dim % 4 == 0 && dim <= 8192) {        // four values a thread and step (every operand is a tensor's start: 16 bytes)
     const Filters none{};
-#define SRMSV(R) stream_rms_vec_kernel<R, 0><<<(unsigned)rows, 256, 0, s>>>(x32, d1, dt1, d2, dt2, row, w1, w2, dtw, y1, y2, dim, eps, dt_out, none)
-    if (dim <= 1024) SRMSV(1);
-    else if (dim <= 2048) SRMSV(2);
-    else if (dim <= 4096) SRMSV(4);
-    else SRMSV(8);
+    const int one = one_type(d1, dt1, d2, dt2, w1, dtw, dt_out);
+#define SRMSV(...) stream_rms_vec_kernel<__VA_ARGS__><<<(unsigned)rows, 256, 0, s>>>(x32, d1, dt1, d2, dt2, row, w1, w2, dtw, y1, y2, dim, eps, dt_out, none)
+#define SRMSV_BY_TYPE(R)                                 \
+  do {                                                   \
+    if (one == HOLON_BF16) SRMSV(R, 0, HOLON_BF16, true); \
+    else if (one == HOLON_F32) SRMSV(R, 0, HOLON_F32, true); \
+    else SRMSV(R, 0);                                    \
+  } while (0)
+    if (dim <= 1024) SRMSV_BY_TYPE(1);
+    else if (dim <= 2048) SRMSV_BY_TYPE(2);
+    else if (dim <= 4096) SRMSV_BY_TYPE(4);
+    else SRMSV(8, 0);
+#undef SRMSV_BY_TYPE
 #undef SRMSV
     HOLON_LAUNCH_OK();
     return 0;
@@ -413,9 +510,16 @@ extern "C" int holon_stream_rms_filter(float* x32, const void* d1, int dt1, cons
   if (rows == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const Filters f{cw1, cw2, held1, held2, slots, starts, taps};
+  const bool ahead = dim <= 4096 && one_type(d1, dt1, d2, dt2, w1, dtw, dt_out) == dt_out;
 #define SRMSF(R, K)                                                                                                  \
   do {                                                                                                               \
-    if (dt_out == HOLON_F32)                                                                                         \
+    if (ahead && R <= 4 && dt_out == HOLON_F32)                                                                      \
+      stream_rms_vec_kernel<R <= 4 ? R : 4, K, HOLON_F32, true><<<(unsigned)rows, 256, 0, s>>>(                      \
+          x32, d1, dt1, d2, dt2, row, w1, w2, dtw, y1, y2, dim, eps, dt_out, f);                                     \
+    else if (ahead && R <= 4)                                                                                        \
+      stream_rms_vec_kernel<R <= 4 ? R : 4, K, HOLON_BF16, true><<<(unsigned)rows, 256, 0, s>>>(                     \
+          x32, d1, dt1, d2, dt2, row, w1, w2, dtw, y1, y2, dim, eps, dt_out, f);                                     \
+    else if (dt_out == HOLON_F32)                                                                                         \
       stream_rms_vec_kernel<R, K, HOLON_F32><<<(unsigned)rows, 256, 0, s>>>(x32, d1, dt1, d2, dt2, row, w1, w2, dtw, \
                                                                             y1, y2, dim, eps, dt_out, f);            \
     else                                                                                                             \

@@ -1859,3 +1859,35 @@ def test_decode_rows_of_every_last_block(hip, geometry, softcap):
         assert torch.equal(outs[-1], outs[-2]) and torch.isfinite(outs[-1].float()).all()
         want = PLAIN.paged_attention(q.double(), pages.double(), table, attn, page, d ** -0.5, 0, softcap=softcap)
         assert H.op_budget_usage(outs[-1], want, dtype, d + 64) <= 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim", [4, 1020, 1028, 2048, 4092, 4096, 4100])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_stream_rows_of_one_type_are_those_of_several(hip, dtype, dim):
+    """A pass over stream rows whose operands are of one type and asked for ahead gives the bits of the general one (taken here by a term
+    of the other type that holds the same values, or by a weight that does): with and without terms, vector, second weight, filters."""
+    import holon_amd.parts.parallel_block  # noqa: F401  (brings the operations)
+    other = torch.float32 if dtype == torch.bfloat16 else torch.bfloat16
+    rows = 3
+    x, row = _randn(rows, dim, dtype=torch.float32, seed=220), _randn(dim, dtype=torch.float32, seed=221)
+    t1, t2 = (_randn(rows, dim, dtype=torch.bfloat16, seed=s).to(dtype) for s in (222, 223))
+    w1, w2 = (_randn(dim, dtype=torch.bfloat16, seed=s).to(dtype) for s in (224, 225))
+    c1, c2 = (_randn(dim, 3, dtype=torch.bfloat16, seed=s).to(dtype) for s in (226, 227))
+    held = _randn(2, rows, 2, dim, dtype=torch.bfloat16, seed=228).to(dtype)
+    slots, starts = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([2, 0, 1], [5, 0, 1]))
+    for terms in ([], [t1], [t1, t2]):
+        for added in (None, row):
+            for second in (None, w2):
+                got = []
+                for to_terms, to_weights in ((dtype, dtype), (dtype, other)) + (((other, dtype),) if terms else ()):
+                    xs, hs = x.clone(), held.clone()
+                    args = (xs, [(t.to(to_terms), 1.0) for t in terms], added, w1.to(to_weights),
+                            None if second is None else second.to(to_weights), 1e-6, dtype)
+                    y = [*hip.stream_rms(*args), xs]
+                    args[0].copy_(x)
+                    y += [*hip.stream_rms_filter(*args, c1, c2 if second is not None else None, hs[0], hs[1] if second is not None else None,
+                                                 slots, starts), xs.clone(), hs]
+                    got.append([v for v in y if v is not None])
+                for one in got[1:]:
+                    assert all(torch.equal(a, b) for a, b in zip(one, got[0], strict=True)), (len(terms), added is None, second is None)

@@ -78,8 +78,8 @@ def softmax_attention_plain(q, pages, table, rows, token_row, positions, kv_head
 
 def _float64_sums_serve(heads, kv_heads, dim, vdim, page_size):
     """What the library's `holon_softmax_attention_f64_supported` answers. That kernel takes every float32 step of such heads, prompts (four
-    times as fast) and decode rows (1.2 to 1.4 times the general one's time) alike: their orders of sums differ, and a position has the
-    same bits whatever step it comes in only if one of the two takes them all."""
+    times as fast) and decode rows (1.2 to 1.4 times the general one's time, where neither has its waves in blocks of their own) alike:
+    their orders of sums differ, and a position has the same bits whatever step it comes in only if one of the two takes them all."""
     return dim == vdim and dim in (64, 128) and page_size % 16 == 0 and heads % kv_heads == 0 \
         and kv_heads * -(-(heads // kv_heads) // 16) <= 65535
 

@@ -59,7 +59,7 @@ def dispatches(path: str) -> list[tuple]:
 
 
 CLASSES = (("attention", ("attn_", "sigmoid_attention", "softmax_attention", "latent_attention", "latent_prefill", "latent_decode",
-                          "latent_merge")),
+                          "latent_merge", "sigmoid_merge", "attention_generic", "attention_f64")),
            ("matrix products", ("gemm_", "Cijk_", "Custom_Cijk_", "hipBLASLt", "head_linear", "moe_up_few", "moe_down_few")),
            ("recurrent scans", ("memory_scan", "delta_scan", "delta_blocks", "delta_chain", "delta_walk", "mlstm_scan", "mlstm_chunk", "mlstm_pieces", "mlstm_gates", "ssd_", "gla_")),
            ("elementwise", ("rmsnorm", "gated_mul", "qk_norm_rope", "v_write", "kv_write", "embedding", "sum_parts",

@@ -31,7 +31,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
-from .products import Product, drive
+from .products import FEW_ROWS, Product, drive
 from .softmax_attention import attend, to_half_split
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -141,7 +141,8 @@ class DiffAttention(Part):
         held = site.paged[self.state_name]
         view = step.paged[held.group]
         table = getattr(self.position, "table", None)
-        qkv, = yield [Product(self.qkv, x)]
+        few = x.shape[0] <= FEW_ROWS
+        qkv = (yield [Product(self.qkv, x)])[0] if few else self.qkv(x)
         if self.own_kv:
             q = k.head_prepare(qkv, 2 * self.heads, 2 * self.kv_heads, self.dim, self.vdim, self.q_norm,
                                self.k_norm, self.eps, table, step.positions, held.pages, view.write_page,
@@ -151,7 +152,7 @@ class DiffAttention(Part):
                                self.eps, table, step.positions, None, None, None, view.page_size)
         maps = attend(k, q, held, view, step, 2 * self.kv_heads, self.vdim, None, self.scale, 0, value_share=2)
         out = k.diff_combine(maps, self.heads, self.kv_heads, self.vdim, self.lam, self.eps, 1.0 - self.diff)
-        return (yield [Product(self.o, out)])[0]
+        return (yield [Product(self.o, out)])[0] if few else self.o(out)
 
     def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]

@@ -12,7 +12,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, Stream
 from .linear import Linear
 from .norms import Normed
-from .products import Product, Routing, drive
+from .products import FEW_ROWS, Product, Routing, drive
 
 
 @register_part("ffn", "swiglu")
@@ -528,8 +528,10 @@ class PolyNormFFN(Part):
         self.declare("act", (4,), kind=FLOAT32, init="unit")
 
     def products(self, x: torch.Tensor, step=None):
-        up, = yield [Product(self.up_proj, x)]
-        return (yield [Product(self.down_proj, self.kernels.polynorm(up, self.act, self.eps))])[0]
+        few = x.shape[0] <= FEW_ROWS
+        up = (yield [Product(self.up_proj, x)])[0] if few else self.up_proj(x)
+        y = self.kernels.polynorm(up, self.act, self.eps)
+        return (yield [Product(self.down_proj, y)])[0] if few else self.down_proj(y)
 
     def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step))[0]
@@ -553,8 +555,10 @@ class DenseFFN(Part):
         self.attach("down_proj", Linear(build, inp=inter, out=hidden))
 
     def products(self, x: torch.Tensor, step=None):
-        y, = yield [Product(self.up_proj, x, relu2=True)]
-        return (yield [Product(self.down_proj, y)])[0]
+        few = x.shape[0] <= FEW_ROWS
+        up = Product(self.up_proj, x, relu2=True)
+        y = (yield [up])[0] if few else up.alone()
+        return (yield [Product(self.down_proj, y)])[0] if few else self.down_proj(y)
 
     def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step))[0]
@@ -668,7 +672,7 @@ class MoE(Part):
         else:
             route = Routing(k, x, self.router, self.correction if self.has_bias else None, self.experts, self.top, self.groups, self.keep,
                             scale=self.scale)
-        weights, = yield [route]
+        weights = (yield [route])[0] if x.shape[0] <= FEW_ROWS else route.alone()
         up, down = self.gate_up, self.all_down
         if x.dtype == torch.float32 and moe_f32_takes(x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top):
             y = k.moe_f32(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",

@@ -15,7 +15,7 @@ from ..kernels.registry import KernelOp, register_kernel
 from ..registry import register_part
 from .base import FLOAT32, Build, Part, SlotState
 from .linear import Linear
-from .products import Product, drive
+from .products import FEW_ROWS, Product, drive
 from .recurrent import MAX_KEY_DIM, _need, _rows, gated_out_plain, scan_pieces
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -197,8 +197,9 @@ class GatedLinearAttention(Part):
     def products(self, x: torch.Tensor, step, site, rows: torch.Tensor | None = None, at: int = 0):
         """`rows`: the input's projections, this mixer's from column `at` on (None: made here from `x`)."""
         k = self.kernels
+        few = x.shape[0] <= FEW_ROWS
         if rows is None:
-            rows, = yield [Product(self.inp, x)]
+            rows = (yield [Product(self.inp, x)])[0] if few else self.inp(x)
         c, n = self.heads * self.dim, self.heads * self.vdim
         q, kk = rows[:, at: at + c], rows[:, at + c: at + 2 * c]
         v, gate = rows[:, at + 2 * c: at + 2 * c + n], rows[:, at + 2 * c + n: at + 2 * c + 2 * n]
@@ -207,11 +208,12 @@ class GatedLinearAttention(Part):
         if step.rows.in_order and gla_step_serves(self.dim, self.vdim):       # single tokens: one kernel
             y = k.gla_step(q, kk, v, gate, a, self.scale, self.a2t, self.a2_bias, self.tau, self.norm, self.eps, state,
                            step.slots, step.starts, self.heads)
-            return (yield [Product(self.o, y)])[0]
+            return (yield [Product(self.o, y)])[0] if few else self.o(y)
         alpha = k.gla_decay(a, self.a2t, self.a2_bias, self.tau)
         o = k.gla_scan(q, kk, v, self.scale, alpha, state, step.slots, step.starts, step.query_start, step.n_rows,
                        self.heads, scan_pieces(step, PIECE, PIECES_FROM))
-        return (yield [Product(self.o, k.gated_out(o, gate, self.norm, False, self.eps, self.build.dtype))])[0]
+        y = k.gated_out(o, gate, self.norm, False, self.eps, self.build.dtype)
+        return (yield [Product(self.o, y)])[0] if few else self.o(y)
 
     def forward(self, x: torch.Tensor, step, site, rows: torch.Tensor | None = None, at: int = 0) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step, site, rows, at))[0]

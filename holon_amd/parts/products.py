@@ -6,12 +6,15 @@ down in. A part may therefore say what it does as a generator (`products`, with 
 `Product`s, is sent their results, and returns what `forward` returns. `drive` runs such parts side by side: in steps of few
 rows it collects what all of them ask for and runs it as one operation (`linear_group`); in other steps, and for parts
 without a generator, one after the other: products of one size in one launch where they fill the chip together
-(`linear_block_group`), each other product as it always was.
+(`linear_block_group`), each other product as it always was. (A list, its products and the generator's way cost the host 3 us, as
+much as two launches of a step that the host bounds: a part that has one or two products to ask for runs them itself in such steps.)
 """
 from __future__ import annotations
 
 import ctypes
 import dataclasses
+import functools
+from collections.abc import Sequence
 from typing import Any
 
 import torch
@@ -25,7 +28,7 @@ BLOCK_ROWS = (129, 3072)      # this many rows: products of one size run togethe
 BLOCK_MOST = 4                # so many of them
 
 
-@dataclasses.dataclass
+@dataclasses.dataclass(slots=True)
 class Product:
     """x W^T of one projection: in the rows' dtype, as `dtype`, or (`relu2`) its max(z, 0)^2."""
 
@@ -42,7 +45,7 @@ class Product:
         return k.relu2(linear(self.x)) if y is None else y
 
 
-@dataclasses.dataclass
+@dataclasses.dataclass(slots=True)
 class Routing:
     """A mixture's router (`moe_router_top`, or with `scale` set `moe_router`): which experts each row of x takes, and their weights."""
 
@@ -74,10 +77,15 @@ class Routing:
                                           and (self.scale is not None or self.top <= self.keep * (e // self.groups)))))
 
 
+@functools.cache
+def _says_products(cls: type) -> bool:
+    owner = next((c for c in cls.__mro__ if "forward" in vars(c) or "products" in vars(c)), None)
+    return owner is not None and "products" in vars(owner)
+
+
 def products_of(part, *args, **kwargs):
     """The part's generator, where the class that says what `forward` does says it as one too; else one that runs `forward`."""
-    owner = next((c for c in type(part).__mro__ if "forward" in vars(c) or "products" in vars(c)), None)
-    if owner is not None and "products" in vars(owner):
+    if _says_products(type(part)):
         return part.products(*args, **kwargs)
 
     def whole():
@@ -86,9 +94,11 @@ def products_of(part, *args, **kwargs):
     return whole()
 
 
-def drive(kernels, rows: int, *parts) -> list:
+def drive(kernels, rows: int, *parts) -> Sequence:
     """What each generator returns."""
     if rows > FEW_ROWS:
+        if len(parts) == 1:
+            return (_by_itself(kernels, parts[0]),)
         return [_by_itself(kernels, part) for part in parts]
     results, asked = [None] * len(parts), {}
 
@@ -109,13 +119,12 @@ def drive(kernels, rows: int, *parts) -> list:
 
 
 def _by_itself(kernels, part):
-    send = None
-    while True:
-        try:
-            asked = part.send(send)
-            send = [p.alone() for p in asked] if len(asked) < BLOCK_MOST else kernels.linear_block_group(asked)
-        except StopIteration as end:
-            return end.value
+    try:
+        asked = part.send(None)
+        while True:
+            asked = part.send([p.alone() for p in asked] if len(asked) < BLOCK_MOST else kernels.linear_block_group(asked))
+    except StopIteration as end:
+        return end.value
 
 
 def linear_group_plain(products: list[Product | Routing]) -> list[torch.Tensor]:

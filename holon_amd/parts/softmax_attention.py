@@ -21,7 +21,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
-from .products import Product, drive
+from .products import FEW_ROWS, Product, drive
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -624,7 +624,8 @@ class SoftmaxAttention(Part):
         held = site.paged[self.state_name]
         view = step.paged[held.group]
         table = getattr(self.position, "table", None)
-        qkv = (yield [Product(self.qkv, x)])[0] if rows is None else rows
+        few = x.shape[0] <= FEW_ROWS
+        qkv = rows if rows is not None else (yield [Product(self.qkv, x)])[0] if few else self.qkv(x)
         if self.whole_norm is not None:
             q = k.whole_norm_prepare(qkv, self.heads, self.kv_heads, self.dim, self.vdim, self.q_norm,
                                      self.k_norm, self.whole_norm, held.pages, view.write_page, view.write_off,
@@ -639,7 +640,7 @@ class SoftmaxAttention(Part):
         out = attend(k, q, held, view, step, self.kv_heads, self.vdim, sink, self.scale,
                      self.sees, self.softcap, (self.r1, self.r2) if self.distance_bias else None, self.keep_first,
                      head_gate=gates)
-        out, = yield [Product(self.o, out)]
+        out = (yield [Product(self.o, out)])[0] if few else self.o(out)
         return k.add_bias(out, self.o_bias) if self.has_o_bias and add_row else out
 
     def forward(self, x: torch.Tensor, step, site, add_row: bool = True, rows: torch.Tensor | None = None) -> torch.Tensor:
@@ -776,7 +777,8 @@ class LatentAttention(Part):
                              "another run's")
         held = site.paged[self.state_name]
         view = step.paged[held.group]
-        both, = yield [Product(self.down, x)]
+        few = t <= FEW_ROWS
+        both = (yield [Product(self.down, x)])[0] if few else self.down(x)
         if self.q_rank == 0:                      # norm, rotation and the cache write in one kernel
             table = getattr(self.position, "table", None)
             if self.own_kv:
@@ -797,7 +799,7 @@ class LatentAttention(Part):
                 c = self.dkv_norm(both[:, self.q_rank:].contiguous()).view(t, 1, self.kv_rank)
                 k.kv_write(c, c, held.pages.view(-1, 2, 1, view.page_size * self.kv_rank), view.write_page,
                            view.write_off, view.page_size)
-            uq, = yield [Product(self.uq, cq)]
+            uq = (yield [Product(self.uq, cq)])[0] if few else self.uq(cq)
             q = k.head_linear(uq.view(t, self.heads, self.dim), self.uk_t)
         sink = self.sink if self.has_sink else None
         if self.entries == 1:
@@ -808,7 +810,8 @@ class LatentAttention(Part):
                            ).view(t, self.heads, self.width)
         gate = both[:, self.gate_at: self.gate_at + self.heads * self.vdim] if self.has_gate else None
         out = k.head_linear(mixed, self.uv_h, gate=gate) if gate is not None else k.head_linear(mixed, self.uv_h)
-        return (yield [Product(self.o, out.view(t, self.heads * self.vdim))])[0]
+        out = out.view(t, self.heads * self.vdim)
+        return (yield [Product(self.o, out)])[0] if few else self.o(out)
 
     def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]

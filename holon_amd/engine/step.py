@@ -26,8 +26,9 @@ from .batch import PagedView, Step, StepRow
 BUCKETS = (1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256)    # core/holon/core/executor.py:28
 LEN_BUCKET_MIN = 1024
 LEN_BUCKET_SHORT = 256        # rows up to here have a bucket of their own in steps of up to 16: an attention kernel takes their keys in one
-                              # block and needs no merge, one row over 100 keys 7.9 us in place of 6.3 + 3.9 at heads of 128, 12.5 in place of 9.6 + 4.0 at 256 (not
-                              # for a model whose sums keep their order, `HipKernels.configured`: the launch's shape decides it)
+                              # block and needs no merge. One row over 100 keys, in one block against sixteen and a merge, us: 5.6 | 7.5 at
+                              # 16 heads of 128, 7.6 | 9.1 at 256; over 250 keys 6.8 | 7.5 and 9.9 | 9.0 (not for a model whose sums keep
+                              # their order, `HipKernels.configured`: the launch's shape decides it)
 
 
 @dataclasses.dataclass

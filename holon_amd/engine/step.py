@@ -25,10 +25,6 @@ from .batch import PagedView, Step, StepRow
 
 BUCKETS = (1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256)    # core/holon/core/executor.py:28
 LEN_BUCKET_MIN = 1024
-LEN_BUCKET_SHORT = 256        # rows up to here have a bucket of their own in steps of up to 16: an attention kernel takes their keys in one
-                              # block and needs no merge. One row over 100 keys, in one block against sixteen and a merge, us: 5.6 | 7.5 at
-                              # 16 heads of 128, 7.6 | 9.1 at 256; over 250 keys 6.8 | 7.5 and 9.9 | 9.0 (not for a model whose sums keep
-                              # their order, `HipKernels.configured`: the launch's shape decides it)
 
 
 @dataclasses.dataclass
@@ -254,7 +250,7 @@ class StepRunner:
         n = len(checked[0])
         bucket = next(b for b in BUCKETS if b >= n)
         slots, starts, counts, tokens, _, take = self._padded(checked, bucket - n)
-        len_bucket = _len_bucket(int((starts + counts).max()), bucket <= 16 and not getattr(self.kernels, "settled", False))
+        len_bucket = _len_bucket(int((starts + counts).max()))
         arrays, facts = self._arrays(slots, starts, counts, tokens, take)
         facts["max_decode_len"] = len_bucket       # launch shapes are the bucket's, whatever the rows' lengths
         key = (bucket, len_bucket)
@@ -283,9 +279,7 @@ class StepRunner:
         return g.logits[:n]
 
 
-def _len_bucket(longest: int, short: bool = True) -> int:
-    if short and longest <= LEN_BUCKET_SHORT:
-        return LEN_BUCKET_SHORT
+def _len_bucket(longest: int) -> int:
     return max(LEN_BUCKET_MIN, 1 << (max(longest, 1) - 1).bit_length())
 
 

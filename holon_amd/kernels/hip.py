@@ -767,7 +767,7 @@ class HipKernels:
                            _ptr(sink), *mod, self._stream())
             if rows.n_decode:
                 span = rows.max_decode_len if not window else min(rows.max_decode_len, abs(window) + 31)
-                splits, per, waves = self.decode_splits(rows.n_decode * hkv * ((hq // hkv + 15) // 16), span, d, one_block=not self.settled)
+                splits, per, waves = self.decode_splits(rows.n_decode * hkv * ((hq // hkv + 15) // 16), span, d)
                 part_o, part_ml = self._decode_parts(rows.n_decode * hq * (splits // waves), d, q.device)
                 self._call(self.lib.holon_attention_decode_mod_bf16, *common, rows.decode_rows.data_ptr(),
                            rows.n_decode, rows.max_decode_len, hq, hkv, d, page_size, float(scale), int(window),
@@ -784,7 +784,7 @@ class HipKernels:
                            _ptr(sink), self._stream())
             if rows.n_decode:
                 span = rows.max_decode_len if not window else min(rows.max_decode_len, abs(window) + 31)
-                splits, per, waves = self.decode_splits(rows.n_decode * hkv * ((hq // hkv + 15) // 16), span, d, one_block=not self.settled)
+                splits, per, waves = self.decode_splits(rows.n_decode * hkv * ((hq // hkv + 15) // 16), span, d)
                 part_o, part_ml = self._decode_parts(rows.n_decode * hq * (splits // waves), d, q.device)
                 self._call(self.lib.holon_attention_decode_sink_bf16, *common, rows.decode_rows.data_ptr(),
                            rows.n_decode, rows.max_decode_len, hq, hkv, d, page_size, float(scale), int(window),
@@ -842,7 +842,7 @@ class HipKernels:
                        _ptr(sink), *mod, self._stream())
         if rows.n_decode:
             span = rows.max_decode_len if not window else min(rows.max_decode_len, abs(window) + 31)
-            splits, per, waves = self.decode_splits(rows.n_decode * hkv * ((hq // hkv + 15) // 16), span, d, one_block=not self.settled)
+            splits, per, waves = self.decode_splits(rows.n_decode * hkv * ((hq // hkv + 15) // 16), span, d)
             part_o, part_ml = self._decode_parts(rows.n_decode * hq * (splits // waves), d, q.device)
             self._call(self.lib.holon_attention_decode_shared_bf16, *common, rows.decode_rows.data_ptr(),
                        rows.n_decode, rows.max_decode_len, hq, hkv, d, page_size, float(scale), int(window),
@@ -907,7 +907,7 @@ class HipKernels:
 
     @staticmethod
     def decode_splits(pairs: int, span: int, head_dim: int = 128, target_waves: int = 2048, min_keys: int = 64,
-                      blocks: int | None = None, one_block: bool = True) -> tuple[int, int, int]:
+                      blocks: int | None = None) -> tuple[int, int, int]:
         """How a decode row's keys are cut over waves: (splits, keys per split, waves a block). `pairs`: (row, kv head)
         tiles in the launch. Enough waves to fill the GPU but at least `min_keys` keys each (a multiple of 32); the
         waves of a block combine their partials through LDS, so as many of a row's splits share a block as leave
@@ -921,8 +921,6 @@ class HipKernels:
         per = max(min_keys, -(-span // want))
         per = -(-per // 32) * 32
         splits = max(1, -(-span // per))
-        if splits <= 4 and per == min_keys and one_block:      # no merge: fewer waves at work cost less than a kernel
-            return splits, per, splits
         cap = max(1, min(8, (64 * 1024 // 4) // (16 * head_dim + 32) + 1))
         outer = min(splits, max(1, -(-blocks // max(1, pairs))))
         waves = min(cap, -(-splits // outer))

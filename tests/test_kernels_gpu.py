@@ -1840,7 +1840,7 @@ def test_products_of_many_rows_in_one_launch(hip, m, n, k):
 @pytest.mark.parametrize("softcap", [0.0, 20.0])
 @pytest.mark.parametrize("geometry", [(8, 2, 64), (16, 4, 128), (16, 1, 256)])
 def test_decode_rows_of_every_last_block(hip, geometry, softcap):
-    """Decode rows of 1 to 64 keys, NaN in every cache slot behind them, alone in their block and over its four waves: each row within its
+    """Decode rows of 1 to 64 keys, NaN in every cache slot behind them, in one wave and over four: each row within its
     budget of the plain form in float64, and bit for bit what it is with zeros there."""
     heads, kv_heads, d = geometry
     page, dtype, rows = 16, torch.bfloat16, [(n, 1) for n in range(64)]

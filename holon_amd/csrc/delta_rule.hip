@@ -1,5 +1,5 @@
 // The gated delta rule over prompt rows, in blocks of 16 tokens on the float32 matrix cores. Token by token (recurrent.hip, which
-// keeps decode rows) the rule is S <- g_t S; u_t = beta_t (v_t - S^T k_t); S <- S + k_t u_t^T; o_t = S^T q_t. Over a block that
+// keeps decode rows and short portions, also where a step has longer rows beside them) the rule is S <- g_t S; u_t = beta_t (v_t - S^T k_t); S <- S + k_t u_t^T; o_t = S^T q_t. Over a block that
 // starts from S0, with G_t the product of g up to t, f(t, i) the product of g behind i up to t and E_i = f(last, i):
 //   u   = T R,  R_t = beta_t v_t - beta_t G_t S0^T k_t,  T = (I + L)^-1,  L[t][i] = beta_t f(t, i) k_t . k_i below the diagonal
 //   o_t = G_t S0^T q_t + sum over i <= t of (f(t, i) q_t . k_i) u_i
@@ -42,12 +42,15 @@ struct DeltaRows {
   const int32_t* query_start;
   int heads, kv_heads, dim, vdim;
   int piece;                   // tokens a piece, a multiple of 16
+  const int32_t* piece_of;     // [rows]: the same row by row, 0: the row goes token by token; null: `piece` for all
   const int32_t* base;         // [rows]: the number of row b's first piece among all pieces of the step
   float* blocks;               // [T / 16 + rows, H, BLOCK_FLOATS]
   float* a;                    // [pieces, H, KD, KD], the key size padded with zeros
   float* sin;                  // [pieces, H, D, V]: B, then the state behind the piece; a row's last piece's place: the state it starts from
 };
 
+__device__ __forceinline__ int piece_tokens(const DeltaRows& r, int b) { return r.piece_of ? r.piece_of[b] : r.piece; }
+__device__ __forceinline__ int pieces_of(int tokens, int piece) { return piece > 0 ? (tokens + piece - 1) / piece : 0; }
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
 __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -73,7 +76,7 @@ __global__ void __launch_bounds__(THREADS) delta_blocks_kernel(DeltaRows r) {
   __shared__ __attribute__((aligned(16))) double below[NW][TB][TB];
   const int b = blockIdx.x, h = blockIdx.y, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, g4 = lane / 16, c = lane % 16;
   const int lo = r.query_start[b], hi = r.query_start[b + 1], t0 = lo + (blockIdx.z * NW + wave) * TB;
-  if (t0 >= hi) return;                                    // (waves of a block share nothing)
+  if (t0 >= hi || piece_tokens(r, b) == 0) return;         // (waves of a block share nothing)
   const int n = min(TB, hi - t0), hk = h / (r.heads / r.kv_heads);
   const bool in = c < n;
   const int64_t row = ((int64_t)(t0 + min(c, n - 1)) * r.kv_heads + hk) * r.dim;
@@ -143,10 +146,10 @@ __global__ void __launch_bounds__(THREADS, KD <= 128 ? 2 : 1) delta_chain_kernel
   const int columns = OUT ? vdim : vdim + dim, col_blocks = (columns + 16 * NW - 1) / (16 * NW);
   const int piece = blockIdx.z / col_blocks, j = (blockIdx.z % col_blocks) * 16 * NW + 16 * wave + c;      // this lane's column
   int lo = r.query_start[b], hi = r.query_start[b + 1];
-  const int pieces = (hi - lo + r.piece - 1) / r.piece;
+  const int tokens = piece_tokens(r, b), pieces = pieces_of(hi - lo, tokens);
   if (piece >= pieces || (!OUT && piece == pieces - 1)) return;
-  lo += piece * r.piece;
-  hi = min(hi, lo + r.piece);
+  lo += piece * tokens;
+  hi = min(hi, lo + tokens);
   const int64_t piece_no = r.base[b] + piece;
   float* held = state + ((int64_t)r.slots[b] * r.heads + h) * dim * vdim;
   const float* before = pieces == 1 ? held : r.sin + ((piece_no + (piece == 0 ? pieces : 0) - 1) * r.heads + h) * dim * vdim;
@@ -305,7 +308,7 @@ __global__ void __launch_bounds__(THREADS) delta_walk_kernel(const float* __rest
   __shared__ __attribute__((aligned(16))) float st[2][16 * SP];
   const int b = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * 16, wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, g4 = lane / 16, c = lane % 16;
   const int dim = r.dim, vdim = r.vdim, j = j0 + c;
-  const int pieces = (r.query_start[b + 1] - r.query_start[b] + r.piece - 1) / r.piece;
+  const int pieces = pieces_of(r.query_start[b + 1] - r.query_start[b], piece_tokens(r, b));
   if (pieces < 2) return;
   const float* held = state + ((int64_t)r.slots[b] * r.heads + h) * dim * vdim;
   const bool carried = r.starts[b] > 0;
@@ -377,14 +380,14 @@ void chain(int pass, dim3 grid, hipStream_t s, const void* qkv, int stride, int 
 }
 }  // namespace
 
-// The rows of holon_delta_scan that are not single tokens (it has checked the arguments).
+// The rows of holon_delta_scan that `piece_of` gives pieces (null: every row; it has checked the arguments).
 int holon_delta_scan_pieces(const float* qn, const float* kn, const void* qkv, int qkv_stride, int v_offset, const float* beta,
                             const float* g, float* state, float* out, const int32_t* slots, const int32_t* starts,
                             const int32_t* query_start, int rows, int heads, int kv_heads, int dim, int vdim, int dtype,
-                            int piece_tokens, int max_pieces, const int32_t* piece_base, float* blocks, float* a, float* sin,
-                            void* stream) {
+                            int piece_tokens, int max_pieces, const int32_t* piece_base, const int32_t* piece_of, float* blocks,
+                            float* a, float* sin, void* stream) {
   hipStream_t s = (hipStream_t)stream;
-  const DeltaRows r{qn, kn, beta, g, slots, starts, query_start, heads, kv_heads, dim, vdim, piece_tokens, piece_base, blocks, a, sin};
+  const DeltaRows r{qn, kn, beta, g, slots, starts, query_start, heads, kv_heads, dim, vdim, piece_tokens, piece_of, piece_base, blocks, a, sin};
   const bool whole = dim % 4 == 0 && (((uintptr_t)qn | (uintptr_t)kn) & 15) == 0;
   const int64_t groups = ((int64_t)max_pieces * piece_tokens / TB + NW - 1) / NW;
   const int out_cols = (vdim + 16 * NW - 1) / (16 * NW), all_cols = (vdim + dim + 16 * NW - 1) / (16 * NW);

@@ -261,7 +261,8 @@ template <int KD, int ARRAYS> struct ScanChunk {
 };
 
 // Per (row, head): S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q. Lane 8 c + p owns rows
-// p KD/8 .. (p + 1) KD/8 - 1 of column c of S. (Longer rows go in blocks of tokens on the matrix cores: delta_rule.hip.)
+// p KD/8 .. (p + 1) KD/8 - 1 of column c of S. (Longer rows go in blocks of tokens on the matrix cores: delta_rule.hip; `piece_of`, nullable,
+// says which rows do.)
 template <int KD, typename T>
 __global__ void __launch_bounds__(WAVE) delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
                                                           const T* __restrict__ qkv, int qkv_stride, int v_offset,
@@ -269,13 +270,15 @@ __global__ void __launch_bounds__(WAVE) delta_scan_kernel(const float* __restric
                                                           float* __restrict__ state, float* __restrict__ out,
                                                           const int32_t* __restrict__ slots,
                                                           const int32_t* __restrict__ starts,
-                                                          const int32_t* __restrict__ query_start, int heads,
-                                                          int kv_heads, int dim, int vdim) {
+                                                          const int32_t* __restrict__ query_start,
+                                                          const int32_t* __restrict__ piece_of, int heads, int kv_heads, int dim,
+                                                          int vdim) {
   constexpr int KQ = KD / SCAN_PARTS, TC = ScanChunk<KD, 2>::kTokens, N = TC * KD, PER = (N + WAVE - 1) / WAVE;
   constexpr int VPER = (TC * SCAN_COLS + WAVE - 1) / WAVE;
   __shared__ __attribute__((aligned(16))) float ks[2][N], qs[2][N];
   __shared__ float vs[2][TC * SCAN_COLS], gs[2][TC], bs[2][TC];
   const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  if (piece_of && piece_of[b] > 0) return;               // (uniform over the block)
   const int col_block = blockIdx.z;
   const int part = lane % SCAN_PARTS, col = lane / SCAN_PARTS, j = col_block * SCAN_COLS + col;
   const int hk = h / (heads / kv_heads);
@@ -657,10 +660,10 @@ extern "C" int holon_delta_prepare(const void* qkv, const void* ab, const float*
 template <typename T, int KD>
 static void launch_delta(dim3 grid, hipStream_t s, const float* qn, const float* kn, const void* qkv,
                          int stride, int voff, const float* beta, const float* g, float* state, float* out,
-                         const int32_t* slots, const int32_t* starts, const int32_t* qs, int heads, int kv_heads, int dim,
-                         int vdim) {
+                         const int32_t* slots, const int32_t* starts, const int32_t* qs, const int32_t* piece_of, int heads,
+                         int kv_heads, int dim, int vdim) {
   delta_scan_kernel<KD, T><<<grid, WAVE, 0, s>>>(qn, kn, (const T*)qkv, stride, voff, beta, g, state, out, slots,
-                                                    starts, qs, heads, kv_heads, dim, vdim);
+                                                    starts, qs, piece_of, heads, kv_heads, dim, vdim);
 }
 
 #define BY_KEY_SIZE(dim, CALL)                                  \
@@ -678,14 +681,14 @@ static void launch_delta(dim3 grid, hipStream_t s, const float* qn, const float*
 int holon_delta_scan_pieces(const float* qn, const float* kn, const void* qkv, int qkv_stride, int v_offset, const float* beta,
                             const float* g, float* state, float* out, const int32_t* slots, const int32_t* starts,
                             const int32_t* query_start, int rows, int heads, int kv_heads, int dim, int vdim, int dtype,
-                            int piece_tokens, int max_pieces, const int32_t* piece_base, float* blocks, float* a, float* sin,
-                            void* stream);
+                            int piece_tokens, int max_pieces, const int32_t* piece_base, const int32_t* piece_of, float* blocks,
+                            float* a, float* sin, void* stream);
 
 extern "C" int holon_delta_scan(const float* qn, const float* kn, const void* qkv, int qkv_stride, int v_offset,
                                 const float* beta, const float* g, float* state, float* out, const int32_t* slots,
                                 const int32_t* starts, const int32_t* query_start, int rows, int heads, int kv_heads,
                                 int dim, int vdim, int state_slots, int dtype, int piece_tokens, int max_pieces,
-                                const int32_t* piece_base, float* blocks, float* a, float* sin, void* stream) {
+                                const int32_t* piece_base, const int32_t* piece_of, float* blocks, float* a, float* sin, void* stream) {
   HOLON_CHECK(rows >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "delta_scan: %d/%d heads", heads, kv_heads);
   HOLON_CHECK(dim > 0 && dim <= 256 && vdim > 0 && vdim <= 1024, "delta_scan: key size %d (at most 256), value size %d "
               "(at most 1024)", dim, vdim);
@@ -695,13 +698,17 @@ extern "C" int holon_delta_scan(const float* qn, const float* kn, const void* qk
                                     (max_pieces == 1 || (a && sin)) && (((uintptr_t)blocks | (uintptr_t)a) & 15) == 0),
               "delta_scan: rows in pieces of %d tokens (a multiple of 16) need the pieces' table and workspace", piece_tokens);
   if (rows == 0) return 0;
-  if (piece_tokens > 0)
-    return holon_delta_scan_pieces(qn, kn, qkv, qkv_stride, v_offset, beta, g, state, out, slots, starts, query_start, rows, heads,
-                                   kv_heads, dim, vdim, dtype, piece_tokens, max_pieces, piece_base, blocks, a, sin, stream);
+  if (piece_tokens > 0) {
+    const int failed = holon_delta_scan_pieces(qn, kn, qkv, qkv_stride, v_offset, beta, g, state, out, slots, starts, query_start, rows,
+                                               heads, kv_heads, dim, vdim, dtype, piece_tokens, max_pieces, piece_base, piece_of, blocks,
+                                               a, sin, stream);
+    if (failed || !piece_of) return failed;
+  }
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid(rows, heads, (vdim + SCAN_COLS - 1) / SCAN_COLS);      // a wave for every 8 value columns
   BY_DTYPE(dtype, BY_KEY_SIZE(dim, (launch_delta<T, KD>(grid, s, qn, kn, qkv, qkv_stride, v_offset, beta, g, state, out, slots,
-                                                         starts, query_start, heads, kv_heads, dim, vdim))));
+                                                         starts, query_start, piece_tokens > 0 ? piece_of : nullptr, heads, kv_heads,
+                                                         dim, vdim))));
   HOLON_LAUNCH_OK();
   return 0;
 }

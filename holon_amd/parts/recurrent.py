@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 
+import numpy as np
 import torch
 
 from ..kernels.registry import KernelOp, register_kernel
@@ -21,9 +22,9 @@ from .products import FEW_ROWS, Product, drive
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
 MAX_KEY_DIM = 256             # the scans keep a column of D values in registers
-# The delta rule's rows in blocks of 16 tokens, from a longest row of this many (16 heads of 128 by 128, us, against token by token:
-# 32 tokens 22 / 24, 64 28 / 41, 300 70 / 170). The 32-bit path keeps the token's own order of sums in shorter steps, so that its logits do
-# not depend on how a prompt of up to that many tokens is cut.
+# The delta rule's rows of this many tokens and more go in blocks of 16 tokens (16 heads of 128 by 128, us, against token by token:
+# 32 tokens 22 / 24, 64 28 / 41, 300 70 / 170), whatever other rows a step has. The 32-bit path keeps the token's own order of sums in
+# shorter rows, so that the rule's results do not depend on how a prompt is cut into portions below that many tokens.
 DELTA_FROM = {torch.bfloat16: 32, torch.float32: 512}
 
 
@@ -73,7 +74,7 @@ def _delta_prepare_hip(launch, qkv, ab, a_log, dt_bias, heads, kv_heads, dim, vd
 def delta_scan_plain(qn, kn, qkv, beta, g, state, slots, starts, query_start, n_rows, heads, vdim, pieces=None):
     """Per row and head, along the row's tokens: S <- g S; u = beta (v - S^T k); S <- S + k u^T; o = S^T q.
     qn, kn [T, G, D] float32; v is the last H V columns of qkv; state [slots, H, D, V] float32, read unless the row
-    starts at position 0 and written back. -> o [T, H, V] float32. `pieces` as for `memory_scan`."""
+    starts at position 0 and written back. -> o [T, H, V] float32. `pieces` as for `memory_scan`, or what `delta_pieces` answers."""
     t, kv_heads, dim = qn.shape
     v = qkv[:, qkv.shape[1] - heads * vdim:].float().view(t, heads, vdim)
     out = torch.empty((t, heads, vdim), dtype=torch.float32, device=qn.device)
@@ -102,16 +103,16 @@ def _delta_scan_hip(launch, qn, kn, qkv, beta, g, state, slots, starts, query_st
     _need(dim <= MAX_KEY_DIM and vdim <= 1024, f"delta_scan: key size {dim} (at most {MAX_KEY_DIM}), value size {vdim} "
           "(at most 1024)")
     out = torch.empty((t, heads, vdim), dtype=torch.float32, device=qn.device)
-    extra = (0, 0, None, None, None, None)
+    extra = (0, 0, None, None, None, None, None)
     if pieces is not None:
-        tokens, most, base, total = pieces
+        tokens, most, base, total, each = *pieces, *(None,) * (5 - len(pieces))
         f32 = dict(dtype=torch.float32, device=qn.device)
         blocks, a, sin = torch.empty((t // 16 + n_rows, heads, 576), **f32), None, None
         if most > 1:
             kd = next(size for size in (32, 64, 128, 256) if dim <= size)
             a = torch.empty((total, heads, kd, kd), **f32)
             sin = torch.empty((total, heads, dim, vdim), **f32)
-        extra = (tokens, most, base.data_ptr(), blocks.data_ptr(), _ptr(a), _ptr(sin))
+        extra = (tokens, most, base.data_ptr(), _ptr(each), blocks.data_ptr(), _ptr(a), _ptr(sin))
     launch(qn.data_ptr(), kn.data_ptr(), qkv.data_ptr(), qkv.shape[1], qkv.shape[1] - heads * vdim, beta.data_ptr(),
            g.data_ptr(), state.data_ptr(), out.data_ptr(), slots.data_ptr(), starts.data_ptr(), query_start.data_ptr(),
            n_rows, heads, kv_heads, dim, vdim, state.shape[0], _DT[qkv.dtype], *extra)
@@ -249,18 +250,30 @@ def _memory_scan_hip(launch, r, k, v, w, u, state, slots, starts, query_start, n
 
 
 def delta_pieces(step, columns: int, dtype: torch.dtype):
-    """`scan_pieces` for the delta rule over `columns` value columns of all heads: pieces of 256 tokens, or of 512 where no row is
-    longer or the step's columns fill the GPU by themselves (the pass that makes pieces independent runs on D + V columns:
-    16 heads of 128 by 128, us in pieces of 256 / 512: one row of 300 tokens 104 / 70, of 1,024 120 / 177, of 2,048 159 / 188,
-    of 4,000 261 / 238, eight of 500 173 / 117, four of 700 to 1,400 299 / 259)."""
-    full = step.rows.max_chunk_query <= 512 or step.n_tokens * columns > 2560 * 2048
-    return scan_pieces(step, 512 if full else 256, DELTA_FROM[dtype])
+    """What `scan_pieces` answers, for the delta rule over `columns` value columns of all heads, and each row's own tokens a piece [rows]
+    int32 on the device (None: the first number for all). A row's length alone decides its form, so that its sums do not depend on what
+    else a step holds: below `DELTA_FROM` token by token, else pieces of 256 tokens, or of 512 where the row is no longer or fills the GPU
+    by itself (the pass that makes pieces independent runs on D + V columns: 16 heads of 128 by 128, us in pieces of 256 / 512: one
+    row of 300 tokens 104 / 70, of 1,024 120 / 177, of 2,048 159 / 188, of 4,000 261 / 238; four of 700 to 1,400 in a step, which keep the
+    form that one of them has alone, 299 / 259)."""
+    least = DELTA_FROM[dtype]
+    if step.rows.max_chunk_query < least:
+        return None
+    cache = step.__dict__.setdefault("_scan_pieces", {})
+    key = ("delta", least, columns)
+    if key not in cache:
+        n = step.h_counts.astype("int64")
+        each = np.where(n < least, 0, np.where((n <= 512) | (n * columns > 2560 * 2048), 512, 256))
+        pieces = np.where(each > 0, -(-n // np.maximum(each, 1)), 0)
+        two = torch.from_numpy(np.stack((pieces.cumsum() - pieces, each)).astype("int32")).to(step.slots.device, non_blocking=True)
+        cache[key] = (int(each.max()), int(pieces.max()), two[0], int(pieces.sum()), None if (each == each[0]).all() else two[1])
+    return cache[key]
 
 
 register_kernel(KernelOp("delta_prepare", delta_prepare_plain, "holon_delta_prepare",
                          [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I], _delta_prepare_hip))
 register_kernel(KernelOp("delta_scan", delta_scan_plain, "holon_delta_scan",
-                         [_P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P],
+                         [_P, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P],
                          _delta_scan_hip))
 register_kernel(KernelOp("gated_out", gated_out_plain, "holon_gated_out",
                          [_P, _P, _P, _P, _I, _I, _I, _I, _F, _I, ctypes.c_int64, _I, _P], _gated_out_hip))

@@ -10,6 +10,7 @@ import json
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 import torch
 
@@ -496,3 +497,64 @@ def test_the_delta_rule_in_blocks_of_tokens(heads, kv, dim, vdim, dtype):
             got = run(48, kk, vv)[0]
             assert torch.equal(got[:at], ref[:at]), (at, value)
             assert torch.equal(got.isfinite(), run(0, kk, vv)[0].isfinite()), (at, value)
+
+
+def _step_of(counts, device="cpu"):
+    """What the scans read of a step whose rows have these numbers of tokens."""
+    from types import SimpleNamespace
+    return SimpleNamespace(h_counts=np.array(counts, dtype=np.int32), n_tokens=sum(counts), slots=torch.zeros(1, device=device),
+                           rows=SimpleNamespace(max_chunk_query=max([c for c in counts if c > 1], default=0)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("columns", [64, 2048, 4096])
+def test_a_rows_pieces_do_not_depend_on_the_rows_beside_it(dtype, columns):
+    """`delta_pieces` gives every row of a step the tokens a piece that it has alone (none below the block form's border), and
+    each row's pieces places of their own in order."""
+    from holon_amd.parts.recurrent import DELTA_FROM, delta_pieces
+    least = DELTA_FROM[dtype]
+    counts = [1, 2, least - 1, least, 511, 512, 513, 1281, 2560, 2561, 9000, 1]
+
+    def form(counts):
+        got = delta_pieces(_step_of(counts), columns, dtype)
+        if got is None:
+            return [0] * len(counts), None
+        tokens, most, base, total, each = got
+        return ([tokens] * len(counts) if each is None else each.tolist()), (tokens, most, base.tolist(), total)
+    each, (tokens, most, base, total) = form(counts)
+    assert each == [form([c])[0][0] for c in counts] and all(e in ((256, 512) if c >= least else (0,)) for c, e in zip(counts, each))
+    pieces = [-(-c // e) if e else 0 for c, e in zip(counts, each)]
+    assert (tokens, most, total) == (max(each), max(pieces), sum(pieces)) and base == [sum(pieces[:b]) for b in range(len(counts))]
+    assert form([1, 1, least - 1])[1] is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(2, 1, 32, 64), (1, 1, 128, 72)])
+def test_the_delta_rule_of_a_row_does_not_depend_on_the_rows_beside_it(heads, kv, dim, vdim, dtype):
+    """Rows of one token to several pieces in one step, bit for bit what each of them is alone: below the block form's border, at it,
+    in one piece and in several, carried and not."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    from holon_amd.parts.recurrent import delta_pieces
+    k, dev = load_hip(), torch.device("cuda")
+    gen = torch.Generator().manual_seed(dim)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
+    counts, starts = [1, 20, 31, 32, 300, 511, 600, 1], [9, 0, 4, 1, 0, 2, 3, 0]
+    t, n = sum(counts), len(counts)
+    norm = lambda x: x / x.norm(dim=-1, keepdim=True)                          # noqa: E731
+    qn, kn = norm(rn(t, kv, dim)), norm(rn(t, kv, dim))
+    qkv = rn(t, 2 * kv * dim + heads * vdim).to(dtype)
+    beta, g = torch.rand(t, heads, generator=gen).to(dev), torch.exp(-rn(t, heads).abs())
+    state = rn(n, heads, dim, vdim)
+    together, lo = state.clone(), 0
+    out = k.delta_scan(qn, kn, qkv, beta, g, together, i32(list(range(n))), i32(starts), i32([sum(counts[:b]) for b in range(n + 1)]), n,
+                       heads, vdim, delta_pieces(_step_of(counts, dev), heads * vdim, dtype))
+    for b, c in enumerate(counts):
+        alone, own = state.clone(), slice(lo, lo + c)
+        got = k.delta_scan(qn[own].contiguous(), kn[own].contiguous(), qkv[own].contiguous(), beta[own].contiguous(), g[own].contiguous(),
+                           alone, i32([b]), i32([starts[b]]), i32([0, c]), 1, heads, vdim,
+                           delta_pieces(_step_of([c], dev), heads * vdim, dtype))
+        assert torch.equal(got, out[own]) and torch.equal(alone[b], together[b]), (b, c)
+        lo += c

@@ -236,7 +236,8 @@ __global__ void __launch_bounds__(THREADS, KD <= 128 ? 2 : 1) delta_chain_kernel
       from = d0 ? from + fs : fs;
     }
     // A row of R or u that is not finite belongs into its own token's and the later ones': the products, where it would meet the
-    // earlier ones' zeros, go without it, and it is added below them.
+    // earlier ones' zeros, go without it, and it is added below them: T from the row behind its own, as its diagonal is left out of `m` and
+    // R itself is added to u (an infinity stays one, for its token's u and for the state), and never in rows behind the portion's end.
     const auto lower = [&](const f32x4& a, const f32x4& x, int matrix) {
       f32x4 clean, sum = {0.f, 0.f, 0.f, 0.f};
       bool all_finite = true;
@@ -256,7 +257,7 @@ __global__ void __launch_bounds__(THREADS, KD <= 128 ? 2 : 1) delta_chain_kernel
           const float val = __shfl(mine, (n / 4) * 16 + c, WAVE);
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (!finite(val) && n <= 4 * g4 + i) sum[i] += m[(4 * g4 + i) * TB + n] * val;
+            if (!finite(val) && n < 4 * g4 + i + matrix && t0 + 4 * g4 + i < hi) sum[i] += m[(4 * g4 + i) * TB + n] * val;
         }
       }
       return sum;

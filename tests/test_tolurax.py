@@ -558,3 +558,36 @@ def test_the_delta_rule_of_a_row_does_not_depend_on_the_rows_beside_it(heads, kv
                            delta_pieces(_step_of([c], dev), heads * vdim, dtype))
         assert torch.equal(got, out[own]) and torch.equal(alone[b], together[b]), (b, c)
         lo += c
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(2, 1, 32, 64), (1, 1, 6, 5), (1, 1, 128, 72)])
+def test_an_infinite_value_of_a_rows_last_token_is_infinite_in_its_state(heads, kv, dim, vdim):
+    """`delta_scan` in blocks of tokens, a row's last token with a value of infinity: its column of the state is what the
+    token-by-token scan leaves there (infinities of the key's signs), every other column what it is without it; rows that end with a
+    block, inside one, and of one token."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    k, dev = load_hip(), torch.device("cuda")
+    gen = torch.Generator().manual_seed(dim)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
+    counts = [1, 16, 33, 47]
+    t, n = sum(counts), len(counts)
+    base = [sum(counts[:b]) for b in range(n + 1)]
+    norm = lambda x: x / x.norm(dim=-1, keepdim=True)                          # noqa: E731
+    qn, kn = norm(rn(t, kv, dim)), norm(rn(t, kv, dim))
+    qkv, beta, g = rn(t, 2 * kv * dim + heads * vdim), 0.1 + torch.rand(t, heads, generator=gen).to(dev), torch.exp(-rn(t, heads).abs())
+    state, at = rn(n, heads, dim, vdim), 2 * kv * dim + 3                      # (the first head's column 3)
+    for sign in (1.0, -1.0):
+        val = qkv.clone()
+        val[[b - 1 for b in base[1:]], at] = sign * float("inf")
+        after = []
+        for v, pieces in ((val, None), (val, (48, 1, i32([0, 1, 2, 3]), 4)), (qkv, (48, 1, i32([0, 1, 2, 3]), 4))):
+            held = state.clone()
+            k.delta_scan(qn, kn, v, beta, g, held, i32(list(range(n))), i32([1] * n), i32(base), n, heads, vdim, pieces)
+            after.append(held)
+        tokens, blocks, without = after
+        assert torch.equal(blocks[:, 0, :, 3], tokens[:, 0, :, 3]) and blocks[:, 0, :, 3].isinf().all()
+        blocks[:, 0, :, 3] = without[:, 0, :, 3]
+        assert torch.equal(blocks, without)

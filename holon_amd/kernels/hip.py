@@ -57,6 +57,26 @@ def glu_block_pays(rows: int, inter: int, hidden: int) -> bool:
     return rows > 128 and rows * inter >= 0.62 * rounds * 256 * 256 * 128
 
 
+def heads_a_block(group: int, head_dim: int) -> int:
+    """How many heads of a group share a block of the general attention kernel (as its launch decides)."""
+    return 1 if head_dim > 256 else next(n for n in (4, 2, 1) if group % n == 0)
+
+
+def general_split_pays(blocks: int, head_dim: int, span: int) -> bool:
+    """Whether decode rows of the general attention kernel, in `blocks` blocks of eight waves (a token and one to four heads) over up to
+    `span` keys, have every wave in a block of its own and a second kernel behind them (the same bits): where the blocks leave compute units
+    idle and the waves have enough to do that the second kernel, 4.7 us, and the partial sums' way through memory are made up for. By
+    what there is in flight (`blocks` times `head_dim`) and the keys. Measured, us, whole | split, float32 unless noted, by blocks x head size:
+    16 x 128 (four heads a block) over 128 / 192 / 256 / 512 keys 15.8 | 15.6, 16.3 | 15.7, 17.2 | 15.7, 19.6 | 15.8; 64 x 128 256 / 512 / 1,024 keys
+    17.5 | 19.6, 23.7 | 20.0, 48 | 32; 128 x 128 22 | 24, 30 | 27, 50 | 42; 256 x 128 25 | 44, 32 | 48, 59 | 82; one head a block 24 x 128
+    192 / 256 / 512 10.5 | 10.7, 11.7 | 10.7, 12.9 | 10.8, 96 x 128 256 / 512 12.0 | 12.2, 13.6 | 12.7, 192 x 128 12.4 | 22, 18 | 21, 36 | 39; 32 x 64
+    (four heads) 192 / 256 / 512 12.0 | 11.9, 12.2 | 11.5, 14.7 | 12.0, 128 x 64 256 / 512 12.4 | 13.3, 15.4 | 13.4, 256 x 64 512 / 1,024 16.2 | 18.4,
+    27.5 | 27.6; 4,544 x 64 (71 heads on one) 98 | 127, 181 | 225; 16 x 256 192 / 256 / 512 23.7 | 23.8, 24.1 | 23.7, 28.6 | 23.8, 32 x 256 256 / 512
+    24 | 32, 34 | 32; 16 x 512 39 | 41, 53 | 41, 64 x 512 39 | 61, 55 | 61; bfloat16 48 x 96 192 / 512 / 1,024 10.4 | 10.1, 10.9 | 9.9, 18.5 | 14.9."""
+    few = blocks * head_dim <= 4096
+    return blocks <= 128 and blocks * head_dim <= 16384 and span > (128 if few and 64 < head_dim <= 128 else 256 if few else 384)
+
+
 class HipKernels:
     name = "hip-gfx950"
     settled = False           # see `configured`
@@ -796,7 +816,7 @@ class HipKernels:
                               f"not at head_dim {d}, page {page_size}, {q.dtype}")
         general, parts = self.lib.holon_attention_generic, ()
         span = min(rows.max_decode_len, abs(window)) if window else rows.max_decode_len
-        if rows.n_chunk == 0 and t * hkv <= 64 and span > 128:      # decode rows that leave compute units idle: a wave a block
+        if rows.n_chunk == 0 and general_split_pays(t * hq // heads_a_block(hq // hkv, d), d, span):      # a wave a block
             f64 = torch.float64 if q.dtype == torch.float32 else torch.float32
             general, parts = self.lib.holon_attention_generic_split, (
                 torch.empty((t, hq, 8, d), dtype=f64, device=q.device), torch.empty((t, hq, 8, 2), dtype=torch.float32, device=q.device))

@@ -1891,3 +1891,26 @@ def test_stream_rows_of_one_type_are_those_of_several(hip, dtype, dim):
                     got.append([v for v in y if v is not None])
                 for one in got[1:]:
                     assert all(torch.equal(a, b) for a, b in zip(one, got[0], strict=True)), (len(terms), added is None, second is None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,kv,dim,t,longest,split", [(16, 4, 128, 4, 128, False), (16, 4, 128, 4, 129, True), (16, 4, 128, 16, 384, False),
+                                                          (16, 4, 128, 16, 385, True), (71, 1, 72, 2, 700, False), (71, 1, 72, 1, 385, True),
+                                                          (12, 2, 96, 33, 700, False), (8, 2, 512, 16, 700, False), (8, 2, 512, 2, 385, True)])
+def test_decode_rows_at_the_borders_of_a_wave_a_block(hip, dtype, heads, kv, dim, t, longest, split, monkeypatch):
+    """`paged_attention` by the general kernel on both sides of the rule that gives every wave a block, by the blocks that a step really
+    has: the form named, within its budget of the plain form, and no bigger a workspace than a few MB."""
+    page = 5 if dtype == torch.bfloat16 else 16
+    rows = [(longest - 1 - i * 7 % 60, 1) for i in range(t)]
+    q, pages, table, attn = _paged_case(rows, heads, kv, dim, page, dtype, seed=230, max_seqs=t)
+    called, made, empty = [], [], torch.empty
+    call = hip._call
+    with monkeypatch.context() as m:
+        m.setattr(hip, "_call", lambda fn, *a: called.append(fn.__name__) or call(fn, *a))
+        m.setattr(torch, "empty", lambda *a, **kw: made.append(empty(*a, **kw)) or made[-1])
+        got = hip.paged_attention(q, pages, table, attn, page, dim ** -0.5, 0)
+    assert called == ["holon_attention_generic_split" if split else "holon_attention_generic"]
+    assert sum(x.numel() * x.element_size() for x in made) <= 5 << 20 and (split or not made)
+    want = PLAIN.paged_attention(q.double(), pages.double(), table, attn, page, dim ** -0.5, 0)
+    assert H.op_budget_usage(got, want, dtype, dim + longest) <= 1

@@ -14,6 +14,7 @@ from __future__ import annotations
 import ctypes
 import dataclasses
 import functools
+import inspect
 from collections.abc import Sequence
 from typing import Any
 
@@ -79,8 +80,10 @@ class Routing:
 
 @functools.cache
 def _says_products(cls: type) -> bool:
-    owner = next((c for c in cls.__mro__ if "forward" in vars(c) or "products" in vars(c)), None)
-    return owner is not None and "products" in vars(owner)
+    """Whether the class that says what a call of the part does (the nearest that has `__call__`, `forward` or `products`) says it as a
+    generator too."""
+    owner = next((vars(c) for c in cls.__mro__ if not vars(c).keys().isdisjoint(("__call__", "forward", "products"))), {})
+    return inspect.isgeneratorfunction(owner.get("products"))
 
 
 def products_of(part, *args, **kwargs):

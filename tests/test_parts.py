@@ -692,3 +692,40 @@ def test_a_norm_and_an_embedding_that_implement_only_their_base_class(device, dt
         unregister_part("norm", "test-centred")
         unregister_part("embed", "test-scaled-table")
         unregister_part("test-family", "thing")
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("rows", [3, 40])
+def test_a_part_that_overrides_how_it_is_called_is_called(device, rows):
+    """A part whose base says what it does as a generator of products: a subclass with a `__call__` of its own, with a `forward` beside it,
+    or with a method `products` that is something else is what a block's side-by-side run calls."""
+    from holon_amd.parts import DenseFFN, drive, products_of
+
+    class Called(DenseFFN):
+        def __call__(self, x, step=None):
+            return 2 * super().__call__(x, step)
+
+    class Forward(DenseFFN):
+        def forward(self, x, step=None):
+            return 3 * super().forward(x, step)
+        __call__ = forward
+
+    class Named(DenseFFN):
+        def products(self, x):
+            return [x]
+
+        def __call__(self, x, step=None):
+            return x
+
+    class Plain(DenseFFN):
+        pass
+    build = _build(device, torch.float32)
+    results = {}
+    for cls in (DenseFFN, Plain, Called, Forward, Named):
+        part = cls(build, hidden=64, inter=32, layer=0)
+        _fill(part, 5, torch.float32, device)
+        x = torch.randn(rows, 64, generator=torch.Generator().manual_seed(6)).to(device)
+        results[cls], again = drive(part.kernels, rows, products_of(part, x), products_of(part, x))
+        assert torch.equal(results[cls], again) and torch.equal(results[cls], part(x))
+    assert torch.equal(results[Plain], results[DenseFFN]) and torch.equal(results[Called], 2 * results[DenseFFN])
+    assert torch.equal(results[Forward], 3 * results[DenseFFN])

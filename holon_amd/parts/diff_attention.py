@@ -31,7 +31,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
-from .products import FEW_ROWS, Product, drive
+from .products import Product, drive, together
 from .softmax_attention import attend, to_half_split
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -141,7 +141,7 @@ class DiffAttention(Part):
         held = site.paged[self.state_name]
         view = step.paged[held.group]
         table = getattr(self.position, "table", None)
-        few = x.shape[0] <= FEW_ROWS
+        few = together(x, self.qkv)
         qkv = (yield [Product(self.qkv, x)])[0] if few else self.qkv(x)
         if self.own_kv:
             q = k.head_prepare(qkv, 2 * self.heads, 2 * self.kv_heads, self.dim, self.vdim, self.q_norm,

@@ -12,7 +12,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, Stream
 from .linear import Linear
 from .norms import Normed
-from .products import FEW_ROWS, Product, Routing, drive
+from .products import Product, Routing, drive, together
 
 
 @register_part("ffn", "swiglu")
@@ -528,7 +528,7 @@ class PolyNormFFN(Part):
         self.declare("act", (4,), kind=FLOAT32, init="unit")
 
     def products(self, x: torch.Tensor, step=None):
-        few = x.shape[0] <= FEW_ROWS
+        few = together(x, self.down_proj)
         up = (yield [Product(self.up_proj, x)])[0] if few else self.up_proj(x)
         y = self.kernels.polynorm(up, self.act, self.eps)
         return (yield [Product(self.down_proj, y)])[0] if few else self.down_proj(y)
@@ -555,7 +555,7 @@ class DenseFFN(Part):
         self.attach("down_proj", Linear(build, inp=inter, out=hidden))
 
     def products(self, x: torch.Tensor, step=None):
-        few = x.shape[0] <= FEW_ROWS
+        few = together(x, self.down_proj)
         up = Product(self.up_proj, x, relu2=True)
         y = (yield [up])[0] if few else up.alone()
         return (yield [Product(self.down_proj, y)])[0] if few else self.down_proj(y)
@@ -672,7 +672,7 @@ class MoE(Part):
         else:
             route = Routing(k, x, self.router, self.correction if self.has_bias else None, self.experts, self.top, self.groups, self.keep,
                             scale=self.scale)
-        weights = (yield [route])[0] if x.shape[0] <= FEW_ROWS else route.alone()
+        weights = (yield [route])[0] if together(x) else route.alone()
         up, down = self.gate_up, self.all_down
         if x.dtype == torch.float32 and moe_f32_takes(x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top):
             y = k.moe_f32(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",

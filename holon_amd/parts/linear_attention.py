@@ -15,7 +15,7 @@ from ..kernels.registry import KernelOp, register_kernel
 from ..registry import register_part
 from .base import FLOAT32, Build, Part, SlotState
 from .linear import Linear
-from .products import FEW_ROWS, Product, drive
+from .products import Product, drive, together
 from .recurrent import MAX_KEY_DIM, _need, _rows, gated_out_plain, scan_pieces
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -197,7 +197,7 @@ class GatedLinearAttention(Part):
     def products(self, x: torch.Tensor, step, site, rows: torch.Tensor | None = None, at: int = 0):
         """`rows`: the input's projections, this mixer's from column `at` on (None: made here from `x`)."""
         k = self.kernels
-        few = x.shape[0] <= FEW_ROWS
+        few = together(x, self.o)
         if rows is None:
             rows = (yield [Product(self.inp, x)])[0] if few else self.inp(x)
         c, n = self.heads * self.dim, self.heads * self.vdim

@@ -7,7 +7,8 @@ down in. A part may therefore say what it does as a generator (`products`, with 
 rows it collects what all of them ask for and runs it as one operation (`linear_group`); in other steps, and for parts
 without a generator, one after the other: products of one size in one launch where they fill the chip together
 (`linear_block_group`), each other product as it always was. (A list, its products and the generator's way cost the host 3 us, as
-much as two launches of a step that the host bounds: a part that has one or two products to ask for runs them itself in such steps.)
+much as two launches of a step that the host bounds: a part that has one or two products to ask for runs them itself in steps that
+cannot share a launch, which is what `together` says of its input, and a launch for one product alone is not asked for.)
 """
 from __future__ import annotations
 
@@ -78,6 +79,13 @@ class Routing:
                                           and (self.scale is not None or self.top <= self.keep * (e // self.groups)))))
 
 
+def together(x, linear: Linear | None = None) -> bool:
+    """Whether a product over these rows (of `linear`, if it is one's) may share a launch: few of them, in the type that it serves, over
+    a tiled copy. Else whoever asks for it gains nothing from the list, and runs it."""
+    return x.shape[0] <= FEW_ROWS and getattr(x, "dtype", None) == torch.bfloat16 and \
+        (linear is None or getattr(linear, "tiled", None) is not None)
+
+
 @functools.cache
 def _says_products(cls: type) -> bool:
     """Whether the class that says what a call of the part does (the nearest that has `__call__`, `forward` or `products`) says it as a
@@ -115,10 +123,16 @@ def drive(kernels, rows: int, *parts) -> Sequence:
         go(i, None)
     while asked:
         waiting = dict(asked)
-        done = iter(kernels.linear_group([p for i in waiting for p in waiting[i]]))
+        todo = [p for i in waiting for p in waiting[i]]
+        done = iter(kernels.linear_group(todo) if _share(todo) else [p.alone() for p in todo])
         for i, products in waiting.items():
             go(i, [next(done) for _ in products])
     return results
+
+
+def _share(products: list[Product | Routing]) -> bool:
+    """Whether any of the products may find another one to run beside."""
+    return len(products) > 1 and any(isinstance(p, Product) and together(p.x, p.linear) for p in products)
 
 
 def _by_itself(kernels, part):

@@ -17,7 +17,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, SlotState
 from .convs import CausalConv
 from .linear import Linear
-from .products import FEW_ROWS, Product, drive
+from .products import Product, drive, together
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -343,7 +343,7 @@ class GatedDelta(Part):
         o = k.delta_scan(qn, kn, qkv, beta, g, site.slot_state[self.prefix + "S"], step.slots, step.starts,
                          step.query_start, step.n_rows, self.heads, self.vdim, delta_pieces(step, self.heads * self.vdim, self.build.dtype))
         y = k.gated_out(o, gate, self.norm, False, self.eps, self.build.dtype)
-        return (yield [Product(self.o, y)])[0] if x.shape[0] <= FEW_ROWS else self.o(y)
+        return (yield [Product(self.o, y)])[0] if together(x, self.o) else self.o(y)
 
     def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
@@ -410,7 +410,7 @@ class DecayMemory(Part):
         o = k.memory_scan(r, kk, v, decay, self.u, site.slot_state[self.prefix + "S"], *rows, step.n_rows, self.heads,
                           scan_pieces(step))
         y = k.gated_out(o, gate, self.norm, True, self.eps, self.build.dtype)
-        return (yield [Product(self.o, y)])[0] if x.shape[0] <= FEW_ROWS else self.o(y)
+        return (yield [Product(self.o, y)])[0] if together(x, self.o) else self.o(y)
 
     def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]

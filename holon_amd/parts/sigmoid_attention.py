@@ -18,7 +18,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
-from .products import FEW_ROWS, Product, drive
+from .products import Product, drive, together
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -260,7 +260,7 @@ class SigmoidWindowAttention(Part):
         out = k.sigmoid_attention(q, held.pages, view.table, step.rows, step.token_row, step.positions,
                                   self.kv_heads, self.vdim, view.page_size, self.pb if self.head_bias else None,
                                   self.scale, self.window, *(gate or (None,)))
-        return (yield [Product(self.o, out)])[0] if x.shape[0] <= FEW_ROWS else self.o(out)
+        return (yield [Product(self.o, out)])[0] if together(x, self.o) else self.o(out)
 
     def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
         return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]

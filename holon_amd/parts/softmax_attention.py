@@ -21,7 +21,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
-from .products import FEW_ROWS, Product, drive
+from .products import Product, drive, together
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -624,7 +624,7 @@ class SoftmaxAttention(Part):
         held = site.paged[self.state_name]
         view = step.paged[held.group]
         table = getattr(self.position, "table", None)
-        few = x.shape[0] <= FEW_ROWS
+        few = together(x, self.o)
         qkv = rows if rows is not None else (yield [Product(self.qkv, x)])[0] if few else self.qkv(x)
         if self.whole_norm is not None:
             q = k.whole_norm_prepare(qkv, self.heads, self.kv_heads, self.dim, self.vdim, self.q_norm,
@@ -777,7 +777,7 @@ class LatentAttention(Part):
                              "another run's")
         held = site.paged[self.state_name]
         view = step.paged[held.group]
-        few = t <= FEW_ROWS
+        few = together(x, self.o)
         both = (yield [Product(self.down, x)])[0] if few else self.down(x)
         if self.q_rank == 0:                      # norm, rotation and the cache write in one kernel
             table = getattr(self.position, "table", None)

@@ -729,3 +729,33 @@ def test_a_part_that_overrides_how_it_is_called_is_called(device, rows):
         assert torch.equal(results[cls], again) and torch.equal(results[cls], part(x))
     assert torch.equal(results[Plain], results[DenseFFN]) and torch.equal(results[Called], 2 * results[DenseFFN])
     assert torch.equal(results[Forward], 3 * results[DenseFFN])
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("dtype,copies,rows,asked", [(torch.float32, True, 3, 0), (torch.bfloat16, False, 3, 0), (torch.bfloat16, True, 16, 2),
+                                                     (torch.bfloat16, True, 17, 0)])
+def test_products_that_cannot_share_a_launch_are_run_by_their_part(device, dtype, copies, rows, asked, monkeypatch):
+    """Few rows in a type or over weights that no launch of several products serves are not collected for one, and neither is a product
+    that nothing else is asked for beside: two feed-forwards side by side, one by itself, three products of one part."""
+    from holon_amd.parts import DenseFFN, Product, drive, products_of
+    build = _build(device, dtype, decode_copy=copies)
+    part = DenseFFN(build, hidden=256, inter=512, layer=0)
+    _fill(part, 7, dtype, device)
+    if device == "cpu" and copies and dtype == torch.bfloat16:                 # (the plain functions read none, and have no layout for one)
+        part.up_proj.tiled, part.down_proj.tiled = part.up_proj.weight, part.down_proj.weight
+    x = torch.randn(rows, 256, generator=torch.Generator().manual_seed(8)).to(dtype).to(device)
+    calls = []
+
+    def group(products):
+        calls.append(len(products))
+        return [p.alone() for p in products]
+    monkeypatch.setattr(part.kernels, "linear_group", group)
+
+    def three():
+        return (yield [Product(part.up_proj, x)] * 3)
+    want = part(x)
+    assert not calls
+    one, two = drive(part.kernels, rows, products_of(part, x), products_of(part, x))
+    assert calls == [2] * asked and torch.equal(one, want) and torch.equal(two, want)
+    assert all(torch.equal(y, part.up_proj(x)) for y in drive(part.kernels, rows, three())[0])
+    assert calls[asked:] == [3] * (asked > 0)

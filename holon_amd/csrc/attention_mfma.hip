@@ -2146,7 +2146,7 @@ extern "C" int holon_sigmoid_attention_prefill_bf16(const void* q, void* out, co
   return 0;
 }
 
-// Decode rows of the same: the window's keys over `blocks` blocks a (row, kv head) and their waves (up to 8). With more than one, part_o
+// Decode rows of the same: the window's keys over `blocks` blocks a (row, kv head) of `waves` waves (up to 8). With more than one block, part_o
 // [n_rows, heads, blocks, D] takes their sums (float32), which a second kernel adds. What bounds a block is what its compute unit reads (16 KB
 // for every 32 keys at D = 128, about 42 KB a us), so a long window goes over several units; a short one not, as the second kernel takes 4 us.
 extern "C" int holon_sigmoid_attention_decode_bf16(const void* q, void* out, const void* pages, const int32_t* table,
@@ -2154,7 +2154,7 @@ extern "C" int holon_sigmoid_attention_decode_bf16(const void* q, void* out, con
                                                    const int32_t* query_start, const int32_t* row_ids, int n_rows,
                                                    int max_len, int heads, int kv_heads, int head_dim, int page_size,
                                                    float scale, int window, const float* head_bias, const void* gate,
-                                                   int rows_in_order, int blocks, float* part_o, void* stream) {
+                                                   int rows_in_order, int blocks, int waves, float* part_o, void* stream) {
   HOLON_CHECK((head_dim == 64 || head_dim == 128) && mfma_serves(head_dim, page_size),
               "sigmoid attention (matrix cores): head_dim %d / page %d not served", head_dim, page_size);
   HOLON_CHECK(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && window >= 0 && table_stride > 0 && max_len >= 0,
@@ -2162,9 +2162,7 @@ extern "C" int holon_sigmoid_attention_decode_bf16(const void* q, void* out, con
   if (n_rows <= 0) return 0;
   HOLON_CHECK(blocks == 1 || (blocks > 1 && blocks <= 64 && part_o != nullptr && (uintptr_t)part_o % 16 == 0),
               "sigmoid attention: %d blocks a row without room for their sums", blocks);
-  const int span = window > 0 ? (window < max_len ? window + 31 : max_len) : max_len;
-  int waves = ((span + blocks - 1) / blocks + 31) / 32;      // 32 keys a wave, or more
-  waves = waves < 1 ? 1 : (waves > 8 ? 8 : waves);
+  HOLON_CHECK(waves >= 1 && waves <= 8, "sigmoid attention: blocks of %d waves", waves);
   AttnArgs a{};
   a.q = (const bf16_t*)q; a.out = (bf16_t*)out; a.pages = (const bf16_t*)pages; a.table = table;
   a.table_stride = table_stride; a.slots = slots; a.lens = lens; a.qstart = query_start; a.row_ids = row_ids;

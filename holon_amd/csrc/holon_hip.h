@@ -308,14 +308,14 @@ int holon_sigmoid_attention_prefill_bf16(const void* q, void* out, const void* p
                                          const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_query,
                                          int max_len, int heads, int kv_heads, int head_dim, int page_size, float scale,
                                          int window, const float* head_bias, const void* gate, void* stream);
-// The decode rows (one token each) on the matrix cores, the same sizes; a row's keys over `blocks` blocks (1 to 64), with more than one
+// The decode rows (one token each) on the matrix cores, the same sizes; a row's keys over `blocks` blocks (1 to 64) of `waves` (1 to 8), with more than one block
 // part_o [n_rows, heads, blocks, D] float32.
 int holon_sigmoid_attention_decode_bf16(const void* q, void* out, const void* pages, const int32_t* table,
                                         int table_stride, const int32_t* slots, const int32_t* lens,
                                         const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_len,
                                         int heads, int kv_heads, int head_dim, int page_size, float scale, int window,
                                         const float* head_bias, const void* gate, int rows_in_order, int blocks,
-                                        float* part_o, void* stream);
+                                        int waves, float* part_o, void* stream);
 
 // -- Dynamic Tanh and the adds around it (dyt.hip) ------------------------------------------------------------------------
 // x [rows, dim] (float32 when anything is added): x += scale * (tanh(a1 term) w1 + b1) (with a term), x += extra (with

@@ -151,6 +151,20 @@ def decode_blocks(pairs: int, span: int) -> int:
     return 1 if span <= 256 else max(1, min(64, -(-span // 128), 256 // max(1, pairs)))
 
 
+def decode_waves(pairs: int, span: int, blocks: int) -> int:
+    """Waves of each of these blocks. Where a compute unit has a block or none, 32 keys a wave, up to what a unit's loads keep busy: 4 waves, 5
+    from 256 keys, 8 from 1,024. Where it has several they cover one another's latencies, and waves only add their start, their partial sums and the
+    registers that keep the next block out: 128 keys a wave, up to 4. Measured, 32 | 128 keys a wave (up to 8), us: 1,024 pairs of heads of 128
+    over 100 / 200 / 300 / 400 / 700 / 3,000 keys 21 | 18, 41 | 24, 51 | 33, 55 | 39, 85 | 83, 260 | 260 (4 waves 69 and 253 for the last two), 512
+    pairs 11 | 13, 22 | 16, 28 | 20, 30 | 23, 40 | 39 (33); 256 pairs of 200 / 300 keys 10.5 | 11.3, 14.0 | 13.8 (4 waves 10.0, 13.3); heads of
+    64, 128 pairs of 400 / 700 / 3,000 keys by 4 / 5 / 8 waves 8.4 / 7.8 / 8.4, 10.0 / 9.5 / 9.8, 27.6 / 27.3 / 22.0. Several blocks a row: 64 pairs
+    over 400 / 700 keys by 4 | 8 waves 8.7 | 11.5, 11.1 | 11.7."""
+    if pairs > 256:
+        return max(1, min(4, -(-span // 128)))
+    most = 4 if blocks > 1 or span <= 256 else 5 if span < 1024 else 8
+    return max(1, min(most, -(-(-(-span // blocks)) // 32)))
+
+
 def _sigmoid_attention_hip(launch, q, pages, table, rows, token_row, positions, kv_heads, vdim, page_size, bias,
                            scale, window, gate):
     t, heads, dim = q.shape
@@ -176,11 +190,12 @@ def _sigmoid_attention_hip(launch, q, pages, table, rows, token_row, positions, 
                  _ptr(bias), _ptr(gate))
         if rows.n_decode:
             span = min(rows.max_decode_len, window + 31) if window > 0 else rows.max_decode_len
-            blocks = decode_blocks(rows.n_decode * kv_heads * (-(-(heads // kv_heads) // 16)), span)
+            pairs = rows.n_decode * kv_heads * (-(-(heads // kv_heads) // 16))
+            blocks = decode_blocks(pairs, span)
             parts = torch.empty((rows.n_decode, heads, blocks, dim), dtype=torch.float32, device=q.device) if blocks > 1 else None
             narrow(*common, rows.lens.data_ptr(), rows.query_start.data_ptr(), rows.decode_rows.data_ptr(),
                    rows.n_decode, rows.max_decode_len, heads, kv_heads, dim, page_size, float(scale), int(window),
-                   _ptr(bias), _ptr(gate), int(rows.in_order and rows.n_decode == t), blocks, _ptr(parts))
+                   _ptr(bias), _ptr(gate), int(rows.in_order and rows.n_decode == t), blocks, decode_waves(pairs, span, blocks), _ptr(parts))
     else:
         general(*common, token_row.data_ptr(), positions.data_ptr(), None, None, t, *tail)
     return out
@@ -194,7 +209,7 @@ register_kernel(KernelOp("sigmoid_attention", sigmoid_attention_plain,
                           "holon_sigmoid_attention_decode_bf16"),
                          ([_P, _P, _P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _F, _I, _P, _I],
                           [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P],
-                          [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _P]),
+                          [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _P, _I, _I, _I, _P]),
                          _sigmoid_attention_hip))
 
 

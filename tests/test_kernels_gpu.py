@@ -1914,3 +1914,25 @@ def test_decode_rows_at_the_borders_of_a_wave_a_block(hip, dtype, heads, kv, dim
     assert sum(x.numel() * x.element_size() for x in made) <= 5 << 20 and (split or not made)
     want = PLAIN.paged_attention(q.double(), pages.double(), table, attn, page, dim ** -0.5, 0)
     assert H.op_budget_usage(got, want, dtype, dim + longest) <= 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv,dim", [(4, 2, 128), (3, 3, 64), (34, 2, 64)])
+@pytest.mark.parametrize("t,longest,window", [(1, 256, 0), (1, 257, 0), (3, 1100, 0), (50, 300, 1024), (129, 1023, 0), (129, 1024, 0), (140, 640, 129)])
+def test_sigmoid_decode_rows_by_the_rules_of_blocks_and_waves(hip, heads, kv, dim, t, longest, window):
+    """`sigmoid_attention` of decode rows on both sides of the lines that blocks and waves are chosen by (256, 257, 1,023 and 1,024 keys; up to 256
+    (row, kv head) pairs and more): float32 sums of up to 1,100 bfloat16 products, rounded once (2^-9)."""
+    from holon_amd.kernels.registry import kernel_op
+    import holon_amd.parts  # noqa: F401  (brings the operations)
+    page, lens = 16, [max(1, longest - 37 * i % longest) for i in range(t)]
+    per = -(-longest // page)
+    pages = _randn(t * per, kv * page * 2 * dim, dtype=torch.bfloat16, seed=240)
+    table = torch.arange(t * per, dtype=torch.int32, device="cuda").view(t, per)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")          # noqa: E731
+    order = i32(list(range(t)))
+    q, gate = _randn(t, heads, dim, dtype=torch.bfloat16, seed=241), _randn(t, heads * dim, dtype=torch.bfloat16, seed=242)
+    rows = AttnRows(slots=order, lens=i32(lens), query_start=i32(list(range(t + 1))), decode_rows=order, chunk_rows=i32([]), n_decode=t,
+                    n_chunk=0, max_decode_len=longest, max_chunk_query=0, max_chunk_len=0, in_order=True)
+    args = (q, pages, table, rows, order, i32([v - 1 for v in lens]), kv, dim, page, _randn(heads, dtype=torch.float32, seed=243), dim ** -0.5,
+            window, gate)
+    assert H.rel_rms(hip.sigmoid_attention(*args), kernel_op("sigmoid_attention").plain(*args)) < 2.0 ** -8

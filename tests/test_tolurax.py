@@ -591,3 +591,12 @@ def test_an_infinite_value_of_a_rows_last_token_is_infinite_in_its_state(heads, 
         assert torch.equal(blocks[:, 0, :, 3], tokens[:, 0, :, 3]) and blocks[:, 0, :, 3].isinf().all()
         blocks[:, 0, :, 3] = without[:, 0, :, 3]
         assert torch.equal(blocks, without)
+
+
+def test_sigmoid_decode_rows_keep_few_waves_where_units_have_several_blocks():
+    """`decode_waves`: a wave for every 32 keys only up to 256 (row, kv head) pairs, and then one for every 128, never more than four."""
+    from holon_amd.parts.sigmoid_attention import decode_blocks, decode_waves
+    assert [decode_waves(4, n, 1) for n in (1, 32, 33, 128, 256, 257, 1023, 1024, 5000)] == [1, 1, 2, 4, 4, 5, 5, 8, 8]
+    assert [decode_waves(257, n, 1) for n in (1, 128, 129, 300, 400, 512, 5000)] == [1, 1, 2, 3, 4, 4, 4]
+    for pairs in (1, 16, 64, 128):
+        assert all(decode_waves(pairs, n, decode_blocks(pairs, n)) == min(4, -(-(-(-n // decode_blocks(pairs, n))) // 32)) for n in (257, 700, 9000))

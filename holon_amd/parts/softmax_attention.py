@@ -84,11 +84,18 @@ def _float64_sums_serve(heads, kv_heads, dim, vdim, page_size):
         and kv_heads * -(-(heads // kv_heads) // 16) <= 65535
 
 
-def f64_split_pays(blocks: int, longest: int, window: int) -> bool:
-    """Whether a step of decode rows alone, in `blocks` blocks of eight waves over up to `longest` keys, has every wave in a block of its
-    own (the same bits): where the blocks leave compute units idle and a wave has more than a tile or two (one row behind 700 tokens 28 us
-    in place of 45; behind 150 a block takes 16 and the second kernel alone 4.6)."""
-    return blocks <= 128 and (min(longest, abs(window)) if window else longest) > 256
+def f64_split_pays(tokens: int, heads: int, kv_heads: int, dim: int, longest: int, window: int) -> bool:
+    """Whether a step of decode rows alone, over up to `longest` keys, has each of its blocks' eight waves in a block of its own (the same bits):
+    where every one of them has a SIMD of the 1,024 to itself, counted with the places that the grid is filled up to, and a wave has more than a tile or two. Measured, us, whole | split, heads of 128: 4 blocks over 257 / 512 / 1,024 keys 20.7 | 15.1,
+    30.8 | 18.3, 55.6 | 30.6; 112 blocks 22.5 | 19.3, 33.4 | 22.7, 60.0 | 35.9; 128 in a grid of 132 22.7 | 19.9, 33.6 | 23.2, 60.2 | 36.1, in one of 144
+    22.8 | 23.2, 33.3 | 35.7, 60.1 | 60.5; 104 in one of 160 22.6 | 22.6, 32.9 | 35.1, 59.6 | 60.0. Heads of 64: 64 blocks over 257 / 512 12.8 | 12.3, 18.1 | 14.5; 112 blocks 257 / 384 / 512
+    12.6 | 13.0, 15.2 | 13.3, 18.5 | 15.4 (20 heads on one, 72 blocks, 12.8 | 13.6, 15.1 | 14.0, 18.7 | 15.4), 128 in a grid of 132
+    13.0 | 14.7, 15.4 | 16.7, 18.7 | 20.3, 104 in one of 160 12.8 | 14.1, 15.0 | 16.2, 18.5 | 19.9."""
+    group = heads // kv_heads
+    per, blocks = 16 // min(group, 16), kv_heads * -(-group // 16)                # tokens a block takes; blocks a token
+    grid = (-(-tokens // per) | 1) * per * blocks
+    span = min(longest, abs(window)) if window else longest
+    return grid <= (128 if dim == 64 else 132) and span > (320 if dim == 64 and tokens * blocks > 64 else 256)
 
 
 def _softmax_attention_hip(launch, q, pages, table, rows, token_row, positions, kv_heads, vdim, page_size, sink,
@@ -112,7 +119,7 @@ def _softmax_attention_hip(launch, q, pages, table, rows, token_row, positions, 
         and _float64_sums_serve(heads, kv_heads, dim, vdim, page_size) and q.data_ptr() % 16 == 0 and pages.data_ptr() % 16 == 0 \
         else general
     parts = ()
-    if kernel is wide and rows.n_chunk == 0 and f64_split_pays(t * kv_heads * -(-(heads // kv_heads) // 16), rows.max_decode_len, window):
+    if kernel is wide and rows.n_chunk == 0 and f64_split_pays(t, heads, kv_heads, dim, rows.max_decode_len, window):
         kernel, parts = split, (torch.empty((t, heads, 8, dim), dtype=torch.float64, device=q.device),
                                 torch.empty((t, heads, 8, 2), dtype=torch.float32, device=q.device))
     kernel(q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), table.shape[1], table.shape[0],

@@ -1936,3 +1936,39 @@ def test_sigmoid_decode_rows_by_the_rules_of_blocks_and_waves(hip, heads, kv, di
     args = (q, pages, table, rows, order, i32([v - 1 for v in lens]), kv, dim, page, _randn(heads, dtype=torch.float32, seed=243), dim ** -0.5,
             window, gate)
     assert H.rel_rms(hip.sigmoid_attention(*args), kernel_op("sigmoid_attention").plain(*args)) < 2.0 ** -8
+
+
+F64_BORDERS = [(16, 4, 128, 1, 256, False), (16, 4, 128, 1, 257, True), (16, 4, 128, 28, 300, True), (16, 4, 128, 29, 300, False),
+               (32, 8, 128, 12, 300, True), (32, 8, 128, 13, 300, False), (16, 4, 64, 16, 257, True), (16, 4, 64, 17, 320, False),
+               (16, 4, 64, 17, 321, True), (40, 2, 64, 31, 321, True), (40, 2, 64, 32, 700, False), (4, 4, 64, 32, 700, False),
+               (4, 1, 128, 128, 300, True), (4, 1, 128, 133, 300, False), (4, 1, 64, 128, 700, False)]
+
+
+def test_float64_decode_rows_are_split_where_their_blocks_fit():
+    from holon_amd.parts.softmax_attention import f64_split_pays
+    assert [f64_split_pays(t, h, kv, dim, longest, 0) for h, kv, dim, t, longest, _ in F64_BORDERS] == [b[-1] for b in F64_BORDERS]
+    assert not f64_split_pays(1, 16, 4, 128, 700, 256) and f64_split_pays(1, 16, 4, 128, 700, -257)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv,dim,t,longest,split", F64_BORDERS)
+def test_float64_decode_rows_at_the_borders_of_a_wave_a_block(hip, heads, kv, dim, t, longest, split, monkeypatch):
+    """`softmax_attention` of float32 decode rows on both sides of the rule that gives every wave a block: the form named, and its result that of
+    the plain form in float64 within float32 exponentials and one rounding."""
+    from holon_amd.kernels.registry import kernel_op
+    import holon_amd.parts  # noqa: F401  (brings the operations)
+    page, lens = 16, [longest - 7 * i % 60 for i in range(t)]
+    per = -(-longest // page)
+    pages = _randn(t * per, 2 * kv * page * dim, dtype=torch.float32, seed=250)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")          # noqa: E731
+    table, order = torch.arange(t * per, dtype=torch.int32, device="cuda").view(t, per), i32(list(range(t)))
+    rows = AttnRows(slots=order, lens=i32(lens), query_start=i32(list(range(t + 1))), decode_rows=order, chunk_rows=i32([]), n_decode=t,
+                    n_chunk=0, max_decode_len=longest, max_chunk_query=0, max_chunk_len=0, in_order=True)
+    q, positions, made, empty = _randn(t, heads, dim, dtype=torch.float32, seed=251), i32([v - 1 for v in lens]), [], torch.empty
+    rest = (rows, order, positions, kv, dim, page, None, dim ** -0.5, 0)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", lambda *a, **kw: made.append(kw.get("dtype")) or empty(*a, **kw))
+        got = hip.softmax_attention(q, pages, table, *rest)
+    assert (torch.float64 in made) == split
+    want = kernel_op("softmax_attention").plain(q.double(), pages.double(), table, *rest)
+    assert H.rel_rms(got, want) < 1e-6

@@ -517,12 +517,15 @@ __global__ void shift_keep_kernel(const T* __restrict__ x, T* __restrict__ state
 
 // exp(-exp(tanh(a) w2^T + w0)) on the float32 matrix cores, whose sums are the chain of multiply-adds in ascending order. A block takes 16
 // tokens and 256 channels, a wave 64 of them: lane l's four neighbouring channels are column l % 16 of four tiles, so that one load of w2
-// (transposed, [rank, channels]) serves them all. The tokens' tanh values lie in LDS. VEC: channels come in whole fours.
+// (transposed, [rank, channels]) serves them all. The tokens' tanh values lie in LDS. FOURS: there are four channels; a lane whose four would
+// end behind the last channel takes the last four, which a neighbour has as well: the same sums, stored twice. (Loads and stores of four
+// are aligned as one value is, so that any number of channels takes them; value by value 17 tokens of 1,030 channels of rank 30 took 7.6 us, so 5.2.)
+// A lane's four results of a tile are tokens g, 4 + g, 8 + g and 12 + g, so that a step of up to four tokens has one for every lane.
 // 2,048 tokens by 2,048 channels of rank 64 17 us and one token 4.9 (on the vector unit, a token's value read from LDS for every
 // multiply-add, 27 and 8.4).
 __host__ __device__ constexpr int lora_pitch(int rank) { return (rank + 3) / 4 * 4 + (rank < 1000 ? 1 : 0); }      // (at most 64 KB of LDS)
 constexpr int LORA_TOKENS = 16, LORA_MAX_RANK = 1024, LORA_AHEAD = 8;      // LORA_AHEAD: steps of four ranks whose weights are asked for at a time
-template <bool VEC, typename T>
+template <bool FOURS, typename T>
 __global__ void __launch_bounds__(256) decay_lora_kernel(const float* __restrict__ a, const T* __restrict__ w2t,
                                                          const float* __restrict__ w0, float* __restrict__ y, int tokens,
                                                          int channels, int rank) {
@@ -530,17 +533,17 @@ __global__ void __launch_bounds__(256) decay_lora_kernel(const float* __restrict
   typedef float f32x4 __attribute__((ext_vector_type(4)));
   const int steps = (rank + 3) / 4, pitch = lora_pitch(rank);
   const int t0 = blockIdx.x * LORA_TOKENS, lane = threadIdx.x % WAVE, g = lane / 16, c = lane % 16;
-  const int c0 = blockIdx.y * 256 + threadIdx.x / WAVE * 64 + 4 * c;
+  const int first = blockIdx.y * 256 + threadIdx.x / WAVE * 64 + 4 * c, c0 = FOURS ? min(first, channels - 4) : first;
   T next[LORA_AHEAD][4];
   const auto ask = [&](int s0) {
 #pragma unroll
     for (int u = 0; u < LORA_AHEAD; ++u) {
       const int64_t row = (int64_t)min(4 * (s0 + u) + g, rank - 1) * channels;
-      if constexpr (VEC) {
-        typedef T vec __attribute__((ext_vector_type(4)));
-        const vec v = *reinterpret_cast<const vec*>(w2t + row + min(c0, channels - 4));
+      if constexpr (FOURS) {
+        struct Four { T v[4]; };
+        const Four v = *reinterpret_cast<const Four*>(w2t + row + c0);
 #pragma unroll
-        for (int n = 0; n < 4; ++n) next[u][n] = v[n];
+        for (int n = 0; n < 4; ++n) next[u][n] = v.v[n];
       } else {
 #pragma unroll
         for (int n = 0; n < 4; ++n) next[u][n] = w2t[row + min(c0 + n, channels - 1)];
@@ -566,7 +569,7 @@ __global__ void __launch_bounds__(256) decay_lora_kernel(const float* __restrict
 #pragma unroll
     for (int u = 0; u < LORA_AHEAD; ++u) {
       if (s0 + u >= steps) break;
-      const float x = th[c * pitch + 4 * (s0 + u) + g];
+      const float x = th[(c % 4 * 4 + c / 4) * pitch + 4 * (s0 + u) + g];
 #pragma unroll
       for (int n = 0; n < 4; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, w[u][n], acc[n], 0, 0, 0);
     }
@@ -575,18 +578,18 @@ __global__ void __launch_bounds__(256) decay_lora_kernel(const float* __restrict
 #pragma unroll
   for (int n = 0; n < 4; ++n) off[n] = w0[min(c0 + n, channels - 1)];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {                            // lane: tokens 4 g + i of its four channels
-    const int t = t0 + 4 * g + i;
+  for (int i = 0; i < 4; ++i) {                            // lane: tokens 4 i + g of its four channels
+    const int t = t0 + 4 * i + g;
     if (t >= tokens) continue;
-    f32x4 o;
+    struct Four { float v[4]; } o;
 #pragma unroll
-    for (int n = 0; n < 4; ++n) o[n] = expf(-expf(acc[n][i] + off[n]));
-    if constexpr (VEC) {
-      if (c0 < channels) *reinterpret_cast<f32x4*>(y + (int64_t)t * channels + c0) = o;
+    for (int n = 0; n < 4; ++n) o.v[n] = expf(-expf(acc[n][i] + off[n]));
+    if constexpr (FOURS) {
+      if (first < channels) *reinterpret_cast<Four*>(y + (int64_t)t * channels + c0) = o;
     } else {
 #pragma unroll
       for (int n = 0; n < 4; ++n)
-        if (c0 + n < channels) y[(int64_t)t * channels + c0 + n] = o[n];
+        if (c0 + n < channels) y[(int64_t)t * channels + c0 + n] = o.v[n];
     }
   }
 }
@@ -798,7 +801,7 @@ extern "C" int holon_decay_lora(const float* a, const void* w2t, const float* w0
   HOLON_CHECK(grid.y <= 65535, "decay_lora: %d channels exceed one launch", channels);
   const size_t lds = (size_t)LORA_TOKENS * lora_pitch(rank) * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
-  if (channels % 4 == 0 && (((uintptr_t)w2t | (uintptr_t)y) & 15) == 0)
+  if (channels >= 4)
     BY_DTYPE(dtype, (decay_lora_kernel<true, T><<<grid, 256, lds, s>>>(a, (const T*)w2t, w0, y, tokens, channels, rank)));
   else
     BY_DTYPE(dtype, (decay_lora_kernel<false, T><<<grid, 256, lds, s>>>(a, (const T*)w2t, w0, y, tokens, channels, rank)));

@@ -1972,3 +1972,17 @@ def test_float64_decode_rows_at_the_borders_of_a_wave_a_block(hip, heads, kv, di
     assert (torch.float64 in made) == split
     want = kernel_op("softmax_attention").plain(q.double(), pages.double(), table, *rest)
     assert H.rel_rms(got, want) < 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,channels,rank", [(1, 1030, 30), (4, 255, 64), (5, 257, 9), (17, 7, 4), (33, 5, 16), (2, 4, 3), (20, 3, 5)])
+def test_decay_projection_of_any_number_of_channels(hip, dtype, tokens, channels, rank):
+    """Channels that do not come in fours: bit for bit those of a call whose channels do, and nothing behind them is written."""
+    more = -(-channels // 4) * 4 + 4
+    a, w2t = _randn(tokens, rank, dtype=torch.float32, seed=260), _randn(rank, more, dtype=dtype, seed=261, scale=0.3 * rank ** -0.5)
+    w0, w = _randn(more, dtype=torch.float32, seed=262), w2t[:, :channels].contiguous()
+    y = torch.full((tokens * channels + 4,), 7.0, dtype=torch.float32, device="cuda")
+    hip._call(hip.lib.holon_decay_lora, a.data_ptr(), w.data_ptr(), w0.data_ptr(), y.data_ptr(), tokens, channels, rank,
+              int(dtype == torch.bfloat16), hip._stream())
+    assert torch.equal(y[:-4].view(tokens, channels), hip.decay_lora(a, w2t, w0)[:, :channels]) and (y[-4:] == 7.0).all()

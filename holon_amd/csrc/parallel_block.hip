@@ -475,6 +475,7 @@ extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void*
   } while (0)
     if (dim <= 1024) SRMSV_BY_TYPE(1);
     else if (dim <= 2048) SRMSV_BY_TYPE(2);
+    else if (dim <= 3072) SRMSV_BY_TYPE(3);
     else if (dim <= 4096) SRMSV_BY_TYPE(4);
     else SRMSV(8, 0);
 #undef SRMSV_BY_TYPE

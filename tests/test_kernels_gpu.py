@@ -1862,7 +1862,7 @@ def test_decode_rows_of_every_last_block(hip, geometry, softcap):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dim", [4, 1020, 1028, 2048, 4092, 4096, 4100])
+@pytest.mark.parametrize("dim", [4, 1020, 1028, 2048, 2560, 3072, 3076, 4092, 4096, 4100])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_stream_rows_of_one_type_are_those_of_several(hip, dtype, dim):
     """A pass over stream rows whose operands are of one type and asked for ahead gives the bits of the general one (taken here by a term

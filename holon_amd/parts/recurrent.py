@@ -22,10 +22,12 @@ from .products import Product, drive, together
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
 MAX_KEY_DIM = 256             # the scans keep a column of D values in registers
-# The delta rule's rows of this many tokens and more go in blocks of 16 tokens (16 heads of 128 by 128, us, against token by token:
-# 32 tokens 22 / 24, 64 28 / 41, 300 70 / 170), whatever other rows a step has. The 32-bit path keeps the token's own order of sums in
+# The delta rule's rows of this many tokens and more go in blocks of 16 tokens, whatever other rows a step has. Measured, us, against token by
+# token: 16 heads of 128 by 128 32 tokens 21 / 23, 64 28 / 40, 300 70 / 170; of 64 by 64 32 tokens 14.6 / 13.7, 48 16.7 / 18.7, 64 18.5 / 23.6. Beside
+# shorter rows the two forms are launches of their own: fifteen single tokens and 32 / 48 / 64 tokens of 64 by 64 20.9 / 15.6, 22.8 / 20.8,
+# 24.9 / 26.5, 32 heads of 32 by 64 the same, 8 heads of 128 30 / 26, 34 / 36, 37 / 45: from 64 on no mix of rows loses. The 32-bit path keeps the token's own order of sums in
 # shorter rows, so that the rule's results do not depend on how a prompt is cut into portions below that many tokens.
-DELTA_FROM = {torch.bfloat16: 32, torch.float32: 512}
+DELTA_FROM = {torch.bfloat16: 64, torch.float32: 512}
 
 
 def _ptr(t):

@@ -541,7 +541,7 @@ def test_the_delta_rule_of_a_row_does_not_depend_on_the_rows_beside_it(heads, kv
     gen = torch.Generator().manual_seed(dim)
     rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)             # noqa: E731
-    counts, starts = [1, 20, 31, 32, 300, 511, 600, 1], [9, 0, 4, 1, 0, 2, 3, 0]
+    counts, starts = [1, 20, 63, 64, 300, 511, 600, 1, 512], [9, 0, 4, 1, 0, 2, 3, 0, 5]
     t, n = sum(counts), len(counts)
     norm = lambda x: x / x.norm(dim=-1, keepdim=True)                          # noqa: E731
     qn, kn = norm(rn(t, kv, dim)), norm(rn(t, kv, dim))

@@ -1729,7 +1729,7 @@ def test_decay_projection(hip, dtype, tokens, channels, rank):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("heads,kv,dim,page", [(8, 2, 128, 16), (3, 3, 72, 5), (2, 1, 512, 8)])
+@pytest.mark.parametrize("heads,kv,dim,page", [(8, 2, 128, 16), (3, 3, 72, 5), (2, 1, 512, 8), (4, 2, 64, 16), (6, 1, 192, 8), (8, 2, 256, 16)])
 @pytest.mark.parametrize("window", [0, 300, -128])
 def test_decode_rows_a_wave_a_block_are_the_same_bits(hip, dtype, heads, kv, dim, page, window):
     """The general attention kernel's waves in blocks of their own against the whole block: rows of one key, of a tile and one more, of more

@@ -12,7 +12,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, Stream
 from .linear import Linear
 from .norms import Normed
-from .products import Product, Routing, drive, together
+from .products import Product, Routing, by_itself, together
 
 
 @register_part("ffn", "swiglu")
@@ -534,7 +534,7 @@ class PolyNormFFN(Part):
         return (yield [Product(self.down_proj, y)])[0] if few else self.down_proj(y)
 
     def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
-        return drive(self.kernels, x.shape[0], self.products(x, step))[0]
+        return by_itself(self.kernels, self.products(x, step))
 
     __call__ = forward
 
@@ -561,7 +561,7 @@ class DenseFFN(Part):
         return (yield [Product(self.down_proj, y)])[0] if few else self.down_proj(y)
 
     def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
-        return drive(self.kernels, x.shape[0], self.products(x, step))[0]
+        return by_itself(self.kernels, self.products(x, step))
 
     __call__ = forward
 
@@ -694,7 +694,7 @@ class MoE(Part):
         return down(between(up(x), weights, self.inter, self.shared, shared_weight=self.shared_gated))
 
     def forward(self, x: torch.Tensor, step=None) -> torch.Tensor:
-        return drive(self.kernels, x.shape[0], self.products(x, step))[0]
+        return by_itself(self.kernels, self.products(x, step))
 
     def _own_rows(self, rows: int) -> bool:
         """Whether the engine's product choices leave a step of many rows to `moe_rows`: pins of either product over all experts keep

@@ -15,7 +15,7 @@ from ..kernels.registry import KernelOp, register_kernel
 from ..registry import register_part
 from .base import FLOAT32, Build, Part, SlotState
 from .linear import Linear
-from .products import Product, drive, together
+from .products import Product, by_itself, together
 from .recurrent import MAX_KEY_DIM, _need, _rows, gated_out_plain, scan_pieces
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
@@ -216,6 +216,6 @@ class GatedLinearAttention(Part):
         return (yield [Product(self.o, y)])[0] if few else self.o(y)
 
     def forward(self, x: torch.Tensor, step, site, rows: torch.Tensor | None = None, at: int = 0) -> torch.Tensor:
-        return drive(self.kernels, x.shape[0], self.products(x, step, site, rows, at))[0]
+        return by_itself(self.kernels, self.products(x, step, site, rows, at))
 
     __call__ = forward

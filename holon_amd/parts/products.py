@@ -107,10 +107,8 @@ def products_of(part, *args, **kwargs):
 
 def drive(kernels, rows: int, *parts) -> Sequence:
     """What each generator returns."""
-    if rows > FEW_ROWS:
-        if len(parts) == 1:
-            return (_by_itself(kernels, parts[0]),)
-        return [_by_itself(kernels, part) for part in parts]
+    if rows > FEW_ROWS or len(parts) == 1:
+        return [by_itself(kernels, part) for part in parts]
     results, asked = [None] * len(parts), {}
 
     def go(i: int, send) -> None:
@@ -123,25 +121,31 @@ def drive(kernels, rows: int, *parts) -> Sequence:
         go(i, None)
     while asked:
         waiting = dict(asked)
-        todo = [p for i in waiting for p in waiting[i]]
-        done = iter(kernels.linear_group(todo) if _share(todo) else [p.alone() for p in todo])
+        done = iter(_results(kernels, [p for i in waiting for p in waiting[i]]))
         for i, products in waiting.items():
             go(i, [next(done) for _ in products])
     return results
 
 
-def _share(products: list[Product | Routing]) -> bool:
-    """Whether any of the products may find another one to run beside."""
-    return len(products) > 1 and any(isinstance(p, Product) and together(p.x, p.linear) for p in products)
-
-
-def _by_itself(kernels, part):
+def by_itself(kernels, part):
+    """What one generator returns, with nothing beside it."""
     try:
         asked = part.send(None)
         while True:
-            asked = part.send([p.alone() for p in asked] if len(asked) < BLOCK_MOST else kernels.linear_block_group(asked))
+            asked = part.send(_results(kernels, asked))
     except StopIteration as end:
         return end.value
+
+
+def _results(kernels, products: list[Product | Routing]) -> list[torch.Tensor]:
+    if len(products) < 2:
+        return [p.alone() for p in products]
+    if products[0].x.shape[0] > FEW_ROWS:
+        if len(products) >= BLOCK_MOST:
+            return kernels.linear_block_group(products)
+    elif any(isinstance(p, Product) and together(p.x, p.linear) for p in products):
+        return kernels.linear_group(products)
+    return [p.alone() for p in products]
 
 
 def linear_group_plain(products: list[Product | Routing]) -> list[torch.Tensor]:

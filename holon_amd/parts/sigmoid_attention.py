@@ -18,7 +18,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
-from .products import Product, drive, together
+from .products import Product, by_itself, together
 
 _P, _I, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -278,6 +278,6 @@ class SigmoidWindowAttention(Part):
         return (yield [Product(self.o, out)])[0] if together(x, self.o) else self.o(out)
 
     def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
-        return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
+        return by_itself(self.kernels, self.products(x, step, site))
 
     __call__ = forward

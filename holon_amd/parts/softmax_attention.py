@@ -21,7 +21,7 @@ from ..registry import register_part
 from ..spec import PartRef
 from .base import FLOAT32, Build, PagedState, Part
 from .linear import Linear
-from .products import Product, drive, together
+from .products import Product, by_itself, together
 
 _P, _I, _L, _F = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
 _DT = {torch.float32: 0, torch.bfloat16: 1}
@@ -651,7 +651,7 @@ class SoftmaxAttention(Part):
         return k.add_bias(out, self.o_bias) if self.has_o_bias and add_row else out
 
     def forward(self, x: torch.Tensor, step, site, add_row: bool = True, rows: torch.Tensor | None = None) -> torch.Tensor:
-        return drive(self.kernels, x.shape[0], self.products(x, step, site, add_row, rows))[0]
+        return by_itself(self.kernels, self.products(x, step, site, add_row, rows))
 
     __call__ = forward
 
@@ -821,6 +821,6 @@ class LatentAttention(Part):
         return (yield [Product(self.o, out)])[0] if few else self.o(out)
 
     def forward(self, x: torch.Tensor, step, site) -> torch.Tensor:
-        return drive(self.kernels, x.shape[0], self.products(x, step, site))[0]
+        return by_itself(self.kernels, self.products(x, step, site))
 
     __call__ = forward

@@ -153,13 +153,27 @@ def linear_group_plain(products: list[Product | Routing]) -> list[torch.Tensor]:
     return [p.alone() for p in products]
 
 
+def group_pays(m: int, n: int, k: int) -> bool:
+    """Whether a product of m rows over an [n, k] weight joins a launch of several. Not where few waves share its K and each has a long run of it:
+    the launch holds two to sixteen such tiles a block and a wave four loads at a time, which leaves units idle that the product by itself fills.
+    And not the widest weights, which fill the chip by themselves, in blocks that hold two tiles above eight rows. Measured, us, beside
+    2,048 x 2,048, together | one after the other at 1 / 16 rows: 4,096 columns of K 2,816 (8 waves, 11 steps of 32 each) 9.9 | 10.9 and less, 1,408 (4, 11)
+    10.2 | 10.1 at 16 rows, 3,840 (8, 15) 13.9 | 13.8 at 16; 4,352 (8, 17) 16.0 | 14.9 at 16, 11,008 (8, 43) 25.6 | 20.4 and 35.5 | 25.8, 5,504 (4, 43) 20.2 | 15.0
+    and 33.6 | 17.1, 1,440 (1, 45) 18.9 | 10.1 and 25.5 | 11.6; two of 8,192 x 8,192 (8, 32) faster together at any rows, 12,288 x 4,096 at 4 rows, but 42.8 | 41.6 at
+    16; 9,216 x 4,096 27.0 | 25.5, 16,384 x 2,048 15.0 | 15.0 at 4 rows and 19.9 | 17.6 at 16, two of 24,576 x 2,048 35.0 | 33.7 and 45.5 | 35.8."""
+    most = 16 if n < 5120 else 8                            # waves a tile, as the kernels' `skinny_waves` has them
+    waves = next(w for w in (16, 8, 4, 2, 1) if w <= most and k % (32 * w) == 0)
+    return n <= (12288 if m <= 8 else 8192) and (waves == most or k // (32 * waves) <= 15)
+
+
 def _served(p: Product) -> bool:
-    """Whether the few-row product over a tiled copy serves it (what `linear` and `linear_relu2` would run)."""
+    """Whether the few-row product over a tiled copy serves it (what `linear` and `linear_relu2` would run), and a launch of several pays."""
     x, w, tiled = p.x, p.linear.weight, p.linear.tiled
     return (tiled is not None and p.linear.folded is None and x.is_cuda and x.dtype == tiled.dtype == torch.bfloat16 and x.dim() == 2
             and 1 <= x.shape[0] <= FEW_ROWS and x.is_contiguous() and tiled.is_contiguous() and tiled.shape == w.shape
             and x.shape[1] == w.shape[1] and w.shape[0] % 16 == 0 and w.shape[1] % 32 == 0 and w.shape[1] >= 256
-            and x.data_ptr() % 16 == 0 and p.dtype in (None, torch.bfloat16, torch.float32) and not (p.relu2 and p.dtype == torch.float32))
+            and x.data_ptr() % 16 == 0 and p.dtype in (None, torch.bfloat16, torch.float32) and not (p.relu2 and p.dtype == torch.float32)
+            and group_pays(x.shape[0], *w.shape))
 
 
 SCORES = {"softmax": 0, "sigmoid": 1, "sigmoid_squared": 2}
@@ -209,7 +223,9 @@ def block_group_pays(count: int, m: int, n: int, k: int) -> bool:
     library's four take 100. Four products against the library's, inside a graph: 36 | 36 us at 129 rows of 2,048 x 2,048, 37 | 44
     at 400, 42 | 65 at 1,024, 103 | 127 at 3,000, 123 | 155 at 4,096; 2,560 x 2,560: 43 | 43 at 129, 57 | 104 at 1,024, 187 | 221 at
     4,096; 4,096 x 4,096: 71 | 88 at 129, 114 | 181 at 1,024, 308 | 347 at 3,000, then 406 | 385 at 4,096, where one product fills
-    the chip by itself. Two or three gain little or lose at most sizes (three of 4,096 x 4,096 at 1,400 rows 155 | 153)."""
+    the chip by itself. Wider weights gain on the library as long, tile for tile: 8,192 x 2,048 40 | 52 at 129 rows, 102 | 135 at 1,024, 200 | 203 at 2,048 (256
+    tiles a product), 244 | 306 and 288 | 343 at 2,560 and 3,072; 8,192 x 4,096 75 | 96, 197 | 253, 369 | 386, 481 | 547, 577 | 622; 8,192 x 1,024 115 | 123 at 2,048; 5,120 x
+    2,560 226 | 231 at 3,072. 1,024 x 2,048 at 129 and 256 rows 34.7 | 32.7 and 35.2 | 34.5, at 400 35.9 | 38.5. Two or three gain little or lose at most sizes (three of 4,096 x 4,096 at 1,400 rows 155 | 153)."""
     return count == BLOCK_MOST and BLOCK_ROWS[0] <= m <= BLOCK_ROWS[1] and 1024 <= n <= 8192 and 1024 <= k < 8192 and k % 128 == 0 and n % 16 == 0
 
 

@@ -759,3 +759,11 @@ def test_products_that_cannot_share_a_launch_are_run_by_their_part(device, dtype
     assert calls == [2] * asked and torch.equal(one, want) and torch.equal(two, want)
     assert all(torch.equal(y, part.up_proj(x)) for y in drive(part.kernels, rows, three())[0])
     assert calls[asked:] == [3] * (asked > 0)
+
+
+def test_products_join_a_launch_of_several_where_that_pays():
+    """`group_pays` on both sides of its lines: long runs of K to few waves, wide weights by the rows."""
+    from holon_amd.parts.products import group_pays
+    assert all(group_pays(m, n, k) for m in (1, 16) for n, k in ((64, 256), (2048, 8192), (512, 480), (4096, 2816), (5104, 3840), (8192, 8192), (8192, 3840)))
+    assert not any(group_pays(m, n, k) for m in (1, 16) for n, k in ((512, 512 + 32), (2048, 4352), (2048, 11008), (4096, 5504), (8192, 5504), (512, 1440)))
+    assert [group_pays(m, n, 2048) for m, n in ((8, 12288), (8, 12304), (9, 8192), (9, 8208))] == [True, False, True, False]

@@ -172,8 +172,9 @@ __device__ __forceinline__ void widen4(const ushort4& h, float (&v)[4]) {
 // through its causal filter of TAPS taps before it is stored (see `filter4`).
 // AHEAD: the terms, the weights and the results are of one type (DT), and everything that the row needs is asked for before any of it is
 // read: a step of few rows is a block or a few, and what it takes is one memory latency after the other, where a branch on a type
-// stands around each load. One row of 2,048 (two terms, one weight) 3.1 us -> 2.5, with the added vector, two weights and filters 4.6 ->
-// 3.7; of 4,096 4.4 -> 3.1 and 7.2 -> 5.4; 2,048 rows of 2,048 9.2 -> 8.7. Rows beyond 4,096 would hold more than the registers are worth.
+// stands around each load (a weight of another type than the terms, as a norm's float32 weight beside bfloat16, takes the general
+// form). One row of 2,048 (two terms, one weight) 3.1 us -> 2.5, with the added vector, two weights and filters 4.6 -> 3.7; of 4,096 4.4 ->
+// 3.1 and 7.2 -> 5.4; 2,048 rows of 2,048 9.2 -> 8.7. Rows beyond 4,096 would hold more than the registers are worth.
 template <int REGS, int TAPS, int DT = HOLON_BF16, bool AHEAD = false>     // DT: read when TAPS > 0 or AHEAD
 __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__ x32, const void* __restrict__ d1, int dt1,
                                                              const void* __restrict__ d2, int dt2,

@@ -48,7 +48,9 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 def glu_block_pays(rows: int, inter: int, hidden: int) -> bool:
     """Whether a gated first product of many rows with its activation takes this package's 256 x 256 tiles (128 gates and their ups each):
     where the rounds of one tile a compute unit that it takes are filled to 0.62 and more (`hidden` does not enter: either side's time
-    is in proportion to it; tiles of 192 columns, taken where their rounds end sooner, make the line a cautious one). Measured on MI355X, us,
+    is in proportion to it). Tiles of 192 columns, taken where their rounds end sooner, are not counted: the line leaves
+    products to the library that are shorter here, 8,192 x 2,048 at 400 rows and 9,728 x 2,560 at 1,024 below, and at the same filling
+    12,288 x 4,096 at 600, which is not. Measured on MI355X, us,
     against the vendor library's product and the kernel of the activation: 12,288 x 4,096 at 520 / 600 / 1,024 / 2,048 / 4,096 rows (filled
     0.76 / 0.44 / 0.75 / 1 / 1) 97 / 134 / 153 / 280 / 551 and 124 / 124 / 176 / 307 / 596; 8,192 x 2,048 at 400 / 768 / 1,024 / 2,048 (0.39 /
     0.75 / 1 / 1) 34 / 45 / 52 / 101 and 39 / 52 / 65 / 122; 9,728 x 2,560 at 1,024 / 1,500 (0.59 / 0.87) 104 / 122 and 114 / 142."""

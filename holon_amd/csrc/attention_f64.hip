@@ -22,6 +22,8 @@
 // behind 500 41 and 70. Each head its own keys, a column a token: 37 / 700 tokens 21 / 142 and 10 / 412.
 #include <float.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "holon_hip.h"
 
@@ -94,13 +96,17 @@ __global__ void __launch_bounds__(SPLIT ? WAVE : WAVES * WAVE, SPLIT ? 1 : 2) at
   const int first = pos >= 0 ? max(0, first_seen(pos, a.window)) : 0;
 
   int last = live ? pos : -1, least = live ? pos : 0x7fffffff, from = live ? first : 0x7fffffff, whole_from = live ? first : 0;
-#pragma unroll
-  for (int o = 1; o < 16; o *= 2) {
-    last = max(last, __shfl_xor(last, o, WAVE));
-    least = min(least, __shfl_xor(least, o, WAVE));
-    from = min(from, __shfl_xor(from, o, WAVE));
-    whole_from = max(whole_from, __shfl_xor(whole_from, o, WAVE));
-  }
+  const auto columns = [&](auto distance) {                // over the 16 lanes of a group of columns
+    constexpr int O = decltype(distance)::value;
+    last = max(last, lane_xor<O>(last));
+    least = min(least, lane_xor<O>(least));
+    from = min(from, lane_xor<O>(from));
+    whole_from = max(whole_from, lane_xor<O>(whole_from));
+  };
+  columns(std::integral_constant<int, 1>{});
+  columns(std::integral_constant<int, 2>{});
+  columns(std::integral_constant<int, 4>{});
+  columns(std::integral_constant<int, 8>{});
   last = __builtin_amdgcn_readfirstlane(last);
   from = __builtin_amdgcn_readfirstlane(from);
   const int slot = min(max(a.slots[row], 0), a.table_rows - 1);
@@ -154,8 +160,8 @@ __global__ void __launch_bounds__(SPLIT ? WAVE : WAVES * WAVE, SPLIT ? 1 : 2) at
         if (MOD && a.r1 != nullptr) s[r] -= b1 * log1pf(b2 * (float)max(pos - mine0 - r, 0));
         if (seen[r]) mx = fmaxf(mx, s[r]);
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+      mx = xor_max<16>(mx);
+      mx = xor_max<32>(mx);
       const float m_new = fmaxf(m, mx), at = m_new == -INFINITY ? 0.f : m_new;    // (a score that is NaN stays one)
       const float alpha = expf(m - at);
       float p[4], sum = 0.f;
@@ -164,8 +170,8 @@ __global__ void __launch_bounds__(SPLIT ? WAVE : WAVES * WAVE, SPLIT ? 1 : 2) at
         p[r] = seen[r] ? expf(s[r] - at) : 0.f;
         sum += p[r];
       }
-      sum += __shfl_xor(sum, 16, WAVE);
-      sum += __shfl_xor(sum, 32, WAVE);
+      sum = xor_sum<16>(sum);
+      sum = xor_sum<32>(sum);
       l = l * alpha + sum;
       if (__any(m_new != m)) {
 #pragma unroll

@@ -160,8 +160,8 @@ __global__ void __launch_bounds__(SPLIT ? WAVE : WAVES * WAVE) attention_generic
       }
 #pragma unroll
       for (int h = 0; h < HG; ++h) {
-        dot[h] += __shfl_xor(dot[h], 1, WAVE);
-        dot[h] += __shfl_xor(dot[h], 2, WAVE);
+        dot[h] += lane_xor<1>(dot[h]);
+        dot[h] += lane_xor<2>(dot[h]);
         if (r == part && key <= pos) s[h] = (float)dot[h] * scale;
       }
     }

@@ -458,8 +458,8 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(AttnArgs a) {
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     float lt = l[t];
-    lt += __shfl_xor(lt, 16, WAVE);
-    lt += __shfl_xor(lt, 32, WAVE);
+    lt = xor_sum<16>(lt);
+    lt = xor_sum<32>(lt);
     if (!rr[t].valid) continue;
     lt = with_sink(a, rr[t].token, rr[t].head, lt, m[t]);
     const float inv = lt > 0.f ? 1.0f / lt : 0.f;
@@ -662,8 +662,8 @@ __global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       float lt = l[t];
-      lt += __shfl_xor(lt, 16, WAVE);
-      lt += __shfl_xor(lt, 32, WAVE);
+      lt = xor_sum<16>(lt);
+      lt = xor_sum<32>(lt);
       if (!rr[t].valid) continue;
       lt = with_sink(a, rr[t].token, rr[t].head, lt, m[t]);
       const float inv = lt > 0.f ? 1.0f / lt : 0.f;
@@ -935,7 +935,7 @@ __global__ void __launch_bounds__(256, D == 128 ? 2 : 3) attn_prefill_wide_kerne
     } else {
       stage(std::true_type{}, kb, 0, r1);
     }
-    float lt = l + __shfl_xor(l, 32, WAVE);
+    float lt = xor_sum<32>(l);
     if (valid) {
       if (!SIG) lt = with_sink(a, token, head, lt, m);
       const float inv = SIG ? 1.0f : (lt > 0.f ? 1.0f / lt : 0.f);
@@ -1271,7 +1271,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dma_kernel(AttnArgs a) {
       buf = SC::after(buf);
     }
     stage(std::true_type{}, kb_last, buf, key_hi);
-    float lt = l + __shfl_xor(l, 32, WAVE);
+    float lt = xor_sum<32>(l);
     if (valid) {
       lt = with_sink(a, token, head, lt, m);
       const float inv = lt > 0.f ? 1.0f / lt : 0.f;
@@ -1519,7 +1519,7 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_pair_kernel(AttnArgs a) {
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      float lt = l[t] + __shfl_xor(l[t], 32, WAVE);
+      float lt = xor_sum<32>(l[t]);
       if (valid[t]) {
         lt = with_sink(a, token[t], head, lt, m[t]);
         const float inv = lt > 0.f ? 1.0f / lt : 0.f;
@@ -1585,8 +1585,7 @@ struct NewKeyValue {
       float ss = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss += v[j] * v[j];
-#pragma unroll
-      for (int o = LPH / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, WAVE);
+      ss = lanes_sum<LPH>(ss);
       const float inv = 1.0f / sqrtf(ss / (float)D + f.eps);
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = (float)(__bf16)((v[j] * inv) * bf16_to_float(w[j]));
@@ -1600,7 +1599,7 @@ struct NewKeyValue {
       *reinterpret_cast<float4*>(si + 4) = *reinterpret_cast<const float4*>(cs + D / 2 + 4);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float other = __shfl_xor(v[j], LPH / 2, WAVE);
+        const float other = lane_xor<LPH / 2>(v[j]);
         v[j] = li < LPH / 2 ? v[j] * co[j] - other * si[j] : v[j] * co[j] + other * si[j];
       }
     }
@@ -1732,8 +1731,8 @@ __global__ void __launch_bounds__(D == 256 ? 256 : 512) attn_decode_kernel(AttnA
           }
         }
         if (f.q_weight != nullptr) {     // the sum of squares over the four lane groups, then round((x inv) w)
-          ss += __shfl_xor(ss, 16, WAVE);
-          ss += __shfl_xor(ss, 32, WAVE);
+          ss = xor_sum<16>(ss);
+          ss = xor_sum<32>(ss);
           const float inv = 1.0f / sqrtf(ss / (float)D + f.eps);
 #pragma unroll
           for (int ks = 0; ks < D / 32; ++ks) {
@@ -1776,8 +1775,8 @@ __global__ void __launch_bounds__(D == 256 ? 256 : 512) attn_decode_kernel(AttnA
     }
   }
   float lt = l[0];
-  lt += __shfl_xor(lt, 16, WAVE);
-  lt += __shfl_xor(lt, 32, WAVE);
+  lt = xor_sum<16>(lt);
+  lt = xor_sum<32>(lt);
   float mt = m[0];
   if (waves > 1) {                       // the block's partials, added up in wave order by wave 0
     if (wave > 0) {
@@ -1876,7 +1875,7 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict
     const float big = wave_max(m_s);
     const float w_s = l_s > 0.f ? exp2f(m_s - big) : 0.f;
     float denom = 0.f;                     // in split order
-    for (int s = 0; s < splits; ++s) denom += __shfl(w_s * l_s, s, WAVE);
+    for (int s = 0; s < splits; ++s) denom += of_lane(w_s * l_s, s);
     if (sink != nullptr && big != -INFINITY) denom += exp2f(sink[h] * 1.4426950408889634f - big);
     if (hgate != nullptr) denom *= 1.0f + __expf(-bf16_to_float(hgate[(int64_t)token * hgate_stride + h]));
     weight[tid] = w_s;

@@ -49,15 +49,72 @@ template <int ACT, typename T> __device__ __forceinline__ float gate_act(float z
   else return silu<T>(z);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-  return v;
+// What lane ^ O holds (O a power of two below 64), by register moves instead of the shuffles' way through LDS (each of them
+// about a tenth of a microsecond that a row's sum waits for): inside a quad and inside a row of 16 lanes by data-parallel
+// moves, between rows of 16 and halves of the wave by gfx950's swaps. Every lane of the wave has to be there (and blocks are of one
+// dimension, as all of this package's are). Measured over whole traces, the same bits: four rows a step in 68 kernels 25.74 ms ->
+// 25.20, sixteen rows 12.99 -> 12.81, float32 rows 10.53 -> 10.42.
+template <int O>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  static_assert(O == 1 || O == 2 || O == 4 || O == 8 || O == 16 || O == 32, "a power of two inside the wave");
+  if constexpr (O == 1) return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);           // quad_perm:[1,0,3,2]
+  else if constexpr (O == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);      // quad_perm:[2,3,0,1]
+  else if constexpr (O == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);     // row_ror:8
+  else if constexpr (O == 4) {                             // quads 0, 2 of a row look four lanes up, quads 1, 3 four down
+    const uint32_t up = __builtin_amdgcn_update_dpp(0, v, 0x104, 0xf, 0x5, false);
+    return __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false);
+  } else if constexpr (O == 16) {                          // [0]: what the even rows hold, twice; [1]: the odd rows
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return threadIdx.x & 16 ? r[0] : r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return threadIdx.x & 32 ? r[0] : r[1];
+  }
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-  return v;
+template <int O> __device__ __forceinline__ float lane_xor(float v) { return __uint_as_float(lane_xor<O>(__float_as_uint(v))); }
+template <int O> __device__ __forceinline__ int lane_xor(int v) { return (int)lane_xor<O>((uint32_t)v); }
+template <int O> __device__ __forceinline__ double lane_xor(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)lane_xor<O>((uint32_t)(b >> 32)) << 32 | lane_xor<O>((uint32_t)b));
+}
+// op(a lane's value, what lane ^ O holds), the same number in both lanes; for an op that may take its operands either way round.
+template <int O, typename Op>
+__device__ __forceinline__ float with_xor(float v, Op op) {
+  if constexpr (O == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (O == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else {
+    return op(v, lane_xor<O>(v));
+  }
+}
+// Over groups of N neighbouring lanes, by N / 2, N / 4, .. 1, every lane its group's: the very sums that shuffles by those
+// distances give. (Below a step by 8 the row holds everything twice, so the step by 4 may turn the row instead of swapping quads.)
+template <int N, typename Op>
+__device__ __forceinline__ float over_lanes(float v, Op op) {
+  static_assert(N == 2 || N == 4 || N == 8 || N == 16 || N == 32 || N == 64, "a power of two inside the wave");
+  if constexpr (N >= 64) v = with_xor<32>(v, op);
+  if constexpr (N >= 32) v = with_xor<16>(v, op);
+  if constexpr (N >= 16) {
+    v = with_xor<8>(v, op);
+    v = op(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x124, 0xf, 0xf, true)));   // row_ror:4
+  } else if constexpr (N == 8) {
+    v = with_xor<4>(v, op);
+  }
+  if constexpr (N >= 4) v = with_xor<2>(v, op);
+  return with_xor<1>(v, op);
+}
+template <int N> __device__ __forceinline__ float lanes_sum(float v) { return over_lanes<N>(v, [](float a, float b) { return a + b; }); }
+template <int N> __device__ __forceinline__ float lanes_max(float v) { return over_lanes<N>(v, [](float a, float b) { return fmaxf(a, b); }); }
+template <int O> __device__ __forceinline__ float xor_sum(float v) { return with_xor<O>(v, [](float a, float b) { return a + b; }); }
+template <int O> __device__ __forceinline__ float xor_max(float v) { return with_xor<O>(v, [](float a, float b) { return fmaxf(a, b); }); }
+__device__ __forceinline__ float wave_sum(float v) { return lanes_sum<WAVE>(v); }
+__device__ __forceinline__ float wave_max(float v) { return lanes_max<WAVE>(v); }
+// What lane `from` (the same in all lanes) holds.
+__device__ __forceinline__ float of_lane(float v, int from) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), from));
 }
 
 // A copy from memory straight into LDS (global_load_lds_dwordx4): 16 bytes a lane, the wave's 64 lanes into one

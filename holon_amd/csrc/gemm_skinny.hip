@@ -74,9 +74,7 @@ struct RowSums {
 // l ^ 8, l ^ 16, l ^ 32, in that order), then column c out of lane c / 4. Every lane of column c gets the same sum.
 __device__ __forceinline__ float row_sum_of_column(f32x4_t v, int c) {
 #pragma unroll
-  for (int o = 4; o < WAVE; o <<= 1)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] += __shfl_xor(v[i], o, WAVE);
+  for (int i = 0; i < 4; ++i) v[i] = xor_sum<32>(xor_sum<16>(xor_sum<8>(xor_sum<4>(v[i]))));
   const float t0 = __shfl(v[0], c / 4, WAVE), t1 = __shfl(v[1], c / 4, WAVE), t2 = __shfl(v[2], c / 4, WAVE),
               t3 = __shfl(v[3], c / 4, WAVE);
   return c % 4 == 0 ? t0 : (c % 4 == 1 ? t1 : (c % 4 == 2 ? t2 : t3));

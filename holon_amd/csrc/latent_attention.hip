@@ -334,8 +334,8 @@ __global__ void __launch_bounds__(512, 2) latent_prefill_kernel(LatArgs a) {
     wait_loads_but<0>();                                 // the next stage has landed (this wave's share of it)
     lds_barrier();
   }
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
+  l = xor_sum<16>(l);
+  l = xor_sum<32>(l);
   if (g == 0) max_s[kh][rt * 16 + c] = l;
   if (g == 0 && kh == 0) alpha_s[rt * 16 + c] = valid && a.sink ? __builtin_amdgcn_exp2f(a.sink[head] * 1.4426950408889634f - m) : 0.f;
   lds_barrier();
@@ -451,8 +451,8 @@ __global__ void __launch_bounds__(256, 2) latent_decode_kernel(LatArgs a) {
       }
     }
   }
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
+  l = xor_sum<16>(l);
+  l = xor_sum<32>(l);
   lds_barrier();                                         // every wave has read the last maxima
   if (g == 0) red_s[wave][c] = l;
   lds_barrier();

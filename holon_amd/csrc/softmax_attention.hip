@@ -282,10 +282,7 @@ __global__ void __launch_bounds__(256) head_linear_kernel(const T* __restrict__ 
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       float v = acc[r];
-      v += __shfl_xor(v, 1, WAVE);
-      v += __shfl_xor(v, 2, WAVE);
-      v += __shfl_xor(v, 4, WAVE);
-      v += __shfl_xor(v, 8, WAVE);
+      v = xor_sum<8>(xor_sum<4>(xor_sum<2>(xor_sum<1>(v))));
       if (part == 0 && b < B && t0 + r < rows) {
         if (gate) v *= 1.0f / (1.0f + expf(-Elem<T>::load(gate[(t0 + r) * gate_stride + (int64_t)h * B + b])));
         y[((int64_t)(t0 + r) * heads + h) * y_head + b] = Elem<T>::store(v);

@@ -1986,3 +1986,32 @@ def test_decay_projection_of_any_number_of_channels(hip, dtype, tokens, channels
     hip._call(hip.lib.holon_decay_lora, a.data_ptr(), w.data_ptr(), w0.data_ptr(), y.data_ptr(), tokens, channels, rank,
               int(dtype == torch.bfloat16), hip._stream())
     assert torch.equal(y[:-4].view(tokens, channels), hip.decay_lora(a, w2t, w0)[:, :channels]) and (y[-4:] == 7.0).all()
+
+
+@pytest.mark.parametrize("waves", [1, 16])
+def test_moves_between_lanes_are_the_shuffles(waves):
+    """Bit for bit what lane ^ o holds and what sums and maxima over steps by n / 2 .. 1 are; infinities, both zeros, tiny values."""
+    import ctypes
+    import pathlib
+    from holon_amd.kernels import build
+    source = pathlib.Path(__file__).parent / "kernels" / "lanes.hip"
+    fn = ctypes.CDLL(str(build.source_library(source) or build.build_source(source))).test_lanes
+    fn.argtypes, fn.restype = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p], ctypes.c_int
+    rng = np.random.default_rng(waves)
+    x = (rng.standard_normal((waves, 64)) * 10.0 ** rng.integers(-8, 8, (waves, 64))).astype(np.float32)
+    x[:, 3], x[:, 17], x[:, 40], x[:, 55] = np.float32(np.inf), 0.0, -0.0, np.finfo(np.float32).min
+    out = torch.full((waves, 7, 6, 64), torch.nan, device="cuda")
+    given = torch.from_numpy(x).cuda()
+    assert fn(given.data_ptr(), out.data_ptr(), waves, torch.cuda.current_stream().cuda_stream) == 0
+    got, lane = out.cpu().numpy(), np.arange(64)
+    for n, o in enumerate((1, 2, 4, 8, 16, 32)):
+        other = x[:, lane ^ o]
+        total, top = x, x
+        for step in (s for s in (32, 16, 8, 4, 2, 1) if s <= o):
+            total, top = total + total[:, lane ^ step], np.maximum(top, top[:, lane ^ step])
+        want = (other, x + other, np.maximum(x, other), total, top, np.broadcast_to((lane ^ o).astype(np.float32), x.shape),
+                np.broadcast_to(x[:, 2 * o - 1: 2 * o], x.shape))
+        for k, w in enumerate(want):
+            have, w = got[:, k, n], np.ascontiguousarray(w, np.float32)
+            same = have == w if k in (2, 4) else have.view(np.uint32) == w.view(np.uint32)      # (a maximum: either zero)
+            assert same.all(), (k, o)

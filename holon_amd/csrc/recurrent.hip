@@ -9,6 +9,7 @@
 // fixed order. Each token's key and query reach the lanes through LDS. The key size is padded to the next instantiated
 // one with zeros (a zero key writes nothing).
 #include "common.h"
+#include "head_rows.h"
 #include "holon_hip.h"
 
 namespace {
@@ -488,6 +489,33 @@ __global__ void __launch_bounds__(256) gated_out_kernel(const float* __restrict_
   }
 }
 
+// The same for heads of 64, 128 and 256 (LANES 8, 16, 32) on borders of 16 bytes: eight neighbouring values a lane, 64 / LANES cells a wave, every
+// load under way before a sum is taken. The same bits. 2,048 tokens of 32 heads of 64 7.6 us, a value a lane at a time 20.8 (33 MB: 6.8
+// at a copy's rate).
+template <typename T, int LANES>
+__global__ void __launch_bounds__(256) gated_out_rows_kernel(const float* __restrict__ o, const T* __restrict__ gate,
+                                                             const T* __restrict__ weight, T* __restrict__ y, int64_t cells, int heads,
+                                                             int per_head, float eps, int64_t gate_stride, int plain_sigmoid,
+                                                             const float* __restrict__ den) {
+  constexpr int D = LANES * 8, PER = WAVE / LANES;
+  const int lane = threadIdx.x % WAVE, d0 = lane % LANES * 8;
+  const int64_t cell = ((int64_t)blockIdx.x * 4 + threadIdx.x / WAVE) * PER + lane / LANES, at = min(cell, cells - 1);
+  const int h = (int)(at % heads);
+  float v[8], wv[8], gv[8];
+  head_rows::load8(o + at * D + d0, v);
+  head_rows::load8(weight + (per_head ? h * D : 0) + d0, wv);
+  head_rows::load8(gate + (at / heads) * gate_stride + (int64_t)h * D + d0, gv);
+  if (den) {
+    const float under = den[at];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = v[j] / under;
+  }
+  const float r = 1.0f / sqrtf(head_rows::sum_of_squares<LANES>(v, lane) / (float)D + eps);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = v[j] * r * wv[j] * (plain_sigmoid ? 1.0f / (1.0f + expf(-gv[j])) : silu<T>(gv[j]));
+  if (cell < cells) head_rows::store8(y + cell * D + d0, v);
+}
+
 template <typename T>
 __global__ void shift_mix_kernel(const T* __restrict__ x, const T* __restrict__ mu, T* __restrict__ state,
                                  T* __restrict__ y, const int32_t* __restrict__ slots, const int32_t* __restrict__ starts,
@@ -504,6 +532,31 @@ __global__ void shift_mix_kernel(const T* __restrict__ x, const T* __restrict__ 
   for (int s = 0; s < mixes; ++s)
     y[((int64_t)s * tokens + t) * width + c] = Elem<T>::store(cur + (prev - cur) * Elem<T>::load(mu[(int64_t)s * width + c]));
   if (keep) state[(int64_t)slots[b] * width + c] = x[(int64_t)t * width + c];
+}
+
+// The same, eight neighbouring channels a thread: 2,048 tokens of 2,048, mixed five times, 12.1 us, a channel a thread 23.
+template <typename T>
+__global__ void __launch_bounds__(256) shift_mix_rows_kernel(const T* __restrict__ x, const T* __restrict__ mu, T* __restrict__ state,
+                                                             T* __restrict__ y, const int32_t* __restrict__ slots,
+                                                             const int32_t* __restrict__ starts, const int32_t* __restrict__ query_start,
+                                                             const int32_t* __restrict__ token_row, int tokens, int width, int mixes,
+                                                             int keep) {
+  const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
+  const int t = blockIdx.y;
+  if (c >= width) return;
+  const int b = keep ? t : token_row[t];
+  float prev[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, cur[8];
+  head_rows::load8(x + (int64_t)t * width + c, cur);
+  if (!keep && t > query_start[b]) head_rows::load8(x + (int64_t)(t - 1) * width + c, prev);
+  else if (starts[b] > 0) head_rows::load8(state + (int64_t)slots[b] * width + c, prev);
+  for (int s = 0; s < mixes; ++s) {
+    float m[8];
+    head_rows::load8(mu + (int64_t)s * width + c, m);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m[j] = cur[j] + (prev[j] - cur[j]) * m[j];
+    head_rows::store8(y + ((int64_t)s * tokens + t) * width + c, m);
+  }
+  if (keep) head_rows::store8(state + (int64_t)slots[b] * width + c, cur);
 }
 
 template <typename T>
@@ -763,9 +816,19 @@ extern "C" int holon_gated_out(const float* o, const void* gate, const void* wei
   const int64_t cells = (int64_t)tokens * heads;
   if (cells == 0) return 0;
   HOLON_CHECK((cells + 3) / 4 <= 0x7fffffff, "gated_out: %lld cells exceed one launch", (long long)cells);
-  BY_DTYPE(dtype, (gated_out_kernel<T><<<(unsigned)((cells + 3) / 4), 256, 0, (hipStream_t)stream>>>(
-                      o, (const T*)gate, (const T*)weight, (T*)y, cells, heads, vdim, per_head, eps, gate_stride,
-                      plain_sigmoid, den)));
+  hipStream_t s = (hipStream_t)stream;
+#define GATED_ROWS(LANES)                                                                                                         \
+  BY_DTYPE(dtype, (gated_out_rows_kernel<T, LANES><<<(unsigned)((cells * LANES + 255) / 256), 256, 0, s>>>(                         \
+                      o, (const T*)gate, (const T*)weight, (T*)y, cells, heads, per_head, eps, gate_stride, plain_sigmoid, den)))
+  const bool pieces = gate_stride % 8 == 0 && head_rows::on16(o) && head_rows::on16(gate) && head_rows::on16(weight) && head_rows::on16(y);
+  if (pieces && vdim == 64) GATED_ROWS(8);
+  else if (pieces && vdim == 128) GATED_ROWS(16);
+  else if (pieces && vdim == 256) GATED_ROWS(32);
+  else
+    BY_DTYPE(dtype, (gated_out_kernel<T><<<(unsigned)((cells + 3) / 4), 256, 0, s>>>(
+                        o, (const T*)gate, (const T*)weight, (T*)y, cells, heads, vdim, per_head, eps, gate_stride,
+                        plain_sigmoid, den)));
+#undef GATED_ROWS
   HOLON_LAUNCH_OK();
   return 0;
 }
@@ -782,9 +845,14 @@ extern "C" int holon_shift_mix(const void* x, const void* mu, void* state, void*
   const dim3 block(256), grid_t((width + 255) / 256, tokens), grid_b((width + 255) / 256, rows);
   HOLON_CHECK(!rows_in_order || tokens == rows, "shift_mix: rows in order means one token a row, got %d in %d", tokens,
               rows);
-  BY_DTYPE(dtype, (shift_mix_kernel<T><<<grid_t, block, 0, s>>>((const T*)x, (const T*)mu, (T*)state, (T*)y, slots, starts,
-                                                                query_start, token_row, tokens, width, mixes,
-                                                                rows_in_order)));
+  if (width % 8 == 0 && head_rows::on16(x) && head_rows::on16(mu) && head_rows::on16(state) && head_rows::on16(y))
+    BY_DTYPE(dtype, (shift_mix_rows_kernel<T><<<dim3((width + 2047) / 2048, tokens), block, 0, s>>>(
+                        (const T*)x, (const T*)mu, (T*)state, (T*)y, slots, starts, query_start, token_row, tokens, width, mixes,
+                        rows_in_order)));
+  else
+    BY_DTYPE(dtype, (shift_mix_kernel<T><<<grid_t, block, 0, s>>>((const T*)x, (const T*)mu, (T*)state, (T*)y, slots, starts,
+                                                                  query_start, token_row, tokens, width, mixes,
+                                                                  rows_in_order)));
   HOLON_LAUNCH_OK();
   if (rows_in_order) return 0;                           // the one kernel has kept each row's token
   BY_DTYPE(dtype, (shift_keep_kernel<T><<<grid_b, block, 0, s>>>((const T*)x, (T*)state, slots, query_start, width)));

@@ -2015,3 +2015,80 @@ def test_moves_between_lanes_are_the_shuffles(waves):
             have, w = got[:, k, n], np.ascontiguousarray(w, np.float32)
             same = have == w if k in (2, 4) else have.view(np.uint32) == w.view(np.uint32)      # (a maximum: either zero)
             assert same.all(), (k, o)
+
+
+def _moved(t, by=1):
+    """The same values where no border of 16 bytes is: kernels that take pieces of eight values leave them to the general form."""
+    return torch.empty(t.numel() + by, dtype=t.dtype, device=t.device)[by:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_heads_in_pieces_are_the_heads_value_by_value(hip, dtype, dim):
+    """q, k and v prepared, read-outs normed and gated, two maps combined: eight values a lane bit for bit as a value a lane; heads that do
+    not fill a wave, every rotated width on and off the middle of a head, tokens without a place in the cache."""
+    heads, kv, page_size, t, pages_n = 5, 2, 16, 19, 3
+    positions = torch.arange(t, dtype=torch.int32).cuda() * 7 % 40
+    write_page = (torch.arange(t, dtype=torch.int32) // page_size).cuda()
+    write_off = (torch.arange(t, dtype=torch.int32) % page_size).cuda()
+    write_page[3], write_off[5] = -1, page_size
+    for rot in (0, 16, 48, dim // 2, dim):
+        table = _randn(40, rot, dtype=torch.float32, seed=200) if rot else None
+        for normed, biased, values, share, vdim in ((True, False, "own", 1, dim), (False, False, "own", 2, 24), (True, True, "own", 1, 40),
+                                                    (False, True, "keys", 1, dim)):
+            width = (heads + kv) * dim + (0 if values == "keys" else kv // share * vdim)
+            qkv = _randn(t, width + 8, dtype=dtype, seed=201, scale=2.0)
+            weights = [1 + 0.2 * _randn(dim, dtype=dtype, seed=202 + i) for i in range(2)] if normed else [None, None]
+            bias = _randn(width, dtype=torch.float32, seed=204) if biased else None
+            v_heads = kv if values == "keys" else kv // share
+            made = []
+            for rows in (qkv, _moved(qkv)):
+                pages = torch.zeros(pages_n, kv * page_size * dim + v_heads * page_size * vdim, dtype=dtype, device="cuda")
+                q = hip.head_prepare(rows, heads, kv, dim, vdim, *weights, 1e-5, table, positions, pages, write_page, write_off, page_size,
+                                     bias=bias, values=values, value_share=share)
+                made.append((q, pages))
+            assert all(torch.equal(a, b) for a, b in zip(*made)), (rot, normed, biased, values, share)
+    for cells in (1, 7, 33):
+        o, gate = _randn(cells, heads, dim, dtype=torch.float32, seed=205), _randn(cells, heads * dim + 8, dtype=dtype, seed=206)
+        den = _randn(cells, heads, dtype=torch.float32, seed=207).abs() + 0.1
+        for per_head in (False, True):
+            w = 1 + 0.2 * _randn(heads * dim if per_head else dim, dtype=dtype, seed=208)
+            for act, under in (("silu", None), ("sigmoid", den)):
+                got, want = (hip.gated_out(x, gate[:, : heads * dim], w, per_head, 1e-6, dtype, act=act, den=under) for x in (o, _moved(o)))
+                assert torch.equal(got, want), (cells, per_head, act)
+        y = _randn(cells, 2 * 4 * dim, dtype=dtype, seed=209)
+        got, want = (hip.diff_combine(x, 4, 2, dim, 0.35, 1e-5, 0.65) for x in (y, _moved(y)))
+        assert torch.equal(got, want), cells
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_in_pieces_are_the_rows_value_by_value(hip, dtype):
+    """Token shifts and a latent's entries and queries: eight values a thread bit for bit as a value a thread."""
+    for width in (8, 2040, 2048, 2056):
+        counts = [1, 5, 17]
+        starts, slots = torch.tensor([0, 3, 9], dtype=torch.int32).cuda(), torch.tensor([2, 0, 3], dtype=torch.int32).cuda()
+        first = torch.tensor([0, 1, 6, 23], dtype=torch.int32).cuda()
+        row = torch.repeat_interleave(torch.arange(3), torch.tensor(counts)).to(torch.int32).cuda()
+        x, mu = _randn(23, width, dtype=dtype, seed=210), _randn(5, width, dtype=dtype, seed=211)
+        made = []
+        for rows in (x, _moved(x)):
+            state = _randn(4, width, dtype=dtype, seed=212)
+            y = hip.shift_mix(rows, mu, state, slots, starts, first, row, 3)
+            step = hip.shift_mix(rows[:3].clone() if rows is x else _moved(rows[:3]), mu, state, slots, starts, first, row, 3, in_order=True)
+            made.append((y, step, state))
+        assert all(torch.equal(a, b) for a, b in zip(*made)), width
+    t, page_size = 257, 16
+    positions = (torch.arange(t, dtype=torch.int32) % 50).cuda()
+    write_page = (torch.arange(t, dtype=torch.int32) // page_size).cuda()
+    write_off = (torch.arange(t, dtype=torch.int32) % page_size).cuda()
+    write_page[7] = 99
+    for heads, dim, rot, rank, rd, copies in ((3, 128, 64, 192, 64, 1), (16, 8, 16, 24, 16, 2), (5, 72, 24, 512, 16, 2), (2, 64, 0, 64, 0, 1)):
+        both = _randn(t, heads * (dim + rot) + rank + rot + 8, dtype=dtype, seed=213)
+        table = _randn(50, rd, dtype=torch.float32, seed=214) if rd else None
+        weight, made = 1 + 0.2 * _randn(rank, dtype=dtype, seed=215), []
+        for rows in (both, _moved(both)):
+            pages = torch.zeros(-(-t // page_size), copies * page_size * (rank + rot), dtype=dtype, device="cuda")
+            q, full = hip.latent_rope_prepare(rows, heads, dim, rot, rank, weight, 1e-5, table, positions, pages, write_page, write_off, page_size,
+                                              copies=copies)
+            made.append((q, full[..., rank:].clone(), pages))
+        assert all(torch.equal(a, b) for a, b in zip(*made)), (heads, dim, rot, rank, rd, copies)

@@ -1,5 +1,7 @@
 // The elementwise steps of two feed-forward kinds: the PolyNorm activation of a dense one, and the router's choice and
 // the gated activation of a mixture of experts. float32 inside; sums over a row in an order its width alone decides.
+#include <type_traits>
+
 #include "common.h"
 #include "holon_hip.h"
 #include "moe_router.h"
@@ -191,6 +193,81 @@ __global__ void __launch_bounds__(moe_router::BLOCK_WAVES * WAVE) moe_router_few
     int width, int experts, int rows_r, int top, int groups, int keep, int score, float scale) {
   __shared__ moe_router::Lds lds;
   moe_router::few_token<T, PARTS>(lds, blockIdx.x, x, router, bias, weights, width, experts, rows_r, top, groups, keep, score, scale);
+}
+
+// The router of up to 64 experts for many rows, both kinds: TOK tokens a wave, so that TOK rows share what is read of the router (128 KB a
+// token at 8 experts of 4,096: more than all else a step of many rows reads here), E of its rows at a time, the next loads under way
+// while the last are multiplied. Logits are added up and the choice is made as moe_router.h has them. Rows of 4,096 over 8 experts:
+// 4,096 of them 21 us, 2,154 20, a block a token 76 and 41; 1,800 of 2,048 over 9 (PARTS 4) 16, a block a token 22.
+template <typename T, int PARTS, int TOK, int E>
+__global__ void __launch_bounds__(256) moe_router_rows_kernel(const T* __restrict__ x, const float* __restrict__ router,
+                                                              const float* __restrict__ bias, float* __restrict__ weights, int64_t rows,
+                                                              int width, int experts, int rows_r, int top, int groups, int keep, int score,
+                                                              float scale) {
+  __shared__ moe_router::Lds lds[4][TOK];
+  struct Four { T v[4]; };                                  // (aligned as T is; one load all the same)
+  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const int64_t t0 = ((int64_t)blockIdx.x * 4 + wave) * TOK;
+  const T* row[TOK];
+#pragma unroll
+  for (int n = 0; n < TOK; ++n) row[n] = x + min(t0 + n, rows - 1) * width;
+  for (int e0 = 0; e0 < rows_r; e0 += E) {
+    float acc[TOK][E][PARTS];
+#pragma unroll
+    for (int n = 0; n < TOK; ++n)
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+#pragma unroll
+        for (int q = 0; q < PARTS; ++q) acc[n][e][q] = 0.f;
+    Four r[2][TOK];
+    float4 w[2][E];
+    const auto ask = [&](auto set, int step) {              // (behind the row's end its last values: not used)
+      constexpr int B = decltype(set)::value;
+      const int i = min((step * WAVE + lane) * 4, width - 4);
+#pragma unroll
+      for (int n = 0; n < TOK; ++n) r[B][n] = *reinterpret_cast<const Four*>(row[n] + i);
+#pragma unroll
+      for (int e = 0; e < E; ++e) w[B][e] = *reinterpret_cast<const float4*>(router + (int64_t)min(e0 + e, rows_r - 1) * width + i);
+    };
+    const auto use = [&](auto set, int step, auto part) {
+      constexpr int B = decltype(set)::value, Q = decltype(part)::value % PARTS;
+      if ((step * WAVE + lane) * 4 >= width) return;
+#pragma unroll
+      for (int n = 0; n < TOK; ++n) {
+        const float x0 = Elem<T>::load(r[B][n].v[0]), x1 = Elem<T>::load(r[B][n].v[1]), x2 = Elem<T>::load(r[B][n].v[2]),
+                    x3 = Elem<T>::load(r[B][n].v[3]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[n][e][Q] += dot4(x0, x1, x2, x3, w[B][e]);
+      }
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    const int steps = (width + 4 * WAVE - 1) / (4 * WAVE);
+    ask(even, 0);
+    for (int step = 0; step < steps; step += 4) {
+      ask(odd, step + 1);
+      use(even, step, even);
+      ask(even, step + 2);
+      use(odd, step + 1, odd);
+      ask(odd, step + 3);
+      use(even, step + 2, std::integral_constant<int, 2>{});
+      ask(even, step + 4);
+      use(odd, step + 3, std::integral_constant<int, 3>{});
+    }
+#pragma unroll
+    for (int n = 0; n < TOK; ++n)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        float sum = wave_sum(acc[n][e][0]);
+#pragma unroll
+        for (int q = 1; q < PARTS; ++q) sum += wave_sum(acc[n][e][q]);
+        if (lane == 0 && e0 + e < rows_r) lds[wave][n].z[e0 + e] = sum;
+      }
+  }
+#pragma unroll
+  for (int n = 0; n < TOK; ++n)
+    if (t0 + n < rows)
+      moe_router::choose(lds[wave][n], bias, weights + (t0 + n) * rows_r, experts, rows_r, top, groups, keep, score, scale);
 }
 
 // y[t, c] = round(round(silu(gate)) * up) * weight of the column's expert, 0 where that weight is 0; columns from
@@ -459,17 +536,31 @@ extern "C" int holon_moe_route(const float* logits, const float* correction, flo
   return 0;
 }
 
-// Up to 256 rows a block a token leaves the chip with idle units, which more waves a token use; with more (4,096 rows of 4,096 over
-// 8 experts: 57 us a wave a token, 58 so) there is nothing left to gain.
-static bool router_few_serves(int64_t rows, int experts) { return rows <= 256 && experts <= WAVE; }
-static int router_few(const void* x, const float* router, const float* bias, float* weights, int64_t rows, int width,
-                      int experts, int rows_r, int top, int groups, int keep, int score, float scale, int dtype,
-                      hipStream_t s) {
+// Up to 64 experts: a block of 16 waves a token up to 256 rows, which a block of four a token would leave idle units; from there on rows that
+// share what they read of the router, by the wave, as many as leave a block for every unit.
+static bool router_waves_serve(int64_t rows, int width, int experts, const float* router) {
+  return experts <= WAVE && (rows <= 256 || (width % 4 == 0 && (uintptr_t)router % 16 == 0 && rows <= 0x7fffffff));
+}
+static int router_waves(const void* x, const float* router, const float* bias, float* weights, int64_t rows, int width,
+                        int experts, int rows_r, int top, int groups, int keep, int score, float scale, int dtype,
+                        hipStream_t s) {
 #define ROUTER(T, PARTS)                                                                                                   \
   moe_router_few_kernel<T, PARTS><<<(unsigned)rows, 1024, 0, s>>>((const T*)x, router, bias, weights, width, experts, rows_r, \
                                                                   top, groups, keep, score, scale)
-  if (score < 0) { if (dtype == HOLON_F32) ROUTER(float, 1); else ROUTER(bf16_t, 1); }
-  else { if (dtype == HOLON_F32) ROUTER(float, 4); else ROUTER(bf16_t, 4); }
+#define ROUTER_ROWS(T, PARTS, TOK, E)                                                                                      \
+  moe_router_rows_kernel<T, PARTS, TOK, E><<<(unsigned)((rows + 4 * TOK - 1) / (4 * TOK)), 256, 0, s>>>(                     \
+      (const T*)x, router, bias, weights, rows, width, experts, rows_r, top, groups, keep, score, scale)
+#define ROUTER_FOR(T)                                                                                                      \
+  do {                                                                                                                     \
+    if (rows <= 256) { if (score < 0) ROUTER(T, 1); else ROUTER(T, 4); }                                                   \
+    else if (rows < 1024) { if (score < 0) ROUTER_ROWS(T, 1, 1, 8); else ROUTER_ROWS(T, 4, 1, 8); }                          \
+    else if (rows < 2048) { if (score < 0) ROUTER_ROWS(T, 1, 2, 8); else ROUTER_ROWS(T, 4, 2, 8); }                          \
+    else { if (score < 0) ROUTER_ROWS(T, 1, 4, 8); else ROUTER_ROWS(T, 4, 4, 4); }                                           \
+  } while (0)
+  if (dtype == HOLON_F32) ROUTER_FOR(float);
+  else ROUTER_FOR(bf16_t);
+#undef ROUTER_FOR
+#undef ROUTER_ROWS
 #undef ROUTER
   HOLON_LAUNCH_OK();
   return 0;
@@ -486,8 +577,8 @@ extern "C" int holon_moe_router(const void* x, const float* router, const float*
               "moe_router: %d experts in %d groups of which %d stay open", experts, groups, keep);
   if (rows == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  if (router_few_serves(rows, experts))
-    return router_few(x, router, correction, weights, rows, width, experts, experts, top, groups, keep, -1, scale, dtype, s);
+  if (router_waves_serve(rows, width, experts, router))
+    return router_waves(x, router, correction, weights, rows, width, experts, experts, top, groups, keep, -1, scale, dtype, s);
   const size_t lds = (size_t)width * sizeof(float);
   if (dtype == HOLON_F32)
     moe_router_kernel<float><<<(unsigned)rows, 256, lds, s>>>((const float*)x, router, correction, weights, width,
@@ -538,8 +629,8 @@ extern "C" int holon_moe_router_top(const void* x, const float* router, const fl
               "moe_router_top: top %d of %d experts in %d groups of which %d stay open", top, experts, groups, keep);
   if (rows == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  if (router_few_serves(rows, experts))
-    return router_few(x, router, bias, weights, rows, width, experts, router_rows, top, groups, keep, score, 1.f, dtype, s);
+  if (router_waves_serve(rows, width, experts, router))
+    return router_waves(x, router, bias, weights, rows, width, experts, router_rows, top, groups, keep, score, 1.f, dtype, s);
   if (dtype == HOLON_F32)
     moe_router_top_kernel<float><<<(unsigned)rows, 256, 0, s>>>((const float*)x, router, bias, weights, width, experts,
                                                                router_rows, top, groups, keep, score);

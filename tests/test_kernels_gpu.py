@@ -2092,3 +2092,20 @@ def test_rows_in_pieces_are_the_rows_value_by_value(hip, dtype):
                                               copies=copies)
             made.append((q, full[..., rank:].clone(), pages))
         assert all(torch.equal(a, b) for a, b in zip(*made)), (heads, dim, rot, rank, rd, copies)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_routers_of_many_rows_are_those_of_few(hip, dtype):
+    """Tokens that share what a wave reads of the router (one, two or four of them, by the rows) have bit for bit the weights of a token by
+    itself: rows on both sides of the lines, experts that do not come in eights, widths that do not fill a wave's step."""
+    for rows, width, experts, top, groups, keep in ((257, 2048, 8, 2, 1, 1), (1023, 260, 9, 3, 1, 1), (1024, 4, 1, 1, 1, 1), (2047, 1028, 17, 4, 1, 1),
+                                                    (2048, 2044, 64, 6, 8, 3), (2061, 512, 12, 2, 4, 2)):
+        x = _randn(rows, width, dtype=dtype, seed=220)
+        router = _randn(experts + 1, width, dtype=torch.float32, seed=221, scale=width ** -0.5)
+        bias = _randn(experts, dtype=torch.float32, seed=222, scale=0.2)
+        calls = [(hip.moe_router, (router[:experts].contiguous(), bias, top, groups, keep, 1.5), {})]
+        calls += [(hip.moe_router_top, (r, bias, experts, top, groups, keep), dict(score=how))
+                  for r, how in ((router, "softmax"), (router[:experts].contiguous(), "sigmoid"), (router, "sigmoid_squared"))]
+        for op, args, how in calls:
+            want = torch.cat([op(x[at: at + 256].contiguous(), *args, **how) for at in range(0, rows, 256)])
+            assert torch.equal(op(x, *args, **how), want), (rows, width, experts, how)

@@ -459,6 +459,10 @@ int holon_moe_up_few_bf16(const void* x, const void* w_tiled, void* act, int row
                           int gated, const float* weights, int wstride, int shared_col, void* stream);
 int holon_moe_down_few_bf16(const void* act, const void* w_tiled, void* y, int rows, int hidden, int experts, int ff,
                             int shared, const float* weights, int wstride, void* stream);
+// The same with py [rows, N] = px [rows, K] pw^T over a tiled weight in the same launch (form as in holon_gemm_skinny_bf16: 0, 2 or 4).
+int holon_moe_down_beside_bf16(const void* act, const void* w_tiled, void* y, int rows, int hidden, int experts, int ff,
+                               int shared, const float* weights, int wstride, const void* px, const void* pw, void* py, int N, int K,
+                               int form, void* stream);
 // The experts for steps of many bfloat16 rows, every expert over the rows that chose it alone: y [rows, hidden] from x, the
 // first projections `up` and the second ones `down` as they come (untiled), with the activations and roundings of the few-row
 // form. At most `top` weights a row are not 0. Scratch as the definition says.

@@ -12,7 +12,7 @@ from ..registry import register_part
 from .base import FLOAT32, Build, Part, Stream
 from .linear import Linear
 from .norms import Normed
-from .products import Product, Routing, by_itself, together
+from .products import ExpertsDown, Product, Routing, by_itself, together
 
 
 @register_part("ffn", "swiglu")
@@ -367,7 +367,7 @@ def moe_few_pays(rows: int, hidden: int, experts: int, ff: int, gated: bool, top
     return 1 + 0.01 * rows * experts + 0.25 * (experts - left) < column * ff * left
 
 
-def _moe_few_hip(launch, x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight=False):
+def _moe_up_few_hip(launch, x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight=False):
     t, hidden = x.shape
     cols = experts * ff + shared
     if up_tiled is None or down_tiled is None or x.dtype != torch.bfloat16 or not moe_few_serves(t, hidden, experts, ff, shared):
@@ -379,18 +379,46 @@ def _moe_few_hip(launch, x, weights, up_tiled, down_tiled, experts, ff, shared, 
           f"moe_few: rows {tuple(x.shape)}, weights {tuple(weights.shape)}, projections {tuple(up_tiled.shape)} and "
           f"{tuple(down_tiled.shape)} for {experts} experts of {ff} and {shared} shared columns")
     act = torch.empty((t, cols), dtype=x.dtype, device=x.device)
-    y = torch.empty((t, hidden), dtype=x.dtype, device=x.device)
-    up, down = launch
-    up(x.data_ptr(), up_tiled.data_ptr(), act.data_ptr(), t, hidden, experts, ff, shared, int(bool(gated)), weights.data_ptr(),
-       weights.shape[1], experts if shared_weight else -1)
-    down(act.data_ptr(), down_tiled.data_ptr(), y.data_ptr(), t, hidden, experts, ff, shared, weights.data_ptr(),
-         weights.shape[1])
+    launch(x.data_ptr(), up_tiled.data_ptr(), act.data_ptr(), t, hidden, experts, ff, shared, int(bool(gated)), weights.data_ptr(),
+           weights.shape[1], experts if shared_weight else -1)
+    return act
+
+
+def _moe_down_few_hip(launch, act, weights, down_tiled, experts, ff, shared):
+    t, hidden = act.shape[0], down_tiled.shape[0]
+    cols = experts * ff + shared
+    _need(act.is_cuda and act.is_contiguous() and act.dtype == down_tiled.dtype == torch.bfloat16 and weights.is_contiguous()
+          and weights.dtype == torch.float32 and weights.dim() == 2 and weights.shape[0] == t and weights.shape[1] >= experts
+          and down_tiled.is_contiguous() and moe_few_serves(t, hidden, experts, ff, shared)
+          and tuple(act.shape) == (t, cols) and tuple(down_tiled.shape) == (hidden, cols),
+          f"moe_down_few: activations {tuple(act.shape)}, weights {tuple(weights.shape)}, projection {tuple(down_tiled.shape)} for {experts} "
+          f"experts of {ff} and {shared} shared columns")
+    y = torch.empty((t, hidden), dtype=act.dtype, device=act.device)
+    launch(act.data_ptr(), down_tiled.data_ptr(), y.data_ptr(), t, hidden, experts, ff, shared, weights.data_ptr(),
+           weights.shape[1])
     return y
 
 
-register_kernel(KernelOp("moe_few", moe_few_plain, ("holon_moe_up_few_bf16", "holon_moe_down_few_bf16"),
-                         ([_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I], [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I]),
+def _moe_few_hip(launch, x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight=False):
+    act = _moe_up_few_hip(launch[0], x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight)
+    return None if act is None else _moe_down_few_hip(launch[1], act, weights, down_tiled, experts, ff, shared)
+
+
+def moe_up_few_plain(x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight=False):
+    """The first product of `moe_few` and its activation, or None."""
+    return None
+
+
+def moe_down_few_plain(act, weights, down_tiled, experts, ff, shared):
+    """The second product of `moe_few`, over what `moe_up_few` left (the plain form of which leaves nothing)."""
+    raise NotImplementedError("moe_down_few: there is no plain form of a tiled projection")
+
+
+_MOE_UP_FEW, _MOE_DOWN_FEW = [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I], [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I]
+register_kernel(KernelOp("moe_few", moe_few_plain, ("holon_moe_up_few_bf16", "holon_moe_down_few_bf16"), (_MOE_UP_FEW, _MOE_DOWN_FEW),
                          _moe_few_hip))
+register_kernel(KernelOp("moe_up_few", moe_up_few_plain, "holon_moe_up_few_bf16", _MOE_UP_FEW, _moe_up_few_hip))
+register_kernel(KernelOp("moe_down_few", moe_down_few_plain, "holon_moe_down_few_bf16", _MOE_DOWN_FEW, _moe_down_few_hip))
 
 
 def moe_rows_plain(x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
@@ -680,10 +708,11 @@ class MoE(Part):
             if y is not None:
                 return y
         if moe_few_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.act == "silu", self.top):
-            y = k.moe_few(x, weights, up.tiled, down.tiled, self.experts, self.inter, self.shared, self.act == "silu",
-                          shared_weight=self.shared_gated)
-            if y is not None:
-                return y
+            act = k.moe_up_few(x, weights, up.tiled, down.tiled, self.experts, self.inter, self.shared, self.act == "silu",
+                               shared_weight=self.shared_gated)
+            if act is not None:
+                rest = ExpertsDown(k, act, weights, down.tiled, self.experts, self.inter, self.shared)
+                return (yield [rest])[0] if together(x) else rest.alone()
         if moe_rows_pays(x.shape[0], x.shape[1], self.experts, self.inter, self.shared, self.act == "silu", self.top) \
                 and self._own_rows(x.shape[0]):
             y = k.moe_rows(x, weights, up.weight, down.weight, self.experts, self.top, self.inter, self.shared, self.act == "silu",

@@ -79,6 +79,30 @@ class Routing:
                                           and (self.scale is not None or self.top <= self.keep * (e // self.groups)))))
 
 
+@dataclasses.dataclass(slots=True)
+class ExpertsDown:
+    """The second product of a mixture's chosen experts (`moe_down_few`) over x, their activations [T, experts ff + shared]."""
+
+    kernels: Any
+    x: torch.Tensor
+    weights: torch.Tensor
+    tiled: torch.Tensor
+    experts: int
+    ff: int
+    shared: int
+
+    def alone(self) -> torch.Tensor:
+        return self.kernels.moe_down_few(self.x, self.weights, self.tiled, self.experts, self.ff, self.shared)
+
+    def served(self) -> bool:
+        """Whether a product's launch takes it along: what the operation by itself accepts."""
+        x, w, t, cols = self.x, self.weights, self.tiled, self.experts * self.ff + self.shared
+        return (x.is_cuda and x.dtype == t.dtype == torch.bfloat16 and x.is_contiguous() and t.is_contiguous() and w.is_contiguous()
+                and w.dtype == torch.float32 and w.dim() == 2 and w.shape[0] == x.shape[0] and 1 <= x.shape[0] <= FEW_ROWS
+                and w.shape[1] >= self.experts and tuple(x.shape[1:]) == (cols,) and tuple(t.shape[1:]) == (cols,) and t.shape[0] % 32 == 0
+                and self.experts <= 1024 and self.ff % 32 == 0 and self.shared % 32 == 0)
+
+
 def together(x, linear: Linear | None = None) -> bool:
     """Whether a product over these rows (of `linear`, if it is one's) may share a launch: few of them, in the type that it serves, over
     a tiled copy. Else whoever asks for it gains nothing from the list, and runs it."""
@@ -137,7 +161,7 @@ def by_itself(kernels, part):
         return end.value
 
 
-def _results(kernels, products: list[Product | Routing]) -> list[torch.Tensor]:
+def _results(kernels, products: list[Product | Routing | ExpertsDown]) -> list[torch.Tensor]:
     if len(products) < 2:
         return [p.alone() for p in products]
     if products[0].x.shape[0] > FEW_ROWS:
@@ -148,8 +172,9 @@ def _results(kernels, products: list[Product | Routing]) -> list[torch.Tensor]:
     return [p.alone() for p in products]
 
 
-def linear_group_plain(products: list[Product | Routing]) -> list[torch.Tensor]:
-    """The results of products (and a mixture's routing) that do not read one another's, in order; each with the roundings it has alone."""
+def linear_group_plain(products: list[Product | Routing | ExpertsDown]) -> list[torch.Tensor]:
+    """The results of products (and of a mixture's routing or its experts' second product) that do not read one another's, in order; each
+    with the roundings it has alone."""
     return [p.alone() for p in products]
 
 
@@ -179,20 +204,25 @@ def _served(p: Product) -> bool:
 SCORES = {"softmax": 0, "sigmoid": 1, "sigmoid_squared": 2}
 
 
-def _linear_group_hip(launch, products: list[Product | Routing]) -> list[torch.Tensor]:
+def _linear_group_hip(launch, products: list[Product | Routing | ExpertsDown]) -> list[torch.Tensor]:
+    launch, launch_beside = launch
     out: list = [None] * len(products)
     by_rows: dict[int, list[int]] = {}
     routes: dict[int, list[int]] = {}
+    downs: dict[int, list[int]] = {}
     for i, p in enumerate(products):
-        if isinstance(p, Routing):
+        if isinstance(p, (Routing, ExpertsDown)):
             if p.served():
-                routes.setdefault(p.x.shape[0], []).append(i)
+                (routes if isinstance(p, Routing) else downs).setdefault(p.x.shape[0], []).append(i)
         elif _served(p):
             by_rows.setdefault(p.x.shape[0], []).append(i)
     for rows, which in by_rows.items():
         for group in (which[at: at + MOST] for at in range(0, len(which), MOST)):
             route = routes[rows].pop(0) if routes.get(rows) else None
             if len(group) == 1 and route is None:
+                if downs.get(rows):                       # a mixture's experts beside it (several products fill the chip by themselves)
+                    at = downs[rows].pop(0)
+                    out[group[0]], out[at] = _beside(launch_beside, products[group[0]], products[at])
                 continue
             items = []
             for i in group:
@@ -212,8 +242,21 @@ def _linear_group_hip(launch, products: list[Product | Routing]) -> list[torch.T
     return [y if y is not None else p.alone() for y, p in zip(out, products)]
 
 
-register_kernel(KernelOp("linear_group", linear_group_plain, "holon_gemm_skinny_group_bf16",
-                         [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_float], _linear_group_hip))
+def _beside(launch, p: Product, d: ExpertsDown) -> tuple[torch.Tensor, torch.Tensor]:
+    """A product and a mixture's second one, in one launch."""
+    form = 4 if p.relu2 else 2 if p.dtype == torch.float32 else 0
+    rows, (n, k), hidden = p.x.shape[0], p.linear.weight.shape, d.tiled.shape[0]
+    y = torch.empty((rows, n), dtype=torch.float32 if form == 2 else torch.bfloat16, device=p.x.device)
+    out = torch.empty((rows, hidden), dtype=torch.bfloat16, device=p.x.device)
+    launch(d.x.data_ptr(), d.tiled.data_ptr(), out.data_ptr(), rows, hidden, d.experts, d.ff, d.shared, d.weights.data_ptr(),
+           d.weights.shape[1], p.x.data_ptr(), p.linear.tiled.data_ptr(), y.data_ptr(), n, k, form)
+    return y, out
+
+
+_P, _I = ctypes.c_void_p, ctypes.c_int
+register_kernel(KernelOp("linear_group", linear_group_plain, ("holon_gemm_skinny_group_bf16", "holon_moe_down_beside_bf16"),
+                         ([_P, _I, _I, _P, ctypes.c_float], [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _I, _I, _I]),
+                         _linear_group_hip))
 
 
 def block_group_pays(count: int, m: int, n: int, k: int) -> bool:

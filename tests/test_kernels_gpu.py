@@ -2109,3 +2109,35 @@ def test_routers_of_many_rows_are_those_of_few(hip, dtype):
         for op, args, how in calls:
             want = torch.cat([op(x[at: at + 256].contiguous(), *args, **how) for at in range(0, rows, 256)])
             assert torch.equal(op(x, *args, **how), want), (rows, width, experts, how)
+
+
+@pytest.mark.parametrize("rows", [1, 6, 16])
+@pytest.mark.parametrize("hidden,experts,ff,shared", [(256, 8, 32, 0), (2048, 8, 256, 512), (512, 70, 544, 32), (288, 5, 96, 0)])
+def test_experts_beside_a_product_are_both(hip, rows, hidden, experts, ff, shared):
+    """A mixture's second product and another one in one launch, bit for bit what either is by itself: tiles of 16, 8, 4, 2 and 1 waves
+    that do and do not fill a block, every output form; a product that joins no launch, and none at all."""
+    from holon_amd.parts.products import ExpertsDown, Product
+    bf, cols, gen = torch.bfloat16, experts * ff + shared, torch.Generator(device="cuda").manual_seed(rows)
+    down_t = hip.tile_weight(_randn(hidden, cols, dtype=bf, seed=230, scale=ff ** -0.5))
+    weights = (torch.rand(rows, experts, generator=gen, device="cuda") * (torch.rand(rows, experts, generator=gen, device="cuda") < 0.3)).contiguous()
+    act = _randn(rows, cols, dtype=bf, seed=231)
+    act[:, : experts * ff] *= (weights != 0).repeat_interleave(ff, 1)
+    down = ExpertsDown(hip, act, weights, down_t, experts, ff, shared)
+    whole = hip.linear(act, _randn(hidden, cols, dtype=bf, seed=230, scale=ff ** -0.5), tiled=down_t)
+    assert torch.equal(down.alone(), whole) and torch.equal(hip.linear_group([down])[0], whole)
+
+    class Weights:                                # what a projection holds
+        folded, kernels = None, hip
+
+        def __init__(self, n, kk):
+            self.weight = (0.05 * torch.randn(n, kk, generator=gen, device="cuda")).bfloat16()
+            self.tiled = hip.tile_weight(self.weight)
+
+        def __call__(self, x, dtype=None):
+            return hip.linear(x, self.weight, dtype, self.tiled)
+    for i, (n, kk) in enumerate(((2048, 2048), (16, 512), (5136, 512), (80, 1184), (80, 288), (528, 352), (48, 192))):
+        p = Product(Weights(n, kk), torch.randn(rows, kk, generator=gen, device="cuda").bfloat16(), **({}, {"dtype": torch.float32}, {"relu2": True})[i % 3])
+        for products in ([p, down], [down, p]):
+            got = dict(zip(map(id, products), hip.linear_group(products)))
+            want = p.alone()
+            assert got[id(p)].dtype == want.dtype and torch.equal(got[id(p)], want) and torch.equal(got[id(down)], whole), (n, kk)

@@ -170,12 +170,12 @@ __device__ __forceinline__ void widen4(const ushort4& h, float (&v)[4]) {
 // The same pass as stream_rms_kernel with four neighbouring values a thread and step (dim a multiple of 4, at most
 // 1024 REGS values a row, which stay in registers). FILTER: the step's rows are single tokens, and each result goes
 // through its causal filter of TAPS taps before it is stored (see `filter4`).
-// AHEAD: the terms, the weights and the results are of one type (DT), and everything that the row needs is asked for before any of it is
-// read: a step of few rows is a block or a few, and what it takes is one memory latency after the other, where a branch on a type
-// stands around each load (a weight of another type than the terms, as a norm's float32 weight beside bfloat16, takes the general
-// form). One row of 2,048 (two terms, one weight) 3.1 us -> 2.5, with the added vector, two weights and filters 4.6 -> 3.7; of 4,096 4.4 ->
+// AHEAD: the terms and the results are of one type (DT), the weights of another (DW) or the same, and everything that the row needs is asked
+// for before any of it is read: a step of few rows is a block or a few, and what it takes is one memory latency after the other, where a
+// branch on a type stands around each load. Four rows of 2,048 of bfloat16 terms under a float32 weight
+// 3.2 us -> 2.4. One row of 2,048 (two terms, one weight) 3.1 us -> 2.5, with the added vector, two weights and filters 4.6 -> 3.7; of 4,096 4.4 ->
 // 3.1 and 7.2 -> 5.4; 2,048 rows of 2,048 9.2 -> 8.7. Rows beyond 4,096 would hold more than the registers are worth.
-template <int REGS, int TAPS, int DT = HOLON_BF16, bool AHEAD = false>     // DT: read when TAPS > 0 or AHEAD
+template <int REGS, int TAPS, int DT = HOLON_BF16, bool AHEAD = false, int DW = DT>     // DT: read when TAPS > 0 or AHEAD
 __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__ x32, const void* __restrict__ d1, int dt1,
                                                              const void* __restrict__ d2, int dt2,
                                                              const float* __restrict__ row, const void* __restrict__ w1,
@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__
   float held[REGS][4];
   float sq = 0.f;
   constexpr bool FILTER = TAPS > 0;
-  Four<DT> g1[AHEAD ? REGS : 1], g2[AHEAD ? REGS : 1];
+  Four<DW> g1[AHEAD ? REGS : 1], g2[AHEAD ? REGS : 1];
   Filter4<FILTER ? TAPS : 1, DT> f1[FILTER ? REGS : 1], f2[FILTER ? REGS : 1];
   auto ask_filters = [&]() {
     const int slot = f.slots[blockIdx.x];
@@ -223,11 +223,11 @@ __global__ void __launch_bounds__(256) stream_rms_vec_kernel(float* __restrict__
     }
     if (w1) {
 #pragma unroll
-      for (int e = 0; e < REGS; ++e) g1[e] = raw4<DT>(w1, at[e]);
+      for (int e = 0; e < REGS; ++e) g1[e] = raw4<DW>(w1, at[e]);
     }
     if (w2) {
 #pragma unroll
-      for (int e = 0; e < REGS; ++e) g2[e] = raw4<DT>(w2, at[e]);
+      for (int e = 0; e < REGS; ++e) g2[e] = raw4<DW>(w2, at[e]);
     }
     if constexpr (FILTER) ask_filters();
     __builtin_amdgcn_sched_barrier(0);
@@ -467,11 +467,13 @@ extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void*
   if (dim % 4 == 0 && dim <= 8192) {        // four values a thread and step (every operand is a tensor's start: 16 bytes)
     const Filters none{};
     const int one = one_type(d1, dt1, d2, dt2, w1, dtw, dt_out);
+    const bool wide_weights = w1 && dtw == HOLON_F32 && one_type(d1, dt1, d2, dt2, w1, dt_out, dt_out) == HOLON_BF16;
 #define SRMSV(...) stream_rms_vec_kernel<__VA_ARGS__><<<(unsigned)rows, 256, 0, s>>>(x32, d1, dt1, d2, dt2, row, w1, w2, dtw, y1, y2, dim, eps, dt_out, none)
 #define SRMSV_BY_TYPE(R)                                 \
   do {                                                   \
     if (one == HOLON_BF16) SRMSV(R, 0, HOLON_BF16, true); \
     else if (one == HOLON_F32) SRMSV(R, 0, HOLON_F32, true); \
+    else if (wide_weights) SRMSV(R, 0, HOLON_BF16, true, HOLON_F32); \
     else SRMSV(R, 0);                                    \
   } while (0)
     if (dim <= 1024) SRMSV_BY_TYPE(1);

@@ -1840,7 +1840,9 @@ __global__ void __launch_bounds__(D == 256 ? 256 : 512) attn_decode_kernel(AttnA
 // out[row, head, :] = sum_i 2^(m_i - M) o_i / sum_i 2^(m_i - M) l_i over the splits (at most 64). One block of four
 // waves per (row, head): thread (group, d4) adds the partials of splits group, group + NG, ... for four dims, all of
 // its loads under way at once; the groups' sums are then added in group order. The order of every sum depends on
-// the number of splits and the head size alone.
+// the number of splits and the head size alone. Bound by latencies one behind the other: every wave works the splits'
+// weights out for itself (by one wave for all, the block met once more), which over traces of one and four rows is
+// 0.2 to 0.3 us a merge; loads left out where there are fewer splits cost a branch each (1 us at 32 splits).
 template <int D>
 __global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict__ part_o,
                                                          const float* __restrict__ part_ml, bf16_t* __restrict__ out,
@@ -1852,7 +1854,6 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict
   constexpr int LANES = D / 4;            // threads across one partial
   constexpr int NG = 256 / LANES;         // groups of splits
   constexpr int PER = (64 + NG - 1) / NG; // splits a thread may own
-  __shared__ float weight[64];
   __shared__ float inv_denom;
   __shared__ f32x4_t sums[NG][LANES];
   const int ri = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
@@ -1864,29 +1865,27 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(const float* __restrict
 #pragma unroll
   for (int i = 0; i < PER; ++i)            // asked for before the weights are known: an empty split's values are dropped
     v[i] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)min(group + i * NG, splits - 1) * D + d0);
+  const int lane = tid % WAVE;
+  float m_s = -INFINITY, l_s = 0.f;
+  if (lane < splits) {
+    const float2 x = *reinterpret_cast<const float2*>(ml + 2 * lane);
+    m_s = x.x;
+    l_s = x.y;
+  }
+  if (!(l_s > 0.f)) m_s = -INFINITY;
+  const float big = wave_max(m_s);
+  const float w_s = l_s > 0.f ? exp2f(m_s - big) : 0.f;
   if (tid < WAVE) {
-    float m_s = -INFINITY, l_s = 0.f;
-    if (tid < splits) {
-      const float2 x = *reinterpret_cast<const float2*>(ml + 2 * tid);
-      m_s = x.x;
-      l_s = x.y;
-    }
-    if (!(l_s > 0.f)) m_s = -INFINITY;
-    const float big = wave_max(m_s);
-    const float w_s = l_s > 0.f ? exp2f(m_s - big) : 0.f;
     float denom = 0.f;                     // in split order
     for (int s = 0; s < splits; ++s) denom += of_lane(w_s * l_s, s);
     if (sink != nullptr && big != -INFINITY) denom += exp2f(sink[h] * 1.4426950408889634f - big);
     if (hgate != nullptr) denom *= 1.0f + __expf(-bf16_to_float(hgate[(int64_t)token * hgate_stride + h]));
-    weight[tid] = w_s;
     if (tid == 0) inv_denom = denom > 0.f ? 1.0f / denom : 0.f;
   }
-  __syncthreads();
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int sp = group + i * NG;
-    const float w = sp < splits ? weight[sp] : 0.f;
+    const float w = __shfl(w_s, group + i * NG, WAVE);      // (of a split that is not there: 0)
     if (w > 0.f) acc += w * v[i];
   }
   sums[group][tid % LANES] = acc;

@@ -73,18 +73,17 @@ __global__ void __launch_bounds__(SHARES * WAVE) gemm_f32_half_kernel(const floa
   store4(y, sum, c, n0 + 4 * g, M, N);
 }
 
-template <int SIDE, bool VEC>
-__global__ void __launch_bounds__(SIDE * 256) gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                              float* __restrict__ y, int M, int N, int K) {
-  __shared__ __attribute__((aligned(16))) Stage<SIDE> stage;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64, r0 = threadIdx.x % 256 / 8;
-  const float *xr[2], *wr[2];
+template <int SIDE, int MT, int NT, How HOW>
+__global__ void __launch_bounds__(SIDE * 256, SIDE > 1 ? 4 : (MT == 2 && NT == 2 && HOW == DIRECT ? 5 : 1)) gemm_f32_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y, int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) Stage<SIDE, MT, NT> stage;
+  const int m0 = blockIdx.y * 32 * MT, n0 = blockIdx.x * 32 * NT, r0 = threadIdx.x % 256 / 8;
+  const float *xr[MT], *wr[NT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    xr[i] = x + (int64_t)min(m0 + r0 + 32 * i, M - 1) * K;
-    wr[i] = w + (int64_t)min(n0 + r0 + 32 * i, N - 1) * K;
-  }
-  tile_sums<SIDE, VEC>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) { store4(y, sum, m0 + row, n0 + column, M, N); });
+  for (int i = 0; i < MT; ++i) xr[i] = x + (int64_t)min(m0 + r0 + 32 * i, M - 1) * K;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) wr[i] = w + (int64_t)min(n0 + r0 + 32 * i, N - 1) * K;
+  tile_sums<SIDE, MT, NT, HOW>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) { store4(y, sum, m0 + row, n0 + column, M, N); });
 }
 
 // Long sums into many columns: one running sum over k = 0, 1, 2, ... (v_mfma_f32_32x32x2_f32 adds its two k one after the
@@ -161,36 +160,41 @@ __global__ void __launch_bounds__(256) gemm_f32_in_order_kernel(const float* __r
   }
 }
 
-// Which form a product takes: the one that is done first by a fit over K = 48 to 18,432, N = 64 to 16,384 and M = 17 to 2,048 on
-// MI355X (1,149 products, each in all forms, weights from memory): in us, a start and so much for every round of one block a CU, both
-// linear in K. Where the best form takes more than 15 us the choice is 0.1 % from it on average and 6 % at most. In us, best and others:
-// 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10; with a 64 x 64 tile a block and no split of K it took 118), quarters side by side
-// from 300 rows (42; one after the other 54, 2 x 2 tiles 50), one after the other at 2,048 (157; 163); 2048 x 9248 and 2048 x 18432 at
-// 704 rows quarters side by side (345 and 672; 2 x 4 tiles, which a fit up to K = 4,096 took there, 396 and 767); 16384 x 2048 1 x 1
-// tiles up to 16 rows (5.0 TB/s at one row), quarters side by side from 64 (46; 58), one after the other from 150 (125; 130); 9248 x 256
-// at 2,048 rows one after the other (103; side by side 180).
+// Which form a product takes: the one that is done first by a fit on MI355X (weights from memory), in us: a start, and so much for every
+// round of one block a CU, linear in K. Tiles straight from memory (1,149 products) add a part of K to that; of staged ones (170 products, K =
+// 64 to 18,432, N = 64 to 16,384, M = 17 to 2,048) a block that has its unit to itself takes longer than its share of a full one, `alone`
+// a k. The choice is 0.7 % from the best form on average and 12 % at most. In us, best and others: 2048 x 2048 takes 1 x 1
+// tiles up to 32 rows (10; with a 64 x 64 tile a block and no split of K it took 118), quarters side by side from 300 rows (38; one after
+// the other 46), blocks of 32 rows at 700 (65; of 64 rows 76, whose second round is mostly empty); 2048 x 9248 at 704 rows blocks of 32
+// (268; of 64 313); 16384 x 2048 1 x 1 tiles up to 16 rows (5.0 TB/s at one row), quarters side by side at 64 (42; one after the other
+// 53), blocks of 32 at 150 (108; 113), of 64 at 825 (480; of 32 571); 9248 x 256 at 2,048 rows one after the other (95; side by side 139).
 struct Form { int mt, nt; float start, start_k, round, round_k; };
-constexpr Form FORMS[6] = {{1, 1, 2.6f, 2e-4f, 0.43f, 3.25e-3f}, {1, 2, 2.5f, 2e-4f, 0.63f, 5.0e-3f},
-                           {2, 2, 2.5f, 7e-4f, 0.90f, 7.35e-3f}, {2, 4, 1.2f, 5e-4f, 3.0f, 1.31e-2f},
-                           {4, 4, 1.2f, 0.f, 3.2f, 1.86e-2f},    {4, 4, 2.1f, 8.0e-3f, 1.1f, 1.66e-2f}};
+enum { SIDE_BY_SIDE = 4, IN_TURN = 5, IN_TURN_32 = 6, KINDS = 7 };
+constexpr Form FORMS[KINDS] = {{1, 1, 2.6f, 2e-4f, 0.43f, 3.25e-3f},   {1, 2, 2.5f, 2e-4f, 0.63f, 5.0e-3f},    {2, 2, 2.5f, 7e-4f, 0.90f, 7.35e-3f},
+                               {2, 4, 1.2f, 5e-4f, 3.0f, 1.31e-2f},    {4, 4, 2.5f, 1.66e-2f, 2.86f, 1.7e-2f}, {4, 4, 3.3f, 2.06e-2f, 0.56f, 1.8e-2f},
+                               {2, 4, 2.95f, 1.42e-2f, 0.33f, 1.02e-2f}};
+// Operands that cannot be copied straight into LDS (K off a multiple of 32, or not on 16 bytes) pass registers, in tiles of 64 x 64.
+constexpr Form BY_REGISTERS[2] = {{4, 4, 1.2f, 0.f, 3.2f, 1.86e-2f}, {4, 4, 2.1f, 8.0e-3f, 1.1f, 1.66e-2f}};
 
-int pick_form(int M, int N, int K) {
+int pick_form(int M, int N, int K, bool direct) {
   int best = 0;
   float least = INFINITY;
-  for (int i = 0; i < 6; ++i) {
-    const Form& f = FORMS[i];
+  for (int i = 0; i < (direct ? KINDS : KINDS - 1); ++i) {
+    const bool staged = i >= SIDE_BY_SIDE;
+    const Form& f = staged && !direct ? BY_REGISTERS[i - SIDE_BY_SIDE] : FORMS[i];
     if (i > 0 && M <= 16) break;
     if (f.mt < 4 && (M + 16 * f.mt - 1) / (16 * f.mt) > 65535) continue;
     const int64_t blocks = (int64_t)((M + 16 * f.mt - 1) / (16 * f.mt)) * ((N + 16 * f.nt - 1) / (16 * f.nt));
-    const float cost = f.start + f.start_k * K + (float)((blocks + 255) / 256) * (f.round + f.round_k * K);
+    const float rounds = (float)((blocks + 255) / 256) * (f.round + f.round_k * K), lone = f.start_k * K;
+    const float cost = f.start + (staged && direct ? fmaxf(lone, rounds) : lone + rounds);
     if (cost < least) { least = cost; best = i; }
   }
   return best;
 }
 
-template <bool VEC>
+template <bool VEC, How HOW>
 void launch(const float* x, const float* w, float* y, int M, int N, int K, hipStream_t s) {
-  const int best = pick_form(M, N, K);
+  const int best = pick_form(M, N, K, HOW == DIRECT);
   const dim3 grid((N + 16 * FORMS[best].nt - 1) / (16 * FORMS[best].nt), (M + 16 * FORMS[best].mt - 1) / (16 * FORMS[best].mt));
   switch (best) {
     case 0:
@@ -200,15 +204,23 @@ void launch(const float* x, const float* w, float* y, int M, int N, int K, hipSt
     case 1: gemm_f32_rows_kernel<1, 2, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
     case 2: gemm_f32_rows_kernel<2, 2, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
     case 3: gemm_f32_rows_kernel<2, 4, 1, VEC><<<grid, SHARES * WAVE, 0, s>>>(x, w, y, M, N, K); break;
-    case 4: gemm_f32_kernel<4, VEC><<<grid, 1024, 0, s>>>(x, w, y, M, N, K); break;
-    default: gemm_f32_kernel<1, VEC><<<grid, 256, 0, s>>>(x, w, y, M, N, K); break;
+    case SIDE_BY_SIDE: gemm_f32_kernel<4, 2, 2, HOW><<<grid, 1024, 0, s>>>(x, w, y, M, N, K); break;
+    case IN_TURN_32:
+      if constexpr (HOW == DIRECT) gemm_f32_kernel<1, 1, 2, HOW><<<grid, 256, 0, s>>>(x, w, y, M, N, K);
+      break;
+    default: gemm_f32_kernel<1, 2, 2, HOW><<<grid, 256, 0, s>>>(x, w, y, M, N, K); break;
   }
 }
 }  // namespace
 
-// Which form serves M rows: 0 to 3 tiles of 1 x 1, 1 x 2, 2 x 2 and 2 x 4 a block, 4 quarters of K side by side, 5 one after the
-// other; -1 one running sum.
-extern "C" int holon_gemm_f32_form(int M, int N, int K) { return sums_in_order(N, K) ? -1 : pick_form(M, N, K); }
+// Which form serves M rows of operands on 16 bytes: 0 to 3 tiles of 1 x 1, 1 x 2, 2 x 2 and 2 x 4 a block; 4 and 5 staged tiles, 4 for outputs
+// of few (the quarters of K side by side, or blocks of 32 rows) and 5 for outputs of many (64 x 64, the quarters one after the other); -1 one
+// running sum.
+extern "C" int holon_gemm_f32_form(int M, int N, int K) {
+  if (sums_in_order(N, K)) return -1;
+  const int form = pick_form(M, N, K, K % CHUNK == 0);
+  return form == IN_TURN_32 ? SIDE_BY_SIDE : form;
+}
 
 extern "C" int holon_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, void* stream) {
   HOLON_CHECK(M >= 0 && N > 0 && K > 0, "gemm (float32): M=%d N=%d K=%d", M, N, K);
@@ -220,8 +232,9 @@ extern "C" int holon_gemm_f32(const void* x, const void* w, void* y, int M, int 
     hipStream_t s = (hipStream_t)stream;
     if (vec) gemm_f32_in_order_kernel<true><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, (float*)y, M, N, K);
     else gemm_f32_in_order_kernel<false><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, (float*)y, M, N, K);
-  } else if (vec) launch<true>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
-  else launch<false>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
+  } else if (vec && K % CHUNK == 0) launch<true, DIRECT>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
+  else if (vec) launch<true, BY_FOUR>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
+  else launch<false, BY_VALUE>((const float*)x, (const float*)w, (float*)y, M, N, K, (hipStream_t)stream);
   HOLON_LAUNCH_OK();
   return 0;
 }

@@ -127,10 +127,10 @@ __device__ __forceinline__ bool take(const MoeRows& p, int routed_cols, int shar
 
 // act of an expert's rows (routed: [rows * top, ff] in the order of the lists) and of the shared one ([rows, shared]): tiles of 64 rows
 // by 64 columns, GATED 32 gates and the same 32 ups.
-template <bool GATED>
-__global__ void __launch_bounds__(256) moe_up_rows_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+template <bool GATED, How HOW>
+__global__ void __launch_bounds__(256, HOW == DIRECT ? 5 : 1) moe_up_rows_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                               float* __restrict__ act, float* __restrict__ act_shared, MoeRows p) {
-  __shared__ __attribute__((aligned(16))) Stage<1> stage;
+  __shared__ __attribute__((aligned(16))) Stage<1, 2, 2> stage;
   constexpr int COLS = GATED ? 32 : 64;
   const auto tiles = [](int n) { return (n + COLS - 1) / COLS; };
   Taken t;
@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(256) moe_up_rows_f32_kernel(const float* __res
   }
   float* out = t.routed ? act + (int64_t)t.rows.first * p.ff : act_shared;
   if constexpr (!GATED) {
-    tile_sums<1, true>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) {
+    tile_sums<1, 2, 2, HOW>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) {
       const int r = t.rows.row0 + row;
       if (r >= t.rows.count || n0 + column >= width) return;
       const float weight = weight_of(p, token(r), t.rows.expert);
@@ -156,9 +156,9 @@ __global__ void __launch_bounds__(256) moe_up_rows_f32_kernel(const float* __res
       *reinterpret_cast<f32x4_t*>(out + (int64_t)r * width + n0 + column) = sum;
     });
   } else {
-    float* both = &stage[0][0][0][0];                      // [64 rows][64 columns and 4]: gates, then ups
+    float* both = &stage[0][0][0];                      // [64 rows][64 columns and 4]: gates, then ups
     static_assert(sizeof(stage) >= ROWS * 68 * sizeof(float), "a tile's gates and ups");
-    tile_sums<1, true>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) {      // (behind the last barrier of the sums)
+    tile_sums<1, 2, 2, HOW>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) {      // (behind the last barrier of the sums)
       *reinterpret_cast<f32x4_t*>(both + row * 68 + column) = sum;
     });
     __syncthreads();
@@ -175,9 +175,10 @@ __global__ void __launch_bounds__(256) moe_up_rows_f32_kernel(const float* __res
 }
 
 // parts [rows * top + rows, hidden]: an expert's share of the results of its rows, then the shared expert's; slots as in moe_rows.hip.
-__global__ void __launch_bounds__(256) moe_down_rows_f32_kernel(const float* __restrict__ act, const float* __restrict__ act_shared,
+template <How HOW>
+__global__ void __launch_bounds__(256, HOW == DIRECT ? 5 : 1) moe_down_rows_f32_kernel(const float* __restrict__ act, const float* __restrict__ act_shared,
                                                                 const float* __restrict__ w, float* __restrict__ parts, MoeRows p) {
-  __shared__ __attribute__((aligned(16))) Stage<1> stage;
+  __shared__ __attribute__((aligned(16))) Stage<1, 2, 2> stage;
   const int per = (p.hidden + 63) / 64;
   Taken t;
   if (!take(p, per, per, t)) return;
@@ -196,7 +197,7 @@ __global__ void __launch_bounds__(256) moe_down_rows_f32_kernel(const float* __r
     p.slots[(int64_t)(entry & ((1u << TOKEN_BITS) - 1)) * p.top + (entry >> TOKEN_BITS)] = t.rows.first + r;
   }
   float* out = parts + (int64_t)(t.routed ? t.rows.first : (int64_t)p.rows * p.top) * p.hidden;
-  tile_sums<1, true>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) {
+  tile_sums<1, 2, 2, HOW>(stage, xr, wr, K, [&](f32x4_t sum, int row, int column) {
     const int r = t.rows.row0 + row;
     if (r < t.rows.count && n0 + column < p.hidden) *reinterpret_cast<f32x4_t*>(out + (int64_t)r * p.hidden + n0 + column) = sum;
   });
@@ -242,9 +243,13 @@ extern "C" int holon_moe_f32(const void* x, const void* up, const void* down, vo
   const auto blocks = [&](int64_t n) { return (unsigned)(tiles(n, XCDS) * XCDS); };      // every XCD as many
   const unsigned up_blocks = blocks(routed * tiles(ff, width) + shared_rows * tiles(shared, width));
   make_lists(p, s);
-  if (gated) moe_up_rows_f32_kernel<true><<<up_blocks, 256, 0, s>>>(xf, wu, a, act_shared, p);
-  else moe_up_rows_f32_kernel<false><<<up_blocks, 256, 0, s>>>(xf, wu, a, act_shared, p);
-  moe_down_rows_f32_kernel<<<blocks((routed + shared_rows) * tiles(hidden, 64)), 256, 0, s>>>(a, act_shared, wd, parts, p);
+#define UP(GATED, HOW) moe_up_rows_f32_kernel<GATED, HOW><<<up_blocks, 256, 0, s>>>(xf, wu, a, act_shared, p)
+  if (hidden % CHUNK == 0) { if (gated) UP(true, DIRECT); else UP(false, DIRECT); }
+  else { if (gated) UP(true, BY_FOUR); else UP(false, BY_FOUR); }
+#undef UP
+  const unsigned down_blocks = blocks((routed + shared_rows) * tiles(hidden, 64));
+  if (ff % CHUNK == 0 && shared % CHUNK == 0) moe_down_rows_f32_kernel<DIRECT><<<down_blocks, 256, 0, s>>>(a, act_shared, wd, parts, p);
+  else moe_down_rows_f32_kernel<BY_FOUR><<<down_blocks, 256, 0, s>>>(a, act_shared, wd, parts, p);
   add_parts(p, parts, (float*)y, s);
   HOLON_LAUNCH_OK();
   return 0;

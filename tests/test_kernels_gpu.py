@@ -1577,6 +1577,21 @@ def test_float32_product_of_long_sums_takes_the_form_that_is_done_first(hip):
             assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), (m, n, k, row)
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 130, 96), (97, 4160, 1056), (161, 1000, 544), (300, 2048, 4128), (700, 2048, 2048), (705, 2049, 2016),
+                                   (825, 3072, 1024), (825, 16384, 64), (1030, 2100, 32), (33, 9248, 160)])
+def test_float32_products_copied_straight_into_lds(hip, m, n, k):
+    """Blocks of 64 and of 32 rows, edges of both, K that ends in each quarter: bit for bit what operands give that pass registers (those
+    off a border of 16 bytes) and what a row is alone; against the float64 product."""
+    x, w = _randn(m, k, dtype=torch.float32, seed=142), _randn(n, k, dtype=torch.float32, seed=143)
+    got, want = hip.linear(x, w), x.double() @ w.double().T
+    bound = (-(-k // 512) * 32 + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((got.double() - want).abs() <= bound).all()
+    off = torch.empty(m * k + 1, dtype=torch.float32, device="cuda")[1:].view(m, k).copy_(x)
+    assert off.data_ptr() % 16 and torch.equal(hip.linear(off, w), got)
+    for row in (0, 31, m - 1):
+        assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), row
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("heads,kv,d", [(6, 2, 48), (8, 8, 24), (4, 1, 272), (4, 2, 80)])
 def test_general_attention_of_short_rows(hip, dtype, heads, kv, d):

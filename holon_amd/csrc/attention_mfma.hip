@@ -476,31 +476,34 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(AttnArgs a) {
   }
 }
 
-// Prompt portions, staged through LDS: a block of four waves owns 4*NT consecutive tiles (for four heads a group: 32
+// Prompt portions, staged through LDS: a block of WAVES waves owns WAVES*NT consecutive tiles (for four heads a group and four waves: 32
 // positions with NT = 2) and walks the keys in stages of 32; each stage's keys and transposed values are copied from
 // the pages into LDS once per block (double buffered: the next stage's loads are in flight while this one is
 // multiplied) and every wave takes its matrix-core operands from there, so a key is read from the cache once per
 // block, not once per wave. Keys are stored in LDS in the order the two score products want their rows (lane c reads
 // row c, then row 16 + c), which with a row pitch of D + 8 makes the 16-byte reads conflict-free; value rows have a
 // pitch of 40. To even out the causal mask, a block does two position ranges: the b-th from the start and the b-th
-// from the end.
-template <int D, int NT>
-__global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
+// from the end (unpaired: a block each).
+// Heads of 256 take eight waves a block (74 KB of LDS a block, two waves a SIMD): the bits of the kernel that reads them straight from the
+// cache, whose every wave waits for its own 32 KB a stage. What bounds it is those 32 KB a wave and stage out of LDS.
+template <int D, int NT, int WAVES = 4>
+__global__ void __launch_bounds__(WAVES * WAVE) attn_prefill_lds_kernel(AttnArgs a) {
   constexpr int KP = D + 8;    // pitch of a key row in LDS (elements)
   constexpr int VP = 40;       // pitch of a value row: 32 keys + 8
+  constexpr int EARLY = D == 256 ? 8 : 0;      // values asked of LDS in front of the scores, as many as registers hold (137 us and 140)
   __shared__ __attribute__((aligned(16))) bf16_t k_lds[2][32 * KP];
   __shared__ __attribute__((aligned(16))) bf16_t v_lds[2][D * VP];
   constexpr int PG = 4096;     // the row's first block-table entries, kept in LDS: page lookups then do not queue
   __shared__ int32_t pg_lds[PG];   // behind the vector loads in flight
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, tid = threadIdx.x;
   const int g = lane / 16, c = lane % 16;
-  const int b = a.row_ids[blockIdx.z];
+  const int b = a.row_ids[a.unpaired ? blockIdx.z / 2 : blockIdx.z];
   const int group = a.heads / a.kv_heads;
   const TileMap tm = tile_map(group);
   const int hk = blockIdx.y / tm.head_blocks, hb = blockIdx.y % tm.head_blocks;
   const int qs = a.qstart[b], nq = a.qstart[b + 1] - qs, n = a.lens[b];
   const int n_tiles = (nq + tm.pos_per_tile - 1) / tm.pos_per_tile;
-  constexpr int TPB = 4 * NT;                                  // tiles a block owns per range
+  constexpr int TPB = WAVES * NT;                               // tiles a block owns per range
   const int n_ranges = (n_tiles + TPB - 1) / TPB;
   if (n <= 0 || (int)blockIdx.x >= (n_ranges + 1) / 2) return;   // uniform over the block
   const int32_t* trow = a.table + (int64_t)a.slots[b] * a.table_stride;
@@ -513,15 +516,15 @@ __global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
 
   // every entry a stage can ask for: the last stage's second half may lie one page past the row's tokens (the table
   // holds a valid page id there, the null page or any other: the keys are masked), so the whole row is copied
-  for (int i = tid; i < min(PG, a.table_stride); i += 256) pg_lds[i] = trow[i];
-  // this thread's share of a stage's copy: D/64 chunks of keys and as many of values, 16 bytes each
+  for (int i = tid; i < min(PG, a.table_stride); i += WAVES * WAVE) pg_lds[i] = trow[i];
+  // this thread's share of a stage's copy: chunks of keys and as many of values, 16 bytes each
   constexpr int KCH = D / 8;                                   // chunks per key row
-  constexpr int ROUNDS = D / 64;                               // 32 keys x D and D x 32 values: 4 D chunks each, 256 threads
-  static_assert(D == 64 || D == 128, "the LDS kernel copies one or two chunks of each kind per thread");
+  constexpr int ROUNDS = D / 16 / WAVES;                       // 32 keys x D and D x 32 values: 4 D chunks each
+  static_assert(ROUNDS == 1 || ROUNDS == 2, "the LDS kernel copies one or two chunks of each kind per thread");
   int k_key[ROUNDS], k_col[ROUNDS], k_dst[ROUNDS], v_d[ROUNDS], v_kc[ROUNDS], v_dst[ROUNDS];
 #pragma unroll
   for (int i = 0; i < ROUNDS; ++i) {
-    const int q = tid + 256 * i;
+    const int q = tid + WAVES * WAVE * i;
     k_key[i] = q / KCH;
     k_col[i] = (q % KCH) * 8;
     const int j = k_key[i];
@@ -532,11 +535,12 @@ __global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
     v_dst[i] = v_d[i] * VP + v_kc[i] * 8;
   }
 
-  for (int pass = 0; pass < 2; ++pass) {
+  const int pass_lo = a.unpaired ? 1 - (int)(blockIdx.z % 2) : 0, pass_hi = a.unpaired ? pass_lo + 1 : 2;      // (the longer ranges first)
+  for (int pass = pass_lo; pass < pass_hi; ++pass) {
     const int range = pass == 0 ? (int)blockIdx.x : n_ranges - 1 - (int)blockIdx.x;
     if (pass == 1 && range <= (int)blockIdx.x) break;          // an odd count: the middle range was done in pass 0
     bf16x8_t qf[NT][D / 32];
-    int qpos[NT], tile_last[NT], tile_first[NT], seen_from[NT], whole_from[NT];
+    int qpos[NT], tile_last[NT], tile_first[NT], seen_from[NT], whole_from[NT], tile_from[NT];
     RowRef rr[NT];
     int key_hi = -1, key_lo = 0x7fffffff;                      // over the whole block (all waves walk the same stages)
     {
@@ -555,6 +559,7 @@ __global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
       tile_first[t] = n - nq + p0;
       seen_from[t] = first_seen(qpos[t], a.window);
       whole_from[t] = first_seen(tile_last[t], a.window);
+      tile_from[t] = max(0, first_seen(tile_first[t], a.window)) / 32 * 32;      // the stage of the first key that a row of the tile sees
       const bf16_t* qp = a.q + ((int64_t)rr[t].token * a.heads + rr[t].head) * D + 8 * g;
 #pragma unroll
       for (int ks = 0; ks < D / 32; ++ks) {
@@ -610,7 +615,7 @@ __global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
     auto stage = [&](int kb, int buf, Regs& next) {
       bool any = false;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) any = any || kb <= tile_last[t];
+      for (int t = 0; t < NT; ++t) any = any || (kb >= tile_from[t] && kb <= tile_last[t]);
       if (any) {
         bf16x8_t kf0[D / 32], kf1[D / 32];
 #pragma unroll
@@ -618,10 +623,16 @@ __global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
           kf0[ks] = *reinterpret_cast<const bf16x8_t*>(&k_lds[buf][c * KP + ks * 32 + 8 * g]);
           kf1[ks] = *reinterpret_cast<const bf16x8_t*>(&k_lds[buf][(16 + c) * KP + ks * 32 + 8 * g]);
         }
+        bf16x8_t vf[D / 16];
+        const auto read_value = [&](int ds) { vf[ds] = *reinterpret_cast<const bf16x8_t*>(&v_lds[buf][(ds * 16 + c) * VP + 8 * g]); };
+        if constexpr (EARLY > 0) {
+#pragma unroll
+          for (int ds = 0; ds < EARLY; ++ds) read_value(ds);
+        }
         bf16x8_t pb[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          if (kb > tile_last[t]) continue;
+          if (kb < tile_from[t] || kb > tile_last[t]) continue;
           f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int ks = 0; ks < D / 32; ++ks) {
@@ -635,12 +646,13 @@ __global__ void __launch_bounds__(256) attn_prefill_lds_kernel(AttnArgs a) {
         }
 #pragma unroll
         for (int ds = 0; ds < D / 16; ++ds) {
-          bf16x8_t vf = *reinterpret_cast<const bf16x8_t*>(&v_lds[buf][(ds * 16 + c) * VP + 8 * g]);
-          if (kb + 31 > key_hi) zero_after(vf, kb + 8 * g, key_hi);
+          if (ds >= EARLY) read_value(ds);
+          const int last = NT == 1 ? tile_last[0] : key_hi;          // (what lies behind the tile's tokens may be anything)
+          if (kb + 31 > last) zero_after(vf[ds], kb + 8 * g, last);
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
-            if (kb > tile_last[t]) continue;
-            o[t][ds] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pb[t], o[t][ds], 0, 0, 0);
+            if (kb < tile_from[t] || kb > tile_last[t]) continue;
+            o[t][ds] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[ds], pb[t], o[t][ds], 0, 0, 0);
           }
         }
       }
@@ -2071,6 +2083,17 @@ static int prefill_launch(const void* q, void* out, const void* pages, const int
       if (head_dim == 64) attn_prefill_lds_kernel<64, 1><<<lgrid, 256, 0, ls>>>(a);
       else attn_prefill_lds_kernel<128, 1><<<lgrid, 256, 0, ls>>>(a);
     }
+    HOLON_LAUNCH_OK();
+    return 0;
+  }
+  // Heads of 256 in the order of 32 keys a product that short rows have (`staged_256` off, or more than 32 heads a group): staged from 512
+  // keys on, the same bits. 16 heads over one, us, straight from the cache against staged: prompts of 300 tokens 27 / 29, 512 41 / 40, 1,024
+  // 78 / 68, 4,096 591 / 314, four of 700 to 1,500 224 / 137, eight of 100 15 / 17; 64 tokens behind 8,000 546 / 430, 20 behind 600 49 / 46.
+  if (head_dim == 256 && tiles >= 16 && max_len >= 512 && max_len <= 4096 * page_size) {
+    const int ranges = (tiles + 7) / 8;
+    a.unpaired = (int64_t)((ranges + 1) / 2) * kv_heads * tm.head_blocks * n_rows < UNPAIR_BELOW ? 1 : 0;
+    dim3 lgrid((ranges + 1) / 2, kv_heads * tm.head_blocks, a.unpaired ? 2 * n_rows : n_rows);
+    attn_prefill_lds_kernel<256, 1, 8><<<lgrid, 512, 0, (hipStream_t)stream>>>(a);
     HOLON_LAUNCH_OK();
     return 0;
   }

@@ -1618,6 +1618,39 @@ def test_general_attention_of_short_rows(hip, dtype, heads, kv, d):
         assert H.rel_rms(got, want) < tight and H.rel_rms(hip.paged_attention(q, pages, table, rows(1), page, d ** -0.5, window), want) < tight
 
 
+@pytest.mark.parametrize("heads,kv,window", [(16, 1, 0), (16, 1, 200), (20, 1, 0), (8, 2, 0), (6, 2, -160), (34, 1, 96), (3, 3, 33)])
+def test_heads_of_256_staged_are_the_bits_of_short_portions(hip, heads, kv, window):
+    """Two prompts in one step, the longer one beyond the length from which stages go through LDS, behind cached tokens or not: every row
+    bit for bit what portions give that are too short for it, under sinks and windows of either kind, whatever later tokens' values are."""
+    d, page, bf = 256, 16, torch.bfloat16
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                      # noqa: E731
+    hip = hip.configured()
+    hip.settled = True
+    short = 16 // min(heads // kv, 16) * 15                                                # (15 tiles of 16 rows)
+    sink = _randn(heads, dtype=torch.float32, seed=172)
+    for behind, lens in ((0, (533, 97)), (37, (641, 17)), (490, (27 * short // 16, 300))):
+        total = [behind + n for n in lens]
+        pages_each = -(-max(total) // page)
+        pages = _randn(2 * pages_each, 2, kv, page * d, dtype=bf, seed=170)
+        table = torch.arange(2 * pages_each, dtype=torch.int32, device="cuda").flip(0).view(2, pages_each).contiguous()
+        q = _randn(sum(lens), heads, d, dtype=bf, seed=171)
+        rows = AttnRows(slots=i32([0, 1]), lens=i32(total), query_start=i32([0, lens[0], sum(lens)]), decode_rows=None,
+                        chunk_rows=i32([0, 1]), n_decode=0, n_chunk=2, max_decode_len=0, max_chunk_query=max(lens),
+                        max_chunk_len=max(total))
+        last = total[0] - 1                                                                # (rows of its own tile weigh it by zero: left out below)
+        pages[table[0, last // page].long(), 1].view(kv, d, page)[:, :, last % page] = torch.inf
+        got = hip.paged_attention(q, pages, table, rows, page, d ** -0.5, window, sink=sink)
+        for b, first in ((0, 0), (1, lens[0])):
+            for s in range(0, lens[b], short):
+                n = min(short, lens[b] - s)
+                one = AttnRows(slots=i32([b]), lens=i32([behind + s + n]), query_start=i32([0, n]), decode_rows=None, chunk_rows=i32([0]),
+                               n_decode=0, n_chunk=1, max_decode_len=0, max_chunk_query=n, max_chunk_len=behind + s + n)
+                part = slice(first + s, first + s + n)
+                want = hip.paged_attention(q[part].contiguous(), pages, table, one, page, d ** -0.5, window, sink=sink)
+                mine = slice(0, max(0, n - 16) if b == 0 and s + n == lens[0] else n)
+                assert torch.equal(got[part][mine], want[mine]) and torch.isfinite(want[mine]).all(), (behind, b, s)
+
+
 def test_few_row_products_whose_steps_leave_a_rest(hip):
     """A wave's steps of 32 are multiplied in sets of 2, 4 or 8, and what is left over in a set by itself: every remainder of each, none
     among them, fewer steps than a set, for each number of waves a tile, both weight layouts and the gated form, against float64; a

@@ -264,13 +264,14 @@ __global__ void __launch_bounds__(WAVE) mlstm_scan_kernel(const T* __restrict__ 
 // scores in float64: a score's rounding is shared by all of the token's columns, and made results lie 1.2 times as far from 64 bits as
 // the token-by-token scan's (16 heads of 128 by 128 over 2,048 tokens: 1.56e-7 against 1.31e-7; so 1.14e-7, for 5 % of the time).
 // Bound by the float32 matrix cores (two products with S a token), by the barriers around a chunk, and in the second pass by its
-// registers: keys of 128 need all 256 and spill 42 of them (172 bytes a lane), keys of 256 138, with the LDS for two waves a SIMD (one
-// block a unit) to hide that; the first pass spills at keys of 256 alone (36). Two layers of 16 heads of 128 by 128 over steps of 4,096
+// registers: keys of 128 need all 256 and spill 42 of them (172 bytes a lane; 13 with bfloat16 keys and queries in pieces of 16 bytes,
+// PIECES, four prompts of 700 to 1,500 tokens of 16 heads 103 us and 95), keys of 256 138, with the LDS for two waves a SIMD (one
+// block a unit) to hide that; the first pass spills at keys of 256 alone (36; pieces would make it 83, so they go value by value). Two layers of 16 heads of 128 by 128 over steps of 4,096
 // and 304 tokens: 150 us for the first passes and 400 for the second ones (368 without the scores in float64 and the branch for
 // values that are not finite); token by token, a wave 8 columns with S in registers, 3,400 in all.
 // Operands: lane (g4, c) of A holds row c, of B column c, and product i of a group of 16 takes inner index 4 g4 + i, so that
 // a result's registers are the B operands of the products over its rows.
-template <int KD, int PASS, typename T>
+template <int KD, int PASS, bool PIECES, typename T>
 __global__ void __launch_bounds__(512) mlstm_chunk_kernel(const T* __restrict__ proj, int width, int q_off, int k_off,
                                                           int v_off, float* __restrict__ S_all, float* __restrict__ out,
                                                           float* __restrict__ den_out, const int32_t* __restrict__ slots,
@@ -279,7 +280,10 @@ __global__ void __launch_bounds__(512) mlstm_chunk_kernel(const T* __restrict__ 
                                                           int vdim, int col_blocks, MlstmPieces pc) {
   constexpr bool OUT = PASS == 2;
   constexpr int C = KD <= 128 ? 64 : 32, CT = C / 16, DT = KD / 16, QS = KD + 4, MS = C + 4, THREADS = 512;
-  constexpr int PER = C * KD / THREADS, TPT = THREADS / C;                  // staged values a thread; threads a token
+  constexpr int VEC = PIECES ? 16 / (int)sizeof(T) : 1;      // values of a load
+  constexpr int PER = C * KD / THREADS / VEC, TPT = THREADS / C;            // staged pieces a thread; threads a token
+  static_assert(!PIECES || PER >= 1, "a piece a thread");
+  struct alignas(VEC * sizeof(T)) Piece { T v[VEC]; };
   __shared__ __attribute__((aligned(16))) float qs[OUT ? C * QS : 4], ks[C * QS];
   __shared__ __attribute__((aligned(16))) float score[OUT ? C * MS : 4], fade[OUT ? C * MS : 4];
   __shared__ __attribute__((aligned(16))) float p_s[C], e_s[C];      // (read 16 bytes at a time, as those above)
@@ -316,15 +320,16 @@ __global__ void __launch_bounds__(512) mlstm_chunk_kernel(const T* __restrict__ 
   const float q_scale = 1.0f / sqrtf((float)dim);
   // what a chunk needs, on its way to registers: places that do not exist are read from ones that do and made harmless
   // when the values are used, so that nothing here waits for a load
-  T nq[OUT ? PER : 1], nk[PER], nv[CT][4];
+  Piece nq[OUT ? PER : 1], nk[PER];
+  T nv[CT][4];
   float ng[3];
   auto ask = [&](int t0) {
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      const int idx = tid + e * THREADS, t = min(t0 + idx / KD, hi - 1), d = min(idx % KD, dim - 1);
+      const int idx = (tid + e * THREADS) * VEC, t = min(t0 + idx / KD, hi - 1), d = PIECES ? idx % KD : min(idx % KD, dim - 1);
       const T* row = proj + (int64_t)t * width + h * dim + d;
-      nk[e] = row[k_off];
-      if constexpr (OUT) nq[e] = row[q_off];
+      nk[e] = *reinterpret_cast<const Piece*>(row + k_off);
+      if constexpr (OUT) nq[e] = *reinterpret_cast<const Piece*>(row + q_off);
     }
 #pragma unroll
     for (int tt = 0; tt < CT; ++tt)
@@ -338,10 +343,13 @@ __global__ void __launch_bounds__(512) mlstm_chunk_kernel(const T* __restrict__ 
   for (int t0 = lo; t0 < hi; t0 += C) {
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      const int idx = tid + e * THREADS;
-      const bool ok = t0 + idx / KD < hi && idx % KD < dim;
-      ks[idx / KD * QS + idx % KD] = ok ? Elem<T>::load(nk[e]) : 0.f;
-      if constexpr (OUT) qs[idx / KD * QS + idx % KD] = ok ? Elem<T>::load(nq[e]) * q_scale : 0.f;
+      const int idx = (tid + e * THREADS) * VEC, at = idx / KD * QS + idx % KD;
+      const bool ok = t0 + idx / KD < hi && (PIECES || idx % KD < dim);
+#pragma unroll
+      for (int x = 0; x < VEC; ++x) {
+        ks[at + x] = ok ? Elem<T>::load(nk[e].v[x]) : 0.f;
+        if constexpr (OUT) qs[at + x] = ok ? Elem<T>::load(nq[e].v[x]) * q_scale : 0.f;
+      }
     }
     if (tid < C) {
       const bool ok = t0 + tid < hi;                       // (a token that is not there keeps everything and adds nothing)
@@ -512,12 +520,22 @@ template <typename T, int KD>
 void launch_chunks(int pass, dim3 grid, hipStream_t s, const void* proj, int width, int q_off, int k_off, int v_off, float* S,
                    float* out, float* den, const int32_t* slots, const int32_t* starts, const int32_t* qs, int heads,
                    int dim, int vdim, int col_blocks, MlstmPieces pc) {
-  if (pass == 1)
-    mlstm_chunk_kernel<KD, 1, T><<<grid, 512, 0, s>>>((const T*)proj, width, q_off, k_off, v_off, S, out, den, slots, starts,
-                                                      qs, heads, dim, vdim, col_blocks, pc);
-  else
-    mlstm_chunk_kernel<KD, 2, T><<<grid, 512, 0, s>>>((const T*)proj, width, q_off, k_off, v_off, S, out, den, slots, starts,
-                                                      qs, heads, dim, vdim, col_blocks, pc);
+  // keys and queries in pieces of 16 bytes, where all of a head's values are there and lie on such borders
+  constexpr int V = 16 / (int)sizeof(T);
+  const bool pieces = dim == KD && width % V == 0 && q_off % V == 0 && k_off % V == 0 && (uintptr_t)proj % 16 == 0;
+#define CHUNKS(PASS, PIECES)                                                                                                       \
+  mlstm_chunk_kernel<KD, PASS, PIECES, T><<<grid, 512, 0, s>>>((const T*)proj, width, q_off, k_off, v_off, S, out, den, slots, starts, \
+                                                               qs, heads, dim, vdim, col_blocks, pc)
+  if constexpr (KD == 64 || KD == 128) {
+    if (pieces) {
+      if (pass == 1) CHUNKS(1, true);
+      else CHUNKS(2, true);
+      return;
+    }
+  }
+  if (pass == 1) CHUNKS(1, false);
+  else CHUNKS(2, false);
+#undef CHUNKS
 }
 }  // namespace
 

@@ -686,6 +686,33 @@ def test_the_matrix_memory_in_pieces_at_its_edges(heads, d, v, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads,d", [(2, 64), (3, 128)])
+def test_keys_and_queries_in_pieces_of_16_bytes_are_the_same_bits(heads, d, dtype):
+    """Rows whose width keeps every head on a border of 16 bytes against the same values in rows one longer; portions that end inside
+    a chunk, at its end and one behind it, infinities among the keys."""
+    import holon_amd.parts  # noqa: F401  (registers the parts' operations)
+    from holon_amd.kernels import load_hip
+    k, dev, piece = load_hip(), torch.device("cuda"), 128
+    gen = torch.Generator().manual_seed(d)
+    rn = lambda *s: torch.randn(s, generator=gen).to(dev)                      # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)             # noqa: E731
+    counts = [256, 193, 63, 128]
+    t, hd, copies = sum(counts), heads * d, -(-(d + 1) // 8)
+    npc = [-(-n // piece) for n in counts]
+    proj, gb = rn(t, 4 * hd + 16).to(dtype), rn(2 * heads)
+    proj[300, hd + 5] = torch.inf
+    state = [rn(4, heads, d, d + 1), rn(4, heads, 1).expand(4, heads, copies).contiguous()]
+    rows = (i32([3, 0, 1, 2]), i32([0, 9, 5, 0]), i32([sum(counts[:b]) for b in range(5)]), 4, heads, d, d)
+    cut = (piece, max(npc), i32([sum(npc[:b]) for b in range(4)]), sum(npc))
+    seen = []
+    for rows_of in (proj, torch.nn.functional.pad(proj, (0, 1))):
+        held = [x.clone() for x in state]
+        seen.append([*k.mlstm_scan(rows_of, 0, hd, 2 * hd, 3 * hd, gb, 12.0, *held, *rows, cut), *held])
+    assert all(torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)) for a, b in zip(*seen))
+
+
+@pytest.mark.gpu
 def test_prompts_keep_the_orders_of_sums_they_have():
     """A matrix memory's norm brings a read-out near nothing to unit length, so that any other order of a sum in front of it can move a
     row by more than rounding does: a model with one keeps the forms of 17 rows and more that its logits have been compared in (the

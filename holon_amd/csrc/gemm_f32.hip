@@ -167,7 +167,7 @@ __global__ void __launch_bounds__(256) gemm_f32_in_order_kernel(const float* __r
 // tiles up to 32 rows (10; with a 64 x 64 tile a block and no split of K it took 118), quarters side by side from 300 rows (38; one after
 // the other 46), blocks of 32 rows at 700 (65; of 64 rows 76, whose second round is mostly empty); 2048 x 9248 at 704 rows blocks of 32
 // (268; of 64 313); 16384 x 2048 1 x 1 tiles up to 16 rows (5.0 TB/s at one row), quarters side by side at 64 (42; one after the other
-// 53), blocks of 32 at 150 (108; 113), of 64 at 825 (480; of 32 571); 9248 x 256 at 2,048 rows one after the other (95; side by side 139).
+// 53), blocks of 32 at 150 (108; 116), of 64 at 825 (502; of 32 571); 9248 x 256 at 2,048 rows one after the other (95; side by side 139).
 struct Form { int mt, nt; float start, start_k, round, round_k; };
 enum { SIDE_BY_SIDE = 4, IN_TURN = 5, IN_TURN_32 = 6, KINDS = 7 };
 constexpr Form FORMS[KINDS] = {{1, 1, 2.6f, 2e-4f, 0.43f, 3.25e-3f},   {1, 2, 2.5f, 2e-4f, 0.63f, 5.0e-3f},    {2, 2, 2.5f, 7e-4f, 0.90f, 7.35e-3f},

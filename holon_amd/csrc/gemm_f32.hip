@@ -213,14 +213,10 @@ void launch(const float* x, const float* w, float* y, int M, int N, int K, hipSt
 }
 }  // namespace
 
-// Which form serves M rows of operands on 16 bytes: 0 to 3 tiles of 1 x 1, 1 x 2, 2 x 2 and 2 x 4 a block; 4 and 5 staged tiles, 4 for outputs
-// of few (the quarters of K side by side, or blocks of 32 rows) and 5 for outputs of many (64 x 64, the quarters one after the other); -1 one
-// running sum.
-extern "C" int holon_gemm_f32_form(int M, int N, int K) {
-  if (sums_in_order(N, K)) return -1;
-  const int form = pick_form(M, N, K, K % CHUNK == 0);
-  return form == IN_TURN_32 ? SIDE_BY_SIDE : form;
-}
+// Which form serves M rows of operands on 16 bytes: 0 to 3 tiles of 1 x 1, 1 x 2, 2 x 2 and 2 x 4 a block straight from memory; 4 to 6 staged
+// ones, 64 x 64 a block with the quarters of K side by side (4) or one after the other (5), and 32 x 64 one after the other (6, whole
+// chunks of K alone); -1 one running sum.
+extern "C" int holon_gemm_f32_form(int M, int N, int K) { return sums_in_order(N, K) ? -1 : pick_form(M, N, K, K % CHUNK == 0); }
 
 extern "C" int holon_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K, void* stream) {
   HOLON_CHECK(M >= 0 && N > 0 && K > 0, "gemm (float32): M=%d N=%d K=%d", M, N, K);

@@ -1561,14 +1561,15 @@ def test_float32_product_of_short_sums(hip):
 
 
 def test_float32_product_of_long_sums_takes_the_form_that_is_done_first(hip):
-    """Some hundred rows over K beyond 4,096 take 64 x 64 tiles with the quarters of K side by side (tiles of 32 x 64 straight from
-    memory take 15 % longer), few rows narrow tiles, wide weights one running sum; against the float64 product, each row bit for bit
-    what it is alone."""
+    """Some hundred rows over K beyond 4,096 take staged tiles, 32 x 64 a block where 64 x 64 would leave a last round mostly empty, else
+    64 x 64 with the quarters of K side by side; few rows narrow tiles straight from memory, wide weights one running sum. Each of these
+    forms against the float64 product, each row bit for bit what it is alone."""
     form = hip.lib.holon_gemm_f32_form
-    assert [form(m, 2048, 18432) for m in (1, 17, 704)] == [0, 0, 4]
-    assert [form(704, 2048, 9248), form(500, 3072, 12288), form(300, 4096, 18432), form(2048, 2048, 2048)] == [4, 4, 4, 5]
+    assert [form(m, 2048, 18432) for m in (1, 17, 704)] == [0, 0, 6]
+    assert [form(704, 2048, 9248), form(500, 3072, 12288), form(300, 4096, 18432), form(2048, 2048, 2048)] == [6, 6, 6, 5]
     assert [form(m, n, k) for m, n, k in ((1, 6144, 4096), (704, 4097, 4096), (704, 4096, 4096))] == [-1, -1, 4]
-    for m, n, k in ((130, 2048, 4608), (400, 2048, 5120), (300, 1056, 9248), (67, 4096, 6150)):
+    for m, n, k, taken in ((130, 2048, 4608, 3), (400, 2048, 5120, 4), (300, 1056, 9248, 3), (67, 4096, 6150, 3), (500, 3072, 4160, 6)):
+        assert form(m, n, k) == taken, (m, n, k)
         x, w = _randn(m, k, dtype=torch.float32, seed=140), _randn(n, k, dtype=torch.float32, seed=141)
         got, want = hip.linear(x, w), x.double() @ w.double().T
         bound = (-(-k // 512) * 32 + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
@@ -1577,14 +1578,17 @@ def test_float32_product_of_long_sums_takes_the_form_that_is_done_first(hip):
             assert torch.equal(hip.linear(x[row: row + 1].contiguous(), w)[0], got[row]), (m, n, k, row)
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 130, 96), (97, 4160, 1056), (161, 1000, 544), (300, 2048, 4128), (700, 2048, 2048), (705, 2049, 2016),
-                                   (825, 3072, 1024), (825, 16384, 64), (1030, 2100, 32), (33, 9248, 160)])
-def test_float32_products_copied_straight_into_lds(hip, m, n, k):
-    """Blocks of 64 and of 32 rows, edges of both, K that ends in each quarter: bit for bit what operands give that pass registers (those
-    off a border of 16 bytes) and what a row is alone; against the float64 product."""
+@pytest.mark.parametrize("m,n,k,form", [(33, 4160, 64, 6), (825, 16384, 64, 5), (97, 16384, 160, 5), (500, 2100, 288, 6), (705, 16384, 416, 5),
+                                        (65, 9248, 512, 6), (705, 3072, 544, 6), (300, 3072, 704, 4), (33, 9248, 800, 4), (825, 3072, 1024, 6),
+                                        (97, 4160, 1056, 4), (705, 2049, 2016, 6), (1030, 9248, 2016, 5), (700, 2048, 2048, 6), (300, 2048, 4128, 4)])
+def test_float32_products_copied_straight_into_lds(hip, m, n, k, form):
+    """Each of the staged forms (blocks of 64 and of 32 rows, the quarters of K side by side where it is long enough for that), edges of
+    their tiles, K that ends in each quarter: bit for bit what operands give that pass registers (those off a border of 16 bytes) and what
+    a row is alone; against the float64 product."""
+    assert hip.lib.holon_gemm_f32_form(m, n, k) == form
     x, w = _randn(m, k, dtype=torch.float32, seed=142), _randn(n, k, dtype=torch.float32, seed=143)
     got, want = hip.linear(x, w), x.double() @ w.double().T
-    bound = (-(-k // 512) * 32 + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    bound = (max(64, -(-k // 512) * 32) + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
     assert ((got.double() - want).abs() <= bound).all()
     off = torch.empty(m * k + 1, dtype=torch.float32, device="cuda")[1:].view(m, k).copy_(x)
     assert off.data_ptr() % 16 and torch.equal(hip.linear(off, w), got)

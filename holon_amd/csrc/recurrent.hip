@@ -534,29 +534,37 @@ __global__ void shift_mix_kernel(const T* __restrict__ x, const T* __restrict__ 
   if (keep) state[(int64_t)slots[b] * width + c] = x[(int64_t)t * width + c];
 }
 
-// The same, eight neighbouring channels a thread: 2,048 tokens of 2,048, mixed five times, 12.1 us, a channel a thread 23.
+// The same, 16 bytes of neighbouring channels a thread and load, for steps of SHIFT_PIECES_FROM values (tokens times channels) and more: below, a
+// block's round of latency is what a step takes, and a thread with more to do makes it longer. In us, pieces against a channel a thread: 2,048
+// tokens of 2,048 mixed five times 13.3 / 22.9 (bfloat16) and 21.1 / 22.5 (float32), 192 tokens 5.6 / 5.9 and 5.9 / 6.0; 384 of 1,024 5.2 / 5.7 and
+// 5.5 / 5.5; 64 of 2,048 5.1 / 4.7 and 5.2 / 4.7, one 5.1 / 4.5 and 5.1 / 4.4. (Eight float32 channels a thread, 32 bytes apart from the next
+// thread's, took up to 1.29 times as long as one.)
+constexpr int64_t SHIFT_PIECES_FROM = 393216;
 template <typename T>
 __global__ void __launch_bounds__(256) shift_mix_rows_kernel(const T* __restrict__ x, const T* __restrict__ mu, T* __restrict__ state,
                                                              T* __restrict__ y, const int32_t* __restrict__ slots,
                                                              const int32_t* __restrict__ starts, const int32_t* __restrict__ query_start,
                                                              const int32_t* __restrict__ token_row, int tokens, int width, int mixes,
                                                              int keep) {
-  const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
+  constexpr int N = Elem<T>::kVec;
+  struct alignas(16) Piece { T v[N]; };
+  const int c = (blockIdx.x * 256 + threadIdx.x) * N;
   const int t = blockIdx.y;
   if (c >= width) return;
   const int b = keep ? t : token_row[t];
-  float prev[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, cur[8];
-  head_rows::load8(x + (int64_t)t * width + c, cur);
-  if (!keep && t > query_start[b]) head_rows::load8(x + (int64_t)(t - 1) * width + c, prev);
-  else if (starts[b] > 0) head_rows::load8(state + (int64_t)slots[b] * width + c, prev);
+  Piece prev{}, cur = *reinterpret_cast<const Piece*>(x + (int64_t)t * width + c);
+  if (!keep && t > query_start[b]) prev = *reinterpret_cast<const Piece*>(x + (int64_t)(t - 1) * width + c);
+  else if (starts[b] > 0) prev = *reinterpret_cast<const Piece*>(state + (int64_t)slots[b] * width + c);
   for (int s = 0; s < mixes; ++s) {
-    float m[8];
-    head_rows::load8(mu + (int64_t)s * width + c, m);
+    Piece m = *reinterpret_cast<const Piece*>(mu + (int64_t)s * width + c);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) m[j] = cur[j] + (prev[j] - cur[j]) * m[j];
-    head_rows::store8(y + ((int64_t)s * tokens + t) * width + c, m);
+    for (int j = 0; j < N; ++j) {
+      const float now = Elem<T>::load(cur.v[j]), before = Elem<T>::load(prev.v[j]);
+      m.v[j] = Elem<T>::store(now + (before - now) * Elem<T>::load(m.v[j]));
+    }
+    *reinterpret_cast<Piece*>(y + ((int64_t)s * tokens + t) * width + c) = m;
   }
-  if (keep) head_rows::store8(state + (int64_t)slots[b] * width + c, cur);
+  if (keep) *reinterpret_cast<Piece*>(state + (int64_t)slots[b] * width + c) = cur;
 }
 
 template <typename T>
@@ -845,8 +853,10 @@ extern "C" int holon_shift_mix(const void* x, const void* mu, void* state, void*
   const dim3 block(256), grid_t((width + 255) / 256, tokens), grid_b((width + 255) / 256, rows);
   HOLON_CHECK(!rows_in_order || tokens == rows, "shift_mix: rows in order means one token a row, got %d in %d", tokens,
               rows);
-  if (width % 8 == 0 && head_rows::on16(x) && head_rows::on16(mu) && head_rows::on16(state) && head_rows::on16(y))
-    BY_DTYPE(dtype, (shift_mix_rows_kernel<T><<<dim3((width + 2047) / 2048, tokens), block, 0, s>>>(
+  const int piece = dtype == HOLON_F32 ? Elem<float>::kVec : Elem<bf16_t>::kVec;
+  if ((int64_t)tokens * width >= SHIFT_PIECES_FROM && width % piece == 0 && head_rows::on16(x) && head_rows::on16(mu) && head_rows::on16(state) &&
+      head_rows::on16(y))
+    BY_DTYPE(dtype, (shift_mix_rows_kernel<T><<<dim3((width / piece + 255) / 256, tokens), block, 0, s>>>(
                         (const T*)x, (const T*)mu, (T*)state, (T*)y, slots, starts, query_start, token_row, tokens, width, mixes,
                         rows_in_order)));
   else

@@ -2149,6 +2149,36 @@ def test_rows_in_pieces_are_the_rows_value_by_value(hip, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_shifts_of_many_tokens_in_pieces_are_those_channel_by_channel(hip, dtype):
+    """Steps on both sides of the size from which a thread takes 16 bytes of channels (393,216 values), widths that do not fill a block, in one
+    piece of float32 alone, rows of one token and of many, behind kept tokens and not, in order and not: bit for bit what operands off a border of
+    16 bytes give, which go channel by channel; against the plain form a rounding or two of the result's type."""
+    from holon_amd.kernels.registry import kernel_op
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                      # noqa: E731
+    for tokens, width, mixes in ((191, 2048, 5), (192, 2048, 5), (200, 2056, 3), (203, 2060, 2), (96, 4096, 1), (24576, 16, 2), (50, 7872, 2)):
+        counts = [1, 5, tokens - 6]
+        first, row = i32([0, 1, 6, tokens]), torch.repeat_interleave(torch.arange(3), torch.tensor(counts)).to(torch.int32).cuda()
+        x, mu, kept = _randn(tokens, width, dtype=dtype, seed=216), _randn(mixes, width, dtype=dtype, seed=217), _randn(4, width, dtype=dtype, seed=218)
+        made = []
+        for rows in (x, _moved(x)):
+            state = kept.clone()
+            made.append((hip.shift_mix(rows, mu, state, i32([2, 0, 3]), i32([0, 3, 9]), first, row, 3), state))
+        state = kept.clone()
+        want = kernel_op("shift_mix").plain(x, mu, state, i32([2, 0, 3]), i32([0, 3, 9]), first, row, 3), state
+        assert all(torch.equal(a, b) for a, b in zip(*made)) and torch.equal(made[0][1], want[1]), (tokens, width)
+        assert H.rel_rms(made[0][0], want[0]) < (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22), (tokens, width)
+        if tokens > 300:
+            continue
+        made, slots = [], torch.randperm(tokens, generator=torch.Generator().manual_seed(219)).to(torch.int32).cuda()
+        starts, each = i32([n % 3 for n in range(tokens)]), i32(list(range(tokens + 1)))
+        kept = _randn(tokens, width, dtype=dtype, seed=219)
+        for rows in (x, _moved(x)):
+            state = kept.clone()
+            made.append((hip.shift_mix(rows, mu, state, slots, starts, each, each[:-1].contiguous(), tokens, in_order=True), state))
+        assert all(torch.equal(a, b) for a, b in zip(*made)) and torch.equal(made[0][1][slots.long()], x), (tokens, width)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_routers_of_many_rows_are_those_of_few(hip, dtype):
     """Tokens that share what a wave reads of the router (one, two or four of them, by the rows) have bit for bit the weights of a token by
     itself: rows on both sides of the lines, experts that do not come in eights, widths that do not fill a wave's step."""

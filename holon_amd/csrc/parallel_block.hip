@@ -455,6 +455,16 @@ static int one_type(const void* d1, int dt1, const void* d2, int dt2, const void
   return (d1 && dt1 != dt) || (d2 && dt2 != dt) || (w1 && dtw != dt) ? -1 : dt;
 }
 
+// Whether rows of bfloat16 terms under float32 weights ask ahead: a block then holds eight to twelve registers more a step, so that of the
+// 2,048 blocks that the chip holds of the general form some wait for a second round. Where that shows is an added vector without terms from
+// 1,025 rows on (2,048 rows of 2,560 / 3,072 / 4,096 9.4 / 10.8 / 14.8 us, in the general form 9.0 / 9.9 / 12.6), and about 2,048 rows of up to 2,560
+// (one term, two weights 12.5 / 11.9). Elsewhere it is 0.71 to 1.03 of the general form's time: four rows of 2,048 2.4 / 3.2, 512 with two terms
+// 0.84, 8,192 0.96.
+static bool wide_ahead_pays(int64_t rows, int dim, bool terms, bool added) {
+  if (rows > 2048) return true;
+  return added && !terms ? rows <= 1024 || dim <= 2048 : rows <= 1792 || dim <= 1536 || dim > 2560;
+}
+
 extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void* d2, int dt2, const float* row,
                                 const void* w1, const void* w2, int dtw, void* y1, void* y2, int64_t rows, int dim,
                                 float eps, int dt_out, void* stream) {
@@ -467,7 +477,8 @@ extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void*
   if (dim % 4 == 0 && dim <= 8192) {        // four values a thread and step (every operand is a tensor's start: 16 bytes)
     const Filters none{};
     const int one = one_type(d1, dt1, d2, dt2, w1, dtw, dt_out);
-    const bool wide_weights = w1 && dtw == HOLON_F32 && one_type(d1, dt1, d2, dt2, w1, dt_out, dt_out) == HOLON_BF16;
+    const bool wide_weights = w1 && dtw == HOLON_F32 && one_type(d1, dt1, d2, dt2, w1, dt_out, dt_out) == HOLON_BF16 &&
+                              wide_ahead_pays(rows, dim, d1 != nullptr, row != nullptr);
 #define SRMSV(...) stream_rms_vec_kernel<__VA_ARGS__><<<(unsigned)rows, 256, 0, s>>>(x32, d1, dt1, d2, dt2, row, w1, w2, dtw, y1, y2, dim, eps, dt_out, none)
 #define SRMSV_BY_TYPE(R)                                 \
   do {                                                   \

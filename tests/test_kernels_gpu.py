@@ -1919,8 +1919,10 @@ def test_decode_rows_of_every_last_block(hip, geometry, softcap):
 @pytest.mark.parametrize("dim", [4, 1020, 1028, 2048, 2560, 3072, 3076, 4092, 4096, 4100])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_stream_rows_of_one_type_are_those_of_several(hip, dtype, dim):
-    """A pass over stream rows whose operands are of one type and asked for ahead gives the bits of the general one (taken here by a term
-    of the other type that holds the same values, or by a weight that does): with and without terms, vector, second weight, filters."""
+    """A pass over stream rows whose operands are asked for ahead gives the bits of the general one: of one type, or bfloat16 under float32
+    weights that hold the same values (without filters; float32 rows under bfloat16 weights take the general form). The general one is
+    taken by a term of the other type that holds the same values, and without terms by results in float32, rounded here: with and without
+    terms, vector, second weight, filters."""
     import holon_amd.parts.parallel_block  # noqa: F401  (brings the operations)
     other = torch.float32 if dtype == torch.bfloat16 else torch.bfloat16
     rows = 3
@@ -1943,8 +1945,27 @@ def test_stream_rows_of_one_type_are_those_of_several(hip, dtype, dim):
                     y += [*hip.stream_rms_filter(*args, c1, c2 if second is not None else None, hs[0], hs[1] if second is not None else None,
                                                  slots, starts), xs.clone(), hs]
                     got.append([v for v in y if v is not None])
+                if dtype == torch.bfloat16 and not terms:
+                    y = [v.bfloat16() for v in hip.stream_rms(x.clone(), [], added, w1, second, 1e-6, torch.float32) if v is not None]
+                    assert all(torch.equal(a, b) for a, b in zip(y, got[0])), (added is None, second is None)
                 for one in got[1:]:
                     assert all(torch.equal(a, b) for a, b in zip(one, got[0], strict=True)), (len(terms), added is None, second is None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1024, 1025, 1792, 1793, 2048, 2049])
+def test_many_stream_rows_under_float32_weights(hip, rows):
+    """bfloat16 terms under float32 weights on both sides of the rows and widths from which they are not asked for ahead: bit for bit the
+    general form (taken by results in float32 under bfloat16 weights, rounded here)."""
+    import holon_amd.parts.parallel_block  # noqa: F401  (brings the operations)
+    for dim in (1536, 1540, 2048, 2052, 2560, 2564, 4096):
+        x, row = _randn(rows, dim, dtype=torch.float32, seed=229), _randn(dim, dtype=torch.float32, seed=230)
+        t1, (w1, w2) = _randn(rows, dim, dtype=torch.bfloat16, seed=231), (_randn(dim, dtype=torch.bfloat16, seed=s) for s in (232, 233))
+        for terms, added, second in (([], None, None), ([], row, w2), ([t1], None, w2), ([t1, t1], row, None)):
+            a, b = x.clone(), x.clone()
+            got = hip.stream_rms(a, [(t, 1.0) for t in terms], added, w1.float(), None if second is None else second.float(), 1e-6, torch.bfloat16)
+            want = hip.stream_rms(b, [(t, 1.0) for t in terms], added, w1, second, 1e-6, torch.float32)
+            assert torch.equal(a, b) and all(torch.equal(g, w.bfloat16()) for g, w in zip(got, want) if w is not None), (dim, len(terms))
 
 
 @pytest.mark.gpu

@@ -18,6 +18,10 @@
 // Softmax is online, float32, in base 2 with log2(e) folded into the scale.
 #include <mutex>
 
+#include <stdlib.h>
+
+#include <algorithm>
+
 #include "common.h"
 #include "holon_hip.h"
 
@@ -484,8 +488,8 @@ __global__ void __launch_bounds__(256) attn_prefill_kernel(AttnArgs a) {
 // row c, then row 16 + c), which with a row pitch of D + 8 makes the 16-byte reads conflict-free; value rows have a
 // pitch of 40. To even out the causal mask, a block does two position ranges: the b-th from the start and the b-th
 // from the end (unpaired: a block each).
-// Heads of 256 take eight waves a block (74 KB of LDS a block, two waves a SIMD): the bits of the kernel that reads them straight from the
-// cache, whose every wave waits for its own 32 KB a stage. What bounds it is those 32 KB a wave and stage out of LDS.
+// Heads of 256 take eight waves a block (89 KB of LDS, so one block a unit, two waves a SIMD): the bits of the kernel that reads them straight from
+// the cache, whose every wave waits for its own 32 KB a stage. What bounds it is those 32 KB a wave and stage out of LDS.
 template <int D, int NT, int WAVES = 4>
 __global__ void __launch_bounds__(WAVES * WAVE) attn_prefill_lds_kernel(AttnArgs a) {
   constexpr int KP = D + 8;    // pitch of a key row in LDS (elements)
@@ -1984,11 +1988,47 @@ struct ScoreMod {
   int keep_first;
 };
 
+// Heads of 256 in the order of 32 keys a product that short rows have (`staged_256` off below, or more than 32 heads a group): how a step's
+// portions run. Straight from the cache a wave walks its own 16 rows' keys; staged, a block walks those of all of its eight waves, holds a
+// unit to itself, and costs its launch also where a row is too short to have it.
+struct Staged256 {
+  bool pays;
+  int ranges, unpaired;
+};
+// Without a window staged from 576 keys on, or from 512 where tiles outnumber the SIMDs (16 heads over one, us, straight from the cache against
+// staged: prompts of 300 tokens 27 / 29, 512 42 / 41, 600 49 / 47, 1,024 78 / 68, 4,096 591 / 314, eight of 512 124 / 83, 64 tokens behind 8,000
+// 546 / 430; 16 over 16, 512 tokens 42 / 45, 600 49 / 47, eight of 512 156 / 88). Under a window a wave's walk is short, so only where the tiles
+// outnumber the SIMDs and the window is 512 keys and more, or 100 and more with tiles for every group of heads and a quarter of the launched
+// blocks at work (16 over one within 128: 1,024 tokens 20 / 24, 2,048 38 / 26; 32 over 8 within 128, 1,500 tokens beside twelve of 40 80 / 108,
+// four of 700 to 1,500 78 / 63 of 16 over one; within 512, 1,500 beside twelve of 40 84 / 55). Over 1,110 steps nothing was longer than
+// straight from the cache by more than 5 %; staged from 512 keys on whatever else, half of them were, up to 1.9 times.
+static Staged256 stages_256(int heads, int kv_heads, int n_rows, int max_query, int max_len, int window, int tokens) {
+  const TileMap tm = tile_map(heads / kv_heads);
+  const int64_t most = (int64_t)n_rows * max_query, positions = tokens > 0 && tokens < most ? tokens : most;
+  const int tiles = (max_query + tm.pos_per_tile - 1) / tm.pos_per_tile, groups = kv_heads * tm.head_blocks, ranges = (tiles + 7) / 8;
+  const int64_t waves = std::min<int64_t>((int64_t)n_rows * tiles, positions / tm.pos_per_tile + n_rows) * groups;
+  const int64_t pairs = std::min<int64_t>((int64_t)n_rows * ((ranges + 1) / 2), positions / (16 * tm.pos_per_tile) + n_rows) * groups;
+  Staged256 f{false, ranges, pairs < UNPAIR_BELOW && n_rows <= 32767 ? 1 : 0};
+  if (tiles < 16 || max_len < 512) return f;
+  const int64_t launched = (int64_t)n_rows * ((ranges + 1) / 2) * (f.unpaired ? 2 : 1) * groups;
+  const int64_t real = std::min<int64_t>(launched, (positions / (8 * tm.pos_per_tile) + n_rows) * groups), span = std::abs((int64_t)window);
+  if (span == 0) f.pays = max_len >= 576 || waves > 1024;
+  else f.pays = waves > 1024 && (span >= 512 || (span >= 100 && waves > 1024 * tm.head_blocks && 4 * real >= launched));
+  return f;
+}
+
+// Whether portions of heads of 256 in that order go through LDS.
+extern "C" int holon_attention_prefill_one_order_staged(int heads, int kv_heads, int n_rows, int max_query, int max_len, int page_size, int window,
+                                                        int tokens) {
+  return heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && max_len <= (int64_t)4096 * page_size &&
+         stages_256(heads, kv_heads, n_rows, max_query, max_len, window, tokens).pays;
+}
+
 static int prefill_launch(const void* q, void* out, const void* pages, const int32_t* table, int table_stride,
                           const int32_t* slots, const int32_t* lens, const int32_t* query_start, const int32_t* row_ids,
                           int n_rows, int max_query, int max_len, int heads, int kv_heads, int head_dim, int page_size,
                           float scale, int window, const float* sink, void* stream, const ScoreMod* mod = nullptr,
-                          int v_share = 1, const void* hgate = nullptr, int64_t hgate_stride = 0, bool staged_256 = true) {
+                          int v_share = 1, const void* hgate = nullptr, int64_t hgate_stride = 0, bool staged_256 = true, int tokens = 0) {
   HOLON_CHECK(mfma_serves(head_dim, page_size), "attention (matrix cores): head_dim %d / page %d not served", head_dim,
               page_size);
   HOLON_CHECK(heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && window > -0x7fffffff && table_stride > 0,
@@ -2086,13 +2126,10 @@ static int prefill_launch(const void* q, void* out, const void* pages, const int
     HOLON_LAUNCH_OK();
     return 0;
   }
-  // Heads of 256 in the order of 32 keys a product that short rows have (`staged_256` off, or more than 32 heads a group): staged from 512
-  // keys on, the same bits. 16 heads over one, us, straight from the cache against staged: prompts of 300 tokens 27 / 29, 512 41 / 40, 1,024
-  // 78 / 68, 4,096 591 / 314, four of 700 to 1,500 224 / 137, eight of 100 15 / 17; 64 tokens behind 8,000 546 / 430, 20 behind 600 49 / 46.
-  if (head_dim == 256 && tiles >= 16 && max_len >= 512 && max_len <= 4096 * page_size) {
-    const int ranges = (tiles + 7) / 8;
-    a.unpaired = (int64_t)((ranges + 1) / 2) * kv_heads * tm.head_blocks * n_rows < UNPAIR_BELOW ? 1 : 0;
-    dim3 lgrid((ranges + 1) / 2, kv_heads * tm.head_blocks, a.unpaired ? 2 * n_rows : n_rows);
+  if (head_dim == 256 && holon_attention_prefill_one_order_staged(heads, kv_heads, n_rows, max_query, max_len, page_size, window, tokens)) {
+    const Staged256 f = stages_256(heads, kv_heads, n_rows, max_query, max_len, window, tokens);
+    a.unpaired = f.unpaired;
+    dim3 lgrid((f.ranges + 1) / 2, kv_heads * tm.head_blocks, f.unpaired ? 2 * n_rows : n_rows);
     attn_prefill_lds_kernel<256, 1, 8><<<lgrid, 512, 0, (hipStream_t)stream>>>(a);
     HOLON_LAUNCH_OK();
     return 0;
@@ -2126,15 +2163,16 @@ extern "C" int holon_attention_prefill_sink_bf16(const void* q, void* out, const
                         heads, kv_heads, head_dim, page_size, scale, window, sink, stream);
 }
 
-// The same with the operands of heads of 256 straight from the cache whatever the rows' length, in the order of sums that short rows have.
-extern "C" int holon_attention_prefill_from_cache_bf16(const void* q, void* out, const void* pages, const int32_t* table,
+// The same with one order of sums for heads of 256 whatever the rows' length, the one that short rows have; `tokens`: how many the portions hold
+// in all, or more (0: not known).
+extern "C" int holon_attention_prefill_one_order_bf16(const void* q, void* out, const void* pages, const int32_t* table,
                                                        int table_stride, const int32_t* slots, const int32_t* lens,
                                                        const int32_t* query_start, const int32_t* row_ids, int n_rows,
                                                        int max_query, int max_len, int heads, int kv_heads, int head_dim,
                                                        int page_size, float scale, int window, const float* sink,
-                                                       void* stream) {
+                                                       int tokens, void* stream) {
   return prefill_launch(q, out, pages, table, table_stride, slots, lens, query_start, row_ids, n_rows, max_query, max_len,
-                        heads, kv_heads, head_dim, page_size, scale, window, sink, stream, nullptr, 1, nullptr, 0, false);
+                        heads, kv_heads, head_dim, page_size, scale, window, sink, stream, nullptr, 1, nullptr, 0, false, tokens);
 }
 
 // Prompt portions of windowed attention with sigmoid weights (head sizes 64 and 128, keys and values of one width,

@@ -84,13 +84,15 @@ int holon_attention_prefill_sink_bf16(const void* q, void* out, const void* page
                                       const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_query,
                                       int max_len, int heads, int kv_heads, int head_dim, int page_size, float scale,
                                       int window, const float* sink, void* stream);
-// The prompt entry point with heads of 256 read straight from the cache whatever the rows' length (a row of more than 192 tokens has its
-// stages copied into LDS otherwise, in another order of sums).
-int holon_attention_prefill_from_cache_bf16(const void* q, void* out, const void* pages, const int32_t* table,
-                                            int table_stride, const int32_t* slots, const int32_t* lens,
-                                            const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_query,
-                                            int max_len, int heads, int kv_heads, int head_dim, int page_size, float scale,
-                                            int window, const float* sink, void* stream);
+// The prompt entry point with one order of sums for heads of 256 whatever the rows' length (a row of more than 192 tokens has 16 keys a
+// product otherwise, and 32 below). tokens: how many the portions hold in all, or more (0: not known), which decides the form alone.
+int holon_attention_prefill_one_order_bf16(const void* q, void* out, const void* pages, const int32_t* table,
+                                           int table_stride, const int32_t* slots, const int32_t* lens,
+                                           const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_query,
+                                           int max_len, int heads, int kv_heads, int head_dim, int page_size, float scale,
+                                           int window, const float* sink, int tokens, void* stream);
+int holon_attention_prefill_one_order_staged(int heads, int kv_heads, int n_rows, int max_query, int max_len, int page_size, int window,
+                                             int tokens);      // whether such heads of 256 go through LDS there
 int holon_attention_decode_sink_bf16(const void* q, void* out, const void* pages, const int32_t* table,
                                      int table_stride, const int32_t* slots, const int32_t* lens,
                                      const int32_t* query_start, const int32_t* row_ids, int n_rows, int max_len,

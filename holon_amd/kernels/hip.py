@@ -129,8 +129,8 @@ class HipKernels:
                                                   _P, _P, _I, _I, _I, _I, _P],
             "holon_attention_prefill_sink_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
                                                   _P, _P],
-            "holon_attention_prefill_from_cache_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
-                                                        _P, _P],
+            "holon_attention_prefill_one_order_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
+                                                       _P, _I, _P],
             "holon_attention_decode_sink_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I,
                                                  _P, _P, _I, _I, _I, _I, _P, _P],
             "holon_attention_prefill_mod_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _I,
@@ -186,7 +186,7 @@ class HipKernels:
         library, and the record of tiled weights by shape, are shared; what a product took is per engine
         (`plan.taken`). `settled` (set on the result, by whoever puts a model with an amplifying part together): steps of
         17 rows and more keep the forms whose order of sums such a model's logits have been compared in: no 256 x 256
-        tiles, no narrow products in one launch, heads of 256 straight from the cache."""
+        tiles, no narrow products in one launch, heads of 256 in the order of sums that short rows have."""
         other = copy.copy(self)
         other.plan = ProductPlan(products, pins)
         return other
@@ -800,10 +800,11 @@ class HipKernels:
             common = (q.data_ptr(), out.data_ptr(), pages.data_ptr(), table.data_ptr(), table.shape[1],
                       rows.slots.data_ptr(), rows.lens.data_ptr(), rows.query_start.data_ptr())
             if rows.n_chunk:
-                prefill = self.lib.holon_attention_prefill_from_cache_bf16 if self.settled else self.lib.holon_attention_prefill_sink_bf16
+                prefill, more = (self.lib.holon_attention_prefill_one_order_bf16, (t - rows.n_decode,)) if self.settled else \
+                    (self.lib.holon_attention_prefill_sink_bf16, ())
                 self._call(prefill, *common, rows.chunk_rows.data_ptr(), rows.n_chunk,
                            rows.max_chunk_query, rows.max_chunk_len, hq, hkv, d, page_size, float(scale), int(window),
-                           _ptr(sink), self._stream())
+                           _ptr(sink), *more, self._stream())
             if rows.n_decode:
                 span = rows.max_decode_len if not window else min(rows.max_decode_len, abs(window) + 31)
                 splits, per, waves = self.decode_splits(rows.n_decode * hkv * ((hq // hkv + 15) // 16), span, d)

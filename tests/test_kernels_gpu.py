@@ -1624,18 +1624,23 @@ def test_general_attention_of_short_rows(hip, dtype, heads, kv, d):
         assert H.rel_rms(got, want) < tight and H.rel_rms(hip.paged_attention(q, pages, table, rows(1), page, d ** -0.5, window), want) < tight
 
 
-@pytest.mark.parametrize("heads,kv,window", [(16, 1, 0), (16, 1, 200), (20, 1, 0), (8, 2, 0), (6, 2, -160), (34, 1, 96), (3, 3, 33)])
-def test_heads_of_256_staged_are_the_bits_of_short_portions(hip, heads, kv, window):
-    """Two prompts in one step, the longer one beyond the length from which stages go through LDS, behind cached tokens or not: every row
-    bit for bit what portions give that are too short for it, under sinks and windows of either kind, whatever later tokens' values are."""
+@pytest.mark.parametrize("heads,kv,window,steps", [
+    (16, 1, 0, ((0, (540, 530)), (37, (641, 17)), (560, (25, 300)))), (16, 1, 200, ((0, (1030, 97)), (37, (1100, 17)))), (20, 1, 0, ((0, (577, 97)),)),
+    (8, 2, 0, ((0, (577, 97)), (490, (130, 300)))), (6, 2, -160, ((0, (2700, 60)),)), (34, 1, 0, ((37, (641, 17)),)), (34, 1, 128, ((0, (1100, 17)),)),
+    (3, 3, 0, ((0, (641, 500)),)), (3, 3, 128, ((0, (5600, 40)),)), (3, 3, 513, ((600, (5600, 900)),))])
+def test_heads_of_256_staged_are_the_bits_of_short_portions(hip, heads, kv, window, steps):
+    """Two prompts in one step that takes its stages through LDS, behind cached tokens or not: every row bit for bit what portions give
+    that are too short for it, under sinks and windows of either kind, whatever later tokens' values are."""
     d, page, bf = 256, 16, torch.bfloat16
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                      # noqa: E731
     hip = hip.configured()
     hip.settled = True
     short = 16 // min(heads // kv, 16) * 15                                                # (15 tiles of 16 rows)
     sink = _randn(heads, dtype=torch.float32, seed=172)
-    for behind, lens in ((0, (533, 97)), (37, (641, 17)), (490, (27 * short // 16, 300))):
+    for behind, lens in steps:
         total = [behind + n for n in lens]
+        staged = hip.lib.holon_attention_prefill_one_order_staged
+        assert staged(heads, kv, 2, max(lens), max(total), page, window, sum(lens)) and not staged(heads, kv, 1, short, max(total), page, window, short)
         pages_each = -(-max(total) // page)
         pages = _randn(2 * pages_each, 2, kv, page * d, dtype=bf, seed=170)
         table = torch.arange(2 * pages_each, dtype=torch.int32, device="cuda").flip(0).view(2, pages_each).contiguous()
@@ -1655,6 +1660,21 @@ def test_heads_of_256_staged_are_the_bits_of_short_portions(hip, heads, kv, wind
                 want = hip.paged_attention(q[part].contiguous(), pages, table, one, page, d ** -0.5, window, sink=sink)
                 mine = slice(0, max(0, n - 16) if b == 0 and s + n == lens[0] else n)
                 assert torch.equal(got[part][mine], want[mine]) and torch.isfinite(want[mine]).all(), (behind, b, s)
+
+
+def test_which_portions_of_heads_of_256_go_through_lds(hip):
+    """Both sides of the lines: keys without a window, tiles for the SIMDs, windows too narrow, groups of more heads than a tile has rows, a long
+    portion among short ones, rows of more pages than LDS holds."""
+    staged = hip.lib.holon_attention_prefill_one_order_staged
+
+    def of(lens, heads, kv, window=0, behind=0, known=True, page=16):
+        return staged(heads, kv, len(lens), max(lens), behind + max(lens), page, window, sum(lens) if known else 0)
+    assert [of([n], 16, 1) for n in (511, 575, 576)] == [0, 0, 1] and [of([512] * n, 16, 1) for n in (2, 3)] == [0, 1]
+    assert [of([n], 16, 16, behind=600) for n in (240, 241)] == [0, 1]                      # (fewer than 16 tiles)
+    assert [of([n], 16, 1, w) for n, w in ((1024, 128), (1100, 128), (1100, 99), (1100, 512), (1024, 512))] == [0, 1, 0, 1, 0]
+    assert [of([n], 34, 1, 128) for n in (1024, 1100)] == [0, 1] and of([600], 34, 1, -512) == 1
+    assert of([600] + [40] * 7, 16, 1, 128) == 0 and of([600] + [40] * 7, 16, 1, 128, known=False) == 1 and of([1500] + [40] * 12, 32, 8, 128) == 0
+    assert of([64], 16, 1, behind=65536 - 64) == 1 and of([64], 16, 1, behind=65536 - 63) == 0 and of([64], 16, 1, behind=65536 - 63, page=32) == 1
 
 
 def test_few_row_products_whose_steps_leave_a_rest(hip):

@@ -186,9 +186,34 @@ def group_pays(m: int, n: int, k: int) -> bool:
     10.2 | 10.1 at 16 rows, 3,840 (8, 15) 13.9 | 13.8 at 16; 4,352 (8, 17) 16.0 | 14.9 at 16, 11,008 (8, 43) 25.6 | 20.4 and 35.5 | 25.8, 5,504 (4, 43) 20.2 | 15.0
     and 33.6 | 17.1, 1,440 (1, 45) 18.9 | 10.1 and 25.5 | 11.6; two of 8,192 x 8,192 (8, 32) faster together at any rows, 12,288 x 4,096 at 4 rows, but 42.8 | 41.6 at
     16; 9,216 x 4,096 27.0 | 25.5, 16,384 x 2,048 15.0 | 15.0 at 4 rows and 19.9 | 17.6 at 16, two of 24,576 x 2,048 35.0 | 33.7 and 45.5 | 35.8."""
-    most = 16 if n < 5120 else 8                            # waves a tile, as the kernels' `skinny_waves` has them
-    waves = next(w for w in (16, 8, 4, 2, 1) if w <= most and k % (32 * w) == 0)
-    return n <= (12288 if m <= 8 else 8192) and (waves == most or k // (32 * waves) <= 15)
+    waves = few_row_waves(n, k)
+    return n <= (12288 if m <= 8 else 8192) and (waves == (16 if n < 5120 else 8) or k // (32 * waves) <= 15)
+
+
+def few_row_waves(n: int, k: int) -> int:
+    """Waves a tile of 16 columns of a few-row product over an [n, k] weight, as the kernels' `skinny_waves` has them."""
+    return next(w for w in (16, 8, 4, 2, 1) if w <= (16 if n < 5120 else 8) and k % (32 * w) == 0)
+
+
+def beside_pays(m: int, hidden: int, n: int, k: int) -> bool:
+    """Whether a mixture's second product into `hidden` columns and a product of the same m rows over an [n, k] weight share a launch: a block of
+    eight waves for 16 of the mixture's columns, and one for one to eight tiles of the other's. It saves a launch, and where both leave units
+    idle a round of blocks; but blocks that do not fit beside one another wait, the other product's for all of its K. So wherever the blocks of
+    both take fewer rounds of 256 together (0.66 to 0.93 of the time apart), or a wave's loads come in full sets to their end (K a
+    multiple of 4,096); else the narrower the mixture and the more rows, the longer a K may be. Over 2,500 steps (2,048 to 5,120 columns, 8 to
+    128 experts, 1 to 16 rows) nothing so chosen took over 2 % longer than apart, of all of them 5 % did, up to 7 %. Measured, us, together | apart, 8
+    experts unless noted: 2,048 columns beside 2,048 x 2,048 10.1 | 13.9 at one row and 42.5 | 48.1 at 16 (128 experts), 12,288 x 2,048
+    18.2 | 22.3, 2,560 x 5,120 19.2 | 18.0 at two; 2,304 beside 512 x 2,048 6.5 | 10.1 and 3,072 x 1,024 10.4 | 9.9 at one; 2,560 (64 experts) beside
+    2,048 x 6,144 17.5 | 17.3 at one and 30.3 | 38.2 at eight; 3,072 beside 2,048 x 2,816 13.6 | 18.0 at four; 3,584 beside 2,048 x 1,024 15.8 | 14.9 at
+    three; 4,096 (64 experts) beside 4,096 x 2,048 14.1 | 14.1 at one and 52.8 | 51.0 at 16, beside 4,096 x 4,096 16.1 | 17.5 and 54.8 | 56.7."""
+    mixture, product = hidden // 16, -(-(n // 16) // (8 // min(few_row_waves(n, k), 8)))
+    if -(-(mixture + product) // 256) < -(-mixture // 256) + -(-product // 256) or k % 4096 == 0:
+        return True
+    if hidden <= 2048:
+        return k < 4096 or m > 3
+    if hidden <= 2560:
+        return (m > 1 or k >= 1408) and (k < 4096 or m >= 8)
+    return hidden < 4096 and m > 1 and mixture + product <= 336 and 1024 < k < 4096
 
 
 def _served(p: Product) -> bool:
@@ -220,9 +245,11 @@ def _linear_group_hip(launch, products: list[Product | Routing | ExpertsDown]) -
         for group in (which[at: at + MOST] for at in range(0, len(which), MOST)):
             route = routes[rows].pop(0) if routes.get(rows) else None
             if len(group) == 1 and route is None:
-                if downs.get(rows):                       # a mixture's experts beside it (several products fill the chip by themselves)
-                    at = downs[rows].pop(0)
-                    out[group[0]], out[at] = _beside(launch_beside, products[group[0]], products[at])
+                p = products[group[0]]
+                at = next((d for d in downs.get(rows, ()) if beside_pays(rows, products[d].tiled.shape[0], *p.linear.weight.shape)), None)
+                if at is not None:                        # a mixture's experts beside it (several products fill the chip by themselves)
+                    downs[rows].remove(at)
+                    out[group[0]], out[at] = _beside(launch_beside, p, products[at])
                 continue
             items = []
             for i in group:

@@ -2238,9 +2238,10 @@ def test_routers_of_many_rows_are_those_of_few(hip, dtype):
 
 @pytest.mark.parametrize("rows", [1, 6, 16])
 @pytest.mark.parametrize("hidden,experts,ff,shared", [(256, 8, 32, 0), (2048, 8, 256, 512), (512, 70, 544, 32), (288, 5, 96, 0)])
-def test_experts_beside_a_product_are_both(hip, rows, hidden, experts, ff, shared):
+def test_experts_beside_a_product_are_both(hip, rows, hidden, experts, ff, shared, monkeypatch):
     """A mixture's second product and another one in one launch, bit for bit what either is by itself: tiles of 16, 8, 4, 2 and 1 waves
-    that do and do not fill a block, every output form; a product that joins no launch, and none at all."""
+    that do and do not fill a block, every output form; a product that joins no launch, one beside which it does not pay, and none at all."""
+    from holon_amd.parts import products as pr
     from holon_amd.parts.products import ExpertsDown, Product
     bf, cols, gen = torch.bfloat16, experts * ff + shared, torch.Generator(device="cuda").manual_seed(rows)
     down_t = hip.tile_weight(_randn(hidden, cols, dtype=bf, seed=230, scale=ff ** -0.5))
@@ -2266,3 +2267,8 @@ def test_experts_beside_a_product_are_both(hip, rows, hidden, experts, ff, share
             got = dict(zip(map(id, products), hip.linear_group(products)))
             want = p.alone()
             assert got[id(p)].dtype == want.dtype and torch.equal(got[id(p)], want) and torch.equal(got[id(down)], whole), (n, kk)
+        with monkeypatch.context() as m:
+            m.setattr(pr, "beside_pays", lambda *a: False)
+            m.setattr(pr, "_beside", lambda *a: pytest.fail("a launch that does not pay"))
+            apart = hip.linear_group([p, down])
+        assert torch.equal(apart[0], want) and torch.equal(apart[1], whole), (n, kk)

@@ -767,3 +767,16 @@ def test_products_join_a_launch_of_several_where_that_pays():
     assert all(group_pays(m, n, k) for m in (1, 16) for n, k in ((64, 256), (2048, 8192), (512, 480), (4096, 2816), (5104, 3840), (8192, 8192), (8192, 3840)))
     assert not any(group_pays(m, n, k) for m in (1, 16) for n, k in ((512, 512 + 32), (2048, 4352), (2048, 11008), (4096, 5504), (8192, 5504), (512, 1440)))
     assert [group_pays(m, n, 2048) for m, n in ((8, 12288), (8, 12304), (9, 8192), (9, 8208))] == [True, False, True, False]
+
+
+def test_which_products_a_mixture_shares_a_launch_with():
+    """`beside_pays` on both sides of its lines: rounds of blocks that are saved, full sets of loads, widths of the mixture, rows, long and short K."""
+    from holon_amd.parts.products import beside_pays
+    assert all(beside_pays(m, 2048, n, k) for m in (1, 16) for n, k in ((2048, 2048), (512, 256), (4096, 4096), (12288, 2048), (8192, 8192), (2048, 6144)))
+    assert [beside_pays(m, 2048, 2560, 5120) for m in (1, 3, 4)] == [False, False, True]                                    # (288 blocks)
+    assert [beside_pays(m, 2560, 2048, k) for m, k in ((1, 1024), (2, 1024), (1, 1408), (1, 6144), (7, 6144), (8, 6144))] == [False, True, True, False, False, True]
+    assert beside_pays(1, 2304, 512, 2048) and not beside_pays(1, 2304, 3072, 1024)
+    assert [beside_pays(m, 3072, 2048, k) for m, k in ((1, 2048), (2, 2048), (2, 1024), (16, 6144), (1, 4096))] == [False, True, False, False, True]
+    assert not beside_pays(2, 3072, 4096, 2048) and beside_pays(2, 3584, 1024, 2048)
+    assert [beside_pays(m, 4096, n, k) for m in (1, 16) for n, k in ((2048, 2048), (4096, 4096), (2048, 6144), (4096, 2048))] == [False, True, False, False] * 2
+    assert beside_pays(1, 5120, 2048, 2048)                                                                                 # (320 and 128: two rounds, not three)

@@ -340,13 +340,6 @@ register_kernel(KernelOp("linear_relu2", linear_relu2_plain, "holon_gemm_skinny_
                          _linear_relu2_hip))
 
 
-def moe_few_plain(x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight=False):
-    """The experts' two products and the activation between them for steps of few rows, reading the chosen experts' weights
-    alone, with the roundings of `linear`, `moe_gate` (`gated`) or `moe_relu2`, and `linear`; None where they are not served
-    (the caller then composes the three). The plain form never does."""
-    return None
-
-
 def moe_few_serves(rows: int, hidden: int, experts: int, ff: int, shared: int) -> bool:
     """What the library's `holon_moe_few_supported` answers."""
     return 1 <= rows <= 16 and hidden % 32 == 0 and experts <= 1024 and ff % 32 == 0 and shared % 32 == 0
@@ -376,7 +369,7 @@ def _moe_up_few_hip(launch, x, weights, up_tiled, down_tiled, experts, ff, share
           and tuple(weights.shape) == (t, experts + int(bool(shared_weight)))
           and all(w.is_contiguous() and w.dtype == x.dtype for w in (up_tiled, down_tiled))
           and tuple(up_tiled.shape) == ((2 if gated else 1) * cols, hidden) and tuple(down_tiled.shape) == (hidden, cols),
-          f"moe_few: rows {tuple(x.shape)}, weights {tuple(weights.shape)}, projections {tuple(up_tiled.shape)} and "
+          f"moe_up_few: rows {tuple(x.shape)}, weights {tuple(weights.shape)}, projections {tuple(up_tiled.shape)} and "
           f"{tuple(down_tiled.shape)} for {experts} experts of {ff} and {shared} shared columns")
     act = torch.empty((t, cols), dtype=x.dtype, device=x.device)
     launch(x.data_ptr(), up_tiled.data_ptr(), act.data_ptr(), t, hidden, experts, ff, shared, int(bool(gated)), weights.data_ptr(),
@@ -399,26 +392,23 @@ def _moe_down_few_hip(launch, act, weights, down_tiled, experts, ff, shared):
     return y
 
 
-def _moe_few_hip(launch, x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight=False):
-    act = _moe_up_few_hip(launch[0], x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight)
-    return None if act is None else _moe_down_few_hip(launch[1], act, weights, down_tiled, experts, ff, shared)
-
-
 def moe_up_few_plain(x, weights, up_tiled, down_tiled, experts, ff, shared, gated, shared_weight=False):
-    """The first product of `moe_few` and its activation, or None."""
+    """The experts' first product and the activation behind it for steps of few rows, reading the chosen experts' weights alone, with the
+    roundings of `linear` and `moe_gate` (`gated`) or `moe_relu2`: [T, experts ff + shared], columns of experts that no row chose left as
+    the memory was; None where the two products are not served (the caller then composes them with those). The plain form never does."""
     return None
 
 
 def moe_down_few_plain(act, weights, down_tiled, experts, ff, shared):
-    """The second product of `moe_few`, over what `moe_up_few` left (the plain form of which leaves nothing)."""
-    raise NotImplementedError("moe_down_few: there is no plain form of a tiled projection")
+    """The second product over what `moe_up_few` left, reading the chosen experts' weights alone, with the rounding of `linear`."""
+    n, k = down_tiled.shape
+    down = down_tiled.view(n // 16, k // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(n, k)          # (16 rows of 32 columns lie together)
+    used = torch.cat(((weights[:, :experts] != 0).repeat_interleave(ff, 1), weights.new_ones(act.shape[0], shared).bool()), 1)
+    return (torch.where(used, act, 0).float() @ down.float().T).to(act.dtype)
 
 
-_MOE_UP_FEW, _MOE_DOWN_FEW = [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I], [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I]
-register_kernel(KernelOp("moe_few", moe_few_plain, ("holon_moe_up_few_bf16", "holon_moe_down_few_bf16"), (_MOE_UP_FEW, _MOE_DOWN_FEW),
-                         _moe_few_hip))
-register_kernel(KernelOp("moe_up_few", moe_up_few_plain, "holon_moe_up_few_bf16", _MOE_UP_FEW, _moe_up_few_hip))
-register_kernel(KernelOp("moe_down_few", moe_down_few_plain, "holon_moe_down_few_bf16", _MOE_DOWN_FEW, _moe_down_few_hip))
+register_kernel(KernelOp("moe_up_few", moe_up_few_plain, "holon_moe_up_few_bf16", [_P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _I, _I], _moe_up_few_hip))
+register_kernel(KernelOp("moe_down_few", moe_down_few_plain, "holon_moe_down_few_bf16", [_P, _P, _P, _I, _I, _I, _I, _I, _P, _I], _moe_down_few_hip))
 
 
 def moe_rows_plain(x, weights, up, down, experts, top, ff, shared, gated, shared_weight=False):
@@ -615,7 +605,7 @@ class MoE(Part):
     is weighted by s * `scale`. All experts' gate and up projections are one product and all down projections
     another: the activations of experts a token did not choose are set to 0 in between (`moe_gate`), so the second
     product adds up exactly the chosen experts' weighted outputs, and the shared expert's columns ride in the same two
-    products. Steps of few rows take the same two products over the chosen experts' columns alone (`moe_few`), steps of many
+    products. Steps of few rows take the same two products over the chosen experts' columns alone (`moe_up_few`, `moe_down_few`), steps of many
     rows each expert's over the rows that chose it (`moe_rows`), where that is done sooner; in float32 every step does the latter
     (`moe_f32`) or none, by the mixture's sizes. Steps of as many rows launch the same kernels whatever was chosen."""
 

@@ -1207,6 +1207,13 @@ def test_nothing_is_collected_while_a_graph_is_recorded():
     assert gc.isenabled()
 
 
+def _moe_few(hip, x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=False):
+    """The two products of a mixture's step of few rows as a model runs them; None where they are not served."""
+    from holon_amd.parts.products import ExpertsDown
+    act = hip.moe_up_few(x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=shared_weight)
+    return None if act is None else ExpertsDown(hip, act, weights, down_t, experts, ff, shared).alone()
+
+
 @pytest.mark.parametrize("hidden,experts,ff,shared,top,gated,own_gate", [
     (256, 8, 32, 0, 1, True, False), (384, 8, 160, 64, 2, True, True), (512, 70, 544, 32, 6, False, False),
     (288, 5, 96, 0, 2, False, False), (2048, 8, 2048, 2048, 2, True, True)])
@@ -1230,7 +1237,7 @@ def test_chosen_experts_alone(hip, hidden, experts, ff, shared, top, gated, own_
         weights = weights.cuda()
         garbage = torch.full((m, cols), float("nan"), dtype=bf, device="cuda")
         del garbage                            # what no row chose must not be read
-        got = hip.moe_few(x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=own_gate)
+        got = _moe_few(hip, x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=own_gate)
         between = hip.moe_gate if gated else hip.moe_relu2
         whole = hip.linear(between(hip.linear(x, up_w, tiled=up_t), weights, ff, shared, shared_weight=own_gate), down_w,
                            tiled=down_t)
@@ -1243,10 +1250,10 @@ def test_chosen_experts_alone(hip, hidden, experts, ff, shared, top, gated, own_
         apart = H.rel_rms(got, want) if want.any() else got.abs().max().item()
         assert apart < 5 * 2.0 ** -9, (m, apart)
         for row in (0, m // 2, m - 1):
-            alone = hip.moe_few(x[row: row + 1].contiguous(), weights[row: row + 1].contiguous(), up_t, down_t, experts, ff, shared,
-                                gated, shared_weight=own_gate)
+            alone = _moe_few(hip, x[row: row + 1].contiguous(), weights[row: row + 1].contiguous(), up_t, down_t, experts, ff, shared,
+                             gated, shared_weight=own_gate)
             assert torch.equal(alone[0], got[row]), (m, row)
-    assert hip.moe_few(_randn(17, hidden, dtype=bf), weights, up_t, down_t, experts, ff, shared, gated) is None
+    assert _moe_few(hip, _randn(17, hidden, dtype=bf), weights, up_t, down_t, experts, ff, shared, gated) is None
 
 
 @pytest.mark.parametrize("hidden,experts,ff,shared,top,gated,own_gate", [
@@ -1442,7 +1449,7 @@ def test_a_shared_expert_whose_gate_is_shut(hip, gated, shared):
         weights = weights.cuda()
         garbage = torch.full((m, cols), float("nan"), dtype=bf, device="cuda")
         del garbage                            # what the next allocation of this size finds
-        got = hip.moe_few(x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=True)
+        got = _moe_few(hip, x, weights, up_t, down_t, experts, ff, shared, gated, shared_weight=True)
         whole = hip.linear(between(hip.linear(x, up_w, tiled=up_t), weights, ff, shared, shared_weight=True), down_w,
                            tiled=down_t)
         assert torch.equal(got, whole), (m, open_rows)
@@ -2241,6 +2248,7 @@ def test_routers_of_many_rows_are_those_of_few(hip, dtype):
 def test_experts_beside_a_product_are_both(hip, rows, hidden, experts, ff, shared, monkeypatch):
     """A mixture's second product and another one in one launch, bit for bit what either is by itself: tiles of 16, 8, 4, 2 and 1 waves
     that do and do not fill a block, every output form; a product that joins no launch, one beside which it does not pay, and none at all."""
+    from holon_amd.kernels.registry import kernel_op
     from holon_amd.parts import products as pr
     from holon_amd.parts.products import ExpertsDown, Product
     bf, cols, gen = torch.bfloat16, experts * ff + shared, torch.Generator(device="cuda").manual_seed(rows)
@@ -2251,6 +2259,8 @@ def test_experts_beside_a_product_are_both(hip, rows, hidden, experts, ff, share
     down = ExpertsDown(hip, act, weights, down_t, experts, ff, shared)
     whole = hip.linear(act, _randn(hidden, cols, dtype=bf, seed=230, scale=ff ** -0.5), tiled=down_t)
     assert torch.equal(down.alone(), whole) and torch.equal(hip.linear_group([down])[0], whole)
+    plain = kernel_op("moe_down_few").plain(act, weights, down_t, experts, ff, shared)
+    assert H.rel_rms(whole, plain) < 2.0 ** -8 if plain.any() else not whole.any()
 
     class Weights:                                # what a projection holds
         folded, kernels = None, hip

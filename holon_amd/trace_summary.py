@@ -60,12 +60,13 @@ def dispatches(path: str) -> list[tuple]:
 
 CLASSES = (("attention", ("attn_", "sigmoid_attention", "softmax_attention", "latent_attention", "latent_prefill", "latent_decode",
                           "latent_merge", "sigmoid_merge", "attention_generic", "attention_f64")),
-           ("matrix products", ("gemm_", "Cijk_", "Custom_Cijk_", "hipBLASLt", "head_linear", "moe_up_few", "moe_down_few")),
+           ("matrix products", ("gemm_", "Cijk_", "Custom_Cijk_", "hipBLASLt", "head_linear", "moe_up_", "moe_down_")),
            ("recurrent scans", ("memory_scan", "delta_scan", "delta_blocks", "delta_chain", "delta_walk", "mlstm_scan", "mlstm_chunk", "mlstm_pieces", "mlstm_gates", "ssd_", "gla_")),
            ("elementwise", ("rmsnorm", "gated_mul", "qk_norm_rope", "v_write", "kv_write", "embedding", "sum_parts",
                             "row_sumsq", "scatter_rows", "stream_norm", "dyt_stream", "widen_", "narrow_", "pair_rows", "softcap", "causal_conv",
                             "head_prepare", "delta_prepare", "gated_out", "shift_mix", "shift_keep", "decay_lora", "stream_rms", "latent_rope_prepare", "gated_parts_norm",
-                            "moe_gate", "moe_router", "moe_relu2", "relu2", "keep_last_token")),
+                            "moe_gate", "moe_route", "moe_relu2", "moe_lists", "moe_add_parts", "relu2", "polynorm", "keep_last_token", "scale_rows",
+                            "latent_prepare", "whole_norm_prepare", "head_gate", "diff_combine", "add_bias", "tile_weight")),
            ("sampling", ("argmax", "sample_kernel", "store_tokens", "logprobs")))
 
 

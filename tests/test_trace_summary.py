@@ -54,3 +54,16 @@ def test_a_step_by_class_of_kernel(tmp_path, capsys):
     assert table == {"matrix products": 60.0, "attention": 40.0, "elementwise": 9.0, "sampling": 6.0,
                      "other (copies, library elementwise)": 3.0, "between kernels": 3.5}
     assert trace_summary.kernel_class("_ZN12_GLOBAL__N_116gemm_rows_kernelILi4E") == "matrix products"
+
+
+def test_every_kernel_of_the_library_has_its_class():
+    """By the names in the sources: none is counted among copies and a library's elementwise kernels."""
+    import pathlib
+    import re
+    csrc, names = pathlib.Path(trace_summary.__file__).parent / "csrc", set()
+    for source in [*csrc.glob("*.hip"), *csrc.glob("*.h")]:
+        names.update(re.findall(r"__global__ void(?:\s+__launch_bounds__\((?:[^()]|\([^()]*\))*\))?\s+(\w+)\(", source.read_text()))
+    assert len(names) > 100 and not [n for n in names if trace_summary.kernel_class(n).startswith("other")]
+    products = ("moe_down_beside_kernel", "moe_down_few_kernel", "moe_up_rows_kernel", "moe_down_rows_f32_kernel")
+    assert {trace_summary.kernel_class(n) for n in products} == {"matrix products"}
+    assert trace_summary.kernel_class("moe_router_rows_kernel") == trace_summary.kernel_class("moe_add_parts_kernel") == "elementwise"

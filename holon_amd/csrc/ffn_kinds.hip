@@ -197,8 +197,8 @@ __global__ void __launch_bounds__(moe_router::BLOCK_WAVES * WAVE) moe_router_few
 
 // The router of up to 64 experts for many rows, both kinds: TOK tokens a wave, so that TOK rows share what is read of the router (128 KB a
 // token at 8 experts of 4,096: more than all else a step of many rows reads here), E of its rows at a time, the next loads under way
-// while the last are multiplied. Logits are added up and the choice is made as moe_router.h has them. Rows of 4,096 over 8 experts:
-// 4,096 of them 21 us, 2,154 20, a block a token 76 and 41; 1,800 of 2,048 over 9 (PARTS 4) 16, a block a token 22.
+// while the last are multiplied. Logits are added up and the choice is made as moe_router.h has them. Rows of 4,096 over 8 experts
+// back to back: 4,096 of them 16.6 us (PARTS 4 19.7), a block a token 56 and 38; 2,047 of 2,048 7.6 and 8.7, a block a token 14.1 and 16.4.
 template <typename T, int PARTS, int TOK, int E>
 __global__ void __launch_bounds__(256) moe_router_rows_kernel(const T* __restrict__ x, const float* __restrict__ router,
                                                               const float* __restrict__ bias, float* __restrict__ weights, int64_t rows,
@@ -537,7 +537,13 @@ extern "C" int holon_moe_route(const float* logits, const float* correction, flo
 }
 
 // Up to 64 experts: a block of 16 waves a token up to 256 rows, which a block of four a token would leave idle units; from there on rows that
-// share what they read of the router, by the wave, as many as leave a block for every unit.
+// share what they read of the router, by the wave: one token a wave up to 1,023 rows, two up to 2,047, four beyond (PARTS 4: half as many experts at a
+// time, for its registers). A block has four waves, so just above either line half of the units have no block, 257 rows have 65 blocks in all, and yet
+// nothing takes longer than a block a token did (whose blocks read the router 4 to 16 times as often): 128 sizes of 257 to 8,192 rows of
+// 2,048 and 4,096 over 8 to 64 experts, both kinds, 0.23 to 1.02 of its time. In us, against a block a token, rows of 4,096, PARTS 1 and 4: over 8
+// experts 257 rows 7.4 / 8.9 and 8.0 / 9.2, 1,023 8.2 / 16.5 and 8.7 / 12.1, 1,024 9.5 / 16.4 and 10.6 / 12.2, 2,048 14.8 / 27.5 and 17.9 / 23.4; over 64
+// 257 rows 41 / 41 and 45 / 50, 1,023 43 / 77 and 46 / 58, 1,024 51 / 76 and 59 / 58, 2,048 82 / 139 and 110 / 121, 8,192 135 / 515 and 188 / 393 (back
+// to back, the router in the cache).
 static bool router_waves_serve(int64_t rows, int width, int experts, const float* router) {
   return experts <= WAVE && (rows <= 256 || (width % 4 == 0 && (uintptr_t)router % 16 == 0 && rows <= 0x7fffffff));
 }

@@ -117,9 +117,9 @@ __device__ __forceinline__ void half_sums(f32x4_t& acc, const float* wr, const f
 // other: several blocks share a unit, so that one's first loads and its stores lie under the others' products; that is the better
 // one where there are tiles for it, the more the shorter K. Either ends at K (what lies behind it would add zeros).
 // Whole chunks of K go from memory straight into LDS: no register holds them on their way, which leaves room for five blocks of 64 x 64 a
-// unit instead of four, no instruction writes LDS, and a chunk has one barrier. Against the form that passes registers, us back to back:
-// 825 x 16384 x 2048 539 -> 476 (360 at the rate of a large product; behind the kernels of a model 553 and 551), 825 x 2048 x 8192
-// 303 -> 278, 2048 x 2048 x 2048 162 -> 149, 2048 x 9248 x 256 111 -> 95. What is left there is mostly the last round of blocks; 128 x 64 a
+// unit instead of four, no instruction writes LDS, and a chunk has one barrier. Against the form that passes registers, us, weights from memory:
+// 825 x 16384 x 2048 550 -> 493 (360 at the rate of a large product; in a model's trace 553 -> 526 to 562, for a reason not found), 825 x 2048 x 8192
+// 304 -> 279, 2048 x 2048 x 2048 164 -> 152, 2048 x 9248 x 256 115 -> 102. What is left there is mostly the last round of blocks; 128 x 64 a
 // block (three blocks a unit) takes 6 to 17 % longer, and an XCD a run of columns of its own gained nothing that a model shows.
 // Every thread of the block comes here. `xr`, `wr`: the rows of either operand that the thread stages, row tid / 8 of 32 and those 32
 // further on (tid: the thread within its quarter). emit(sums, row, column): four results of a row, once each, behind the block's last

@@ -164,17 +164,18 @@ __global__ void __launch_bounds__(256) gemm_f32_in_order_kernel(const float* __r
 // 17 to 2,048, weights from memory (1.6 GB of them in turn: back to back over three weights that stay in the last-level cache, staged forms
 // look up to a third faster than behind a model's other products), in us: a start, and so much for every round of one block a CU, linear in K.
 // Tiles straight from memory add a part of K to that; of staged ones a block that has its unit to itself takes longer than its share of a full
-// one, `start_k` a k. The choice is 0.4 % from the best form on average and 14 % at most (1.4 us). In us, best and others: 2048 x 2048 takes
-// 1 x 1 tiles up to 32 rows (10; with a 64 x 64 tile a block and no split of K it took 118), 1 x 2 at 64 (16), 2 x 4 at 145 (34; staged 39 to
-// 48), quarters side by side from 300 rows (39; one after the other 48), blocks of 32 rows at 700 (65; of 64 rows 76, whose second round is
-// mostly empty); 2048 x 9248 at 704 rows blocks of 32 (274; of 64 312); 16384 x 2048 1 x 1 tiles up to 16 rows (5.0 TB/s at one row), blocks of
-// 32 at 150 (117; of 64 122), of 64 at 825 (493; of 32 596); 9248 x 256 at 2,048 rows of 64 one after the other (102; side by side 143).
+// one, `start_k` a k. The choice is 0.3 % from the best form on average and 9 % at most, 0.1 and 5 % of those above 60 us; over 160 products
+// that the fit has not seen 0.3 and 9 %. In us, best and others: 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10; with a 64 x 64 tile a
+// block and no split of K it took 118), 1 x 2 at 64 (16), 2 x 4 at 145 (34; staged 39 to 48), quarters side by side from 300 rows (39; one
+// after the other 48), blocks of 32 rows at 700 (65; of 64 rows 76, whose second round is mostly empty); 2048 x 9248 at 704 rows blocks of
+// 32 (274; of 64 312); 16384 x 2048 1 x 1 tiles up to 16 rows (5.0 TB/s at one row), blocks of 32 at 150 (117; of 64 122), of 64 at 825
+// (493; of 32 596); 9248 x 256 at 2,048 rows of 64 one after the other (102; side by side 143).
 struct Form { int mt, nt; float start, start_k, round, round_k; };
 enum { SIDE_BY_SIDE = 4, IN_TURN = 5, IN_TURN_32 = 6, KINDS = 7 };
-constexpr Form FORMS[KINDS] = {{1, 1, 2.03f, 6.67e-4f, 0.425f, 3.27e-3f}, {1, 2, 2.13f, 8.34e-4f, 0.613f, 5.15e-3f},
-                               {2, 2, 2.34f, 1.28e-3f, 0.911f, 7.33e-3f}, {2, 4, 1.0f, 1.28e-3f, 3.15f, 1.36e-2f},
-                               {4, 4, 1.0f, 6.47e-3f, 3.33f, 1.69e-2f},   {4, 4, 3.17f, 2.16e-2f, 0.634f, 1.81e-2f},
-                               {2, 4, 1.73f, 1.98e-2f, 0.694f, 1.03e-2f}};
+constexpr Form FORMS[KINDS] = {{1, 1, 1.7f, 6.67e-4f, 0.425f, 3.27e-3f},  {1, 2, 2.06f, 7.5e-4f, 0.613f, 5.89e-3f},
+                               {2, 2, 2.34f, 1.28e-3f, 0.911f, 7.33e-3f}, {2, 4, 1.0f, 1.24e-3f, 3.19f, 1.36e-2f},
+                               {4, 4, 0.872f, 6.47e-3f, 3.39f, 1.69e-2f}, {4, 4, 3.63f, 2.16e-2f, 0.607f, 1.72e-2f},
+                               {2, 4, 1.73f, 1.98e-2f, 0.657f, 1.03e-2f}};
 // Operands that cannot be copied straight into LDS (K off a multiple of 32, or not on 16 bytes) pass registers, in tiles of 64 x 64: a fit of
 // their own (1,149 products), each time the sum of all its terms; within 1 % of the best on average over the 400 above, too.
 constexpr Form BY_REGISTERS[KINDS - 1] = {{1, 1, 2.6f, 2e-4f, 0.43f, 3.25e-3f}, {1, 2, 2.5f, 2e-4f, 0.63f, 5.0e-3f},

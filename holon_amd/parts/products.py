@@ -190,11 +190,13 @@ def group_pays(m: int, n: int, k: int) -> bool:
     return n <= (12288 if m <= 8 else 8192) and (waves == (16 if n < 5120 else 8) or k // (32 * waves) <= 15)
 
 
+@functools.lru_cache(maxsize=1024)
 def few_row_waves(n: int, k: int) -> int:
     """Waves a tile of 16 columns of a few-row product over an [n, k] weight, as the kernels' `skinny_waves` has them."""
     return next(w for w in (16, 8, 4, 2, 1) if w <= (16 if n < 5120 else 8) and k % (32 * w) == 0)
 
 
+@functools.lru_cache(maxsize=1024)
 def beside_pays(m: int, hidden: int, n: int, k: int) -> bool:
     """Whether a mixture's second product into `hidden` columns and a product of the same m rows over an [n, k] weight share a launch: a block of
     eight waves for 16 of the mixture's columns, and one for one to eight tiles of the other's. It saves a launch, and where both leave units

@@ -494,7 +494,9 @@ template <int D, int NT, int WAVES = 4>
 __global__ void __launch_bounds__(WAVES * WAVE) attn_prefill_lds_kernel(AttnArgs a) {
   constexpr int KP = D + 8;    // pitch of a key row in LDS (elements)
   constexpr int VP = 40;       // pitch of a value row: 32 keys + 8
-  constexpr int EARLY = D == 256 ? 8 : 0;      // values asked of LDS in front of the scores, as many as registers hold (137 us and 140)
+  constexpr bool ONE_ORDER = D == 256;         // the bits of the kernel that reads the cache
+  static_assert(!ONE_ORDER || NT == 1, "a tile a wave");
+  constexpr int EARLY = ONE_ORDER ? 8 : 0;     // values asked of LDS in front of the scores, as many as registers hold (137 us and 140)
   __shared__ __attribute__((aligned(16))) bf16_t k_lds[2][32 * KP];
   __shared__ __attribute__((aligned(16))) bf16_t v_lds[2][D * VP];
   constexpr int PG = 4096;     // the row's first block-table entries, kept in LDS: page lookups then do not queue
@@ -614,12 +616,14 @@ __global__ void __launch_bounds__(WAVES * WAVE) attn_prefill_lds_kernel(AttnArgs
         *reinterpret_cast<bf16x8_t*>(&v_lds[buf][v_dst[i]]) = r.v[i];
       }
     };
+    // stages that none of the tile's rows sees (those before its window: left out in the one order alone, where they cost more than the question)
+    const auto outside = [&](int t, int kb) { return (ONE_ORDER && kb < tile_from[t]) || kb > tile_last[t]; };
     // One stage: LDS buffer `buf` holds the keys kb .. kb+31. `next` holds stage kb+32, which goes to the other
     // buffer after the products and is then refilled with stage kb+96 (`other` holds kb+64 meanwhile).
     auto stage = [&](int kb, int buf, Regs& next) {
       bool any = false;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) any = any || (kb >= tile_from[t] && kb <= tile_last[t]);
+      for (int t = 0; t < NT; ++t) any = any || !outside(t, kb);
       if (any) {
         bf16x8_t kf0[D / 32], kf1[D / 32];
 #pragma unroll
@@ -636,7 +640,7 @@ __global__ void __launch_bounds__(WAVES * WAVE) attn_prefill_lds_kernel(AttnArgs
         bf16x8_t pb[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          if (kb < tile_from[t] || kb > tile_last[t]) continue;
+          if (outside(t, kb)) continue;
           f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int ks = 0; ks < D / 32; ++ks) {
@@ -651,11 +655,11 @@ __global__ void __launch_bounds__(WAVES * WAVE) attn_prefill_lds_kernel(AttnArgs
 #pragma unroll
         for (int ds = 0; ds < D / 16; ++ds) {
           if (ds >= EARLY) read_value(ds);
-          const int last = NT == 1 ? tile_last[0] : key_hi;          // (what lies behind the tile's tokens may be anything)
+          const int last = ONE_ORDER ? tile_last[0] : key_hi;        // (what lies behind the tile's tokens may be anything)
           if (kb + 31 > last) zero_after(vf[ds], kb + 8 * g, last);
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
-            if (kb < tile_from[t] || kb > tile_last[t]) continue;
+            if (outside(t, kb)) continue;
             o[t][ds] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[ds], pb[t], o[t][ds], 0, 0, 0);
           }
         }

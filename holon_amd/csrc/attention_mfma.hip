@@ -2004,8 +2004,8 @@ struct Staged256 {
 // 546 / 430; 16 over 16, 512 tokens 42 / 45, 600 49 / 47, eight of 512 156 / 88). Under a window a wave's walk is short, so only where the tiles
 // outnumber the SIMDs and the window is 512 keys and more, or 100 and more with tiles for every group of heads and a quarter of the launched
 // blocks at work (16 over one within 128: 1,024 tokens 20 / 24, 2,048 38 / 26; 32 over 8 within 128, 1,500 tokens beside twelve of 40 80 / 108,
-// four of 700 to 1,500 78 / 63 of 16 over one; within 512, 1,500 beside twelve of 40 84 / 55). Over 1,110 steps nothing was longer than
-// straight from the cache by more than 5 %; staged from 512 keys on whatever else, half of them were, up to 1.9 times.
+// four of 700 to 1,500 78 / 63 of 16 over one; within 512, 1,500 beside twelve of 40 84 / 55). Over 1,245 steps nothing was longer than
+// straight from the cache by more than 5 %; staged from 512 keys on whatever else, 549 of them were by more than 2 %, up to 1.9 times.
 static Staged256 stages_256(int heads, int kv_heads, int n_rows, int max_query, int max_len, int window, int tokens) {
   const TileMap tm = tile_map(heads / kv_heads);
   const int64_t most = (int64_t)n_rows * max_query, positions = tokens > 0 && tokens < most ? tokens : most;

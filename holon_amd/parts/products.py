@@ -201,9 +201,9 @@ def beside_pays(m: int, hidden: int, n: int, k: int) -> bool:
     """Whether a mixture's second product into `hidden` columns and a product of the same m rows over an [n, k] weight share a launch: a block of
     eight waves for 16 of the mixture's columns, and one for one to eight tiles of the other's. It saves a launch, and where both leave units
     idle a round of blocks; but blocks that do not fit beside one another wait, the other product's for all of its K. So wherever the blocks of
-    both take fewer rounds of 256 together (0.66 to 0.93 of the time apart), or a wave's loads come in full sets to their end (K a
+    both take fewer rounds of 256 together (0.58 to 0.93 of the time apart), or a wave's loads come in full sets to their end (K a
     multiple of 4,096); else the narrower the mixture and the more rows, the longer a K may be. Over 2,500 steps (2,048 to 5,120 columns, 8 to
-    128 experts, 1 to 16 rows) nothing so chosen took over 2 % longer than apart, of all of them 5 % did, up to 7 %. Measured, us, together | apart, 8
+    128 experts, 1 to 16 rows) nothing so chosen took over 2 % longer than apart, of all of them 9 % did, up to 10 %. Measured, us, together | apart, 8
     experts unless noted: 2,048 columns beside 2,048 x 2,048 10.1 | 13.9 at one row and 42.5 | 48.1 at 16 (128 experts), 12,288 x 2,048
     18.2 | 22.3, 2,560 x 5,120 19.2 | 18.0 at two; 2,304 beside 512 x 2,048 6.5 | 10.1 and 3,072 x 1,024 10.4 | 9.9 at one; 2,560 (64 experts) beside
     2,048 x 6,144 17.5 | 17.3 at one and 30.3 | 38.2 at eight; 3,072 beside 2,048 x 2,816 13.6 | 18.0 at four; 3,584 beside 2,048 x 1,024 15.8 | 14.9 at

@@ -2001,11 +2001,14 @@ struct Staged256 {
 };
 // Without a window staged from 576 keys on, or from 512 where tiles outnumber the SIMDs (16 heads over one, us, straight from the cache against
 // staged: prompts of 300 tokens 27 / 29, 512 42 / 41, 600 49 / 47, 1,024 78 / 68, 4,096 591 / 314, eight of 512 124 / 83, 64 tokens behind 8,000
-// 546 / 430; 16 over 16, 512 tokens 42 / 45, 600 49 / 47, eight of 512 156 / 88). Under a window a wave's walk is short, so only where the tiles
-// outnumber the SIMDs and the window is 512 keys and more, or 100 and more with tiles for every group of heads and a quarter of the launched
-// blocks at work (16 over one within 128: 1,024 tokens 20 / 24, 2,048 38 / 26; 32 over 8 within 128, 1,500 tokens beside twelve of 40 80 / 108,
-// four of 700 to 1,500 78 / 63 of 16 over one; within 512, 1,500 beside twelve of 40 84 / 55). Over 1,245 steps nothing was longer than
-// straight from the cache by more than 5 %; staged from 512 keys on whatever else, 549 of them were by more than 2 %, up to 1.9 times.
+// 546 / 430; 16 over 16, 512 tokens 42 / 45, 600 49 / 47, eight of 512 156 / 88). Under a window the one that is done first by a fit, in us: a start,
+// and for every round of blocks (of four waves, one of eight a unit) the keys that a wave, or a block, walks; blocks that a long row's grid launches for
+// the short ones cost a little, and more than half of such leave units with two others. Over 17,000 steps of 17 to 4,000 tokens behind up to 7,900, 4 to 48 heads over 1
+// to 16 and windows of 64 to 4,096 or none, two thirds of them not those of the fit, the choice is 1.1 % from the better form on average: 0.1 % where rows are
+// about as long (22 % at most), 2.1 % where a few are long among short ones, whose blocks the launch lays out as it comes (2.1 times at most). Staged
+// always is 6.9 % from it, from the cache always 31 %; under windows only where tiles outnumber the SIMDs 5.3 %, up to 2.5 times. 16 over one: 304
+// tokens behind 600 within 128 17 / 20, within 512 43 / 42; 1,500 within 128 33 / 23, 384 67 / 36, 1,024 84 / 70; 700 to 1,500 together within 128
+// 72 / 60; 32 over 8, 1,500 beside twelve of 40 within 128 78 / 106.
 static Staged256 stages_256(int heads, int kv_heads, int n_rows, int max_query, int max_len, int window, int tokens) {
   const TileMap tm = tile_map(heads / kv_heads);
   const int64_t most = (int64_t)n_rows * max_query, positions = tokens > 0 && tokens < most ? tokens : most;
@@ -2014,10 +2017,17 @@ static Staged256 stages_256(int heads, int kv_heads, int n_rows, int max_query, 
   const int64_t pairs = std::min<int64_t>((int64_t)n_rows * ((ranges + 1) / 2), positions / (16 * tm.pos_per_tile) + n_rows) * groups;
   Staged256 f{false, ranges, pairs < UNPAIR_BELOW && n_rows <= 32767 ? 1 : 0};
   if (tiles < 16 || max_len < 512) return f;
-  const int64_t launched = (int64_t)n_rows * ((ranges + 1) / 2) * (f.unpaired ? 2 : 1) * groups;
-  const int64_t real = std::min<int64_t>(launched, (positions / (8 * tm.pos_per_tile) + n_rows) * groups), span = std::abs((int64_t)window);
-  if (span == 0) f.pays = max_len >= 576 || waves > 1024;
-  else f.pays = waves > 1024 && (span >= 512 || (span >= 100 && waves > 1024 * tm.head_blocks && 4 * real >= launched));
+  const int64_t span = std::abs((int64_t)window);
+  if (span == 0 || span >= max_len) {
+    f.pays = max_len >= 576 || waves > 1024;
+    return f;
+  }
+  const int64_t launched_waves = (int64_t)n_rows * tiles * groups, launched = (int64_t)n_rows * ((ranges + 1) / 2) * (f.unpaired ? 2 : 1) * groups;
+  const float blocks = fminf((float)launched, (positions / (8 * tm.pos_per_tile) + 0.5f * n_rows) * groups);
+  const float cache_rounds = ceilf(waves * (launched_waves > 2 * waves ? 1.4f : 1.f) / 1024), rounds = ceilf(blocks / 256) * (f.unpaired ? 1 : 2);
+  const auto walk = [&](int positions_too) { return (float)std::min<int64_t>(span + positions_too, max_len); };
+  f.pays = 3.9f + rounds * (9.8f + 0.055f * walk(8 * tm.pos_per_tile)) + 2.f * launched / 256 <
+           1.9f + cache_rounds * (6.4f + 0.0677f * walk(tm.pos_per_tile)) + 0.1f * launched_waves / 1024;
   return f;
 }
 

@@ -1634,7 +1634,8 @@ def test_general_attention_of_short_rows(hip, dtype, heads, kv, d):
 @pytest.mark.parametrize("heads,kv,window,steps", [
     (16, 1, 0, ((0, (540, 530)), (37, (641, 17)), (560, (25, 300)))), (16, 1, 200, ((0, (1030, 97)), (37, (1100, 17)))), (20, 1, 0, ((0, (577, 97)),)),
     (8, 2, 0, ((0, (577, 97)), (490, (130, 300)))), (6, 2, -160, ((0, (2700, 60)),)), (34, 1, 0, ((37, (641, 17)),)), (34, 1, 128, ((0, (1100, 17)),)),
-    (3, 3, 0, ((0, (641, 500)),)), (3, 3, 128, ((0, (5600, 40)),)), (3, 3, 513, ((600, (5600, 900)),))])
+    (3, 3, 0, ((0, (641, 500)),)), (3, 3, 128, ((0, (5600, 40)),)), (3, 3, 513, ((600, (5600, 900)),)),
+    (16, 1, 1024, ((1200, (304, 25)), (1500, (17, 20)))), (32, 8, -768, ((900, (300, 17)),)), (34, 1, 600, ((700, (65, 20)),))])
 def test_heads_of_256_staged_are_the_bits_of_short_portions(hip, heads, kv, window, steps):
     """Two prompts in one step that takes its stages through LDS, behind cached tokens or not: every row bit for bit what portions give
     that are too short for it, under sinks and windows of either kind, whatever later tokens' values are."""
@@ -1670,17 +1671,19 @@ def test_heads_of_256_staged_are_the_bits_of_short_portions(hip, heads, kv, wind
 
 
 def test_which_portions_of_heads_of_256_go_through_lds(hip):
-    """Both sides of the lines: keys without a window, tiles for the SIMDs, windows too narrow, groups of more heads than a tile has rows, a long
-    portion among short ones, rows of more pages than LDS holds."""
+    """Both sides of the lines: keys without a window, tiles for the SIMDs, windows that are narrow, wide or wider than the rows, groups of more
+    heads than a tile has rows, a long portion among short ones, rows of more pages than LDS holds."""
     staged = hip.lib.holon_attention_prefill_one_order_staged
 
     def of(lens, heads, kv, window=0, behind=0, known=True, page=16):
         return staged(heads, kv, len(lens), max(lens), behind + max(lens), page, window, sum(lens) if known else 0)
     assert [of([n], 16, 1) for n in (511, 575, 576)] == [0, 0, 1] and [of([512] * n, 16, 1) for n in (2, 3)] == [0, 1]
     assert [of([n], 16, 16, behind=600) for n in (240, 241)] == [0, 1]                      # (fewer than 16 tiles)
-    assert [of([n], 16, 1, w) for n, w in ((1024, 128), (1100, 128), (1100, 99), (1100, 512), (1024, 512))] == [0, 1, 0, 1, 0]
-    assert [of([n], 34, 1, 128) for n in (1024, 1100)] == [0, 1] and of([600], 34, 1, -512) == 1
-    assert of([600] + [40] * 7, 16, 1, 128) == 0 and of([600] + [40] * 7, 16, 1, 128, known=False) == 1 and of([1500] + [40] * 12, 32, 8, 128) == 0
+    assert [of([n], 16, 1, w) for n, w in ((1024, 128), (1025, 128), (1100, 99), (1100, 512), (1024, 512))] == [0, 1, 1, 1, 0]
+    assert [of([304], 16, 1, w, behind=1200) for w in (384, 440, 480, 512, 1024, -1024)] == [0, 0, 1, 1, 1, 1]
+    assert [of([n], 16, 1, 512, behind=600) for n in (816, 820, 1024, 1028)] == [1, 0, 0, 1] and [of([576], 16, 1, w) for w in (128, 576, 600)] == [0, 1, 1]
+    assert [of([n], 34, 1, 128, behind=300) for n in (341, 342)] == [0, 1] and of([600], 34, 1, -512) == 1 and of([1500] + [40] * 12, 32, 8, 128) == 0
+    assert [of([n] + [40] * 7, 16, 1, 128) for n in (300, 600, 1500)] == [0, 1, 1] and [of([600] + [17] * 7, 16, 1, 128, known=k) for k in (True, False)] == [0, 1]
     assert of([64], 16, 1, behind=65536 - 64) == 1 and of([64], 16, 1, behind=65536 - 63) == 0 and of([64], 16, 1, behind=65536 - 63, page=32) == 1
 
 

@@ -197,25 +197,21 @@ def few_row_waves(n: int, k: int) -> int:
 
 
 @functools.lru_cache(maxsize=1024)
-def beside_pays(m: int, hidden: int, n: int, k: int) -> bool:
-    """Whether a mixture's second product into `hidden` columns and a product of the same m rows over an [n, k] weight share a launch: a block of
-    eight waves for 16 of the mixture's columns, and one for one to eight tiles of the other's. It saves a launch, and where both leave units
-    idle a round of blocks; but blocks that do not fit beside one another wait, the other product's for all of its K. So wherever the blocks of
-    both take fewer rounds of 256 together (0.58 to 0.93 of the time apart), or a wave's loads come in full sets to their end (K a
-    multiple of 4,096); else the narrower the mixture and the more rows, the longer a K may be. Over 2,500 steps (2,048 to 5,120 columns, 8 to
-    128 experts, 1 to 16 rows) nothing so chosen took over 2 % longer than apart, of all of them 9 % did, up to 10 %. Measured, us, together | apart, 8
-    experts unless noted: 2,048 columns beside 2,048 x 2,048 10.1 | 13.9 at one row and 42.5 | 48.1 at 16 (128 experts), 12,288 x 2,048
-    18.2 | 22.3, 2,560 x 5,120 19.2 | 18.0 at two; 2,304 beside 512 x 2,048 6.5 | 10.1 and 3,072 x 1,024 10.4 | 9.9 at one; 2,560 (64 experts) beside
-    2,048 x 6,144 17.5 | 17.3 at one and 30.3 | 38.2 at eight; 3,072 beside 2,048 x 2,816 13.6 | 18.0 at four; 3,584 beside 2,048 x 1,024 15.8 | 14.9 at
-    three; 4,096 (64 experts) beside 4,096 x 2,048 14.1 | 14.1 at one and 52.8 | 51.0 at 16, beside 4,096 x 4,096 16.1 | 17.5 and 54.8 | 56.7."""
-    mixture, product = hidden // 16, -(-(n // 16) // (8 // min(few_row_waves(n, k), 8)))
-    if -(-(mixture + product) // 256) < -(-mixture // 256) + -(-product // 256) or k % 4096 == 0:
-        return True
-    if hidden <= 2048:
-        return k < 4096 or m > 3
-    if hidden <= 2560:
-        return (m > 1 or k >= 1408) and (k < 4096 or m >= 8)
-    return hidden < 4096 and m > 1 and mixture + product <= 336 and 1024 < k < 4096
+def beside_pays(hidden: int, n: int, k: int) -> bool:
+    """Whether a mixture's second product into `hidden` columns and a product of the same rows over an [n, k] weight share a launch: a block of
+    eight waves for 16 of the mixture's columns, and one for one to eight tiles of the other's. It saves a launch, and where either leaves units
+    idle a round of blocks. Where neither is so, the mixture's blocks full rounds of 256 and no round fewer together, the other product's blocks
+    wait for the mixture's units; what they then win is that their loads follow one another without a gap, which takes more than four steps of K
+    a wave. Over 21,700 steps (1,024 to 8,192 columns, 8 to 128 experts, 512 to 12,288 columns of the other, K of 256 to 8,192, 1 to 16 rows, weights from
+    memory) the choice is 0.3 % from the better on average and takes 0.86 of the time apart (always together 0.6 %, never 18 %); 4 % are more than 2 %
+    longer than apart, most of them beside 12,288 columns, up to 21 % beside a small mixture there. In us, 8 experts, one row unless noted, together |
+    apart: 2,048 columns beside 2,048 x 2,048 12.6 | 16.3 and 31.2 | 36.3 at 16, 12,288 x 2,048 16.3 | 19.4; 2,560 beside 2,560 x 1,024 10.4 | 11.3;
+    3,072 beside 2,048 x 1,024 10.7 | 12.5; 3,584 beside 1,024 x 3,584 12.7 | 17.3, 12,288 x 1,024 14.1 | 12.3; 5,120 beside 12,288 x 2,048 at three 32.7 | 42.8;
+    4,096 beside 4,096 x 4,096 15.5 | 16.4, 4,096 x 8,192 at four 26.0 | 26.6, and what stays apart: 4,096 x 2,048 9.7 | 9.8 and 24.7 | 23.2 at 16,
+    2,048 x 1,024 9.4 | 8.6; 8,192 beside 4,096 x 1,024 20.2 | 19.7."""
+    mixture, waves = hidden // 16, few_row_waves(n, k)
+    product = -(-(n // 16) // (8 // min(waves, 8)))
+    return mixture % 256 != 0 or k > 4 * 32 * waves or -(-(mixture + product) // 256) < -(-mixture // 256) + -(-product // 256)
 
 
 def _served(p: Product) -> bool:
@@ -248,7 +244,7 @@ def _linear_group_hip(launch, products: list[Product | Routing | ExpertsDown]) -
             route = routes[rows].pop(0) if routes.get(rows) else None
             if len(group) == 1 and route is None:
                 p = products[group[0]]
-                at = next((d for d in downs.get(rows, ()) if beside_pays(rows, products[d].tiled.shape[0], *p.linear.weight.shape)), None)
+                at = next((d for d in downs.get(rows, ()) if beside_pays(products[d].tiled.shape[0], *p.linear.weight.shape)), None)
                 if at is not None:                        # a mixture's experts beside it (several products fill the chip by themselves)
                     downs[rows].remove(at)
                     out[group[0]], out[at] = _beside(launch_beside, p, products[at])

@@ -770,13 +770,11 @@ def test_products_join_a_launch_of_several_where_that_pays():
 
 
 def test_which_products_a_mixture_shares_a_launch_with():
-    """`beside_pays` on both sides of its lines: rounds of blocks that are saved, full sets of loads, widths of the mixture, rows, long and short K."""
+    """`beside_pays` on both sides of its lines: mixtures whose blocks fill rounds of units and not, rounds that are saved, short and long K of one to
+    sixteen waves a tile."""
     from holon_amd.parts.products import beside_pays
-    assert all(beside_pays(m, 2048, n, k) for m in (1, 16) for n, k in ((2048, 2048), (512, 256), (4096, 4096), (12288, 2048), (8192, 8192), (2048, 6144)))
-    assert [beside_pays(m, 2048, 2560, 5120) for m in (1, 3, 4)] == [False, False, True]                                    # (288 blocks)
-    assert [beside_pays(m, 2560, 2048, k) for m, k in ((1, 1024), (2, 1024), (1, 1408), (1, 6144), (7, 6144), (8, 6144))] == [False, True, True, False, False, True]
-    assert beside_pays(1, 2304, 512, 2048) and not beside_pays(1, 2304, 3072, 1024)
-    assert [beside_pays(m, 3072, 2048, k) for m, k in ((1, 2048), (2, 2048), (2, 1024), (16, 6144), (1, 4096))] == [False, True, False, False, True]
-    assert not beside_pays(2, 3072, 4096, 2048) and beside_pays(2, 3584, 1024, 2048)
-    assert [beside_pays(m, 4096, n, k) for m in (1, 16) for n, k in ((2048, 2048), (4096, 4096), (2048, 6144), (4096, 2048))] == [False, True, False, False] * 2
-    assert beside_pays(1, 5120, 2048, 2048)                                                                                 # (320 and 128: two rounds, not three)
+    assert all(beside_pays(hidden, n, k) for hidden in (32, 2048, 2560, 4064, 4128, 5120) for n, k in ((2048, 2048), (512, 256), (12288, 1024), (16, 32)))
+    assert [beside_pays(4096, n, k) for n, k in ((2048, 2048), (2048, 2560), (4096, 2048), (4096, 4096), (4096, 2080), (12288, 1024), (12288, 1280))] == \
+        [False, True, False, True, True, False, True]
+    assert [beside_pays(8192, 2048, k) for k in (96, 128, 160, 2048, 4096)] == [False, False, True, False, True]      # (one wave a tile, four, one, 16)
+    assert not beside_pays(4096, 4608, 2048)                          # (256 and 288 blocks: three rounds either way)

@@ -2001,12 +2001,13 @@ struct Staged256 {
 };
 // Without a window staged from 576 keys on, or from 512 where tiles outnumber the SIMDs (16 heads over one, us, straight from the cache against
 // staged: prompts of 300 tokens 27 / 29, 512 42 / 41, 600 49 / 47, 1,024 78 / 68, 4,096 591 / 314, eight of 512 124 / 83, 64 tokens behind 8,000
-// 546 / 430; 16 over 16, 512 tokens 42 / 45, 600 49 / 47, eight of 512 156 / 88). Under a window the one that is done first by a fit, in us: a start,
-// and for every round of blocks (of four waves, one of eight a unit) the keys that a wave, or a block, walks; blocks that a long row's grid launches for
-// the short ones cost a little, and more than half of such leave units with two others. Over 17,000 steps of 17 to 4,000 tokens behind up to 7,900, 4 to 48 heads over 1
-// to 16 and windows of 64 to 4,096 or none, two thirds of them not those of the fit, the choice is 1.1 % from the better form on average: 0.1 % where rows are
-// about as long (22 % at most), 2.1 % where a few are long among short ones, whose blocks the launch lays out as it comes (2.1 times at most). Staged
-// always is 6.9 % from it, from the cache always 31 %; under windows only where tiles outnumber the SIMDs 5.3 %, up to 2.5 times. 16 over one: 304
+// 546 / 430; 16 over 16, 512 tokens 42 / 45, 600 49 / 47, eight of 512 156 / 88). Under a window the one that is done first by a fit, in us: a
+// start, for every round of blocks (of four waves from the cache, of eight staged, one a unit) so much a key that a wave or a block walks, and a little
+// for blocks that a long row's grid launches for short ones. Where more than half of the launched have nothing to do, some units get two of the
+// others, as if there were 1.4 times as many. Over 17,000 steps of 17 to 4,000 tokens behind up to 7,900, 4 to 48 heads over 1 to 16 and windows
+// of 64 to 4,096 or none, two thirds of them not those of the fit, the choice is 1.1 % from the better form on average: 0.1 % where rows are about as
+// long (22 % at most), 2.1 % where a few are long among short ones (2.1 times at most: where their blocks land is not known here). Staged always is
+// 6.9 % from it, from the cache always 31 %; under windows staged only where tiles outnumber the SIMDs 5.3 %, up to 2.5 times. 16 over one: 304
 // tokens behind 600 within 128 17 / 20, within 512 43 / 42; 1,500 within 128 33 / 23, 384 67 / 36, 1,024 84 / 70; 700 to 1,500 together within 128
 // 72 / 60; 32 over 8, 1,500 beside twelve of 40 within 128 78 / 106.
 static Staged256 stages_256(int heads, int kv_heads, int n_rows, int max_query, int max_len, int window, int tokens) {

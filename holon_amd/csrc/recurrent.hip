@@ -535,11 +535,12 @@ __global__ void shift_mix_kernel(const T* __restrict__ x, const T* __restrict__ 
 }
 
 // The same, 16 bytes of neighbouring channels a thread and load, for steps of SHIFT_PIECES_FROM values (tokens times channels) and more: below, a
-// block's round of latency is what a step takes, and a thread with more to do makes it longer. In us, pieces against a channel a thread: 2,048
-// tokens of 2,048 mixed five times 13.3 / 22.9 (bfloat16) and 21.1 / 22.5 (float32), 192 tokens 5.6 / 5.9 and 5.9 / 6.0; 384 of 1,024 5.2 / 5.7 and
-// 5.5 / 5.5; 64 of 2,048 5.1 / 4.7 and 5.2 / 4.7, one 5.1 / 4.5 and 5.1 / 4.4. (Eight float32 channels a thread, 32 bytes apart from the next
-// thread's, took up to 1.29 times as long as one.)
-constexpr int64_t SHIFT_PIECES_FROM = 393216;
+// block's round of latency is what a step takes, and a thread with more to do makes it longer. A row's blocks are as many as 256 threads each need,
+// of as many waves as an even share takes. Over 10,560 steps the choice is 0.3 % from the better form on average and up to 14 % (3,136 float32 channels, six
+// mixes). In us, pieces against a channel a thread: 2,058 tokens of 2,048 mixed five times 14.2 / 23.7 (bfloat16), 1,913 20.2 / 21.9 (float32), 196 of
+// 1,920 5.4 / 5.9 and 209 of 2,048 5.8 / 6.0; 383 of 1,024 5.5 / 5.8 and 350 of 1,088 5.8 / 5.9; 69 of 2,048 5.1 / 4.7 and 67 5.1 / 4.6. (Eight
+// float32 channels a thread, 32 bytes apart from the next thread's, took up to 1.29 times as long as one.)
+constexpr int64_t SHIFT_PIECES_FROM = 196608, SHIFT_PIECES_FROM_F32 = 262144;
 template <typename T>
 __global__ void __launch_bounds__(256) shift_mix_rows_kernel(const T* __restrict__ x, const T* __restrict__ mu, T* __restrict__ state,
                                                              T* __restrict__ y, const int32_t* __restrict__ slots,
@@ -548,7 +549,7 @@ __global__ void __launch_bounds__(256) shift_mix_rows_kernel(const T* __restrict
                                                              int keep) {
   constexpr int N = Elem<T>::kVec;
   struct alignas(16) Piece { T v[N]; };
-  const int c = (blockIdx.x * 256 + threadIdx.x) * N;
+  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * N;
   const int t = blockIdx.y;
   if (c >= width) return;
   const int b = keep ? t : token_row[t];
@@ -853,10 +854,10 @@ extern "C" int holon_shift_mix(const void* x, const void* mu, void* state, void*
   const dim3 block(256), grid_t((width + 255) / 256, tokens), grid_b((width + 255) / 256, rows);
   HOLON_CHECK(!rows_in_order || tokens == rows, "shift_mix: rows in order means one token a row, got %d in %d", tokens,
               rows);
-  const int piece = dtype == HOLON_F32 ? Elem<float>::kVec : Elem<bf16_t>::kVec;
-  if ((int64_t)tokens * width >= SHIFT_PIECES_FROM && width % piece == 0 && head_rows::on16(x) && head_rows::on16(mu) && head_rows::on16(state) &&
-      head_rows::on16(y))
-    BY_DTYPE(dtype, (shift_mix_rows_kernel<T><<<dim3((width / piece + 255) / 256, tokens), block, 0, s>>>(
+  const int piece = dtype == HOLON_F32 ? Elem<float>::kVec : Elem<bf16_t>::kVec, per = width / piece, across = (per + 255) / 256;
+  if ((int64_t)tokens * width >= (dtype == HOLON_F32 ? SHIFT_PIECES_FROM_F32 : SHIFT_PIECES_FROM) && width % piece == 0 && head_rows::on16(x) &&
+      head_rows::on16(mu) && head_rows::on16(state) && head_rows::on16(y))
+    BY_DTYPE(dtype, (shift_mix_rows_kernel<T><<<dim3(across, tokens), ((per + across - 1) / across + 63) / 64 * 64, 0, s>>>(
                         (const T*)x, (const T*)mu, (T*)state, (T*)y, slots, starts, query_start, token_row, tokens, width, mixes,
                         rows_in_order)));
   else

@@ -2202,12 +2202,13 @@ def test_rows_in_pieces_are_the_rows_value_by_value(hip, dtype):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_shifts_of_many_tokens_in_pieces_are_those_channel_by_channel(hip, dtype):
-    """Steps on both sides of the size from which a thread takes 16 bytes of channels (393,216 values), widths that do not fill a block, in one
-    piece of float32 alone, rows of one token and of many, behind kept tokens and not, in order and not: bit for bit what operands off a border of
+    """Steps on both sides of the size from which a thread takes 16 bytes of channels (196,608 values, 262,144 in float32), widths that do not fill
+    a block or two, in pieces of float32 alone, rows of one token and of many, behind kept tokens and not, in order and not: bit for bit what operands off a border of
     16 bytes give, which go channel by channel; against the plain form a rounding or two of the result's type."""
     from holon_amd.kernels.registry import kernel_op
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")                      # noqa: E731
-    for tokens, width, mixes in ((191, 2048, 5), (192, 2048, 5), (200, 2056, 3), (203, 2060, 2), (96, 4096, 1), (24576, 16, 2), (50, 7872, 2)):
+    for tokens, width, mixes in ((95, 2048, 5), (96, 2048, 5), (127, 2048, 2), (128, 2048, 5), (200, 2056, 3), (203, 2060, 2), (96, 4096, 1), (24576, 16, 2), (50, 7872, 2),
+                                 (260, 1032, 2)):
         counts = [1, 5, tokens - 6]
         first, row = i32([0, 1, 6, tokens]), torch.repeat_interleave(torch.arange(3), torch.tensor(counts)).to(torch.int32).cuda()
         x, mu, kept = _randn(tokens, width, dtype=dtype, seed=216), _randn(mixes, width, dtype=dtype, seed=217), _randn(4, width, dtype=dtype, seed=218)

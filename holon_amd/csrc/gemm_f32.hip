@@ -164,8 +164,8 @@ __global__ void __launch_bounds__(256) gemm_f32_in_order_kernel(const float* __r
 // 17 to 2,048, weights from memory (1.6 GB of them in turn: back to back over three weights that stay in the last-level cache, staged forms
 // look up to a third faster than behind a model's other products), in us: a start, and so much for every round of one block a CU, linear in K.
 // Tiles straight from memory add a part of K to that; of staged ones a block that has its unit to itself takes longer than its share of a full
-// one, `start_k` a k. The choice is 0.3 % from the best form on average and 9 % at most, 0.1 and 5 % of those above 60 us; over 160 products
-// that the fit has not seen 0.3 and 9 %. In us, best and others: 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10; with a 64 x 64 tile a
+// one, `start_k` a k. The choice is 0.3 % from the best form on average and 9 % at most; over 2,850 products that the fit has not seen 0.6 and 11 %
+// from K = 512 on, up to 24 % below (of 3 to 15 us, where K is 64 or less). In us, best and others: 2048 x 2048 takes 1 x 1 tiles up to 32 rows (10; with a 64 x 64 tile a
 // block and no split of K it took 118), 1 x 2 at 64 (16), 2 x 4 at 145 (34; staged 39 to 48), quarters side by side from 300 rows (39; one
 // after the other 48), blocks of 32 rows at 700 (65; of 64 rows 76, whose second round is mostly empty); 2048 x 9248 at 704 rows blocks of
 // 32 (274; of 64 312); 16384 x 2048 1 x 1 tiles up to 16 rows (5.0 TB/s at one row), blocks of 32 at 150 (117; of 64 122), of 64 at 825

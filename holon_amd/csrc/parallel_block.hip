@@ -456,13 +456,16 @@ static int one_type(const void* d1, int dt1, const void* d2, int dt2, const void
 }
 
 // Whether rows of bfloat16 terms under float32 weights ask ahead: a block then holds eight to twelve registers more a step, so that of the
-// 2,048 blocks that the chip holds of the general form some wait for a second round. Where that shows is an added vector without terms from
-// 1,025 rows on (2,048 rows of 2,560 / 3,072 / 4,096 9.4 / 10.8 / 14.8 us, in the general form 9.0 / 9.9 / 12.6), and about 2,048 rows of up to 2,560
-// (one term, two weights 12.5 / 11.9). Elsewhere it is 0.71 to 1.03 of the general form's time: four rows of 2,048 2.4 / 3.2, 512 with two terms
-// 0.84, 8,192 0.96.
-static bool wide_ahead_pays(int64_t rows, int dim, bool terms, bool added) {
-  if (rows > 2048) return true;
-  return added && !terms ? rows <= 1024 || dim <= 2048 : rows <= 1792 || dim <= 1536 || dim > 2560;
+// 2,048 blocks that the chip holds of the general form some wait for a second round. Where that shows, rows that come from memory, us, ahead against
+// the general form: an added vector without terms from 1,025 rows on and 2,052 to 3,072 values (2,009 rows of 2,548 13.6 / 13.1, with two weights 1,997
+// of 2,576 18.1 / 16.9; 1,996 of 3,680 21.0 / 21.5), and from 1,793 rows on with two weights and at most one term, up to 2,560 values (2,004 of 1,592
+// 12.9 / 11.1, without a term 2,006 of 2,328 11.9 / 11.2; two terms and one weight 1,990 of 2,052 14.0 / 14.8). Over 6,900 steps of 1,025 to 2,048
+// rows there the general form is 0.96 of the time ahead on average, and where it is not taken 1.02. Elsewhere ahead is 0.71 to 1.03 of the
+// general form's time: four rows of 2,048 2.4 / 3.2, 512 with two terms 0.84, 8,192 0.96.
+static bool wide_ahead_pays(int64_t rows, int dim, int terms, bool added, bool second) {
+  if (rows <= 1024 || rows > 2048) return true;
+  if (added && terms == 0) return dim <= 2048 || dim > 3072;
+  return terms == 2 || !second || rows <= 1792 || dim <= 1536 || dim > 2560;
 }
 
 extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void* d2, int dt2, const float* row,
@@ -478,7 +481,7 @@ extern "C" int holon_stream_rms(float* x32, const void* d1, int dt1, const void*
     const Filters none{};
     const int one = one_type(d1, dt1, d2, dt2, w1, dtw, dt_out);
     const bool wide_weights = w1 && dtw == HOLON_F32 && one_type(d1, dt1, d2, dt2, w1, dt_out, dt_out) == HOLON_BF16 &&
-                              wide_ahead_pays(rows, dim, d1 != nullptr, row != nullptr);
+                              wide_ahead_pays(rows, dim, (d1 != nullptr) + (d2 != nullptr), row != nullptr, w2 != nullptr);
 #define SRMSV(...) stream_rms_vec_kernel<__VA_ARGS__><<<(unsigned)rows, 256, 0, s>>>(x32, d1, dt1, d2, dt2, row, w1, w2, dtw, y1, y2, dim, eps, dt_out, none)
 #define SRMSV_BY_TYPE(R)                                 \
   do {                                                   \

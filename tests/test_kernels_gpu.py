@@ -1989,7 +1989,7 @@ def test_many_stream_rows_under_float32_weights(hip, rows):
     """bfloat16 terms under float32 weights on both sides of the rows and widths from which they are not asked for ahead: bit for bit the
     general form (taken by results in float32 under bfloat16 weights, rounded here)."""
     import holon_amd.parts.parallel_block  # noqa: F401  (brings the operations)
-    for dim in (1536, 1540, 2048, 2052, 2560, 2564, 4096):
+    for dim in (1536, 1540, 2048, 2052, 2560, 2564, 3072, 3076, 4096):
         x, row = _randn(rows, dim, dtype=torch.float32, seed=229), _randn(dim, dtype=torch.float32, seed=230)
         t1, (w1, w2) = _randn(rows, dim, dtype=torch.bfloat16, seed=231), (_randn(dim, dtype=torch.bfloat16, seed=s) for s in (232, 233))
         for terms, added, second in (([], None, None), ([], row, w2), ([t1], None, w2), ([t1, t1], row, None)):
